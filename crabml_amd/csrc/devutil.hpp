@@ -20,6 +20,14 @@ __device__ __forceinline__ unsigned short f2h(float f) {
   __builtin_memcpy(&h, &x, 2);
   return h;
 }
+// eight f16 x f16 products, exact in f32, added to s one after the other
+__device__ __forceinline__ float dot_f16x8(i32x4 a, i32x4 b, float s) {
+  typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+  const h8 x = __builtin_bit_cast(h8, a), y = __builtin_bit_cast(h8, b);
+#pragma unroll
+  for (int e = 0; e < 8; e++) s = __builtin_fmaf((float)x[e], (float)y[e], s);
+  return s;
+}
 // bfloat16: the upper half of an f32 (exact), and back with round-to-nearest-even
 __device__ __forceinline__ float bf2f(unsigned short h) { return __builtin_bit_cast(float, (unsigned)h << 16); }
 __device__ __forceinline__ unsigned short f2bf(float f) {

@@ -23,6 +23,7 @@
 #include "fused_common.hpp"
 #include "fused_attention.hpp"
 #include "fused_ffn.hpp"
+#include "gemm_bf16.hpp"
 #include "prefill_rows.hpp"
 #include "lazy.hpp"
 
@@ -185,6 +186,7 @@ struct crabml_hip_llama {
   char *pf_act_dim = nullptr, *pf_act_hid = nullptr;
   float* pf_split = nullptr;  // ... and pf_split_floats of scratch for the partial tiles of its k pieces
   size_t pf_split_floats = 0;
+  unsigned* pf_ticks = nullptr;  // (F16 layers) GEMM_TICKS counters of tiles whose k is cut, zero between launches
   void* pf_xh2 = nullptr;  // a second one: the gate | up launch reads pf_xh while its epilogue writes ffn_down's
   void* pf_xh = nullptr;  // the fast pass's f16 GEMMs: the current rhs rows as pre-scaled f16 (gemm_f16w.hip), gemm_f16w_xh_bytes(cap, max(dim, hidden))
   float* pf_scores = nullptr;          // long prompts: [PF_LONG_ROWS][n_heads][seq_len] f32 scores
@@ -1068,6 +1070,12 @@ int prefill_alloc(crabml_hip_llama* c, size_t cap) {
     CH_TRY(A(c->pf_split_floats * 4, (void**)&c->pf_split));
     CH_HIP(c->dev, hipMemsetAsync(c->pf_xh, 0, xb, c->dev->stream));
   }
+  if (c->qt == CRABML_HIP_F16 && !c->dev->strict_order) {  // (pieces of k of a short pass's GEMMs: gemm_f16.hip)
+    c->pf_split_floats = (size_t)8 << 20;
+    CH_TRY(A(c->pf_split_floats * 4, (void**)&c->pf_split));
+    CH_TRY(A(GEMM_TICKS * sizeof(unsigned), (void**)&c->pf_ticks));
+    CH_HIP(c->dev, hipMemsetAsync(c->pf_ticks, 0, GEMM_TICKS * sizeof(unsigned), c->dev->stream));
+  }
   c->pf_cap = cap;
   return 0;
 }
@@ -1228,6 +1236,19 @@ int prefill_chunk(crabml_hip_llama* c, const uint32_t* tokens, size_t B, size_t 
     xh_order = order;
     return planes;
   };
+  // F16 weights on the fast device: matrix cores from two rows on, q | k | v and gate | up as one launch each (false: not covered)
+  auto gemm_f16 = [&](std::initializer_list<const crabml_hip_buf*> w, std::initializer_list<size_t> n, size_t k, const void* act,
+                      std::initializer_list<float*> out) -> bool {
+    if (strict || c->qt != CRABML_HIP_F16) return false;
+    const void* wp[3];
+    int i = 0;
+    for (const crabml_hip_buf* b : w) {
+      if (b->dtype != CRABML_HIP_F16) return false;
+      wp[i++] = b->ptr;
+    }
+    return launch_gemm_f16(dev, nullptr, wp, n.begin(), i, k, act, act_layout(CRABML_HIP_F16, k).total, B, out.begin(),
+                           GemmScratch{c->pf_split, c->pf_split_floats, c->pf_ticks});
+  };
   // defer (nullable): a GEMM cut into k pieces may leave the sum of its pieces to the row kernel that consumes `out` (pf_split holds them)
   auto gemm = [&](const crabml_hip_buf* w, int m, int k, const void* act, float* out, int* defer = nullptr) -> int {
     if (defer) *defer = 0;
@@ -1237,6 +1258,7 @@ int prefill_chunk(crabml_hip_llama* c, const uint32_t* tokens, size_t B, size_t 
       const size_t mm = (size_t)m;
       if (launch_gemm_f16w(dev, &w, &mm, 1, (size_t)k, c->pf_xh, B, &out, c->pf_split, c->pf_split_floats, nullptr, nullptr, defer)) return 0;
     }
+    if (gemm_f16({w}, {(size_t)m}, (size_t)k, act, {out})) return 0;
     if (!strict) {
       return launch_gemv(dev, w, m, k, act, B, out, nullptr, !gemm_exact_hook);
     }
@@ -1346,6 +1368,8 @@ int prefill_chunk(crabml_hip_llama* c, const uint32_t* tokens, size_t B, size_t 
       float* outs[3] = {c->pf_q, c->pf_k, c->pf_v};
       qkv_done = launch_gemm_f16w(dev, ws, ms, 3, (size_t)dim, c->pf_xh, B, outs, c->pf_split, c->pf_split_floats);
     }
+    if (!qkv_done)
+      qkv_done = gemm_f16({c->wq[l], c->wk[l], c->wv[l]}, {(size_t)dim, (size_t)kv_dim, (size_t)kv_dim}, (size_t)dim, a, {c->pf_q, c->pf_k, c->pf_v});
     if (!qkv_done) {
       CH_TRY(gemm(c->wq[l], dim, dim, a, c->pf_q));
       CH_TRY(gemm(c->wk[l], kv_dim, dim, a, c->pf_k));
@@ -1426,6 +1450,7 @@ int prefill_chunk(crabml_hip_llama* c, const uint32_t* tokens, size_t B, size_t 
         xh_order = hq_order;
       }
     }
+    if (!gu_done) gu_done = gemm_f16({c->gate[l], c->up[l]}, {(size_t)hidden, (size_t)hidden}, (size_t)dim, a, {c->pf_g, c->pf_u});
     if (!gu_done) {
       CH_TRY(gemm(c->gate[l], hidden, dim, a, c->pf_g));
       CH_TRY(gemm(c->up[l], hidden, dim, a, c->pf_u));

@@ -6,23 +6,8 @@
 
 namespace crabml_hip {
 
-// 16 bytes per lane from memory into LDS at l + 16 lane (l: wave-uniform).  As assembly, because the compiler would wait for ALL of them
-// in front of the next LDS read (it cannot tell the buffers apart); who waits for what is landed_barrier's business.
-// (m0, the LDS address of such a load, needs one wait state behind its write; nothing else here uses it.)
-__device__ __forceinline__ void lds_dma16(const void* g, const void* l) {
-  const unsigned at = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(size_t)(const __attribute__((address_space(3))) void*)l);
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(at) : "memory");
-}
 // four values as f32 / as bf16 planes (16- and 8-byte stores)
 __device__ __forceinline__ void store4(float* p, const float (&v)[4]) { *(f32x4*)p = f32x4{v[0], v[1], v[2], v[3]}; }
-
-// S > 1: k is cut into S pieces, one workgroup each.  A workgroup leaves its accumulators in ws (write-through) and counts itself in; the
-// one that comes last adds the others' pieces to its own, in piece order, and goes on to the epilogue.  The counter is left at zero.
-// waits until at most N of this wave's memory requests are outstanding, then for the workgroup.  (__syncthreads would drain them all.)
-template <int N>
-__device__ __forceinline__ void landed_barrier() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
-}
 
 // (NS: GEMM_OUT_STREAMS with up to that many streams)
 template <int BM, int BN, int WGM, int WGN, int ST, int P, int OUT, int NS>
@@ -106,44 +91,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_bf16(const GemmBf16 g, 
     }
     buf = buf + 1 == ST ? 0 : buf + 1;
   }
-  if (S > 1) {
-    constexpr int FRAG = TM * TN * 2;  // 8-byte halves of a lane's accumulators
-    unsigned long long* base = (unsigned long long*)ws + (size_t)tile * S * NT * FRAG + tid;
-    unsigned long long* mine = base + (size_t)piece * NT * FRAG;
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-      for (int j = 0; j < TN; j++)
-#pragma unroll
-        for (int e = 0; e < 2; e++) {
-          const f32x2 v = {acc[i][j][2 * e], acc[i][j][2 * e + 1]};
-          __hip_atomic_store(mine + ((i * TN + j) * 2 + e) * NT, __builtin_bit_cast(unsigned long long, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's write-through stores have been acknowledged
-    __shared__ unsigned s_last;
-    __syncthreads();
-    if (tid == 0) s_last = __hip_atomic_fetch_add(tick + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(S - 1);
-    __syncthreads();
-    if (!s_last) return;
-    if (tid == 0) __hip_atomic_store(tick + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-      for (int j = 0; j < TN; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int q = 0; q < S; q++) {  // (its own piece from memory as well: one order of addition, whoever is last)
-      const unsigned long long* p = base + (size_t)q * NT * FRAG;
-#pragma unroll
-      for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++)
-#pragma unroll
-          for (int e = 0; e < 2; e++) {
-            const f32x2 v = __builtin_bit_cast(f32x2, __hip_atomic_load(p + ((i * TN + j) * 2 + e) * NT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-            acc[i][j][2 * e] += v[0];
-            acc[i][j][2 * e + 1] += v[1];
-          }
-    }
-  }
+  if (S > 1 && !add_pieces<TM * TN, NT>((f32x4*)acc, S, piece, tile, ws, tick)) return;
   // epilogue: the tile goes through LDS in slabs of HR rows, so that a thread has eight neighbouring columns of a row
   float* lc = (float*)lds;            // [HR][LC]
   float* lf = lc + HR * LC;           // [BM] row factors
@@ -395,21 +343,17 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_bf16(const GemmBf16 g, 
 
 // Tile and k pieces.  A CU's time for a step of 64 (tile by tile, one workgroup after the other or side by side) and a workgroup's own
 // chain of steps are what was measured; a cut of k costs the hand-over of the pieces.
-struct GemmPlan {
-  int bm, S;
-};
 struct TileCost {
   int bm, resident;     // workgroups of this tile a CU holds
   double step, chain;   // us per step of 64: a workgroup's share of a busy CU; the latency of one alone
 };
-static GemmPlan plan(const GemmBf16& g, int planes, int n_cu, size_t ws_floats) {
+GemmPlan gemm_plan(int M, int col_tiles, int steps, int n_cu, size_t ws_floats) {
   static const TileCost costs[] = {{256, 1, 1.03, 1.03}, {128, 1, 0.68, 0.68}, {64, 2, 0.42, 0.51}, {32, 2, 0.41, 0.41}};
   GemmPlan best{128, 1};
   double best_cost = 1e30;
-  const int steps = g.K / 64 * planes;
   for (const TileCost& t : costs) {
-    if (t.bm > 32 && g.M <= t.bm / 2) continue;
-    const int tiles = ((g.M + t.bm - 1) / t.bm) * ((g.N + 127) / 128);
+    if (t.bm > 32 && M <= t.bm / 2) continue;
+    const int tiles = ((M + t.bm - 1) / t.bm) * col_tiles;
     for (int S : {1, 2, 3, 4, 6, 8}) {
       if (S > 1 && (steps / S < 6 || (size_t)tiles * S * t.bm * 128 > ws_floats || tiles > GEMM_TICKS)) break;
       const double per = (double)steps / S, wgs = (double)tiles * S, rounds = ceil(wgs / (n_cu * t.resident));
@@ -427,7 +371,7 @@ static GemmPlan plan(const GemmBf16& g, int planes, int n_cu, size_t ws_floats) 
     return h && h[0] == '1' && e ? atoi(e) : 0;
   }();
   if (force) {
-    const int bm = force / 100, S = force % 100, tiles = ((g.M + bm - 1) / bm) * ((g.N + 127) / 128);
+    const int bm = force / 100, S = force % 100, tiles = ((M + bm - 1) / bm) * col_tiles;
     if ((bm == 256 || bm == 128 || bm == 64 || bm == 32) && S >= 1 && S <= steps && (S == 1 || ((size_t)tiles * S * bm * 128 <= ws_floats && tiles <= GEMM_TICKS))) return {bm, S};
   }
   return best;
@@ -435,7 +379,7 @@ static GemmPlan plan(const GemmBf16& g, int planes, int n_cu, size_t ws_floats) 
 
 template <int P, int OUT, int NS = 0>
 static void launch_t(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemmBf16& g, int n_cu, const GemmScratch& w) {
-  const GemmPlan p = plan(g, P, n_cu, w.floats);
+  const GemmPlan p = gemm_plan(g.M, (g.N + 127) / 128, g.K / 64 * P, n_cu, w.floats);
   const dim3 grid(((g.M + p.bm - 1) / p.bm) * ((g.N + 127) / 128) * p.S);
   if (p.bm == 256)
     launch_k(st, rec, k_gemm_bf16<256, 128, 4, 2, 3, P, OUT, NS>, grid, dim3(512), 0, g, p.S, w.partials, w.ticks);

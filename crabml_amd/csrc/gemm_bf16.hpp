@@ -82,6 +82,58 @@ __device__ __forceinline__ void read8(const float* p, float (&o)[8]) {
   }
 }
 
+// 16 bytes per lane from memory into LDS at l + 16 lane (l: wave-uniform).  As assembly, because the compiler would wait for ALL of them
+// in front of the next LDS read (it cannot tell the buffers apart); who waits for what is landed_barrier's business.
+// (m0, the LDS address of such a load, needs one wait state behind its write; nothing else here uses it.)
+__device__ __forceinline__ void lds_dma16(const void* g, const void* l) {
+  const unsigned at = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(size_t)(const __attribute__((address_space(3))) void*)l);
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(at) : "memory");
+}
+// waits until at most N of this wave's memory requests are outstanding, then for the workgroup.  (__syncthreads would drain them all.)
+template <int N>
+__device__ __forceinline__ void landed_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+// S > 1: k is cut into S pieces, one workgroup each.  A workgroup leaves its accumulators (F fragments a thread, NT threads) in ws
+// (write-through) and counts itself in; the one that comes last adds all pieces in piece order, whoever it is, and goes on to the epilogue
+// (true).  The counter is left at zero.
+template <int F, int NT>
+__device__ __forceinline__ bool add_pieces(f32x4* acc, int S, int piece, int tile, float* ws, unsigned* tick) {
+  constexpr int FRAG = F * 2;  // 8-byte halves of a thread's accumulators
+  const int tid = threadIdx.x;
+  unsigned long long* base = (unsigned long long*)ws + (size_t)tile * S * NT * FRAG + tid;
+  unsigned long long* mine = base + (size_t)piece * NT * FRAG;
+#pragma unroll
+  for (int i = 0; i < F; i++)
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+      const f32x2 v = {acc[i][2 * e], acc[i][2 * e + 1]};
+      __hip_atomic_store(mine + (i * 2 + e) * NT, __builtin_bit_cast(unsigned long long, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's write-through stores have been acknowledged
+  __shared__ unsigned s_last;
+  __syncthreads();
+  if (tid == 0) s_last = __hip_atomic_fetch_add(tick + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(S - 1);
+  __syncthreads();
+  if (!s_last) return false;
+  if (tid == 0) __hip_atomic_store(tick + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+  for (int i = 0; i < F; i++) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int q = 0; q < S; q++) {
+    const unsigned long long* p = base + (size_t)q * NT * FRAG;
+#pragma unroll
+    for (int i = 0; i < F; i++)
+#pragma unroll
+      for (int e = 0; e < 2; e++) {
+        const f32x2 v = __builtin_bit_cast(f32x2, __hip_atomic_load(p + (i * 2 + e) * NT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        acc[i][2 * e] += v[0];
+        acc[i][2 * e + 1] += v[1];
+      }
+  }
+  return true;
+}
+
 struct GemmBf16 {
   const unsigned short* a = nullptr;  // [planes][rows padded][k]
   size_t a_plane = 0;                 // elements between planes
@@ -117,6 +169,22 @@ struct GemmScratch {
   float* partials = nullptr;
   size_t floats = 0;
   unsigned* ticks = nullptr;
+};
+// rows of a tile and pieces of k for M rows x col_tiles tiles of 128 columns, `steps` steps of 64
+struct GemmPlan {
+  int bm, S;
+};
+GemmPlan gemm_plan(int M, int col_tiles, int steps, int n_cu, size_t ws_floats);
+
+// gemm_f16.hip: F16 weights
+struct GemmF16 {
+  const void* a = nullptr;  // rows of f16, a_stride bytes apart (a multiple of 16)
+  size_t a_stride = 0;
+  const unsigned short* w[3] = {nullptr, nullptr, nullptr};  // [n][K]
+  float* out[3] = {nullptr, nullptr, nullptr};               // [M][n]
+  int n[3] = {0, 0, 0};
+  int end[3] = {0, 0, 0};  // column tiles up to and with this matrix
+  int M = 0, K = 0;
 };
 // planes: 1 or 3 (GEMM_OUT_ACT_BF16 goes with one, GEMM_OUT_ACT_F32 with three)
 void launch_gemm_bf16(crabml_hip_device* dev, crabml_hip_device::ProfRec* rec, int planes, int out, const GemmBf16& g, const GemmScratch& w);

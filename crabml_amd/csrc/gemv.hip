@@ -16,7 +16,7 @@
 // CPU loop (lane-strided partial sums + a 64-lane butterfly), which is why logits carry an fp tolerance.
 // The kernel is HBM-bound (~3.6 flop/byte): no LDS round trip, no MFMA; x is re-read from L1/L2.
 #include "gemv_core.hpp"
-#include "gemv_bf16.hpp"
+#include "gemm_bf16.hpp"
 
 namespace crabml_hip {
 
@@ -238,9 +238,59 @@ __global__ __launch_bounds__(256) void k_gemv_f32(const float* __restrict__ w, c
   acc = wave_sum_f32(acc);
   if (lane == 0) out[row] = acc;
 }
-__global__ __launch_bounds__(256) void k_gemv_f16(const unsigned short* __restrict__ w,
-                                                  const unsigned short* __restrict__ x16, float* __restrict__ out,
-                                                  int m, int k) {
+// F16 rows: a lane takes 16 bytes of R neighbouring rows and of the rhs at a time (UN steps of 512 elements in flight), products are exact in
+// f32 (v_fma_mix_f32: no conversions), sums f32.  Bound by the weights' bytes: 32000 x 2048 25.9 us (5.1 TB/s; two bytes a lane at a time:
+// 68.6), 8192 x 2048 7.8 (9.3), 2048 x 8192 10.4 (36).
+template <int R>
+__global__ __launch_bounds__(256) void k_gemv_f16(const unsigned short* __restrict__ w, const unsigned short* __restrict__ x16,
+                                                  float* __restrict__ out, int m, int k) {
+  constexpr int UN = R >= 4 ? 2 : 4;
+  const int lane = threadIdx.x & 63;
+  const int row0 = (blockIdx.x * (blockDim.x >> 6) + wave_in_wg()) * R;
+  if (row0 >= m) return;
+  const unsigned short* wr[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) wr[r] = w + (size_t)(row0 + r < m ? row0 + r : m - 1) * k;
+  i32x4 wv[UN][R], xv[UN];
+  auto request = [&](int k0) {
+#pragma unroll
+    for (int u = 0; u < UN; u++) {
+      int i = k0 + u * 512 + lane * 8;
+      i = i < k ? i : 0;  // (a lane past the end requests the row's start and never uses it)
+#pragma unroll
+      for (int r = 0; r < R; r++) wv[u][r] = __builtin_nontemporal_load((const i32x4*)(wr[r] + i));
+      xv[u] = *(const i32x4*)(x16 + i);
+    }
+  };
+  request(0);
+  float acc[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) acc[r] = 0.f;
+  for (int k0 = 0; k0 < k; k0 += UN * 512) {
+    i32x4 wc[UN][R], xc[UN];
+#pragma unroll
+    for (int u = 0; u < UN; u++) {
+#pragma unroll
+      for (int r = 0; r < R; r++) wc[u][r] = wv[u][r];
+      xc[u] = xv[u];
+    }
+    if (k0 + UN * 512 < k) request(k0 + UN * 512);
+#pragma unroll
+    for (int u = 0; u < UN; u++)
+      if (k0 + u * 512 + lane * 8 < k) {
+#pragma unroll
+        for (int r = 0; r < R; r++) acc[r] = dot_f16x8(wc[u][r], xc[u], acc[r]);
+      }
+  }
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const float s = wave_sum_f32(acc[r]);
+    if (lane == 0 && row0 + r < m) out[row0 + r] = s;
+  }
+}
+// F16 rows that are not whole 16-byte pieces
+__global__ __launch_bounds__(256) void k_gemv_f16_any(const unsigned short* __restrict__ w, const unsigned short* __restrict__ x16,
+                                                      float* __restrict__ out, int m, int k) {
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * (blockDim.x >> 6) + wave_in_wg();
   if (row >= m) return;
@@ -298,6 +348,10 @@ int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m_, size
     g.nb = (int)b;
     launch_gemv_bf16<GEMV_IN_PLAIN, GEMV_OUT_STORE>(st, rec0, g);
     return 0;
+  }
+  if (w->dtype == CRABML_HIP_F16 && b >= 2) {
+    const void* ws[1] = {wp};
+    if (launch_gemm_f16(dev, rec0, ws, &m_, 1, k_, act, al.total, b, &out, GemmScratch{})) return 0;
   }
   if (b >= 16 && launch_gemm_mfma(dev, w, m_, k_, act, b, out, rec0, nullptr, fused_add)) return 0;
   for (size_t bi = 0; bi < b; bi++) {
@@ -428,8 +482,15 @@ int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m_, size
         break;
       }
       case CRABML_HIP_F16: {
-        int grid = (m + 3) / 4;
-        launch_k(st, rec, k_gemv_f16, dim3(grid), dim3(256), 0, (const unsigned short*)wp, (const unsigned short*)ap, o, m, k);
+        const unsigned short *wh = (const unsigned short*)wp, *xh = (const unsigned short*)ap;
+        if (k % 8 != 0)
+          launch_k(st, rec, k_gemv_f16_any, dim3((m + 3) / 4), dim3(256), 0, wh, xh, o, m, k);
+        else if (m >= 16384)  // (enough rows to give a wave four and still fill the chip)
+          launch_k(st, rec, k_gemv_f16<4>, dim3((m + 15) / 16), dim3(256), 0, wh, xh, o, m, k);
+        else if (m >= 2048)
+          launch_k(st, rec, k_gemv_f16<2>, dim3((m + 7) / 8), dim3(256), 0, wh, xh, o, m, k);
+        else
+          launch_k(st, rec, k_gemv_f16<1>, dim3((m + 3) / 4), dim3(256), 0, wh, xh, o, m, k);
         break;
       }
       case CRABML_HIP_BF16: {

@@ -76,6 +76,11 @@ bool launch_gemm_f16w(crabml_hip_device* dev, const crabml_hip_buf* const* w, co
 // defer_parts (one matrix): a launch cut into k pieces leaves piece 0 in out and pieces 1.. in ws (b * m floats apart) and returns
 // their number instead of launching the reduce: the row kernel that consumes out adds them first, in piece order (prefill_rows.hpp)
 // gu_exp_tab / gu_done (two matrices = ffn_gate, ffn_up): the launch may store h = silu(g) * u to out[0] instead of g and u (*gu_done = 1)
+// gemm_f16.hip: F16 weights x f16 rows (act_stride bytes apart), up to three matrices of one rhs; without scratch k stays whole.
+// false = not covered (one row, rows that are not whole 16-byte pieces)
+struct GemmScratch;
+bool launch_gemm_f16(crabml_hip_device* dev, crabml_hip_device::ProfRec* rec, const void* const* w, const size_t* n, int nw, size_t k,
+                     const void* act, size_t act_stride, size_t rows, float* const* out, const GemmScratch& ws);
 // batched rhs on the matrix cores (gemm_mfma.hip); false = not covered
 bool launch_gemm_mfma(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m, size_t k, const void* act, size_t b, float* out,
                       crabml_hip_device::ProfRec* rec, int* dbg = nullptr, bool fused_add = false);

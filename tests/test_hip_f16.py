@@ -1,0 +1,51 @@
+"""F16 weights on the fast device: the row kernel (one row of the rhs) and the matrix-core GEMM (two rows and more) behind matmul_vec and the
+prompt pass, against float64 on the rhs as the reference rounds it (f16, buf_f16.rs:83-97)."""
+import numpy as np
+import pytest
+
+from crabml_amd import synth
+from tests.helpers import FAST_TOL, GEMV_REL
+
+pytestmark = pytest.mark.gpu
+
+# (m, k, rows): one row; ragged m and rows; a tail of k shorter than a step of 64; k that is not whole 16-byte pieces; every tile height
+SHAPES = [(1, 8, 1), (5, 72, 1), (16385, 520, 1), (2050, 4104, 1), (33, 70, 1), (33, 70, 3), (1, 8, 2), (130, 72, 33), (128, 64, 2), (257, 328, 129),
+          (300, 512, 256), (96, 4096, 300), (1027, 136, 65), (2048, 2048, 31)]
+
+
+@pytest.mark.parametrize("m,k,rows", SHAPES)
+def test_matmul_vec_f16(ca, hdev, m, k, rows):
+    rng = np.random.default_rng(m * 31 + k * 7 + rows)
+    w = rng.standard_normal((m, k)).astype(np.float16)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    t = ca.HipTensor.from_cpu(w.view(np.uint8).reshape(-1), [m, k], ca.GGMLType.F16, hdev)
+    got = t.matmul_vec(ca.HipTensor.new(x.reshape(-1), [rows, k], hdev)).export().reshape(rows, m)
+    wd, xd = w.astype(np.float64), x.astype(np.float16).astype(np.float64)
+    assert np.all(np.abs(got - xd @ wd.T) <= GEMV_REL * (np.abs(xd) @ np.abs(wd).T))
+
+
+def test_matmul_vec_f16_infinite_and_nan_rows_stay_apart(ca, hdev):
+    """a row of the rhs that holds an infinity or a NaN changes that row's results only; so do the weights' rows"""
+    rng = np.random.default_rng(3)
+    w, x = rng.standard_normal((37, 72)).astype(np.float16), rng.standard_normal((35, 72)).astype(np.float32)
+    w[36, 71], x[34, 71], x[5, 0] = np.inf, np.nan, np.inf
+    t = ca.HipTensor.from_cpu(w.view(np.uint8).reshape(-1), [37, 72], ca.GGMLType.F16, hdev)
+    got = t.matmul_vec(ca.HipTensor.new(x.reshape(-1), [35, 72], hdev)).export().reshape(35, 37)
+    rows = [r for r in range(35) if r not in (5, 34)]
+    assert np.isfinite(got[rows][:, :36]).all() and np.isinf(got[rows][:, 36]).all()
+    assert np.isnan(got[34]).all() and not np.isfinite(got[5]).any()
+
+
+@pytest.mark.parametrize("rows", [2, 65, 203])
+def test_prompt_pass_equals_the_token_loop(ca, rows):
+    """one prompt pass (k of its GEMMs cut into pieces at this width) against the same tokens one by one"""
+    shape = synth.ModelShape("f16", 2048, 2304, 1, 16, 4, 1000, 256)
+    dev = ca.HipTensorDevice(0)
+    conf, w = synth.to_hip(synth.build_model(shape, synth.F16, seed=4), dev)
+    toks = [(13 * i + 5) % 1000 for i in range(rows)]
+    a, b = ca.HipLlamaRunner(conf, w, dev, 256, True), ca.HipLlamaRunner(conf, w, dev, 256, True)
+    want = [b.forward(t, i) for i, t in enumerate(toks)][-1]
+    for _ in range(2):  # (the pieces' counters are left at zero)
+        got = a.prefill(toks)
+        assert np.max(np.abs(got - want)) <= FAST_TOL["F16"][1] * np.max(np.abs(want))
+        a.reset()
