@@ -23,6 +23,7 @@
 #include "fused_common.hpp"
 #include "fused_attention.hpp"
 #include "fused_ffn.hpp"
+#include "fused_f16.hpp"
 #include "gemm_bf16.hpp"
 #include "prefill_rows.hpp"
 #include "lazy.hpp"
@@ -134,6 +135,7 @@ struct crabml_hip_llama {
   bool tp_dry = false;       // CRABML_HIP_LLAMA_TP_DRY_RUN: a lone rank that skips the all-reduces (timing only)
   bool k_norm_in = false;    // fast Q4_K step: gate | up normalizes and quantizes wo's f32 row itself (k_gateup_k_lds<.., NORMIN>)
   bool kfused = false;       // Q4_K layers, fast mode: fused GEMV kernels with the Q4_K inner loop (enqueue_segment_k)
+  bool f16_step = false;     // F16 layers, fast mode, one GPU: the linears with their row operations folded in (enqueue_segment_f16)
   bool generic = false;      // per-op launches (strict-order device, or a weight format without fused kernels)
   bool ord = false;          // strict-order device, Q4_0 / Q8_0 / Q4_1 layers: the fused launches with block-ordered sums (k_*_ord)
   uint32_t qt = 0, out_qt = 0;  // vec_dot_rhs_dtype of the layer weights / of the classifier
@@ -390,6 +392,61 @@ void enqueue_attention(crabml_hip_llama* c, int l, signed char* xq, unsigned sho
   if (prof) prof_end(dev, &ar);
 }
 
+// ---- F16 layers on the fast device (fused_f16.hpp) ---------------------------------------------------------
+// Rows a wave takes: two (gate and up: two of each) where that still leaves eight waves per CU, else one -- a launch is over in one round
+// either way, and a short one wants more waves rather than longer ones.
+template <int R, int UN, int IN, int OUT>
+void launch_step_f16_t(crabml_hip_device* dev, crabml_hip_device::ProfRec* rec, const StepF16& a, const QkvEpi& e) {
+  const int per_wg = 4 * (OUT == F16_OUT_GU ? R / 2 : R);
+  const dim3 grid((unsigned)((a.m + per_wg - 1) / per_wg));
+  const size_t lds = IN == F16_IN_HALF ? 0 : ((size_t)a.k * 2 + 15) & ~(size_t)15;
+  if constexpr (IN != F16_IN_HALF) {
+    if (a.k > 4096) {
+      launch_k(dev->stream, rec, k_step_f16<R, UN, 8, IN, OUT>, grid, dim3(256), lds, a, e);
+      return;
+    }
+  }
+  launch_k(dev->stream, rec, k_step_f16<R, UN, 2, IN, OUT>, grid, dim3(256), lds, a, e);
+}
+template <int IN, int OUT>
+void launch_step_f16(crabml_hip_device* dev, crabml_hip_device::ProfRec* rec, const StepF16& a, const QkvEpi& e = QkvEpi{}) {
+  const bool wide = a.m >= 16 * dev->n_cu;
+  if constexpr (OUT == F16_OUT_QKV)
+    launch_step_f16_t<2, 4, IN, OUT>(dev, rec, a, e);
+  else if constexpr (OUT == F16_OUT_GU) {
+    if (wide)
+      launch_step_f16_t<4, 2, IN, OUT>(dev, rec, a, e);
+    else
+      launch_step_f16_t<2, 4, IN, OUT>(dev, rec, a, e);
+  } else if constexpr (OUT == F16_OUT_STORE) {  // (a classifier)
+    if (wide)
+      launch_step_f16_t<4, 2, IN, OUT>(dev, rec, a, e);
+    else
+      launch_step_f16_t<1, 4, IN, OUT>(dev, rec, a, e);
+  } else {
+    if (wide)
+      launch_step_f16_t<2, 4, IN, OUT>(dev, rec, a, e);
+    else
+      launch_step_f16_t<1, 8, IN, OUT>(dev, rec, a, e);
+  }
+}
+constexpr size_t STEP_F16_MAX_K = 16384;  // the longest normalized row (eight pieces of 8 per thread)
+StepF16 step_f16(const crabml_hip_llama* c, std::initializer_list<const crabml_hip_buf*> w, int m, int k, const float* x, const float* gain, float eps, float* out) {
+  StepF16 a;
+  int i = 0;
+  for (const crabml_hip_buf* b : w) a.w[i++] = (const unsigned short*)b->ptr;
+  a.m = m;
+  a.k = k;
+  a.x = x;
+  a.gain = gain;
+  a.eps = eps;
+  a.out = out;
+  a.h16 = (unsigned short*)c->act_hid;
+  a.x16 = (const unsigned short*)c->act_hid;
+  a.exp_tab = (const unsigned short*)c->dev->exp_table;
+  return a;
+}
+
 // the tail of the final segment: classifier GEMV over this rank's rows (all of them unless the vocabulary is split,
 // llama2.rs:199-208) + greedy sampler + advance
 int enqueue_classifier_and_sampler(crabml_hip_llama* c, const void* cls_act, crabml_hip_device::ProfRec* R) {
@@ -399,7 +456,9 @@ int enqueue_classifier_and_sampler(crabml_hip_llama* c, const void* cls_act, cra
   const int dim = (int)g.embedding_dim;
   int *token_d = c->state, *pos_d = c->state + 1, *step_d = c->state + 2;
   float* out = c->logits + c->vocab_off;
-  if (dev->strict_order)
+  if (cls_act == nullptr)  // (F16 step: the final norm is this launch's own)
+    launch_step_f16<F16_IN_NORM, F16_OUT_STORE>(dev, R, step_f16(c, {c->output}, c->vocab_l, dim, c->x, (const float*)c->rms_final->ptr, g.rms_norm_eps, out));
+  else if (dev->strict_order)
     CH_TRY(launch_gemv_strict(dev, c->output, (size_t)c->vocab_l, dim, cls_act, 1, out));
   else
     CH_TRY(launch_gemv(dev, c->output, (size_t)c->vocab_l, dim, cls_act, 1, out, R));
@@ -768,6 +827,63 @@ int enqueue_segment_generic(crabml_hip_llama* c, int seg) {
   return 0;
 }
 
+// F16 layers (fast mode, one GPU): five launches per layer (six past attn_long_from where the attention merges in a launch of its own)
+int enqueue_segment_f16(crabml_hip_llama* c, int seg) {
+  crabml_hip_device* dev = c->dev;
+  hipStream_t st = dev->stream;
+  const auto& g = c->cfg;
+  const int dim = (int)g.embedding_dim, dim_l = c->dim_l, kv_dim_l = c->kv_dim_l, hidden_l = c->hidden_l, hd = c->hd, L = (int)g.n_layers;
+  const bool prof = dev->prof_on && !c->use_graph && !c->capturing;
+  crabml_hip_device::ProfRec pr{};
+  crabml_hip_device::ProfRec* R = prof ? &pr : nullptr;
+  auto P0 = [&](uint32_t stage, double rows, double k) { return prof ? prof_begin(dev, &pr, CRABML_HIP_F16, stage, 2.0 * rows * k + 4.0 * k + 4.0 * rows) : 0; };
+  auto P1 = [&]() { return prof ? prof_end(dev, &pr) : 0; };
+  if (seg == 2 * L) {
+    const void* act = nullptr;  // (an F16 classifier normalizes the row itself)
+    if (c->output->dtype != CRABML_HIP_F16) {
+      if (dim <= 4096)
+        k_norm_f32<4><<<1, 1024, norm_lds_bytes(dim), st>>>(c->x, nullptr, (const float*)c->rms_final->ptr, dim, g.rms_norm_eps, c->xn, 1);
+      else
+        k_norm_f32<12><<<1, 1024, norm_lds_bytes(dim), st>>>(c->x, nullptr, (const float*)c->rms_final->ptr, dim, g.rms_norm_eps, c->xn, 1);
+      act = c->xn;
+      if (c->out_qt != CRABML_HIP_F32) {
+        launch_quantize_act(st, c->out_qt, c->xn, (size_t)dim, c->act_dim);
+        act = c->act_dim;
+      }
+    }
+    if (prof)
+      CH_TRY(prof_begin(dev, &pr, c->output->dtype, 5,
+                        (double)c->vocab_l * (double)(dim / block_elems(c->output->dtype)) * (double)block_bytes(c->output->dtype) + 4.0 * dim +
+                            4.0 * c->vocab_l));
+    CH_TRY(enqueue_classifier_and_sampler(c, act, R));
+    return P1();
+  }
+  const int l = seg / 2;
+  if ((seg & 1) == 0) {
+    if (l == 0)
+      k_embed<<<(dim + 255) / 256, 256, 0, st>>>((const char*)c->token_embed->ptr, (int)c->token_embed->dtype, c->token_embed->wl.off_scale, c->state, dim, c->x);
+    const QkvEpi e{c->qbuf, c->kc[l], c->vc[l], c->rope, c->state + 1, 1.0f / std::sqrt((float)hd), dim_l, kv_dim_l, hd,
+                   (int)g.rope_dim, c->npairs, (int)g.seq_len, g.use_f16_kv_cache ? 1 : 0};
+    CH_TRY(P0(1, dim_l + 2.0 * kv_dim_l, dim));
+    launch_step_f16<F16_IN_NORM, F16_OUT_QKV>(dev, R, step_f16(c, {c->wq[l], c->wk[l], c->wv[l]}, dim_l + 2 * kv_dim_l, dim, c->x,
+                                                               (const float*)c->rms_att[l]->ptr, g.rms_norm_eps, nullptr), e);
+    CH_TRY(P1());
+    enqueue_attention(c, l, nullptr, nullptr, nullptr, PrefetchPlan{}, 0, prof);
+    CH_TRY(P0(2, dim, dim_l));
+    launch_step_f16<F16_IN_ROUND, F16_OUT_RES>(dev, R, step_f16(c, {c->wo[l]}, dim, dim_l, c->attn, nullptr, 0.f, c->x));
+    CH_TRY(P1());
+  } else {
+    CH_TRY(P0(3, 2.0 * hidden_l, dim));
+    launch_step_f16<F16_IN_NORM, F16_OUT_GU>(dev, R, step_f16(c, {c->gate[l], c->up[l]}, hidden_l, dim, c->x, (const float*)c->rms_ffn[l]->ptr, 1e-5f, nullptr));
+    CH_TRY(P1());
+    CH_TRY(P0(4, dim, hidden_l));
+    launch_step_f16<F16_IN_HALF, F16_OUT_RES>(dev, R, step_f16(c, {c->down[l]}, dim, hidden_l, nullptr, nullptr, 0.f, c->x));
+    CH_TRY(P1());
+  }
+  CH_HIP(dev, hipGetLastError());
+  return 0;
+}
+
 // Q4_K and Q4_1 layers (fast mode): the fused GEMV kernels with the format's inner loop against Q8_K / Q8_1
 // activation planes.  The rhs quantizer is its own launch here (a Q8_K super-block spans 256 rows: eight 32-row
 // workgroups; Q8_1 keeps the same structure), so a layer is 11 launches instead of the per-op path's 18.
@@ -980,6 +1096,7 @@ int enqueue_segment_k(crabml_hip_llama* c, int seg) {
 int enqueue_segment(crabml_hip_llama* c, int seg) {
   if (c->kfused)
     return c->wtype == CRABML_HIP_Q4_K ? enqueue_segment_k<CRABML_HIP_Q4_K>(c, seg) : enqueue_segment_k<CRABML_HIP_Q4_1>(c, seg);
+  if (c->f16_step) return enqueue_segment_f16(c, seg);
   if (c->generic) return enqueue_segment_generic(c, seg);
   return c->wtype == CRABML_HIP_Q4_0   ? enqueue_segment_t<CRABML_HIP_Q4_0>(c, seg)
          : c->wtype == CRABML_HIP_Q8_0 ? enqueue_segment_t<CRABML_HIP_Q8_0>(c, seg)
@@ -1887,6 +2004,8 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
   if (ordk) ord = true;
   if (ordk && mixed) generic = false;
   c->generic = generic;
+  // (dims are multiples of 32 and heads of 2 by now; a longer row does not fit the launches that normalize it: the per-op segments)
+  c->f16_step = !dev->strict_order && wt == CRABML_HIP_F16 && !mixed && tp == 1 && g.embedding_dim <= STEP_F16_MAX_K && dim_l <= STEP_F16_MAX_K;
   c->ord = ord;
   // Q4_K always; Q4_1 when it cannot take the 5-kernel path (mixed classifier format) or for the A/B flag
   c->kfused = ordk ||

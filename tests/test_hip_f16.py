@@ -49,3 +49,27 @@ def test_prompt_pass_equals_the_token_loop(ca, rows):
         got = a.prefill(toks)
         assert np.max(np.abs(got - want)) <= FAST_TOL["F16"][1] * np.max(np.abs(want))
         a.reset()
+
+
+# dim, hidden, heads, kv heads, vocab: rows shorter than a wave's step; ragged rows everywhere; rows past the 4096 elements that two pieces a
+# thread hold; classifiers on either side of the row count that gives a wave four rows
+@pytest.mark.parametrize("dim,hidden,heads,kv,vocab", [(96, 32, 3, 1, 50), (352, 544, 4, 2, 4097), (4160, 4128, 32, 8, 77), (512, 4128, 8, 8, 50)])
+@pytest.mark.parametrize("kv_f16", [True, False])
+def test_decode_step_against_the_scalar_order(ca, dim, hidden, heads, kv, vocab, kv_f16):
+    """the fast step against the strict device (the reference's sums, its own launches) on the same tokens; the graph replays itself"""
+    shape = synth.ModelShape("f16", dim, hidden, 2, heads, kv, vocab, 128, 1e-5, dim // heads // 2 * 2)
+    model = synth.build_model(shape, synth.F16, seed=5)
+    logits = []
+    for strict in (True, False):
+        dev = ca.HipTensorDevice(0, False, 0, strict)
+        conf, w = synth.to_hip(model, dev)
+        r = ca.HipLlamaRunner(conf, w, dev, 128, kv_f16)
+        logits.append(np.array([r.forward((7 * i + 3) % vocab, i) for i in range(12)]))
+        if not strict:
+            r.reset()
+            first = r.forward(3 % vocab, 0)
+            assert np.array_equal(first, logits[1][0])  # (a replay leaves nothing behind that changes the next one)
+    # 2-norms; two orders of a sum flip roundings to f16 (every rhs, cached rows, the exponential's levels), each 2^-11 of an element: up to
+    # 1.2e-3 over these models where the fast device takes one launch per op, four such steps allowed
+    err = np.linalg.norm(logits[1] - logits[0], axis=1) / np.linalg.norm(logits[0], axis=1)
+    assert np.max(err) <= 4 * 2.0 ** -11, err
