@@ -19,6 +19,10 @@ enum {
                       // applied to the finished dots: W (s x) = s (W x)
   GEMV_IN_SPLIT = 2,  // elements from k_split on still want their RMS normalization; their sum of squares arrives in pieces (ss)
   GEMV_IN_RMSV = 3,   // GEMV_IN_RMS with a gain per element (gain: K numbers), applied while the row is staged
+  // the matrix-core form with one plane: rows that their producer left as bf16 (x16)
+  GEMV_IN_BF16 = 4,
+  GEMV_IN_BF16_RMS = 5,    // times gain (nullable: 1) over the root mean square, its sum of squares in pieces (ss); gains per element are in x16
+  GEMV_IN_BF16_SPLIT = 6,  // GEMV_IN_SPLIT: the dots of the elements from k_split on are normalized
 };
 // what happens to a dot product on the way out
 enum {
@@ -94,9 +98,17 @@ __device__ __forceinline__ V stream_apply(const StreamMix& m, float* x, const V 
 struct GemvBf16 {
   const unsigned short* w = nullptr;  // [N][ldw]
   const float* x = nullptr;           // [nb][ldx]
-  float* out = nullptr;               // [nb][ldo]
+  const unsigned short* x16 = nullptr;  // GEMV_IN_BF16*: the same as bf16
+  float* out = nullptr;                 // [nb][ldo]
+  // on the matrix cores (nullable): where the results go as bf16 -- XIELU, GLU: instead; RESIDUAL, STREAMS: what the next linear reads, times
+  // gain_out (nullable) and with its square sums by 16 columns
+  unsigned short* out16 = nullptr;
+  const float* gain_out = nullptr;
+  float* ss_out = nullptr;  // [nb][n_ss_out]
+  int n_ss_out = 0;
   int N = 0, K = 0, ldw = 0, ldx = 0, ldo = 0, nb = 1;  // K % 8 == 0
   // GEMV_IN_RMS: elements the mean is over, eps, the gain (device); GEMV_IN_SPLIT: the same for the tail, with ss[b][n_ss] pieces
+  // (GEMV_IN_BF16_RMS: such pieces too)
   int mean_n = 1;
   float eps = 0.f;
   const float* gain = nullptr;
@@ -147,17 +159,20 @@ __device__ __forceinline__ float gelu_tanh(float z) {
 }
 __device__ __forceinline__ float soft_cap(float z, float cap) { return cap > 0.0f ? cap * tanhf(z / cap) : z; }
 
+__device__ __forceinline__ float gemv_residual(const GemvBf16& a, int row, int b, float v) {
+  float* o = a.out + (size_t)b * a.ldo + row;
+  float s = *o + v;
+  if (a.add_rows) s += a.add_rows[(size_t)b * a.ld_add + row];
+  if (a.add_vec) s += a.add_vec[row];
+  *o = s;
+  return s;
+}
 template <int OUT>
 __device__ __forceinline__ void gemv_out(const GemvBf16& a, int row, int b, float v) {
   float* o = a.out + (size_t)b * a.ldo + row;
   if constexpr (OUT == GEMV_OUT_STORE) *o = v;
   if constexpr (OUT == GEMV_OUT_ACT) *o = act_ranges(a.bias ? v + a.bias[row] : v, row, a.act);
-  if constexpr (OUT == GEMV_OUT_RESIDUAL) {
-    float s = *o + v;
-    if (a.add_rows) s += a.add_rows[(size_t)b * a.ld_add + row];
-    if (a.add_vec) s += a.add_vec[row];
-    *o = s;
-  }
+  if constexpr (OUT == GEMV_OUT_RESIDUAL) (void)gemv_residual(a, row, b, v);
   if constexpr (OUT == GEMV_OUT_XIELU) *o = xielu_apply(v, a.xielu[0], a.xielu[1]);
   if constexpr (OUT == GEMV_OUT_SOFTCAP) *o = soft_cap(v, a.cap);
 }
@@ -170,8 +185,22 @@ __device__ __forceinline__ void stream_elem_load(const GemvBf16& a, int row, int
   stream_load(a.sm, a.out + (size_t)b * a.ldo + row, e.old);
   if (a.bias) e.bias = a.bias[row];
 }
+__device__ __forceinline__ float stream_elem_mix(const GemvBf16& a, int row, int b, const StreamElem& e, float v) {
+  return stream_apply(a.sm, a.out + (size_t)b * a.ldo + row, e.old, v + e.bias);
+}
 __device__ __forceinline__ void stream_elem_out(const GemvBf16& a, int row, int b, const StreamElem& e, float v) {
-  a.u[(size_t)b * a.ldo + row] = stream_apply(a.sm, a.out + (size_t)b * a.ldo + row, e.old, v + e.bias);
+  a.u[(size_t)b * a.ldo + row] = stream_elem_mix(a, row, b, e, v);
+}
+// v of 16 neighbouring columns in 16 lanes (zero outside the matrix): what the next linear reads, and its square sum.  Without out16: as f32.
+__device__ __forceinline__ void rows16_out(const GemvBf16& a, int row, int b, float v) {
+  const bool in = b < a.nb && row < a.N;
+  if (!a.out16) {
+    if (in) a.u[(size_t)b * a.ldo + row] = v;
+    return;
+  }
+  if (in) a.out16[(size_t)b * a.ldo + row] = f2bf(a.gain_out ? v * a.gain_out[row] : v);
+  const float s = row16_sum_f32(v * v);
+  if (in && (row & 15) == 0) a.ss_out[(size_t)b * a.n_ss_out + (row >> 4)] = s;
 }
 
 #define GEMV_BF16_LDS_FLOATS 8192  // rhs elements staged at a time, all rows together: a cut segment is a multiple of the steps in flight
@@ -347,133 +376,220 @@ __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
 }
 
 // ---- the same linear for 3 .. 16 rhs rows: one pass over the weights on the matrix cores ---------------------------------------------
-// A 512-thread workgroup owns 16 RT weight rows; its eight waves take the 64-element pieces of k in turn and their tiles are added
-// through LDS at the end.  Both operands come straight from memory in fragment order (16 rows x 64 bytes per request; the rhs, a few
-// hundred KB, lives in L2), the next piece's requests out before the current one is multiplied.  The rhs becomes bf16 on the way:
-// rounded (SPL = 1), or as three exact pieces (SPL = 3; see split_store in gemm_bf16.hpp).  K is a multiple of 64.
+// A workgroup of W waves owns 16 RT weight rows; the waves take the 64-element pieces of k in turn, D pieces of requests out each, and their
+// tiles are added through LDS at the end.  The rhs becomes bf16 on the way: rounded (SPL = 1), or as three exact pieces (SPL = 3; see
+// split_store in gemm_bf16.hpp) -- or arrives as bf16 (GEMV_IN_BF16).  K is a multiple of 64.
+//
+// A fragment of the matrix instruction has a row per lane, so neighbouring lanes' 16 bytes would come from different cache lines: 64 line
+// accesses per request, and that -- not the bytes -- was the bound (2048 x 8192, 16 rows: 23.2 us, 20 of them 128 pieces x 6 requests x
+// 64 accesses of one CU).  Here eight (f32 rhs: sixteen) neighbouring lanes take a row's 128 (256) bytes and the tile goes through the
+// wave's own 2 KB of LDS, 16-byte pieces permuted by (row / 2) % 8 as in gemm_bf16.hip; no barrier, a wave's LDS accesses are in order.
+// 16 rows, before -> after, with bf16 rows: 2048 x 8192 23.2 -> 12.7 us, 2048 x 4096 17.5 -> 8.6, 5632 x 2048 19.3 -> 13.9, 8192 x 2048
+// 14.1 -> 10.2, 32000 x 2048 35.4 -> 30.3 (4.3 TB/s); what is left is a launch's ramp, two rounds of memory latency and the hand-over.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 // f32 -> its upper, middle and lower eight significand bits as bf16: their sum is exact
+__device__ __forceinline__ void split3(float v, unsigned short& hi, unsigned short& mid, unsigned short& lo) {
+  const float a = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, v) & 0xffff0000u), r = v - a;
+  const float b = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, r) & 0xffff0000u);
+  hi = (unsigned short)(__builtin_bit_cast(unsigned, a) >> 16);
+  mid = (unsigned short)(__builtin_bit_cast(unsigned, b) >> 16);
+  lo = f2bf(r - b);
+}
 __device__ __forceinline__ void split3(const float (&v)[8], bf16x8& hi, bf16x8& mid, bf16x8& lo) {
   unsigned short h[8], m[8], l[8];
 #pragma unroll
-  for (int e = 0; e < 8; e++) {
-    const float a = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, v[e]) & 0xffff0000u), r = v[e] - a;
-    const float b = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, r) & 0xffff0000u);
-    h[e] = (unsigned short)(__builtin_bit_cast(unsigned, a) >> 16);
-    m[e] = (unsigned short)(__builtin_bit_cast(unsigned, b) >> 16);
-    l[e] = f2bf(r - b);
-  }
+  for (int e = 0; e < 8; e++) split3(v[e], h[e], m[e], l[e]);
   __builtin_memcpy(&hi, h, 16);
   __builtin_memcpy(&mid, m, 16);
   __builtin_memcpy(&lo, l, 16);
 }
+// what this wave has written to LDS is there for its other lanes (a wave's LDS accesses are in order; the compiler is told)
+__device__ __forceinline__ void wave_lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 
-template <int RT, int SPL, int IN, int OUT>
-__global__ __launch_bounds__(512) void k_gemv16_bf16(const GemvBf16 a) {
-  constexpr int W = 8, LD = 20;
-  __shared__ __attribute__((aligned(16))) float tile[W][RT][16 * LD];
+template <int RT, int SPL, int W, int D, int IN, int OUT>
+__global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
+  constexpr int LD = 20, NT = 64 * W;
+  constexpr bool XB = IN == GEMV_IN_BF16 || IN == GEMV_IN_BF16_RMS || IN == GEMV_IN_BF16_SPLIT, NORM = IN == GEMV_IN_RMS || IN == GEMV_IN_RMSV;
+  constexpr bool PIECES = IN == GEMV_IN_BF16_RMS || IN == GEMV_IN_BF16_SPLIT, TAIL = IN == GEMV_IN_BF16_SPLIT;
+  constexpr int XR = XB ? 2 : 4;  // requests for a piece of the rhs
+  static_assert(!XB || SPL == 1, "a bf16 rhs has one piece");
+  union Lds {
+    unsigned short in[W][RT + SPL][16 * 64];  // a wave's tiles: weights, rhs
+    float tile[W][RT][16 * LD];
+  };
+  __shared__ __attribute__((aligned(16))) Lds lds;
   __shared__ float sums[W][16], scale[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_wg(), fr = lane & 15, fk = lane >> 4;
   const int row0 = blockIdx.x * 16 * RT;
-  const unsigned short* wr[RT];
+  // where this lane's part of a request lies: 16 bytes, eight lanes a row (f32: sixteen)
+  const int r8 = lane >> 3, c8 = lane & 7, r16 = lane >> 4, c16 = lane & 15;
+  // (32-bit offsets from a scalar base)
+  const char *wb = (const char*)(a.w + (size_t)row0 * a.ldw), *xbase = XB ? (const char*)a.x16 : (const char*)a.x, *gb = (const char*)a.gain;
+  unsigned wo[RT][2], xo[XR];
 #pragma unroll
-  for (int t = 0; t < RT; t++) {
-    const int row = row0 + t * 16 + fr;
-    wr[t] = a.w + (size_t)(row < a.N ? row : a.N - 1) * a.ldw + fk * 8;
-  }
-  const float* xr = a.x + (size_t)(fr < a.nb ? fr : a.nb - 1) * a.ldx + fk * 8;
-  bf16x8 wv[2][RT];
-  f32x4 xv[2][2], gv[2][2];
-  auto request = [&](int k) {
+  for (int t = 0; t < RT; t++)
 #pragma unroll
-    for (int u = 0; u < 2; u++) {
-#pragma unroll
-      for (int t = 0; t < RT; t++) wv[u][t] = *(const bf16x8*)(wr[t] + k + u * 32);
-      xv[u][0] = *(const f32x4*)(xr + k + u * 32);
-      xv[u][1] = *(const f32x4*)(xr + k + u * 32 + 4);
-      if constexpr (IN == GEMV_IN_RMSV) {
-        gv[u][0] = *(const f32x4*)(a.gain + k + u * 32 + fk * 8);
-        gv[u][1] = *(const f32x4*)(a.gain + k + u * 32 + fk * 8 + 4);
-      }
+    for (int j = 0; j < 2; j++) {
+      const int row = t * 16 + j * 8 + r8;
+      wo[t][j] = (unsigned)(row0 + row < a.N ? row : a.N - 1 - row0) * (unsigned)a.ldw * 2 + c8 * 16;
     }
+#pragma unroll
+  for (int j = 0; j < XR; j++) {
+    const int b = XB ? j * 8 + r8 : j * 4 + r16;
+    xo[j] = (unsigned)(b < a.nb ? b : a.nb - 1) * (unsigned)a.ldx * (XB ? 2 : 4) + (XB ? c8 : c16) * 16;
+  }
+  i32x4 wv[D][RT][2], xv[D][XR];
+  f32x4 gv[D];
+  auto request = [&](int d, int i) {
+    const char *w = wb + i * 128, *x = xbase + i * (XB ? 128 : 256);
+#pragma unroll
+    for (int t = 0; t < RT; t++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) wv[d][t][j] = *(const i32x4*)(w + wo[t][j]);
+#pragma unroll
+    for (int j = 0; j < XR; j++) xv[d][j] = *(const i32x4*)(x + xo[j]);
+    if constexpr (IN == GEMV_IN_RMSV) gv[d] = *(const f32x4*)(gb + i * 256 + (unsigned)c16 * 16);
   };
-  const int n = a.K / 64;
-  if (wave < n) request(wave * 64);
-  StreamElem elem[(RT + 1) / 2];  // of this thread's results: element tid + 512 i of the tile
+  const int n = a.K / 64, last = n - 1;
+  // a row's sum of squares: NT / 16 threads, its first pieces requested ahead of the weights (loads come back in order)
+  constexpr int QT = NT / 16, QP = 4;
+  const int q_row = tid / QT, q_at = tid % QT;
+  const float* q_ss = PIECES ? a.ss + (size_t)(q_row < a.nb ? q_row : a.nb - 1) * a.n_ss : nullptr;
+  float q_v[QP];
+  if constexpr (PIECES) {
+#pragma unroll
+    for (int u = 0; u < QP; u++) q_v[u] = q_ss[q_at + u * QT < a.n_ss ? q_at + u * QT : 0];
+  }
+  if (wave < n) {
+#pragma unroll
+    for (int d = 0; d < D; d++) request(d, wave + d * W < n ? wave + d * W : last);  // (clamped: no branch between the requests)
+  }
+  constexpr int ELEMS = (RT * 256 + NT - 1) / NT;
+  StreamElem elem[ELEMS];  // of this thread's results: element tid + NT i of the tile
   if constexpr (OUT == GEMV_OUT_STREAMS) {
 #pragma unroll
-    for (int i = 0; i < (RT + 1) / 2; i++) {
-      const int j = tid + i * 512, b = (j >> 4) & 15, row = row0 + (j >> 8) * 16 + (j & 15);
+    for (int i = 0; i < ELEMS; i++) {
+      const int j = tid + i * NT, b = (j >> 4) & 15, row = row0 + (j >> 8) * 16 + (j & 15);
       if (j < RT * 256 && b < a.nb && row < a.N) stream_elem_load(a, row, b, elem[i]);
     }
   }
-  float tail = 1.f, sq = 0.f;
-  if constexpr (IN == GEMV_IN_SPLIT) {
-    float s = 0.f;
-    for (int i = fk; i < a.n_ss; i += 4) s += a.ss[(size_t)(fr < a.nb ? fr : a.nb - 1) * a.n_ss + i];
-    s += __shfl_xor(s, 16, 64);
-    s += __shfl_xor(s, 32, 64);
-    tail = 1.0f / sqrtf(s / (float)a.mean_n + a.eps);
+  float tail[4], sq[4];  // of row 4 j + r16
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    tail[j] = 1.f;
+    sq[j] = 0.f;
+    if constexpr (IN == GEMV_IN_SPLIT) {
+      const int b = j * 4 + r16;
+      float t = 0.f;
+      for (int i = c16; i < a.n_ss; i += 16) t += a.ss[(size_t)(b < a.nb ? b : a.nb - 1) * a.n_ss + i];
+      tail[j] = 1.0f / sqrtf(row16_sum_f32(t) / (float)a.mean_n + a.eps);
+    }
   }
-  f32x4 acc[RT];
+  f32x4 acc[RT], acc2[RT];  // (TAIL: what is normalized apart)
 #pragma unroll
-  for (int t = 0; t < RT; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int i = wave; i < n; i += W) {
-    bf16x8 wc[2][RT];
-    f32x4 xc[2][2], gc[2][2];
+  for (int t = 0; t < RT; t++) acc[t] = acc2[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  unsigned short(*mine)[16 * 64] = lds.in[wave];
+  auto multiply = [&](const i32x4 (&wc)[RT][2], const i32x4 (&xc)[XR], const f32x4& gc, int i) {
 #pragma unroll
-    for (int u = 0; u < 2; u++) {
+    for (int t = 0; t < RT; t++)
 #pragma unroll
-      for (int t = 0; t < RT; t++) wc[u][t] = wv[u][t];
-      xc[u][0] = xv[u][0];
-      xc[u][1] = xv[u][1];
-      if constexpr (IN == GEMV_IN_RMSV) {
-        gc[u][0] = gv[u][0];
-        gc[u][1] = gv[u][1];
+      for (int j = 0; j < 2; j++) {
+        const int r = j * 8 + r8;
+        *(i32x4*)&mine[t][r * 64 + ((c8 ^ ((r >> 1) & 7)) * 8)] = wc[t][j];
+      }
+    if constexpr (XB) {
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        const int r = j * 8 + r8;
+        *(i32x4*)&mine[RT][r * 64 + ((c8 ^ ((r >> 1) & 7)) * 8)] = xc[j];
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int r = j * 4 + r16;
+        f32x4 v = __builtin_bit_cast(f32x4, xc[j]);
+        if constexpr (NORM) {
+#pragma unroll
+          for (int e = 0; e < 4; e++) sq[j] = __builtin_fmaf(v[e], v[e], sq[j]);
+        }
+        if constexpr (IN == GEMV_IN_RMSV) v *= gc;
+        if constexpr (IN == GEMV_IN_SPLIT) v *= i * 64 >= a.k_split ? tail[j] : 1.f;  // (k_split is a multiple of 64)
+        unsigned short p[SPL][4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          if constexpr (SPL == 1)
+            p[0][e] = f2bf(v[e]);
+          else
+            split3(v[e], p[0][e], p[1][e], p[2][e]);
+        }
+#pragma unroll
+        for (int q = 0; q < SPL; q++) {
+          i32x2 w;
+          __builtin_memcpy(&w, p[q], 8);
+          *(i32x2*)&mine[RT + q][r * 64 + (((c16 >> 1) ^ ((r >> 1) & 7)) * 8) + (c16 & 1) * 4] = w;
+        }
       }
     }
-    if (i + W < n) request((i + W) * 64);
+    wave_lds_order();
 #pragma unroll
     for (int u = 0; u < 2; u++) {
-      float v[8] = {xc[u][0][0], xc[u][0][1], xc[u][0][2], xc[u][0][3], xc[u][1][0], xc[u][1][1], xc[u][1][2], xc[u][1][3]};
-      if constexpr (IN == GEMV_IN_RMS || IN == GEMV_IN_RMSV) {
+      const int at = fr * 64 + (((u * 4 + fk) ^ ((fr >> 1) & 7)) * 8);
+      bf16x8 x[SPL];
 #pragma unroll
-        for (int e = 0; e < 8; e++) sq = __builtin_fmaf(v[e], v[e], sq);
-      }
-      if constexpr (IN == GEMV_IN_RMSV) {
+      for (int q = 0; q < SPL; q++) x[q] = *(const bf16x8*)&mine[RT + q][at];
 #pragma unroll
-        for (int e = 0; e < 8; e++) v[e] *= gc[u][e >> 2][e & 3];
-      }
-      if constexpr (IN == GEMV_IN_SPLIT) {
-        const float f = i * 64 >= a.k_split ? tail : 1.f;  // (k_split is a multiple of 64)
+      for (int t = 0; t < RT; t++) {
+        const bf16x8 w = *(const bf16x8*)&mine[t][at];
+        if (TAIL && i * 64 >= a.k_split)
+          acc2[t] = mfma_bf16(w, x[0], acc2[t]);
+        else
 #pragma unroll
-        for (int e = 0; e < 8; e++) v[e] *= f;
-      }
-      if constexpr (SPL == 1) {
-        bf16x8 b;
-#pragma unroll
-        for (int e = 0; e < 8; e++) b[e] = (__bf16)v[e];
-#pragma unroll
-        for (int t = 0; t < RT; t++) acc[t] = mfma_bf16(wc[u][t], b, acc[t]);
-      } else {
-        bf16x8 h, m, l;
-        split3(v, h, m, l);
-#pragma unroll
-        for (int t = 0; t < RT; t++) acc[t] = mfma_bf16(wc[u][t], h, mfma_bf16(wc[u][t], m, mfma_bf16(wc[u][t], l, acc[t])));
+          for (int q = SPL - 1; q >= 0; q--) acc[t] = mfma_bf16(w, x[q], acc[t]);  // (the smallest piece first)
       }
     }
+    wave_lds_order();
+  };
+  for (int i = wave; i < n; i += D * W) {
+    if (i + D * W < n) {
+#pragma unroll
+      for (int d = 0; d < D; d++) {
+        multiply(wv[d], xv[d], gv[d], i + d * W);
+        request(d, i + (D + d) * W < n ? i + (D + d) * W : last);
+      }
+    } else {
+#pragma unroll
+      for (int d = 0; d < D; d++)
+        if (i + d * W < n) multiply(wv[d], xv[d], gv[d], i + d * W);
+    }
+  }
+  if constexpr (NORM) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const float t = row16_sum_f32(sq[j]);
+      if (c16 == 0) sums[wave][j * 4 + r16] = t;
+    }
+  }
+  if constexpr (PIECES) {
+    float t = 0.f;
+#pragma unroll
+    for (int u = 0; u < QP; u++) t += q_at + u * QT < a.n_ss ? q_v[u] : 0.f;
+    for (int i = q_at + QP * QT; i < a.n_ss; i += QT) t += q_ss[i];
+    t = row16_sum_f32(t);
+    t += __shfl_xor(t, 16, 64);
+    if constexpr (QT == 64) t += __shfl_xor(t, 32, 64);
+    if (q_at == 0) scale[q_row] = (!TAIL && a.gain ? *a.gain : 1.0f) / sqrtf(t / (float)a.mean_n + a.eps);
+  }
+  __syncthreads();  // (the tiles of results take the place of the operands')
+  if constexpr (TAIL) {
+#pragma unroll
+    for (int t = 0; t < RT; t++) acc[t] += acc2[t] * scale[fr];
   }
   // lane: weight rows 4 fk .. of rhs row fr
 #pragma unroll
-  for (int t = 0; t < RT; t++) *(f32x4*)&tile[wave][t][fr * LD + fk * 4] = acc[t];
-  if constexpr (IN == GEMV_IN_RMS || IN == GEMV_IN_RMSV) {
-    sq += __shfl_xor(sq, 16, 64);
-    sq += __shfl_xor(sq, 32, 64);
-    if (fk == 0) sums[wave][fr] = sq;
-  }
+  for (int t = 0; t < RT; t++) *(f32x4*)&lds.tile[wave][t][fr * LD + fk * 4] = acc[t];
   __syncthreads();
-  if constexpr (IN == GEMV_IN_RMS || IN == GEMV_IN_RMSV) {
+  if constexpr (NORM) {
     if (tid < 16) {
       float s = 0.f;
 #pragma unroll
@@ -483,53 +599,89 @@ __global__ __launch_bounds__(512) void k_gemv16_bf16(const GemvBf16 a) {
     __syncthreads();
   }
   if constexpr (OUT == GEMV_OUT_GLU) {
-    for (int i = tid; i < RT * 128; i += 512) {
+    for (int i = tid; i < RT * 128; i += NT) {
       const int t = i >> 7, b = (i >> 3) & 15, r = (i & 7) * 2, row = row0 + t * 16 + r;
       float gate = 0.f, up = 0.f;
 #pragma unroll
       for (int w = 0; w < W; w++) {
-        gate += tile[w][t][b * LD + r];
-        up += tile[w][t][b * LD + r + 1];
+        gate += lds.tile[w][t][b * LD + r];
+        up += lds.tile[w][t][b * LD + r + 1];
       }
-      if constexpr (IN == GEMV_IN_RMS || IN == GEMV_IN_RMSV) {
+      if constexpr (NORM || IN == GEMV_IN_BF16_RMS) {
         gate *= scale[b];
         up *= scale[b];
       }
-      if (b < a.nb && row < a.N) a.out[(size_t)b * a.ldo + row / 2] = gelu_tanh(gate) * up;
+      if (b < a.nb && row < a.N) {
+        const size_t o = (size_t)b * a.ldo + row / 2;
+        if (a.out16)
+          a.out16[o] = f2bf(gelu_tanh(gate) * up);
+        else
+          a.out[o] = gelu_tanh(gate) * up;
+      }
     }
     return;
   }
   if constexpr (OUT == GEMV_OUT_STREAMS) {
 #pragma unroll
-    for (int i = 0; i < (RT + 1) / 2; i++) {
-      const int j = tid + i * 512, t = j >> 8, b = (j >> 4) & 15, r = j & 15, row = row0 + t * 16 + r;
-      if (j < RT * 256 && b < a.nb && row < a.N) {
+    for (int i = 0; i < ELEMS; i++) {
+      const int j = tid + i * NT, t = j >> 8, b = (j >> 4) & 15, r = j & 15, row = row0 + t * 16 + r;
+      if (j >= RT * 256) break;  // (whole waves)
+      float u = 0.f;
+      if (b < a.nb && row < a.N) {
         float v = 0.f;
 #pragma unroll
-        for (int w = 0; w < W; w++) v += tile[w][t][b * LD + r];
-        stream_elem_out(a, row, b, elem[i], v);
+        for (int w = 0; w < W; w++) v += lds.tile[w][t][b * LD + r];
+        u = stream_elem_mix(a, row, b, elem[i], v);
       }
+      rows16_out(a, row, b, u);
     }
     return;
   }
-  for (int i = tid; i < RT * 256; i += 512) {
+  for (int i = tid; i < RT * 256; i += NT) {
     const int t = i >> 8, b = (i >> 4) & 15, r = i & 15, row = row0 + t * 16 + r;
     float v = 0.f;
 #pragma unroll
-    for (int w = 0; w < W; w++) v += tile[w][t][b * LD + r];
-    if constexpr (IN == GEMV_IN_RMS || IN == GEMV_IN_RMSV) v *= scale[b];
-    if (b < a.nb && row < a.N) gemv_out<OUT>(a, row, b, v);
+    for (int w = 0; w < W; w++) v += lds.tile[w][t][b * LD + r];
+    if constexpr (NORM || IN == GEMV_IN_BF16_RMS) v *= scale[b];
+    if constexpr (OUT == GEMV_OUT_RESIDUAL) {
+      float x = 0.f;
+      if (b < a.nb && row < a.N) x = gemv_residual(a, row, b, v);
+      if (a.out16) rows16_out(a, row, b, x);
+      continue;
+    }
+    if (b < a.nb && row < a.N) {
+      if constexpr (OUT == GEMV_OUT_XIELU) {
+        if (a.out16) {
+          a.out16[(size_t)b * a.ldo + row] = f2bf(xielu_apply(v, a.xielu[0], a.xielu[1]));
+          continue;
+        }
+      }
+      gemv_out<OUT>(a, row, b, v);
+    }
   }
 }
 
-template <int IN, int OUT>
-inline void launch_gemv16_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a, bool exact) {
-  const bool two = a.N >= 16384;
-  const dim3 grid((a.N + (two ? 31 : 15)) / (two ? 32 : 16));
-  if (exact)
-    launch_k(st, rec, two ? k_gemv16_bf16<2, 3, IN, OUT> : k_gemv16_bf16<1, 3, IN, OUT>, grid, dim3(512), 0, a);
-  else
-    launch_k(st, rec, two ? k_gemv16_bf16<2, 1, IN, OUT> : k_gemv16_bf16<1, 1, IN, OUT>, grid, dim3(512), 0, a);
+// 32 rows a workgroup where that still fills the chip, else 16; sixteen waves where 16 rows leave CUs without a workgroup and k is long
+// enough for each of them to have a few steps.  One piece of the rhs: bf16 rows, but for a classifier behind a prompt pass.
+template <int RT, int SPL, int W, int IN, int OUT>
+inline void launch_gemv16_t(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a) {
+  constexpr int D = IN < GEMV_IN_BF16 || RT == 2 ? 2 : OUT == GEMV_OUT_STREAMS ? 3 : 4;  // (registers: sixteen waves a CU)
+  launch_k(st, rec, k_gemv16_bf16<RT, SPL, W, D, IN, OUT>, dim3((a.N + 16 * RT - 1) / (16 * RT)), dim3(64 * W), 0, a);
+}
+template <int SPL, int IN, int OUT>
+inline void launch_gemv16_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a, int n_cu) {
+  const bool two = a.N >= 16384, deep = !two && (a.N + 15) / 16 < n_cu && a.K >= 2048;
+  if (two) {
+    launch_gemv16_t<2, SPL, 8, IN, OUT>(st, rec, a);
+    return;
+  }
+  if constexpr (IN >= GEMV_IN_BF16) {
+    if (deep) {
+      launch_gemv16_t<1, SPL, 16, IN, OUT>(st, rec, a);
+      return;
+    }
+  }
+  launch_gemv16_t<1, SPL, 8, IN, OUT>(st, rec, a);
 }
 
 template <int NB, int R, int IN, int OUT>

@@ -69,6 +69,11 @@ struct crabml_hip_hybrid {
   StepSeq* st_seq = nullptr;
   int* st_count = nullptr;
   float *st_x = nullptr, *st_emb = nullptr, *st_proj = nullptr, *st_cat = nullptr, *st_u = nullptr, *st_ss = nullptr, *st_part = nullptr, *st_logits = nullptr;
+  // a step's rows as bf16 where its linears take them so (rows16): what a norm reads, with its square sums by 16 columns; the mixers' results;
+  // the feed-forward's middle
+  unsigned short *st_x16 = nullptr, *st_cat16 = nullptr, *st_u16 = nullptr;
+  float* st_xss = nullptr;
+  int n_xss = 0;
   float *st_in = nullptr, *st_vk = nullptr, *st_q = nullptr, *st_lpart = nullptr;  // streams: what the next linear reads; kept values; latent queries, partials
   int ld_vk = 0, ld_kv = 0, ld_lat = 0, ld_rot = 0;
   size_t hist = 0;  // earlier positions a latent layer can see
@@ -420,13 +425,18 @@ struct Prof {
   crabml_hip_device::ProfRec* rec() { return on ? &r : nullptr; }
 };
 
-// a decode linear: up to two rows on the vector kernel, more on the matrix cores
-template <int IN, int OUT>
+// More than two rows in bf16 compute: the matrix-core linears, whose rows are bf16 all the way -- every producer leaves them rounded as the
+// linear would round them on the way in, with the square sums a norm needs -- half the bytes, and none of the conversions in every workgroup.
+bool rows16(const Ctx* c, int B) { return B > 2 && !c->f32; }
+// a decode linear: up to two rows on the vector kernel, more on the matrix cores (IN16: its form for rows16)
+template <int IN, int IN16, int OUT>
 void step_linear(Ctx* c, crabml_hip_device::ProfRec* rec, const GemvBf16& g) {
   if (g.nb <= 2)
     launch_gemv_bf16<IN, OUT>(c->dev->stream, rec, g);
+  else if (c->f32)
+    launch_gemv16_bf16<3, IN, OUT>(c->dev->stream, rec, g, c->dev->n_cu);
   else
-    launch_gemv16_bf16<IN, OUT>(c->dev->stream, rec, g, c->f32);
+    launch_gemv16_bf16<1, IN16, OUT>(c->dev->stream, rec, g, c->dev->n_cu);
 }
 
 MixStep mix_step(const Ctx* c, const Run& run, int B) {
@@ -438,6 +448,7 @@ MixStep mix_step(const Ctx* c, const Run& run, int B) {
   m.seq = c->st_seq;
   m.proj = c->st_proj;
   m.cat = c->st_cat;
+  m.cat16 = rows16(c, B) ? c->st_cat16 : nullptr;
   m.ss = c->st_ss;
   m.part = c->st_part;
   m.tick = c->st_tick;
@@ -491,15 +502,29 @@ StreamMix streams_at_start(const Ctx* c, size_t stride) {
 }
 // an RMS norm and a linear behind it
 template <int OUT>
-void normed_linear(Ctx* c, crabml_hip_device::ProfRec* rec, const GemvBf16& g) {
+void normed_linear(Ctx* c, crabml_hip_device::ProfRec* rec, GemvBf16 g) {
+  if (rows16(c, g.nb)) {
+    g.x16 = c->st_x16;
+    g.ss = c->st_xss;
+    g.n_ss = c->n_xss;
+    if (c->streams) g.gain = nullptr;  // (in the rows already)
+  }
   if (c->streams)
-    step_linear<GEMV_IN_RMSV, OUT>(c, rec, g);
+    step_linear<GEMV_IN_RMSV, GEMV_IN_BF16_RMS, OUT>(c, rec, g);
   else
-    step_linear<GEMV_IN_RMS, OUT>(c, rec, g);
+    step_linear<GEMV_IN_RMS, GEMV_IN_BF16_RMS, OUT>(c, rec, g);
+}
+// a linear into the residual leaves the rows that the next norm and linear read
+void next_rows16(Ctx* c, GemvBf16* g, const float* gain) {
+  if (!rows16(c, g->nb)) return;
+  g->out16 = c->st_x16;
+  g->gain_out = c->streams ? gain : nullptr;
+  g->ss_out = c->st_xss;
+  g->n_ss_out = c->n_xss;
 }
 
-// the classifier on f32 rows
-void head_rows(Ctx* c, const float* x, int B, bool prof) {
+// the classifier on f32 rows, or (a step's own, f32_rows = false) on the rows the last linear left
+void head_rows(Ctx* c, const float* x, int B, bool prof, bool f32_rows) {
   GemvBf16 g;
   g.w = c->head;
   g.x = x;
@@ -512,6 +537,13 @@ void head_rows(Ctx* c, const float* x, int B, bool prof) {
   g.gain = c->final_norm;
   g.cap = c->cfg.logit_softcap;
   Prof p(c->dev, prof, ST_STEP + ST_HEAD, (double)c->vocab * c->ldx * 2);
+  if (f32_rows && rows16(c, B)) {
+    if (c->streams)
+      launch_gemv16_bf16<1, GEMV_IN_RMSV, GEMV_OUT_SOFTCAP>(c->dev->stream, p.rec(), g, c->dev->n_cu);
+    else
+      launch_gemv16_bf16<1, GEMV_IN_RMS, GEMV_OUT_SOFTCAP>(c->dev->stream, p.rec(), g, c->dev->n_cu);
+    return;
+  }
   normed_linear<GEMV_OUT_SOFTCAP>(c, p.rec(), g);
 }
 
@@ -527,6 +559,7 @@ int latent_step(Ctx* c, const Run& run, int B, bool prof) {
   m.q = c->st_q;
   m.part = c->st_lpart;
   m.cat = c->st_cat;
+  m.cat16 = rows16(c, B) ? c->st_cat16 : nullptr;
   m.B = B;
   m.ldp = L.n_in;
   m.ldc = L.ldc;
@@ -554,7 +587,9 @@ int enqueue_step(Ctx* c, int B, bool sample, bool prof) {
   const float* next_gain = nullptr;
   float* x_in = c->streams ? c->st_in : c->st_x;  // what a norm reads
   k_embed_step<<<dim3((c->width + 255) / 256, B), 256, 0, st>>>(c->embed, c->st_seq, c->width, c->ldx, c->cfg.embed_scale, c->freq, c->st_x,
-                                                               c->keep_emb ? c->st_emb : nullptr, c->runs[0].add_vec, streams_at_start(c, stride), c->st_in);
+                                                               c->keep_emb ? c->st_emb : nullptr, c->runs[0].add_vec, streams_at_start(c, stride), c->st_in,
+                                                               rows16(c, B) ? c->st_x16 : nullptr, c->streams ? c->layers[c->runs[0].layer].norm1 : nullptr,
+                                                               c->st_xss, c->n_xss);
   for (size_t r = 0; r < c->runs.size(); r++) {
     const Run& run = c->runs[r];
     const Layer& L = c->layers[run.layer];
@@ -609,10 +644,13 @@ int enqueue_step(Ctx* c, int B, bool sample, bool prof) {
         g.bias = L.bias_o;
         g.sm = streams_behind(c, r, 0, stride, &next_gain);
         g.u = c->st_in;
-        step_linear<GEMV_IN_SPLIT, GEMV_OUT_STREAMS>(c, p.rec(), g);
-      } else {
-        step_linear<GEMV_IN_SPLIT, GEMV_OUT_RESIDUAL>(c, p.rec(), g);
       }
+      next_rows16(c, &g, next_gain);
+      if (rows16(c, B)) g.x16 = c->st_cat16;
+      if (c->streams)
+        step_linear<GEMV_IN_SPLIT, GEMV_IN_BF16_SPLIT, GEMV_OUT_STREAMS>(c, p.rec(), g);
+      else
+        step_linear<GEMV_IN_SPLIT, GEMV_IN_BF16_SPLIT, GEMV_OUT_RESIDUAL>(c, p.rec(), g);
     }
     if (!L.ff) continue;
     {
@@ -628,6 +666,7 @@ int enqueue_step(Ctx* c, int B, bool sample, bool prof) {
       g.eps = eps;
       g.gain = L.norm2;
       g.xielu = L.xielu;
+      if (rows16(c, B)) g.out16 = c->st_u16;
       Prof p(dev, prof, ST_STEP + ST_UP, (double)g.N * c->ldx * 2);
       if (L.glu)
         normed_linear<GEMV_OUT_GLU>(c, p.rec(), g);
@@ -649,13 +688,16 @@ int enqueue_step(Ctx* c, int B, bool sample, bool prof) {
       if (c->streams) {
         g.sm = streams_behind(c, r, 1, stride, &next_gain);
         g.u = c->st_in;
-        step_linear<GEMV_IN_PLAIN, GEMV_OUT_STREAMS>(c, p.rec(), g);
-      } else {
-        step_linear<GEMV_IN_PLAIN, GEMV_OUT_RESIDUAL>(c, p.rec(), g);
       }
+      next_rows16(c, &g, next_gain);
+      if (rows16(c, B)) g.x16 = c->st_u16;
+      if (c->streams)
+        step_linear<GEMV_IN_PLAIN, GEMV_IN_BF16, GEMV_OUT_STREAMS>(c, p.rec(), g);
+      else
+        step_linear<GEMV_IN_PLAIN, GEMV_IN_BF16, GEMV_OUT_RESIDUAL>(c, p.rec(), g);
     }
   }
-  head_rows(c, x_in, B, prof);
+  head_rows(c, x_in, B, prof, false);
   if (sample) {
     k_argmax_partial<<<dim3(ARGMAX_BLOCKS, B), 256, 0, st>>>(c->st_logits, c->vocab, c->am_val, c->am_idx, 0, c->vocab);
     k_argmax_rows_step<<<B, 64, 0, st>>>(c->am_val, c->am_idx, ARGMAX_BLOCKS, c->st_seq, c->st_count, c->st_out, (int)c->st_out_cap);
@@ -997,7 +1039,7 @@ int run_pass(Ctx* c, const std::vector<Part>& parts, float** logits) {
     if (n <= 8) {  // the decode step's classifier
       float* x = c->streams ? c->st_in : c->st_x;
       k_gather_rows<0><<<(unsigned)n, 256, 0, st>>>(c->pf_x, c->ldx, c->width, dw + w0, x, nullptr, 0, nullptr, 0, sum, nullptr);
-      head_rows(c, x, (int)n, true);
+      head_rows(c, x, (int)n, true, true);
       src = c->st_logits;
     } else {
       const size_t gp = LOGIT_ROWS * (size_t)c->ldx;
@@ -1121,6 +1163,13 @@ int create_impl(Ctx* c, const crabml_hip_hybrid_layer_t* layers, const crabml_hi
   CH_TRY(dalloc_n(c, B * c->ld_proj, &c->st_proj));
   CH_TRY(dalloc_n(c, B * c->ld_cat, &c->st_cat));
   CH_TRY(dalloc_n(c, B * c->ld_u, &c->st_u));
+  if (!c->f32) {
+    c->n_xss = (c->width + 15) / 16;
+    CH_TRY(dalloc_n(c, B * c->ldx, &c->st_x16));
+    CH_TRY(dalloc_n(c, B * c->n_xss, &c->st_xss));
+    CH_TRY(dalloc_n(c, B * c->ld_cat, &c->st_cat16));
+    CH_TRY(dalloc_n(c, B * c->ld_u, &c->st_u16));
+  }
   CH_TRY(dalloc_n(c, ss, &c->st_ss));
   CH_TRY(dalloc_n(c, part, &c->st_part));
   CH_TRY(dalloc_n(c, tick, &c->st_tick));

@@ -105,6 +105,7 @@ struct LatStep {
   float* q = nullptr;           // [B][H][rank + rot]
   float* part = nullptr;        // [B][H][LAT_SPLITS][rank + 2]: unnormalized sums, maximum, denominator
   float* cat = nullptr;         // [B][ldc]
+  unsigned short* cat16 = nullptr;  // the same as bf16, instead (nullable)
   int B = 0, ldp = 0, ldc = 0;
   int splits = LAT_SPLITS;
 };
@@ -431,7 +432,7 @@ __global__ __launch_bounds__(256) void k_latent_value(const LatStep a) {
       s = wave_sum_f32(s);
     else
       for (int o = 1; o < lpr; o <<= 1) s += __shfl_xor(s, o, 64);
-    if (k0 == 0 && v < v1 && j * rows + sub < RW) a.cat[(size_t)b * a.ldc + h * g.V + v] = s * g.out_scale;
+    if (k0 == 0 && v < v1 && j * rows + sub < RW) cat_out(a.cat, a.cat16, (size_t)b * a.ldc + h * g.V + v, s * g.out_scale);
   }
 }
 

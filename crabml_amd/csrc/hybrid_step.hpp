@@ -23,22 +23,30 @@ struct StepSeq {
 
 __global__ __launch_bounds__(256) void k_embed_step(const unsigned short* __restrict__ table, const StepSeq* __restrict__ seq, int width, int ldx,
                                                     float scale, const double* __restrict__ freq, float* __restrict__ x, float* __restrict__ emb,
-                                                    const float* __restrict__ add_vec, const StreamMix sm, float* __restrict__ u) {
+                                                    const float* __restrict__ add_vec, const StreamMix sm, float* __restrict__ u,
+                                                    unsigned short* __restrict__ x16, const float* __restrict__ gain, float* __restrict__ xss, int n_xss) {
   const int c = blockIdx.x * 256 + threadIdx.x, b = blockIdx.y;
-  if (c >= width) return;
+  const bool in = c < width;
   const StepSeq s = seq[b];
-  const float v = __builtin_fmaf(bf2f(table[(size_t)s.token * width + c]), scale, position_entry(s.pos, c, freq));
-  if (sm.n) {  // every stream starts as the embedding
-    float r = 0.f;
-    for (int t = 0; t < sm.n; t++) {
-      x[t * sm.stride + (size_t)b * ldx + c] = v;
-      r = __builtin_fmaf(sm.in[t], v, r);
+  float r = 0.f;  // what the first norm reads
+  if (in) {
+    const float v = __builtin_fmaf(bf2f(table[(size_t)s.token * width + c]), scale, position_entry(s.pos, c, freq));
+    if (sm.n) {  // every stream starts as the embedding
+      for (int t = 0; t < sm.n; t++) {
+        x[t * sm.stride + (size_t)b * ldx + c] = v;
+        r = __builtin_fmaf(sm.in[t], v, r);
+      }
+      if (!x16) u[(size_t)b * ldx + c] = r;
+    } else {
+      if (emb) emb[(size_t)b * ldx + c] = v;
+      r = add_vec ? v + add_vec[c] : v;
+      x[(size_t)b * ldx + c] = r;
     }
-    u[(size_t)b * ldx + c] = r;
-    return;
   }
-  if (emb) emb[(size_t)b * ldx + c] = v;
-  x[(size_t)b * ldx + c] = add_vec ? v + add_vec[c] : v;
+  if (!x16) return;
+  if (in) x16[(size_t)b * ldx + c] = f2bf(gain ? r * gain[c] : r);
+  const float q = row16_sum_f32(r * r);
+  if (in && (c & 15) == 0) xss[(size_t)b * n_xss + (c >> 4)] = q;
 }
 
 struct MixStep {
@@ -48,6 +56,7 @@ struct MixStep {
   const StepSeq* seq = nullptr;
   const float* proj = nullptr;  // [B][ldp]
   float* cat = nullptr;         // [B][ldc]: attention columns from 0, linear columns from lin_off
+  unsigned short* cat16 = nullptr;  // the same as bf16, instead (nullable)
   float* ss = nullptr;          // [B][H * slices] square sums of the linear branch
   float* part = nullptr;        // attention partials
   float* v_kept = nullptr;      // [B][ld_vk] values that VMIX_KEEP leaves
@@ -57,6 +66,13 @@ struct MixStep {
 };
 // floats of one partial: per head its V sums, the running maximum and the denominator
 __host__ __device__ inline int mix_part_floats(int V) { return MIX_HEADS * (V + 2); }
+
+__device__ __forceinline__ void cat_out(float* cat, unsigned short* cat16, size_t at, float v) {
+  if (cat16)
+    cat16[at] = f2bf(v);
+  else
+    cat[at] = v;
+}
 
 // One workgroup: up to MIX_HEADS query heads of one kv head over MIX_KEYS cached rows; heads up to CLS wide.  Everything it needs from
 // memory is requested up front; the rest is register and LDS work.  (The launch runs cold: its code is kept short.)
@@ -265,7 +281,7 @@ __device__ __forceinline__ void mix_attention(const MixStep& a, int blk, float* 
         }
       }
     }
-    a.cat[(size_t)b * a.ldc + h0 * g.V + i] = o / l * g_s[i];
+    cat_out(a.cat, a.cat16, (size_t)b * a.ldc + h0 * g.V + i, o / l * g_s[i]);
   }
 }
 
@@ -325,7 +341,7 @@ __device__ __forceinline__ void mix_linear(const MixStep& a, int blk, float* lds
     const bool in = lane < LIN_SLICE && oc < g.V;
     const float ss = wave_sum_f32(in ? r * r : 0.f);
     if (lane == 0) a.ss[(size_t)b * g.H * g.slices + h * g.slices + slice] = ss;
-    if (in) a.cat[(size_t)b * a.ldc + a.lin_off + occ] = r * factor;
+    if (in) cat_out(a.cat, a.cat16, (size_t)b * a.ldc + a.lin_off + occ, r * factor);
   }
 }
 

@@ -1,0 +1,42 @@
+"""The matrix-core linears of a decode step (3 to 16 sequences) at sizes that reach every form of them -- 32 weight rows a workgroup, sixteen
+waves, rows and pieces of k that do not divide -- on one-layer models of both designs against the plain implementations."""
+import numpy as np
+import pytest
+
+from crabml_amd import synth_bifazen as sb
+from crabml_amd import synth_hybrid as sh
+from tests import bifazen_oracle as bo
+from tests import hybrid_oracle as ho
+
+pytestmark = pytest.mark.gpu
+
+
+def nilivik(width, ff, vocab):
+    return sh.config(width, vocab, [sh.layer(4, 2, 24, 40, 100, 3, 16, 24, ff)]), sh.random_tensors, ho
+
+
+def bifazen(width, ff, vocab):
+    return sb.config(width, vocab, [sb.latent(4, 16, 6, 24, 40, 50, ff), sb.attention(4, 2, 24, 40, 50, ff)], streams=3), sb.random_tensors, bo
+
+
+# width, ff, vocab: everything on 16 rows and eight waves; sixteen waves in front of the residual; 32 rows (the vocabulary, Bifazen's gate | up)
+@pytest.mark.parametrize("width,ff,vocab", [(72, 90, 50), (2090, 4104, 60), (328, 8200, 16401)])
+@pytest.mark.parametrize("design", [nilivik, bifazen])
+@pytest.mark.parametrize("f32", [False, True])
+def test_batched_steps(ca, hdev, tmp_path, design, width, ff, vocab, f32):
+    config, tensors, oracle = design(width, ff, vocab)
+    bits = tensors(config, 11, pool=1 << 20)
+    r = ca.load_model(sh.write_model(config, bits, str(tmp_path)), hdev, seq_len=16, f32=f32)
+    floats = {k: sh.from_bf16(v) for k, v in bits.items()}
+    rng = np.random.default_rng(width)
+    toks = rng.integers(0, vocab, (16, 3))
+    want = [oracle.forward(config, floats, t) for t in toks[:3]]
+    for batch in (1, 3, 16, 2):  # (the forms for few rows in between: they share the step's buffers)
+        seqs = [r.open() for _ in range(batch)]
+        got = np.array([r.step([(s, [int(toks[i, t])], [0]) for i, s in enumerate(seqs)]) for t in range(3)])  # [step, sequence, vocab]
+        for s in seqs:
+            r.close(s)
+        for i in range(min(batch, 3)):
+            d = got[:, i] - want[i]
+            # the bounds of the designs' own tests
+            assert np.sqrt((d * d).mean(axis=1)).max() <= (2e-5 if f32 else 2.5e-2) * np.sqrt((want[i] ** 2).mean()), (batch, i)
