@@ -21,11 +21,12 @@
 namespace crabml_hip {
 
 // ---- Q4_0 x Q8_0 ---------------------------------------------------------------------------------
-template <int R>
+template <int R, bool ROWS = false>
 __global__ __launch_bounds__(256) void k_gemv_q4_0(const i32x4* __restrict__ wq, const unsigned short* __restrict__ wd,
-                                                   ActQ8_0 act, float* __restrict__ out, int m, int nb) {
+                                                   ActQ8_0 act, float* __restrict__ out, int m, int nb, RhsRows rr) {
+  RHS_ROW(act, out, m)
   const int lane = threadIdx.x & 63;
-  const int wave = blockIdx.x * (blockDim.x >> 6) + wave_in_wg();
+  const int wave = tile * (blockDim.x >> 6) + wave_in_wg();
   const int row0 = wave * R;
   if (row0 >= m) return;
   float acc[R];
@@ -58,11 +59,12 @@ __global__ __launch_bounds__(256) void k_gemv_q4_0(const i32x4* __restrict__ wq,
 }
 
 // ---- Q8_0 x Q8_0 ---------------------------------------------------------------------------------
-template <int R>
+template <int R, bool ROWS = false>
 __global__ __launch_bounds__(256) void k_gemv_q8_0(const i32x4* __restrict__ wq, const unsigned short* __restrict__ wd,
-                                                   ActQ8_0 act, float* __restrict__ out, int m, int nb) {
+                                                   ActQ8_0 act, float* __restrict__ out, int m, int nb, RhsRows rr) {
+  RHS_ROW(act, out, m)
   const int lane = threadIdx.x & 63;
-  const int wave = blockIdx.x * (blockDim.x >> 6) + wave_in_wg();
+  const int wave = tile * (blockDim.x >> 6) + wave_in_wg();
   const int row0 = wave * R;
   if (row0 >= m) return;
   float acc[R];
@@ -75,11 +77,12 @@ __global__ __launch_bounds__(256) void k_gemv_q8_0(const i32x4* __restrict__ wq,
 }
 
 // ---- Q4_1 x Q8_1 ---------------------------------------------------------------------------------
-template <int R>
+template <int R, bool ROWS = false>
 __global__ __launch_bounds__(256) void k_gemv_q4_1(const i32x4* __restrict__ wq, const unsigned* __restrict__ wdm,
-                                                   ActQ8_1 act, float* __restrict__ out, int m, int nb) {
+                                                   ActQ8_1 act, float* __restrict__ out, int m, int nb, RhsRows rr) {
+  RHS_ROW(act, out, m)
   const int lane = threadIdx.x & 63;
-  const int wave = blockIdx.x * (blockDim.x >> 6) + wave_in_wg();
+  const int wave = tile * (blockDim.x >> 6) + wave_in_wg();
   const int row0 = wave * R;
   if (row0 >= m) return;
   float acc[R];
@@ -99,11 +102,12 @@ __global__ __launch_bounds__(256) void k_gemv_q4_1(const i32x4* __restrict__ wq,
 // (one 128-byte request per wave) and the 6-bit (scale, min) pairs are unpacked in registers.  (Widening the
 // 6-bit fields to bytes at upload -- 20-byte headers, two dword loads, 20 fewer VALU ops -- measured SLOWER:
 // gate/up 8.98 -> 10.88 us; the loop is bound by memory instructions, not by VALU.)
-template <int R>
+template <int R, bool ROWS = false>
 __global__ __launch_bounds__(256) void k_gemv_q4_k(const i32x4* __restrict__ wq, const i32x4* __restrict__ wh, ActQ8_K act,
-                                                   float* __restrict__ out, int m, int nsb) {
+                                                   float* __restrict__ out, int m, int nsb, RhsRows rr) {
+  RHS_ROW(act, out, m)
   const int lane = threadIdx.x & 63;
-  const int wave = blockIdx.x * (blockDim.x >> 6) + wave_in_wg();
+  const int wave = tile * (blockDim.x >> 6) + wave_in_wg();
   const int row0 = wave * R;
   if (row0 >= m) return;
   float acc[R];
@@ -116,11 +120,12 @@ __global__ __launch_bounds__(256) void k_gemv_q4_k(const i32x4* __restrict__ wq,
 }
 
 // ---- Q5_K x Q8_K (buf_q5_k.rs:229-325; rows_partial_q5k, gemv_core.hpp) ---------------------------------------------------------
-template <int R>
+template <int R, bool ROWS = false>
 __global__ __launch_bounds__(256) void k_gemv_q5_k(const char* __restrict__ w, size_t off_qh, ActQ8_K act, float* __restrict__ out, int m,
-                                                   int nsb) {
+                                                   int nsb, RhsRows rr) {
+  RHS_ROW(act, out, m)
   const int lane = threadIdx.x & 63;
-  const int wave = blockIdx.x * (blockDim.x >> 6) + wave_in_wg();
+  const int wave = tile * (blockDim.x >> 6) + wave_in_wg();
   const int row0 = wave * R;
   if (row0 >= m) return;
   float acc[R];
@@ -133,11 +138,12 @@ __global__ __launch_bounds__(256) void k_gemv_q5_k(const char* __restrict__ w, s
 }
 
 // ---- Q5_0 / Q5_1 / Q2_K / Q3_K (piece policies, gemv_core.hpp) -------------------------------------------------------------
-template <class P, int R>
+template <class P, int R, bool ROWS = false>
 __global__ __launch_bounds__(256) void k_gemv_pieces(const char* __restrict__ w, size_t off, size_t n, typename P::Act act,
-                                                     float* __restrict__ out, int m, int nbr) {
+                                                     float* __restrict__ out, int m, int nbr, RhsRows rr) {
+  RHS_ROW(act, out, m)
   const int lane = threadIdx.x & 63;
-  const int wave = blockIdx.x * (blockDim.x >> 6) + wave_in_wg();
+  const int wave = tile * (blockDim.x >> 6) + wave_in_wg();
   const int row0 = wave * R;
   if (row0 >= m) return;
   float acc[R];
@@ -169,11 +175,12 @@ __global__ void k_block_dots_pieces(const char* __restrict__ w, size_t off, size
 // 4 bits of two 16-element scale groups -- low nibbles: elements 128 h + 32 a + 16 p + [0, 16), high nibbles: the
 // same + 64 -- and the matching 2-bit planes sit in qh[32 h + 16 p .. +16) at bit 2 a and 2 a + 4
 // (buf_q6_k.rs:21-48).  6-bit values are rebuilt as bytes for v_dot4; the -32 offset is applied as -32 * bsum.
-template <int R>
+template <int R, bool ROWS = false>
 __global__ __launch_bounds__(256) void k_gemv_q6_k(const char* __restrict__ w, size_t off_qh, ActQ8_K act,
-                                                   float* __restrict__ out, int m, int nsb) {
+                                                   float* __restrict__ out, int m, int nsb, RhsRows rr) {
+  RHS_ROW(act, out, m)
   const int lane = threadIdx.x & 63;
-  const int wave = blockIdx.x * (blockDim.x >> 6) + wave_in_wg();
+  const int wave = tile * (blockDim.x >> 6) + wave_in_wg();
   const int row0 = wave * R;
   if (row0 >= m) return;
   float acc[R];
@@ -188,11 +195,12 @@ __global__ __launch_bounds__(256) void k_gemv_q6_k(const char* __restrict__ w, s
 // ---- Q8_K x Q8_K ---------------------------------------------------------------------------------
 // planes: qs[n][256] | d[n] f32.  A lane owns one 32-element group; the 8 lanes of a super-block add
 // their integer partials (exact) before the single f32 scaling `sum_i as f32 * d_a * d_b`.
-template <int R>
+template <int R, bool ROWS = false>
 __global__ __launch_bounds__(256) void k_gemv_q8_k(const i32x4* __restrict__ wq, const float* __restrict__ wd,
-                                                   ActQ8_K act, float* __restrict__ out, int m, int nsb) {
+                                                   ActQ8_K act, float* __restrict__ out, int m, int nsb, RhsRows rr) {
+  RHS_ROW(act, out, m)
   const int lane = threadIdx.x & 63;
-  const int wave = blockIdx.x * (blockDim.x >> 6) + wave_in_wg();
+  const int wave = tile * (blockDim.x >> 6) + wave_in_wg();
   const int row0 = wave * R;
   if (row0 >= m) return;
   float acc[R];
@@ -227,10 +235,12 @@ __global__ __launch_bounds__(256) void k_gemv_q8_k(const i32x4* __restrict__ wq,
 }
 
 // ---- F32 / F16 weights ---------------------------------------------------------------------------
+template <bool ROWS = false>
 __global__ __launch_bounds__(256) void k_gemv_f32(const float* __restrict__ w, const float* __restrict__ x,
-                                                  float* __restrict__ out, int m, int k) {
+                                                  float* __restrict__ out, int m, int k, RhsRows rr) {
+  RHS_ROW(x, out, m)
   const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * (blockDim.x >> 6) + wave_in_wg();
+  const int row = tile * (blockDim.x >> 6) + wave_in_wg();
   if (row >= m) return;
   const float* wr = w + (size_t)row * k;
   float acc = 0.f;
@@ -241,12 +251,13 @@ __global__ __launch_bounds__(256) void k_gemv_f32(const float* __restrict__ w, c
 // F16 rows: a lane takes 16 bytes of R neighbouring rows and of the rhs at a time (UN steps of 512 elements in flight), products are exact in
 // f32 (v_fma_mix_f32: no conversions), sums f32.  Bound by the weights' bytes: 32000 x 2048 25.9 us (5.1 TB/s; two bytes a lane at a time:
 // 68.6), 8192 x 2048 7.8 (9.3), 2048 x 8192 10.4 (36).
-template <int R>
+template <int R, bool ROWS = false>
 __global__ __launch_bounds__(256) void k_gemv_f16(const unsigned short* __restrict__ w, const unsigned short* __restrict__ x16,
-                                                  float* __restrict__ out, int m, int k) {
+                                                  float* __restrict__ out, int m, int k, RhsRows rr) {
+  RHS_ROW(x16, out, m)
   constexpr int UN = R >= 4 ? 2 : 4;
   const int lane = threadIdx.x & 63;
-  const int row0 = (blockIdx.x * (blockDim.x >> 6) + wave_in_wg()) * R;
+  const int row0 = (tile * (blockDim.x >> 6) + wave_in_wg()) * R;
   if (row0 >= m) return;
   const unsigned short* wr[R];
 #pragma unroll
@@ -289,10 +300,12 @@ __global__ __launch_bounds__(256) void k_gemv_f16(const unsigned short* __restri
   }
 }
 // F16 rows that are not whole 16-byte pieces
+template <bool ROWS = false>
 __global__ __launch_bounds__(256) void k_gemv_f16_any(const unsigned short* __restrict__ w, const unsigned short* __restrict__ x16,
-                                                      float* __restrict__ out, int m, int k) {
+                                                      float* __restrict__ out, int m, int k, RhsRows rr) {
+  RHS_ROW(x16, out, m)
   const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * (blockDim.x >> 6) + wave_in_wg();
+  const int row = tile * (blockDim.x >> 6) + wave_in_wg();
   if (row >= m) return;
   const unsigned short* wr = w + (size_t)row * k;
   float acc = 0.f;
@@ -302,10 +315,12 @@ __global__ __launch_bounds__(256) void k_gemv_f16_any(const unsigned short* __re
 }
 
 // bfloat16 rows of any length x f32 (rows whose k the vectorized kernel of gemv_bf16.hpp does not take)
+template <bool ROWS = false>
 __global__ __launch_bounds__(256) void k_gemv_bf16_any(const unsigned short* __restrict__ w, const float* __restrict__ x,
-                                                       float* __restrict__ out, int m, int k) {
+                                                       float* __restrict__ out, int m, int k, RhsRows rr) {
+  RHS_ROW(x, out, m)
   const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * (blockDim.x >> 6) + wave_in_wg();
+  const int row = tile * (blockDim.x >> 6) + wave_in_wg();
   if (row >= m) return;
   const unsigned short* wr = w + (size_t)row * k;
   float acc = 0.f;
@@ -328,6 +343,15 @@ static void launch_rows(hipStream_t st, int m, int n_cu, F&& f) {
   (void)n_cu;
 }
 
+// one row of the rhs, or all of `rows` in one launch
+#define GEMV_LAUNCH(ONE_, ROWS_, tiles_, tpb_, ...)                                                                                            \
+  do {                                                                                                                                       \
+    const int tiles__ = (tiles_);                                                                                                            \
+    if (rows == 1)                                                                                                                           \
+      launch_k(st, rec, ONE_, dim3((unsigned)tiles__), dim3(tpb_), 0, __VA_ARGS__, RhsRows{});                                               \
+    else                                                                                                                                     \
+      launch_k(st, rec, ROWS_, dim3(rhs_rows_grid((unsigned)tiles__, rows)), dim3(tpb_), 0, __VA_ARGS__, RhsRows{tiles__, (int)rows, act_stride}); \
+  } while (0)
 int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m_, size_t k_, const void* act, size_t b,
                 float* out, crabml_hip_device::ProfRec* rec0, bool fused_add) {
   hipStream_t st = dev->stream;
@@ -354,19 +378,20 @@ int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m_, size
     if (launch_gemm_f16(dev, rec0, ws, &m_, 1, k_, act, al.total, b, &out, GemmScratch{})) return 0;
   }
   if (b >= 16 && launch_gemm_mfma(dev, w, m_, k_, act, b, out, rec0, nullptr, fused_add)) return 0;
-  for (size_t bi = 0; bi < b; bi++) {
-    const char* ap = (const char*)act + bi * act_stride;
-    float* o = out + bi * m_;
-    crabml_hip_device::ProfRec* rec = bi == 0 ? rec0 : nullptr;
+  for (size_t b0 = 0; b0 < b; b0 += RHS_ROWS_MAX) {
+    const size_t rows = b - b0 < RHS_ROWS_MAX ? b - b0 : RHS_ROWS_MAX;
+    const char* ap = (const char*)act + b0 * act_stride;
+    float* o = out + b0 * m_;
+    crabml_hip_device::ProfRec* rec = b0 == 0 ? rec0 : nullptr;
     switch (w->dtype) {
       case CRABML_HIP_Q4_0: {
         ActQ8_0 a{(const i32x4*)ap, (const unsigned short*)(ap + al.off_d), (const int*)(ap + al.off_aux)};
         const int nb = k / 32;
         launch_rows(st, m, dev->n_cu, [&](int R, int grid, int tpb) {
           if (R == 2)
-            launch_k(st, rec, k_gemv_q4_0<2>, dim3(grid), dim3(tpb), 0, (const i32x4*)wp, (const unsigned short*)(wp + w->wl.off_scale), a, o, m, nb);
+            GEMV_LAUNCH((k_gemv_q4_0<2>), (k_gemv_q4_0<2, true>), grid, tpb, (const i32x4*)wp, (const unsigned short*)(wp + w->wl.off_scale), a, o, m, nb);
           else
-            launch_k(st, rec, k_gemv_q4_0<1>, dim3(grid), dim3(tpb), 0, (const i32x4*)wp, (const unsigned short*)(wp + w->wl.off_scale), a, o, m, nb);
+            GEMV_LAUNCH((k_gemv_q4_0<1>), (k_gemv_q4_0<1, true>), grid, tpb, (const i32x4*)wp, (const unsigned short*)(wp + w->wl.off_scale), a, o, m, nb);
         });
         break;
       }
@@ -375,9 +400,9 @@ int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m_, size
         const int nb = k / 32;
         launch_rows(st, m, dev->n_cu, [&](int R, int grid, int tpb) {
           if (R == 2)
-            launch_k(st, rec, k_gemv_q8_0<2>, dim3(grid), dim3(tpb), 0, (const i32x4*)wp, (const unsigned short*)(wp + w->wl.off_scale), a, o, m, nb);
+            GEMV_LAUNCH((k_gemv_q8_0<2>), (k_gemv_q8_0<2, true>), grid, tpb, (const i32x4*)wp, (const unsigned short*)(wp + w->wl.off_scale), a, o, m, nb);
           else
-            launch_k(st, rec, k_gemv_q8_0<1>, dim3(grid), dim3(tpb), 0, (const i32x4*)wp, (const unsigned short*)(wp + w->wl.off_scale), a, o, m, nb);
+            GEMV_LAUNCH((k_gemv_q8_0<1>), (k_gemv_q8_0<1, true>), grid, tpb, (const i32x4*)wp, (const unsigned short*)(wp + w->wl.off_scale), a, o, m, nb);
         });
         break;
       }
@@ -386,9 +411,9 @@ int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m_, size
         const int nb = k / 32;
         launch_rows(st, m, dev->n_cu, [&](int R, int grid, int tpb) {
           if (R == 2)
-            launch_k(st, rec, k_gemv_q4_1<2>, dim3(grid), dim3(tpb), 0, (const i32x4*)wp, (const unsigned*)(wp + w->wl.off_scale), a, o, m, nb);
+            GEMV_LAUNCH((k_gemv_q4_1<2>), (k_gemv_q4_1<2, true>), grid, tpb, (const i32x4*)wp, (const unsigned*)(wp + w->wl.off_scale), a, o, m, nb);
           else
-            launch_k(st, rec, k_gemv_q4_1<1>, dim3(grid), dim3(tpb), 0, (const i32x4*)wp, (const unsigned*)(wp + w->wl.off_scale), a, o, m, nb);
+            GEMV_LAUNCH((k_gemv_q4_1<1>), (k_gemv_q4_1<1, true>), grid, tpb, (const i32x4*)wp, (const unsigned*)(wp + w->wl.off_scale), a, o, m, nb);
         });
         break;
       }
@@ -397,9 +422,9 @@ int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m_, size
         const int nsb = k / 256;
         launch_rows(st, m, dev->n_cu, [&](int R, int grid, int tpb) {
           if (R == 2)
-            launch_k(st, rec, k_gemv_q4_k<2>, dim3(grid), dim3(tpb), 0, (const i32x4*)wp, (const i32x4*)(wp + w->wl.off_scale), a, o, m, nsb);
+            GEMV_LAUNCH((k_gemv_q4_k<2>), (k_gemv_q4_k<2, true>), grid, tpb, (const i32x4*)wp, (const i32x4*)(wp + w->wl.off_scale), a, o, m, nsb);
           else
-            launch_k(st, rec, k_gemv_q4_k<1>, dim3(grid), dim3(tpb), 0, (const i32x4*)wp, (const i32x4*)(wp + w->wl.off_scale), a, o, m, nsb);
+            GEMV_LAUNCH((k_gemv_q4_k<1>), (k_gemv_q4_k<1, true>), grid, tpb, (const i32x4*)wp, (const i32x4*)(wp + w->wl.off_scale), a, o, m, nsb);
         });
         break;
       }
@@ -408,9 +433,9 @@ int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m_, size
         const int nsb = k / 256;
         launch_rows(st, m, dev->n_cu, [&](int R, int grid, int tpb) {
           if (R == 2)
-            launch_k(st, rec, k_gemv_q5_k<2>, dim3(grid), dim3(tpb), 0, wp, w->wl.off_scale, a, o, m, nsb);
+            GEMV_LAUNCH((k_gemv_q5_k<2>), (k_gemv_q5_k<2, true>), grid, tpb, wp, w->wl.off_scale, a, o, m, nsb);
           else
-            launch_k(st, rec, k_gemv_q5_k<1>, dim3(grid), dim3(tpb), 0, wp, w->wl.off_scale, a, o, m, nsb);
+            GEMV_LAUNCH((k_gemv_q5_k<1>), (k_gemv_q5_k<1, true>), grid, tpb, wp, w->wl.off_scale, a, o, m, nsb);
         });
         break;
       }
@@ -419,9 +444,9 @@ int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m_, size
         const int nsb = k / 256;
         launch_rows(st, m, dev->n_cu, [&](int R, int grid, int tpb) {
           if (R == 2)
-            launch_k(st, rec, k_gemv_q6_k<2>, dim3(grid), dim3(tpb), 0, wp, w->wl.off_scale, a, o, m, nsb);
+            GEMV_LAUNCH((k_gemv_q6_k<2>), (k_gemv_q6_k<2, true>), grid, tpb, wp, w->wl.off_scale, a, o, m, nsb);
           else
-            launch_k(st, rec, k_gemv_q6_k<1>, dim3(grid), dim3(tpb), 0, wp, w->wl.off_scale, a, o, m, nsb);
+            GEMV_LAUNCH((k_gemv_q6_k<1>), (k_gemv_q6_k<1, true>), grid, tpb, wp, w->wl.off_scale, a, o, m, nsb);
         });
         break;
       }
@@ -430,9 +455,9 @@ int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m_, size
         const int nsb = k / 256;
         launch_rows(st, m, dev->n_cu, [&](int R, int grid, int tpb) {
           if (R == 2)
-            launch_k(st, rec, k_gemv_q8_k<2>, dim3(grid), dim3(tpb), 0, (const i32x4*)wp, (const float*)(wp + w->wl.off_scale), a, o, m, nsb);
+            GEMV_LAUNCH((k_gemv_q8_k<2>), (k_gemv_q8_k<2, true>), grid, tpb, (const i32x4*)wp, (const float*)(wp + w->wl.off_scale), a, o, m, nsb);
           else
-            launch_k(st, rec, k_gemv_q8_k<1>, dim3(grid), dim3(tpb), 0, (const i32x4*)wp, (const float*)(wp + w->wl.off_scale), a, o, m, nsb);
+            GEMV_LAUNCH((k_gemv_q8_k<1>), (k_gemv_q8_k<1, true>), grid, tpb, (const i32x4*)wp, (const float*)(wp + w->wl.off_scale), a, o, m, nsb);
         });
         break;
       }
@@ -440,9 +465,9 @@ int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m_, size
         ActQ8_0 a{(const i32x4*)ap, (const unsigned short*)(ap + al.off_d), (const int*)(ap + al.off_aux)};
         launch_rows(st, m, dev->n_cu, [&](int R, int grid, int tpb) {
           if (R == 2)
-            launch_k(st, rec, k_gemv_pieces<PieceQ5_0, 2>, dim3(grid), dim3(tpb), 0, wp, w->wl.off_scale, w->wl.n_blocks, a, o, m, k / 32);
+            GEMV_LAUNCH((k_gemv_pieces<PieceQ5_0, 2>), (k_gemv_pieces<PieceQ5_0, 2, true>), grid, tpb, wp, w->wl.off_scale, w->wl.n_blocks, a, o, m, k / 32);
           else
-            launch_k(st, rec, k_gemv_pieces<PieceQ5_0, 1>, dim3(grid), dim3(tpb), 0, wp, w->wl.off_scale, w->wl.n_blocks, a, o, m, k / 32);
+            GEMV_LAUNCH((k_gemv_pieces<PieceQ5_0, 1>), (k_gemv_pieces<PieceQ5_0, 1, true>), grid, tpb, wp, w->wl.off_scale, w->wl.n_blocks, a, o, m, k / 32);
         });
         break;
       }
@@ -450,9 +475,9 @@ int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m_, size
         ActQ8_1 a{(const i32x4*)ap, (const unsigned short*)(ap + al.off_d), (const unsigned short*)(ap + al.off_aux)};
         launch_rows(st, m, dev->n_cu, [&](int R, int grid, int tpb) {
           if (R == 2)
-            launch_k(st, rec, k_gemv_pieces<PieceQ5_1, 2>, dim3(grid), dim3(tpb), 0, wp, w->wl.off_scale, w->wl.n_blocks, a, o, m, k / 32);
+            GEMV_LAUNCH((k_gemv_pieces<PieceQ5_1, 2>), (k_gemv_pieces<PieceQ5_1, 2, true>), grid, tpb, wp, w->wl.off_scale, w->wl.n_blocks, a, o, m, k / 32);
           else
-            launch_k(st, rec, k_gemv_pieces<PieceQ5_1, 1>, dim3(grid), dim3(tpb), 0, wp, w->wl.off_scale, w->wl.n_blocks, a, o, m, k / 32);
+            GEMV_LAUNCH((k_gemv_pieces<PieceQ5_1, 1>), (k_gemv_pieces<PieceQ5_1, 1, true>), grid, tpb, wp, w->wl.off_scale, w->wl.n_blocks, a, o, m, k / 32);
         });
         break;
       }
@@ -460,9 +485,9 @@ int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m_, size
         const ActQ8_K a = act_q8k_at(ap, al.off_d, al.off_aux, al.off_p);
         launch_rows(st, m, dev->n_cu, [&](int R, int grid, int tpb) {
           if (R == 2)
-            launch_k(st, rec, k_gemv_pieces<PieceQ2_K, 2>, dim3(grid), dim3(tpb), 0, wp, w->wl.off_scale, w->wl.n_blocks, a, o, m, k / 256);
+            GEMV_LAUNCH((k_gemv_pieces<PieceQ2_K, 2>), (k_gemv_pieces<PieceQ2_K, 2, true>), grid, tpb, wp, w->wl.off_scale, w->wl.n_blocks, a, o, m, k / 256);
           else
-            launch_k(st, rec, k_gemv_pieces<PieceQ2_K, 1>, dim3(grid), dim3(tpb), 0, wp, w->wl.off_scale, w->wl.n_blocks, a, o, m, k / 256);
+            GEMV_LAUNCH((k_gemv_pieces<PieceQ2_K, 1>), (k_gemv_pieces<PieceQ2_K, 1, true>), grid, tpb, wp, w->wl.off_scale, w->wl.n_blocks, a, o, m, k / 256);
         });
         break;
       }
@@ -470,31 +495,31 @@ int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m_, size
         const ActQ8_K a = act_q8k_at(ap, al.off_d, al.off_aux, al.off_p);
         launch_rows(st, m, dev->n_cu, [&](int R, int grid, int tpb) {
           if (R == 2)
-            launch_k(st, rec, k_gemv_pieces<PieceQ3_K, 2>, dim3(grid), dim3(tpb), 0, wp, w->wl.off_scale, w->wl.n_blocks, a, o, m, k / 256);
+            GEMV_LAUNCH((k_gemv_pieces<PieceQ3_K, 2>), (k_gemv_pieces<PieceQ3_K, 2, true>), grid, tpb, wp, w->wl.off_scale, w->wl.n_blocks, a, o, m, k / 256);
           else
-            launch_k(st, rec, k_gemv_pieces<PieceQ3_K, 1>, dim3(grid), dim3(tpb), 0, wp, w->wl.off_scale, w->wl.n_blocks, a, o, m, k / 256);
+            GEMV_LAUNCH((k_gemv_pieces<PieceQ3_K, 1>), (k_gemv_pieces<PieceQ3_K, 1, true>), grid, tpb, wp, w->wl.off_scale, w->wl.n_blocks, a, o, m, k / 256);
         });
         break;
       }
       case CRABML_HIP_F32: {
         int grid = (m + 3) / 4;
-        launch_k(st, rec, k_gemv_f32, dim3(grid), dim3(256), 0, (const float*)wp, (const float*)ap, o, m, k);
+        GEMV_LAUNCH((k_gemv_f32<>), (k_gemv_f32<true>), grid, 256, (const float*)wp, (const float*)ap, o, m, k);
         break;
       }
       case CRABML_HIP_F16: {
         const unsigned short *wh = (const unsigned short*)wp, *xh = (const unsigned short*)ap;
         if (k % 8 != 0)
-          launch_k(st, rec, k_gemv_f16_any, dim3((m + 3) / 4), dim3(256), 0, wh, xh, o, m, k);
+          GEMV_LAUNCH((k_gemv_f16_any<>), (k_gemv_f16_any<true>), (m + 3) / 4, 256, wh, xh, o, m, k);
         else if (m >= 16384)  // (enough rows to give a wave four and still fill the chip)
-          launch_k(st, rec, k_gemv_f16<4>, dim3((m + 15) / 16), dim3(256), 0, wh, xh, o, m, k);
+          GEMV_LAUNCH((k_gemv_f16<4>), (k_gemv_f16<4, true>), (m + 15) / 16, 256, wh, xh, o, m, k);
         else if (m >= 2048)
-          launch_k(st, rec, k_gemv_f16<2>, dim3((m + 7) / 8), dim3(256), 0, wh, xh, o, m, k);
+          GEMV_LAUNCH((k_gemv_f16<2>), (k_gemv_f16<2, true>), (m + 7) / 8, 256, wh, xh, o, m, k);
         else
-          launch_k(st, rec, k_gemv_f16<1>, dim3((m + 3) / 4), dim3(256), 0, wh, xh, o, m, k);
+          GEMV_LAUNCH((k_gemv_f16<1>), (k_gemv_f16<1, true>), (m + 3) / 4, 256, wh, xh, o, m, k);
         break;
       }
       case CRABML_HIP_BF16: {
-        launch_k(st, rec, k_gemv_bf16_any, dim3((m + 3) / 4), dim3(256), 0, (const unsigned short*)wp, (const float*)ap, o, m, k);
+        GEMV_LAUNCH((k_gemv_bf16_any<>), (k_gemv_bf16_any<true>), (m + 3) / 4, 256, (const unsigned short*)wp, (const float*)ap, o, m, k);
         break;
       }
       default:

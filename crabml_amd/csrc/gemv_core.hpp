@@ -60,6 +60,42 @@ __host__ __device__ inline ActQ8_K act_q8k_at(const char* planes, size_t off_d, 
   return ActQ8_K{(const i32x4*)planes, (const float*)(planes + off_d), (const short*)(planes + off_aux), (const i32x4*)(planes + off_p)};
 }
 
+// ---- a row kernel on several rows of the rhs (short prompts, formats without a matrix-core kernel): one launch.  A weight tile's rows of
+// the rhs run back to back on one XCD (block id % 8), so the tile comes from memory once and then from that XCD's L2.
+struct RhsRows {
+  int tiles = 0, rows = 1;
+  size_t stride = 0;  // bytes between the rows' activation planes
+};
+inline unsigned rhs_rows_grid(unsigned tiles, size_t rows) { return rows == 1 ? tiles : (unsigned)((tiles + 7) / 8 * 8 * rows); }
+constexpr size_t RHS_ROWS_MAX = 256;  // of one launch
+template <bool ROWS>
+__device__ __forceinline__ bool rhs_row(const RhsRows& r, int* tile, int* row) {
+  *tile = blockIdx.x;
+  *row = 0;
+  if constexpr (ROWS) {
+    const int j = (int)blockIdx.x >> 3;
+    *tile = j / r.rows * 8 + ((int)blockIdx.x & 7);
+    *row = j % r.rows;
+    return *tile < r.tiles;
+  }
+  return true;
+}
+template <typename T>
+__device__ __forceinline__ const T* rhs_at(const T* p, size_t bytes) {
+  return (const T*)((const char*)p + bytes);
+}
+__device__ __forceinline__ ActQ8_0 rhs_at(ActQ8_0 a, size_t n) { return {rhs_at(a.q, n), rhs_at(a.d, n), rhs_at(a.isum, n)}; }
+__device__ __forceinline__ ActQ8_1 rhs_at(ActQ8_1 a, size_t n) { return {rhs_at(a.q, n), rhs_at(a.d, n), rhs_at(a.s, n)}; }
+__device__ __forceinline__ ActQ8_K rhs_at(ActQ8_K a, size_t n) { return {rhs_at(a.q, n), rhs_at(a.d, n), rhs_at(a.bsums, n), rhs_at(a.qp, n)}; }
+// in front of a row kernel's body: `act` and `out` become this workgroup's row's, the wave's index counts its tile's waves
+#define RHS_ROW(act_, out_, m_)                                   \
+  int tile, rhs_i;                                                \
+  if (!rhs_row<ROWS>(rr, &tile, &rhs_i)) return;                  \
+  if constexpr (ROWS) {                                           \
+    act_ = rhs_at(act_, rhs_i * rr.stride);                       \
+    out_ += (size_t)rhs_i * m_;                                   \
+  }
+
 // ---- the fast step's hop-free norm: 1 / rms applied by the CONSUMER of the quantized row ------------------------------------
 // RMSNorm divides the whole row by one number, and the truncating rhs quantizer's levels q = trunc(v / (max|v| / 127))
 // (buf_q8_0.rs:119-124) do not depend on a common factor of v.  So the wo / ffn_down launch that produces the residual row x

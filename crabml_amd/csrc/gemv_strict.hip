@@ -14,10 +14,13 @@
 
 namespace crabml_hip {
 
+template <bool ROWS = false>
 __global__ __launch_bounds__(64) void k_gemv_strict(const char* __restrict__ w, int dtype, size_t off_scale,
                                                     const char* __restrict__ act, size_t off_d, size_t off_aux,
-                                                    float* __restrict__ out, const float* add, int m, int k) {
-  const int row = blockIdx.x * blockDim.x + threadIdx.x;
+                                                    float* __restrict__ out, const float* add, int m, int k, RhsRows rr) {
+  RHS_ROW(act, out, m)
+  if constexpr (ROWS) add += add ? (size_t)rhs_i * m : 0;
+  const int row = tile * blockDim.x + threadIdx.x;
   if (row >= m) return;
   float sumf = 0.0f;
   switch (dtype) {
@@ -314,12 +317,14 @@ __device__ __forceinline__ void exact_chain_store(const float* __restrict__ T, i
   }
 }
 
-template <int FMT, int R>
+template <int FMT, int R, bool ROWS = false>
 __global__ __launch_bounds__(256) void k_gemv_exact_blk(const i32x4* __restrict__ wq, const unsigned short* __restrict__ wd,
-                                                        typename ActOf<FMT>::type act, float* __restrict__ out, const float* add, int m, int nb) {
+                                                        typename ActOf<FMT>::type act, float* __restrict__ out, const float* add, int m, int nb, RhsRows rr) {
+  RHS_ROW(act, out, m)
+  if constexpr (ROWS) add += add ? (size_t)rhs_i * m : 0;
   extern __shared__ __attribute__((aligned(16))) float exact_terms[];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int wave = blockIdx.x * (blockDim.x >> 6) + wv;
+  const int wave = tile * (blockDim.x >> 6) + wv;
   const int row0 = wave * R;
   if (row0 >= m) return;
   const int nt = (nb + 3) & ~3;  // row stride of the term table (16-byte aligned rows)
@@ -328,12 +333,14 @@ __global__ __launch_bounds__(256) void k_gemv_exact_blk(const i32x4* __restrict_
   exact_chain_store<R>(T, nb, nt, row0, m, lane, out, add);
 }
 
-template <class P, int R>
+template <class P, int R, bool ROWS = false>
 __global__ __launch_bounds__(256) void k_gemv_exact_pieces(const char* __restrict__ w, size_t off, size_t n, typename P::Act act,
-                                                           float* __restrict__ out, const float* add, int m, int nbr) {
+                                                           float* __restrict__ out, const float* add, int m, int nbr, RhsRows rr) {
+  RHS_ROW(act, out, m)
+  if constexpr (ROWS) add += add ? (size_t)rhs_i * m : 0;
   extern __shared__ __attribute__((aligned(16))) float exact_terms[];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int wave = blockIdx.x * (blockDim.x >> 6) + wv;
+  const int wave = tile * (blockDim.x >> 6) + wv;
   const int row0 = wave * R;
   if (row0 >= m) return;
   const int nt = (nbr + 3) & ~3;
@@ -363,12 +370,14 @@ __global__ __launch_bounds__(256) void k_gemv_exact_pieces(const char* __restric
   exact_chain_store<R>(T, nbr, nt, row0, m, lane, out, add);
 }
 
-template <int R>
+template <int R, bool ROWS = false>
 __global__ __launch_bounds__(256) void k_gemv_exact_q8k(const i32x4* __restrict__ wq, const float* __restrict__ wd, ActQ8_K act,
-                                                        float* __restrict__ out, const float* add, int m, int nsb) {
+                                                        float* __restrict__ out, const float* add, int m, int nsb, RhsRows rr) {
+  RHS_ROW(act, out, m)
+  if constexpr (ROWS) add += add ? (size_t)rhs_i * m : 0;
   extern __shared__ __attribute__((aligned(16))) float exact_terms[];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int wave = blockIdx.x * (blockDim.x >> 6) + wv;
+  const int wave = tile * (blockDim.x >> 6) + wv;
   const int row0 = wave * R;
   if (row0 >= m) return;
   const int nt = (nsb + 3) & ~3;
@@ -404,12 +413,14 @@ __global__ __launch_bounds__(256) void k_gemv_exact_q8k(const i32x4* __restrict_
 // fast kernel does, splits its v_dot4 sums by byte position (byte k of dword i is element class 4 (i & 1) + k: the activation dword
 // is masked to one byte per v_dot4), the eight lanes of a super-block add their integers (DPP), and the first of them parks the nine
 // terms in LDS; one lane per row then runs the nine chains over the super-blocks in order.  Bit-identical to k_gemv_strict's case.
-template <bool Q5, int R>
+template <bool Q5, int R, bool ROWS = false>
 __global__ __launch_bounds__(256) void k_gemv_exact_q4k(const char* __restrict__ w, size_t off_scale, ActQ8_K act, float* __restrict__ out, const float* add, int m,
-                                                        int nsb) {
+                                                        int nsb, RhsRows rr) {
+  RHS_ROW(act, out, m)
+  if constexpr (ROWS) add += add ? (size_t)rhs_i * m : 0;
   extern __shared__ __attribute__((aligned(16))) float exact_terms[];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int wave = blockIdx.x * (blockDim.x >> 6) + wv;
+  const int wave = tile * (blockDim.x >> 6) + wv;
   const int row0 = wave * R;
   if (row0 >= m) return;
   const size_t n5 = off_scale / 128;  // (Q5_K: blocks in the tensor; planes qs | qh | hdr)
@@ -517,12 +528,14 @@ __global__ __launch_bounds__(256) void k_gemv_exact_q4k(const char* __restrict__
 
 // ---- Q6_K (buf_q6_k.rs:183-234): eight f32 lanes as above, no minimum term; the levels are made signed bytes (q6 - 32) so that the
 // byte-split v_dot4 sums are the reference's products directly.  planes ql | qh | scales | d (common.hpp), n = off_scale / 128 blocks.
-template <int R>
+template <int R, bool ROWS = false>
 __global__ __launch_bounds__(256) void k_gemv_exact_q6k(const char* __restrict__ w, size_t off_qh, ActQ8_K act, float* __restrict__ out, const float* add, int m,
-                                                        int nsb) {
+                                                        int nsb, RhsRows rr) {
+  RHS_ROW(act, out, m)
+  if constexpr (ROWS) add += add ? (size_t)rhs_i * m : 0;
   extern __shared__ __attribute__((aligned(16))) float exact_terms[];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int wave = blockIdx.x * (blockDim.x >> 6) + wv;
+  const int wave = tile * (blockDim.x >> 6) + wv;
   const int row0 = wave * R;
   if (row0 >= m) return;
   const size_t n = off_qh / 128;
@@ -618,12 +631,14 @@ __global__ __launch_bounds__(256) void k_gemv_exact_q6k(const char* __restrict__
 // ---- Q3_K (buf_q3_k.rs:238-329): eight i32 lanes per super-block (element e feeds lane e % 8), `sums[l] += d * aux32[l]`, the sums
 // reduced in order at the end.  A lane takes one 16-byte qs piece = four 16-element scale groups (PieceQ3_K, gemv_core.hpp); the levels
 // (2 low bits | hmask bit << 2) - 4 are made signed bytes and the v_dot4 sums split by byte position as for Q4_K.
-template <int R>
+template <int R, bool ROWS = false>
 __global__ __launch_bounds__(256) void k_gemv_exact_q3k(const char* __restrict__ w, size_t off, size_t n, ActQ8_K act, float* __restrict__ out,
-                                                        const float* add, int m, int nsb) {
+                                                        const float* add, int m, int nsb, RhsRows rr) {
+  RHS_ROW(act, out, m)
+  if constexpr (ROWS) add += add ? (size_t)rhs_i * m : 0;
   extern __shared__ __attribute__((aligned(16))) float exact_terms[];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int wave = blockIdx.x * (blockDim.x >> 6) + wv;
+  const int wave = tile * (blockDim.x >> 6) + wv;
   const int row0 = wave * R;
   if (row0 >= m) return;
   const int stride = nsb * 8;
@@ -696,6 +711,15 @@ __global__ __launch_bounds__(256) void k_gemv_exact_q3k(const char* __restrict__
   }
 }
 
+// one row of the rhs, or all of `rows` in one launch
+#define STRICT_LAUNCH(ONE_, ROWS_, tiles_, tpb_, lds_, ...)                                                                                     \
+  do {                                                                                                                                       \
+    const unsigned tiles__ = (tiles_);                                                                                                       \
+    if (rows == 1)                                                                                                                           \
+      launch_k(dev->stream, nullptr, ONE_, dim3(tiles__), dim3(tpb_), lds_, __VA_ARGS__, RhsRows{});                                         \
+    else                                                                                                                                     \
+      launch_k(dev->stream, nullptr, ROWS_, dim3(rhs_rows_grid(tiles__, rows)), dim3(tpb_), lds_, __VA_ARGS__, RhsRows{(int)tiles__, (int)rows, act_stride}); \
+  } while (0)
 int launch_gemv_strict(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m, size_t k, const void* act, size_t b,
                        float* out, const float* add_all) {
   const uint32_t qt = vec_dot_rhs_dtype(w->dtype);
@@ -713,10 +737,11 @@ int launch_gemv_strict(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m
     const char* e = getenv("CRABML_HIP_STRICT_SCALAR");
     return h && h[0] == '1' && e && e[0] == '1';
   }();
-  for (size_t bi = 0; bi < b; bi++) {
-    const char* ap = (const char*)act + bi * act_stride;
-    float* o = out + bi * m;
-    const float* add = add_all ? add_all + bi * m : nullptr;  // the residual row of THIS batch row
+  for (size_t b0 = 0; b0 < b; b0 += RHS_ROWS_MAX) {
+    const size_t rows = b - b0 < RHS_ROWS_MAX ? b - b0 : RHS_ROWS_MAX;
+    const char* ap = (const char*)act + b0 * act_stride;
+    float* o = out + b0 * m;
+    const float* add = add_all ? add_all + b0 * m : nullptr;  // the residual rows of these batch rows
     bool done = false;
     if (!scalar_only && lds <= 48 * 1024 && block_elems(w->dtype) > 1) {
       done = true;
@@ -725,22 +750,22 @@ int launch_gemv_strict(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m
       const ActQ8_K ak = act_q8k_at(ap, al.off_d, al.off_aux, al.off_p);
       switch (w->dtype) {
         case CRABML_HIP_Q4_0:
-          k_gemv_exact_blk<CRABML_HIP_Q4_0, R><<<grid, 64 * WAVES, lds, dev->stream>>>((const i32x4*)wp, (const unsigned short*)(wp + w->wl.off_scale), a0, o, add, (int)m, (int)(k / 32));
+          STRICT_LAUNCH((k_gemv_exact_blk<CRABML_HIP_Q4_0, R>), (k_gemv_exact_blk<CRABML_HIP_Q4_0, R, true>), grid, 64 * WAVES, lds, (const i32x4*)wp, (const unsigned short*)(wp + w->wl.off_scale), a0, o, add, (int)m, (int)(k / 32));
           break;
         case CRABML_HIP_Q8_0:
-          k_gemv_exact_blk<CRABML_HIP_Q8_0, R><<<grid, 64 * WAVES, lds, dev->stream>>>((const i32x4*)wp, (const unsigned short*)(wp + w->wl.off_scale), a0, o, add, (int)m, (int)(k / 32));
+          STRICT_LAUNCH((k_gemv_exact_blk<CRABML_HIP_Q8_0, R>), (k_gemv_exact_blk<CRABML_HIP_Q8_0, R, true>), grid, 64 * WAVES, lds, (const i32x4*)wp, (const unsigned short*)(wp + w->wl.off_scale), a0, o, add, (int)m, (int)(k / 32));
           break;
         case CRABML_HIP_Q4_1:
-          k_gemv_exact_blk<CRABML_HIP_Q4_1, R><<<grid, 64 * WAVES, lds, dev->stream>>>((const i32x4*)wp, (const unsigned short*)(wp + w->wl.off_scale), a1, o, add, (int)m, (int)(k / 32));
+          STRICT_LAUNCH((k_gemv_exact_blk<CRABML_HIP_Q4_1, R>), (k_gemv_exact_blk<CRABML_HIP_Q4_1, R, true>), grid, 64 * WAVES, lds, (const i32x4*)wp, (const unsigned short*)(wp + w->wl.off_scale), a1, o, add, (int)m, (int)(k / 32));
           break;
         case CRABML_HIP_Q5_0:
-          k_gemv_exact_pieces<PieceQ5_0, R><<<grid, 64 * WAVES, lds, dev->stream>>>(wp, w->wl.off_scale, w->wl.n_blocks, a0, o, add, (int)m, (int)(k / 32));
+          STRICT_LAUNCH((k_gemv_exact_pieces<PieceQ5_0, R>), (k_gemv_exact_pieces<PieceQ5_0, R, true>), grid, 64 * WAVES, lds, wp, w->wl.off_scale, w->wl.n_blocks, a0, o, add, (int)m, (int)(k / 32));
           break;
         case CRABML_HIP_Q5_1:
-          k_gemv_exact_pieces<PieceQ5_1, R><<<grid, 64 * WAVES, lds, dev->stream>>>(wp, w->wl.off_scale, w->wl.n_blocks, a1, o, add, (int)m, (int)(k / 32));
+          STRICT_LAUNCH((k_gemv_exact_pieces<PieceQ5_1, R>), (k_gemv_exact_pieces<PieceQ5_1, R, true>), grid, 64 * WAVES, lds, wp, w->wl.off_scale, w->wl.n_blocks, a1, o, add, (int)m, (int)(k / 32));
           break;
         case CRABML_HIP_Q2_K:
-          k_gemv_exact_pieces<PieceQ2_K, R><<<grid, 64 * WAVES, lds, dev->stream>>>(wp, w->wl.off_scale, w->wl.n_blocks, ak, o, add, (int)m, (int)(k / 256));
+          STRICT_LAUNCH((k_gemv_exact_pieces<PieceQ2_K, R>), (k_gemv_exact_pieces<PieceQ2_K, R, true>), grid, 64 * WAVES, lds, wp, w->wl.off_scale, w->wl.n_blocks, ak, o, add, (int)m, (int)(k / 256));
           break;
         case CRABML_HIP_Q4_K:
         case CRABML_HIP_Q5_K: {
@@ -748,9 +773,9 @@ int launch_gemv_strict(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m
           if (lk > 48 * 1024) {
             done = false;
           } else if (w->dtype == CRABML_HIP_Q4_K) {
-            k_gemv_exact_q4k<false, R><<<grid, 64 * WAVES, lk, dev->stream>>>(wp, w->wl.off_scale, ak, o, add, (int)m, (int)(k / 256));
+            STRICT_LAUNCH((k_gemv_exact_q4k<false, R>), (k_gemv_exact_q4k<false, R, true>), grid, 64 * WAVES, lk, wp, w->wl.off_scale, ak, o, add, (int)m, (int)(k / 256));
           } else {
-            k_gemv_exact_q4k<true, R><<<grid, 64 * WAVES, lk, dev->stream>>>(wp, w->wl.off_scale, ak, o, add, (int)m, (int)(k / 256));
+            STRICT_LAUNCH((k_gemv_exact_q4k<true, R>), (k_gemv_exact_q4k<true, R, true>), grid, 64 * WAVES, lk, wp, w->wl.off_scale, ak, o, add, (int)m, (int)(k / 256));
           }
           break;
         }
@@ -759,7 +784,7 @@ int launch_gemv_strict(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m
           if (lk > 48 * 1024)
             done = false;
           else
-            k_gemv_exact_q6k<R><<<grid, 64 * WAVES, lk, dev->stream>>>(wp, w->wl.off_scale, ak, o, add, (int)m, (int)(k / 256));
+            STRICT_LAUNCH((k_gemv_exact_q6k<R>), (k_gemv_exact_q6k<R, true>), grid, 64 * WAVES, lk, wp, w->wl.off_scale, ak, o, add, (int)m, (int)(k / 256));
           break;
         }
         case CRABML_HIP_Q3_K: {
@@ -767,17 +792,17 @@ int launch_gemv_strict(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m
           if (lk > 48 * 1024)
             done = false;
           else
-            k_gemv_exact_q3k<R><<<grid, 64 * WAVES, lk, dev->stream>>>(wp, w->wl.off_scale, w->wl.n_blocks, ak, o, add, (int)m, (int)(k / 256));
+            STRICT_LAUNCH((k_gemv_exact_q3k<R>), (k_gemv_exact_q3k<R, true>), grid, 64 * WAVES, lk, wp, w->wl.off_scale, w->wl.n_blocks, ak, o, add, (int)m, (int)(k / 256));
           break;
         }
         case CRABML_HIP_Q8_K:
-          k_gemv_exact_q8k<R><<<grid, 64 * WAVES, lds, dev->stream>>>((const i32x4*)wp, (const float*)(wp + w->wl.off_scale), ak, o, add, (int)m, (int)(k / 256));
+          STRICT_LAUNCH((k_gemv_exact_q8k<R>), (k_gemv_exact_q8k<R, true>), grid, 64 * WAVES, lds, (const i32x4*)wp, (const float*)(wp + w->wl.off_scale), ak, o, add, (int)m, (int)(k / 256));
           break;
         default: done = false;
       }
     }
     if (!done)
-      k_gemv_strict<<<(unsigned)((m + 63) / 64), 64, 0, dev->stream>>>(wp, (int)w->dtype, w->wl.off_scale, ap, al.off_d, al.off_aux, o, add, (int)m, (int)k);
+      STRICT_LAUNCH((k_gemv_strict<>), (k_gemv_strict<true>), (unsigned)((m + 63) / 64), 64, 0, wp, (int)w->dtype, w->wl.off_scale, ap, al.off_d, al.off_aux, o, add, (int)m, (int)k);
   }
   return 0;
 }

@@ -1,0 +1,30 @@
+"""matmul_vec on several rows of the rhs in one launch of the row kernels: bit for bit what a call per row gives, for every format, on both
+devices.  (From 16 rows on the fast device has matrix-core kernels for some formats: those counts are left to the formats without one.)"""
+import numpy as np
+import pytest
+
+from crabml_amd import synth
+from tests.test_hip_gemv import HT
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("fmt", ["Q4_0", "Q8_0", "Q4_1", "Q5_0", "Q5_1", "Q2_K", "Q3_K", "Q4_K", "Q5_K", "Q6_K", "Q8_K", "F32", "F16"])
+@pytest.mark.parametrize("strict", [False, True])
+# rows of the matrix: less than a tile, tiles that do not divide by the eight XCDs, two rows a wave; rows of the rhs: past one launch's share
+@pytest.mark.parametrize("m,k,rows", [(1, 256, 2), (77, 768, 15), (8210, 512, 5), (9, 256, 259)])
+def test_rows_equal_single_calls(ca, fmt, strict, m, k, rows):
+    if rows > 15 and not strict and fmt in ("Q4_0", "Q8_0", "Q4_1", "Q4_K", "Q6_K", "Q8_K"):
+        rows = 15
+    if fmt == "F16":
+        k += 0 if strict else 2  # (fast: rows of whole 16-byte pieces take the matrix cores)
+    rng = np.random.default_rng(m + rows)
+    typ = synth.TYPE_BY_NAME[fmt]
+    dev = ca.HipTensorDevice(0, False, 0, strict)
+    w = ca.HipTensor.from_cpu(synth.random_blocks(rng, m * k, typ), [m, k], getattr(ca.GGMLType, HT[fmt]), dev)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    got = w.matmul_vec(ca.HipTensor.new(x.reshape(-1), [rows, k], dev)).export().reshape(rows, m)
+    picks = sorted({0, 1, rows // 2, rows - 1})
+    for r in picks:
+        one = w.matmul_vec(ca.HipTensor.new(x[r], [k], dev)).export()
+        assert np.array_equal(got[r].view(np.uint32), one.view(np.uint32)), r
