@@ -155,13 +155,13 @@ struct crabml_hip_llama {
   int vocab_l = 0, vocab_off = 0;
   int* am_best = nullptr;   // {max bits, index} of this rank's shard (single-device simulation: combined by the driver)
   size_t kv_len = 0;
-  // [0]: one attention workgroup per head; [1]: the long-context attention kernels (from attn_long_from positions)
-  hipGraph_t graph[3] = {nullptr, nullptr, nullptr};
-  hipGraphExec_t exec[3] = {nullptr, nullptr, nullptr};
+  // by attn_variant
+  hipGraph_t graph[4] = {nullptr, nullptr, nullptr, nullptr};
+  hipGraphExec_t exec[4] = {nullptr, nullptr, nullptr, nullptr};
   bool use_graph = false;
   bool capturing = false;
   int attn_variant = 0;         // which of them the next enqueue emits: 0 = one workgroup per head, 1 = the long-context kernels,
-                                // 2 = split-KV attention with the merge inside the launch (ticket form: the mid range)
+                                // 2 = split-KV attention with the merge inside the launch (ticket form: the mid range), 3 = k_attn_short
   size_t flash_ticket_until = 0;  // > 0: positions [attn_long_from, this) run variant 2
   bool attn_long_ok = false;    // f16 cache, head_dim % 32 == 0, group size in {1, 2, 4, 8}; and seq_len % 8 == 0 (exact kernels) or k_attn_flash
   bool exact_long_ok = false;   // the exact long-context kernels (score / probability rows of seq_len elements read as 16-byte vectors)
@@ -176,6 +176,8 @@ struct crabml_hip_llama {
   float* flash_part = nullptr;  // [n_kv_l][flash_S][G][hd + 2] partial {O, m, l}
   unsigned* flash_tick = nullptr;  // [n_kv_l] arrival counters (monotonic)
   int gu_rows = 0;              // > 0 (tensor-parallel ranks): gate/up leaves h as f32 from workgroups of this many rows, ffn_down quantizes it
+  // cached positions (pos + 1) [from, until) run k_attn_short: as variant 0 where from = 0, else as variant 3
+  size_t attn_short_from = SIZE_MAX, attn_short_until = SIZE_MAX;
   int attn_s_rows = 0;          // > 0: variant 0 runs k_attn_s (K / V staged through LDS) with room for this many cached rows
   size_t attn_s_lds = 0;
   float* scores_g = nullptr;    // [n_heads_l][seq_len] f32
@@ -318,6 +320,7 @@ FlashFn flash_kernel(int grp, int hd, bool q81, bool ticket) {
 }
 // which attention form serves cache position `pos` (see attn_variant)
 int variant_of(const crabml_hip_llama* c, size_t pos) {
+  if (pos + 1 >= c->attn_short_from && pos + 1 < c->attn_short_until) return c->attn_short_from == 0 ? 0 : 3;
   if (!(c->attn_long_ok && pos + 1 >= c->attn_long_from)) return 0;
   return c->flash_ticket_until > 0 && pos + 1 < c->flash_ticket_until ? 2 : 1;
 }
@@ -355,6 +358,15 @@ void enqueue_attention(crabml_hip_llama* c, int l, signed char* xq, unsigned sho
   hipStream_t st = dev->stream;
   const int hd = c->hd, seq_cap = (int)c->cfg.seq_len, n_heads = c->n_heads_l, n_kv = c->n_kv_l;
   const int* pos_d = c->state + 1;
+  crabml_hip_device::ProfRec ar{};
+  crabml_hip_device::ProfRec* AR = prof ? &ar : nullptr;
+  if (c->attn_variant == 3 || (c->attn_variant == 0 && c->attn_short_from == 0)) {
+    if (prof) prof_begin(dev, &ar, CRABML_HIP_F32, 7, 0.0);
+    launch_k(st, AR, attn_short_kernel(hd), dim3(n_heads + spare), dim3(512), 0, (const float*)c->qbuf, (const unsigned short*)c->kc[l], (const unsigned short*)c->vc[l],
+             pos_d, c->attn, xq, xd, xisum, n_heads, n_kv, hd, seq_cap, pf, c->qt == CRABML_HIP_Q8_1 ? 1 : 0);
+    if (prof) prof_end(dev, &ar);
+    return;
+  }
   if (c->attn_variant >= 1 && c->attn_flash) {
     launch_attn_flash(c, l, xq, xd, xisum, prof);
     return;
@@ -370,8 +382,6 @@ void enqueue_attention(crabml_hip_llama* c, int l, signed char* xq, unsigned sho
   }
   const size_t attn_lds = (size_t)(seq_cap + hd) * sizeof(float);
   const int sbit = dev->strict_order ? 256 : 0;  // strict device: sequential softmax row sums at any length (softmax.rs:43-48)
-  crabml_hip_device::ProfRec ar{};
-  crabml_hip_device::ProfRec* AR = prof ? &ar : nullptr;
   if (prof) prof_begin(dev, &ar, CRABML_HIP_F32, 7, 0.0);
   if (c->attn_s_rows > 0 && hd == 128)
     launch_k(st, AR, k_attn_s<128>, dim3(n_heads + spare), dim3(256), c->attn_s_lds, (const float*)c->qbuf, (const unsigned short*)c->kc[l],
@@ -2186,7 +2196,18 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
       }
       (void)hipGetLastError();
     }
-    // short-context attention with K / V staged through LDS (f16 cache): variant 0 serves positions < S
+    // A head per workgroup with f32 sums (k_attn_short): from the start on the fast step of Q4_0 / Q8_0 layers, whose RMS norms leave the
+    // reference's summation order as well; elsewhere where k_attn_flash would leave it.  Us per layer of the 8B shape, k_attn_short against
+    // what ran before: 4.7 against 6.5 at 40 cached positions, 5.4 against 8.8 at 88.  Against k_attn_flash, a step and layer: 33.1 / 35.6 at
+    // 128, 34.1 / 36.0 at 256, 35.4 / 36.3 at 384, 36.4 / 36.3 at 512, 38.3 / 36.9 at 768 (16 / 4 heads x 128: even at 600; 32 / 32 x 64:
+    // at 1000) -- one workgroup reads a head's rows at a CU's rate.  A caller's own attn_long_from is the long kernels' from there on.
+    if (g.use_f16_kv_cache && hd % 8 == 0 && hd <= 256 && !dev->strict_order &&
+        !(g.flags & (CRABML_HIP_LLAMA_EXACT_ATTENTION | CRABML_HIP_LLAMA_NO_LONG_ATTENTION | CRABML_HIP_LLAMA_NO_STAGED_ATTENTION))) {
+      const bool flash = c->attn_flash && g.attn_long_from == 0;
+      c->attn_short_from = wt == CRABML_HIP_Q4_0 || wt == CRABML_HIP_Q8_0 ? 0 : flash ? c->attn_long_from : SIZE_MAX;
+      c->attn_short_until = flash ? 512 : c->attn_long_ok ? c->attn_long_from : SIZE_MAX;
+    }
+    // everything else: K / V staged through LDS, the reference's bits; variant 0 serves positions < S
     if (g.use_f16_kv_cache && hd % 8 == 0 && !(g.flags & CRABML_HIP_LLAMA_NO_STAGED_ATTENTION)) {
       const size_t S = c->attn_long_ok && c->attn_long_from < g.seq_len ? c->attn_long_from : g.seq_len;
       const size_t lds = attn_s_lds_bytes((int)S, (int)hd);
@@ -2277,9 +2298,11 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
   const bool want_graph = !(g.flags & CRABML_HIP_LLAMA_NO_GRAPH) &&
                           (tp == 1 || c->tp_dry || p2p_comm || (c->comm != nullptr && (g.flags & CRABML_HIP_LLAMA_TP_GRAPH)));
   if (want_graph) {
-    const int nvar = c->attn_long_ok ? (c->flash_ticket_until > 0 ? 3 : 2) : 1;
+    const bool has[4] = {true, c->attn_long_ok, c->attn_long_ok && c->flash_ticket_until > 0,
+                         c->attn_short_from > 0 && c->attn_short_from < g.seq_len};
     bool ok = true;
-    for (int v = 0; v < nvar && ok; v++) {
+    for (int v = 0; v < 4 && ok; v++) {
+      if (!has[v]) continue;
       ok = false;
       hipError_t e = hipStreamBeginCapture(dev->stream, hipStreamCaptureModeThreadLocal);
       if (e != hipSuccess) break;
@@ -2333,7 +2356,7 @@ int crabml_hip_llama_destroy(crabml_hip_llama_t* c) {
     (void)hipSetDevice(c->dev->ordinal);
     (void)hipStreamSynchronize(c->dev->stream);
   }
-  for (int v = 0; v < 3; v++) {
+  for (int v = 0; v < 4; v++) {
     if (c->exec[v]) (void)hipGraphExecDestroy(c->exec[v]);
     if (c->graph[v]) (void)hipGraphDestroy(c->graph[v]);
   }
@@ -2509,6 +2532,38 @@ int crabml_hip_llama_debug_kv(crabml_hip_llama_t* c, size_t layer, int32_t which
 }
 
 // parity hook (crabml_hip_debug.h): k_attn_flash by itself, on caller-supplied q / K / V
+int crabml_hip_debug_short_attention(crabml_hip_device_t* dev, const float* q, const uint16_t* k, const uint16_t* v, size_t n_heads,
+                                     size_t n_kv, size_t head_dim, size_t seq, size_t seq_cap, float* out) {
+  if (!dev || !q || !k || !v || !out || seq == 0 || seq > seq_cap || seq_cap > (1u << 24) || n_kv == 0 || n_heads == 0 || n_heads % n_kv != 0 || n_heads > 4096 ||
+      head_dim == 0 || head_dim % 8 != 0 || head_dim > 256)
+    return CRABML_HIP_BAD_INPUT;
+  CH_LIVE(dev);
+  CH_USE(dev);
+  CH_FLUSH(dev);
+  const size_t nq = n_heads * head_dim * 4, nkv = n_kv * seq_cap * head_dim * 2;
+  const size_t o_k = align_up(nq, 256), o_v = align_up(o_k + nkv, 256), o_out = align_up(o_v + nkv, 256), o_pos = align_up(o_out + nq, 256);
+  char* base = nullptr;
+  CH_HIP(dev, hipMalloc((void**)&base, o_pos + 256));
+  hipStream_t st = dev->stream;
+  const int pos = (int)seq - 1;
+  hipError_t e = hipMemcpyAsync(base, q, nq, hipMemcpyHostToDevice, st);
+  if (e == hipSuccess) e = hipMemcpyAsync(base + o_k, k, nkv, hipMemcpyHostToDevice, st);
+  if (e == hipSuccess) e = hipMemcpyAsync(base + o_v, v, nkv, hipMemcpyHostToDevice, st);
+  if (e == hipSuccess) e = hipMemcpyAsync(base + o_pos, &pos, 4, hipMemcpyHostToDevice, st);
+  if (e == hipSuccess) e = hipStreamSynchronize(st);  // (`pos` leaves scope)
+  if (e == hipSuccess) {
+    launch_k(st, nullptr, attn_short_kernel((int)head_dim), dim3((unsigned)n_heads), dim3(512), 0, (const float*)base, (const unsigned short*)(base + o_k),
+             (const unsigned short*)(base + o_v), (const int*)(base + o_pos), (float*)(base + o_out), (signed char*)nullptr,
+             (unsigned short*)nullptr, (void*)nullptr, (int)n_heads, (int)n_kv, (int)head_dim, (int)seq_cap, PrefetchPlan{}, 0);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipMemcpyAsync(out, base + o_out, nq, hipMemcpyDeviceToHost, st);
+  const hipError_t e2 = hipStreamSynchronize(st);
+  (void)hipFree(base);
+  CH_HIP(dev, e != hipSuccess ? e : e2);
+  return 0;
+}
+
 int crabml_hip_debug_flash_attention(crabml_hip_device_t* dev, const float* q, const uint16_t* k, const uint16_t* v, size_t n_heads,
                                      size_t n_kv, size_t head_dim, size_t seq, size_t slices, float* out, float* out2) {
   if (!dev || !q || !k || !v || !out || seq == 0 || n_kv == 0 || n_heads % n_kv != 0) return CRABML_HIP_BAD_INPUT;

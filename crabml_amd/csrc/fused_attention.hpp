@@ -2,6 +2,9 @@
 // Part of the fused decode step (fused.hip includes the three fused_*.hpp files once, in order; they are not stand-alone
 // translation units: the kernels are launched from fused.hip's host code).
 #pragma once
+#include <cfloat>
+#include <type_traits>
+
 #include "fused_common.hpp"
 
 namespace crabml_hip {
@@ -183,6 +186,35 @@ __global__ __launch_bounds__(256) void k_attn(const float* __restrict__ q, const
     }
   }
   stamp(5);
+}
+
+// quantize the head's output for wo: a 32-element block = the 16 lanes of one DPP row, two columns each (whole waves: hd % 32 == 0, so a
+// row of 16 lanes is all live or all dead); e: the lane's first element
+__device__ __forceinline__ void quantize_pair(bool live, int e, float v0, float v1, int q81, signed char* __restrict__ xq,
+                                              unsigned short* __restrict__ xd, void* __restrict__ xisum) {
+  const float a0 = live ? v0 : 0.f, a1 = live ? v1 : 0.f;
+  const float amax = row16_max_f32(fmaxf(fabsf(a0), fabsf(a1)));
+  const float dd = amax / 127.0f;
+  int q0, q1, aux;
+  if (!q81) {  // buf_q8_0.rs:87-134: q = trunc(x / d) (`as i8` of the i32 wraps), aux = the block's quant sum
+    q0 = (int)(signed char)(unsigned char)((unsigned)rs_f32_as_i32(a0 / dd) & 0xffu);
+    q1 = (int)(signed char)(unsigned char)((unsigned)rs_f32_as_i32(a1 / dd) & 0xffu);
+    aux = row16_sum_i32(live ? q0 + q1 : 0);
+  } else {  // buf_q8_1.rs:90-129: clamp, NaN -> -128, s = f16(d * sum q)
+    q0 = (int)fminf(fmaxf(a0 / dd, -128.0f), 127.0f);
+    q1 = (int)fminf(fmaxf(a1 / dd, -128.0f), 127.0f);
+    const int sum = row16_sum_i32(live ? q0 + q1 : 0);
+    aux = (int)f2h((float)sum * dd);
+  }
+  if (!live) return;
+  *(unsigned short*)(xq + e) = (unsigned short)(((unsigned)q0 & 0xffu) | (((unsigned)q1 & 0xffu) << 8));
+  if ((threadIdx.x & 15) == 0) {
+    xd[e >> 5] = f2h(dd);
+    if (q81)
+      store_qaux<true>(xisum, e >> 5, aux);
+    else
+      store_qaux<false>(xisum, e >> 5, aux);
+  }
 }
 
 // ---- attention at short context with K / V staged through LDS ---------------------------------------------------------
@@ -405,39 +437,169 @@ __global__ __launch_bounds__(256) void k_attn_s(const float* __restrict__ q, con
     __syncthreads();
     if (wave == 0) q8k_exchange_store(k8.ex, qs, head * hd, hd, lane, xq, k8.d, k8.bs, k8.qp);
   } else if (xq != nullptr && wave * 64 < npair) {
-  // ---- quantize the head's output for wo: a 32-element block = the 16 lanes of one DPP row (two columns each)  // whole waves (hd % 32 == 0 here: rows of 16 lanes are all-live or all-dead)
-    const bool live = tid < npair;
-    const float a0 = live ? v0 : 0.f, a1 = live ? v1 : 0.f;
-    const float amax = row16_max_f32(fmaxf(fabsf(a0), fabsf(a1)));
-    const float dd = amax / 127.0f;
-    int q0, q1, aux;
-    if (!q81) {  // buf_q8_0.rs:87-134: q = trunc(x / d) (`as i8` of the i32 wraps), aux = the block's quant sum
-      q0 = (int)(signed char)(unsigned char)((unsigned)rs_f32_as_i32(a0 / dd) & 0xffu);
-      q1 = (int)(signed char)(unsigned char)((unsigned)rs_f32_as_i32(a1 / dd) & 0xffu);
-      aux = row16_sum_i32(live ? q0 + q1 : 0);
-    } else {  // buf_q8_1.rs:90-129: clamp, NaN -> -128, s = f16(d * sum q)
-      q0 = (int)fminf(fmaxf(a0 / dd, -128.0f), 127.0f);
-      q1 = (int)fminf(fmaxf(a1 / dd, -128.0f), 127.0f);
-      const int sum = row16_sum_i32(live ? q0 + q1 : 0);
-      aux = (int)f2h((float)sum * dd);
-    }
-    if (live) {
-      const int e = head * hd + 2 * tid;
-      *(unsigned short*)(xq + e) = (unsigned short)(((unsigned)q0 & 0xffu) | (((unsigned)q1 & 0xffu) << 8));
-      if ((tid & 15) == 0) {
-        xd[e >> 5] = f2h(dd);
-        if (q81)
-          store_qaux<true>(xisum, e >> 5, aux);
-        else
-          store_qaux<false>(xisum, e >> 5, aux);
-      }
-    }
+    quantize_pair(tid < npair, head * hd + 2 * tid, v0, v1, q81, xq, xd, xisum);
   }
   stamp(5);
 }
 __host__ __device__ inline size_t attn_s_lds_bytes(int S, int hd) {
   return (size_t)(((S + 3) & ~3) + hd) * sizeof(float) + (size_t)S * (hd + 8) * 2 + (size_t)S * hd * 2;
 }
+
+// ---- fast-mode attention at short context: a head per workgroup, the cached rows over its eight waves ---------------------------
+// k_attn_s is a chain: 128 dependent products per score, a softmax on one wave, an f16 sum over the positions one after the other.  Here a
+// row is LPR lanes x 16 bytes and a wave instruction takes 64 / LPR rows, straight from the cache into registers: every lane multiplies its
+// eight elements, the LPR lanes of a row add up, and the wave sums p * v over its rows with the weights e^(s - its own maximum); the lanes
+// of one column meet through swaps of half waves and rows, the eight waves once, in LDS.  The arithmetic is k_attn_flash's (q rounded to
+// f16; exact products, f32 exp, weights and sums): closer to exact than the f16 chain, not its bits -- so for the layers whose fast step
+// already leaves the reference's bits (Q4_0 / Q8_0, attn_short in fused.hip), everything else keeps k_attn_s.
+// The first 64 rows are requested before the position is known (rows past it are cache memory: read, never used).
+// hd: a multiple of 8, at most 8 LPR (lanes past it hold zeros).
+template <int LPR>
+__global__ __launch_bounds__(512) void k_attn_short(const float* __restrict__ q, const unsigned short* __restrict__ kc,
+                                                    const unsigned short* __restrict__ vc, const int* __restrict__ pos_d, float* __restrict__ out,
+                                                    signed char* __restrict__ xq, unsigned short* __restrict__ xd, void* __restrict__ xisum,
+                                                    int n_heads, int n_kv, int hd, int seq_cap, PrefetchPlan pf, int q81) {
+  if ((int)blockIdx.x >= n_heads) {
+    prefetch_wg(pf, blockIdx.x - n_heads, gridDim.x - n_heads);
+    return;
+  }
+  constexpr int NW = 8, RPI = 64 / LPR, RR = NW * RPI;        // rows of a wave's request / of one from every wave
+  constexpr int U0 = 64 / RR > 0 ? 64 / RR : 1, U1 = 128 / RR;  // requests: before the position is known / of a round after that
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  __shared__ f32x2 s_acc[NW][LPR * 4];
+  __shared__ float s_m[NW], s_l[NW];
+  const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_wg();
+  const int rc = lane / LPR, dl = lane % LPR, head = blockIdx.x, kvh = head / (n_heads / n_kv);
+  const bool col = dl * 8 < hd;
+  const int c0 = col ? dl * 8 : 0;
+  const unsigned short *kb = kc + (size_t)kvh * seq_cap * hd + c0, *vb = vc + (size_t)kvh * seq_cap * hd + c0;
+  const f32x4 qa = *(const f32x4*)(q + head * hd + c0), qb = *(const f32x4*)(q + head * hd + c0 + 4);
+  i32x4 k0[U0], v0[U0];
+#pragma unroll
+  for (int u = 0; u < U0; u++) {
+    const int row = u * RR + wave * RPI + rc, rowc = row < seq_cap ? row : seq_cap - 1;
+    k0[u] = *(const i32x4*)(kb + (size_t)rowc * hd);
+    v0[u] = *(const i32x4*)(vb + (size_t)rowc * hd);
+  }
+  int seq = *pos_d + 1;
+  seq = seq < seq_cap ? seq : seq_cap;
+  float qf[8];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {  // rounded to f16 (batch_matmul.rs:39)
+    qf[i] = col ? h2f(f2h(qa[i])) : 0.f;
+    qf[i + 4] = col ? h2f(f2h(qb[i])) : 0.f;
+  }
+  float m = -FLT_MAX, l = 0.f, acc[8];  // m: the same in all lanes of the wave (a row of -inf scores has weight 0)
+#pragma unroll
+  for (int i = 0; i < 8; i++) acc[i] = 0.f;
+  auto take = [&](const auto& kk, const auto& vv, auto n, int row0) {  // the wave's rows row0 + u RR + rc
+    constexpr int U = decltype(n)::value;
+    float s[U], mc = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      float d = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const h2 k = __builtin_bit_cast(h2, col ? (unsigned)kk[u][i] : 0u);
+        d = __builtin_fmaf(qf[2 * i], (float)k[0], d);
+        d = __builtin_fmaf(qf[2 * i + 1], (float)k[1], d);
+      }
+      d += dpp_f<0xB1>(d);
+      d += dpp_f<0x4E>(d);
+      d += dpp_f<0x141>(d);
+      if constexpr (LPR >= 16) d += dpp_f<0x140>(d);
+      if constexpr (LPR == 32) d += __shfl_xor(d, 16, 64);
+      s[u] = row0 + u * RR + rc < seq ? d : -INFINITY;
+      mc = fmaxf(mc, s[u]);
+    }
+    const float mn = fmaxf(m, wave_max_f32(mc)), alpha = __expf(m - mn);
+    m = mn;
+    l *= alpha;
+#pragma unroll
+    for (int i = 0; i < 8; i++) acc[i] *= alpha;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const bool live = row0 + u * RR + rc < seq;
+      const float p = __expf(s[u] - mn);
+      l += p;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const h2 v = __builtin_bit_cast(h2, live ? (unsigned)vv[u][i] : 0u);
+        acc[2 * i] = __builtin_fmaf(p, (float)v[0], acc[2 * i]);
+        acc[2 * i + 1] = __builtin_fmaf(p, (float)v[1], acc[2 * i + 1]);
+      }
+    }
+  };
+  const int first = wave * RPI;
+  if (first < seq) take(k0, v0, std::integral_constant<int, U0>{}, first);
+#pragma unroll 1
+  for (int r0 = U0 * RR + first; r0 < seq; r0 += U1 * RR) {
+    i32x4 k1[U1], v1[U1];
+#pragma unroll
+    for (int u = 0; u < U1; u++) {
+      const int row = r0 + u * RR + rc, rowc = row < seq ? row : seq - 1;
+      k1[u] = *(const i32x4*)(kb + (size_t)rowc * hd);
+      v1[u] = *(const i32x4*)(vb + (size_t)rowc * hd);
+    }
+    take(k1, v1, std::integral_constant<int, U1>{}, r0);
+  }
+  // ---- the wave's row classes: lanes < 32 end up with the sums of elements 0-3, the others of 4-7, and (LPR < 32) odd rows of 16 lanes
+  // with the upper two of those
+  auto meet32 = [](float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+    const unsigned lo = r[0], hi = r[1];
+    return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+  };
+  auto meet16 = [](float a, float b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+    const unsigned lo = r[0], hi = r[1];
+    return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+  };
+#pragma unroll
+  for (int i = 0; i < 4; i++) acc[i] = meet32(acc[i], acc[i + 4]);
+  l = meet32(l, l);
+  if constexpr (LPR == 32) {
+    s_acc[wave][dl * 4 + (lane >> 5) * 2] = f32x2{acc[0], acc[1]};
+    s_acc[wave][dl * 4 + (lane >> 5) * 2 + 1] = f32x2{acc[2], acc[3]};
+  } else {
+    acc[0] = meet16(acc[0], acc[2]);
+    acc[1] = meet16(acc[1], acc[3]);
+    l = meet16(l, l);
+    if constexpr (LPR == 8) {  // two rows' lanes in 16
+      acc[0] += dpp_f<0x128>(acc[0]);
+      acc[1] += dpp_f<0x128>(acc[1]);
+      l += dpp_f<0x128>(l);
+    }
+    if (LPR == 16 || (lane & 8) == 0) s_acc[wave][dl * 4 + (lane >> 5) * 2 + ((lane >> 4) & 1)] = f32x2{acc[0], acc[1]};
+  }
+  if (lane == 0) {
+    s_m[wave] = first < seq ? m : -INFINITY;
+    s_l[wave] = l;
+  }
+  __syncthreads();
+  const int npair = hd >> 1;
+  if (wave * 64 >= npair) return;
+  float M = s_m[0], L = 0.f;
+#pragma unroll
+  for (int w = 1; w < NW; w++) M = fmaxf(M, s_m[w]);
+  const int pair = tid < npair ? tid : npair - 1;
+  f32x2 o = {0.f, 0.f};
+#pragma unroll
+  for (int w = 0; w < NW; w++) {
+    const float e = __expf(s_m[w] - M);
+    const f32x2 a = s_acc[w][pair];
+    L = __builtin_fmaf(s_l[w], e, L);
+    o[0] = __builtin_fmaf(a[0], e, o[0]);
+    o[1] = __builtin_fmaf(a[1], e, o[1]);
+  }
+  o[0] /= L;
+  o[1] /= L;
+  const int e = head * hd + 2 * tid;
+  if (tid < npair) *(f32x2*)(out + e) = o;
+  if (xq != nullptr) quantize_pair(tid < npair, e, o[0], o[1], q81, xq, xd, xisum);
+}
+
+inline auto attn_short_kernel(int hd) { return hd <= 64 ? k_attn_short<8> : hd <= 128 ? k_attn_short<16> : k_attn_short<32>; }
 
 // ---- attention at long context: the same arithmetic over every CU ----------------------------------------------
 // One workgroup per head streams its whole K and V through one CU (~26 GB/s): 223 us per layer at 4000 cached

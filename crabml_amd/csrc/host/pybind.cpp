@@ -122,6 +122,18 @@ PYBIND11_MODULE(_host, m) {
                                                       out.mutable_data(), out2.mutable_data()));
              return py::make_tuple(out, out2);
            })
+      .def("debug_short_attention",
+           [](HipTensorDevice& d, py::array_t<float, py::array::c_style | py::array::forcecast> q,
+              py::array_t<uint16_t, py::array::c_style | py::array::forcecast> k,
+              py::array_t<uint16_t, py::array::c_style | py::array::forcecast> v, size_t n_heads, size_t n_kv, size_t head_dim,
+              size_t seq, size_t seq_cap) {
+             if ((size_t)q.size() != n_heads * head_dim || (size_t)k.size() != n_kv * seq_cap * head_dim || k.size() != v.size())
+               throw Error(ErrorKind::BadInput, "debug_short_attention: array sizes");
+             py::array_t<float> out(n_heads * head_dim);
+             d.check(crabml_hip_debug_short_attention(d.raw(), q.data(), k.data(), v.data(), n_heads, n_kv, head_dim, seq, seq_cap,
+                                                      out.mutable_data()));
+             return out;
+           })
       .def("debug_flash_attention_rows",
            [](HipTensorDevice& d, py::array_t<float, py::array::c_style | py::array::forcecast> q,
               py::array_t<uint16_t, py::array::c_style | py::array::forcecast> k,

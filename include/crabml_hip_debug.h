@@ -69,6 +69,11 @@ int crabml_hip_debug_read_ceiling(crabml_hip_device_t* dev, size_t bytes, int32_
 int crabml_hip_debug_flash_attention(crabml_hip_device_t* dev, const float* q, const uint16_t* k, const uint16_t* v, size_t n_heads,
                                      size_t n_kv, size_t head_dim, size_t seq, size_t slices, float* out, float* out2);
 
+/* The fast step's short-context attention (k_attn_short) by itself: as above, head_dim a multiple of 8 up to 256, one workgroup per head;
+ * k, v: [n_kv][seq_cap][head_dim], of which the first `seq` rows count. */
+int crabml_hip_debug_short_attention(crabml_hip_device_t* dev, const float* q, const uint16_t* k, const uint16_t* v, size_t n_heads,
+                                     size_t n_kv, size_t head_dim, size_t seq, size_t seq_cap, float* out);
+
 /* The fast prompt pass's causal attention (k_attn_flash_rows: flash attention on the f16 matrix cores) by itself.  q: rows *
  * n_heads * head_dim f32 (row r is the prompt row at position pos0 + r); k, v: [n_kv][seq_cap][head_dim] f16 bits (the cache
  * after the pass's appends: positions 0 .. pos0 + rows - 1 are live, whatever lies beyond must not matter); out: rows * n_heads *

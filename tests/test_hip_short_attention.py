@@ -1,0 +1,82 @@
+"""k_attn_short -- the fast decode step's attention at short contexts (a head per workgroup, f32 sums) -- against float64 arithmetic on the
+same f16 inputs, and the step that uses it against the exact chain."""
+import numpy as np
+import pytest
+
+from crabml_amd import synth
+
+pytestmark = pytest.mark.gpu
+EXACT = 4194304  # CRABML_HIP_LLAMA_EXACT_ATTENTION
+
+
+def attend(dev, q, k, v, n_heads, n_kv, hd, seq, cap):
+    """the kernel on a cache whose rows past `seq` are NaN; float64 on the rows that count"""
+    kc, vc = (np.full((n_kv, cap, hd), np.nan, np.float16) for _ in range(2))
+    kc[:, :seq], vc[:, :seq] = k, v
+    got = dev.debug_short_attention(q, kc.view(np.uint16).reshape(-1), vc.view(np.uint16).reshape(-1), n_heads, n_kv, hd, seq, cap)
+    q16 = q.astype(np.float16).astype(np.float64).reshape(n_heads, hd)
+    ref = np.zeros((n_heads, hd))
+    with np.errstate(invalid="ignore", over="ignore"):
+        for h in range(n_heads):
+            s = k[h // (n_heads // n_kv)].astype(np.float64) @ q16[h]
+            p = np.exp(s - s.max())
+            ref[h] = (p / p.sum()) @ v[h // (n_heads // n_kv)].astype(np.float64)
+    return got.reshape(n_heads, hd), ref
+
+
+# a row of 8 / 16 / 32 lanes, full and with dead lanes; positions at the edges of a wave's request, of the speculative 64 and of a round
+@pytest.mark.parametrize("n_heads,n_kv,hd", [(6, 6, 8), (4, 2, 40), (6, 6, 48), (8, 1, 64), (6, 2, 96), (32, 8, 128), (4, 4, 136), (4, 1, 256)])
+@pytest.mark.parametrize("spread", [1.0, 8.0])
+def test_against_float64(ca, n_heads, n_kv, hd, spread):
+    dev = ca.HipTensorDevice(0)
+    rng = np.random.default_rng(hd)
+    for seq in (1, 2, 3, 4, 5, 7, 8, 9, 15, 16, 17, 31, 33, 63, 64, 65, 127, 128, 129, 191, 192, 193, 511, 700):
+        for cap in (seq, seq + 200):
+            q = (rng.standard_normal(n_heads * hd) * spread / np.sqrt(hd)).astype(np.float32)
+            k, v = (rng.standard_normal((n_kv, seq, hd)).astype(np.float16) for _ in range(2))
+            got, ref = attend(dev, q, k, v, n_heads, n_kv, hd, seq, cap)
+            # exp's argument carries the score's f32 error, hd roundings of |score| <= 32: 2e-5 of the largest output, as for the long kernels
+            assert np.max(np.abs(got - ref)) <= 2e-5 * np.max(np.abs(ref)), (seq, cap)
+
+
+@pytest.mark.parametrize("hd", [48, 128])
+def test_infinities_and_nan(ca, hd):
+    """a score of -inf has weight zero wherever it lies, +inf and NaN scores make the head NaN, an infinite v stays in its column"""
+    dev = ca.HipTensorDevice(0)
+    rng = np.random.default_rng(5)
+    for seq, at in ((3, 0), (40, 33), (130, 129), (300, 64)):
+        q = np.abs(rng.standard_normal(hd)).astype(np.float32)
+        k, v = (rng.standard_normal((1, seq, hd)).astype(np.float16) for _ in range(2))
+        k[0, at, 3] = -np.inf
+        got, ref = attend(dev, q, k, v, 1, 1, hd, seq, seq + 8)
+        assert np.max(np.abs(got - ref)) <= 2e-5 * np.max(np.abs(ref)), seq
+        v[0, at ^ 1, 5] = np.inf
+        got, ref = attend(dev, q, k, v, 1, 1, hd, seq, seq + 8)
+        assert np.isposinf(got[0, 5]) and np.isfinite(np.delete(got[0], 5)).all(), seq
+        for bad in (np.inf, np.nan):
+            k[0, at, 3] = bad
+            assert np.isnan(attend(dev, q, k, v, 1, 1, hd, seq, seq + 8)[0]).all(), (seq, bad)
+
+
+@pytest.mark.parametrize("fmt", ["Q8_0", "F16", "Q4_K"])
+def test_step_across_the_switches(ca, fmt):
+    """positions 0 .. 529: k_attn_short from the start (Q8_0) or from 96 (the others) up to 512, k_attn_flash behind -- graph and eager agree
+    bit for bit, and stay as close to the exact chain as k_attn_flash is required to"""
+    model = synth.build_model(synth.SHAPES["tiny-hd128"], synth.TYPE_BY_NAME[fmt], seed=78)
+    dev = ca.HipTensorDevice(0)
+    conf, w = synth.to_hip(model, dev)
+    a, e, x = ca.HipLlamaRunner(conf, w, dev, 533, True), ca.HipLlamaRunner(conf, w, dev, 533, True, False), ca.HipLlamaRunner(conf, w, dev, 533, True, extra_flags=EXACT)
+    check = {0, 94, 95, 96, 97, 128, 510, 511, 512, 529}
+    errs = []
+    for i in range(530):
+        t = (5 * i + 2) % 1000
+        if i not in check:
+            for r in (a, e, x):
+                r.forward_async(t, i)
+            continue
+        got, eager, exact = a.forward(t, i).copy(), e.forward(t, i).copy(), x.forward(t, i).copy()
+        assert np.array_equal(got.view(np.uint32), eager.view(np.uint32)), i
+        if fmt != "Q8_0" and i < 95:
+            assert np.array_equal(got.view(np.uint32), exact.view(np.uint32)), i
+        errs.append(np.max(np.abs(got - exact)) / np.max(np.abs(exact)))
+    assert max(errs) <= 7.5e-2, errs  # (the widest of the long kernels' bounds, helpers.FAST_TOL: a flipped level of the quantized row)
