@@ -98,6 +98,49 @@ __device__ __forceinline__ float rl_f(float v, int lane) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
 }
 // full-wave (64 lanes): every lane gets the result
+// half waves / neighbouring rows of 16 lanes swap and add: the first half (even rows) gets a's sum, the other half (odd rows) b's
+__device__ __forceinline__ float meet32(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+  const unsigned lo = r[0], hi = r[1];
+  return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+}
+__device__ __forceinline__ float meet16(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+  const unsigned lo = r[0], hi = r[1];
+  return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+}
+// Sums over the 64 / LPR groups of LPR lanes.  Of a lane's eight columns it is left with the sums of two -- pair 2 (lane / 32) + (lane / 16) % 2
+// of the four -- in acc[0], acc[1] (LPR = 32: of four, half lane / 32 of the eight).  LPR = 8: lanes 8-15 of a row hold what lanes 0-7 do.
+template <int LPR>
+__device__ __forceinline__ void sum_groups(float (&acc)[8]) {
+#pragma unroll
+  for (int i = 0; i < 4; i++) acc[i] = meet32(acc[i], acc[i + 4]);
+  if constexpr (LPR < 32) {
+    acc[0] = meet16(acc[0], acc[2]);
+    acc[1] = meet16(acc[1], acc[3]);
+  }
+  if constexpr (LPR == 8) {
+    acc[0] += dpp_f<0x128>(acc[0]);
+    acc[1] += dpp_f<0x128>(acc[1]);
+  }
+}
+template <int LPR>
+__device__ __forceinline__ float sum_groups(float v) {
+  v = meet32(v, v);
+  if constexpr (LPR < 32) v = meet16(v, v);
+  if constexpr (LPR == 8) v += dpp_f<0x128>(v);
+  return v;
+}
+// the sum over a group's lanes, in all of them
+template <int LPR>
+__device__ __forceinline__ float group_sum(float v) {
+  v += dpp_f<0xB1>(v);
+  v += dpp_f<0x4E>(v);
+  v += dpp_f<0x141>(v);
+  if constexpr (LPR >= 16) v += dpp_f<0x140>(v);
+  if constexpr (LPR == 32) v = meet16(v, v);
+  return v;
+}
 __device__ __forceinline__ float wave_sum_f32(float v) {
   v = row16_sum_f32(v);
   return (rl_f(v, 0) + rl_f(v, 16)) + (rl_f(v, 32) + rl_f(v, 48));

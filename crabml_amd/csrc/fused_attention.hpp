@@ -504,11 +504,7 @@ __global__ __launch_bounds__(512) void k_attn_short(const float* __restrict__ q,
         d = __builtin_fmaf(qf[2 * i], (float)k[0], d);
         d = __builtin_fmaf(qf[2 * i + 1], (float)k[1], d);
       }
-      d += dpp_f<0xB1>(d);
-      d += dpp_f<0x4E>(d);
-      d += dpp_f<0x141>(d);
-      if constexpr (LPR >= 16) d += dpp_f<0x140>(d);
-      if constexpr (LPR == 32) d += __shfl_xor(d, 16, 64);
+      d = group_sum<LPR>(d);
       s[u] = row0 + u * RR + rc < seq ? d : -INFINITY;
       mc = fmaxf(mc, s[u]);
     }
@@ -543,34 +539,13 @@ __global__ __launch_bounds__(512) void k_attn_short(const float* __restrict__ q,
     }
     take(k1, v1, std::integral_constant<int, U1>{}, r0);
   }
-  // ---- the wave's row classes: lanes < 32 end up with the sums of elements 0-3, the others of 4-7, and (LPR < 32) odd rows of 16 lanes
-  // with the upper two of those
-  auto meet32 = [](float a, float b) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
-    const unsigned lo = r[0], hi = r[1];
-    return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
-  };
-  auto meet16 = [](float a, float b) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
-    const unsigned lo = r[0], hi = r[1];
-    return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
-  };
-#pragma unroll
-  for (int i = 0; i < 4; i++) acc[i] = meet32(acc[i], acc[i + 4]);
-  l = meet32(l, l);
+  sum_groups<LPR>(acc);
+  l = sum_groups<LPR>(l);
   if constexpr (LPR == 32) {
     s_acc[wave][dl * 4 + (lane >> 5) * 2] = f32x2{acc[0], acc[1]};
     s_acc[wave][dl * 4 + (lane >> 5) * 2 + 1] = f32x2{acc[2], acc[3]};
-  } else {
-    acc[0] = meet16(acc[0], acc[2]);
-    acc[1] = meet16(acc[1], acc[3]);
-    l = meet16(l, l);
-    if constexpr (LPR == 8) {  // two rows' lanes in 16
-      acc[0] += dpp_f<0x128>(acc[0]);
-      acc[1] += dpp_f<0x128>(acc[1]);
-      l += dpp_f<0x128>(l);
-    }
-    if (LPR == 16 || (lane & 8) == 0) s_acc[wave][dl * 4 + (lane >> 5) * 2 + ((lane >> 4) & 1)] = f32x2{acc[0], acc[1]};
+  } else if (LPR == 16 || (lane & 8) == 0) {
+    s_acc[wave][dl * 4 + (lane >> 5) * 2 + ((lane >> 4) & 1)] = f32x2{acc[0], acc[1]};
   }
   if (lane == 0) {
     s_m[wave] = first < seq ? m : -INFINITY;

@@ -7,14 +7,17 @@
 //   k_gemv_bf16<PLAIN, RESIDUAL>  down projection + residual (+ what a pass adds)
 // Tokens, positions and the sequences' state pointers are read from device memory, so a captured graph serves every step.
 #pragma once
+#include <cfloat>
+
 #include "hybrid_common.hpp"
 #include "sampler.hpp"
 
 namespace crabml_hip {
 
 #define HYB_STEP_ROWS 16
-#define MIX_KEYS 64   // cached rows per attention workgroup
-#define MIX_HEADS 8   // query heads per attention workgroup
+#define MIX_ONE 256   // up to so many cached rows one workgroup takes them all
+#define MIX_KEYS 128  // ... and past that so many per workgroup
+#define MIX_HEADS 4   // query heads per attention workgroup
 
 struct StepSeq {
   int token, pos;
@@ -62,7 +65,7 @@ struct MixStep {
   float* v_kept = nullptr;      // [B][ld_vk] values that VMIX_KEEP leaves
   int ld_vk = 0;
   unsigned* tick = nullptr;     // arrivals per (sequence, kv head, head block); the last one puts it back to zero
-  int B = 0, ldp = 0, ldc = 0, lin_off = 0, splits = 0, head_blocks = 0;
+  int B = 0, ldp = 0, ldc = 0, lin_off = 0, splits = 0, head_blocks = 0, heads = 0;
 };
 // floats of one partial: per head its V sums, the running maximum and the denominator
 __host__ __device__ inline int mix_part_floats(int V) { return MIX_HEADS * (V + 2); }
@@ -74,12 +77,17 @@ __device__ __forceinline__ void cat_out(float* cat, unsigned short* cat16, size_
     cat[at] = v;
 }
 
-// One workgroup: up to MIX_HEADS query heads of one kv head over MIX_KEYS cached rows; heads up to CLS wide.  Everything it needs from
-// memory is requested up front; the rest is register and LDS work.  (The launch runs cold: its code is kept short.)
-template <typename T, int CLS>
+// One workgroup: up to MIX_HEADS query heads of one kv head over its share of the cached rows; heads up to CLS wide.  What bounds it is the
+// chain position -> rows -> scores -> softmax -> sums of a cold launch, so the chain has one barrier where the heads' operands are laid out and
+// one where the waves meet: a row is LPR lanes x 8 elements and a wave instruction takes 64 / LPR rows; a wave keeps K and V of its rows in
+// registers, scores them for every head, takes its own maximum, and adds up p * v over its rows.  (64 rows a round and four heads: 128 registers,
+// so that two workgroups -- the linear branch's are as large -- share a CU.)  Four barriers, a wave per head's softmax and LDS exchanges between
+// 256 threads before that: 13.0 -> 9.4 us a launch (one sequence, 33 to 81 rows, normed q and k), 15.4 -> 13.2 (16 sequences, 90 to 154 rows,
+// linear branch beside it).  Up to MIX_ONE rows stay in one workgroup:
+// handing partial sums over costs 3 us, a second round of 128 rows 0.6.
+template <typename T, int CLS, int NT>
 __device__ __forceinline__ void mix_attention(const MixStep& a, int blk, float* lds) {
-  constexpr int NU = CLS / 32;                             // K: four lanes per row, their octets interleaved
-  constexpr int CP = CLS / 8, GR = 256 / CP, NV = MIX_KEYS / GR;  // V: CP lanes across the columns, GR groups of rows
+  constexpr int LPR = CLS / 8, RPI = 64 / LPR, NW = NT / 64, RR = NW * RPI, U = 64 / RR < 4 ? 64 / RR : 4;
   const AttnGeom& g = a.at;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_wg();
   const int split = blk % a.splits;
@@ -89,35 +97,63 @@ __device__ __forceinline__ void mix_attention(const MixStep& a, int blk, float* 
   const int kvh = rest % g.G, b = rest / g.G;
   const StepSeq sq = a.seq[b];
   const int hpg = g.H / g.G, h0 = kvh * hpg + hb * MIX_HEADS;
-  const int nh = hpg - hb * MIX_HEADS < MIX_HEADS ? hpg - hb * MIX_HEADS : MIX_HEADS;
+  const int nh = hpg - hb * MIX_HEADS < MIX_HEADS ? hpg - hb * MIX_HEADS : MIX_HEADS, heads = a.heads;
   const float* pr = a.proj + (size_t)b * a.ldp;
-  float* ml = lds;                          // [MIX_HEADS][2]: maximum, denominator
-  float* hp_s = ml + 2 * MIX_HEADS;         // [3][MIX_HEADS]: penalty factor, its rate, sink; then the waves' square sums of q and k
-  T* kn_s = (T*)(hp_s + 5 * MIX_HEADS);     // [CLS], [CLS]: the new token's row as the cache holds it
+  float* m_s = lds;                       // [NW][MIX_HEADS] the waves' maxima
+  float* l_s = m_s + NW * MIX_HEADS;      // ... and denominators
+  float* hp_s = l_s + NW * MIX_HEADS;     // [3][MIX_HEADS]: penalty factor, its rate, sink; then the waves' square sums of q and k
+  T* kn_s = (T*)(hp_s + 3 * MIX_HEADS + 2 * NW);  // [CLS], [CLS]: the new token's row as the cache holds it
   T* vn_s = kn_s + CLS;
-  float* g_s = (float*)(vn_s + CLS);        // [MIX_HEADS][V]: gates
-  float* q_s = g_s + MIX_HEADS * g.V;       // [MIX_HEADS][D]
-  float* p_s = q_s + MIX_HEADS * g.D;       // [MIX_HEADS][MIX_KEYS]
-  float* o_s = p_s + MIX_HEADS * MIX_KEYS;  // [4 waves][MIX_HEADS][V]
-  // what does not depend on the position: on its way together with it
+  float* g_s = (float*)(vn_s + CLS);      // [heads][V]: gates
+  float* q_s = g_s + heads * g.V;         // [heads][D]
+  float* o_s = q_s + heads * g.D;         // [NW][heads][V]
+  // the new token's row, and the rows it sees: its chunk's up to itself, or the whole ring once the window has gone round
+  const int in_chunk = sq.pos % g.span, n_rows = g.window && sq.pos >= g.span ? g.span : in_chunk + 1;
+  const int keys = n_rows <= MIX_ONE ? MIX_ONE : MIX_KEYS, r0 = split * keys;
+  if (r0 >= n_rows) return;  // (whole workgroup)
+  const int active = (n_rows + keys - 1) / keys, r1 = r0 + keys < n_rows ? r0 + keys : n_rows;
+  T* kc = (T*)(sq.slab + a.rs.k) + (size_t)kvh * g.rows * g.D;
+  T* vc = (T*)(sq.slab + a.rs.v) + (size_t)kvh * g.rows * g.V;
+  const bool own_new = in_chunk >= r0 && in_chunk < r1;
+  const int rc = lane / LPR, c = lane % LPR * 8;
+  const bool kcol = c < g.D, vcol = c < g.V;
+  Oct<T> kr[U], vr[U];
+  auto fetch = [&](int base) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int row = base + u * RR + rc;
+      const bool in = row < r1 && row != in_chunk;
+      kr[u] = vr[u] = oct_zero<T>();
+      if (in && kcol) kr[u] = oct_load(kc + (size_t)row * g.D + c);
+      if (in && vcol) vr[u] = oct_load(vc + (size_t)row * g.V + c);
+    }
+  };
+  const int first = r0 + wave * RPI;
+  fetch(first);
   float q_f = g.scale, k_f = 1.f;
   if (g.q_norm) {  // (the same for the whole workgroup)
     float sq2 = 0.f, sk2 = 0.f;
-    for (int i = tid; i < g.H * g.D; i += 256) sq2 = __builtin_fmaf(pr[g.cq + i], pr[g.cq + i], sq2);
-    for (int i = tid; i < g.G * g.D; i += 256) sk2 = __builtin_fmaf(pr[g.ck + i], pr[g.ck + i], sk2);
+    for (int i = tid; i < g.H * g.D; i += NT) sq2 = __builtin_fmaf(pr[g.cq + i], pr[g.cq + i], sq2);
+    for (int i = tid; i < g.G * g.D; i += NT) sk2 = __builtin_fmaf(pr[g.ck + i], pr[g.ck + i], sk2);
     sq2 = wave_sum_f32(sq2);
     sk2 = wave_sum_f32(sk2);
     float* red = hp_s + 3 * MIX_HEADS;
     if (lane == 0) {
       red[wave] = sq2;
-      red[4 + wave] = sk2;
+      red[NW + wave] = sk2;
     }
     __syncthreads();
-    q_f *= 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)g.q_mean + g.eps);
-    k_f = 1.0f / sqrtf(((red[4] + red[5]) + (red[6] + red[7])) / (float)g.k_mean + g.eps);
+    sq2 = sk2 = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      sq2 += red[w];
+      sk2 += red[NW + w];
+    }
+    q_f *= 1.0f / sqrtf(sq2 / (float)g.q_mean + g.eps);
+    k_f = 1.0f / sqrtf(sk2 / (float)g.k_mean + g.eps);
   }
-  for (int i = tid; i < nh * g.D; i += 256) q_s[i] = pr[g.cq + h0 * g.D + i] * (g.q_norm ? q_f * g.q_norm[h0 * g.D + i] : q_f);
-  for (int i = tid; i < nh * g.V; i += 256)
+  for (int i = tid; i < nh * g.D; i += NT) q_s[i] = pr[g.cq + h0 * g.D + i] * (g.q_norm ? q_f * g.q_norm[h0 * g.D + i] : q_f);
+  for (int i = tid; i < nh * g.V; i += NT)
     g_s[i] = (g.gate == GATE_ELEMENT ? pr[g.cg + h0 * g.V + i] : g.gate == GATE_HEAD ? pr[g.cg + h0 + i / g.V] : 1.f) * g.out_scale;
   if (tid < g.D) kn_s[tid] = kv_from<T>(pr[g.ck + kvh * g.D + tid] * (g.k_norm ? k_f * g.k_norm[kvh * g.D + tid] : 1.f));
   float v_raw = 0.f;
@@ -135,102 +171,83 @@ __device__ __forceinline__ void mix_attention(const MixStep& a, int blk, float* 
     hp_s[MIX_HEADS + tid] = g.amp ? g.rate[h0 + tid] : 0.f;
     hp_s[2 * MIX_HEADS + tid] = g.sink ? g.sink[h0 + tid] : -INFINITY;
   }
-  // the new token's row, and the rows it sees: its chunk's up to itself, or the whole ring once the window has gone round
-  const int in_chunk = sq.pos % g.span, n_rows = g.window && sq.pos >= g.span ? g.span : in_chunk + 1;
-  const int r0 = split * MIX_KEYS;
-  if (r0 >= n_rows) return;  // (whole workgroup)
-  const int active = (n_rows + MIX_KEYS - 1) / MIX_KEYS;
-  const int nk = n_rows - r0 < MIX_KEYS ? n_rows - r0 : MIX_KEYS;
-  T* kc = (T*)(sq.slab + a.rs.k) + (size_t)kvh * g.rows * g.D;
-  T* vc = (T*)(sq.slab + a.rs.v) + (size_t)kvh * g.rows * g.V;
-  const bool own_new = in_chunk >= r0 && in_chunk < r0 + MIX_KEYS;
-  const int key = tid >> 2, part = tid & 3, vcol = tid % CP * 8, vgrp = tid / CP;
-  Oct<T> kr[NU], vr[NV];
-#pragma unroll
-  for (int u = 0; u < NU; u++) {
-    const int c = part * 8 + u * 32;
-    kr[u] = oct_zero<T>();
-    if (c < g.D && key < nk && r0 + key != in_chunk) kr[u] = oct_load(kc + (size_t)(r0 + key) * g.D + c);
-  }
-#pragma unroll
-  for (int u = 0; u < NV; u++) {
-    const int k = vgrp + u * GR;
-    vr[u] = oct_zero<T>();
-    if (k < nk && vcol < g.V && r0 + k != in_chunk) vr[u] = oct_load(vc + (size_t)(r0 + k) * g.V + vcol);
-  }
   __syncthreads();
-  if (own_new) {  // the new row: appended to the cache by one head block, taken from LDS by all
-    if (hb == 0) {
-      if (tid < g.D) kc[(size_t)in_chunk * g.D + tid] = kn_s[tid];
-      if (tid < g.V) vc[(size_t)in_chunk * g.V + tid] = vn_s[tid];
-      if (g.vmix == VMIX_KEEP && tid < g.V) a.v_kept[(size_t)b * a.ld_vk + kvh * g.V + tid] = v_raw;
-    }
-    if (r0 + key == in_chunk) {
-#pragma unroll
-      for (int u = 0; u < NU; u++)
-        if (part * 8 + u * 32 < g.D) kr[u] = oct_load(kn_s + part * 8 + u * 32);
-    }
-#pragma unroll
-    for (int u = 0; u < NV; u++)
-      if (r0 + vgrp + u * GR == in_chunk && vcol < g.V) vr[u] = oct_load(vn_s + vcol);
+  if (own_new && hb == 0) {  // the new row: appended to the cache by one head block, taken from LDS by all
+    if (tid < g.D) kc[(size_t)in_chunk * g.D + tid] = kn_s[tid];
+    if (tid < g.V) vc[(size_t)in_chunk * g.V + tid] = vn_s[tid];
+    if (g.vmix == VMIX_KEEP && tid < g.V) a.v_kept[(size_t)b * a.ld_vk + kvh * g.V + tid] = v_raw;
   }
-  {
-    const int behind = in_chunk - (r0 + key);
-    const float dist = (float)(g.window && behind < 0 ? behind + g.span : behind);
-    float kk[NU][8];
+  float m[MIX_HEADS], l[MIX_HEADS], o[MIX_HEADS][8];  // m: the same in all lanes of the wave (a row of -inf scores has weight 0)
 #pragma unroll
-    for (int u = 0; u < NU; u++) oct_floats(kr[u], kk[u]);
-    for (int h = 0; h < nh; h++) {
-      const float* q = q_s + h * g.D + part * 8;
-      float s = 0.f;
+  for (int h = 0; h < MIX_HEADS; h++) {
+    m[h] = -FLT_MAX;
+    l[h] = 0.f;
 #pragma unroll
-      for (int u = 0; u < NU; u++) {
-        if (part * 8 + u * 32 < g.D) {
-          const f32x4 q0 = *(const f32x4*)(q + u * 32), q1 = *(const f32x4*)(q + u * 32 + 4);
+    for (int e = 0; e < 8; e++) o[h][e] = 0.f;
+  }
+#pragma unroll 1
+  for (int base = first; base < r1; base += U * RR) {
+    float kf[U][8], vf[U][8], dist[U];
 #pragma unroll
-          for (int e = 0; e < 4; e++) s = __builtin_fmaf(q0[e], kk[u][e], __builtin_fmaf(q1[e], kk[u][e + 4], s));
-        }
+    for (int u = 0; u < U; u++) {
+      const int row = base + u * RR + rc, behind = in_chunk - row;
+      if (row == in_chunk) {
+        if (kcol) kr[u] = oct_load(kn_s + c);
+        if (vcol) vr[u] = oct_load(vn_s + c);
       }
-      s += dpp_f<0xB1>(s);
-      s += dpp_f<0x4E>(s);
-      s -= hp_s[h] * __logf(__builtin_fmaf(hp_s[MIX_HEADS + h], dist > 0.f ? dist : 0.f, 1.0f));
-      if (part == 0) p_s[h * MIX_KEYS + key] = key < nk ? s : -INFINITY;
+      oct_floats(kr[u], kf[u]);
+      oct_floats(vr[u], vf[u]);
+      const int back = g.window && behind < 0 ? behind + g.span : behind;
+      dist[u] = (float)(back > 0 ? back : 0);
+    }
+    if (base + U * RR < r1) fetch(base + U * RR);  // (the next round's, while this one is worked on)
+#pragma unroll
+    for (int h = 0; h < MIX_HEADS; h++) {
+      if (h >= nh) break;  // (uniform)
+      f32x4 q0 = {0.f, 0.f, 0.f, 0.f}, q1 = q0;
+      if (kcol) {
+        q0 = *(const f32x4*)(q_s + h * g.D + c);
+        q1 = *(const f32x4*)(q_s + h * g.D + c + 4);
+      }
+      float s[U], mc = -INFINITY;
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        float d = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; e++) d = __builtin_fmaf(q0[e], kf[u][e], __builtin_fmaf(q1[e], kf[u][e + 4], d));
+        d = group_sum<LPR>(d);
+        if (g.amp) d -= hp_s[h] * __logf(__builtin_fmaf(hp_s[MIX_HEADS + h], dist[u], 1.0f));
+        s[u] = base + u * RR + rc < r1 ? d : -INFINITY;
+        mc = fmaxf(mc, s[u]);
+      }
+      const float mn = fmaxf(m[h], wave_max_f32(mc)), alpha = __expf(m[h] - mn);
+      m[h] = mn;
+      l[h] *= alpha;
+#pragma unroll
+      for (int e = 0; e < 8; e++) o[h][e] *= alpha;
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const float w = __expf(s[u] - mn);
+        l[h] += w;
+#pragma unroll
+        for (int e = 0; e < 8; e++) o[h][e] = __builtin_fmaf(w, vf[u][e], o[h][e]);
+      }
     }
   }
-  __syncthreads();
-  for (int h = wave; h < nh; h += 4) {  // one wave per head: MIX_KEYS = 64 scores
-    const float s = p_s[h * MIX_KEYS + lane];
-    const float m = wave_max_f32(s);
-    const float e = __expf(s - m);
-    p_s[h * MIX_KEYS + lane] = e;
-    const float l = wave_sum_f32(e);
+#pragma unroll
+  for (int h = 0; h < MIX_HEADS; h++) {
+    if (h >= nh) break;
+    sum_groups<LPR>(o[h]);
+    l[h] = sum_groups<LPR>(l[h]);
+    float* d = o_s + (wave * heads + h) * g.V + c + (lane >> 5) * 4;
+    if (LPR == 32) {
+      if (vcol) *(f32x4*)d = f32x4{o[h][0], o[h][1], o[h][2], o[h][3]};
+    } else if (vcol && (LPR == 16 || (lane & 8) == 0)) {
+      *(f32x2*)(d + ((lane >> 4) & 1) * 2) = f32x2{o[h][0], o[h][1]};
+    }
     if (lane == 0) {
-      ml[2 * h] = m;
-      ml[2 * h + 1] = l;
-    }
-  }
-  __syncthreads();
-  {  // weighted value rows, added over the wave's row groups by lane exchange, over the waves through LDS
-    float vv[NV][8];
-#pragma unroll
-    for (int u = 0; u < NV; u++) oct_floats(vr[u], vv[u]);
-    for (int h = 0; h < nh; h++) {
-      float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int u = 0; u < NV; u++) {
-        const float w = p_s[h * MIX_KEYS + vgrp + u * GR];
-#pragma unroll
-        for (int e = 0; e < 8; e++) o[e] = __builtin_fmaf(w, vv[u][e], o[e]);
-      }
-#pragma unroll
-      for (int x = CP; x < 64; x <<= 1)
-#pragma unroll
-        for (int e = 0; e < 8; e++) o[e] += __shfl_xor(o[e], x, 64);
-      if (lane < CP && vcol < g.V) {
-        float* d = o_s + (wave * MIX_HEADS + h) * g.V + vcol;
-        *(f32x4*)d = f32x4{o[0], o[1], o[2], o[3]};
-        *(f32x4*)(d + 4) = f32x4{o[4], o[5], o[6], o[7]};
-      }
+      m_s[wave * MIX_HEADS + h] = first < r1 ? m[h] : -INFINITY;
+      l_s[wave * MIX_HEADS + h] = l[h];
     }
   }
   __syncthreads();
@@ -238,11 +255,31 @@ __device__ __forceinline__ void mix_attention(const MixStep& a, int blk, float* 
   const int wstr = MIX_HEADS * g.V, pf = mix_part_floats(g.V), n_out = nh * g.V;
   float* base = a.part + (size_t)slot * a.splits * pf;
   __shared__ unsigned s_last;
+  auto met = [&](int i, float& M, float& L) {  // output i of the workgroup's rows: its sum, the head's maximum and denominator
+    const int h = i / g.V;
+    M = m_s[h];
+#pragma unroll
+    for (int w = 1; w < NW; w++) M = fmaxf(M, m_s[w * MIX_HEADS + h]);
+    L = 0.f;
+    float r = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      const float e = __expf(m_s[w * MIX_HEADS + h] - M);
+      L = __builtin_fmaf(l_s[w * MIX_HEADS + h], e, L);
+      r = __builtin_fmaf(o_s[w * heads * g.V + i], e, r);
+    }
+    return r;
+  };
   if (active > 1) {  // partials through write-through stores; whoever arrives last merges them in row order
     float* mine = base + (size_t)split * pf;
-    for (int i = tid; i < n_out; i += 256)
-      __hip_atomic_store(mine + i, (o_s[i] + o_s[wstr + i]) + (o_s[2 * wstr + i] + o_s[3 * wstr + i]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (tid < 2 * nh) __hip_atomic_store(mine + wstr + tid, ml[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int i = tid; i < n_out; i += NT) {
+      float M, L;
+      __hip_atomic_store(mine + i, met(i, M, L), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (i % g.V == 0) {
+        __hip_atomic_store(mine + wstr + 2 * (i / g.V), M, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(mine + wstr + 2 * (i / g.V) + 1, L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's write-through stores have been acknowledged
     __syncthreads();
     if (tid == 0) s_last = __hip_atomic_fetch_add(a.tick + slot, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(active - 1);
@@ -250,13 +287,14 @@ __device__ __forceinline__ void mix_attention(const MixStep& a, int blk, float* 
     if (!s_last) return;
     if (tid == 0) __hip_atomic_store(a.tick + slot, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  for (int i = tid; i < n_out; i += 256) {
+  for (int i = tid; i < n_out; i += NT) {
     const int h = i / g.V;
     float m = hp_s[2 * MIX_HEADS + h], l = m == -INFINITY ? 0.f : 1.f, o = 0.f;  // the sink: a key without a value (or none)
     if (active == 1) {
-      const float mx = fmaxf(m, ml[2 * h]), w = __expf(ml[2 * h] - mx);
-      l = __builtin_fmaf(l, __expf(m - mx), ml[2 * h + 1] * w);
-      o = ((o_s[i] + o_s[wstr + i]) + (o_s[2 * wstr + i] + o_s[3 * wstr + i])) * w;
+      float M, L;
+      const float r = met(i, M, L), mx = fmaxf(m, M), w = __expf(M - mx);
+      l = __builtin_fmaf(l, __expf(m - mx), L * w);
+      o = r * w;
     } else {
       for (int s0 = 0; s0 < active; s0 += 16) {
         float ps[16], ms[16], ls[16], mx = m;
@@ -285,10 +323,15 @@ __device__ __forceinline__ void mix_attention(const MixStep& a, int blk, float* 
   }
 }
 
-// one head's slice of value columns: 8 threads x 4 columns, 32 groups of key rows
+// one head's slice of value columns: 8 threads x 4 columns, 32 groups of key rows; 256 threads a slice
+template <int NT>
 __device__ __forceinline__ void mix_linear(const MixStep& a, int blk, float* lds) {
   const LinGeom& g = a.li;
-  const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_wg();
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = wave_in_wg() & 3, part = wave_in_wg() >> 2;
+  const int n = a.B * g.H * g.slices, unit = blk * (NT / 256) + part;
+  const bool used = unit < n;  // (the last workgroup's second slice may be none)
+  blk = used ? unit : n - 1;
+  lds += part * (2 * g.D + 32 * 36);
   const int slice = blk % g.slices, h = (blk / g.slices) % g.H, b = blk / (g.slices * g.H);
   const StepSeq sq = a.seq[b];
   float* S = (float*)(sq.slab + a.rs.s) + (size_t)h * g.D * g.V;
@@ -297,7 +340,7 @@ __device__ __forceinline__ void mix_linear(const MixStep& a, int blk, float* lds
   float* q_s = k_s + g.D;  // [D]
   float* o_s = q_s + g.D;  // [32][32 + 4]
   const int c = slice * LIN_SLICE + (tid & 7) * 4, grp = tid >> 3;
-  const bool live = c < g.V;
+  const bool live = used && c < g.V;
   const bool fresh = sq.pos == 0;  // a sequence's first token: whatever the slab holds, the state is zero
   f32x4 s[8];  // (at most 256 key rows)
 #pragma unroll
@@ -338,28 +381,32 @@ __device__ __forceinline__ void mix_linear(const MixStep& a, int blk, float* lds
 #pragma unroll
       for (int i = 0; i < 32; i++) r += o_s[i * 36 + lane];
     }
-    const bool in = lane < LIN_SLICE && oc < g.V;
+    const bool in = used && lane < LIN_SLICE && oc < g.V;
     const float ss = wave_sum_f32(in ? r * r : 0.f);
-    if (lane == 0) a.ss[(size_t)b * g.H * g.slices + h * g.slices + slice] = ss;
+    if (used && lane == 0) a.ss[(size_t)b * g.H * g.slices + h * g.slices + slice] = ss;
     if (in) cat_out(a.cat, a.cat16, (size_t)b * a.ldc + a.lin_off + occ, r * factor);
   }
 }
 
-template <typename T, int CLS>
-__global__ __launch_bounds__(256) void k_mix_step(const MixStep a) {
+template <typename T, int CLS, int NT>
+__global__ __launch_bounds__(NT, NT == 512 && sizeof(T) == 2 ? 4 : 2) void k_mix_step(const MixStep a) {
   extern __shared__ __attribute__((aligned(16))) float mix_lds[];
   const int n_attn = a.at.H ? a.B * a.at.G * a.head_blocks * a.splits : 0;
   if ((int)blockIdx.x < n_attn)
-    mix_attention<T, CLS>(a, blockIdx.x, mix_lds);
+    mix_attention<T, CLS, NT>(a, blockIdx.x, mix_lds);
   else
-    mix_linear(a, blockIdx.x - n_attn, mix_lds);
+    mix_linear<NT>(a, blockIdx.x - n_attn, mix_lds);
 }
 template <typename T, int CLS>
-inline void launch_mix_step_t(hipStream_t st, crabml_hip_device::ProfRec* rec, const MixStep& a) {
-  const size_t at = a.at.H ? 7 * MIX_HEADS + 2 * CLS * sizeof(T) / 4 + (size_t)MIX_HEADS * (a.at.D + MIX_KEYS + 5 * a.at.V) : 0;
-  const size_t li = a.li.H ? (size_t)(2 * a.li.D + 32 * 36) : 0;
-  const unsigned grid = (unsigned)(a.B * ((a.at.H ? a.at.G * a.head_blocks * a.splits : 0) + a.li.H * a.li.slices));
-  launch_k(st, rec, k_mix_step<T, CLS>, dim3(grid), dim3(256), (at > li ? at : li) * sizeof(float), a);  // (at most 57 KiB)
+inline void launch_mix_step_t(hipStream_t st, crabml_hip_device::ProfRec* rec, MixStep a) {
+  constexpr int NT = CLS == 256 ? 256 : 512, NW = NT / 64;  // (the waves' sums of 256 columns would not fit twice)
+  const int hpg = a.at.H ? a.at.H / a.at.G : 0;
+  a.heads = hpg < MIX_HEADS ? hpg : MIX_HEADS;
+  const size_t at = a.at.H ? (2 * NW + 3) * MIX_HEADS + 2 * NW + 2 * CLS * sizeof(T) / 4 + (size_t)a.heads * (a.at.D + (NW + 1) * a.at.V) : 0;
+  const size_t li = a.li.H ? (size_t)(2 * a.li.D + 32 * 36) * (NT / 256) : 0;
+  const int units = a.B * a.li.H * a.li.slices;
+  const unsigned grid = (unsigned)((a.at.H ? a.B * a.at.G * a.head_blocks * a.splits : 0) + (units + NT / 256 - 1) / (NT / 256));
+  launch_k(st, rec, k_mix_step<T, CLS, NT>, dim3(grid), dim3(NT), (at > li ? at : li) * sizeof(float), a);  // (at most 51 KiB)
 }
 template <typename T>
 inline void launch_mix_step(hipStream_t st, crabml_hip_device::ProfRec* rec, const MixStep& a) {
