@@ -1396,6 +1396,9 @@ int prefill_chunk(crabml_hip_llama* c, const uint32_t* tokens, size_t B, size_t 
     }
     if (gemm_f16({w}, {(size_t)m}, (size_t)k, act, {out})) return 0;
     if (!strict) {
+      if (!gemm_exact_hook && B >= 16 && (w->dtype == CRABML_HIP_Q4_0 || w->dtype == CRABML_HIP_Q8_0 || w->dtype == CRABML_HIP_Q4_1) &&
+          launch_gemm_mfma(dev, w, m, k, act, B, out, nullptr, nullptr, true, c->pf_split, c->pf_split_floats, defer))
+        return 0;
       return launch_gemv(dev, w, m, k, act, B, out, nullptr, !gemm_exact_hook);
     }
     // strict order: the Q4_0 / Q8_0 / Q4_1 MFMA GEMM scales its exact integer tiles block by block in the reference's scalar

@@ -688,4 +688,14 @@ bool launch_gemm_f16w(crabml_hip_device* dev, const crabml_hip_buf* const* w, co
   return ok;
 }
 
+void launch_add_parts(hipStream_t st, float* out, const float* ws, size_t n, int nparts) {
+  F16wParts parts{};
+  parts.out[0] = out;
+  parts.part[0] = const_cast<float*>(ws);
+  parts.end4[0] = parts.end4[1] = parts.end4[2] = n / 4;
+  parts.pstride = n;
+  parts.nparts = nparts;
+  k_addn_f32<<<(unsigned)((n / 4 + 255) / 256), 256, 0, st>>>(parts);
+}
+
 }  // namespace crabml_hip

@@ -49,10 +49,13 @@ struct GemmGeo {
 // product and the add as one v_pk_fma_f32 (8 instead of 10 VALU operations per MFMA; one rounding fewer than the reference's
 // expression, the same distance the fast decode step's re-associated sums are allowed).  matmul_vec itself and the strict-order
 // device keep the reference's three roundings (bit-exact, tests/test_hip_gemv.py).
+// pieces > 1 (the fast prompt pass only): that many workgroups per tile, each over its chunks of k; piece s >= 1 leaves its sums in
+// ws + (s - 1) b m, added in piece order behind (a short pass has few tiles: 64 workgroups and a chain of nb / KC chunks otherwise)
 template <int FMT, int NT, bool FMA = false>
 __global__ __launch_bounds__(256) void k_gemm_mfma(const char* __restrict__ wq, const unsigned short* __restrict__ wd,
                                                    const char* __restrict__ act, size_t act_stride, size_t off_d, size_t off_aux,
-                                                   float* __restrict__ out, int m, int nb, int b, int row_tiles) {
+                                                   float* __restrict__ out, int m, int nb, int b, int row_tiles, int pieces,
+                                                   float* __restrict__ ws) {
   using G = GemmGeo<FMT, NT>;
   constexpr int KC = G::KC, APC = G::APC, ARW = G::ARW, BRW = G::BRW, CW = G::CW;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
@@ -62,17 +65,19 @@ __global__ __launch_bounds__(256) void k_gemm_mfma(const char* __restrict__ wq, 
   // 35 MB gate/up GEMM with column-major tile order).  XCD x owns the row tiles rt = x (mod 8); its j-th workgroup
   // is (rt = 8 (j / col_tiles) + x, ct = j % col_tiles).  The activation tiles (8 x 295 KB) stay L2-resident.
   int rt, ct;
+  const int tiles = (int)gridDim.x / pieces, piece = (int)blockIdx.x / tiles, tile = (int)blockIdx.x % tiles;
   {
-    const int col_tiles = (int)gridDim.x / row_tiles;
+    const int col_tiles = tiles / row_tiles;
     if ((row_tiles & 7) == 0) {
-      const int x = (int)blockIdx.x & 7, j = (int)blockIdx.x >> 3;
+      const int x = tile & 7, j = tile >> 3;
       ct = j % col_tiles;
       rt = (j / col_tiles) * 8 + x;
     } else {
-      rt = (int)blockIdx.x % row_tiles;
-      ct = (int)blockIdx.x / row_tiles;
+      rt = tile % row_tiles;
+      ct = tile / row_tiles;
     }
   }
+  if (piece > 0) out = ws + (size_t)(piece - 1) * b * m;
   const int r0 = rt * 64, c0 = ct * CW;
   const int i = lane & 15, g = lane >> 4;
 
@@ -177,16 +182,16 @@ __global__ __launch_bounds__(256) void k_gemm_mfma(const char* __restrict__ wq, 
   using S0 = std::integral_constant<int, 0>;
   using S1 = std::integral_constant<int, 1>;
   using S2 = std::integral_constant<int, 2>;
-  const int nchunks = (nb + KC - 1) / KC;
+  const int all = (nb + KC - 1) / KC, c_lo = all * piece / pieces, nchunks = all * (piece + 1) / pieces - c_lo;
   // every fetch / commit below is unconditional (chunk indices past the end are clamped: they re-read the last
   // chunk and are never multiplied): with a fixed number of loads per iteration the compiler's s_waitcnt vmcnt(n)
   // before a commit waits for exactly the loads of that chunk; with conditional fetches it fell back to waiting
   // for everything in flight, i.e. one HBM round trip per chunk
-  const int last = (nchunks - 1) * KC;
-  fetch(S0{}, 0);
+  const int first = c_lo * KC, last = (c_lo + nchunks - 1) * KC;
+  fetch(S0{}, first);
   commit(S0{}, 0);
-  fetch(S1{}, KC < last ? KC : last);
-  if constexpr (PF == 3) fetch(S2{}, 2 * KC < last ? 2 * KC : last);
+  fetch(S1{}, first + KC < last ? first + KC : last);
+  if constexpr (PF == 3) fetch(S2{}, first + 2 * KC < last ? first + 2 * KC : last);
   __syncthreads();
   // per-lane LDS offsets (words), constant over the k loop: the block index only adds immediates
   const int a_off = (16 * wave + i) * ARW + ((FMT == CRABML_HIP_Q4_0 || FMT == CRABML_HIP_Q4_1) ? g : 2 * g);
@@ -194,9 +199,9 @@ __global__ __launch_bounds__(256) void k_gemm_mfma(const char* __restrict__ wq, 
   // iteration c: request chunk c + PF into the set chunk c used, multiply chunk c (LDS buffer c & 1), commit chunk
   // c + 1 (requested two iterations ago) to the other buffer, barrier
   auto step = [&](auto SET_C, auto SET_N, int c) {
-    const int kb0 = c * KC, buf = c & 1;
+    const int kb0 = first + c * KC, buf = c & 1;
     const int kc = c >= nchunks ? 0 : nb - kb0 < KC ? nb - kb0 : KC;
-    fetch(SET_C, (c + PF) * KC < last ? (c + PF) * KC : last);
+    fetch(SET_C, first + (c + PF) * KC < last ? first + (c + PF) * KC : last);
     const unsigned* sA = (const unsigned*)(lds_raw + (size_t)buf * G::BUF_BYTES);
     const unsigned* sB = sA + G::A_WORDS;
     const float* sAd = (const float*)(sB + G::B_WORDS);
@@ -842,7 +847,8 @@ __global__ __launch_bounds__(256) void k_gemm_mfma_q8k(const i32x4* __restrict__
 
 // returns false when the shape / format is not covered (the caller falls back to one GEMV per batch row)
 bool launch_gemm_mfma(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m, size_t k, const void* act, size_t b, float* out,
-                      crabml_hip_device::ProfRec* rec, int* dbg, bool fused_add) {
+                      crabml_hip_device::ProfRec* rec, int* dbg, bool fused_add, float* ws, size_t ws_floats, int* defer_parts) {
+  if (defer_parts) *defer_parts = 0;
   if (w->dtype != CRABML_HIP_Q4_0 && w->dtype != CRABML_HIP_Q8_0 && w->dtype != CRABML_HIP_Q4_K && w->dtype != CRABML_HIP_Q6_K &&
       w->dtype != CRABML_HIP_Q4_1 && w->dtype != CRABML_HIP_Q8_K)
     return false;
@@ -869,7 +875,7 @@ bool launch_gemm_mfma(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m,
     if (k % 256 != 0) return false;
     const ActLayout alk = act_layout(CRABML_HIP_Q8_K, k);
     const int nsb = (int)(k / 256), rtl = (int)((m + 63) / 64);
-    const bool narrow_k = (size_t)rtl * ((b + 63) / 64) < (size_t)4 * dev->n_cu && b > 16;
+    const bool narrow_k = (size_t)rtl * ((b + 63) / 64) < (size_t)4 * dev->n_cu;
     const int cwk = narrow_k ? 32 : 64, ctl = (int)((b + cwk - 1) / cwk);
     const i32x4* wqk = (const i32x4*)wp;
     const i32x4* whk = (const i32x4*)(wp + w->wl.off_scale);
@@ -892,16 +898,24 @@ bool launch_gemm_mfma(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m,
     const int v = hooks && hooks[0] == '1' && e ? atoi(e) : 4;
     return v >= 0 && v <= 16 ? v : 4;
   }();
-  const bool narrow = (size_t)row_tiles * ((b + 63) / 64) < (size_t)narrow_wgs_per_cu * dev->n_cu && b > 16;
+  const bool narrow = (size_t)row_tiles * ((b + 63) / 64) < (size_t)narrow_wgs_per_cu * dev->n_cu;
   const int cw = narrow ? 32 : 64;
   const int col_tiles = (int)((b + cw - 1) / cw);
   const unsigned short* wd = (const unsigned short*)(wp + w->wl.off_scale);
+  // pieces of k while the tiles leave CUs without work, each at least four chunks long.  24 rows, us a launch without / with the pieces
+  // (and with what adds them): 4096 x 14336 82 / MEAS_A, 4096 x 4096 26 / MEAS_B, 14336 x 4096 27 / MEAS_C
+  const int chunks = (nb + GemmGeo<CRABML_HIP_Q4_0, 2>::KC - 1) / GemmGeo<CRABML_HIP_Q4_0, 2>::KC;
+  int pieces = 1;
+  if (fused_add && !dev->strict_order && ws != nullptr && m % 4 == 0)
+    while (pieces < 8 && (size_t)row_tiles * col_tiles * pieces < (size_t)dev->n_cu * 3 / 2 && chunks / (2 * pieces) >= 4 &&
+           (size_t)(2 * pieces - 1) * b * m <= ws_floats)
+      pieces *= 2;
 #define CRABML_GEMM_LAUNCH(F, N)                                                                                              \
-  launch_k(st, rec, k_gemm_mfma<F, N>, dim3(row_tiles * col_tiles), dim3(256), GemmGeo<F, N>::LDS_BYTES, wp, wd, (const char*)act, \
-           al.total, al.off_d, al.off_aux, out, (int)m, nb, (int)b, row_tiles)
+  launch_k(st, rec, k_gemm_mfma<F, N>, dim3(row_tiles * col_tiles * pieces), dim3(256), GemmGeo<F, N>::LDS_BYTES, wp, wd, (const char*)act, \
+           al.total, al.off_d, al.off_aux, out, (int)m, nb, (int)b, row_tiles, pieces, ws)
 #define CRABML_GEMM_LAUNCH_FMA(F, N)                                                                                                    \
-  launch_k(st, rec, k_gemm_mfma<F, N, true>, dim3(row_tiles * col_tiles), dim3(256), GemmGeo<F, N>::LDS_BYTES, wp, wd, (const char*)act, \
-           al.total, al.off_d, al.off_aux, out, (int)m, nb, (int)b, row_tiles)
+  launch_k(st, rec, k_gemm_mfma<F, N, true>, dim3(row_tiles * col_tiles * pieces), dim3(256), GemmGeo<F, N>::LDS_BYTES, wp, wd, (const char*)act, \
+           al.total, al.off_d, al.off_aux, out, (int)m, nb, (int)b, row_tiles, pieces, ws)
   const bool fma = fused_add && !dev->strict_order;
   if (w->dtype == CRABML_HIP_Q4_0 && fma) {
     if (narrow)
@@ -931,6 +945,10 @@ bool launch_gemm_mfma(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m,
   }
 #undef CRABML_GEMM_LAUNCH
 #undef CRABML_GEMM_LAUNCH_FMA
+  if (pieces > 1 && defer_parts != nullptr)
+    *defer_parts = pieces - 1;  // (the caller's next row kernel adds them)
+  else if (pieces > 1)
+    launch_add_parts(st, out, ws, b * m, pieces - 1);
   return true;
 }
 

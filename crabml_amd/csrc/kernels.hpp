@@ -83,7 +83,10 @@ bool launch_gemm_f16(crabml_hip_device* dev, crabml_hip_device::ProfRec* rec, co
                      const void* act, size_t act_stride, size_t rows, float* const* out, const GemmScratch& ws);
 // batched rhs on the matrix cores (gemm_mfma.hip); false = not covered
 bool launch_gemm_mfma(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m, size_t k, const void* act, size_t b, float* out,
-                      crabml_hip_device::ProfRec* rec, int* dbg = nullptr, bool fused_add = false);
+                      crabml_hip_device::ProfRec* rec, int* dbg = nullptr, bool fused_add = false, float* ws = nullptr, size_t ws_floats = 0,
+                      int* defer_parts = nullptr);  // ws, defer_parts: as launch_gemm_f16w's
+// gemm_f16w.hip: out += ws + s * n, s = 0 .. nparts - 1, element by element in that order (n % 4 == 0)
+void launch_add_parts(hipStream_t st, float* out, const float* ws, size_t n, int nparts);
 int launch_piece_ints(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m, size_t k, size_t row, const void* act, int variant,
                       int32_t* out, float* fout);
 // elementwise.hip: plain streaming read of `bytes` bytes (crabml_hip_debug_read_ceiling), timed by the event pair
