@@ -337,24 +337,27 @@ template <int NT>
 __global__ __launch_bounds__(256) void k_gemm_mfma_q4k(const i32x4* __restrict__ wq, const i32x4* __restrict__ wh,
                                                        const char* __restrict__ act, size_t act_stride, size_t off_d, size_t off_aux,
                                                        size_t off_p, float* __restrict__ out, int m, int nsb, int b, int row_tiles,
-                                                       int* __restrict__ dbg) {
+                                                       int* __restrict__ dbg, int pieces, float* __restrict__ ws) {
   using G = GemmGeoK<NT>;
   constexpr int CW = G::CW;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int i = lane & 15, g = lane >> 4;
   int rt, ct;
+  const int tiles = (int)gridDim.x / pieces, piece = (int)blockIdx.x / tiles, tile = (int)blockIdx.x % tiles;  // pieces of k: as in k_gemm_mfma
   {  // XCD-aware tile order (see k_gemm_mfma)
-    const int col_tiles = (int)gridDim.x / row_tiles;
+    const int col_tiles = tiles / row_tiles;
     if ((row_tiles & 7) == 0) {
-      const int x = (int)blockIdx.x & 7, j = (int)blockIdx.x >> 3;
+      const int x = tile & 7, j = tile >> 3;
       ct = j % col_tiles;
       rt = (j / col_tiles) * 8 + x;
     } else {
-      rt = (int)blockIdx.x % row_tiles;
-      ct = (int)blockIdx.x / row_tiles;
+      rt = tile % row_tiles;
+      ct = tile / row_tiles;
     }
   }
+  const int s_lo = nsb * piece / pieces, s_hi = nsb * (piece + 1) / pieces;
+  if (piece > 0) out = ws + (size_t)(piece - 1) * b * m;
   const int r0 = rt * 64, c0 = ct * CW;
 
   i32x4 ra[G::A_LOADS], rb[G::B_LOADS], rh, rbs;
@@ -434,12 +437,12 @@ __global__ __launch_bounds__(256) void k_gemm_mfma_q4k(const i32x4* __restrict__
 #pragma unroll
   for (int jt = 0; jt < NT; jt++) F[jt][0] = F[jt][1] = f32x2{0.0f, 0.0f};
 
-  fetch(0);
+  fetch(s_lo);
   commit(0);
   __syncthreads();
-  for (int sb = 0; sb < nsb; sb++) {
-    const int buf = sb & 1;
-    fetch(sb + 1 < nsb ? sb + 1 : sb);  // unconditional (the last one re-reads): in flight while this chunk is multiplied
+  for (int sb = s_lo; sb < s_hi; sb++) {
+    const int buf = (sb - s_lo) & 1;
+    fetch(sb + 1 < s_hi ? sb + 1 : sb);  // unconditional (the last one re-reads): in flight while this chunk is multiplied
     const unsigned* S = (const unsigned*)lds_raw + (size_t)buf * G::BUF_WORDS;
     const unsigned* arow = S + (16 * wave + i) * G::ASTR + 2 * g;
     // scales / d / dmin of the four rows this lane's accumulators belong to (rows 4g .. 4g + 3 of the wave's 16)
@@ -855,6 +858,21 @@ bool launch_gemm_mfma(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m,
   if (b < 16 || m == 0 || k % 32 != 0) return false;
   hipStream_t st = dev->stream;
   const char* wp = (const char*)w->ptr;
+  // pieces of k while the tiles leave CUs without work, each at least `least` chunks long.  24 rows, us a launch without / with the pieces:
+  // 4096 x 14336 82 / 21, 4096 x 4096 26 / 9, 1024 x 4096 26 / 7, 14336 x 4096 27 / 21, and 4.5 to add them where no row kernel does;
+  // a layer of the 8B shape 302 -> 174 (Q4_0), 300 -> 184 (Q8_0), 463 -> 219 (Q4_1), 290 -> 178 (Q4_K)
+  auto pieces_of = [&](int tiles, int chunks, int least) {
+    int n = 1;
+    if (fused_add && !dev->strict_order && ws != nullptr && m % 4 == 0)
+      while (n < 8 && (size_t)tiles * n < (size_t)dev->n_cu * 3 / 2 && chunks / (2 * n) >= least && (size_t)(2 * n - 1) * b * m <= ws_floats) n *= 2;
+    return n;
+  };
+  auto add_pieces = [&](int pieces) {
+    if (pieces > 1 && defer_parts != nullptr)
+      *defer_parts = pieces - 1;  // (the caller's next row kernel adds them)
+    else if (pieces > 1)
+      launch_add_parts(st, out, ws, b * m, pieces - 1);
+  };
   if (w->dtype == CRABML_HIP_Q8_K) {
     if (k % 256 != 0) return false;
     const ActLayout alk = act_layout(CRABML_HIP_Q8_K, k);
@@ -879,12 +897,14 @@ bool launch_gemm_mfma(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m,
     const int cwk = narrow_k ? 32 : 64, ctl = (int)((b + cwk - 1) / cwk);
     const i32x4* wqk = (const i32x4*)wp;
     const i32x4* whk = (const i32x4*)(wp + w->wl.off_scale);
+    const int pieces = dbg == nullptr ? pieces_of(rtl * ctl, nsb, 2) : 1;
     if (narrow_k)
-      launch_k(st, rec, k_gemm_mfma_q4k<2>, dim3(rtl * ctl), dim3(256), GemmGeoK<2>::LDS_BYTES, wqk, whk, (const char*)act, alk.total,
-               alk.off_d, alk.off_aux, alk.off_p, out, (int)m, nsb, (int)b, rtl, dbg);
+      launch_k(st, rec, k_gemm_mfma_q4k<2>, dim3(rtl * ctl * pieces), dim3(256), GemmGeoK<2>::LDS_BYTES, wqk, whk, (const char*)act, alk.total,
+               alk.off_d, alk.off_aux, alk.off_p, out, (int)m, nsb, (int)b, rtl, dbg, pieces, ws);
     else
-      launch_k(st, rec, k_gemm_mfma_q4k<4>, dim3(rtl * ctl), dim3(256), GemmGeoK<4>::LDS_BYTES, wqk, whk, (const char*)act, alk.total,
-               alk.off_d, alk.off_aux, alk.off_p, out, (int)m, nsb, (int)b, rtl, dbg);
+      launch_k(st, rec, k_gemm_mfma_q4k<4>, dim3(rtl * ctl * pieces), dim3(256), GemmGeoK<4>::LDS_BYTES, wqk, whk, (const char*)act, alk.total,
+               alk.off_d, alk.off_aux, alk.off_p, out, (int)m, nsb, (int)b, rtl, dbg, pieces, ws);
+    add_pieces(pieces);
     return true;
   }
   const ActLayout al = act_layout(w->dtype == CRABML_HIP_Q4_1 ? CRABML_HIP_Q8_1 : CRABML_HIP_Q8_0, k);
@@ -902,14 +922,7 @@ bool launch_gemm_mfma(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m,
   const int cw = narrow ? 32 : 64;
   const int col_tiles = (int)((b + cw - 1) / cw);
   const unsigned short* wd = (const unsigned short*)(wp + w->wl.off_scale);
-  // pieces of k while the tiles leave CUs without work, each at least four chunks long.  24 rows, us a launch without / with the pieces
-  // (and with what adds them): 4096 x 14336 82 / MEAS_A, 4096 x 4096 26 / MEAS_B, 14336 x 4096 27 / MEAS_C
-  const int chunks = (nb + GemmGeo<CRABML_HIP_Q4_0, 2>::KC - 1) / GemmGeo<CRABML_HIP_Q4_0, 2>::KC;
-  int pieces = 1;
-  if (fused_add && !dev->strict_order && ws != nullptr && m % 4 == 0)
-    while (pieces < 8 && (size_t)row_tiles * col_tiles * pieces < (size_t)dev->n_cu * 3 / 2 && chunks / (2 * pieces) >= 4 &&
-           (size_t)(2 * pieces - 1) * b * m <= ws_floats)
-      pieces *= 2;
+  const int pieces = pieces_of(row_tiles * col_tiles, (nb + GemmGeo<CRABML_HIP_Q4_0, 2>::KC - 1) / GemmGeo<CRABML_HIP_Q4_0, 2>::KC, 4);
 #define CRABML_GEMM_LAUNCH(F, N)                                                                                              \
   launch_k(st, rec, k_gemm_mfma<F, N>, dim3(row_tiles * col_tiles * pieces), dim3(256), GemmGeo<F, N>::LDS_BYTES, wp, wd, (const char*)act, \
            al.total, al.off_d, al.off_aux, out, (int)m, nb, (int)b, row_tiles, pieces, ws)
@@ -945,10 +958,7 @@ bool launch_gemm_mfma(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m,
   }
 #undef CRABML_GEMM_LAUNCH
 #undef CRABML_GEMM_LAUNCH_FMA
-  if (pieces > 1 && defer_parts != nullptr)
-    *defer_parts = pieces - 1;  // (the caller's next row kernel adds them)
-  else if (pieces > 1)
-    launch_add_parts(st, out, ws, b * m, pieces - 1);
+  add_pieces(pieces);
   return true;
 }
 

@@ -387,3 +387,21 @@ def test_fast_prompt_pass_rows_write_their_own_f16_planes(ca, fmt, shape, n):
             assert np.array_equal(la.view(np.uint32), lb.view(np.uint32)), (fmt, shape, chunk, strict)
             nxt = int(np.argmax(la))
             assert list(a.decode_greedy(nxt, 6)) == list(b.decode_greedy(nxt, 6))
+
+
+# short passes whose tiles leave CUs without work: k in 2 / 4 / 8 pieces (26 chunks of four blocks, or 13 super-blocks: pieces of unequal length;
+# an odd first chunk), rows at both ends of the range and a ragged last row tile
+@pytest.mark.parametrize("fmt", ["Q4_0", "Q8_0", "Q4_1", "Q4_K"])
+@pytest.mark.parametrize("rows", [16, 17, 31])
+def test_short_passes_in_pieces_of_k_equal_the_token_loop(ca, fmt, rows):
+    shape = synth.ModelShape("pieces", 3328, 1088 if fmt != "Q4_K" else 1280, 1, 26, 2, 300, 64, 1e-5, None)
+    dev = ca.HipTensorDevice(0)
+    conf, w = synth.to_hip(synth.build_model(shape, synth.TYPE_BY_NAME[fmt], seed=91), dev)
+    a, b = ca.HipLlamaRunner(conf, w, dev, 64, True), ca.HipLlamaRunner(conf, w, dev, 64, True)
+    toks = [(13 * i + 5) % 300 for i in range(rows)]
+    want = [b.forward(t, i) for i, t in enumerate(toks)][-1]
+    first = a.prefill(toks)
+    # the pieces are f32 sums of the same exact block terms; a level of a quantized row that falls the other way sets the bound (FAST_TOL)
+    assert np.max(np.abs(first - want)) <= FAST_TOL[fmt][1] * np.max(np.abs(want))
+    a.reset()
+    assert np.array_equal(a.prefill(toks).view(np.uint32), first.view(np.uint32))  # (added in piece order, whoever ends first)
