@@ -406,7 +406,7 @@ inline void launch_mix_step_t(hipStream_t st, crabml_hip_device::ProfRec* rec, M
   const size_t li = a.li.H ? (size_t)(2 * a.li.D + 32 * 36) * (NT / 256) : 0;
   const int units = a.B * a.li.H * a.li.slices;
   const unsigned grid = (unsigned)((a.at.H ? a.B * a.at.G * a.head_blocks * a.splits : 0) + (units + NT / 256 - 1) / (NT / 256));
-  launch_k(st, rec, k_mix_step<T, CLS, NT>, dim3(grid), dim3(NT), (at > li ? at : li) * sizeof(float), a);  // (at most 51 KiB)
+  launch_k(st, rec, k_mix_step<T, CLS, NT>, dim3(grid), dim3(NT), (at > li ? at : li) * sizeof(float), a);  // (at most 27 KiB)
 }
 template <typename T>
 inline void launch_mix_step(hipStream_t st, crabml_hip_device::ProfRec* rec, const MixStep& a) {
