@@ -378,8 +378,9 @@ int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m_, size
     if (launch_gemm_f16(dev, rec0, ws, &m_, 1, k_, act, al.total, b, &out, GemmScratch{})) return 0;
   }
   if (b >= 16 && launch_gemm_mfma(dev, w, m_, k_, act, b, out, rec0, nullptr, fused_add)) return 0;
-  for (size_t b0 = 0; b0 < b; b0 += RHS_ROWS_MAX) {
-    const size_t rows = b - b0 < RHS_ROWS_MAX ? b - b0 : RHS_ROWS_MAX;
+  const size_t per = rhs_rows_per_launch(m_);
+  for (size_t b0 = 0; b0 < b; b0 += per) {
+    const size_t rows = b - b0 < per ? b - b0 : per;
     const char* ap = (const char*)act + b0 * act_stride;
     float* o = out + b0 * m_;
     crabml_hip_device::ProfRec* rec = b0 == 0 ? rec0 : nullptr;
@@ -680,3 +681,9 @@ void launch_block_dots(hipStream_t st, const crabml_hip_buf* w, size_t k, size_t
 }
 
 }  // namespace crabml_hip
+
+extern "C" int crabml_hip_debug_rhs_rows(size_t m, size_t* rows) {
+  if (!rows || m == 0) return CRABML_HIP_BAD_INPUT;
+  *rows = crabml_hip::rhs_rows_per_launch(m);
+  return 0;
+}

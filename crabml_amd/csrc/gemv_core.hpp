@@ -68,6 +68,12 @@ struct RhsRows {
 };
 inline unsigned rhs_rows_grid(unsigned tiles, size_t rows) { return rows == 1 ? tiles : (unsigned)((tiles + 7) / 8 * 8 * rows); }
 constexpr size_t RHS_ROWS_MAX = 256;  // of one launch
+// Rows of one launch over a matrix of m rows: a launch holds fewer than 2^32 threads (of more, only a part runs), and a row kernel takes at most 64 of them
+// per row of the matrix, in workgroups of up to 256 whose number is padded to a multiple of eight (64 m + 8 * 256 threads at most).
+inline size_t rhs_rows_per_launch(size_t m) {
+  const size_t fit = 0xffffffffu / (64 * m + 8 * 256);
+  return fit < 1 ? 1 : fit < RHS_ROWS_MAX ? fit : RHS_ROWS_MAX;
+}
 template <bool ROWS>
 __device__ __forceinline__ bool rhs_row(const RhsRows& r, int* tile, int* row) {
   *tile = blockIdx.x;

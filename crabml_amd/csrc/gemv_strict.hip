@@ -737,8 +737,9 @@ int launch_gemv_strict(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m
     const char* e = getenv("CRABML_HIP_STRICT_SCALAR");
     return h && h[0] == '1' && e && e[0] == '1';
   }();
-  for (size_t b0 = 0; b0 < b; b0 += RHS_ROWS_MAX) {
-    const size_t rows = b - b0 < RHS_ROWS_MAX ? b - b0 : RHS_ROWS_MAX;
+  const size_t per = rhs_rows_per_launch(m);
+  for (size_t b0 = 0; b0 < b; b0 += per) {
+    const size_t rows = b - b0 < per ? b - b0 : per;
     const char* ap = (const char*)act + b0 * act_stride;
     float* o = out + b0 * m;
     const float* add = add_all ? add_all + b0 * m : nullptr;  // the residual rows of these batch rows

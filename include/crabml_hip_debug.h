@@ -55,6 +55,8 @@ int crabml_hip_debug_superblock_ints(crabml_hip_device_t* dev, const crabml_hip_
  * out (optional, b * m floats) receives the GEMM's f32 result. */
 int crabml_hip_debug_gemm_ints(crabml_hip_device_t* dev, const crabml_hip_buf_t* w, size_t m, size_t k,
                                const crabml_hip_buf_t* x, size_t b, int32_t* dst, float* out);
+/* Rows of the rhs that one launch of the row kernels takes over a matrix of m rows (matmul_vec without a matrix-core kernel).  Host only. */
+int crabml_hip_debug_rhs_rows(size_t m, size_t* rows);
 /* Sustained HBM read rate of this device as a plain streaming kernel reaches it (16-byte non-temporal loads over `bytes`
  * bytes, best of `reps` launches, HIP events on the device stream): the practical ceiling bench.py quotes next to the
  * 8 TB/s datasheet peak. */

@@ -28,3 +28,17 @@ def test_rows_equal_single_calls(ca, fmt, strict, m, k, rows):
     for r in picks:
         one = w.matmul_vec(ca.HipTensor.new(x[r], [k], dev)).export()
         assert np.array_equal(got[r].view(np.uint32), one.view(np.uint32)), r
+
+
+@pytest.mark.parametrize("fmt,strict,m,k", [("F32", False, 262146, 8), ("Q8_0", True, 524304, 32)])
+def test_more_threads_than_a_launch_holds(ca, fmt, strict, m, k):
+    """256 rows of the rhs on matrices whose launch would have 2^32 threads: several launches (of too large a one only a part runs)"""
+    rows = 257
+    rng = np.random.default_rng(9)
+    dev = ca.HipTensorDevice(0, False, 0, strict)
+    w = ca.HipTensor.from_cpu(synth.random_blocks(rng, m * k, synth.TYPE_BY_NAME[fmt]), [m, k], getattr(ca.GGMLType, HT[fmt]), dev)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    got = w.matmul_vec(ca.HipTensor.new(x.reshape(-1), [rows, k], dev)).export().reshape(rows, m)
+    for r in (0, 127, 254, 255, 256):
+        one = w.matmul_vec(ca.HipTensor.new(x[r], [k], dev)).export()
+        assert np.array_equal(got[r].view(np.uint32), one.view(np.uint32)), r
