@@ -2199,18 +2199,7 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
       }
       (void)hipGetLastError();
     }
-    // A head per workgroup with f32 sums (k_attn_short): from the start on the fast step of Q4_0 / Q8_0 layers, whose RMS norms leave the
-    // reference's summation order as well; elsewhere where k_attn_flash would leave it.  Us per layer of the 8B shape, k_attn_short against
-    // what ran before: 4.7 against 6.5 at 40 cached positions, 5.4 against 8.8 at 88.  Against k_attn_flash, a step and layer: 33.1 / 35.6 at
-    // 128, 34.1 / 36.0 at 256, 35.4 / 36.3 at 384, 36.4 / 36.3 at 512, 38.3 / 36.9 at 768 (16 / 4 heads x 128: even at 600; 32 / 32 x 64:
-    // at 1000) -- one workgroup reads a head's rows at a CU's rate.  A caller's own attn_long_from is the long kernels' from there on.
-    if (g.use_f16_kv_cache && hd % 8 == 0 && hd <= 256 && !dev->strict_order &&
-        !(g.flags & (CRABML_HIP_LLAMA_EXACT_ATTENTION | CRABML_HIP_LLAMA_NO_LONG_ATTENTION | CRABML_HIP_LLAMA_NO_STAGED_ATTENTION))) {
-      const bool flash = c->attn_flash && g.attn_long_from == 0;
-      c->attn_short_from = wt == CRABML_HIP_Q4_0 || wt == CRABML_HIP_Q8_0 ? 0 : flash ? c->attn_long_from : SIZE_MAX;
-      c->attn_short_until = flash ? 512 : c->attn_long_ok ? c->attn_long_from : SIZE_MAX;
-    }
-    // everything else: K / V staged through LDS, the reference's bits; variant 0 serves positions < S
+    // K / V staged through LDS, the reference's bits: variant 0 serves positions < S (where k_attn_short does not)
     if (g.use_f16_kv_cache && hd % 8 == 0 && !(g.flags & CRABML_HIP_LLAMA_NO_STAGED_ATTENTION)) {
       const size_t S = c->attn_long_ok && c->attn_long_from < g.seq_len ? c->attn_long_from : g.seq_len;
       const size_t lds = attn_s_lds_bytes((int)S, (int)hd);
@@ -2236,6 +2225,20 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
   c->defer_norm = c->norm_epi && tp == 1 && !ord && !dev->strict_order && (wt == CRABML_HIP_Q4_0 || wt == CRABML_HIP_Q8_0) &&
                   !(g.flags & CRABML_HIP_LLAMA_EXACT_NORM) && (int)(g.embedding_dim / 32) <= dev->n_cu;
   if (c->defer_norm) A(g.embedding_dim / 16 * 4, (void**)&c->rsums);
+  // A head per workgroup with f32 sums (k_attn_short): from the start where the fast step of Q4_0 / Q8_0 layers leaves the reference's summation
+  // order as well (deferred norms; a tensor-parallel rank's wo and ffn_down, whose group adds them up) and no flag asks for more of it;
+  // elsewhere where k_attn_flash would leave it.  Us per layer of the 8B shape, k_attn_short against what ran before: 4.7 against 6.5 at 40
+  // cached positions, 5.4 against 8.8 at 88.  Against k_attn_flash, a step and layer: 33.1 / 35.6 at 128, 34.1 / 36.0 at 256, 35.4 / 36.3 at
+  // 384, 36.4 / 36.3 at 512, 38.3 / 36.9 at 768 (16 / 4 heads x 128: even at 600; 32 / 32 x 64: at 1000) -- one workgroup reads a head's
+  // rows at a CU's rate.  A caller's own attn_long_from is the long kernels' from there on.
+  if (g.use_f16_kv_cache && hd % 8 == 0 && hd <= 256 && !dev->strict_order &&
+      !(g.flags & (CRABML_HIP_LLAMA_EXACT_ATTENTION | CRABML_HIP_LLAMA_NO_LONG_ATTENTION | CRABML_HIP_LLAMA_NO_STAGED_ATTENTION))) {
+    const bool flash = c->attn_flash && g.attn_long_from == 0;
+    const bool own_order = c->defer_norm || (tp > 1 && !generic && (wt == CRABML_HIP_Q4_0 || wt == CRABML_HIP_Q8_0) &&
+                                             !(g.flags & (CRABML_HIP_LLAMA_EXACT_NORM | CRABML_HIP_LLAMA_NO_NORM_EPILOGUE)));
+    c->attn_short_from = own_order ? 0 : flash ? c->attn_long_from : SIZE_MAX;
+    c->attn_short_until = flash ? 512 : c->attn_long_ok ? c->attn_long_from : SIZE_MAX;
+  }
   // A tensor-parallel rank's gate/up: hidden / tp / 32 workgroups of 32 rows would leave most CUs idle.  h stays f32 from workgroups
   // of `gu_rows` rows (the largest even divisor of the rank's rows, at most 32, that gives at least one workgroup per CU) and
   // ffn_down quantizes it in its prologue.

@@ -210,7 +210,7 @@ typedef struct crabml_hip_llama crabml_hip_llama_t;
 #define CRABML_HIP_LLAMA_NO_PREFETCH 2 /* do not warm the Infinity Cache from the latency-bound stages */
 #define CRABML_HIP_LLAMA_TP_GRAPH 8 /* tp_size > 1: capture the RCCL all-reduces into the hipGraph as well
                                        (default for tp: eager launches; falls back to eager if capture fails) */
-#define CRABML_HIP_LLAMA_EXACT_ATTENTION 4194304 /* fast mode, from attn_long_from cached positions (Q4_0 / Q8_0 layers: from the first): keep the reference's serial
+#define CRABML_HIP_LLAMA_EXACT_ATTENTION 4194304 /* fast mode, wherever attention would run with f32 sums (attn_long_from): keep the reference's serial
                                           f16-accumulated PV chain (buf_f16.rs:152-163) instead of the split-KV kernels that
                                           accumulate the same f16 products in f32 (DESIGN.md 2.2 states the deviation and its
                                           measured size).  Strict-order devices always run the exact chain. */
@@ -242,7 +242,7 @@ typedef struct crabml_hip_llama_config { /* crabml-llama2/src/model.rs:30-53 */
   void* tp_comm; /* crabml_hip_tp_comm_t*; NULL with tp_size > 1 = a rank of the single-device simulation */
   size_t attn_long_from; /* cached positions from which attention runs as the multi-workgroup kernels (0 = default: 224 for the
                           * exact kernels; fast step: 512 for the split-KV kernels, the one-workgroup kernel with f32 sums from 96, with
-                          * Q4_0 / Q8_0 layers from the first) */
+                          * Q4_0 / Q8_0 layers from the first unless their norms are asked for, or run, in the reference's order) */
   size_t prefill_chunk;  /* rows per batched prefill pass (0 = default: 1024, 512 on a strict-order device; never more than seq_len) */
 } crabml_hip_llama_config_t;
 typedef struct crabml_hip_llama_weights { /* crabml-llama2/src/model.rs:55-84; per-layer arrays of n_layers */

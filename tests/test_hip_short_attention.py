@@ -80,3 +80,23 @@ def test_step_across_the_switches(ca, fmt):
             assert np.array_equal(got.view(np.uint32), exact.view(np.uint32)), i
         errs.append(np.max(np.abs(got - exact)) / np.max(np.abs(exact)))
     assert max(errs) <= 7.5e-2, errs  # (the widest of the long kernels' bounds, helpers.FAST_TOL: a flipped level of the quantized row)
+
+
+@pytest.mark.parametrize("fmt", ["Q4_0", "Q8_0"])
+@pytest.mark.parametrize("asked", ["exact norm", "norms apart", "mixed layers"])
+def test_steps_that_keep_the_norms_order_keep_the_attentions(ca, fmt, asked):
+    """below 96 cached positions a Q4_0 / Q8_0 step leaves the reference's f16 chain only together with its norms' order: with the norm's
+    division kept in its launch, with norms as launches of their own, and over files whose layers mix formats, EXACT_ATTENTION changes no bit"""
+    model = synth.build_model(synth.SHAPES["tiny-gqa"], synth.TYPE_BY_NAME[fmt], seed=31)
+    if asked == "mixed layers":
+        t = model.tensors["blk.0.attn_v.weight"]
+        t.typ = synth.Q8_0 if fmt == "Q4_0" else synth.Q4_0
+        t.data = synth.random_blocks(np.random.default_rng(1), t.shape[0] * t.shape[1], t.typ)
+    kw, flags = dict(norm_epilogue=asked != "norms apart"), 8388608 if asked == "exact norm" else 0  # CRABML_HIP_LLAMA_EXACT_NORM
+    dev = ca.HipTensorDevice(0)
+    conf, w = synth.to_hip(model, dev)
+    a = ca.HipLlamaRunner(conf, w, dev, 128, True, extra_flags=flags, **kw)
+    b = ca.HipLlamaRunner(conf, w, dev, 128, True, extra_flags=flags + EXACT, **kw)
+    for i in range(95):
+        la, lb = a.forward((7 * i + 3) % 1000, i), b.forward((7 * i + 3) % 1000, i)
+        assert np.array_equal(la.view(np.uint32), lb.view(np.uint32)), i
