@@ -2304,8 +2304,9 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
   const bool want_graph = !(g.flags & CRABML_HIP_LLAMA_NO_GRAPH) &&
                           (tp == 1 || c->tp_dry || p2p_comm || (c->comm != nullptr && (g.flags & CRABML_HIP_LLAMA_TP_GRAPH)));
   if (want_graph) {
-    const bool has[4] = {true, c->attn_long_ok, c->attn_long_ok && c->flash_ticket_until > 0,
-                         c->attn_short_from > 0 && c->attn_short_from < g.seq_len};
+    bool has[4] = {};  // the forms that some position of this context runs (variant_of changes at these numbers of cached positions only)
+    for (size_t n : {(size_t)1, c->attn_short_from, c->attn_short_until, c->attn_long_from, c->flash_ticket_until})
+      if (n >= 1 && n <= g.seq_len) has[variant_of(c, n - 1)] = true;
     bool ok = true;
     for (int v = 0; v < 4 && ok; v++) {
       if (!has[v]) continue;
@@ -2537,7 +2538,15 @@ int crabml_hip_llama_debug_kv(crabml_hip_llama_t* c, size_t layer, int32_t which
   return 0;
 }
 
-// parity hook (crabml_hip_debug.h): k_attn_flash by itself, on caller-supplied q / K / V
+int crabml_hip_llama_debug_graphs(crabml_hip_llama_t* c, size_t pos, int32_t* form, uint32_t* captured) {
+  if (!c || !form || !captured || pos >= c->cfg.seq_len) return CRABML_HIP_BAD_INPUT;
+  *form = variant_of(c, pos);
+  *captured = 0;
+  for (int v = 0; v < 4; v++) *captured |= c->exec[v] ? 1u << v : 0u;
+  return 0;
+}
+
+// parity hook (crabml_hip_debug.h): k_attn_short by itself, on caller-supplied q / K / V
 int crabml_hip_debug_short_attention(crabml_hip_device_t* dev, const float* q, const uint16_t* k, const uint16_t* v, size_t n_heads,
                                      size_t n_kv, size_t head_dim, size_t seq, size_t seq_cap, float* out) {
   if (!dev || !q || !k || !v || !out || seq == 0 || seq > seq_cap || seq_cap > (1u << 24) || n_kv == 0 || n_heads == 0 || n_heads % n_kv != 0 || n_heads > 4096 ||
@@ -2570,6 +2579,7 @@ int crabml_hip_debug_short_attention(crabml_hip_device_t* dev, const float* q, c
   return 0;
 }
 
+// ... and k_attn_flash
 int crabml_hip_debug_flash_attention(crabml_hip_device_t* dev, const float* q, const uint16_t* k, const uint16_t* v, size_t n_heads,
                                      size_t n_kv, size_t head_dim, size_t seq, size_t slices, float* out, float* out2) {
   if (!dev || !q || !k || !v || !out || seq == 0 || n_kv == 0 || n_heads % n_kv != 0) return CRABML_HIP_BAD_INPUT;
@@ -2739,7 +2749,7 @@ int lazy_ctx_segment(crabml_hip_llama* c, int seg) {
 }
 
 // the whole step at once: the context's captured graph (false: this context has none -- the caller enqueues segment by segment)
-bool lazy_ctx_has_graph(const crabml_hip_llama* c) { return !c->dev->dry && c->use_graph && c->exec[0] != nullptr; }
+bool lazy_ctx_has_graph(const crabml_hip_llama* c) { return !c->dev->dry && c->use_graph; }
 int lazy_ctx_step(crabml_hip_llama* c, size_t pos) {
   if (c->dev->dry) return 0;
   return run_step(c, pos);

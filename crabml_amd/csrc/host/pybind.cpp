@@ -461,6 +461,16 @@ PYBIND11_MODULE(_host, m) {
                     return py::array_t<float>(lg.size(), lg.data());
                   })
       .def("forward_async", &HipLlamaRunner::forward_async)
+      .def("debug_graphs",  // (form at pos, [captured forms])
+           [](HipLlamaRunner& r, size_t pos) {
+             int32_t form = 0;
+             uint32_t captured = 0;
+             r.device()->check(crabml_hip_llama_debug_graphs(r.raw(), pos, &form, &captured));
+             py::list forms;
+             for (int v = 0; v < 4; v++)
+               if (captured >> v & 1) forms.append(v);
+             return py::make_tuple(form, forms);
+           })
       .def("debug_kv", [](HipLlamaRunner& r, size_t layer, bool v, bool f16) {
         std::vector<uint8_t> b = r.debug_kv(layer, v, f16);
         return py::array_t<uint8_t>(b.size(), b.data());

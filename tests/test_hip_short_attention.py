@@ -100,3 +100,16 @@ def test_steps_that_keep_the_norms_order_keep_the_attentions(ca, fmt, asked):
     for i in range(95):
         la, lb = a.forward((7 * i + 3) % 1000, i), b.forward((7 * i + 3) % 1000, i)
         assert np.array_equal(la.view(np.uint32), lb.view(np.uint32)), i
+
+
+@pytest.mark.parametrize("fmt", ["Q4_0", "Q4_K", "F16"])
+@pytest.mark.parametrize("shape,seq,long_from", [("tiny-hd128", 64, 0), ("tiny-hd128", 300, 0), ("tiny-hd128", 513, 0), ("tiny-hd128", 1000, 0),
+                                                 ("tiny-hd128", 1000, 1), ("tiny-hd128", 400, 500), ("15m", 600, 0)])
+def test_a_context_captures_the_steps_that_its_positions_run(ca, fmt, shape, seq, long_from):
+    """one graph for every attention form between the first and the last cache position, and none that nothing replays"""
+    if fmt == "Q4_K" and shape == "15m":
+        pytest.skip("width 288 is not whole super-blocks")
+    dev = ca.HipTensorDevice(0)
+    conf, w = synth.to_hip(synth.build_model(synth.SHAPES[shape], synth.TYPE_BY_NAME[fmt], seed=2), dev)
+    r = ca.HipLlamaRunner(conf, w, dev, seq, True, attn_long_from=long_from)
+    assert sorted({r.debug_graphs(p)[0] for p in range(seq)}) == r.debug_graphs(0)[1]
