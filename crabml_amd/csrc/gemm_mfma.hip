@@ -45,17 +45,18 @@ struct GemmGeo {
   static constexpr int A_LOADS = 64 * KC * APC / 256, B_LOADS = CW * KC * 2 / 256, S_LOADS = 64 * KC / 256;
 };
 
-// FMA (the fast prompt pass only, crabml_hip_llama_prefill): sumf = fma(sumi as f32 * d_w, d_x, sumf) -- the block term's second
-// product and the add as one v_pk_fma_f32 (8 instead of 10 VALU operations per MFMA; one rounding fewer than the reference's
+// PASS: the fast prompt pass (crabml_hip_llama_prefill).  Its Q4_0 / Q8_0 sums are sumf = fma(sumi as f32 * d_w, d_x, sumf) -- the block term's
+// second product and the add as one v_pk_fma_f32 (8 instead of 10 VALU operations per MFMA; one rounding fewer than the reference's
 // expression, the same distance the fast decode step's re-associated sums are allowed).  matmul_vec itself and the strict-order
 // device keep the reference's three roundings (bit-exact, tests/test_hip_gemv.py).
-// pieces > 1 (the fast prompt pass only): that many workgroups per tile, each over its chunks of k; piece s >= 1 leaves its sums in
-// ws + (s - 1) b m, added in piece order behind (a short pass has few tiles: 64 workgroups and a chain of nb / KC chunks otherwise)
-template <int FMT, int NT, bool FMA = false>
+// Its k may be cut into gridDim.y pieces (a power of two): that many workgroups per tile, each over its chunks; piece s >= 1 leaves its sums
+// in ws + (s - 1) b m, added in piece order behind (a short pass has few tiles: 64 workgroups and a chain of nb / KC chunks otherwise).
+// matmul_vec's instantiation knows nothing of pieces: with them -- a branch and moved operands in front of the first request -- its
+// launches took 0.3 to 1.5 us more (Q8_0, 24 rows: 1024 x 2048 15.9 -> 16.4, 4096 x 14336 87.4 -> 90.4).
+template <int FMT, int NT, bool PASS = false>
 __global__ __launch_bounds__(256) void k_gemm_mfma(const char* __restrict__ wq, const unsigned short* __restrict__ wd,
                                                    const char* __restrict__ act, size_t act_stride, size_t off_d, size_t off_aux,
-                                                   float* __restrict__ out, int m, int nb, int b, int row_tiles, int pieces,
-                                                   float* __restrict__ ws) {
+                                                   float* __restrict__ out, int m, int nb, int b, int row_tiles, float* __restrict__ ws) {
   using G = GemmGeo<FMT, NT>;
   constexpr int KC = G::KC, APC = G::APC, ARW = G::ARW, BRW = G::BRW, CW = G::CW;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
@@ -65,19 +66,30 @@ __global__ __launch_bounds__(256) void k_gemm_mfma(const char* __restrict__ wq, 
   // 35 MB gate/up GEMM with column-major tile order).  XCD x owns the row tiles rt = x (mod 8); its j-th workgroup
   // is (rt = 8 (j / col_tiles) + x, ct = j % col_tiles).  The activation tiles (8 x 295 KB) stay L2-resident.
   int rt, ct;
-  const int tiles = (int)gridDim.x / pieces, piece = (int)blockIdx.x / tiles, tile = (int)blockIdx.x % tiles;
   {
-    const int col_tiles = tiles / row_tiles;
+    const int col_tiles = (int)gridDim.x / row_tiles;
     if ((row_tiles & 7) == 0) {
-      const int x = tile & 7, j = tile >> 3;
+      const int x = (int)blockIdx.x & 7, j = (int)blockIdx.x >> 3;
       ct = j % col_tiles;
       rt = (j / col_tiles) * 8 + x;
     } else {
-      rt = tile % row_tiles;
-      ct = tile / row_tiles;
+      rt = (int)blockIdx.x % row_tiles;
+      ct = (int)blockIdx.x / row_tiles;
     }
   }
-  if (piece > 0) out = ws + (size_t)(piece - 1) * b * m;
+  // this piece's chunks; below, wq / wd / act begin at its first block and it has `left` blocks of a row's nb in front of it
+  int nchunks = (nb + KC - 1) / KC, left = nb;
+  if constexpr (PASS) {
+    const int piece = (int)blockIdx.y, lg = __builtin_ctz(gridDim.y), c_lo = nchunks * piece >> lg;
+    nchunks = (nchunks * (piece + 1) >> lg) - c_lo;
+    left -= c_lo * KC;
+    if (piece > 0) out = ws + (size_t)(piece - 1) * b * m;
+    wq += (size_t)c_lo * KC * APC * 16;
+    wd += (size_t)c_lo * KC * (FMT == CRABML_HIP_Q4_1 ? 2 : 1);
+    act += (size_t)c_lo * KC * 32;  // 32 bytes of levels a block, 2 of a scale
+    off_d -= (size_t)c_lo * KC * 30;
+    off_aux -= (size_t)c_lo * KC * 30;
+  }
   const int r0 = rt * 64, c0 = ct * CW;
   const int i = lane & 15, g = lane >> 4;
 
@@ -99,21 +111,21 @@ __global__ __launch_bounds__(256) void k_gemm_mfma(const char* __restrict__ wq, 
     for (int u = 0; u < G::A_LOADS; u++) {
       const int t = tid + 256 * u, row = t / (KC * APC), rem = t % (KC * APC), kb = rem / APC, pc = rem % APC;
       const int grow = r0 + row < m ? r0 + row : m - 1;
-      const int gkb = kb0 + kb < nb ? kb0 + kb : nb - 1;  // the tail chunk re-reads the last block (never consumed)
+      const int gkb = kb0 + kb < left ? kb0 + kb : left - 1;  // the tail chunk re-reads the last block (never consumed)
       ra[u] = __builtin_nontemporal_load((const i32x4*)wq + ((size_t)grow * nb + gkb) * APC + pc);
     }
 #pragma unroll
     for (int u = 0; u < G::B_LOADS; u++) {
       const int t = tid + 256 * u, col = t / (KC * 2), rem = t % (KC * 2), kb = rem / 2, pc = rem % 2;
       const int gcol = c0 + col < b ? c0 + col : b - 1;
-      const int gkb = kb0 + kb < nb ? kb0 + kb : nb - 1;
+      const int gkb = kb0 + kb < left ? kb0 + kb : left - 1;
       rb[u] = *((const i32x4*)(act + (size_t)gcol * act_stride) + (size_t)gkb * 2 + pc);
     }
 #pragma unroll
     for (int u = 0; u < G::S_LOADS; u++) {
       const int t = tid + 256 * u, rc = t / KC, kb = t % KC;
       const int grow = r0 + rc < m ? r0 + rc : m - 1, gcol = c0 + rc < b ? c0 + rc : b - 1;
-      const int gkb = kb0 + kb < nb ? kb0 + kb : nb - 1;
+      const int gkb = kb0 + kb < left ? kb0 + kb : left - 1;
       const char* ap = act + (size_t)gcol * act_stride;
       if constexpr (FMT == CRABML_HIP_Q4_1) {
         rad[u] = ((const unsigned*)wd)[(size_t)grow * nb + gkb];
@@ -182,16 +194,15 @@ __global__ __launch_bounds__(256) void k_gemm_mfma(const char* __restrict__ wq, 
   using S0 = std::integral_constant<int, 0>;
   using S1 = std::integral_constant<int, 1>;
   using S2 = std::integral_constant<int, 2>;
-  const int all = (nb + KC - 1) / KC, c_lo = all * piece / pieces, nchunks = all * (piece + 1) / pieces - c_lo;
   // every fetch / commit below is unconditional (chunk indices past the end are clamped: they re-read the last
   // chunk and are never multiplied): with a fixed number of loads per iteration the compiler's s_waitcnt vmcnt(n)
   // before a commit waits for exactly the loads of that chunk; with conditional fetches it fell back to waiting
   // for everything in flight, i.e. one HBM round trip per chunk
-  const int first = c_lo * KC, last = (c_lo + nchunks - 1) * KC;
-  fetch(S0{}, first);
+  const int last = (nchunks - 1) * KC;
+  fetch(S0{}, 0);
   commit(S0{}, 0);
-  fetch(S1{}, first + KC < last ? first + KC : last);
-  if constexpr (PF == 3) fetch(S2{}, first + 2 * KC < last ? first + 2 * KC : last);
+  fetch(S1{}, KC < last ? KC : last);
+  if constexpr (PF == 3) fetch(S2{}, 2 * KC < last ? 2 * KC : last);
   __syncthreads();
   // per-lane LDS offsets (words), constant over the k loop: the block index only adds immediates
   const int a_off = (16 * wave + i) * ARW + ((FMT == CRABML_HIP_Q4_0 || FMT == CRABML_HIP_Q4_1) ? g : 2 * g);
@@ -199,9 +210,9 @@ __global__ __launch_bounds__(256) void k_gemm_mfma(const char* __restrict__ wq, 
   // iteration c: request chunk c + PF into the set chunk c used, multiply chunk c (LDS buffer c & 1), commit chunk
   // c + 1 (requested two iterations ago) to the other buffer, barrier
   auto step = [&](auto SET_C, auto SET_N, int c) {
-    const int kb0 = first + c * KC, buf = c & 1;
-    const int kc = c >= nchunks ? 0 : nb - kb0 < KC ? nb - kb0 : KC;
-    fetch(SET_C, first + (c + PF) * KC < last ? first + (c + PF) * KC : last);
+    const int kb0 = c * KC, buf = c & 1;
+    const int kc = c >= nchunks ? 0 : left - kb0 < KC ? left - kb0 : KC;
+    fetch(SET_C, (c + PF) * KC < last ? (c + PF) * KC : last);
     const unsigned* sA = (const unsigned*)(lds_raw + (size_t)buf * G::BUF_BYTES);
     const unsigned* sB = sA + G::A_WORDS;
     const float* sAd = (const float*)(sB + G::B_WORDS);
@@ -270,7 +281,7 @@ __global__ __launch_bounds__(256) void k_gemm_mfma(const char* __restrict__ wq, 
       for (int jt = 0; jt < NT; jt++) {
         const f32x2 c01 = {(float)D[jt][0], (float)D[jt][1]}, c23 = {(float)D[jt][2], (float)D[jt][3]};
         const f32x2 dxx = {dx[jt], dx[jt]};
-        if constexpr (FMA) {
+        if constexpr (PASS) {
           F[jt][0] = __builtin_elementwise_fma(c01 * dw01, dxx, F[jt][0]);
           F[jt][1] = __builtin_elementwise_fma(c23 * dw23, dxx, F[jt][1]);
         } else {
@@ -337,26 +348,26 @@ template <int NT>
 __global__ __launch_bounds__(256) void k_gemm_mfma_q4k(const i32x4* __restrict__ wq, const i32x4* __restrict__ wh,
                                                        const char* __restrict__ act, size_t act_stride, size_t off_d, size_t off_aux,
                                                        size_t off_p, float* __restrict__ out, int m, int nsb, int b, int row_tiles,
-                                                       int* __restrict__ dbg, int pieces, float* __restrict__ ws) {
+                                                       int* __restrict__ dbg, float* __restrict__ ws) {
   using G = GemmGeoK<NT>;
   constexpr int CW = G::CW;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int i = lane & 15, g = lane >> 4;
   int rt, ct;
-  const int tiles = (int)gridDim.x / pieces, piece = (int)blockIdx.x / tiles, tile = (int)blockIdx.x % tiles;  // pieces of k: as in k_gemm_mfma
+  const int piece = (int)blockIdx.y;  // pieces of k: as in k_gemm_mfma
   {  // XCD-aware tile order (see k_gemm_mfma)
-    const int col_tiles = tiles / row_tiles;
+    const int col_tiles = (int)gridDim.x / row_tiles;
     if ((row_tiles & 7) == 0) {
-      const int x = tile & 7, j = tile >> 3;
+      const int x = (int)blockIdx.x & 7, j = (int)blockIdx.x >> 3;
       ct = j % col_tiles;
       rt = (j / col_tiles) * 8 + x;
     } else {
-      rt = tile % row_tiles;
-      ct = tile / row_tiles;
+      rt = (int)blockIdx.x % row_tiles;
+      ct = (int)blockIdx.x / row_tiles;
     }
   }
-  const int s_lo = nsb * piece / pieces, s_hi = nsb * (piece + 1) / pieces;
+  const int lg = __builtin_ctz(gridDim.y), s_lo = nsb * piece >> lg, s_hi = nsb * (piece + 1) >> lg;
   if (piece > 0) out = ws + (size_t)(piece - 1) * b * m;
   const int r0 = rt * 64, c0 = ct * CW;
 
@@ -899,11 +910,11 @@ bool launch_gemm_mfma(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m,
     const i32x4* whk = (const i32x4*)(wp + w->wl.off_scale);
     const int pieces = dbg == nullptr ? pieces_of(rtl * ctl, nsb, 2) : 1;
     if (narrow_k)
-      launch_k(st, rec, k_gemm_mfma_q4k<2>, dim3(rtl * ctl * pieces), dim3(256), GemmGeoK<2>::LDS_BYTES, wqk, whk, (const char*)act, alk.total,
-               alk.off_d, alk.off_aux, alk.off_p, out, (int)m, nsb, (int)b, rtl, dbg, pieces, ws);
+      launch_k(st, rec, k_gemm_mfma_q4k<2>, dim3(rtl * ctl, pieces), dim3(256), GemmGeoK<2>::LDS_BYTES, wqk, whk, (const char*)act, alk.total,
+               alk.off_d, alk.off_aux, alk.off_p, out, (int)m, nsb, (int)b, rtl, dbg, ws);
     else
-      launch_k(st, rec, k_gemm_mfma_q4k<4>, dim3(rtl * ctl * pieces), dim3(256), GemmGeoK<4>::LDS_BYTES, wqk, whk, (const char*)act, alk.total,
-               alk.off_d, alk.off_aux, alk.off_p, out, (int)m, nsb, (int)b, rtl, dbg, pieces, ws);
+      launch_k(st, rec, k_gemm_mfma_q4k<4>, dim3(rtl * ctl, pieces), dim3(256), GemmGeoK<4>::LDS_BYTES, wqk, whk, (const char*)act, alk.total,
+               alk.off_d, alk.off_aux, alk.off_p, out, (int)m, nsb, (int)b, rtl, dbg, ws);
     add_pieces(pieces);
     return true;
   }
@@ -924,27 +935,32 @@ bool launch_gemm_mfma(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m,
   const unsigned short* wd = (const unsigned short*)(wp + w->wl.off_scale);
   const int pieces = pieces_of(row_tiles * col_tiles, (nb + GemmGeo<CRABML_HIP_Q4_0, 2>::KC - 1) / GemmGeo<CRABML_HIP_Q4_0, 2>::KC, 4);
 #define CRABML_GEMM_LAUNCH(F, N)                                                                                              \
-  launch_k(st, rec, k_gemm_mfma<F, N>, dim3(row_tiles * col_tiles * pieces), dim3(256), GemmGeo<F, N>::LDS_BYTES, wp, wd, (const char*)act, \
-           al.total, al.off_d, al.off_aux, out, (int)m, nb, (int)b, row_tiles, pieces, ws)
-#define CRABML_GEMM_LAUNCH_FMA(F, N)                                                                                                    \
-  launch_k(st, rec, k_gemm_mfma<F, N, true>, dim3(row_tiles * col_tiles * pieces), dim3(256), GemmGeo<F, N>::LDS_BYTES, wp, wd, (const char*)act, \
-           al.total, al.off_d, al.off_aux, out, (int)m, nb, (int)b, row_tiles, pieces, ws)
-  const bool fma = fused_add && !dev->strict_order;
-  if (w->dtype == CRABML_HIP_Q4_0 && fma) {
+  launch_k(st, rec, k_gemm_mfma<F, N>, dim3(row_tiles * col_tiles), dim3(256), GemmGeo<F, N>::LDS_BYTES, wp, wd, (const char*)act, \
+           al.total, al.off_d, al.off_aux, out, (int)m, nb, (int)b, row_tiles, ws)
+#define CRABML_GEMM_LAUNCH_PASS(F, N)                                                                                                    \
+  launch_k(st, rec, k_gemm_mfma<F, N, true>, dim3(row_tiles * col_tiles, pieces), dim3(256), GemmGeo<F, N>::LDS_BYTES, wp, wd, (const char*)act, \
+           al.total, al.off_d, al.off_aux, out, (int)m, nb, (int)b, row_tiles, ws)
+  const bool pass = fused_add && !dev->strict_order;
+  if (w->dtype == CRABML_HIP_Q4_0 && pass) {
     if (narrow)
-      CRABML_GEMM_LAUNCH_FMA(CRABML_HIP_Q4_0, 2);
+      CRABML_GEMM_LAUNCH_PASS(CRABML_HIP_Q4_0, 2);
     else
-      CRABML_GEMM_LAUNCH_FMA(CRABML_HIP_Q4_0, 4);
-  } else if (w->dtype == CRABML_HIP_Q8_0 && fma) {
+      CRABML_GEMM_LAUNCH_PASS(CRABML_HIP_Q4_0, 4);
+  } else if (w->dtype == CRABML_HIP_Q8_0 && pass) {
     if (narrow)
-      CRABML_GEMM_LAUNCH_FMA(CRABML_HIP_Q8_0, 2);
+      CRABML_GEMM_LAUNCH_PASS(CRABML_HIP_Q8_0, 2);
     else
-      CRABML_GEMM_LAUNCH_FMA(CRABML_HIP_Q8_0, 4);
+      CRABML_GEMM_LAUNCH_PASS(CRABML_HIP_Q8_0, 4);
   } else if (w->dtype == CRABML_HIP_Q4_0) {
     if (narrow)
       CRABML_GEMM_LAUNCH(CRABML_HIP_Q4_0, 2);
     else
       CRABML_GEMM_LAUNCH(CRABML_HIP_Q4_0, 4);
+  } else if (w->dtype == CRABML_HIP_Q4_1 && pass) {
+    if (narrow)
+      CRABML_GEMM_LAUNCH_PASS(CRABML_HIP_Q4_1, 2);
+    else
+      CRABML_GEMM_LAUNCH_PASS(CRABML_HIP_Q4_1, 4);
   } else if (w->dtype == CRABML_HIP_Q4_1) {
     if (narrow)
       CRABML_GEMM_LAUNCH(CRABML_HIP_Q4_1, 2);
@@ -957,7 +973,7 @@ bool launch_gemm_mfma(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m,
       CRABML_GEMM_LAUNCH(CRABML_HIP_Q8_0, 4);
   }
 #undef CRABML_GEMM_LAUNCH
-#undef CRABML_GEMM_LAUNCH_FMA
+#undef CRABML_GEMM_LAUNCH_PASS
   add_pieces(pieces);
   return true;
 }
