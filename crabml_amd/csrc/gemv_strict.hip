@@ -802,8 +802,16 @@ int launch_gemv_strict(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m
         default: done = false;
       }
     }
-    if (!done)
-      STRICT_LAUNCH((k_gemv_strict<>), (k_gemv_strict<true>), (unsigned)((m + 63) / 64), 64, 0, wp, (int)w->dtype, w->wl.off_scale, ap, al.off_d, al.off_aux, o, add, (int)m, (int)k);
+    if (!done) {
+      // a lane per row of the matrix: a wave works on 64 cache lines at a time, and a CU's 32 KB of vector L1 hold four waves' (32000 x 2048 of F16, us a
+      // rhs row: 198 with two waves a CU, 154 with four, 269 with six; 4096 x 4096: 24 / 37 / 64 with two / four / six)
+      const size_t wgs = (m + 63) / 64, fit = 4 * (size_t)dev->n_cu / wgs, most = fit < 1 ? 1 : fit, all = rows;
+      for (size_t r0 = 0; r0 < all; r0 += most) {
+        const size_t rows = all - r0 < most ? all - r0 : most;
+        STRICT_LAUNCH((k_gemv_strict<>), (k_gemv_strict<true>), (unsigned)wgs, 64, 0, wp, (int)w->dtype, w->wl.off_scale, ap + r0 * act_stride, al.off_d, al.off_aux,
+                      o + r0 * m, add ? add + r0 * m : add, (int)m, (int)k);
+      }
+    }
   }
   return 0;
 }
