@@ -1,5 +1,5 @@
-// gemm_f16.hip -- f16 rows x f16 weights on the matrix cores: the linears of a prompt pass and matmul_vec's batched rhs where the weights
-// are F16 (fast device; buf_f16.rs:83-97: the rhs is rounded to f16, products are exact in f32, sums are f32).
+// gemm_f16.hip -- f16 rows x f16 weights on the matrix cores: the linears of a prompt pass and matmul_vec's batched rhs of many results where
+// the weights are F16 (fast device; buf_f16.rs:83-97: the rhs is rounded to f16, products are exact in f32, sums are f32).
 //
 //   out[m][row][n] = sum_k a[row][k] w[m][n][k]     up to three matrices of one rhs (q | k | v, gate | up) in one launch
 //
@@ -8,8 +8,8 @@
 // again (its results are not stored), a 16-byte piece past the end of k is a piece of zeros.  Weights are the first operand, so that a
 // lane's four results are neighbouring columns of one row and leave as one 16-byte store, without a way through LDS.
 //
-// Measured (203 rows, width 2048, ff 8192, one layer): q | k | v 16.6 us, wo 16.0, gate | up 31.8, ff_down 28.5 (480 TFLOP/s where the
-// launch fills the chip); before, a launch of the row kernel per row and matrix: 21.3 ms a layer.
+// Measured (203 rows, width 2048, ff 8192, one layer): q | k | v 16.6 us, wo 16.0, gate | up 31.8, ff_down 28.5 (430 TFLOP/s in the
+// gate | up launch); before, a launch of the row kernel per row and matrix: 21.3 ms a layer.
 #include "gemm_bf16.hpp"
 
 namespace crabml_hip {

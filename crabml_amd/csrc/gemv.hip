@@ -373,7 +373,11 @@ int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m_, size
     launch_gemv_bf16<GEMV_IN_PLAIN, GEMV_OUT_STORE>(st, rec0, g);
     return 0;
   }
-  if (w->dtype == CRABML_HIP_F16 && b >= 2) {
+  // F16 on the matrix cores: without scratch k stays whole, 0.41 us a step of 64 whatever the launch, while a row of the rhs costs the row
+  // kernels their weights from L2 (16 TB/s).  Both grow with k: the row kernels take up to 32768 results.  Us, row kernels / matrix cores:
+  // 256 x 16384, 64 rows 43 / 101; 2048 x 8192, 16 rows 37 / 53; 4096 x 4096, 8 rows 21 / 28, 16 rows 32 / 28; 8192 x 2048, 4 rows 13 / 16,
+  // 6 rows 18 / 16; 32000 x 2048, 2 rows 31 / 21.
+  if (w->dtype == CRABML_HIP_F16 && b >= 2 && b * m_ > 32768) {
     const void* ws[1] = {wp};
     if (launch_gemm_f16(dev, rec0, ws, &m_, 1, k_, act, al.total, b, &out, GemmScratch{})) return 0;
   }

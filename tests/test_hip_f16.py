@@ -1,5 +1,5 @@
-"""F16 weights on the fast device: the row kernel (one row of the rhs) and the matrix-core GEMM (two rows and more) behind matmul_vec and the
-prompt pass, against float64 on the rhs as the reference rounds it (f16, buf_f16.rs:83-97)."""
+"""F16 weights on the fast device: the row kernels (one row of the rhs; up to 32768 results of several) and the matrix-core GEMM (past that, and
+the prompt pass from two rows on), against float64 on the rhs as the reference rounds it (f16, buf_f16.rs:83-97)."""
 import numpy as np
 import pytest
 
@@ -8,9 +8,11 @@ from tests.helpers import FAST_TOL, GEMV_REL
 
 pytestmark = pytest.mark.gpu
 
-# (m, k, rows): one row; ragged m and rows; a tail of k shorter than a step of 64; k that is not whole 16-byte pieces; every tile height
+# (m, k, rows): one row; ragged m and rows; a tail of k shorter than a step of 64; k that is not whole 16-byte pieces; every tile height;
+# results on either side of the GEMM's first
 SHAPES = [(1, 8, 1), (5, 72, 1), (16385, 520, 1), (2050, 4104, 1), (33, 70, 1), (33, 70, 3), (1, 8, 2), (130, 72, 33), (128, 64, 2), (257, 328, 129),
-          (300, 512, 256), (96, 4096, 300), (1027, 136, 65), (2048, 2048, 31)]
+          (300, 512, 256), (96, 4096, 300), (1027, 136, 65), (2048, 2048, 31), (16384, 64, 2),
+          (16385, 72, 2), (1100, 200, 33), (4097, 8, 9), (10923, 136, 3)]
 
 
 @pytest.mark.parametrize("m,k,rows", SHAPES)
@@ -24,16 +26,28 @@ def test_matmul_vec_f16(ca, hdev, m, k, rows):
     assert np.all(np.abs(got - xd @ wd.T) <= GEMV_REL * (np.abs(xd) @ np.abs(wd).T))
 
 
-def test_matmul_vec_f16_infinite_and_nan_rows_stay_apart(ca, hdev):
+@pytest.mark.parametrize("m", [37, 1037])  # row kernels, matrix cores
+def test_matmul_vec_f16_infinite_and_nan_rows_stay_apart(ca, hdev, m):
     """a row of the rhs that holds an infinity or a NaN changes that row's results only; so do the weights' rows"""
     rng = np.random.default_rng(3)
-    w, x = rng.standard_normal((37, 72)).astype(np.float16), rng.standard_normal((35, 72)).astype(np.float32)
-    w[36, 71], x[34, 71], x[5, 0] = np.inf, np.nan, np.inf
-    t = ca.HipTensor.from_cpu(w.view(np.uint8).reshape(-1), [37, 72], ca.GGMLType.F16, hdev)
-    got = t.matmul_vec(ca.HipTensor.new(x.reshape(-1), [35, 72], hdev)).export().reshape(35, 37)
+    w, x = rng.standard_normal((m, 72)).astype(np.float16), rng.standard_normal((35, 72)).astype(np.float32)
+    w[m - 1, 71], x[34, 71], x[5, 0] = np.inf, np.nan, np.inf
+    t = ca.HipTensor.from_cpu(w.view(np.uint8).reshape(-1), [m, 72], ca.GGMLType.F16, hdev)
+    got = t.matmul_vec(ca.HipTensor.new(x.reshape(-1), [35, 72], hdev)).export().reshape(35, m)
     rows = [r for r in range(35) if r not in (5, 34)]
-    assert np.isfinite(got[rows][:, :36]).all() and np.isinf(got[rows][:, 36]).all()
+    assert np.isfinite(got[rows][:, :m - 1]).all() and np.isinf(got[rows][:, m - 1]).all()
     assert np.isnan(got[34]).all() and not np.isfinite(got[5]).any()
+
+
+@pytest.mark.parametrize("m,k,rows", [(1, 8, 3), (77, 768, 15), (4096, 512, 8), (16384, 136, 2), (127, 4104, 258)])
+def test_rows_of_few_results_equal_single_calls(ca, hdev, m, k, rows):
+    """up to 32768 results the row kernels take all rows of the rhs in one launch (258: two of them): the bits of a call per row"""
+    rng = np.random.default_rng(m + rows)
+    w, x = rng.standard_normal((m, k)).astype(np.float16), rng.standard_normal((rows, k)).astype(np.float32)
+    t = ca.HipTensor.from_cpu(w.view(np.uint8).reshape(-1), [m, k], ca.GGMLType.F16, hdev)
+    got = t.matmul_vec(ca.HipTensor.new(x.reshape(-1), [rows, k], hdev)).export().reshape(rows, m)
+    for r in sorted({0, 1, rows // 2, rows - 1}):
+        assert np.array_equal(got[r].view(np.uint32), t.matmul_vec(ca.HipTensor.new(x[r], [k], hdev)).export().view(np.uint32)), r
 
 
 @pytest.mark.parametrize("rows", [2, 65, 203])

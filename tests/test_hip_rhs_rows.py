@@ -17,7 +17,7 @@ def test_rows_equal_single_calls(ca, fmt, strict, m, k, rows):
     if rows > 15 and not strict and fmt in ("Q4_0", "Q8_0", "Q4_1", "Q4_K", "Q6_K", "Q8_K"):
         rows = 15
     if fmt == "F16":
-        k += 0 if strict else 2  # (fast: rows of whole 16-byte pieces take the matrix cores)
+        k += 0 if strict else 2  # (fast: rows of whole 16-byte pieces are in test_hip_f16.py, past 32768 results on the matrix cores)
     rng = np.random.default_rng(m + rows)
     typ = synth.TYPE_BY_NAME[fmt]
     dev = ca.HipTensorDevice(0, False, 0, strict)
