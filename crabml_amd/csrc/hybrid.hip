@@ -24,7 +24,7 @@ struct Layer {
   Connection hc[2];  // mixer, feed-forward
   bool glu = false;
   float *bias_in = nullptr, *bias_o = nullptr;
-  int n_in = 0, ldc = 0, lin_off = 0, ff = 0, ldu = 0, splits = 0, head_blocks = 0;
+  int n_in = 0, ldc = 0, lin_off = 0, ff = 0, ldu = 0, head_blocks = 0;
   ActRanges act;
   unsigned short *w_in = nullptr, *w_o = nullptr, *w_up = nullptr, *w_down = nullptr;
   float *norm1 = nullptr, *norm2 = nullptr, *xielu = nullptr;
@@ -283,7 +283,6 @@ int build_layer(Ctx* c, const crabml_hip_hybrid_layer_t& s, Layer& L) {
   L.ldc = L.lin_off + up(Hl * Vl, 64);
   L.ff = (int)s.ff;
   L.ldu = up(s.ff, 64);
-  L.splits = H && !rank ? (a.rows + MIX_KEYS - 1) / MIX_KEYS : 0;
   L.head_blocks = H && !rank ? (int)((H / G + MIX_HEADS - 1) / MIX_HEADS) : 0;
   const size_t ldw = (size_t)c->ldx;
   CH_TRY(alloc_matrix(c, col, ldw, &L.w_in));
@@ -458,7 +457,7 @@ MixStep mix_step(const Ctx* c, const Run& run, int B) {
   m.ldp = L.n_in;
   m.ldc = L.ldc;
   m.lin_off = L.lin_off;
-  m.splits = L.splits;
+  m.splits = L.at.H ? mix_shares(c->dev->n_cu, B * L.at.G * L.head_blocks, L.at.rows) : 0;
   m.head_blocks = L.head_blocks;
   return m;
 }
@@ -1110,7 +1109,10 @@ int create_impl(Ctx* c, const crabml_hip_hybrid_layer_t* layers, const crabml_hi
       c->hist = std::max(c->hist, (size_t)L.at.rows - (L.at.window ? 1 : 0));
     } else if (L.at.H) {
       const size_t slots = (size_t)HYB_STEP_ROWS * L.at.G * L.head_blocks;
-      part = std::max(part, slots * L.splits * mix_part_floats(L.at.V));
+      for (int B = 1; B <= HYB_STEP_ROWS; B++) {
+        const int per = B * L.at.G * L.head_blocks;
+        part = std::max(part, (size_t)per * mix_shares(dev->n_cu, per, L.at.rows) * mix_part_floats(L.at.V));
+      }
       tick = std::max(tick, slots);
     }
     ss = std::max(ss, (size_t)HYB_STEP_ROWS * L.li.H * L.li.slices);
@@ -1363,3 +1365,9 @@ int crabml_hip_hybrid_decode_greedy(crabml_hip_hybrid_t* c, size_t n, const size
 }
 
 }  // extern "C"
+
+extern "C" int crabml_hip_debug_mix_shares(int32_t n_cu, int32_t per, int32_t rows, int32_t* shares) {
+  if (!shares || n_cu < 1 || per < 1 || rows < 1) return CRABML_HIP_BAD_INPUT;
+  *shares = crabml_hip::mix_shares(n_cu, per, rows);
+  return 0;
+}

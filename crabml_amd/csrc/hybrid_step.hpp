@@ -15,9 +15,9 @@
 namespace crabml_hip {
 
 #define HYB_STEP_ROWS 16
-#define MIX_ONE 256   // up to so many cached rows one workgroup takes them all
-#define MIX_KEYS 128  // ... and past that so many per workgroup
-#define MIX_HEADS 4   // query heads per attention workgroup
+#define MIX_ROWS 64  // attention workgroups share cached rows in multiples of this
+#define MIX_HEADS 4  // query heads per attention workgroup
+#define MIX_THREADS 512
 
 struct StepSeq {
   int token, pos;
@@ -67,6 +67,15 @@ struct MixStep {
   unsigned* tick = nullptr;     // arrivals per (sequence, kv head, head block); the last one puts it back to zero
   int B = 0, ldp = 0, ldc = 0, lin_off = 0, splits = 0, head_blocks = 0, heads = 0;
 };
+// Workgroups that may share a (sequence, kv head, head block)'s rows: `per` of those in the launch, `rows` a sequence can hold.  The grid is what the
+// longest sequence needs (positions live on the device), and a workgroup without rows costs its dispatch -- 16 sequences x 16 kv heads x 16
+// shares: 37 us for 10 rows each -- so there are no more of them than CUs beside one per (sequence, kv head, head block).  Us a launch, shares of
+// 128 rows up to capacity / this rule, 16 sequences of 10 and 300 rows: 4 kv heads x 128 20.4 / 9.5 and 35.0 / 15.9, 16 x 64 37.2 / 6.4 and
+// 57.8 / 9.7; one sequence of 690 rows 12.6 / 10.4 and 8.4 / 8.9.  (Twice as many workgroups: 13.7 / 19.7 and 9.3 / 13.6 for 16 sequences.)
+__host__ inline int mix_shares(int n_cu, int per, int rows) {
+  const int most = (rows + MIX_ROWS - 1) / MIX_ROWS, fit = n_cu / per;
+  return fit < 1 ? 1 : fit < most ? fit : most;
+}
 // floats of one partial: per head its V sums, the running maximum and the denominator
 __host__ __device__ inline int mix_part_floats(int V) { return MIX_HEADS * (V + 2); }
 
@@ -77,17 +86,27 @@ __device__ __forceinline__ void cat_out(float* cat, unsigned short* cat16, size_
     cat[at] = v;
 }
 
+// rows of a wave's round: U requests of K and V out; with them and four heads' sums a thread holds at most 128 registers, so that two workgroups
+// of 512 -- the linear branch's are as large -- share a CU
+template <typename T, int CLS>
+struct MixRound {
+  static constexpr int LPR = CLS / 8, RPI = 64 / LPR, RR = 8 * RPI;  // lanes a row, rows of a wave's request, of one from every wave
+  static constexpr int U = sizeof(T) == 2 && CLS >= 128 ? 2 : 1;
+  static constexpr int ONE = CLS == 64 ? 256 : 4 * U * RR < 128 ? 4 * U * RR : 128;  // rows that stay in one workgroup
+};
+
 // One workgroup: up to MIX_HEADS query heads of one kv head over its share of the cached rows; heads up to CLS wide.  What bounds it is the
 // chain position -> rows -> scores -> softmax -> sums of a cold launch, so the chain has one barrier where the heads' operands are laid out and
 // one where the waves meet: a row is LPR lanes x 8 elements and a wave instruction takes 64 / LPR rows; a wave keeps K and V of its rows in
-// registers, scores them for every head, takes its own maximum, and adds up p * v over its rows.  (64 rows a round and four heads: 128 registers,
-// so that two workgroups -- the linear branch's are as large -- share a CU.)  Four barriers, a wave per head's softmax and LDS exchanges between
-// 256 threads before that: 13.0 -> 9.4 us a launch (one sequence, 33 to 81 rows, normed q and k), 15.4 -> 13.2 (16 sequences, 90 to 154 rows,
-// linear branch beside it).  Up to MIX_ONE rows stay in one workgroup:
-// handing partial sums over costs 3 us, a second round of 128 rows 0.6.
-template <typename T, int CLS, int NT>
+// registers, scores them for every head, takes its own maximum, and adds up p * v over its rows.  Four barriers, a wave per head's softmax and LDS
+// exchanges between 256 threads before that: 13.3 -> 9.1 us a launch (one sequence, 60 rows, normed q and k), 22.1 -> 9.5 (16 sequences, 10 rows,
+// linear branch beside it).  A round of 64 rows adds 1.6 us at 128 columns and 0.4 at 64, handing partial sums over 3: two rounds stay in one workgroup (four of 64
+// columns, four short ones of wide heads), longer ranges are shared out evenly (one sequence of 200 rows, one workgroup / four: heads of 128
+// 13.5 / 10.4 us, of 64 6.6 / 7.8).
+template <typename T, int CLS>
 __device__ __forceinline__ void mix_attention(const MixStep& a, int blk, float* lds) {
-  constexpr int LPR = CLS / 8, RPI = 64 / LPR, NW = NT / 64, RR = NW * RPI, U = 64 / RR < 4 ? 64 / RR : 4;
+  using M = MixRound<T, CLS>;
+  constexpr int LPR = M::LPR, RPI = M::RPI, NW = MIX_THREADS / 64, RR = M::RR, U = M::U;
   const AttnGeom& g = a.at;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_wg();
   const int split = blk % a.splits;
@@ -109,9 +128,15 @@ __device__ __forceinline__ void mix_attention(const MixStep& a, int blk, float* 
   float* o_s = q_s + heads * g.D;         // [NW][heads][V]
   // the new token's row, and the rows it sees: its chunk's up to itself, or the whole ring once the window has gone round
   const int in_chunk = sq.pos % g.span, n_rows = g.window && sq.pos >= g.span ? g.span : in_chunk + 1;
-  const int keys = n_rows <= MIX_ONE ? MIX_ONE : MIX_KEYS, r0 = split * keys;
-  if (r0 >= n_rows) return;  // (whole workgroup)
-  const int active = (n_rows + keys - 1) / keys, r1 = r0 + keys < n_rows ? r0 + keys : n_rows;
+  int active = 1, share = n_rows;
+  if (n_rows > M::ONE) {
+    const int want = (n_rows + MIX_ROWS - 1) / MIX_ROWS;
+    active = want < a.splits ? want : a.splits;
+    share = ((n_rows + active - 1) / active + MIX_ROWS - 1) / MIX_ROWS * MIX_ROWS;
+    active = (n_rows + share - 1) / share;
+  }
+  if (split >= active) return;  // (whole workgroup)
+  const int r0 = split * share, r1 = r0 + share < n_rows ? r0 + share : n_rows;
   T* kc = (T*)(sq.slab + a.rs.k) + (size_t)kvh * g.rows * g.D;
   T* vc = (T*)(sq.slab + a.rs.v) + (size_t)kvh * g.rows * g.V;
   const bool own_new = in_chunk >= r0 && in_chunk < r1;
@@ -133,8 +158,8 @@ __device__ __forceinline__ void mix_attention(const MixStep& a, int blk, float* 
   float q_f = g.scale, k_f = 1.f;
   if (g.q_norm) {  // (the same for the whole workgroup)
     float sq2 = 0.f, sk2 = 0.f;
-    for (int i = tid; i < g.H * g.D; i += NT) sq2 = __builtin_fmaf(pr[g.cq + i], pr[g.cq + i], sq2);
-    for (int i = tid; i < g.G * g.D; i += NT) sk2 = __builtin_fmaf(pr[g.ck + i], pr[g.ck + i], sk2);
+    for (int i = tid; i < g.H * g.D; i += MIX_THREADS) sq2 = __builtin_fmaf(pr[g.cq + i], pr[g.cq + i], sq2);
+    for (int i = tid; i < g.G * g.D; i += MIX_THREADS) sk2 = __builtin_fmaf(pr[g.ck + i], pr[g.ck + i], sk2);
     sq2 = wave_sum_f32(sq2);
     sk2 = wave_sum_f32(sk2);
     float* red = hp_s + 3 * MIX_HEADS;
@@ -152,8 +177,8 @@ __device__ __forceinline__ void mix_attention(const MixStep& a, int blk, float* 
     q_f *= 1.0f / sqrtf(sq2 / (float)g.q_mean + g.eps);
     k_f = 1.0f / sqrtf(sk2 / (float)g.k_mean + g.eps);
   }
-  for (int i = tid; i < nh * g.D; i += NT) q_s[i] = pr[g.cq + h0 * g.D + i] * (g.q_norm ? q_f * g.q_norm[h0 * g.D + i] : q_f);
-  for (int i = tid; i < nh * g.V; i += NT)
+  for (int i = tid; i < nh * g.D; i += MIX_THREADS) q_s[i] = pr[g.cq + h0 * g.D + i] * (g.q_norm ? q_f * g.q_norm[h0 * g.D + i] : q_f);
+  for (int i = tid; i < nh * g.V; i += MIX_THREADS)
     g_s[i] = (g.gate == GATE_ELEMENT ? pr[g.cg + h0 * g.V + i] : g.gate == GATE_HEAD ? pr[g.cg + h0 + i / g.V] : 1.f) * g.out_scale;
   if (tid < g.D) kn_s[tid] = kv_from<T>(pr[g.ck + kvh * g.D + tid] * (g.k_norm ? k_f * g.k_norm[kvh * g.D + tid] : 1.f));
   float v_raw = 0.f;
@@ -272,7 +297,7 @@ __device__ __forceinline__ void mix_attention(const MixStep& a, int blk, float* 
   };
   if (active > 1) {  // partials through write-through stores; whoever arrives last merges them in row order
     float* mine = base + (size_t)split * pf;
-    for (int i = tid; i < n_out; i += NT) {
+    for (int i = tid; i < n_out; i += MIX_THREADS) {
       float M, L;
       __hip_atomic_store(mine + i, met(i, M, L), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (i % g.V == 0) {
@@ -287,7 +312,7 @@ __device__ __forceinline__ void mix_attention(const MixStep& a, int blk, float* 
     if (!s_last) return;
     if (tid == 0) __hip_atomic_store(a.tick + slot, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  for (int i = tid; i < n_out; i += NT) {
+  for (int i = tid; i < n_out; i += MIX_THREADS) {
     const int h = i / g.V;
     float m = hp_s[2 * MIX_HEADS + h], l = m == -INFINITY ? 0.f : 1.f, o = 0.f;  // the sink: a key without a value (or none)
     if (active == 1) {
@@ -324,11 +349,10 @@ __device__ __forceinline__ void mix_attention(const MixStep& a, int blk, float* 
 }
 
 // one head's slice of value columns: 8 threads x 4 columns, 32 groups of key rows; 256 threads a slice
-template <int NT>
 __device__ __forceinline__ void mix_linear(const MixStep& a, int blk, float* lds) {
   const LinGeom& g = a.li;
   const int tid = threadIdx.x & 255, lane = tid & 63, wave = wave_in_wg() & 3, part = wave_in_wg() >> 2;
-  const int n = a.B * g.H * g.slices, unit = blk * (NT / 256) + part;
+  const int n = a.B * g.H * g.slices, unit = blk * (MIX_THREADS / 256) + part;
   const bool used = unit < n;  // (the last workgroup's second slice may be none)
   blk = used ? unit : n - 1;
   lds += part * (2 * g.D + 32 * 36);
@@ -388,25 +412,25 @@ __device__ __forceinline__ void mix_linear(const MixStep& a, int blk, float* lds
   }
 }
 
-template <typename T, int CLS, int NT>
-__global__ __launch_bounds__(NT, NT == 512 && sizeof(T) == 2 ? 4 : 2) void k_mix_step(const MixStep a) {
+template <typename T, int CLS>
+__global__ __launch_bounds__(MIX_THREADS, 4) void k_mix_step(const MixStep a) {
   extern __shared__ __attribute__((aligned(16))) float mix_lds[];
   const int n_attn = a.at.H ? a.B * a.at.G * a.head_blocks * a.splits : 0;
   if ((int)blockIdx.x < n_attn)
-    mix_attention<T, CLS, NT>(a, blockIdx.x, mix_lds);
+    mix_attention<T, CLS>(a, blockIdx.x, mix_lds);
   else
-    mix_linear<NT>(a, blockIdx.x - n_attn, mix_lds);
+    mix_linear(a, blockIdx.x - n_attn, mix_lds);
 }
 template <typename T, int CLS>
 inline void launch_mix_step_t(hipStream_t st, crabml_hip_device::ProfRec* rec, MixStep a) {
-  constexpr int NT = CLS == 256 ? 256 : 512, NW = NT / 64;  // (the waves' sums of 256 columns would not fit twice)
+  constexpr int NW = MIX_THREADS / 64;
   const int hpg = a.at.H ? a.at.H / a.at.G : 0;
   a.heads = hpg < MIX_HEADS ? hpg : MIX_HEADS;
   const size_t at = a.at.H ? (2 * NW + 3) * MIX_HEADS + 2 * NW + 2 * CLS * sizeof(T) / 4 + (size_t)a.heads * (a.at.D + (NW + 1) * a.at.V) : 0;
-  const size_t li = a.li.H ? (size_t)(2 * a.li.D + 32 * 36) * (NT / 256) : 0;
+  const size_t li = a.li.H ? (size_t)(2 * a.li.D + 32 * 36) * (MIX_THREADS / 256) : 0;
   const int units = a.B * a.li.H * a.li.slices;
-  const unsigned grid = (unsigned)((a.at.H ? a.B * a.at.G * a.head_blocks * a.splits : 0) + (units + NT / 256 - 1) / (NT / 256));
-  launch_k(st, rec, k_mix_step<T, CLS, NT>, dim3(grid), dim3(NT), (at > li ? at : li) * sizeof(float), a);  // (at most 27 KiB)
+  const unsigned grid = (unsigned)((a.at.H ? a.B * a.at.G * a.head_blocks * a.splits : 0) + (units + MIX_THREADS / 256 - 1) / (MIX_THREADS / 256));
+  launch_k(st, rec, k_mix_step<T, CLS>, dim3(grid), dim3(MIX_THREADS), (at > li ? at : li) * sizeof(float), a);  // (at most 43 KiB)
 }
 template <typename T>
 inline void launch_mix_step(hipStream_t st, crabml_hip_device::ProfRec* rec, const MixStep& a) {

@@ -23,3 +23,14 @@ def test_several_rhs_rows_stay_one_legal_launch(per_wg, threads):
         tiles = -(-tiles // 8) * 8 if rows > 1 else tiles
         assert 1 <= rows <= 256 and tiles * rows * threads < 1 << 32, (m, rows)
     assert rhs_rows(128256) == 256 and rhs_rows(262144) == 255  # (no fewer than fit)
+
+
+@pytest.mark.parametrize("n_cu", [1, 80, 256])
+def test_shares_of_cached_rows(n_cu):
+    """the hybrid step's attention: no more workgroups than CUs beside one per (sequence, kv head, head block), no share without 64 rows to take"""
+    for per in (1, 2, 3, 16, 48, 255, 256, 257, 4096):
+        for rows in (1, 63, 64, 65, 700, 2048, 100000):
+            n = ctypes.c_int32()
+            assert lib.crabml_hip_debug_mix_shares(n_cu, per, rows, ctypes.byref(n)) == 0
+            assert 1 <= n.value <= -(-rows // 64) and n.value * per <= max(n_cu, per)
+            assert n.value == -(-rows // 64) or (n.value + 1) * per > n_cu  # (no fewer than fit)
