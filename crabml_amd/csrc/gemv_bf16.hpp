@@ -407,12 +407,15 @@ __device__ __forceinline__ void split3(const float (&v)[8], bf16x8& hi, bf16x8& 
 __device__ __forceinline__ void wave_lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 
-template <int RT, int SPL, int W, int D, int IN, int OUT>
+// XG: f32 rows are requested and split in groups of four, as many as there are rows -- a group is a request, twelve conversions and three LDS
+// stores a lane and piece, which three rows of four groups paid for in full (f32 compute, us, 4 rows, all groups / one: 11264 x 2048
+// 17.3 / 12.2, gate | up of 16384 x 2048 18.5 / 16.1).
+template <int RT, int SPL, int W, int D, int IN, int OUT, int XG = 4>
 __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
   constexpr int LD = 20, NT = 64 * W;
   constexpr bool XB = IN == GEMV_IN_BF16 || IN == GEMV_IN_BF16_RMS || IN == GEMV_IN_BF16_SPLIT, NORM = IN == GEMV_IN_RMS || IN == GEMV_IN_RMSV;
   constexpr bool PIECES = IN == GEMV_IN_BF16_RMS || IN == GEMV_IN_BF16_SPLIT, TAIL = IN == GEMV_IN_BF16_SPLIT;
-  constexpr int XR = XB ? 2 : 4;  // requests for a piece of the rhs
+  constexpr int XR = XB ? 2 : XG;  // requests for a piece of the rhs
   static_assert(!XB || SPL == 1, "a bf16 rhs has one piece");
   union Lds {
     unsigned short in[W][RT + SPL][16 * 64];  // a wave's tiles: weights, rhs
@@ -461,6 +464,16 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
 #pragma unroll
     for (int u = 0; u < QP; u++) q_v[u] = q_ss[q_at + u * QT < a.n_ss ? q_at + u * QT : 0];
   }
+  float tail[XR], sq[XR];  // of row 4 j + r16
+  const float* t_ss[XR];
+#pragma unroll
+  for (int j = 0; j < XR; j++) {
+    tail[j] = sq[j] = 0.f;
+    if constexpr (IN == GEMV_IN_SPLIT) {  // (the first pieces of every row: ahead of the weights, too)
+      t_ss[j] = a.ss + (size_t)(j * 4 + r16 < a.nb ? j * 4 + r16 : a.nb - 1) * a.n_ss;
+      tail[j] = t_ss[j][c16 < a.n_ss ? c16 : 0];
+    }
+  }
   if (wave < n) {
 #pragma unroll
     for (int d = 0; d < D; d++) request(d, wave + d * W < n ? wave + d * W : last);  // (clamped: no branch between the requests)
@@ -474,15 +487,11 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
       if (j < RT * 256 && b < a.nb && row < a.N) stream_elem_load(a, row, b, elem[i]);
     }
   }
-  float tail[4], sq[4];  // of row 4 j + r16
+  if constexpr (IN == GEMV_IN_SPLIT) {
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
-    tail[j] = 1.f;
-    sq[j] = 0.f;
-    if constexpr (IN == GEMV_IN_SPLIT) {
-      const int b = j * 4 + r16;
-      float t = 0.f;
-      for (int i = c16; i < a.n_ss; i += 16) t += a.ss[(size_t)(b < a.nb ? b : a.nb - 1) * a.n_ss + i];
+    for (int j = 0; j < XR; j++) {
+      float t = c16 < a.n_ss ? tail[j] : 0.f;
+      for (int i = c16 + 16; i < a.n_ss; i += 16) t += t_ss[j][i];
       tail[j] = 1.0f / sqrtf(row16_sum_f32(t) / (float)a.mean_n + a.eps);
     }
   }
@@ -506,7 +515,7 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
       }
     } else {
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
+      for (int j = 0; j < XR; j++) {
         const int r = j * 4 + r16;
         f32x4 v = __builtin_bit_cast(f32x4, xc[j]);
         if constexpr (NORM) {
@@ -565,7 +574,7 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
   }
   if constexpr (NORM) {
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < XR; j++) {
       const float t = row16_sum_f32(sq[j]);
       if (c16 == 0) sums[wave][j * 4 + r16] = t;
     }
@@ -663,25 +672,43 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
 
 // 32 rows a workgroup where that still fills the chip, else 16; sixteen waves where 16 rows leave CUs without a workgroup and k is long
 // enough for each of them to have a few steps.  One piece of the rhs: bf16 rows, but for a classifier behind a prompt pass.
+// Three pieces of more than eight f32 rows: two steps of requests hold 140 registers a thread, one workgroup a CU; where there are more workgroups than
+// CUs, two of them with one step out each are faster (us, 12 rows: 11264 x 2048 18.0 -> 16.4, 8192 x 1024 8.7 -> 6.9), elsewhere they are
+// not (2048 x 8192, 128 workgroups: 16.2 -> 19.8).
 template <int RT, int SPL, int W, int IN, int OUT>
-inline void launch_gemv16_t(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a) {
+inline void launch_gemv16_t(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a, int n_cu) {
   constexpr int D = IN < GEMV_IN_BF16 || RT == 2 ? 2 : OUT == GEMV_OUT_STREAMS ? 3 : 4;  // (registers: sixteen waves a CU)
-  launch_k(st, rec, k_gemv16_bf16<RT, SPL, W, D, IN, OUT>, dim3((a.N + 16 * RT - 1) / (16 * RT)), dim3(64 * W), 0, a);
+  const dim3 grid((a.N + 16 * RT - 1) / (16 * RT));
+  if constexpr (SPL == 3) {
+    if (a.nb <= 4) {
+      launch_k(st, rec, k_gemv16_bf16<RT, SPL, W, D, IN, OUT, 1>, grid, dim3(64 * W), 0, a);
+      return;
+    }
+    if (a.nb <= 8) {
+      launch_k(st, rec, k_gemv16_bf16<RT, SPL, W, D, IN, OUT, 2>, grid, dim3(64 * W), 0, a);
+      return;
+    }
+    if (RT == 1 && (int)grid.x > n_cu) {
+      launch_k(st, rec, k_gemv16_bf16<RT, SPL, W, 1, IN, OUT>, grid, dim3(64 * W), 0, a);
+      return;
+    }
+  }
+  launch_k(st, rec, k_gemv16_bf16<RT, SPL, W, D, IN, OUT>, grid, dim3(64 * W), 0, a);
 }
 template <int SPL, int IN, int OUT>
 inline void launch_gemv16_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a, int n_cu) {
   const bool two = a.N >= 16384, deep = !two && (a.N + 15) / 16 < n_cu && a.K >= 2048;
   if (two) {
-    launch_gemv16_t<2, SPL, 8, IN, OUT>(st, rec, a);
+    launch_gemv16_t<2, SPL, 8, IN, OUT>(st, rec, a, n_cu);
     return;
   }
   if constexpr (IN >= GEMV_IN_BF16) {
     if (deep) {
-      launch_gemv16_t<1, SPL, 16, IN, OUT>(st, rec, a);
+      launch_gemv16_t<1, SPL, 16, IN, OUT>(st, rec, a, n_cu);
       return;
     }
   }
-  launch_gemv16_t<1, SPL, 8, IN, OUT>(st, rec, a);
+  launch_gemv16_t<1, SPL, 8, IN, OUT>(st, rec, a, n_cu);
 }
 
 template <int NB, int R, int IN, int OUT>

@@ -31,7 +31,7 @@ def test_batched_steps(ca, hdev, tmp_path, design, width, ff, vocab, f32):
     rng = np.random.default_rng(width)
     toks = rng.integers(0, vocab, (16, 3))
     want = [oracle.forward(config, floats, t) for t in toks[:3]]
-    for batch in (1, 3, 16, 2):  # (the forms for few rows in between: they share the step's buffers)
+    for batch in (1, 3, 6, 16, 2):  # (f32: one, two and four groups of rows; the forms for few rows in between: they share the step's buffers)
         seqs = [r.open() for _ in range(batch)]
         got = np.array([r.step([(s, [int(toks[i, t])], [0]) for i, s in enumerate(seqs)]) for t in range(3)])  # [step, sequence, vocab]
         for s in seqs:
