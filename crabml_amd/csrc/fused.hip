@@ -2228,16 +2228,18 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
   // A head per workgroup with f32 sums (k_attn_short): from the start where the fast step of Q4_0 / Q8_0 layers leaves the reference's summation
   // order as well (deferred norms; a tensor-parallel rank's wo and ffn_down, whose group adds them up) and no flag asks for more of it;
   // elsewhere where k_attn_flash would leave it.  Us per layer of the 8B shape, k_attn_short against what ran before: 4.7 against 6.5 at 40
-  // cached positions, 5.4 against 8.8 at 88.  Against k_attn_flash, a step and layer: 33.1 / 35.6 at 128, 34.1 / 36.0 at 256, 35.4 / 36.3 at
-  // 384, 36.4 / 36.3 at 512, 38.3 / 36.9 at 768 (16 / 4 heads x 128: even at 600; 32 / 32 x 64: at 1000) -- one workgroup reads a head's
-  // rows at a CU's rate.  A caller's own attn_long_from is the long kernels' from there on.
+  // cached positions, 5.4 against 8.8 at 88.  k_attn_flash overtakes it where a head's rows -- one workgroup reads them at a CU's rate -- are some
+  // 110 KB of K and as much of V: 448 positions of heads of 128, 896 of 64.  A step and layer at 440 / 500 / 600 positions, k_attn_short
+  // against k_attn_flash: 32 / 8 heads x 128 35.2 / 35.8, 36.2 / 35.8, 37.0 / 36.2; 16 / 16 x 128 29.4 / 29.9, 30.4 / 30.0, 31.5 / 30.3;
+  // 64 / 8 x 128 54.9 / 60.9, 55.7 / 60.9, 56.8 / 61.3; at 800 / 900 / 1200: 32 / 32 x 64 29.8 / 30.6, 30.4 / 30.6, 31.4 / 31.2; 12 / 12 x 64
+  // 26.7 / 27.9, 27.4 / 28.0, 29.2 / 28.3.  A caller's own attn_long_from is the long kernels' from there on.
   if (g.use_f16_kv_cache && hd % 8 == 0 && hd <= 256 && !dev->strict_order &&
       !(g.flags & (CRABML_HIP_LLAMA_EXACT_ATTENTION | CRABML_HIP_LLAMA_NO_LONG_ATTENTION | CRABML_HIP_LLAMA_NO_STAGED_ATTENTION))) {
     const bool flash = c->attn_flash && g.attn_long_from == 0;
     const bool own_order = c->defer_norm || (tp > 1 && !generic && (wt == CRABML_HIP_Q4_0 || wt == CRABML_HIP_Q8_0) &&
                                              !(g.flags & (CRABML_HIP_LLAMA_EXACT_NORM | CRABML_HIP_LLAMA_NO_NORM_EPILOGUE)));
     c->attn_short_from = own_order ? 0 : flash ? c->attn_long_from : SIZE_MAX;
-    c->attn_short_until = flash ? 512 : c->attn_long_ok ? c->attn_long_from : SIZE_MAX;
+    c->attn_short_until = flash ? 57344 / hd : c->attn_long_ok ? c->attn_long_from : SIZE_MAX;
   }
   // A tensor-parallel rank's gate/up: hidden / tp / 32 workgroups of 32 rows would leave most CUs idle.  h stays f32 from workgroups
   // of `gu_rows` rows (the largest even divisor of the rank's rows, at most 32, that gives at least one workgroup per CU) and

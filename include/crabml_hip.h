@@ -241,7 +241,7 @@ typedef struct crabml_hip_llama_config { /* crabml-llama2/src/model.rs:30-53 */
   int32_t tp_size, tp_rank;
   void* tp_comm; /* crabml_hip_tp_comm_t*; NULL with tp_size > 1 = a rank of the single-device simulation */
   size_t attn_long_from; /* cached positions from which attention runs as the multi-workgroup kernels (0 = default: 224 for the
-                          * exact kernels; fast step: 512 for the split-KV kernels, the one-workgroup kernel with f32 sums from 96, with
+                          * exact kernels; fast step: 448 for the split-KV kernels, 896 with heads of 64, the one-workgroup kernel with f32 sums from 96, with
                           * Q4_0 / Q8_0 layers from the first unless their norms are asked for, or run, in the reference's order) */
   size_t prefill_chunk;  /* rows per batched prefill pass (0 = default: 1024, 512 on a strict-order device; never more than seq_len) */
 } crabml_hip_llama_config_t;

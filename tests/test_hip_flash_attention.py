@@ -123,13 +123,15 @@ def test_a_cache_length_that_is_no_multiple_of_eight_keeps_the_split_kv_kernels(
     """The exact long-context kernels read score / probability rows of seq_len elements as 16-byte vectors (seq_len % 8 == 0);
     k_attn_flash reads cache rows only.  A cache of 203 positions used to drop the fast step to one workgroup per head past 96
     positions (45 us per layer at 900 positions of the 8B shape); now it runs the same kernels as a cache of 208 -- the cache row
-    stride differs, nothing else: the logits agree bit for bit."""
+    stride differs, nothing else: the logits agree bit for bit.  (attn_long_from = 96: left to itself the step runs k_attn_short there.)"""
     model = synth.build_model(synth.SHAPES["tiny-hd128"], synth.Q4_0, seed=77)
     dev = ca.HipTensorDevice(0)
     conf, w = synth.to_hip(model, dev)
-    odd = ca.HipLlamaRunner(conf, w, dev, 203, True)
-    even = ca.HipLlamaRunner(conf, w, dev, 208, True)
-    odd_eager = ca.HipLlamaRunner(conf, w, dev, 203, True, False)
+    odd = ca.HipLlamaRunner(conf, w, dev, 203, True, attn_long_from=96)
+    even = ca.HipLlamaRunner(conf, w, dev, 208, True, attn_long_from=96)
+    odd_eager = ca.HipLlamaRunner(conf, w, dev, 203, True, False, attn_long_from=96)
+    for r in (odd, even, odd_eager):  # (the split-KV forms: the merge in a launch of its own, in the last workgroup)
+        assert all(r.debug_graphs(i)[0] in (1, 2) for i in range(95, 203)) and r.debug_graphs(94)[0] == 0
     for i in range(200):
         t = (5 * i + 2) % 1000
         a, b, c = odd.forward(t, i).copy(), even.forward(t, i).copy(), odd_eager.forward(t, i).copy()

@@ -7,7 +7,7 @@ length in all three softmax hosts (k_attn, k_attn_s, k_attn_softmax), so the log
 through the multi-workgroup long-context kernels and through the one-workgroup-per-head kernel.  The fast device is held to a
 pinned tolerance at the same positions, with the oracle's own tokens, in both of its long-context forms: the exact kernels
 (CRABML_HIP_LLAMA_EXACT_ATTENTION: the reference's f16 PV chain, block-tree row sum beyond 1024 positions -> FAST_TOL) and the
-default split-KV kernel with f32 accumulation (k_attn_flash, from 224 positions -> FLASH_TOL, round 4).  Q4_K weights (a
+default kernels with f32 accumulation (k_attn_short, k_attn_flash from 896 positions of heads of 64 -> FLASH_TOL).  Q4_K weights (a
 round-to-nearest rhs quantizer: nothing but the attention deviation survives) measure that deviation by itself; Q4_0 shows it
 next to the truncating quantizer's +-1 flips."""
 import numpy as np
@@ -40,7 +40,7 @@ def test_strict_and_fast_decode_equal_the_oracle_up_to_position_4095(ca, fmt):
     fdev = ca.HipTensorDevice(0)
     fconf, fw = synth.to_hip(model, fdev)
     fast = ca.HipLlamaRunner(fconf, fw, fdev, n + 8, True, extra_flags=EXACT)
-    flash = ca.HipLlamaRunner(fconf, fw, fdev, n + 8, True)  # k_attn_flash from 224 cached positions
+    flash = ca.HipLlamaRunner(fconf, fw, fdev, n + 8, True)  # k_attn_short, k_attn_flash from 896 cached positions
     errs, ferrs = [], []
     for i, t in enumerate(toks):
         ref = orr.forward([t], i)

@@ -60,13 +60,14 @@ def test_infinities_and_nan(ca, hd):
 
 @pytest.mark.parametrize("fmt", ["Q8_0", "F16", "Q4_K"])
 def test_step_across_the_switches(ca, fmt):
-    """positions 0 .. 529: k_attn_short from the start (Q8_0) or from 96 (the others) up to 512, k_attn_flash behind -- graph and eager agree
+    """positions 0 .. 529: k_attn_short from the start (Q8_0) or from 96 (the others) up to 448, k_attn_flash behind -- graph and eager agree
     bit for bit, and stay as close to the exact chain as k_attn_flash is required to"""
     model = synth.build_model(synth.SHAPES["tiny-hd128"], synth.TYPE_BY_NAME[fmt], seed=78)
     dev = ca.HipTensorDevice(0)
     conf, w = synth.to_hip(model, dev)
     a, e, x = ca.HipLlamaRunner(conf, w, dev, 533, True), ca.HipLlamaRunner(conf, w, dev, 533, True, False), ca.HipLlamaRunner(conf, w, dev, 533, True, extra_flags=EXACT)
-    check = {0, 94, 95, 96, 97, 128, 510, 511, 512, 529}
+    check = {0, 94, 95, 96, 97, 128, 446, 447, 448, 510, 511, 512, 529}
+    assert [a.debug_graphs(i)[0] for i in (94, 95, 446, 447)] == [0, 0 if fmt == "Q8_0" else 3, 0 if fmt == "Q8_0" else 3, 2]
     errs = []
     for i in range(530):
         t = (5 * i + 2) % 1000

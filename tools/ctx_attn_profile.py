@@ -1,6 +1,6 @@
 """Decode attention at long context: per-stage HIP-event times of the long-context kernels at a few cache fills, Llama-3-8B
-layer shape (8 layers: the per-layer kernels are the same), f16 KV cache.  Stages: the fast step's default k_attn_flash (7) +
-k_attn_flash_merge (8); with FLAGS=4194304 (EXACT_ATTENTION) the exact kernels scores (7) / softmax (8) / pv (9); with
+layer shape (8 layers: the per-layer kernels are the same), f16 KV cache.  Stages: the fast step's default k_attn_short (7) below
+448 positions, k_attn_flash (7) -- with its merge up to 768, then + k_attn_flash_merge (8) --; with FLAGS=4194304 (EXACT_ATTENTION) the exact kernels scores (7) / softmax (8) / pv (9); with
 FLAGS=2097152 (FLASH_TICKET) the single-launch flash form (7).
 usage: [FLAGS=n] python tools/ctx_attn_profile.py [positions ...]"""
 import os

@@ -10,6 +10,7 @@ import numpy as np
 
 sys.path.insert(0, ".")
 os.environ["CRABML_HIP_TEST_HOOKS"] = "1"
+os.environ["CRABML_HIP_FLASH_TICKET_UNTIL"] = "0"  # (else the merge is the last workgroup's below 768 positions, whatever the flags)
 import crabml_amd as ca  # noqa: E402
 from crabml_amd import synth  # noqa: E402
 
