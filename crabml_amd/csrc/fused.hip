@@ -136,6 +136,7 @@ struct crabml_hip_llama {
   bool k_norm_in = false;    // fast Q4_K step: gate | up normalizes and quantizes wo's f32 row itself (k_gateup_k_lds<.., NORMIN>)
   bool kfused = false;       // Q4_K layers, fast mode: fused GEMV kernels with the Q4_K inner loop (enqueue_segment_k)
   bool f16_step = false;     // F16 layers, fast mode, one GPU: the linears with their row operations folded in (enqueue_segment_f16)
+  bool attn_row_apart = false;  // test hook: the attention row of odd head widths through the quantizer's own launch
   bool generic = false;      // per-op launches (strict-order device, or a weight format without fused kernels)
   bool ord = false;          // strict-order device, Q4_0 / Q8_0 / Q4_1 layers: the fused launches with block-ordered sums (k_*_ord)
   uint32_t qt = 0, out_qt = 0;  // vec_dot_rhs_dtype of the layer weights / of the classifier
@@ -718,7 +719,7 @@ int enqueue_segment_t(crabml_hip_llama* c, int seg) {
     enqueue_attention(c, l, attn_quant ? aa.q : (signed char*)nullptr, aa.d, aa.isum, plan(c->wo[l], nullptr, nullptr), attn_spare, prof);
     // heads that are not whole quant blocks (head width 48 of the 15M-parameter model): wo's launch quantizes the row itself -- the same bits, one
     // launch fewer per layer (2 us of quantizer and its boundary: 7.46 -> 7.05 ms for 57 tokens of that model)
-    const bool attn_in_f32 = !attn_quant && defer_wo && !tp && !c->ord && q8_0_lds_bytes(dim_l / 32) <= 60 * 1024;
+    const bool attn_in_f32 = !attn_quant && !c->attn_row_apart && defer_wo && !tp && !c->ord && q8_0_lds_bytes(dim_l / 32) <= 60 * 1024;
     if (!attn_quant && !attn_in_f32) launch_quantize_act(st, qt, c->attn, (size_t)dim_l, c->act_attn);
     // wo (+ residual, llama2.rs:600, 266): k = the local heads' slice
     CH_TRY(gemv_out(c->wo[l], aa, dim_l, 2, (const float*)c->rms_ffn[l]->ptr, 1e-5f, defer_wo, attn_in_f32 ? c->attn : nullptr));
@@ -2026,6 +2027,7 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
   if (ordk) ord = true;
   if (ordk && mixed) generic = false;
   c->generic = generic;
+  if (const char* hooks = getenv("CRABML_HIP_TEST_HOOKS")) c->attn_row_apart = hooks[0] == '1' && getenv("CRABML_HIP_ATTN_ROW_APART") != nullptr;
   // (dims are multiples of 32 and heads of 2 by now; a longer row does not fit the launches that normalize it: the per-op segments)
   c->f16_step = !dev->strict_order && wt == CRABML_HIP_F16 && !mixed && tp == 1 && g.embedding_dim <= STEP_F16_MAX_K && dim_l <= STEP_F16_MAX_K;
   c->ord = ord;
@@ -2550,34 +2552,48 @@ int crabml_hip_llama_debug_graphs(crabml_hip_llama_t* c, size_t pos, int32_t* fo
 
 // parity hook (crabml_hip_debug.h): k_attn_short by itself, on caller-supplied q / K / V
 int crabml_hip_debug_short_attention(crabml_hip_device_t* dev, const float* q, const uint16_t* k, const uint16_t* v, size_t n_heads,
-                                     size_t n_kv, size_t head_dim, size_t seq, size_t seq_cap, float* out) {
+                                     size_t n_kv, size_t head_dim, size_t seq, size_t seq_cap, float* out, uint32_t qtype, int32_t* blocks) {
   if (!dev || !q || !k || !v || !out || seq == 0 || seq > seq_cap || seq_cap > (1u << 24) || n_kv == 0 || n_heads == 0 || n_heads % n_kv != 0 || n_heads > 4096 ||
-      head_dim == 0 || head_dim % 8 != 0 || head_dim > 256)
+      head_dim == 0 || head_dim % 8 != 0 || head_dim > 256 ||
+      (blocks && ((qtype != CRABML_HIP_Q8_0 && qtype != CRABML_HIP_Q8_1) || head_dim % 32 != 0)))
     return CRABML_HIP_BAD_INPUT;
   CH_LIVE(dev);
   CH_USE(dev);
   CH_FLUSH(dev);
-  const size_t nq = n_heads * head_dim * 4, nkv = n_kv * seq_cap * head_dim * 2;
-  const size_t o_k = align_up(nq, 256), o_v = align_up(o_k + nkv, 256), o_out = align_up(o_v + nkv, 256), o_pos = align_up(o_out + nq, 256);
+  const size_t n = n_heads * head_dim, nq = n * 4, nkv = n_kv * seq_cap * head_dim * 2;
+  const ActLayout al = act_layout(blocks ? qtype : CRABML_HIP_Q8_0, n);
+  const size_t o_k = align_up(nq, 256), o_v = align_up(o_k + nkv, 256), o_out = align_up(o_v + nkv, 256), o_pos = align_up(o_out + nq, 256), o_act = o_pos + 256;
   char* base = nullptr;
-  CH_HIP(dev, hipMalloc((void**)&base, o_pos + 256));
+  CH_HIP(dev, hipMalloc((void**)&base, o_act + al.total));
   hipStream_t st = dev->stream;
   const int pos = (int)seq - 1;
+  std::vector<char> act(al.total);
   hipError_t e = hipMemcpyAsync(base, q, nq, hipMemcpyHostToDevice, st);
   if (e == hipSuccess) e = hipMemcpyAsync(base + o_k, k, nkv, hipMemcpyHostToDevice, st);
   if (e == hipSuccess) e = hipMemcpyAsync(base + o_v, v, nkv, hipMemcpyHostToDevice, st);
   if (e == hipSuccess) e = hipMemcpyAsync(base + o_pos, &pos, 4, hipMemcpyHostToDevice, st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);  // (`pos` leaves scope)
   if (e == hipSuccess) {
+    char* a = blocks ? base + o_act : nullptr;
     launch_k(st, nullptr, attn_short_kernel((int)head_dim), dim3((unsigned)n_heads), dim3(512), 0, (const float*)base, (const unsigned short*)(base + o_k),
-             (const unsigned short*)(base + o_v), (const int*)(base + o_pos), (float*)(base + o_out), (signed char*)nullptr,
-             (unsigned short*)nullptr, (void*)nullptr, (int)n_heads, (int)n_kv, (int)head_dim, (int)seq_cap, PrefetchPlan{}, 0);
+             (const unsigned short*)(base + o_v), (const int*)(base + o_pos), (float*)(base + o_out), (signed char*)a,
+             (unsigned short*)(a ? a + al.off_d : nullptr), (void*)(a ? a + al.off_aux : nullptr), (int)n_heads, (int)n_kv, (int)head_dim, (int)seq_cap,
+             PrefetchPlan{}, qtype == CRABML_HIP_Q8_1 ? 1 : 0);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipMemcpyAsync(out, base + o_out, nq, hipMemcpyDeviceToHost, st);
+  if (e == hipSuccess && blocks) e = hipMemcpyAsync(act.data(), base + o_act, al.total, hipMemcpyDeviceToHost, st);
   const hipError_t e2 = hipStreamSynchronize(st);
   (void)hipFree(base);
   CH_HIP(dev, e != hipSuccess ? e : e2);
+  if (blocks) {  // a block: 32 levels, the scale's bits, the sum beside it (Q8_0: the levels' sum; Q8_1: s's bits)
+    int32_t* b = blocks;
+    for (size_t i = 0; i < n / 32; i++, b += 34) {
+      for (int c = 0; c < 32; c++) b[c] = (signed char)act[i * 32 + c];
+      b[32] = ((const uint16_t*)(act.data() + al.off_d))[i];
+      b[33] = qtype == CRABML_HIP_Q8_1 ? (int32_t)((const uint16_t*)(act.data() + al.off_aux))[i] : ((const int32_t*)(act.data() + al.off_aux))[i];
+    }
+  }
   return 0;
 }
 

@@ -122,18 +122,21 @@ PYBIND11_MODULE(_host, m) {
                                                       out.mutable_data(), out2.mutable_data()));
              return py::make_tuple(out, out2);
            })
-      .def("debug_short_attention",
+      .def("debug_short_attention",  // (out, blocks: [n / 32][34], empty without qtype)
            [](HipTensorDevice& d, py::array_t<float, py::array::c_style | py::array::forcecast> q,
               py::array_t<uint16_t, py::array::c_style | py::array::forcecast> k,
               py::array_t<uint16_t, py::array::c_style | py::array::forcecast> v, size_t n_heads, size_t n_kv, size_t head_dim,
-              size_t seq, size_t seq_cap) {
+              size_t seq, size_t seq_cap, uint32_t qtype) {
              if ((size_t)q.size() != n_heads * head_dim || (size_t)k.size() != n_kv * seq_cap * head_dim || k.size() != v.size())
                throw Error(ErrorKind::BadInput, "debug_short_attention: array sizes");
              py::array_t<float> out(n_heads * head_dim);
+             py::array_t<int32_t> blocks(qtype ? n_heads * head_dim / 32 * 34 : 0);
              d.check(crabml_hip_debug_short_attention(d.raw(), q.data(), k.data(), v.data(), n_heads, n_kv, head_dim, seq, seq_cap,
-                                                      out.mutable_data()));
-             return out;
-           })
+                                                      out.mutable_data(), qtype, qtype ? blocks.mutable_data() : nullptr));
+             return py::make_tuple(out, blocks);
+           },
+           py::arg("q"), py::arg("k"), py::arg("v"), py::arg("n_heads"), py::arg("n_kv"), py::arg("head_dim"), py::arg("seq"), py::arg("seq_cap"),
+           py::arg("qtype") = 0)
       .def("debug_flash_attention_rows",
            [](HipTensorDevice& d, py::array_t<float, py::array::c_style | py::array::forcecast> q,
               py::array_t<uint16_t, py::array::c_style | py::array::forcecast> k,

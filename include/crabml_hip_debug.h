@@ -75,9 +75,11 @@ int crabml_hip_debug_flash_attention(crabml_hip_device_t* dev, const float* q, c
                                      size_t n_kv, size_t head_dim, size_t seq, size_t slices, float* out, float* out2);
 
 /* The fast step's short-context attention (k_attn_short) by itself: as above, head_dim a multiple of 8 up to 256, one workgroup per head;
- * k, v: [n_kv][seq_cap][head_dim], of which the first `seq` rows count. */
+ * k, v: [n_kv][seq_cap][head_dim], of which the first `seq` rows count.  blocks (nullable; head_dim % 32 == 0): what the kernel's own quantizer
+ * leaves for wo, qtype Q8_0 or Q8_1, 34 numbers per 32 elements -- the levels, the scale's f16 bits, and the sum of the levels (Q8_0) or the
+ * bits of s (Q8_1). */
 int crabml_hip_debug_short_attention(crabml_hip_device_t* dev, const float* q, const uint16_t* k, const uint16_t* v, size_t n_heads,
-                                     size_t n_kv, size_t head_dim, size_t seq, size_t seq_cap, float* out);
+                                     size_t n_kv, size_t head_dim, size_t seq, size_t seq_cap, float* out, uint32_t qtype, int32_t* blocks);
 
 /* The fast prompt pass's causal attention (k_attn_flash_rows: flash attention on the f16 matrix cores) by itself.  q: rows *
  * n_heads * head_dim f32 (row r is the prompt row at position pos0 + r); k, v: [n_kv][seq_cap][head_dim] f16 bits (the cache

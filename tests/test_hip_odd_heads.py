@@ -27,3 +27,18 @@ def test_decode_against_the_oracle(ca, fmt, dim, hidden, heads, kv, split):
         a, b = got.forward(t, i), want.forward([t], i)
         errs.append(np.max(np.abs(a - b)) / np.max(np.abs(b)))
     assert max(errs) <= FAST_TOL[fmt][1], errs
+
+
+@pytest.mark.parametrize("fmt", ["Q4_0", "Q8_0"])
+@pytest.mark.parametrize("dim,hidden,heads,kv", [(96, 64, 2, 1), (288, 768, 6, 6), (1280, 96, 16, 4)])
+@pytest.mark.parametrize("split", [False, True])
+def test_the_bits_of_the_quantizers_own_launch(ca, monkeypatch, fmt, dim, hidden, heads, kv, split):
+    shape = synth.ModelShape("odd", dim, hidden, 2, heads, kv, 512, 64)
+    dev = ca.HipTensorDevice(0)
+    conf, w = synth.to_hip(synth.build_model(shape, synth.TYPE_BY_NAME[fmt], seed=4), dev)
+    a = ca.HipLlamaRunner(conf, w, dev, 64, True, extra_flags=SPLIT_ALWAYS if split else 0)
+    monkeypatch.setenv("CRABML_HIP_TEST_HOOKS", "1")
+    monkeypatch.setenv("CRABML_HIP_ATTN_ROW_APART", "1")  # (read when a context is made)
+    b = ca.HipLlamaRunner(conf, w, dev, 64, True, extra_flags=SPLIT_ALWAYS if split else 0)
+    for i in range(40):
+        assert np.array_equal(a.forward((7 * i + 1) % 512, i).view(np.uint32), b.forward((7 * i + 1) % 512, i).view(np.uint32)), i

@@ -389,12 +389,15 @@ def test_fast_prompt_pass_rows_write_their_own_f16_planes(ca, fmt, shape, n):
             assert list(a.decode_greedy(nxt, 6)) == list(b.decode_greedy(nxt, 6))
 
 
-# short passes whose tiles leave CUs without work: k in 2 / 4 / 8 pieces (26 chunks of four blocks, or 13 super-blocks: pieces of unequal length;
-# an odd first chunk), rows at both ends of the range and a ragged last row tile
+# short passes whose tiles leave CUs without work.  Width 3328: k in two and four pieces (26 chunks of four blocks, 13 super-blocks: pieces of
+# unequal length; an odd first chunk) and a ragged last row tile, pieces added by their own launch and by the norm behind wo.  Width 4096: eight
+# pieces, ffn_down's left to the next layer's norm.  Rows at both ends of the range.
 @pytest.mark.parametrize("fmt", ["Q4_0", "Q8_0", "Q4_1", "Q4_K"])
 @pytest.mark.parametrize("rows", [16, 17, 31])
-def test_short_passes_in_pieces_of_k_equal_the_token_loop(ca, fmt, rows):
-    shape = synth.ModelShape("pieces", 3328, 1088 if fmt != "Q4_K" else 1280, 1, 26, 2, 300, 64, 1e-5, None)
+@pytest.mark.parametrize("width,layers", [(3328, 1), (4096, 2)])
+def test_short_passes_in_pieces_of_k_equal_the_token_loop(ca, fmt, rows, width, layers):
+    hidden = width if width == 4096 else 1088 if fmt != "Q4_K" else 1280
+    shape = synth.ModelShape("pieces", width, hidden, layers, width // 128, 2, 300, 64, 1e-5, None)
     dev = ca.HipTensorDevice(0)
     conf, w = synth.to_hip(synth.build_model(shape, synth.TYPE_BY_NAME[fmt], seed=91), dev)
     a, b = ca.HipLlamaRunner(conf, w, dev, 64, True), ca.HipLlamaRunner(conf, w, dev, 64, True)

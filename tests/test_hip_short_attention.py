@@ -13,7 +13,7 @@ def attend(dev, q, k, v, n_heads, n_kv, hd, seq, cap):
     """the kernel on a cache whose rows past `seq` are NaN; float64 on the rows that count"""
     kc, vc = (np.full((n_kv, cap, hd), np.nan, np.float16) for _ in range(2))
     kc[:, :seq], vc[:, :seq] = k, v
-    got = dev.debug_short_attention(q, kc.view(np.uint16).reshape(-1), vc.view(np.uint16).reshape(-1), n_heads, n_kv, hd, seq, cap)
+    got, _ = dev.debug_short_attention(q, kc.view(np.uint16).reshape(-1), vc.view(np.uint16).reshape(-1), n_heads, n_kv, hd, seq, cap)
     q16 = q.astype(np.float16).astype(np.float64).reshape(n_heads, hd)
     ref = np.zeros((n_heads, hd))
     with np.errstate(invalid="ignore", over="ignore"):
@@ -56,6 +56,48 @@ def test_infinities_and_nan(ca, hd):
         for bad in (np.inf, np.nan):
             k[0, at, 3] = bad
             assert np.isnan(attend(dev, q, k, v, 1, 1, hd, seq, seq + 8)[0]).all(), (seq, bad)
+
+
+@pytest.mark.parametrize("n_heads,n_kv,hd", [(3, 1, 32), (8, 2, 64), (5, 5, 96), (32, 8, 128), (2, 1, 160), (4, 1, 256)])
+@pytest.mark.parametrize("qtype,name", [(synth.Q8_0, "Q8_0"), (synth.Q8_1, "Q8_1")])
+def test_its_quantizer_is_the_quantizer(ca, n_heads, n_kv, hd, qtype, name):
+    """what the kernel leaves for wo (Q8_0; Q8_1 under Q4_1 layers) is what the stand-alone quantizer makes of its f32 row, bit for bit -- blocks of
+    zeros, of one large element, with infinities and NaN among them"""
+    dev = ca.HipTensorDevice(0)
+    rng = np.random.default_rng(hd + qtype)
+    for seq in (1, 77):
+        q = rng.standard_normal(n_heads * hd).astype(np.float32)
+        k, v = (rng.standard_normal((n_kv, seq, hd)).astype(np.float16) for _ in range(2))
+        v[0, :, 0:32] = 0
+        if hd >= 64:
+            v[-1, :, 32:64], v[-1, :, 40] = 1e-3, 6e4
+        if hd >= 96:
+            v[0, seq - 1, 70] = np.inf
+        if hd >= 128:
+            v[-1, 0, 127] = np.nan
+        out, blocks = dev.debug_short_attention(q, k.view(np.uint16).reshape(-1), v.view(np.uint16).reshape(-1), n_heads, n_kv, hd, seq, seq, qtype=qtype)
+        raw = ca.HipTensor.new(out, [out.size], dev).debug_quantize(getattr(ca.GGMLType, name)).reshape(out.size // 32, -1)
+        blocks = blocks.reshape(-1, 34)
+        assert np.array_equal(blocks[:, :32], raw[:, -32:].view(np.int8)), seq
+        assert np.array_equal(blocks[:, 32], raw[:, :2].copy().view(np.uint16)[:, 0]), seq
+        want = raw[:, -32:].view(np.int8).astype(np.int32).sum(axis=1) if name == "Q8_0" else raw[:, 2:4].copy().view(np.uint16)[:, 0]
+        assert np.array_equal(blocks[:, 33], want), seq
+
+
+def test_q4_1_steps_on_the_short_kernel_equal_the_segment_path(ca):
+    """Q4_1 layers from 96 cached positions: the five-kernel step, whose attention quantizes its own row to Q8_1, against the segments with the
+    quantizer in a launch of its own, bit for bit up to k_attn_flash's first positions"""
+    dev = ca.HipTensorDevice(0)
+    conf, w = synth.to_hip(synth.build_model(synth.SHAPES["tiny-hd128"], synth.Q4_1, seed=62), dev)
+    five = ca.HipLlamaRunner(conf, w, dev, 460, True)
+    segs = ca.HipLlamaRunner(conf, w, dev, 460, True, extra_flags=512)  # CRABML_HIP_LLAMA_Q4_1_SEGMENTS
+    assert [five.debug_graphs(i)[0] for i in (94, 95, 446, 447)] == [0, 3, 3, 2]
+    for i, t in enumerate(int(x) for x in np.random.default_rng(9).integers(0, 1000, size=450)):
+        if 90 <= i < 130 or i >= 440:
+            a, b = five.forward(t, i), segs.forward(t, i)
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), i
+        else:
+            five.forward_async(t, i), segs.forward_async(t, i)
 
 
 @pytest.mark.parametrize("fmt", ["Q8_0", "F16", "Q4_K"])
