@@ -97,7 +97,6 @@ __device__ __forceinline__ int row16_sum_i32(int v) {
 __device__ __forceinline__ float rl_f(float v, int lane) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
 }
-// full-wave (64 lanes): every lane gets the result
 // half waves / neighbouring rows of 16 lanes swap and add: the first half (even rows) gets a's sum, the other half (odd rows) b's
 __device__ __forceinline__ float meet32(float a, float b) {
   const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
@@ -141,6 +140,7 @@ __device__ __forceinline__ float group_sum(float v) {
   if constexpr (LPR == 32) v = meet16(v, v);
   return v;
 }
+// full-wave (64 lanes): every lane gets the result
 __device__ __forceinline__ float wave_sum_f32(float v) {
   v = row16_sum_f32(v);
   return (rl_f(v, 0) + rl_f(v, 16)) + (rl_f(v, 32) + rl_f(v, 48));

@@ -441,7 +441,6 @@ void launch_step_f16(crabml_hip_device* dev, crabml_hip_device::ProfRec* rec, co
       launch_step_f16_t<1, 8, IN, OUT>(dev, rec, a, e);
   }
 }
-constexpr size_t STEP_F16_MAX_K = 16384;  // the longest normalized row (eight pieces of 8 per thread)
 StepF16 step_f16(const crabml_hip_llama* c, std::initializer_list<const crabml_hip_buf*> w, int m, int k, const float* x, const float* gain, float eps, float* out) {
   StepF16 a;
   int i = 0;
@@ -1400,7 +1399,7 @@ int prefill_chunk(crabml_hip_llama* c, const uint32_t* tokens, size_t B, size_t 
       if (!gemm_exact_hook && B >= 16 && (w->dtype == CRABML_HIP_Q4_0 || w->dtype == CRABML_HIP_Q8_0 || w->dtype == CRABML_HIP_Q4_1 || w->dtype == CRABML_HIP_Q4_K) &&
           launch_gemm_mfma(dev, w, m, k, act, B, out, nullptr, nullptr, true, c->pf_split, c->pf_split_floats, defer))
         return 0;
-      return launch_gemv(dev, w, m, k, act, B, out, nullptr, !gemm_exact_hook);
+      return launch_gemv(dev, w, m, k, act, B, out);
     }
     // strict order: the Q4_0 / Q8_0 / Q4_1 MFMA GEMM scales its exact integer tiles block by block in the reference's scalar
     // order, i.e. it IS the strict result (bit for bit) -- the other formats take the scalar-order GEMV row by row
@@ -1521,7 +1520,8 @@ int prefill_chunk(crabml_hip_llama* c, const uint32_t* tokens, size_t B, size_t 
     k_qkv_epi_rows<<<dim3((pairs + 255) / 256, rows), 256, 0, st>>>(c->pf_q, c->pf_k, c->pf_v, e);
     int along = 0;
     // (a pass whose every row sees fewer cached positions than the decode step's switch to the f32 kernels -- attn_long_from --
-    // keeps the exact tile kernel, so that prefill(prompt) and a token loop over the same short prompt agree bit for bit)
+    // keeps the exact tile kernel, so that prefill(prompt) and a token loop over the same short prompt agree bit for bit -- where the step
+    // runs the exact chain there too: not Q4_0 / Q8_0 layers with deferred norms, which run k_attn_short)
     if (c->attn_flash_rows && kv16 && pos0 + B >= c->attn_long_from) {
       // fast step: causal flash attention on the f16 matrix cores (k_attn_flash_rows; the deviation stated for k_attn_flash)
       const dim3 fg((unsigned)((B + 63) / 64), (unsigned)n_heads);
@@ -2028,8 +2028,8 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
   if (ordk && mixed) generic = false;
   c->generic = generic;
   if (const char* hooks = getenv("CRABML_HIP_TEST_HOOKS")) c->attn_row_apart = hooks[0] == '1' && getenv("CRABML_HIP_ATTN_ROW_APART") != nullptr;
-  // (dims are multiples of 32 and heads of 2 by now; a longer row does not fit the launches that normalize it: the per-op segments)
-  c->f16_step = !dev->strict_order && wt == CRABML_HIP_F16 && !mixed && tp == 1 && g.embedding_dim <= STEP_F16_MAX_K && dim_l <= STEP_F16_MAX_K;
+  // (dims are multiples of 32 and heads of 2 by now, rows of at most 12288 elements: the launches that normalize them take 16384)
+  c->f16_step = !dev->strict_order && wt == CRABML_HIP_F16 && !mixed && tp == 1;
   c->ord = ord;
   // Q4_K always; Q4_1 when it cannot take the 5-kernel path (mixed classifier format) or for the A/B flag
   c->kfused = ordk ||

@@ -450,8 +450,9 @@ __host__ __device__ inline size_t attn_s_lds_bytes(int S, int hd) {
 // row is LPR lanes x 16 bytes and a wave instruction takes 64 / LPR rows, straight from the cache into registers: every lane multiplies its
 // eight elements, the LPR lanes of a row add up, and the wave sums p * v over its rows with the weights e^(s - its own maximum); the lanes
 // of one column meet through swaps of half waves and rows, the eight waves once, in LDS.  The arithmetic is k_attn_flash's (q rounded to
-// f16; exact products, f32 exp, weights and sums): closer to exact than the f16 chain, not its bits -- so for the layers whose fast step
-// already leaves the reference's bits (Q4_0 / Q8_0, attn_short in fused.hip), everything else keeps k_attn_s.
+// f16; exact products, f32 exp, weights and sums): closer to exact than the f16 chain, not its bits -- so from the first position only
+// where the fast step already leaves the reference's order (Q4_0 / Q8_0 layers with deferred norms), elsewhere from where k_attn_flash would
+// (attn_short_from in fused.hip); k_attn_s serves what is left.
 // The first 64 rows are requested before the position is known (rows past it are cache memory: read, never used).
 // hd: a multiple of 8, at most 8 LPR (lanes past it hold zeros).
 template <int LPR>

@@ -353,7 +353,7 @@ static void launch_rows(hipStream_t st, int m, int n_cu, F&& f) {
       launch_k(st, rec, ROWS_, dim3(rhs_rows_grid((unsigned)tiles__, rows)), dim3(tpb_), 0, __VA_ARGS__, RhsRows{tiles__, (int)rows, act_stride}); \
   } while (0)
 int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m_, size_t k_, const void* act, size_t b,
-                float* out, crabml_hip_device::ProfRec* rec0, bool fused_add) {
+                float* out, crabml_hip_device::ProfRec* rec0) {
   hipStream_t st = dev->stream;
   const int m = (int)m_, k = (int)k_;
   const char* wp = (const char*)w->ptr;
@@ -381,7 +381,7 @@ int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m_, size
     const void* ws[1] = {wp};
     if (launch_gemm_f16(dev, rec0, ws, &m_, 1, k_, act, al.total, b, &out, GemmScratch{})) return 0;
   }
-  if (b >= 16 && launch_gemm_mfma(dev, w, m_, k_, act, b, out, rec0, nullptr, fused_add)) return 0;
+  if (b >= 16 && launch_gemm_mfma(dev, w, m_, k_, act, b, out, rec0)) return 0;
   const size_t per = rhs_rows_per_launch(m_);
   for (size_t b0 = 0; b0 < b; b0 += per) {
     const size_t rows = b - b0 < per ? b - b0 : per;

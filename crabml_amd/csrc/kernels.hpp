@@ -38,10 +38,8 @@ void launch_quantize_act_rows(hipStream_t st, uint32_t qtype, const float* x, si
 // ---- gemv.hip: W(m,k) x quantized activations (b,k) -> out (b,m)
 // wq: weight planes; aq: activation planes (one set per batch row, stride act_layout(qtype,k).total)
 // rec != nullptr: the (first) kernel is launched with the record's event pair (measurement hook)
-// fused_add (the FAST prompt pass only): a batched rhs's block term takes its second product and the add as one fma -- an explicit
-// argument, never device state: matmul_vec itself is bit-exact and must not pick it up by accident
 int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m, size_t k, const void* act, size_t b,
-                float* out, crabml_hip_device::ProfRec* rec = nullptr, bool fused_add = false);
+                float* out, crabml_hip_device::ProfRec* rec = nullptr);
 // gemv_strict.hip: same contract, block terms added in the reference's scalar order (bit-exact; slow)
 int launch_gemv_strict(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m, size_t k, const void* act, size_t b,
                        float* out, const float* add = nullptr);  // add: out[i] = sum + add[i] (the residual; may alias out)
@@ -76,12 +74,15 @@ bool launch_gemm_f16w(crabml_hip_device* dev, const crabml_hip_buf* const* w, co
 // defer_parts (one matrix): a launch cut into k pieces leaves piece 0 in out and pieces 1.. in ws (b * m floats apart) and returns
 // their number instead of launching the reduce: the row kernel that consumes out adds them first, in piece order (prefill_rows.hpp)
 // gu_exp_tab / gu_done (two matrices = ffn_gate, ffn_up): the launch may store h = silu(g) * u to out[0] instead of g and u (*gu_done = 1)
+
 // gemm_f16.hip: F16 weights x f16 rows (act_stride bytes apart), up to three matrices of one rhs; without scratch k stays whole.
 // false = not covered (one row, rows that are not whole 16-byte pieces)
 struct GemmScratch;
 bool launch_gemm_f16(crabml_hip_device* dev, crabml_hip_device::ProfRec* rec, const void* const* w, const size_t* n, int nw, size_t k,
                      const void* act, size_t act_stride, size_t rows, float* const* out, const GemmScratch& ws);
-// batched rhs on the matrix cores (gemm_mfma.hip); false = not covered
+// batched rhs on the matrix cores (gemm_mfma.hip); false = not covered.  fused_add (the FAST prompt pass only): a Q4_0 / Q8_0 block term takes its
+// second product and the add as one fma, and k may be cut into pieces -- an explicit argument, never device state: matmul_vec itself is
+// bit-exact and must not pick it up by accident
 bool launch_gemm_mfma(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m, size_t k, const void* act, size_t b, float* out,
                       crabml_hip_device::ProfRec* rec, int* dbg = nullptr, bool fused_add = false, float* ws = nullptr, size_t ws_floats = 0,
                       int* defer_parts = nullptr);  // ws, defer_parts: as launch_gemm_f16w's
