@@ -24,7 +24,7 @@ rm -rf $OUT/prof_trait_$TAG
 timeout 400 rocprofv3 --kernel-trace --stats -d $OUT/prof_trait_$TAG -- python $REPO/tools/trait_trace.py 24 > $OUT/trait_trace_$TAG.json 2>> $OUT/prof_$TAG.err
 DB3=$(find $OUT/prof_trait_$TAG -name "*_results.db" | head -1)
 echo "# $TAG the reference's unchanged runner (Llama2Runner<HipTensor>::forward x 24 tokens, 8B shape Q4_0) under rocprofv3 --kernel-trace --stats:" > $OUT/${TAG}_trait_path_kernel_trace.md
-echo "# its ~840 Tensor calls per token are recorded and served by the fused step -- 5 launches per layer (k_qkv, k_attn_s, k_gemv_res_nq x 2, k_gateup_q)" >> $OUT/${TAG}_trait_path_kernel_trace.md
+echo "# its ~840 Tensor calls per token are recorded and served by the fused step -- 5 launches per layer (k_qkv, k_attn_short, k_gemv_res_nq x 2, k_gateup_q)" >> $OUT/${TAG}_trait_path_kernel_trace.md
 echo "# $(cat $OUT/trait_trace_$TAG.json)" >> $OUT/${TAG}_trait_path_kernel_trace.md
 echo >> $OUT/${TAG}_trait_path_kernel_trace.md
 python $REPO/tools/rocpd_summary.py "$DB3" >> $OUT/${TAG}_trait_path_kernel_trace.md 2>> $OUT/prof_$TAG.err
