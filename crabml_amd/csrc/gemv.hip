@@ -515,9 +515,9 @@ int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m_, size
         const unsigned short *wh = (const unsigned short*)wp, *xh = (const unsigned short*)ap;
         if (k % 8 != 0)
           GEMV_LAUNCH((k_gemv_f16_any<>), (k_gemv_f16_any<true>), (m + 3) / 4, 256, wh, xh, o, m, k);
-        else if (m >= 16384)  // (enough rows to give a wave four and still fill the chip)
+        else if (m >= 64 * dev->n_cu)  // (rows a wave: four where that leaves sixteen waves a CU, two where it leaves four)
           GEMV_LAUNCH((k_gemv_f16<4>), (k_gemv_f16<4, true>), (m + 15) / 16, 256, wh, xh, o, m, k);
-        else if (m >= 2048)
+        else if (m >= 8 * dev->n_cu)
           GEMV_LAUNCH((k_gemv_f16<2>), (k_gemv_f16<2, true>), (m + 7) / 8, 256, wh, xh, o, m, k);
         else
           GEMV_LAUNCH((k_gemv_f16<1>), (k_gemv_f16<1, true>), (m + 3) / 4, 256, wh, xh, o, m, k);
