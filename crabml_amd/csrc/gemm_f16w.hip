@@ -3,7 +3,7 @@
 //
 // matmul_vec with a batched rhs is `C[b, m] = W[m, k] . x[b, k]` (matmul_vec.rs:41-76: the (b, k) rhs contract; llama2.rs:111-129).
 // The bit-exact form (gemm_mfma.hip: exact int8 tiles, then the reference's per-block `sumf += (sumi as f32 * d_w) * d_x`) pays
-// 8-10 VALU operations per MFMA for that scaling -- it is VALU-issue-bound at 14 % MfmaUtil (profiles/r05_prefill_gemm_experiments.md).
+// 12-16 VALU operations per MFMA for that scaling -- it is VALU-issue-bound at 14 % MfmaUtil (profiles/r05_prefill_gemm_experiments.md).
 // Here the block scales are folded into the OPERANDS and the sum runs in f32 inside the matrix core across all blocks:
 //   A' = (q_w - 8) * d_w   as f16: q_w - 8 exact, ONE rounding of the product (v_pk_mul_f16)
 //   B' = q_x * d_x         as f16: one rounding (k_q8_0_rows_to_f16: once per activation matrix, not per weight row tile)
@@ -13,7 +13,7 @@
 //
 // Tiling (what round 5's f16 experiment lacked): a wave owns F 16-row fragments x T = 8 column tiles of 16 prompt rows and unpacks
 // each A fragment ONCE per 32 k-slots -- 15 VALU operations -- for T MFMAs: 15 F / (F T) < 2 VALU per MFMA, 0.9 with the staging
-// amortized (the int8 kernel: 10.75).  A fragments come straight from global memory in MFMA layout: lane (i, g) loads the whole
+// amortized (the int8 kernel: 12 for its scaling alone).  A fragments come straight from global memory in MFMA layout: lane (i, g) loads the whole
 // 16-byte block kb0 + g of row i (64 contiguous bytes per row and chunk) and step s = 0..3 of the chunk feeds dword s of every
 // lane -- an MFMA's 32 k-slots then span FOUR blocks (8 elements of each), which the folded scales allow.  B' tiles (128 columns x
 // 128 k-slots x 2 B = 32 KB per chunk) go through LDS, double-buffered, one barrier per chunk, shared by the workgroup's four waves;

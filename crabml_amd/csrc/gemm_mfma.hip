@@ -6,7 +6,7 @@
 // sum_k w[i][k] x[j][k] of the 16 x 16 tile, which are then scaled exactly as the reference's scalar loop does,
 // `sumf += (sumi as f32 * d_w) * d_x` (buf_q4_0.rs:249, buf_q8_0.rs:282), block after block in order -- so each
 // output equals the reference's scalar-order result bit for bit (the per-block scales forbid accumulating across
-// blocks inside the MFMA, which also bounds its utilisation: 4 conversions + 8 f32 ops per lane per MFMA).
+// blocks inside the MFMA, which also bounds its utilisation: 4 conversions + 12 f32 ops per lane per MFMA).
 //
 // MFMA operand layout (16x16x32 i8): lane l supplies, for A, 8 k-slots of row i = l & 15 and, for B, the same 8
 // k-slots of column j = l & 15; k-slot group = l >> 4.  The product is invariant under any permutation of the 32
@@ -46,7 +46,7 @@ struct GemmGeo {
 };
 
 // PASS: the fast prompt pass (crabml_hip_llama_prefill).  Its Q4_0 / Q8_0 sums are sumf = fma(sumi as f32 * d_w, d_x, sumf) -- the block term's
-// second product and the add as one v_pk_fma_f32 (8 instead of 10 VALU operations per MFMA; one rounding fewer than the reference's
+// second product and the add as one v_fma_f32 (12 instead of 16 VALU operations per MFMA; one rounding fewer than the reference's
 // expression, the same distance the fast decode step's re-associated sums are allowed).  matmul_vec itself and the strict-order
 // device keep the reference's three roundings (bit-exact, tests/test_hip_gemv.py).
 // Its k may be cut into gridDim.y pieces (a power of two): that many workgroups per tile, each over its chunks; piece s >= 1 leaves its sums
@@ -180,8 +180,7 @@ __global__ __launch_bounds__(256) void k_gemm_mfma(const char* __restrict__ wq, 
     }
   };
 
-  // accumulators as f32 pairs: the block scaling runs on v_pk_mul_f32 / v_pk_add_f32 (same IEEE operations, two
-  // rows per instruction)
+  // accumulators as f32 pairs, two rows each (the instructions are scalar: packed FP32 is off)
   f32x2 F[NT][2];
   float Fq[NT][4];  // Q4_1 only: scalar accumulators (element-wise updates of the ext-vector ones were miscompiled)
 #pragma unroll
