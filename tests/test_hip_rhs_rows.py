@@ -42,3 +42,18 @@ def test_more_threads_than_a_launch_holds(ca, fmt, strict, m, k):
     for r in (0, 127, 254, 255, 256):
         one = w.matmul_vec(ca.HipTensor.new(x[r], [k], dev)).export()
         assert np.array_equal(got[r].view(np.uint32), one.view(np.uint32)), r
+
+
+@pytest.mark.parametrize("fmt", ["F32", "F16", "Q5_K"])
+# tiles of 64 rows against 256 CUs' room for 1024: seven rows of the rhs a launch and a remainder, one a launch
+@pytest.mark.parametrize("m,rows", [(8210, 16), (65600, 3)])
+def test_lane_per_row_kernel_over_several_launches(ca, fmt, m, rows):
+    """the strict device's lane-per-row kernel takes no more rows of the rhs at once than the CUs hold lines for"""
+    rng = np.random.default_rng(m)
+    dev = ca.HipTensorDevice(0, False, 0, True)
+    w = ca.HipTensor.from_cpu(synth.random_blocks(rng, m * 256, synth.TYPE_BY_NAME[fmt]), [m, 256], getattr(ca.GGMLType, HT[fmt]), dev)
+    x = rng.standard_normal((rows, 256)).astype(np.float32)
+    got = w.matmul_vec(ca.HipTensor.new(x.reshape(-1), [rows, 256], dev)).export().reshape(rows, m)
+    for r in range(rows):
+        one = w.matmul_vec(ca.HipTensor.new(x[r], [256], dev)).export()
+        assert np.array_equal(got[r].view(np.uint32), one.view(np.uint32)), r
