@@ -15,7 +15,7 @@
 //   k_attn         batch_matmul(q,K^T) + softmax_inplace + batch_matmul(p,V) [+ quantize for wo]
 //   k_gemv_res     wo / ffn_down matmul_vec + add_inplace(residual)
 //   k_gateup       ffn_gate/ffn_up matmul_vec + silu_inplace + mul_inplace
-//   k_argmax_step  greedy sampler (last maximum) + token/position advance
+//   k_step_front   greedy sampler (last maximum) + token/position advance, embedding, first norm (+ quantize)
 #include <chrono>
 #include <thread>
 #include <cmath>
@@ -159,8 +159,15 @@ struct crabml_hip_llama {
   // by attn_variant
   hipGraph_t graph[4] = {nullptr, nullptr, nullptr, nullptr};
   hipGraphExec_t exec[4] = {nullptr, nullptr, nullptr, nullptr};
+  // ... and of several steps (multi_steps) behind one another: a graph's two ends cost 6 to 7 us between two launches (measured with 35 and
+  // 140 small kernels), which a greedy run of a small model pays for every token
+  hipGraph_t multi_graph[4] = {nullptr, nullptr, nullptr, nullptr};
+  hipGraphExec_t multi_exec[4] = {nullptr, nullptr, nullptr, nullptr};
+  static constexpr size_t MULTI_STEPS = 8, MULTI_NODES = 384;  // (161 launches a step, 32 layers: the gap is half a percent, two steps)
+  int multi_steps = 1;
   bool use_graph = false;
   bool capturing = false;
+  bool lead = false;  // a step ends with the next one's front (enqueue_front): steps that follow each other on this device without the host
   int attn_variant = 0;         // which of them the next enqueue emits: 0 = one workgroup per head, 1 = the long-context kernels,
                                 // 2 = split-KV attention with the merge inside the launch (ticket form: the mid range), 3 = k_attn_short
   size_t flash_ticket_until = 0;  // > 0: positions [attn_long_from, this) run variant 2
@@ -457,6 +464,63 @@ StepF16 step_f16(const crabml_hip_llama* c, std::initializer_list<const crabml_h
   return a;
 }
 
+PrefetchPlan prefetch_plan(const crabml_hip_llama* c, const crabml_hip_buf* a, const crabml_hip_buf* b, const crabml_hip_buf* cc) {
+  PrefetchPlan pf{};
+  const bool on = !(c->cfg.flags & CRABML_HIP_LLAMA_NO_PREFETCH);
+  const crabml_hip_buf* v[3] = {a, b, cc};
+  for (int i = 0; i < 3; i++) {
+    pf.p[i] = on && v[i] ? v[i]->ptr : nullptr;
+    pf.n[i] = on && v[i] ? (v[i]->wl.total / 16) * 16 : 0;
+  }
+  pf.sink = c->state + 3;
+  return pf;
+}
+
+// The front of a step (k_step_front): embedding, and what the first launch of layer 0 reads.  pick: behind the sampler's partials, for the
+// token they name; otherwise for the token in `state`.
+int enqueue_front(crabml_hip_llama* c, bool pick) {
+  crabml_hip_device* dev = c->dev;
+  const auto& g = c->cfg;
+  const int dim = (int)g.embedding_dim;
+  const bool prof = dev->prof_on && !c->use_graph && !c->capturing;
+  crabml_hip_device::ProfRec nr{};
+  const bool k = c->kfused && c->wtype == CRABML_HIP_Q4_K;
+  const int front = !c->kfused && (c->f16_step || c->generic) ? FRONT_ROW : k ? FRONT_Q8_K : c->wtype == CRABML_HIP_Q4_1 ? FRONT_Q8_1 : FRONT_Q8_0;
+  TokenPick tp;
+  tp.token = c->state;
+  if (pick) {
+    tp.pv = c->am_val;
+    tp.pi = c->am_idx;
+    tp.nparts = ARGMAX_BLOCKS;
+    tp.out_cap = c->out_cap;
+    tp.pos = c->state + 1;
+    tp.step = c->state + 2;
+    tp.serial = c->state + 4;
+    tp.out = c->out_tokens;
+  }
+  const ActLayout al = act_layout(k ? CRABML_HIP_Q8_K : front == FRONT_Q8_1 ? CRABML_HIP_Q8_1 : CRABML_HIP_Q8_0, (size_t)dim);
+  const FrontOut o{(signed char*)c->act_dim, (signed char*)(c->act_dim + al.off_p), (void*)(c->act_dim + al.off_d), (void*)(c->act_dim + al.off_aux)};
+  const bool weights = front == FRONT_Q8_0 || front == FRONT_Q8_1;
+  const PrefetchPlan pf = weights ? prefetch_plan(c, c->wq[0], c->wk[0], c->wv[0]) : PrefetchPlan{};
+  const int spare = weights && !(g.flags & CRABML_HIP_LLAMA_NO_PREFETCH) && dev->n_cu > 1 ? dev->n_cu - 1 : 0;
+  auto go = [&](auto kernel) {
+    launch_k(dev->stream, prof ? &nr : nullptr, kernel, dim3(1 + spare), dim3(1024), front == FRONT_ROW ? 0 : norm_lds_bytes(dim),
+             (const char*)c->token_embed->ptr, (int)c->token_embed->dtype, c->token_embed->wl.off_scale, tp, dim, c->x, (const float*)c->rms_att[0]->ptr,
+             g.rms_norm_eps, o, pf, dev->strict_order ? 0 : 1);
+  };
+  if (prof) CH_TRY(prof_begin(dev, &nr, CRABML_HIP_F32, 6, 8.0 * dim));
+  const bool narrow = dim <= 4096;
+  switch (front) {
+    case FRONT_ROW: narrow ? go(k_step_front<4, FRONT_ROW>) : go(k_step_front<12, FRONT_ROW>); break;
+    case FRONT_Q8_0: narrow ? go(k_step_front<4, FRONT_Q8_0>) : go(k_step_front<12, FRONT_Q8_0>); break;
+    case FRONT_Q8_1: narrow ? go(k_step_front<4, FRONT_Q8_1>) : go(k_step_front<12, FRONT_Q8_1>); break;
+    default: narrow ? go(k_step_front<4, FRONT_Q8_K>) : go(k_step_front<12, FRONT_Q8_K>);
+  }
+  if (prof) CH_TRY(prof_end(dev, &nr));
+  CH_HIP(dev, hipGetLastError());
+  return 0;
+}
+
 // the tail of the final segment: classifier GEMV over this rank's rows (all of them unless the vocabulary is split,
 // llama2.rs:199-208) + greedy sampler + advance
 int enqueue_classifier_and_sampler(crabml_hip_llama* c, const void* cls_act, crabml_hip_device::ProfRec* R) {
@@ -484,6 +548,7 @@ int enqueue_classifier_and_sampler(crabml_hip_llama* c, const void* cls_act, cra
     return 0;
   }
   k_argmax_partial<<<ARGMAX_BLOCKS, 256, 0, st>>>(out, c->vocab_l, c->am_val, c->am_idx, c->vocab_off, 0);
+  if (c->lead) return enqueue_front(c, true);
   if (c->split_vocab && c->comm && c->comm->p2p)
     k_argmax_step_tp<<<1, 64, 0, st>>>(c->am_val, c->am_idx, ARGMAX_BLOCKS, token_d, pos_d, step_d, c->out_tokens, c->out_cap, c->state + 4,
                                        tp_view(c, true), n_segments(c));
@@ -507,7 +572,6 @@ int enqueue_segment_t(crabml_hip_llama* c, int seg) {
   const bool kv16 = g.use_f16_kv_cache != 0;
   const bool tp = c->tp > 1;
   const int L = (int)g.n_layers;
-  int* token_d = c->state;
   int* pos_d = c->state + 1;
   constexpr bool Q81 = FMT == CRABML_HIP_Q4_1;
   const uint32_t qt = c->qt;
@@ -522,16 +586,7 @@ int enqueue_segment_t(crabml_hip_llama* c, int seg) {
   crabml_hip_device::ProfRec pr{};
   crabml_hip_device::ProfRec* R = prof ? &pr : nullptr;
   const bool do_pf = !(g.flags & CRABML_HIP_LLAMA_NO_PREFETCH);
-  auto plan = [&](const crabml_hip_buf* a, const crabml_hip_buf* b, const crabml_hip_buf* cc) {
-    PrefetchPlan pf{};
-    const crabml_hip_buf* v[3] = {a, b, cc};
-    for (int i = 0; i < 3; i++) {
-      pf.p[i] = do_pf && v[i] ? v[i]->ptr : nullptr;
-      pf.n[i] = do_pf && v[i] ? (v[i]->wl.total / 16) * 16 : 0;
-    }
-    pf.sink = c->state + 3;
-    return pf;
-  };
+  auto plan = [&](const crabml_hip_buf* a, const crabml_hip_buf* b, const crabml_hip_buf* cc) { return prefetch_plan(c, a, b, cc); };
   const int spare = do_pf ? (dev->n_cu > 1 ? dev->n_cu - 1 : 0) : 0;
   const size_t norm_lds = norm_lds_bytes(dim);
   // rmsnorm * weight -> act_dim; with tp the previous segment's all-reduced output is folded into x first
@@ -686,12 +741,12 @@ int enqueue_segment_t(crabml_hip_llama* c, int seg) {
   }
   const int l = seg / 2;
   if ((seg & 1) == 0) {
-    if (l == 0)
-      k_embed<<<(dim + 255) / 256, 256, 0, st>>>((const char*)c->token_embed->ptr, (int)c->token_embed->dtype,
-                                                  c->token_embed->wl.off_scale, token_d, dim, c->x);
-    // attention rmsnorm (llama2.rs:230-234)
-    if (!norm_epi || l == 0)
-      norm_quant((const float*)c->rms_att[l]->ptr, g.rms_norm_eps, tp && l > 0, plan(c->wq[l], c->wk[l], c->wv[l]));
+    // embedding and attention rmsnorm (llama2.rs:222-234)
+    if (l == 0) {
+      if (!c->lead) CH_TRY(enqueue_front(c, false));
+    } else if (!norm_epi) {
+      norm_quant((const float*)c->rms_att[l]->ptr, g.rms_norm_eps, tp, plan(c->wq[l], c->wk[l], c->wv[l]));
+    }
     // q, k, v + rope + scale + KV append (llama2.rs:244-256, 542-554, 561-565), local heads only
     QkvEpi e{c->qbuf, c->kc[l], c->vc[l], c->rope, pos_d, 1.0f / std::sqrt((float)hd), dim_l, kv_dim_l, hd,
              (int)g.rope_dim, c->npairs, seq_cap, kv16 ? 1 : 0};
@@ -766,7 +821,6 @@ int enqueue_segment_generic(crabml_hip_llama* c, int seg) {
   const bool strict = dev->strict_order;
   const bool tp = c->tp > 1;
   const int L = (int)g.n_layers;
-  int* token_d = c->state;
   int* pos_d = c->state + 1;
   const bool prof = dev->prof_on && !c->use_graph && !c->capturing && !strict;
   crabml_hip_device::ProfRec pr{};
@@ -808,9 +862,7 @@ int enqueue_segment_generic(crabml_hip_llama* c, int seg) {
   }
   const int l = seg / 2;
   if ((seg & 1) == 0) {
-    if (l == 0)
-      k_embed<<<(dim + 255) / 256, 256, 0, st>>>((const char*)c->token_embed->ptr, (int)c->token_embed->dtype,
-                                                  c->token_embed->wl.off_scale, token_d, dim, c->x);
+    if (l == 0 && !c->lead) CH_TRY(enqueue_front(c, false));
     norm((const float*)c->rms_att[l]->ptr, g.rms_norm_eps, tp && l > 0);
     const void* act = quant(c->xn, dim, c->qt, c->act_dim);
     QkvEpi e{c->qbuf, c->kc[l], c->vc[l], c->rope, pos_d, 1.0f / std::sqrt((float)hd), dim_l, kv_dim_l, hd,
@@ -879,8 +931,7 @@ int enqueue_segment_f16(crabml_hip_llama* c, int seg) {
   }
   const int l = seg / 2;
   if ((seg & 1) == 0) {
-    if (l == 0)
-      k_embed<<<(dim + 255) / 256, 256, 0, st>>>((const char*)c->token_embed->ptr, (int)c->token_embed->dtype, c->token_embed->wl.off_scale, c->state, dim, c->x);
+    if (l == 0 && !c->lead) CH_TRY(enqueue_front(c, false));
     const QkvEpi e{c->qbuf, c->kc[l], c->vc[l], c->rope, c->state + 1, 1.0f / std::sqrt((float)hd), dim_l, kv_dim_l, hd,
                    (int)g.rope_dim, c->npairs, (int)g.seq_len, g.use_f16_kv_cache ? 1 : 0};
     CH_TRY(P0(1, dim_l + 2.0 * kv_dim_l, dim));
@@ -919,7 +970,6 @@ int enqueue_segment_k(crabml_hip_llama* c, int seg) {
   const bool kv16 = g.use_f16_kv_cache != 0;
   const bool tp = c->tp > 1;
   const int L = (int)g.n_layers;
-  int* token_d = c->state;
   int* pos_d = c->state + 1;
   const bool prof = dev->prof_on && !c->use_graph && !c->capturing;
   crabml_hip_device::ProfRec pr{};
@@ -1038,10 +1088,11 @@ int enqueue_segment_k(crabml_hip_llama* c, int seg) {
   }
   const int l = seg / 2;
   if ((seg & 1) == 0) {
-    if (l == 0)
-      k_embed<<<(dim + 255) / 256, 256, 0, st>>>((const char*)c->token_embed->ptr, (int)c->token_embed->dtype,
-                                                  c->token_embed->wl.off_scale, token_d, dim, c->x);
-    if (!nepi || l == 0) norm_quant((const float*)c->rms_att[l]->ptr, g.rms_norm_eps, tp && l > 0, QT);
+    if (l == 0) {
+      if (!c->lead) CH_TRY(enqueue_front(c, false));
+    } else if (!nepi) {
+      norm_quant((const float*)c->rms_att[l]->ptr, g.rms_norm_eps, tp, QT);
+    }
     QkvEpi e{c->qbuf, c->kc[l], c->vc[l], c->rope, pos_d, 1.0f / std::sqrt((float)hd), dim_l, kv_dim_l, hd,
              (int)g.rope_dim, c->npairs, seq_cap, kv16 ? 1 : 0};
     const int total_rows = dim_l + 2 * kv_dim_l;
@@ -1171,6 +1222,46 @@ int run_step(crabml_hip_llama* c, size_t pos) {
   return enqueue_step(c);
 }
 
+
+// `n` decode steps from cache position `pos` on: as many at a time as one graph holds, as long as they take the same attention form
+int run_steps(crabml_hip_llama* c, size_t pos, size_t n) {
+  for (size_t i = 0; i < n;) {
+    const int v = variant_of(c, pos + i);
+    size_t m = 0;
+    if (c->use_graph && c->multi_exec[v] && n - i >= (size_t)c->multi_steps)
+      while (m < (size_t)c->multi_steps && variant_of(c, pos + i + m) == v) m++;
+    if (m > 0 && m == (size_t)c->multi_steps) {
+      CH_HIP(c->dev, hipGraphLaunch(c->multi_exec[v], c->dev->stream));
+      i += m;
+    } else {
+      CH_TRY(run_step(c, pos + i));
+      i++;
+    }
+  }
+  return 0;
+}
+
+// `steps` decode steps of attention form `variant` as a graph (token / pos / step are read from device memory by the kernels)
+bool capture_steps(crabml_hip_llama* c, int variant, int steps, hipGraph_t* graph_out, hipGraphExec_t* exec_out) {
+  hipStream_t st = c->dev->stream;
+  if (hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal) != hipSuccess) return false;
+  c->capturing = true;
+  c->attn_variant = variant;
+  int rc = 0;
+  for (int i = 0; i < steps && rc == 0; i++) rc = enqueue_step(c);
+  c->capturing = false;
+  c->attn_variant = 0;
+  hipGraph_t graph = nullptr;
+  const hipError_t e = hipStreamEndCapture(st, &graph);
+  hipGraphExec_t exec = nullptr;
+  if (rc == 0 && e == hipSuccess && graph && hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) == hipSuccess) {
+    *graph_out = graph;
+    *exec_out = exec;
+    return true;
+  }
+  if (graph) (void)hipGraphDestroy(graph);
+  return false;
+}
 
 // ---- batched prefill ---------------------------------------------------------------------------------------
 // B prompt rows at positions pos0 .. pos0 + B - 1 through every layer as (B, k) matmul_vec calls (launch_gemv: MFMA
@@ -2302,7 +2393,8 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
       return hip_fail(dev, e, "llama init", __FILE__, __LINE__);
     }
   }
-  // capture one decode step into a graph (token / pos / step are read from device memory by the kernels).
+  c->lead = tp == 1 && !c->ext_kv && !c->split_vocab;
+  // capture one decode step into a graph.
   // tp > 1 without a communicator = a rank of the single-device simulation: driven segment by segment, no graph.
   // tp > 1 over RCCL launches eagerly unless CRABML_HIP_LLAMA_TP_GRAPH asks for the collectives to be captured too.
   const bool want_graph = !(g.flags & CRABML_HIP_LLAMA_NO_GRAPH) &&
@@ -2314,31 +2406,15 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
     bool ok = true;
     for (int v = 0; v < 4 && ok; v++) {
       if (!has[v]) continue;
-      ok = false;
-      hipError_t e = hipStreamBeginCapture(dev->stream, hipStreamCaptureModeThreadLocal);
-      if (e != hipSuccess) break;
-      c->capturing = true;
-      c->attn_variant = v;
-      int erc = enqueue_step(c);
-      c->capturing = false;
-      hipGraph_t graph = nullptr;
-      hipError_t e2 = hipStreamEndCapture(dev->stream, &graph);
-      if (erc == 0 && e2 == hipSuccess && graph) {
-        hipGraphExec_t exec = nullptr;
-        if (hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) == hipSuccess) {
-          c->graph[v] = graph;
-          c->exec[v] = exec;
-          ok = true;
-        } else {
-          (void)hipGraphDestroy(graph);
-        }
-      } else if (graph) {
-        (void)hipGraphDestroy(graph);
-      }
+      ok = capture_steps(c, v, 1, &c->graph[v], &c->exec[v]);
+      // several steps in a graph where a step is short enough for the gap between two graphs to show
+      size_t nodes = 0;
+      if (!ok || !c->lead || hipGraphGetNodes(c->graph[v], nullptr, &nodes) != hipSuccess || nodes == 0) continue;
+      if (c->multi_steps == 1) c->multi_steps = (int)std::min({crabml_hip_llama::MULTI_STEPS + 0, crabml_hip_llama::MULTI_NODES / nodes, (size_t)g.seq_len / 2});
+      if (c->multi_steps > 1) (void)capture_steps(c, v, c->multi_steps, &c->multi_graph[v], &c->multi_exec[v]);
     }
     (void)hipGetLastError();
     c->use_graph = ok;
-    c->attn_variant = 0;
     if (!ok && tp == 1) {  // fail loudly: the caller asked for the graph path
       crabml_hip_llama_destroy(c);
       CH_BAIL(dev, CRABML_HIP_UNEXPECTED, "llama: hipGraph capture/instantiate failed");
@@ -2370,6 +2446,8 @@ int crabml_hip_llama_destroy(crabml_hip_llama_t* c) {
   for (int v = 0; v < 4; v++) {
     if (c->exec[v]) (void)hipGraphExecDestroy(c->exec[v]);
     if (c->graph[v]) (void)hipGraphDestroy(c->graph[v]);
+    if (c->multi_exec[v]) (void)hipGraphExecDestroy(c->multi_exec[v]);
+    if (c->multi_graph[v]) (void)hipGraphDestroy(c->multi_graph[v]);
   }
   for (auto& a : c->allocs) pool_free(c->dev, a.first, a.second);
   for (auto* b : c->held) crabml_hip_buf_release(b);
@@ -2397,6 +2475,7 @@ int crabml_hip_llama_forward(crabml_hip_llama_t* c, size_t token, size_t pos, fl
     CH_BAIL(dev, CRABML_HIP_BAD_INPUT, "llama: a tp rank without a communicator is driven by crabml_hip_llama_tp_sim_*");
   CH_TRY(check_step(c, token, pos));
   CH_TRY(set_state(c, token, pos, 0));
+  if (c->lead) CH_TRY(enqueue_front(c, false));
   CH_TRY(run_step(c, pos));
   c->kv_len++;
   if (logits) {
@@ -2423,7 +2502,8 @@ int crabml_hip_llama_decode_greedy(crabml_hip_llama_t* c, size_t token, size_t n
     CH_BAIL(dev, CRABML_HIP_TENSOR_ERROR, "llama: %zu steps do not fit the kv cache (%zu of %zu used)", n_steps, c->kv_len, c->cfg.seq_len);
   if (n_steps == 0) return 0;
   CH_TRY(set_state(c, token, c->kv_len, 0));
-  for (size_t s = 0; s < n_steps; s++) CH_TRY(run_step(c, c->kv_len + s));
+  if (c->lead) CH_TRY(enqueue_front(c, false));
+  CH_TRY(run_steps(c, c->kv_len, n_steps));
   c->kv_len += n_steps;
   int fault = 0;
   CH_HIP(dev, hipMemcpyAsync(out_tokens, c->out_tokens, n_steps * 4, hipMemcpyDeviceToHost, dev->stream));
@@ -2488,6 +2568,7 @@ int crabml_hip_llama_tp_sim_forward(crabml_hip_llama_t* const* ranks, int n, siz
   for (int r = 0; r < n; r++) ptrs.p[r] = ranks[r]->partial;
   const int dim = (int)ranks[0]->cfg.embedding_dim;
   for (int r = 0; r < n; r++) ranks[r]->attn_variant = variant_of(ranks[r], pos);
+  if (ranks[0]->lead) CH_TRY(enqueue_front(ranks[0], false));  // (n == 1)
   for (int s = 0; s < nseg; s++) {
     for (int r = 0; r < n; r++) CH_TRY(enqueue_segment(ranks[r], s));
     if (n > 1 && s + 1 < nseg) k_sim_allreduce<<<(dim + 255) / 256, 256, 0, dev->stream>>>(ptrs, n, dim);

@@ -5,6 +5,8 @@
 #include "dequant.hpp"
 #include "gemv_core.hpp"
 #include "kernels.hpp"
+#include "sampler.hpp"
+#include <type_traits>
 
 namespace crabml_hip {
 
@@ -160,26 +162,12 @@ struct NormLds {  // carved from dynamic LDS: xs[cols] f32 | chunk_sums[cols/32]
 __host__ __device__ inline size_t norm_lds_bytes(int cols) { return (size_t)(cols + cols / 32) * sizeof(float); }
 
 // QUANT = false: the normalized row goes to xn_out as f32 (formats whose rhs is not Q8_0 quantize it afterwards)
-template <int NIT, bool QUANT, bool Q81 = false>  // cols <= NIT * 1024, blockDim.x == 1024; ends with the outputs written
-__device__ __forceinline__ void norm_quant_block(float* __restrict__ x, const float* __restrict__ addv,
-                                                 const float* __restrict__ w, int cols, float eps, NormLds L,
-                                                 float* s_rms, signed char* q, unsigned short* d, void* isum,
-                                                 float* __restrict__ xn_out, int half) {
+// xv, wv: this thread's elements it * 1024 + tid of the row and of the gain (0 past the end); cols <= NIT * 1024, blockDim.x == 1024
+template <int NIT, bool QUANT, bool Q81 = false>
+__device__ __forceinline__ void norm_quant_regs(const float (&xv)[NIT], const float (&wv)[NIT], int cols, float eps, NormLds L, float* s_rms,
+                                                signed char* q, unsigned short* d, void* isum, float* xn_out, int half) {
   const int nchunks = cols / 32;
   const int tid = threadIdx.x;
-  float xv[NIT], wv[NIT];
-#pragma unroll
-  for (int it = 0; it < NIT; it++) {
-    int i = it * 1024 + tid;
-    xv[it] = i < cols ? x[i] : 0.f;
-    wv[it] = i < cols ? w[i] : 0.f;
-    // tensor-parallel: the all-reduced wo / ffn_down output is added to the residual stream here
-    // (x = matmul_out + x, llama2.rs:266 / :636) and written back
-    if (addv != nullptr && i < cols) {
-      xv[it] = addv[i] + xv[it];
-      x[i] = xv[it];
-    }
-  }
 #pragma unroll
   for (int it = 0; it < NIT; it++) {
     int i = it * 1024 + tid;
@@ -244,6 +232,27 @@ __device__ __forceinline__ void norm_quant_block(float* __restrict__ x, const fl
     }
   }
 }
+template <int NIT, bool QUANT, bool Q81 = false>  // cols <= NIT * 1024, blockDim.x == 1024; ends with the outputs written
+__device__ __forceinline__ void norm_quant_block(float* __restrict__ x, const float* __restrict__ addv,
+                                                 const float* __restrict__ w, int cols, float eps, NormLds L,
+                                                 float* s_rms, signed char* q, unsigned short* d, void* isum,
+                                                 float* __restrict__ xn_out, int half) {
+  const int tid = threadIdx.x;
+  float xv[NIT], wv[NIT];
+#pragma unroll
+  for (int it = 0; it < NIT; it++) {
+    int i = it * 1024 + tid;
+    xv[it] = i < cols ? x[i] : 0.f;
+    wv[it] = i < cols ? w[i] : 0.f;
+    // tensor-parallel: the all-reduced wo / ffn_down output is added to the residual stream here
+    // (x = matmul_out + x, llama2.rs:266 / :636) and written back
+    if (addv != nullptr && i < cols) {
+      xv[it] = addv[i] + xv[it];
+      x[i] = xv[it];
+    }
+  }
+  norm_quant_regs<NIT, QUANT, Q81>(xv, wv, cols, eps, L, s_rms, q, d, isum, xn_out, half);
+}
 
 template <int NIT, bool Q81>
 __global__ __launch_bounds__(1024) void k_norm_quant(float* __restrict__ x, const float* __restrict__ addv,
@@ -266,6 +275,105 @@ __global__ __launch_bounds__(1024) void k_norm_f32(float* __restrict__ x, const 
   __shared__ float s_rms;
   NormLds L{lds, lds + cols};
   norm_quant_block<NIT, false>(x, addv, w, cols, eps, L, &s_rms, nullptr, nullptr, nullptr, xn, half);
+}
+
+// ---- the front of a decode step in one launch: sampler's second stage, embedding, first norm, its quantizer -------------
+// These were four launches at a step's two ends (combine the arg-max partials, embedding, norm, quantizer of a Q8_K rhs): each is one
+// round trip to memory behind 1.7 us of launch.  One workgroup does all of it: every wave combines the partials for itself (two
+// requests a lane), so the token is known without a barrier; the row's elements are requested together whatever the table's format is.
+// A context whose steps follow each other on the device (`lead`, fused.hip) runs it at the END of a step, for the next one.
+// With several steps in a graph (run_steps), us a request, before -> after: 57 tokens of the 15M-parameter model in Q8_0 6482 -> 6047, 88 tokens of 8
+// layers of the 8B shape in Q4_0 24840 -> 24232.
+enum { FRONT_ROW = 0, FRONT_Q8_0 = 1, FRONT_Q8_1 = 2, FRONT_Q8_K = 3 };  // what is left beside x: nothing, or the normed row's planes
+struct TokenPick {  // pv == nullptr: the token is *token
+  const float* pv = nullptr;
+  const int* pi = nullptr;
+  int nparts = 0, out_cap = 0;
+  int *token = nullptr, *pos = nullptr, *step = nullptr, *serial = nullptr;
+  unsigned* out = nullptr;
+};
+struct FrontOut {
+  signed char *q = nullptr, *qp = nullptr;  // (qp: class-major copy, Q8_K)
+  void *d = nullptr, *aux = nullptr;        // scales; block sums
+};
+template <int NIT>
+__device__ __forceinline__ void embed_row(const char* __restrict__ w, int dtype, size_t off_scale, size_t base, int dim, float (&v)[NIT]) {
+  // (one format at a time: with the format's switch inside the loop each element's request waited for the one before it)
+  auto all = [&](auto t) {
+#pragma unroll
+    for (int it = 0; it < NIT; it++) {
+      const int i = it * 1024 + (int)threadIdx.x;
+      const float e = dequant_elem(w, decltype(t)::value, off_scale, base + (i < dim ? i : dim - 1));
+      v[it] = i < dim ? e : 0.f;
+    }
+  };
+  switch (dtype) {
+    case CRABML_HIP_Q4_0: all(std::integral_constant<int, CRABML_HIP_Q4_0>()); break;
+    case CRABML_HIP_Q8_0: all(std::integral_constant<int, CRABML_HIP_Q8_0>()); break;
+    case CRABML_HIP_Q4_1: all(std::integral_constant<int, CRABML_HIP_Q4_1>()); break;
+    case CRABML_HIP_Q4_K: all(std::integral_constant<int, CRABML_HIP_Q4_K>()); break;
+    case CRABML_HIP_Q6_K: all(std::integral_constant<int, CRABML_HIP_Q6_K>()); break;
+    case CRABML_HIP_F16: all(std::integral_constant<int, CRABML_HIP_F16>()); break;
+    case CRABML_HIP_F32: all(std::integral_constant<int, CRABML_HIP_F32>()); break;
+    default:
+#pragma unroll 1
+      for (int it = 0; it < NIT; it++) {
+        const int i = it * 1024 + (int)threadIdx.x;
+        v[it] = i < dim ? dequant_elem(w, dtype, off_scale, base + i) : 0.f;
+      }
+  }
+}
+template <int NIT, int FRONT>
+__global__ __launch_bounds__(1024) void k_step_front(const char* __restrict__ table, int dtype, size_t off_scale, TokenPick pick, int dim, float* __restrict__ x,
+                                                     const float* __restrict__ wn, float eps, FrontOut o, PrefetchPlan pf, int half) {
+  if (blockIdx.x > 0) {  // spare workgroups: the first GEMV's weights
+    prefetch_wg(pf, blockIdx.x - 1, gridDim.x - 1);
+    return;
+  }
+  extern __shared__ float lds[];
+  __shared__ float s_rms;
+  const int tid = threadIdx.x, lane = tid & 63;
+  float xv[NIT], wv[NIT];
+  if constexpr (FRONT != FRONT_ROW) {
+#pragma unroll
+    for (int it = 0; it < NIT; it++) wv[it] = it * 1024 + tid < dim ? wn[it * 1024 + tid] : 0.f;
+  }
+  int token;
+  if (pick.pv != nullptr) {
+    float bv = -INFINITY;
+    int bi = -1;
+    for (int i = lane; i < pick.nparts; i += 64) argmax_combine(bv, bi, pick.pv[i], pick.pi[i]);
+    argmax_wave(bv, bi);
+    token = bi;
+    if (tid == 0) {
+      *pick.token = bi;
+      const int st = *pick.step;
+      if (st < pick.out_cap) pick.out[st] = (unsigned)bi;
+      *pick.step = st + 1;
+      *pick.pos = *pick.pos + 1;
+      *pick.serial = *pick.serial + 1;
+    }
+  } else {
+    token = *pick.token;
+  }
+  embed_row<NIT>(table, dtype, off_scale, (size_t)token * dim, dim, xv);
+#pragma unroll
+  for (int it = 0; it < NIT; it++)
+    if (it * 1024 + tid < dim) x[it * 1024 + tid] = xv[it];
+  NormLds L{lds, lds + dim};
+  if constexpr (FRONT == FRONT_Q8_0 || FRONT == FRONT_Q8_1)
+    norm_quant_regs<NIT, true, FRONT == FRONT_Q8_1>(xv, wv, dim, eps, L, &s_rms, o.q, (unsigned short*)o.d, o.aux, nullptr, half);
+  if constexpr (FRONT == FRONT_Q8_K) {
+    norm_quant_regs<NIT, false>(xv, wv, dim, eps, L, &s_rms, nullptr, nullptr, nullptr, L.xs, half);  // (xs has been read by then)
+    __syncthreads();
+    for (int sb = tid >> 6; sb < dim / 256; sb += 16) {  // k_quantize_q8_k's wave per super-block
+      const Q8KLane k = q8k_wave_quant(((const f32x4*)L.xs)[sb * 64 + lane], lane);
+      ((unsigned*)o.q)[sb * 64 + lane] = k.packed;
+      q8k_store_class_major(o.qp + sb * 256, lane, k.packed);
+      if ((lane & 3) == 0) ((short*)o.aux)[sb * 16 + (lane >> 2)] = (short)k.quad_sum;
+      if (lane == 0) ((float*)o.d)[sb] = k.d;
+    }
+  }
 }
 
 // batched prefill, Q8_0 / Q8_1 rhs: x[row] (+= addv[row]: the pending wo / ffn_down output, llama2.rs:266 / :636) -> RMSNorm ->

@@ -1201,12 +1201,7 @@ __global__ __launch_bounds__(64) void k_argmax_step(const float* __restrict__ pv
   float bv = -INFINITY;
   int bi = -1;
   for (int i = threadIdx.x; i < nparts; i += 64) argmax_combine(bv, bi, pv[i], pi[i]);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    float ov = __shfl_xor(bv, o, 64);
-    int oi = __shfl_xor(bi, o, 64);
-    argmax_combine(bv, bi, ov, oi);
-  }
+  argmax_wave(bv, bi);
   if (threadIdx.x == 0) {
     if (best != nullptr) {
       best[0] = __builtin_bit_cast(int, bv);
@@ -1233,12 +1228,7 @@ __global__ __launch_bounds__(64) void k_argmax_step_tp(const float* __restrict__
   float bv = -INFINITY;
   int bi = -1;
   for (int i = lane; i < nparts; i += 64) argmax_combine(bv, bi, pv[i], pi[i]);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    float ov = __shfl_xor(bv, o, 64);
-    int oi = __shfl_xor(bi, o, 64);
-    argmax_combine(bv, bi, ov, oi);
-  }
+  argmax_wave(bv, bi);
   const unsigned serial = (unsigned)(*serial_d);
   const unsigned epoch = serial * (unsigned)nseg + (unsigned)nseg + t.salt;  // segment nseg - 1, + 1
   const int slot = 4 + (int)(serial & 1u);

@@ -47,6 +47,9 @@ enum { ST_IN = 1, ST_MIX = 2, ST_OUT = 3, ST_UP = 4, ST_DOWN = 5, ST_HEAD = 6, S
 
 constexpr size_t LOGIT_ROWS = 256;  // rows of logits a pass keeps on the device at a time
 constexpr int META_SLOTS = 4;
+// steps of a greedy run behind one another in one graph: a graph's two ends cost 6 to 7 us between two launches (measured with graphs of 35 and
+// 140 small kernels)
+constexpr size_t STEPS_A_GRAPH = 8;
 
 }  // namespace
 
@@ -85,7 +88,7 @@ struct crabml_hip_hybrid {
   int ld_proj = 0, ld_cat = 0, ld_u = 0;
   StepSeq* h_seq = nullptr;  // pinned ring of META_SLOTS * HYB_STEP_ROWS
   int h_seq_next = 0;
-  std::map<int, std::pair<hipGraph_t, hipGraphExec_t>> graphs;  // key: rows * 2 + sampler
+  std::map<int, std::pair<hipGraph_t, hipGraphExec_t>> graphs;  // (graph_key)
   // prompt pass (allocated on first use)
   size_t rows_cap = 0, hist_cap = 0, meta_bytes = 0;
   char *meta = nullptr, *h_meta = nullptr;
@@ -578,6 +581,24 @@ int latent_step(Ctx* c, const Run& run, int B, bool prof) {
 }
 
 
+// the front of a step (k_front_rows); pick: behind the sampler's partials
+void enqueue_front(Ctx* c, int B, bool pick) {
+  const size_t stride = (size_t)HYB_STEP_ROWS * c->ldx;
+  RowPick p;
+  if (pick) {
+    p.pv = c->am_val;
+    p.pi = c->am_idx;
+    p.nparts = ARGMAX_BLOCKS;
+    p.out_cap = (int)c->st_out_cap;
+    p.count = c->st_count;
+    p.out = c->st_out;
+  }
+  k_front_rows<<<B, 1024, 0, c->dev->stream>>>(p, c->embed, c->st_seq, c->width, c->ldx, c->cfg.embed_scale, c->freq, c->st_x, c->keep_emb ? c->st_emb : nullptr,
+                                               c->runs[0].add_vec, streams_at_start(c, stride), c->st_in, rows16(c, B) ? c->st_x16 : nullptr,
+                                               c->streams ? c->layers[c->runs[0].layer].norm1 : nullptr, c->st_xss, c->n_xss);
+}
+
+// one step of B rows: front, layers, classifier -- or, with the sampler, layers, classifier, sampler and the next step's front
 int enqueue_step(Ctx* c, int B, bool sample, bool prof) {
   crabml_hip_device* dev = c->dev;
   hipStream_t st = dev->stream;
@@ -585,10 +606,7 @@ int enqueue_step(Ctx* c, int B, bool sample, bool prof) {
   const size_t stride = (size_t)HYB_STEP_ROWS * c->ldx;
   const float* next_gain = nullptr;
   float* x_in = c->streams ? c->st_in : c->st_x;  // what a norm reads
-  k_embed_step<<<dim3((c->width + 255) / 256, B), 256, 0, st>>>(c->embed, c->st_seq, c->width, c->ldx, c->cfg.embed_scale, c->freq, c->st_x,
-                                                               c->keep_emb ? c->st_emb : nullptr, c->runs[0].add_vec, streams_at_start(c, stride), c->st_in,
-                                                               rows16(c, B) ? c->st_x16 : nullptr, c->streams ? c->layers[c->runs[0].layer].norm1 : nullptr,
-                                                               c->st_xss, c->n_xss);
+  if (!sample) enqueue_front(c, B, false);
   for (size_t r = 0; r < c->runs.size(); r++) {
     const Run& run = c->runs[r];
     const Layer& L = c->layers[run.layer];
@@ -699,21 +717,25 @@ int enqueue_step(Ctx* c, int B, bool sample, bool prof) {
   head_rows(c, x_in, B, prof, false);
   if (sample) {
     k_argmax_partial<<<dim3(ARGMAX_BLOCKS, B), 256, 0, st>>>(c->st_logits, c->vocab, c->am_val, c->am_idx, 0, c->vocab);
-    k_argmax_rows_step<<<B, 64, 0, st>>>(c->am_val, c->am_idx, ARGMAX_BLOCKS, c->st_seq, c->st_count, c->st_out, (int)c->st_out_cap);
-    k_step_advance<<<1, 1, 0, st>>>(c->st_count);
+    enqueue_front(c, B, true);
   }
   CH_HIP(dev, hipGetLastError());
   return 0;
 }
 
-// one decode step of B rows from its graph (captured when that batch size first comes up), or eagerly
-int run_step(Ctx* c, int B, bool sample) {
+int graph_key(int B, bool sample, int steps) { return (steps * (HYB_STEP_ROWS + 1) + B) * 2 + (sample ? 1 : 0); }
+// one decode step of B rows, or several of a greedy run, from its graph (captured when that batch size first comes up), or eagerly
+int run_step(Ctx* c, int B, bool sample, int steps = 1) {
   crabml_hip_device* dev = c->dev;
-  if ((c->cfg.flags & CRABML_HIP_HYBRID_NO_GRAPH) || dev->prof_on) return enqueue_step(c, B, sample, true);
-  auto& slot = c->graphs[B * 2 + (sample ? 1 : 0)];
+  if ((c->cfg.flags & CRABML_HIP_HYBRID_NO_GRAPH) || dev->prof_on) {
+    for (int i = 0; i < steps; i++) CH_TRY(enqueue_step(c, B, sample, true));
+    return 0;
+  }
+  auto& slot = c->graphs[graph_key(B, sample, steps)];
   if (!slot.second) {
     CH_HIP(dev, hipStreamBeginCapture(dev->stream, hipStreamCaptureModeThreadLocal));
-    const int rc = enqueue_step(c, B, sample, false);
+    int rc = 0;
+    for (int i = 0; i < steps && rc == 0; i++) rc = enqueue_step(c, B, sample, false);
     hipGraph_t graph = nullptr;
     const hipError_t e = hipStreamEndCapture(dev->stream, &graph);
     hipGraphExec_t exec = nullptr;
@@ -1155,7 +1177,7 @@ int create_impl(Ctx* c, const crabml_hip_hybrid_layer_t* layers, const crabml_hi
   }
   const size_t B = HYB_STEP_ROWS;
   CH_TRY(dalloc_n(c, B, &c->st_seq));
-  CH_TRY(dalloc_n(c, 1, &c->st_count));
+  CH_TRY(dalloc_n(c, HYB_STEP_ROWS, &c->st_count));
   CH_TRY(dalloc_n(c, (c->streams ? c->streams : 1) * B * c->ldx, &c->st_x));
   if (c->streams) CH_TRY(dalloc_n(c, B * c->ldx, &c->st_in));
   if (c->ld_vk) CH_TRY(dalloc_n(c, B * c->ld_vk, &c->st_vk));
@@ -1356,8 +1378,15 @@ int crabml_hip_hybrid_decode_greedy(crabml_hip_hybrid_t* c, size_t n, const size
   }
   if (n_steps == 0) return 0;
   CH_TRY(step_begin(c, n, seqs, tokens));
-  CH_HIP(dev, hipMemsetAsync(c->st_count, 0, sizeof(int), dev->stream));
-  for (size_t s = 0; s < n_steps; s++) CH_TRY(run_step(c, (int)n, true));
+  CH_HIP(dev, hipMemsetAsync(c->st_count, 0, HYB_STEP_ROWS * sizeof(int), dev->stream));
+  enqueue_front(c, (int)n, false);
+  // (a graph of several steps is captured where the run itself earns that back, about a tenth of a millisecond)
+  const bool several = n_steps >= 2 * STEPS_A_GRAPH || c->graphs.count(graph_key((int)n, true, (int)STEPS_A_GRAPH));
+  for (size_t s = 0; s < n_steps;) {
+    const int steps = several && n_steps - s >= STEPS_A_GRAPH ? (int)STEPS_A_GRAPH : 1;
+    CH_TRY(run_step(c, (int)n, true, steps));
+    s += steps;
+  }
   for (size_t i = 0; i < n; i++) c->seqs[seqs[i]].len += n_steps;
   CH_HIP(dev, hipMemcpyAsync(out_tokens, c->st_out, n_steps * n * sizeof(uint32_t), hipMemcpyDeviceToHost, dev->stream));
   CH_HIP(dev, hipStreamSynchronize(dev->stream));

@@ -24,32 +24,70 @@ struct StepSeq {
   char* slab;
 };
 
-__global__ __launch_bounds__(256) void k_embed_step(const unsigned short* __restrict__ table, const StepSeq* __restrict__ seq, int width, int ldx,
-                                                    float scale, const double* __restrict__ freq, float* __restrict__ x, float* __restrict__ emb,
-                                                    const float* __restrict__ add_vec, const StreamMix sm, float* __restrict__ u,
-                                                    unsigned short* __restrict__ x16, const float* __restrict__ gain, float* __restrict__ xss, int n_xss) {
-  const int c = blockIdx.x * 256 + threadIdx.x, b = blockIdx.y;
-  const bool in = c < width;
-  const StepSeq s = seq[b];
-  float r = 0.f;  // what the first norm reads
-  if (in) {
-    const float v = __builtin_fmaf(bf2f(table[(size_t)s.token * width + c]), scale, position_entry(s.pos, c, freq));
-    if (sm.n) {  // every stream starts as the embedding
-      for (int t = 0; t < sm.n; t++) {
-        x[t * sm.stride + (size_t)b * ldx + c] = v;
-        r = __builtin_fmaf(sm.in[t], v, r);
-      }
-      if (!x16) u[(size_t)b * ldx + c] = r;
-    } else {
-      if (emb) emb[(size_t)b * ldx + c] = v;
-      r = add_vec ? v + add_vec[c] : v;
-      x[(size_t)b * ldx + c] = r;
+// A step's front: embedding and what the first norm reads, a workgroup per row.  With pick.pv it runs behind the sampler's partials at a step's end, for
+// the tokens that they name: combining them (every wave for itself), advancing and embedding were three launches of one memory round trip
+// each, 13.6 of the 18.4 us that a 16-row step spent outside its layers and classifier (with several steps in a graph, 16 x 154 tokens of 4 layers of
+// width 2048: 20629 -> 19997 us; one sequence of 81 tokens on latent and windowed layers 12734 -> 12414).
+struct RowPick {
+  const float* pv = nullptr;  // [rows][nparts]
+  const int* pi = nullptr;
+  int nparts = 0, out_cap = 0;
+  int* count = nullptr;  // [rows] steps done
+  unsigned* out = nullptr;
+};
+__global__ __launch_bounds__(1024) void k_front_rows(const RowPick pick, const unsigned short* __restrict__ table, StepSeq* __restrict__ seq, int width, int ldx,
+                                                     float scale, const double* __restrict__ freq, float* __restrict__ x, float* __restrict__ emb,
+                                                     const float* __restrict__ add_vec, const StreamMix sm, float* __restrict__ u,
+                                                     unsigned short* __restrict__ x16, const float* __restrict__ gain, float* __restrict__ xss, int n_xss) {
+  const int b = blockIdx.x, tid = threadIdx.x;
+  int token = seq[b].token, pos = seq[b].pos;
+  if (pick.pv) {
+    float bv = -INFINITY;
+    int bi = -1;
+    for (int i = tid & 63; i < pick.nparts; i += 64) argmax_combine(bv, bi, pick.pv[b * pick.nparts + i], pick.pi[b * pick.nparts + i]);
+    argmax_wave(bv, bi);
+    token = bi < 0 ? 0 : bi;
+    pos++;
+    __syncthreads();  // (every wave has the old position)
+    if (tid == 0) {
+      seq[b].token = token;
+      seq[b].pos = pos;
+      const int n = pick.count[b];
+      const size_t at = (size_t)n * gridDim.x + b;
+      if (at < (size_t)pick.out_cap) pick.out[at] = (unsigned)token;
+      pick.count[b] = n + 1;
     }
   }
-  if (!x16) return;
-  if (in) x16[(size_t)b * ldx + c] = f2bf(gain ? r * gain[c] : r);
-  const float q = row16_sum_f32(r * r);
-  if (in && (c & 15) == 0) xss[(size_t)b * n_xss + (c >> 4)] = q;
+  constexpr int NC = 4;  // columns of a thread that are requested together
+  for (int c0 = tid; c0 - tid < width; c0 += NC * 1024) {
+    unsigned short e[NC];
+#pragma unroll
+    for (int i = 0; i < NC; i++) e[i] = table[(size_t)token * width + (c0 + i * 1024 < width ? c0 + i * 1024 : width - 1)];
+#pragma unroll
+    for (int i = 0; i < NC; i++) {
+      const int c = c0 + i * 1024;
+      const bool in = c < width;
+      float r = 0.f;  // what the first norm reads
+      if (in) {
+        const float v = __builtin_fmaf(bf2f(e[i]), scale, position_entry(pos, c, freq));
+        if (sm.n) {  // every stream starts as the embedding
+          for (int t = 0; t < sm.n; t++) {
+            x[t * sm.stride + (size_t)b * ldx + c] = v;
+            r = __builtin_fmaf(sm.in[t], v, r);
+          }
+          if (!x16) u[(size_t)b * ldx + c] = r;
+        } else {
+          if (emb) emb[(size_t)b * ldx + c] = v;
+          r = add_vec ? v + add_vec[c] : v;
+          x[(size_t)b * ldx + c] = r;
+        }
+      }
+      if (!x16) continue;
+      if (in) x16[(size_t)b * ldx + c] = f2bf(gain ? r * gain[c] : r);
+      const float q = row16_sum_f32(r * r);
+      if (in && (c & 15) == 0) xss[(size_t)b * n_xss + (c >> 4)] = q;
+    }
+  }
 }
 
 struct MixStep {
@@ -442,27 +480,5 @@ inline void launch_mix_step(hipStream_t st, crabml_hip_device::ProfRec* rec, con
   else
     launch_mix_step_t<T, 256>(st, rec, a);
 }
-
-// ---- greedy sampler over the rows of a batch (last maximum, as k_argmax_step) ---------------------------------------------------
-__global__ __launch_bounds__(64) void k_argmax_rows_step(const float* __restrict__ pv, const int* __restrict__ pi, int nparts,
-                                                         StepSeq* __restrict__ seq, const int* __restrict__ step_d, unsigned* __restrict__ out, int out_cap) {
-  const int b = blockIdx.x;
-  float bv = -INFINITY;
-  int bi = -1;
-  for (int i = threadIdx.x; i < nparts; i += 64) argmax_combine(bv, bi, pv[b * nparts + i], pi[b * nparts + i]);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    float ov = __shfl_xor(bv, o, 64);
-    int oi = __shfl_xor(bi, o, 64);
-    argmax_combine(bv, bi, ov, oi);
-  }
-  if (threadIdx.x == 0) {
-    seq[b].token = bi < 0 ? 0 : bi;
-    seq[b].pos++;
-    const size_t at = (size_t)*step_d * gridDim.x + b;
-    if (at < (size_t)out_cap) out[at] = (unsigned)(bi < 0 ? 0 : bi);
-  }
-}
-__global__ void k_step_advance(int* step_d) { *step_d += 1; }
 
 }  // namespace crabml_hip

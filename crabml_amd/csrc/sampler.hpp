@@ -15,6 +15,14 @@ __device__ __forceinline__ void argmax_combine(float& cv, int& ci, float ov, int
     ci = oi;
   }
 }
+__device__ __forceinline__ void argmax_wave(float& v, int& i) {  // over the 64 lanes; every lane gets it
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const float ov = __shfl_xor(v, o, 64);
+    const int oi = __shfl_xor(i, o, 64);
+    argmax_combine(v, i, ov, oi);
+  }
+}
 // base: global index of logits[0] (a vocabulary shard of a tensor-parallel classifier; 0 otherwise).  blockIdx.y: row of a batch
 // (row_stride floats apart; its partials follow the previous row's)
 static __global__ __launch_bounds__(256) void k_argmax_partial(const float* __restrict__ logits, int n, float* __restrict__ pv,
@@ -29,12 +37,7 @@ static __global__ __launch_bounds__(256) void k_argmax_partial(const float* __re
   float bv = -INFINITY;
   int bi = -1;
   for (int i = lo + threadIdx.x; i < hi; i += blockDim.x) argmax_combine(bv, bi, logits[i], base + i);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    float ov = __shfl_xor(bv, o, 64);
-    int oi = __shfl_xor(bi, o, 64);
-    argmax_combine(bv, bi, ov, oi);
-  }
+  argmax_wave(bv, bi);
   if ((threadIdx.x & 63) == 0) {
     sv[threadIdx.x >> 6] = bv;
     si[threadIdx.x >> 6] = bi;

@@ -1,0 +1,69 @@
+"""The two ends of a decode step: sampler, advance, embedding, first norm and its quantizer in one launch behind the classifier, and several steps in
+one graph -- against steps that are given their tokens one at a time, eager ones among them, bit for bit."""
+import numpy as np
+import pytest
+
+from crabml_amd import synth
+from crabml_amd import synth_bifazen as sb
+from crabml_amd import synth_hybrid as sh
+
+pytestmark = pytest.mark.gpu
+
+
+def greedy_by_hand(ca, r, token, pos, n):
+    ids = []
+    for i in range(n):
+        token = ca.sample_argmax(r.forward(token, pos + i))
+        ids.append(token)
+    return ids
+
+
+# (4352: more than four elements a thread; 288: rows that end inside a wave; Q5_K, F32: launches per operation)
+WIDE = synth.ModelShape("wide", 4352, 512, 1, 34, 2, 600, 64, 1e-5, None)
+
+
+@pytest.mark.parametrize("fmt,shape", [("Q4_0", "tiny-hd128"), ("Q8_0", "15m"), ("Q4_1", "tiny-hd128"), ("Q4_K", "tiny-hd128"), ("Q4_K", "tiny-gqa"), ("F16", "15m"),
+                                       ("Q5_K", "tiny-gqa"), ("F32", "tiny-gqa"), ("Q6_K", "tiny-gqa"), ("Q4_0", WIDE), ("Q4_K", WIDE), ("F16", WIDE)])
+@pytest.mark.parametrize("strict", [False, True])
+def test_greedy_runs_equal_single_steps(ca, fmt, shape, strict):
+    dev = ca.HipTensorDevice(0, strict_order=strict)
+    model = synth.build_model(shape if isinstance(shape, synth.ModelShape) else synth.SHAPES[shape], synth.TYPE_BY_NAME[fmt], seed=21)
+    conf, w = synth.to_hip(model, dev)
+    long = fmt in ("Q4_0", "Q8_0") and not isinstance(shape, synth.ModelShape) and not strict
+    seq = 600 if long else 60
+    a, b, e = ca.HipLlamaRunner(conf, w, dev, seq, True), ca.HipLlamaRunner(conf, w, dev, seq, True), ca.HipLlamaRunner(conf, w, dev, seq, True, False)
+    pos, token = 0, 3
+    for n in (1, 7, 8, 9, 17) + ((400, 100) if long else ()):  # (400, 100: runs over the switches of the attention)
+        ids = a.decode_greedy(token, n)
+        assert ids == greedy_by_hand(ca, b, token, pos, n), n
+        assert ids == e.decode_greedy(token, n), n
+        pos, token = pos + n, ids[-1]
+    la, lb, le = a.forward(token, pos), b.forward(token, pos), e.forward(token, pos)
+    assert np.array_equal(la.view(np.uint32), lb.view(np.uint32)) and np.array_equal(la.view(np.uint32), le.view(np.uint32))
+
+
+NILIVIK = sh.config(84, 131, [sh.layer(3, 1, 36, 44, 50, 2, 28, 36, 40)], loop={"start": 0, "stop": 1, "times": 2})
+NILIVIK_WIDE = sh.config(4104, 67, [sh.layer(1, 1, 8, 8, 16, 1, 8, 8, 16)])  # (more than four columns a thread, the last ones in part)
+BIFAZEN = sb.config(200, 131, [sb.latent(2, 12, 4, 12, 20, 30, 40), sb.attention(2, 1, 8, 8, 9, 40)], streams=3)
+
+
+@pytest.mark.parametrize("config,tensors", [(NILIVIK, sh.random_tensors), (NILIVIK_WIDE, sh.random_tensors), (BIFAZEN, sb.random_tensors)])
+@pytest.mark.parametrize("f32", [False, True])
+def test_greedy_batches_equal_single_steps(ca, hdev, tmp_path, config, tensors, f32):
+    folder = sh.write_model(config, tensors(config, 5), str(tmp_path / "m"))
+    g, e, h = (ca.load_model(folder, hdev, seq_len=64, f32=f32, **kw) for kw in ({}, {"use_graph": False}, {}))
+    for rows in (1, 2, 3, 16):
+        seqs = [[r.open() for _ in range(rows)] for r in (g, e, h)]
+        ids = [(7 * i + rows) % 60 for i in range(rows)]
+        for n in (1, 8, 17, 9, 25):
+            a, b = g.decode_batch(seqs[0], ids, n), e.decode_batch(seqs[1], ids, n)
+            assert list(a) == list(b), (rows, n)
+            for k in range(n):
+                ids = [ca.sample_argmax(x) for x in h.step([(s, [t], [0]) for s, t in zip(seqs[2], ids)])]
+                assert ids == list(a[k * rows:(k + 1) * rows]), (rows, n, k)
+        last = [r.step([(s, [t], [0]) for s, t in zip(q, ids)]) for r, q in zip((g, e, h), seqs)]
+        for x in last[1:]:
+            assert np.array_equal(last[0].view(np.uint32), x.view(np.uint32)), rows
+        for r, q in zip((g, e, h), seqs):
+            for s in q:
+                r.close(s)
