@@ -120,6 +120,7 @@ struct GemvBf16 {
   int ld_add = 0;
   float cap = 0.f;
   const float* bias = nullptr;  // [N], nullable (ACT, STREAMS)
+  bool resident = false;  // the weights of all linears that run in turn fit a cache: they are read so that they stay in it (else nontemporal)
   StreamMix sm;                 // STREAMS: out = stream 0, u[b][ldo] = what the next linear reads
   float* u = nullptr;
 };
@@ -205,7 +206,7 @@ __device__ __forceinline__ void rows16_out(const GemvBf16& a, int row, int b, fl
 
 #define GEMV_BF16_LDS_FLOATS 8192  // rhs elements staged at a time, all rows together: a cut segment is a multiple of the steps in flight
 
-template <int NB, int R, int IN, int OUT>
+template <int NB, int R, int IN, int OUT, bool NT>  // NT: weights nontemporal (GemvBf16::resident)
 __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
   extern __shared__ __attribute__((aligned(16))) float gemv_lds[];  // [NB][2][seg / 2]
   __shared__ float red[4][NB];
@@ -227,7 +228,7 @@ __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
       int k = k0 + u * 512 + lane * 8;
       k = k < a.K ? k : 0;  // (a lane past the end requests the row's start and never uses it)
 #pragma unroll
-      for (int r = 0; r < R; r++) wv[u][r] = __builtin_nontemporal_load((const i32x4*)(wr[r] + k));
+      for (int r = 0; r < R; r++) wv[u][r] = ld<NT>((const i32x4*)(wr[r] + k));
     }
   };
   request(0);
@@ -386,8 +387,8 @@ __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
 // wave's own 2 KB of LDS, 16-byte pieces permuted by (row / 2) % 8 as in gemm_bf16.hip; no barrier, a wave's LDS accesses are in order.
 // 16 rows, before -> after, with bf16 rows: 2048 x 8192 23.2 -> 12.7 us, 2048 x 4096 17.5 -> 8.6, 5632 x 2048 19.3 -> 13.9, 8192 x 2048
 // 14.1 -> 10.2, 32000 x 2048 35.4 -> 30.3 (4.3 TB/s); what is left is a launch's ramp, two rounds of memory latency and the hand-over.
-// Weights are read past the L2s' replacement (nontemporal): the 16 rows of the rhs, which every workgroup reads whole, stay in them.  16 x 154 tokens
-// of 4 layers of width 2048 20054 -> 18687 us, 4 x 716 of latent and windowed layers 7443 -> 7283.
+// NTW: weights past the caches' replacement, so that the 16 rows of the rhs, which every workgroup reads whole, stay (GemvBf16::resident).  16 x 154
+// tokens of 4 layers of width 2048 20054 -> 18687 us, 4 x 716 of latent and windowed layers 7443 -> 7283.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 // f32 -> its upper, middle and lower eight significand bits as bf16: their sum is exact
 __device__ __forceinline__ void split3(float v, unsigned short& hi, unsigned short& mid, unsigned short& lo) {
@@ -412,7 +413,7 @@ __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) { return
 // XG: f32 rows are requested and split in groups of four, as many as there are rows -- a group is a request, twelve conversions and three LDS
 // stores a lane and piece, which three rows of four groups paid for in full (f32 compute, us, 4 rows, all groups / one: 11264 x 2048
 // 17.3 / 12.2, gate | up of 16384 x 2048 18.5 / 16.1).
-template <int RT, int SPL, int W, int D, int IN, int OUT, int XG = 4>
+template <int RT, int SPL, int W, int D, int IN, int OUT, bool NTW, int XG = 4>
 __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
   constexpr int LD = 20, NT = 64 * W;
   constexpr bool XB = IN == GEMV_IN_BF16 || IN == GEMV_IN_BF16_RMS || IN == GEMV_IN_BF16_SPLIT, NORM = IN == GEMV_IN_RMS || IN == GEMV_IN_RMSV;
@@ -451,7 +452,7 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
 #pragma unroll
     for (int t = 0; t < RT; t++)
 #pragma unroll
-      for (int j = 0; j < 2; j++) wv[d][t][j] = __builtin_nontemporal_load((const i32x4*)(w + wo[t][j]));
+      for (int j = 0; j < 2; j++) wv[d][t][j] = ld<NTW>((const i32x4*)(w + wo[t][j]));
 #pragma unroll
     for (int j = 0; j < XR; j++) xv[d][j] = *(const i32x4*)(x + xo[j]);
     if constexpr (IN == GEMV_IN_RMSV) gv[d] = *(const f32x4*)(gb + i * 256 + (unsigned)c16 * 16);
@@ -677,47 +678,51 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
 // Three pieces of more than eight f32 rows: two steps of requests hold 140 registers a thread, one workgroup a CU; where there are more workgroups than
 // CUs, two of them with one step out each are faster (us, 12 rows: 11264 x 2048 18.0 -> 16.4, 8192 x 1024 8.7 -> 6.9), elsewhere they are
 // not (2048 x 8192, 128 workgroups: 16.2 -> 19.8).
-template <int RT, int SPL, int W, int IN, int OUT>
+template <int RT, int SPL, int W, int IN, int OUT, bool NTW>
 inline void launch_gemv16_t(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a, int n_cu) {
   constexpr int D = IN < GEMV_IN_BF16 || RT == 2 ? 2 : OUT == GEMV_OUT_STREAMS ? 3 : 4;  // (registers: sixteen waves a CU)
   const dim3 grid((a.N + 16 * RT - 1) / (16 * RT));
   if constexpr (SPL == 3) {
     if (a.nb <= 4) {
-      launch_k(st, rec, k_gemv16_bf16<RT, SPL, W, D, IN, OUT, 1>, grid, dim3(64 * W), 0, a);
+      launch_k(st, rec, k_gemv16_bf16<RT, SPL, W, D, IN, OUT, NTW, 1>, grid, dim3(64 * W), 0, a);
       return;
     }
     if (a.nb <= 8) {
-      launch_k(st, rec, k_gemv16_bf16<RT, SPL, W, D, IN, OUT, 2>, grid, dim3(64 * W), 0, a);
+      launch_k(st, rec, k_gemv16_bf16<RT, SPL, W, D, IN, OUT, NTW, 2>, grid, dim3(64 * W), 0, a);
       return;
     }
     if (RT == 1 && (int)grid.x > n_cu) {
-      launch_k(st, rec, k_gemv16_bf16<RT, SPL, W, 1, IN, OUT>, grid, dim3(64 * W), 0, a);
+      launch_k(st, rec, k_gemv16_bf16<RT, SPL, W, 1, IN, OUT, NTW>, grid, dim3(64 * W), 0, a);
       return;
     }
   }
-  launch_k(st, rec, k_gemv16_bf16<RT, SPL, W, D, IN, OUT>, grid, dim3(64 * W), 0, a);
+  launch_k(st, rec, k_gemv16_bf16<RT, SPL, W, D, IN, OUT, NTW>, grid, dim3(64 * W), 0, a);
 }
-template <int SPL, int IN, int OUT>
-inline void launch_gemv16_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a, int n_cu) {
+template <int SPL, int IN, int OUT, bool NTW>
+inline void launch_gemv16_n(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a, int n_cu) {
   const bool two = a.N >= 16384, deep = !two && (a.N + 15) / 16 < n_cu && a.K >= 2048;
   if (two) {
-    launch_gemv16_t<2, SPL, 8, IN, OUT>(st, rec, a, n_cu);
+    launch_gemv16_t<2, SPL, 8, IN, OUT, NTW>(st, rec, a, n_cu);
     return;
   }
   if constexpr (IN >= GEMV_IN_BF16) {
     if (deep) {
-      launch_gemv16_t<1, SPL, 16, IN, OUT>(st, rec, a, n_cu);
+      launch_gemv16_t<1, SPL, 16, IN, OUT, NTW>(st, rec, a, n_cu);
       return;
     }
   }
-  launch_gemv16_t<1, SPL, 8, IN, OUT>(st, rec, a, n_cu);
+  launch_gemv16_t<1, SPL, 8, IN, OUT, NTW>(st, rec, a, n_cu);
+}
+template <int SPL, int IN, int OUT>
+inline void launch_gemv16_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a, int n_cu) {
+  a.resident ? launch_gemv16_n<SPL, IN, OUT, false>(st, rec, a, n_cu) : launch_gemv16_n<SPL, IN, OUT, true>(st, rec, a, n_cu);
 }
 
 template <int NB, int R, int IN, int OUT>
 inline void launch_gemv_bf16_t(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a) {
   const int cap = GEMV_BF16_LDS_FLOATS / NB, seg = a.K < cap ? a.K : cap;
-  launch_k(st, rec, k_gemv_bf16<NB, R, IN, OUT>, dim3((a.N + 4 * R - 1) / (4 * R), (a.nb + NB - 1) / NB), dim3(256),
-           (size_t)NB * seg * sizeof(float), a);
+  launch_k(st, rec, a.resident ? k_gemv_bf16<NB, R, IN, OUT, false> : k_gemv_bf16<NB, R, IN, OUT, true>,
+           dim3((a.N + 4 * R - 1) / (4 * R), (a.nb + NB - 1) / NB), dim3(256), (size_t)NB * seg * sizeof(float), a);
 }
 // rows of the rhs that share one pass over the weights: as many as there are, up to 8
 template <int IN, int OUT>

@@ -46,6 +46,12 @@ struct Seq {
 enum { ST_IN = 1, ST_MIX = 2, ST_OUT = 3, ST_UP = 4, ST_DOWN = 5, ST_HEAD = 6, ST_LIN = 7, ST_ROWS = 8, ST_LAT = 9, ST_STEP = 10, ST_PASS = 20 };
 
 constexpr size_t LOGIT_ROWS = 256;  // rows of logits a pass keeps on the device at a time
+// Linears whose weights all fit a cache read them so that they stay there from step to step, larger models past its replacement (GemvBf16::resident).
+// One and two rows: the L2s (32 MB); a launch that reads them from the Infinity Cache gains nothing by leaving them there.  More rows, whose
+// workgroups read the rhs beside the weights: the Infinity Cache.  us for 60 steps, kept / past: one row, weights of 16 MB 3049 / 3213, 31 MB 3200 /
+// 3355, 42 MB 4214 / 4036, 112 MB 9049 / 8840; 16 rows, 16 MB 3917 / 4279, 112 MB 10436 / 11523, 134 MB 4262 / 4743, 254 MB 9130 / 9388, 264 MB
+// 8090 / 8149, 394 MB 12280 / 11520, 504 MB 17433 / 17121.
+constexpr size_t RESIDENT_L2 = (size_t)32 << 20, RESIDENT_MALL = (size_t)256 << 20;
 constexpr int META_SLOTS = 4;
 // steps of a greedy run behind one another in one graph: a graph's two ends cost 6 to 7 us between two launches (measured with graphs of 35 and
 // 140 small kernels)
@@ -68,6 +74,7 @@ struct crabml_hip_hybrid {
   int streams = 0;  // 0: one residual row, norms with a single gain; else gains per element
   double* freq = nullptr;
   bool keep_emb = false;
+  size_t weight_bytes = 0;  // of the linears
   // decode step
   StepSeq* st_seq = nullptr;
   int* st_count = nullptr;
@@ -207,7 +214,10 @@ int pack_connection(Ctx* c, const crabml_hip_buf* in, const crabml_hip_buf* out,
   return 0;
 }
 // rows of a weight matrix: padded to 256 so that any tile of the GEMM reads inside it
-int alloc_matrix(Ctx* c, size_t rows, size_t ld, unsigned short** out) { return dalloc_n(c, align_up(rows, 256) * ld, out); }
+int alloc_matrix(Ctx* c, size_t rows, size_t ld, unsigned short** out) {
+  c->weight_bytes += rows * ld * 2;
+  return dalloc_n(c, align_up(rows, 256) * ld, out);
+}
 
 int build_layer(Ctx* c, const crabml_hip_hybrid_layer_t& s, Layer& L) {
   crabml_hip_device* dev = c->dev;
@@ -432,7 +442,8 @@ struct Prof {
 bool rows16(const Ctx* c, int B) { return B > 2 && !c->f32; }
 // a decode linear: up to two rows on the vector kernel, more on the matrix cores (IN16: its form for rows16)
 template <int IN, int IN16, int OUT>
-void step_linear(Ctx* c, crabml_hip_device::ProfRec* rec, const GemvBf16& g) {
+void step_linear(Ctx* c, crabml_hip_device::ProfRec* rec, GemvBf16 g) {
+  g.resident = c->weight_bytes <= (g.nb > 2 ? RESIDENT_MALL : RESIDENT_L2);
   if (g.nb <= 2)
     launch_gemv_bf16<IN, OUT>(c->dev->stream, rec, g);
   else if (c->f32)
@@ -540,6 +551,7 @@ void head_rows(Ctx* c, const float* x, int B, bool prof, bool f32_rows) {
   g.cap = c->cfg.logit_softcap;
   Prof p(c->dev, prof, ST_STEP + ST_HEAD, (double)c->vocab * c->ldx * 2);
   if (f32_rows && rows16(c, B)) {
+    g.resident = c->weight_bytes <= (g.nb > 2 ? RESIDENT_MALL : RESIDENT_L2);
     if (c->streams)
       launch_gemv16_bf16<1, GEMV_IN_RMSV, GEMV_OUT_SOFTCAP>(c->dev->stream, p.rec(), g, c->dev->n_cu);
     else
@@ -1174,6 +1186,10 @@ int create_impl(Ctx* c, const crabml_hip_hybrid_layer_t* layers, const crabml_hi
     CH_TRY(dalloc_n(c, f.size(), &c->freq));
     CH_HIP(dev, hipMemcpyAsync(c->freq, f.data(), f.size() * sizeof(double), hipMemcpyHostToDevice, dev->stream));
     CH_HIP(dev, hipStreamSynchronize(dev->stream));
+  }
+  {
+    const char *h = getenv("CRABML_HIP_TEST_HOOKS"), *e = getenv("CRABML_HIP_STREAM_WEIGHTS");  // test hook: small models through the large ones' loads
+    if (h && h[0] == '1' && e && e[0] == '1') c->weight_bytes = SIZE_MAX;
   }
   const size_t B = HYB_STEP_ROWS;
   CH_TRY(dalloc_n(c, B, &c->st_seq));

@@ -67,3 +67,23 @@ def test_greedy_batches_equal_single_steps(ca, hdev, tmp_path, config, tensors, 
         for r, q in zip((g, e, h), seqs):
             for s in q:
                 r.close(s)
+
+
+@pytest.mark.parametrize("config,tensors", [(NILIVIK, sh.random_tensors), (BIFAZEN, sb.random_tensors)])
+@pytest.mark.parametrize("f32", [False, True])
+def test_weights_past_the_caches_are_the_same_weights(ca, hdev, tmp_path, monkeypatch, config, tensors, f32):
+    """models too large for the caches read their weights with loads of another kind: the same logits from the same model either way"""
+    folder = sh.write_model(config, tensors(config, 6), str(tmp_path / "m"))
+    kept = ca.load_model(folder, hdev, seq_len=64, f32=f32)
+    monkeypatch.setenv("CRABML_HIP_TEST_HOOKS", "1")
+    monkeypatch.setenv("CRABML_HIP_STREAM_WEIGHTS", "1")
+    past = ca.load_model(folder, hdev, seq_len=64, f32=f32)
+    for rows in (1, 2, 3, 8, 16):
+        a, b = [kept.open() for _ in range(rows)], [past.open() for _ in range(rows)]
+        for i in range(6):
+            ids = [(11 * i + 5 * k) % 60 for k in range(rows)]
+            x, y = (r.step([(s, [t], [0]) for s, t in zip(q, ids)]) for r, q in ((kept, a), (past, b)))
+            assert np.array_equal(x.view(np.uint32), y.view(np.uint32)), (rows, i)
+        for r, q in ((kept, a), (past, b)):
+            for s in q:
+                r.close(s)
