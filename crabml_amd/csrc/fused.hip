@@ -363,6 +363,7 @@ void launch_attn_flash(crabml_hip_llama* c, int l, signed char* xq, unsigned sho
 void enqueue_attention(crabml_hip_llama* c, int l, signed char* xq, unsigned short* xd, void* xisum, const PrefetchPlan& pf,
                        int spare, bool prof, const AttnQ8K* k8 = nullptr) {
   crabml_hip_device* dev = c->dev;
+  if (!pf.n) spare = 0;
   hipStream_t st = dev->stream;
   const int hd = c->hd, seq_cap = (int)c->cfg.seq_len, n_heads = c->n_heads_l, n_kv = c->n_kv_l;
   const int* pos_d = c->state + 1;
@@ -464,15 +465,13 @@ StepF16 step_f16(const crabml_hip_llama* c, std::initializer_list<const crabml_h
   return a;
 }
 
-PrefetchPlan prefetch_plan(const crabml_hip_llama* c, const crabml_hip_buf* a, const crabml_hip_buf* b, const crabml_hip_buf* cc) {
+// What workgroups of `rows` consecutive rows each read of a Q4_0 / Q8_0 / Q4_1 matrix (prefetch.hpp)
+PrefetchPlan prefetch_rows(const crabml_hip_llama* c, const crabml_hip_buf* w, int rows) {
   PrefetchPlan pf{};
-  const bool on = !(c->cfg.flags & CRABML_HIP_LLAMA_NO_PREFETCH);
-  const crabml_hip_buf* v[3] = {a, b, cc};
-  for (int i = 0; i < 3; i++) {
-    pf.p[i] = on && v[i] ? v[i]->ptr : nullptr;
-    pf.n[i] = on && v[i] ? (v[i]->wl.total / 16) * 16 : 0;
-  }
-  pf.sink = c->state + 3;
+  if ((c->cfg.flags & CRABML_HIP_LLAMA_NO_PREFETCH) || (w->dtype != CRABML_HIP_Q4_0 && w->dtype != CRABML_HIP_Q8_0 && w->dtype != CRABML_HIP_Q4_1)) return pf;
+  const size_t blocks = w->k / 32 * rows;
+  prefetch_add(pf, w->ptr, blocks * (w->dtype == CRABML_HIP_Q8_0 ? 32 : 16), 0, (int)(w->m / rows));
+  prefetch_add(pf, (const char*)w->ptr + w->wl.off_scale, blocks * (w->dtype == CRABML_HIP_Q4_1 ? 4 : 2), 0, (int)(w->m / rows));
   return pf;
 }
 
@@ -500,13 +499,10 @@ int enqueue_front(crabml_hip_llama* c, bool pick) {
   }
   const ActLayout al = act_layout(k ? CRABML_HIP_Q8_K : front == FRONT_Q8_1 ? CRABML_HIP_Q8_1 : CRABML_HIP_Q8_0, (size_t)dim);
   const FrontOut o{(signed char*)c->act_dim, (signed char*)(c->act_dim + al.off_p), (void*)(c->act_dim + al.off_d), (void*)(c->act_dim + al.off_aux)};
-  const bool weights = front == FRONT_Q8_0 || front == FRONT_Q8_1;
-  const PrefetchPlan pf = weights ? prefetch_plan(c, c->wq[0], c->wk[0], c->wv[0]) : PrefetchPlan{};
-  const int spare = weights && !(g.flags & CRABML_HIP_LLAMA_NO_PREFETCH) && dev->n_cu > 1 ? dev->n_cu - 1 : 0;
   auto go = [&](auto kernel) {
-    launch_k(dev->stream, prof ? &nr : nullptr, kernel, dim3(1 + spare), dim3(1024), front == FRONT_ROW ? 0 : norm_lds_bytes(dim),
+    launch_k(dev->stream, prof ? &nr : nullptr, kernel, dim3(1), dim3(1024), front == FRONT_ROW ? 0 : norm_lds_bytes(dim),
              (const char*)c->token_embed->ptr, (int)c->token_embed->dtype, c->token_embed->wl.off_scale, tp, dim, c->x, (const float*)c->rms_att[0]->ptr,
-             g.rms_norm_eps, o, pf, dev->strict_order ? 0 : 1);
+             g.rms_norm_eps, o, dev->strict_order ? 0 : 1);
   };
   if (prof) CH_TRY(prof_begin(dev, &nr, CRABML_HIP_F32, 6, 8.0 * dim));
   const bool narrow = dim <= 4096;
@@ -585,19 +581,16 @@ int enqueue_segment_t(crabml_hip_llama* c, int seg) {
   auto P1 = [&](crabml_hip_device::ProfRec* r) { return prof ? prof_end(dev, r) : 0; };
   crabml_hip_device::ProfRec pr{};
   crabml_hip_device::ProfRec* R = prof ? &pr : nullptr;
-  const bool do_pf = !(g.flags & CRABML_HIP_LLAMA_NO_PREFETCH);
-  auto plan = [&](const crabml_hip_buf* a, const crabml_hip_buf* b, const crabml_hip_buf* cc) { return prefetch_plan(c, a, b, cc); };
-  const int spare = do_pf ? (dev->n_cu > 1 ? dev->n_cu - 1 : 0) : 0;
   const size_t norm_lds = norm_lds_bytes(dim);
   // rmsnorm * weight -> act_dim; with tp the previous segment's all-reduced output is folded into x first
-  auto norm_quant = [&](const float* wn, float eps, bool add_pending, const PrefetchPlan& pf) {
+  auto norm_quant = [&](const float* wn, float eps, bool add_pending) {
     crabml_hip_device::ProfRec nr{};
     if (prof) prof_begin(dev, &nr, CRABML_HIP_F32, 6, 8.0 * dim);
     const float* addv = add_pending ? c->partial : nullptr;
     if (dim <= 4096)
-      launch_k(st, prof ? &nr : nullptr, k_norm_quant<4, Q81>, dim3(1 + spare), dim3(1024), norm_lds, c->x, addv, wn, dim, eps, ad.q, ad.d, ad.isum, pf, c->ord ? 0 : 1);
+      launch_k(st, prof ? &nr : nullptr, k_norm_quant<4, Q81>, dim3(1), dim3(1024), norm_lds, c->x, addv, wn, dim, eps, ad.q, ad.d, ad.isum, c->ord ? 0 : 1);
     else
-      launch_k(st, prof ? &nr : nullptr, k_norm_quant<12, Q81>, dim3(1 + spare), dim3(1024), norm_lds, c->x, addv, wn, dim, eps, ad.q, ad.d, ad.isum, pf, c->ord ? 0 : 1);
+      launch_k(st, prof ? &nr : nullptr, k_norm_quant<12, Q81>, dim3(1), dim3(1024), norm_lds, c->x, addv, wn, dim, eps, ad.q, ad.d, ad.isum, c->ord ? 0 : 1);
     if (prof) prof_end(dev, &nr);
   };
   // W(dim x k_local) . act -> x (+= residual) or partial (tp)
@@ -729,7 +722,7 @@ int enqueue_segment_t(crabml_hip_llama* c, int seg) {
         launch_quantize_act(st, c->out_qt, c->xn, (size_t)dim, c->act_dim);
       }
     } else if (!norm_epi) {
-      norm_quant((const float*)c->rms_final->ptr, g.rms_norm_eps, tp, plan(nullptr, nullptr, nullptr));
+      norm_quant((const float*)c->rms_final->ptr, g.rms_norm_eps, tp);
     }
     if (prof)
       CH_TRY(prof_begin(dev, &pr, c->output->dtype, 5,
@@ -745,7 +738,7 @@ int enqueue_segment_t(crabml_hip_llama* c, int seg) {
     if (l == 0) {
       if (!c->lead) CH_TRY(enqueue_front(c, false));
     } else if (!norm_epi) {
-      norm_quant((const float*)c->rms_att[l]->ptr, g.rms_norm_eps, tp, plan(c->wq[l], c->wk[l], c->wv[l]));
+      norm_quant((const float*)c->rms_att[l]->ptr, g.rms_norm_eps, tp);
     }
     // q, k, v + rope + scale + KV append (llama2.rs:244-256, 542-554, 561-565), local heads only
     QkvEpi e{c->qbuf, c->kc[l], c->vc[l], c->rope, pos_d, 1.0f / std::sqrt((float)hd), dim_l, kv_dim_l, hd,
@@ -769,8 +762,8 @@ int enqueue_segment_t(crabml_hip_llama* c, int seg) {
     CH_TRY(P1(&pr));
     // attention (llama2.rs:571-590) -> attn (f32) [+ Q8_0 planes for wo]; spare CUs prefetch wo
     const bool attn_quant = (hd % 32) == 0;
-    const int attn_spare = do_pf && dev->n_cu > n_heads_l ? dev->n_cu - n_heads_l : 0;
-    enqueue_attention(c, l, attn_quant ? aa.q : (signed char*)nullptr, aa.d, aa.isum, plan(c->wo[l], nullptr, nullptr), attn_spare, prof);
+    const PrefetchPlan wo = prefetch_rows(c, c->wo[l], norm_epi ? 32 / split_of(dim_l) : 2);
+    enqueue_attention(c, l, attn_quant ? aa.q : (signed char*)nullptr, aa.d, aa.isum, wo, dev->n_cu > n_heads_l ? dev->n_cu - n_heads_l : 0, prof);
     // heads that are not whole quant blocks (head width 48 of the 15M-parameter model): wo's launch quantizes the row itself -- the same bits, one
     // launch fewer per layer (2 us of quantizer and its boundary: 7.46 -> 7.05 ms for 57 tokens of that model)
     const bool attn_in_f32 = !attn_quant && !c->attn_row_apart && defer_wo && !tp && !c->ord && q8_0_lds_bytes(dim_l / 32) <= 60 * 1024;
@@ -779,7 +772,7 @@ int enqueue_segment_t(crabml_hip_llama* c, int seg) {
     CH_TRY(gemv_out(c->wo[l], aa, dim_l, 2, (const float*)c->rms_ffn[l]->ptr, 1e-5f, defer_wo, attn_in_f32 ? c->attn : nullptr));
   } else {
     // ffn rmsnorm, eps = the literal 1e-5 (llama2.rs:611)
-    if (!norm_epi) norm_quant((const float*)c->rms_ffn[l]->ptr, 1e-5f, tp, plan(nullptr, nullptr, nullptr));
+    if (!norm_epi) norm_quant((const float*)c->rms_ffn[l]->ptr, 1e-5f, tp);
     const float* wnext_down = (const float*)(l + 1 < L ? c->rms_att[l + 1] : c->rms_final)->ptr;
     // gate / up + silu * mul (llama2.rs:620-630), local rows
     CH_TRY(P0(&pr, 3, 2.0 * hidden_l, dim));

@@ -26,7 +26,7 @@ __global__ __launch_bounds__(256) void k_attn(const float* __restrict__ q, const
   const int q81 = q81_in & 255;
   const bool strict_sum = (q81_in & 256) != 0;
   if ((int)blockIdx.x >= n_heads) {
-    prefetch_wg(pf, blockIdx.x - n_heads, gridDim.x - n_heads);
+    prefetch_wg(pf, blockIdx.x, n_heads, gridDim.x);
     return;
   }
   auto stamp = [&](int i) {
@@ -245,7 +245,7 @@ __global__ __launch_bounds__(256) void k_attn_s(const float* __restrict__ q, con
   const int q81 = q81_in & 255;  // bit 8: sequential softmax row sum at any length (strict device), as in k_attn
   const bool strict_sum = (q81_in & 256) != 0;
   if ((int)blockIdx.x >= n_heads) {
-    prefetch_wg(pf, blockIdx.x - n_heads, gridDim.x - n_heads);
+    prefetch_wg(pf, blockIdx.x, n_heads, gridDim.x);
     return;
   }
   auto stamp = [&](int i) {
@@ -461,7 +461,7 @@ __global__ __launch_bounds__(512) void k_attn_short(const float* __restrict__ q,
                                                     signed char* __restrict__ xq, unsigned short* __restrict__ xd, void* __restrict__ xisum,
                                                     int n_heads, int n_kv, int hd, int seq_cap, PrefetchPlan pf, int q81) {
   if ((int)blockIdx.x >= n_heads) {
-    prefetch_wg(pf, blockIdx.x - n_heads, gridDim.x - n_heads);
+    prefetch_wg(pf, blockIdx.x, n_heads, gridDim.x);
     return;
   }
   constexpr int NW = 8, RPI = 64 / LPR, RR = NW * RPI;        // rows of a wave's request / of one from every wave

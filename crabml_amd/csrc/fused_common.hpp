@@ -5,6 +5,7 @@
 #include "dequant.hpp"
 #include "gemv_core.hpp"
 #include "kernels.hpp"
+#include "prefetch.hpp"
 #include "sampler.hpp"
 #include <type_traits>
 
@@ -107,36 +108,6 @@ __device__ __forceinline__ void q8k_exchange_store(const Q8KExchange& ex, const 
     if ((lane & 3) == 0) obs[sb * 16 + (lane >> 2)] = (short)o.quad_sum;
   }
   if (lane == 0 && first == sb * 256) od[sb] = o.d;
-}
-
-// ---- weight prefetch into the Infinity Cache ---------------------------------------------------------
-// The norm+quantize and attention stages are latency-bound single-/few-workgroup kernels: HBM idles for
-// ~6-8 us while they run.  Spare workgroups of those launches (one per otherwise idle CU) stream the NEXT
-// GEMV's weights with plain loads and drop them: the lines land in the 256 MiB memory-side Infinity Cache,
-// so the following HBM-bound GEMV starts on warm data.  Pure performance hint: no result depends on it.
-struct PrefetchPlan {
-  const void* p[3];
-  unsigned long long n[3];  // bytes (multiples of 16)
-  int* sink;
-};
-__device__ __forceinline__ void prefetch_wg(const PrefetchPlan& pf, int wg, int nwg) {
-  int acc = 0;
-#pragma unroll 1
-  for (int sp = 0; sp < 3; sp++) {
-    const i32x4* base = (const i32x4*)pf.p[sp];
-    const size_t n16 = pf.n[sp] / 16;
-    if (!base || n16 == 0) continue;
-    const size_t per = (n16 + nwg - 1) / nwg;
-    const size_t lo = (size_t)wg * per, hi = lo + per < n16 ? lo + per : n16;
-    size_t i = lo + threadIdx.x;
-    const size_t st = blockDim.x;
-    for (; i + 3 * st < hi; i += 4 * st) {
-      i32x4 a = base[i], b = base[i + st], c = base[i + 2 * st], d = base[i + 3 * st];
-      acc ^= a[0] ^ b[1] ^ c[2] ^ d[3];
-    }
-    for (; i < hi; i += st) acc ^= base[i][0];
-  }
-  if (acc == 0x7eadbeef) *pf.sink = acc;  // never true in practice; keeps the loads alive
 }
 
 // ---- embedding lookup: copy_rows_from(token_embed, [token]) (llama2.rs:222-223) ----------------------
@@ -258,11 +229,7 @@ template <int NIT, bool Q81>
 __global__ __launch_bounds__(1024) void k_norm_quant(float* __restrict__ x, const float* __restrict__ addv,
                                                     const float* __restrict__ w, int cols, float eps,
                                                     signed char* __restrict__ q, unsigned short* __restrict__ d,
-                                                    void* __restrict__ isum, PrefetchPlan pf, int half) {
-  if (blockIdx.x > 0) {  // spare workgroups: warm the Infinity Cache with the next GEMV's weights
-    prefetch_wg(pf, blockIdx.x - 1, gridDim.x - 1);
-    return;
-  }
+                                                    void* __restrict__ isum, int half) {
   extern __shared__ float lds[];
   __shared__ float s_rms;
   NormLds L{lds, lds + cols};
@@ -325,11 +292,7 @@ __device__ __forceinline__ void embed_row(const char* __restrict__ w, int dtype,
 }
 template <int NIT, int FRONT>
 __global__ __launch_bounds__(1024) void k_step_front(const char* __restrict__ table, int dtype, size_t off_scale, TokenPick pick, int dim, float* __restrict__ x,
-                                                     const float* __restrict__ wn, float eps, FrontOut o, PrefetchPlan pf, int half) {
-  if (blockIdx.x > 0) {  // spare workgroups: the first GEMV's weights
-    prefetch_wg(pf, blockIdx.x - 1, gridDim.x - 1);
-    return;
-  }
+                                                     const float* __restrict__ wn, float eps, FrontOut o, int half) {
   extern __shared__ float lds[];
   __shared__ float s_rms;
   const int tid = threadIdx.x, lane = tid & 63;

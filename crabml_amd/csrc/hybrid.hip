@@ -452,6 +452,16 @@ void step_linear(Ctx* c, crabml_hip_device::ProfRec* rec, GemvBf16 g) {
     launch_gemv16_bf16<1, IN16, OUT>(c->dev->stream, rec, g, c->dev->n_cu);
 }
 
+// What the launch behind a mixer of more than two rows reads, for the mixer's spare workgroups to touch (prefetch.hpp); none where the weights
+// stay in a cache anyway.  One and two rows: the mixer is the longer for it by what the linear gains (8.8 -> 10.9 and 7.0 -> 5.5 us); 16 rows of
+// 4 layers of width 2048 18593 -> 17965 us for 154 tokens each.  (Latent layers, hosted by k_latent_attn: 0.3 %, not kept.)
+PrefetchPlan prefetch_out(const Ctx* c, const Layer& L, int B) {
+  PrefetchPlan pf{};
+  const int rows = c->width >= 16384 ? 32 : 16;  // (a workgroup of launch_gemv16_bf16)
+  if (B > 2 && c->weight_bytes > RESIDENT_MALL) prefetch_add(pf, L.w_o, (size_t)rows * L.ldc * 2, 0, c->width / rows);
+  return pf;
+}
+
 MixStep mix_step(const Ctx* c, const Run& run, int B) {
   const Layer& L = c->layers[run.layer];
   MixStep m;
@@ -644,11 +654,12 @@ int enqueue_step(Ctx* c, int B, bool sample, bool prof) {
       CH_TRY(c->f32 ? latent_step<float>(c, run, B, prof) : latent_step<unsigned short>(c, run, B, prof));
     } else {
       const MixStep m = mix_step(c, run, B);
+      const PrefetchPlan pf = prefetch_out(c, L, B);
       Prof p(dev, prof, ST_STEP + ST_MIX, 0.0);
       if (c->f32)
-        launch_mix_step<float>(st, p.rec(), m);
+        launch_mix_step<float>(st, p.rec(), m, pf, dev->n_cu);
       else
-        launch_mix_step<unsigned short>(st, p.rec(), m);
+        launch_mix_step<unsigned short>(st, p.rec(), m, pf, dev->n_cu);
     }
     {
       GemvBf16 g;

@@ -10,6 +10,7 @@
 #include <cfloat>
 
 #include "hybrid_common.hpp"
+#include "prefetch.hpp"
 #include "sampler.hpp"
 
 namespace crabml_hip {
@@ -450,9 +451,16 @@ __device__ __forceinline__ void mix_linear(const MixStep& a, int blk, float* lds
   }
 }
 
-template <typename T, int CLS>
-__global__ __launch_bounds__(MIX_THREADS, 4) void k_mix_step(const MixStep a) {
+// used: workgroups of the two branches (PF: the others prefetch)
+template <typename T, int CLS, bool PF>
+__global__ __launch_bounds__(MIX_THREADS, 4) void k_mix_step(const MixStep a, int used, const typename PrefetchArg<PF>::type pf) {
   extern __shared__ __attribute__((aligned(16))) float mix_lds[];
+  if constexpr (PF) {
+    if ((int)blockIdx.x >= used) {
+      prefetch_wg(pf, blockIdx.x, used, gridDim.x);
+      return;
+    }
+  }
   const int n_attn = a.at.H ? a.B * a.at.G * a.head_blocks * a.splits : 0;
   if ((int)blockIdx.x < n_attn)
     mix_attention<T, CLS>(a, blockIdx.x, mix_lds);
@@ -460,25 +468,29 @@ __global__ __launch_bounds__(MIX_THREADS, 4) void k_mix_step(const MixStep a) {
     mix_linear(a, blockIdx.x - n_attn, mix_lds);
 }
 template <typename T, int CLS>
-inline void launch_mix_step_t(hipStream_t st, crabml_hip_device::ProfRec* rec, MixStep a) {
+inline void launch_mix_step_t(hipStream_t st, crabml_hip_device::ProfRec* rec, MixStep a, const PrefetchPlan& pf, int spare) {
   constexpr int NW = MIX_THREADS / 64;
   const int hpg = a.at.H ? a.at.H / a.at.G : 0;
   a.heads = hpg < MIX_HEADS ? hpg : MIX_HEADS;
   const size_t at = a.at.H ? (2 * NW + 3) * MIX_HEADS + 2 * NW + 2 * CLS * sizeof(T) / 4 + (size_t)a.heads * (a.at.D + (NW + 1) * a.at.V) : 0;
   const size_t li = a.li.H ? (size_t)(2 * a.li.D + 32 * 36) * (MIX_THREADS / 256) : 0;
   const int units = a.B * a.li.H * a.li.slices;
-  const unsigned grid = (unsigned)((a.at.H ? a.B * a.at.G * a.head_blocks * a.splits : 0) + (units + MIX_THREADS / 256 - 1) / (MIX_THREADS / 256));
-  launch_k(st, rec, k_mix_step<T, CLS>, dim3(grid), dim3(MIX_THREADS), (at > li ? at : li) * sizeof(float), a);  // (at most 43 KiB)
+  const int used = (a.at.H ? a.B * a.at.G * a.head_blocks * a.splits : 0) + (units + MIX_THREADS / 256 - 1) / (MIX_THREADS / 256);
+  const size_t lds = (at > li ? at : li) * sizeof(float);  // (at most 43 KiB)
+  if (pf.n)
+    launch_k(st, rec, k_mix_step<T, CLS, true>, dim3((unsigned)(used + spare)), dim3(MIX_THREADS), lds, a, used, pf);
+  else
+    launch_k(st, rec, k_mix_step<T, CLS, false>, dim3((unsigned)used), dim3(MIX_THREADS), lds, a, used, NoPrefetch{});
 }
 template <typename T>
-inline void launch_mix_step(hipStream_t st, crabml_hip_device::ProfRec* rec, const MixStep& a) {
+inline void launch_mix_step(hipStream_t st, crabml_hip_device::ProfRec* rec, const MixStep& a, const PrefetchPlan& pf, int spare) {
   const int w = a.at.D > a.at.V ? a.at.D : a.at.V;
   if (w <= 64)
-    launch_mix_step_t<T, 64>(st, rec, a);
+    launch_mix_step_t<T, 64>(st, rec, a, pf, spare);
   else if (w <= 128)
-    launch_mix_step_t<T, 128>(st, rec, a);
+    launch_mix_step_t<T, 128>(st, rec, a, pf, spare);
   else
-    launch_mix_step_t<T, 256>(st, rec, a);
+    launch_mix_step_t<T, 256>(st, rec, a, pf, spare);
 }
 
 }  // namespace crabml_hip

@@ -1,0 +1,63 @@
+// prefetch.hpp -- the next launch's weights into the L2 they will be read through, by workgroups of a launch that leaves memory idle
+//
+// Attention, mixers, merges and the front of a step are chains of a few dependent round trips in a few workgroups.  Spare workgroups of those
+// launches touch every 128-byte line of the next linear's weights (one dword a lane: 64 lines a wave instruction, no register traffic).
+// Workgroup i of a launch runs on XCD i mod 8 and each XCD has an L2 of its own (4 MB), so a line helps most where the workgroup that will
+// read it runs: a plan lists the consumer's workgroups with the bytes each reads, and a spare workgroup takes those of its own XCD.
+// A cold launch that reads 8 / 16 / 32 MB takes 3.1 / 4.5 / 6.7 us, behind such a launch 1.7 / 2.0 / 2.7, and 2.6 / 3.8 / 5.9 where the lines
+// were touched from another XCD (they are in the Infinity Cache then).  Above what the L2s hold (64 MB: 10.2 against 12.4) it is not worth
+// its traffic.  No result depends on it, nor on where a workgroup runs.
+#pragma once
+#include "devutil.hpp"
+
+namespace crabml_hip {
+
+struct PrefetchPlan {
+  static constexpr int MAX = 2;
+  const char* p[MAX];       // workgroup first + i of the next launch (i < count) reads `bytes` bytes at p + i * bytes
+  unsigned bytes[MAX];
+  int first[MAX], count[MAX];
+  int n;
+};
+// a kernel that hosts it is a template of PF, so that where there is nothing to prefetch it is the kernel without (its larger arguments alone cost a one-row step 1 %)
+struct NoPrefetch {};
+template <bool PF>
+struct PrefetchArg {
+  typedef NoPrefetch type;
+};
+template <>
+struct PrefetchArg<true> {
+  typedef PrefetchPlan type;
+};
+inline void prefetch_add(PrefetchPlan& pf, const void* p, size_t bytes, int first, int count) {
+  if (pf.n == PrefetchPlan::MAX || bytes < 4 || bytes > (1u << 30) || count < 1) return;
+  pf.p[pf.n] = (const char*)p;
+  pf.bytes[pf.n] = (unsigned)bytes;
+  pf.first[pf.n] = first;
+  pf.count[pf.n++] = count;
+}
+
+// wg: this workgroup's place in the launch (x fastest); the launch's spare ones are [base, all)
+__device__ __forceinline__ void prefetch_wg(const PrefetchPlan& pf, int wg, int base, int all) {
+  const int x = wg & 7, at = base + ((x - base) & 7), nw = blockDim.x >> 6, lane = threadIdx.x & 63;
+  const int waves = ((all - 1 - at) / 8 + 1) * nw, me = ((wg - at) >> 3) * nw + wave_in_wg();  // of this XCD
+  for (int s = 0; s < pf.n; s++) {
+    const char* p = pf.p[s];
+    const unsigned bytes = pf.bytes[s], pieces = (bytes + 8191) >> 13;
+    const int i0 = (x - pf.first[s]) & 7;
+    const unsigned items = pf.count[s] > i0 ? (unsigned)((pf.count[s] - i0 + 7) >> 3) * pieces : 0;
+    for (unsigned j = me; j < items; j += 2 * waves) {
+      unsigned v[2];
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const unsigned k = j + u * waves < items ? j + u * waves : j, i = k / pieces;
+        unsigned o = (k - i * pieces) * 8192 + lane * 128;
+        o = o < bytes - 3 ? o : bytes - 4;  // (the workgroup's last bytes: a line that is read anyway)
+        v[u] = *(const unsigned*)((size_t)(p + (size_t)(i0 + 8 * i) * bytes + o) & ~(size_t)3);
+      }
+      asm volatile("" ::"v"(v[0]), "v"(v[1]));  // (the loads stay; nothing is stored)
+    }
+  }
+}
+
+}  // namespace crabml_hip
