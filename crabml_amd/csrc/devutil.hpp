@@ -4,6 +4,13 @@
 
 namespace crabml_hip {
 
+// A pointer that a kernel reads from memory (a sequence's slab) is generic to the compiler, and generic loads count as LDS accesses too:
+// every wait for LDS then waits for them.  This says that it points to device memory.
+template <typename T>
+__device__ __forceinline__ T* as_global(T* p) {
+  return (T*)(__attribute__((address_space(1))) T*)(size_t)p;
+}
+
 // half crate semantics: from_f32 = IEEE RNE (v_cvt_f16_f32 in the default round mode), to_f32 exact.
 __device__ __forceinline__ float h2f(unsigned short h) {
   _Float16 x;
@@ -107,6 +114,19 @@ __device__ __forceinline__ float meet16(float a, float b) {
   const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
   const unsigned lo = r[0], hi = r[1];
   return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+}
+// the larger of the two, in both
+__device__ __forceinline__ float max32(float a) {
+  const unsigned u = __builtin_bit_cast(unsigned, a);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const unsigned lo = r[0], hi = r[1];
+  return fmaxf(__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi));
+}
+__device__ __forceinline__ float max16(float a) {
+  const unsigned u = __builtin_bit_cast(unsigned, a);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const unsigned lo = r[0], hi = r[1];
+  return fmaxf(__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi));
 }
 // Sums over the 64 / LPR groups of LPR lanes.  Of a lane's eight columns it is left with the sums of two -- pair 2 (lane / 32) + (lane / 16) % 2
 // of the four -- in acc[0], acc[1] (LPR = 32: of four, half lane / 32 of the eight).  LPR = 8: lanes 8-15 of a row hold what lanes 0-7 do.

@@ -841,10 +841,16 @@ struct Part {  // rows of one sequence in one pass
 
 template <typename T, int KC, int VC, bool LAT>
 void launch_attn_cls(Ctx* c, crabml_hip_device::ProfRec* rec, MixRows<T> m, const PassTiles& tiles) {
-  constexpr int big = AttnTile<T, KC, VC>::RT - 1;
+  constexpr int P = sizeof(T) == 2 ? 1 : 3;
+  // 64 query rows a workgroup, or 128: a tile's trip through LDS then serves twice the rows, which pays where two workgroups of them a CU are left.  us,
+  // 64 / 128, 2048 rows: 48 heads of 128 149 / 138, 32 heads of 128 in a window 82 / 71, latent 92 / 82; 16 heads of 128 82 / 94, in a
+  // window 52 / 54; 4 x 500 rows, 32 heads of 128 39 / 45; heads of 64 never (32 of them, 2048 rows: 62 / 72).
+  const bool big = AttnTile<T, KC, VC>::RT == 2 && (size_t)m.at.H * tiles.n[1] >= 2 * (size_t)c->dev->n_cu;
   m.tiles = tiles.list[big];
-  m.n_tiles = (int)tiles.n[big];
-  launch_k(c->dev->stream, rec, k_attn_rows<T, KC, VC, sizeof(T) == 2 ? 1 : 3, LAT>, dim3(m.n_tiles, m.at.H), dim3(256), 0, m);
+  const dim3 grid((unsigned)(tiles.n[big] * m.at.H));
+  if constexpr (AttnTile<T, KC, VC>::RT == 2)
+    if (big) return launch_k(c->dev->stream, rec, k_attn_rows<T, KC, VC, P, LAT, 2>, grid, dim3(256), 0, m);
+  launch_k(c->dev->stream, rec, k_attn_rows<T, KC, VC, P, LAT, 1>, grid, dim3(256), 0, m);
 }
 template <typename T, bool LAT>
 void launch_attn(Ctx* c, const MixRows<T>& m, const PassTiles& tiles) {
@@ -971,6 +977,8 @@ int run_pass(Ctx* c, const std::vector<Part>& parts, float** logits) {
     }
     M += p.n;
   }
+  for (size_t b = 0; b < 2; b++)  // the tiles that see the most keys first
+    std::stable_sort(ht[b], ht[b] + n_tiles[b], [](const PassTile& x, const PassTile& y) { return x.pos + x.n > y.pos + y.n; });
   size_t n_hist = 0;  // earlier positions that latent layers read again
   for (size_t i = 0; i < parts.size(); i++) {
     const int len = (int)c->seqs[parts[i].seq].len, n = (int)std::min(c->hist, (size_t)len);

@@ -37,7 +37,7 @@ __global__ __launch_bounds__(256) void k_latent_rows(const MixRows<T> a) {
   const PassSeq sq = a.seqs[rw.seq];
   if (r >= a.M) {  // an earlier position: zero where this layer no longer sees it (and no longer has it)
     const bool seen = rw.pos >= attn_first(g, sq.pos0);
-    const T* c = (const T*)(sq.slab + a.rs.k) + (size_t)(rw.pos % g.span) * (l.rank + l.rot);
+    const T* c = as_global((const T*)(sq.slab + a.rs.k)) + (size_t)(rw.pos % g.span) * (l.rank + l.rot);
     for (int i = tid; i < l.rank; i += 256) {
       const T v = seen ? c[i] : kv_from<T>(0.f);
       if constexpr (P == 1)
@@ -82,7 +82,7 @@ __global__ __launch_bounds__(256) void k_latent_append(const MixRows<T> a) {
   const PassRow rw = a.rows[r];
   const PassSeq sq = a.seqs[rw.seq];
   if (rw.pos < attn_first(a.at, sq.pos0 + sq.n - 1)) return;
-  T* c = (T*)(sq.slab + a.rs.k) + (size_t)(rw.pos % a.at.span) * (l.rank + l.rot);
+  T* c = as_global((T*)(sq.slab + a.rs.k)) + (size_t)(rw.pos % a.at.span) * (l.rank + l.rot);
   for (int i = tid; i < l.rank; i += 256) c[i] = latent_elem<T, P>(a, r, i);
   for (int i = tid; i < l.rot; i += 256) c[l.rank + i] = a.rot[(size_t)r * l.rot + i];
 }
@@ -136,7 +136,7 @@ __global__ __launch_bounds__(256) void k_latent_query(const LatStep a) {
     const int b = blockIdx.x - g.H * slices, np = l.rot / 2;
     const StepSeq sq = a.seq[b];
     const float* pr = a.proj + (size_t)b * a.ldp;
-    T* c = (T*)(sq.slab + a.rs.k) + (size_t)(sq.pos % g.span) * row_w;
+    T* c = as_global((T*)(sq.slab + a.rs.k)) + (size_t)(sq.pos % g.span) * row_w;
     if (tid < np) {
       const float ang = reduced_angle(sq.pos, l.freq[tid]);
       lat_lds[2 * tid] = cosf(ang);
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(256) void k_latent_attn(const LatStep a) {
   const LatRange rg = latent_range<T>(g, a.splits, sq.pos);
   const int lo = split * rg.per, hi = lo + rg.per < rg.n ? lo + rg.per : rg.n;
   if (lo >= hi) return;  // (whole workgroup)
-  const T* cache = (const T*)(sq.slab + a.rs.k);
+  const T* cache = as_global((const T*)(sq.slab + a.rs.k));
   // a tile's octets in row order, 256 at a time: thread t starts at (row tr0, octet tc0) and goes on by (dr, dc)
   const int tr0 = tid / cpr, tc0 = tid % cpr, dr = 256 / cpr, dc = 256 % cpr;
   constexpr int UN = sizeof(T) == 2 ? 9 : 5;  // octets in flight per thread

@@ -175,59 +175,72 @@ struct MixRows {
   int M = 0;              // rows of this pass
 };
 
-// Shape of the attention kernel for keys up to KC and values up to VC wide: KT keys per tile; RT times 16 query rows per wave.
+// (by value: a choice between two variables is one between their addresses otherwise, and puts them into memory)
+template <typename T>
+__device__ __forceinline__ const T* one_of(bool first, const T* a, const T* b) {
+  return as_global((const T*)(first ? (size_t)a : (size_t)b));
+}
+
+// Shape of the attention kernel for keys up to KC and values up to VC wide: KT keys per tile; up to RT times 16 query rows per wave.
 template <typename T, int KC, int VC>
 struct AttnTile {
   static constexpr int PAD = 16 / sizeof(T), KT = sizeof(T) == 2 ? (KC > 128 ? 32 : 64) : 4096 / KC;
-  static constexpr int RT = sizeof(T) == 2 && KC <= 192 && VC <= 128 ? 2 : 1;
+  static constexpr int RT = sizeof(T) == 2 && KC > 64 && KC <= 192 && VC <= 128 ? 2 : 1;
 };
 
 // One workgroup: 64 RT query rows of one head, four waves of 16 RT.  Keys come in tiles through LDS (K as rows, V transposed), the next
-// tile's rows already on their way into registers while the current one is multiplied.
+// tile's rows already on their way into registers while the current one is multiplied.  What bounds it is the chain of tiles: 64 keys of 128
+// columns take a workgroup 4700 cycles, of which scores 810, softmax 1160, values 1300 and the way through LDS 960, and the last
+// rows of 2048 see 32 of them; so few rows a workgroup (launch_attn_cls), the rows with the most keys first.  16 heads of 128, 2048 rows:
+// 157 -> 82 us, 700 rows in a window 62 -> 33 (latent 64 -> 43), against 128 rows a workgroup, loads through generic pointers (every LDS
+// wait waited for them) and a branch a score.
 // Everything is transposed -- S^T = K Q^T, O^T = V^T P^T -- so that a lane owns one query row (its column): the softmax statistics are
 // one number per lane, and the accumulators of S^T, exponentiated, ARE the operand of the second product: k slot (lane / 16, i) of the
 // matrix instruction stands for key 4 (lane / 16) + i of a 16-key group, and V^T is read from LDS in the same order.  Scores live in
 // the log2 domain.
-template <typename T, int KC, int VC, int P, bool LAT>
-__global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void k_attn_rows(const MixRows<T> a) {
+template <typename T, int KC, int VC, int P, bool LAT, int RT>
+__global__ __launch_bounds__(256, sizeof(T) == 2 ? (RT == 1 && KC <= 128 ? 3 : 2) : 1) void k_attn_rows(const MixRows<T> a) {
   typedef AttnTile<T, KC, VC> A;
-  constexpr int KT = A::KT, RT = A::RT, LK = KC + A::PAD, LV = KT + A::PAD, VT = VC / 16, ST = KT / 16;
+  constexpr int KT = A::KT, LK = KC + A::PAD, LV = KT + A::PAD, VT = VC / 16, ST = KT / 16;
   constexpr int NK = KT * KC / 8 / 256, NV = KT * VC / 8 / 256;  // octets of K and of V per thread and tile
   static_assert(NK >= 1 && NV >= 2 && NV % 2 == 0, "V octets are handled in pairs of keys");
   __shared__ __attribute__((aligned(16))) T ks[KT * LK];
   __shared__ __attribute__((aligned(16))) T vs[VC * LV];
   const AttnGeom& g = a.at;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_wg(), fr = lane & 15, fk = lane >> 4;
-  const PassTile t = a.tiles[a.n_tiles - 1 - blockIdx.x];  // (a sequence's last tiles see the most keys: first)
+  const PassTile t = a.tiles[blockIdx.x / g.H];  // (tiles that see the most keys first)
   const PassSeq sq = a.seqs[t.seq];
-  const int h = blockIdx.y, kvh = h / (g.H / g.G);
+  const int h = blockIdx.x % g.H, kvh = h / (g.H / g.G);
   const int DK = (g.D + 31) & ~31;
   const int lo = attn_first(g, t.pos), hi = t.pos + t.n;  // keys [lo, hi); those before pos0 are cache rows from that of `lo` on
   const int ring = lo % g.span;
-  const T* kc = (const T*)(sq.slab + a.rs.k) + (size_t)kvh * g.rows * g.D;
-  const T* vc = (const T*)(sq.slab + a.rs.v) + (size_t)kvh * g.rows * g.V;
+  const T* kc = as_global((const T*)(sq.slab + a.rs.k)) + (size_t)kvh * g.rows * g.D;
+  const T* vc = as_global((const T*)(sq.slab + a.rs.v)) + (size_t)kvh * g.rows * g.V;
   const T* pk = a.proj + (size_t)sq.row0 * a.ldp + g.ck + kvh * g.D;
   const T* pv = a.proj + (size_t)sq.row0 * a.ldp + g.cv + kvh * g.V;
   const int ldkv = LAT ? g.H * (a.la.dim + g.V) : 0;
-  // position p, column c -> the octet of its key / value
-  auto k_at = [&](int p, int c) -> const T* {
+  // position p, column c -> the octet of its key / value.  Addresses are chosen, not loads: a load under a condition ends the loads in flight.
+  auto k_at = [=](int p, int c) -> const T* {
     if constexpr (LAT) {
       const size_t row = (size_t)((p >= sq.pos0 ? sq.row0 : sq.hist_end) + (p - sq.pos0));
-      return c < a.la.dim ? a.kv + row * ldkv + h * a.la.dim + c : a.rot + row * a.la.rot + (c - a.la.dim);
+      const T *k = a.kv + row * ldkv + h * a.la.dim, *rot = a.rot + row * a.la.rot - a.la.dim;
+      return one_of(c < a.la.dim, k, rot) + c;
     } else {
-      if (p >= sq.pos0) return pk + (size_t)(p - sq.pos0) * a.ldp + c;
+      const bool own = p >= sq.pos0;
       const int r = ring + (p - lo);
-      return kc + (size_t)(r < g.span ? r : r - g.span) * g.D + c;
+      const size_t at = own ? (size_t)(unsigned)(p - sq.pos0) * (unsigned)a.ldp : (size_t)(unsigned)(r < g.span ? r : r - g.span) * (unsigned)g.D;
+      return one_of(own, pk, kc) + at + c;
     }
   };
-  auto v_at = [&](int p, int c) -> const T* {
+  auto v_at = [=](int p, int c) -> const T* {
     if constexpr (LAT) {
       const size_t row = (size_t)((p >= sq.pos0 ? sq.row0 : sq.hist_end) + (p - sq.pos0));
       return a.kv + row * ldkv + g.H * a.la.dim + h * g.V + c;
     } else {
-      if (p >= sq.pos0) return pv + (size_t)(p - sq.pos0) * a.ldp + c;
+      const bool own = p >= sq.pos0;
       const int r = ring + (p - lo);
-      return vc + (size_t)(r < g.span ? r : r - g.span) * g.V + c;
+      const size_t at = own ? (size_t)(unsigned)(p - sq.pos0) * (unsigned)a.ldp : (size_t)(unsigned)(r < g.span ? r : r - g.span) * (unsigned)g.V;
+      return one_of(own, pv, vc) + at + c;
     }
   };
   // this wave's rows, and the keys any of them sees
@@ -265,18 +278,42 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void k_attn_rows(const
   }
   const float amp = g.amp ? g.amp[h] : 0.f, rate = g.amp ? g.rate[h] : 0.f, scale2 = g.scale * 1.44269504f;
   Oct<T> rk[NK], rv[NV];
+  // A tile of this pass's own keys: one base for the workgroup and offsets that stay, where the general form spends some 30 instructions a load
+  unsigned ko[NK], vo[NV];
+#pragma unroll
+  for (int u = 0; u < NK; u++) {
+    const int i = u * 256 + tid, c = i % (KC / 8) * 8, row = i / (KC / 8), cc = c < g.D ? c : 0;
+    ko[u] = LAT ? (cc < a.la.dim ? row * ldkv + cc : row * a.la.rot + cc - a.la.dim) : row * a.ldp + cc;
+  }
+#pragma unroll
+  for (int u = 0; u < NV; u++) {
+    const int i = (u >> 1) * 256 + tid, c = i / (KT / 2) * 8, row = i % (KT / 2) * 2 + (u & 1);
+    vo[u] = row * (LAT ? ldkv : a.ldp) + (c < g.V ? c : 0);
+  }
+  // (past the last key: that one again, which no row's probabilities count; past the last column: column 0, zero in K's tile, unused in V's)
   auto request = [&](int j0) {
+    if (j0 >= sq.pos0 && j0 + KT <= hi) {
+      const size_t row = (size_t)(sq.row0 + (j0 - sq.pos0));
+      const T* kb = LAT ? a.kv + row * ldkv + h * a.la.dim : a.proj + row * a.ldp + g.ck + kvh * g.D;
+      const T* vb = LAT ? a.kv + row * ldkv + g.H * a.la.dim + h * g.V : a.proj + row * a.ldp + g.cv + kvh * g.V;
+#pragma unroll
+      for (int u = 0; u < NK; u++) {
+        const int c = (u * 256 + tid) % (KC / 8) * 8;
+        rk[u] = oct_load((LAT ? one_of(c < a.la.dim || c >= g.D, kb, a.rot + row * a.la.rot) : kb) + ko[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < NV; u++) rv[u] = oct_load(vb + vo[u]);
+      return;
+    }
 #pragma unroll
     for (int u = 0; u < NK; u++) {
       const int i = u * 256 + tid, c = i % (KC / 8) * 8, p = j0 + i / (KC / 8);
-      rk[u] = oct_zero<T>();
-      if (p < hi && c < g.D) rk[u] = oct_load(k_at(p, c));
+      rk[u] = oct_load(k_at(p < hi ? p : hi - 1, c < g.D ? c : 0));
     }
 #pragma unroll
     for (int u = 0; u < NV; u++) {  // octets u, u + 1: the same columns of two neighbouring keys
       const int i = (u >> 1) * 256 + tid, c = i / (KT / 2) * 8, p = j0 + i % (KT / 2) * 2 + (u & 1);
-      rv[u] = oct_zero<T>();
-      if (p < hi && c < g.V) rv[u] = oct_load(v_at(p, c));
+      rv[u] = oct_load(v_at(p < hi ? p : hi - 1, c < g.V ? c : 0));
     }
   };
   request(lo);
@@ -284,8 +321,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void k_attn_rows(const
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < NK; u++) {
-      const int i = u * 256 + tid;
-      oct_store(ks + i / (KC / 8) * LK + i % (KC / 8) * 8, rk[u]);
+      const int i = u * 256 + tid, c = i % (KC / 8) * 8;
+      oct_store(ks + i / (KC / 8) * LK + c, c < g.D ? rk[u] : oct_zero<T>());
     }
 #pragma unroll
     for (int u = 0; u < NV; u += 2) {
@@ -312,7 +349,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void k_attn_rows(const
       if constexpr (sizeof(T) == 2) {
 #pragma unroll
         for (int i = 0; i < KC / 32; i++)
-          if (i * 32 < DK) {
+          if (KC <= 128 || i * 32 < DK) {  // (a check here keeps loads and products of neighbours apart)
             const bf16x8 kf = *(const bf16x8*)(kr + i * 32 + fk * 8);
 #pragma unroll
             for (int r = 0; r < RT; r++) s[r][j] = mfma_bf16(kf, q16[r][i], s[r][j]);
@@ -330,22 +367,30 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void k_attn_rows(const
 #pragma unroll
     for (int r = 0; r < RT; r++) {
       const float d0 = (float)(pos[r] - j0 - fk * 4);  // distance to this lane's first key of the tile
+#pragma unroll
+      for (int j = 0; j < ST; j++) s[r][j] *= scale2;
+      if (g.amp) {
+#pragma unroll
+        for (int j = 0; j < ST; j++)
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+            s[r][j][e] = __builtin_fmaf(-amp, __builtin_amdgcn_logf(__builtin_fmaf(rate, d0 - (float)(j * 16 + e), 1.0f)), s[r][j][e]);
+      }
+      if (edge) {
+#pragma unroll
+        for (int j = 0; j < ST; j++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const int p = j0 + j * 16 + fk * 4 + e;
+            s[r][j][e] = p <= pos[r] && p >= first[r] ? s[r][j][e] : -INFINITY;
+          }
+      }
       float mx = -INFINITY;
 #pragma unroll
       for (int j = 0; j < ST; j++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-          float v = s[r][j][e] * scale2;
-          if (g.amp) v = __builtin_fmaf(-amp, __builtin_amdgcn_logf(__builtin_fmaf(rate, d0 - (float)(j * 16 + e), 1.0f)), v);
-          if (edge) {
-            const int p = j0 + j * 16 + fk * 4 + e;
-            v = p <= pos[r] && p >= first[r] ? v : -INFINITY;
-          }
-          s[r][j][e] = v;
-          mx = fmaxf(mx, v);
-        }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        for (int e = 0; e < 4; e++) mx = fmaxf(mx, s[r][j][e]);
+      mx = max16(max32(mx));
       mx = fmaxf(m[r], mx);
       const float ref = mx == -INFINITY ? 0.f : mx, w = __builtin_amdgcn_exp2f(m[r] - ref);
       m[r] = mx;
@@ -359,8 +404,10 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void k_attn_rows(const
           sum += pe;
         }
       l[r] = __builtin_fmaf(l[r], w, sum);  // (this lane's keys; the four lanes of a row are added at the end)
+      if (!__all(w == 1.f)) {
 #pragma unroll
-      for (int j = 0; j < VT; j++) o[r][j] *= w;
+        for (int j = 0; j < VT; j++) o[r][j] *= w;
+      }
     }
     if constexpr (sizeof(T) == 2) {
 #pragma unroll
@@ -375,7 +422,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void k_attn_rows(const
           }
 #pragma unroll
         for (int j = 0; j < VT; j++)
-          if (j * 16 < g.V) {
+          if (VC <= 128 || j * 16 < g.V) {
             const T* vr = vs + (j * 16 + fr) * LV + jj * 16 + fk * 4;
             bf16x8 vf;
             __builtin_memcpy(&vf, vr, 8);
@@ -400,9 +447,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? 2 : 1) void k_attn_rows(const
   }
 #pragma unroll
   for (int r = 0; r < RT; r++) {
-    float den = l[r];
-    den += __shfl_xor(den, 16, 64);
-    den += __shfl_xor(den, 32, 64);
+    const float v = meet16(l[r], l[r]);
+    float den = meet32(v, v);
     const int row = w0 + r * 16 + fr;
     if (row >= t.n) continue;
     float w = 1.f;
@@ -620,8 +666,8 @@ __global__ __launch_bounds__(256) void k_mix_rows(const MixRows<T> a, float eps)
     const PassSeq sq = a.seqs[rw.seq];
     const int last = sq.pos0 + sq.n - 1;
     if (rw.pos < attn_first(g, last)) return;
-    T* kc = (T*)(sq.slab + a.rs.k);
-    T* vc = (T*)(sq.slab + a.rs.v);
+    T* kc = as_global((T*)(sq.slab + a.rs.k));
+    T* vc = as_global((T*)(sq.slab + a.rs.v));
     const size_t at = (size_t)(rw.pos % g.span);
     for (int i = tid; i < g.G * g.D; i += 256) kc[((size_t)(i / g.D) * g.rows + at) * g.D + i % g.D] = pr[g.ck + i];
     for (int i = tid; i < g.G * g.V; i += 256) vc[((size_t)(i / g.V) * g.rows + at) * g.V + i % g.V] = pr[g.cv + i];

@@ -176,8 +176,8 @@ __device__ __forceinline__ void mix_attention(const MixStep& a, int blk, float* 
   }
   if (split >= active) return;  // (whole workgroup)
   const int r0 = split * share, r1 = r0 + share < n_rows ? r0 + share : n_rows;
-  T* kc = (T*)(sq.slab + a.rs.k) + (size_t)kvh * g.rows * g.D;
-  T* vc = (T*)(sq.slab + a.rs.v) + (size_t)kvh * g.rows * g.V;
+  T* kc = as_global((T*)(sq.slab + a.rs.k)) + (size_t)kvh * g.rows * g.D;
+  T* vc = as_global((T*)(sq.slab + a.rs.v)) + (size_t)kvh * g.rows * g.V;
   const bool own_new = in_chunk >= r0 && in_chunk < r1;
   const int rc = lane / LPR, c = lane % LPR * 8;
   const bool kcol = c < g.D, vcol = c < g.V;
@@ -397,7 +397,7 @@ __device__ __forceinline__ void mix_linear(const MixStep& a, int blk, float* lds
   lds += part * (2 * g.D + 32 * 36);
   const int slice = blk % g.slices, h = (blk / g.slices) % g.H, b = blk / (g.slices * g.H);
   const StepSeq sq = a.seq[b];
-  float* S = (float*)(sq.slab + a.rs.s) + (size_t)h * g.D * g.V;
+  float* S = as_global((float*)(sq.slab + a.rs.s)) + (size_t)h * g.D * g.V;
   const float* pr = a.proj + (size_t)b * a.ldp;
   float* k_s = lds;        // [D]
   float* q_s = k_s + g.D;  // [D]

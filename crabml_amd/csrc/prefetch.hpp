@@ -53,7 +53,7 @@ __device__ __forceinline__ void prefetch_wg(const PrefetchPlan& pf, int wg, int 
         const unsigned k = j + u * waves < items ? j + u * waves : j, i = k / pieces;
         unsigned o = (k - i * pieces) * 8192 + lane * 128;
         o = o < bytes - 3 ? o : bytes - 4;  // (the workgroup's last bytes: a line that is read anyway)
-        v[u] = *(const unsigned*)((size_t)(p + (size_t)(i0 + 8 * i) * bytes + o) & ~(size_t)3);
+        v[u] = *as_global((const unsigned*)((size_t)(p + (size_t)(i0 + 8 * i) * bytes + o) & ~(size_t)3));
       }
       asm volatile("" ::"v"(v[0]), "v"(v[1]));  // (the loads stay; nothing is stored)
     }
