@@ -100,7 +100,7 @@ struct crabml_hip_hybrid {
   size_t rows_cap = 0, hist_cap = 0, meta_bytes = 0;
   char *meta = nullptr, *h_meta = nullptr;
   int h_meta_next = 0;
-  float *pf_x = nullptr, *pf_emb = nullptr, *pf_lin = nullptr, *pf_sq = nullptr, *pf_gsq = nullptr, *pf_logits = nullptr;
+  float *pf_x = nullptr, *pf_emb = nullptr, *pf_lin = nullptr, *pf_states = nullptr, *pf_sq = nullptr, *pf_gsq = nullptr, *pf_logits = nullptr;
   unsigned short *pf_xp = nullptr, *pf_cat = nullptr, *pf_u = nullptr, *pf_gp = nullptr;
   void *pf_proj = nullptr, *pf_vk = nullptr, *pf_rot = nullptr, *pf_kv = nullptr;
   unsigned short* pf_lat = nullptr;
@@ -795,7 +795,11 @@ int pass_alloc(Ctx* c) {
   crabml_hip_device* dev = c->dev;
   const size_t R = align_up(c->cfg.pass_rows ? c->cfg.pass_rows : 2048, 256), P = (size_t)c->planes;
   size_t lin = 0;
-  for (const Layer& L : c->layers) lin = std::max(lin, (size_t)L.li.H * L.li.V);
+  size_t lin_d = 0;
+  for (const Layer& L : c->layers) {
+    lin = std::max(lin, (size_t)L.li.H * L.li.V);
+    if (L.li.H) lin_d = std::max<size_t>(lin_d, L.li.D <= 64 ? 64 : L.li.D <= 128 ? 128 : 256);
+  }
   const size_t S = c->streams ? (size_t)c->streams : 1, e = c->f32 ? 4 : 2, Hc = c->hist ? align_up(std::max(R, c->hist), 256) : 0;
   CH_TRY(dalloc_n(c, S * R * c->ldx, &c->pf_x));
   if (c->keep_emb) CH_TRY(dalloc_n(c, R * c->ldx, &c->pf_emb));
@@ -808,6 +812,7 @@ int pass_alloc(Ctx* c) {
     CH_TRY(dalloc(c, (R + Hc) * c->ld_kv * e, &c->pf_kv));
   }
   CH_TRY(dalloc_n(c, P * R * c->ld_cat, &c->pf_cat));
+  CH_TRY(dalloc_n(c, 2 * dev->n_cu * lin_d * LIN_SLICE, &c->pf_states));  // (lin_segments)
   CH_TRY(dalloc_n(c, R * lin, &c->pf_lin));
   CH_TRY(dalloc_n(c, P * R * c->ld_u, &c->pf_u));
   CH_TRY(dalloc_n(c, R * c->n_sq, &c->pf_sq));
@@ -863,15 +868,22 @@ void launch_attn(Ctx* c, const MixRows<T>& m, const PassTiles& tiles) {
   launch_attn_cls<T, 256, 256, LAT>(c, p.rec(), m, tiles);
 }
 template <typename T, int CLS>
-int launch_linear_cls(Ctx* c, hipStream_t st, crabml_hip_device::ProfRec* rec, const MixRows<T>& m, size_t n_seq) {
+int launch_linear_cls(Ctx* c, hipStream_t st, crabml_hip_device::ProfRec* rec, MixRows<T> m, size_t n_seq, size_t longest) {
   const size_t lds = LinTile<T, CLS>::LDS;
-  CH_HIP(c->dev, raise_dyn_lds(c->dev, (const void*)k_linear_rows<T, CLS>, (int)lds));
-  launch_k(st, rec, k_linear_rows<T, CLS>, dim3(m.li.H * m.li.slices, (unsigned)n_seq), dim3(256), lds, m);
+  m.lin_segs = lin_segments(c->dev->n_cu, (int)(m.li.H * m.li.slices * n_seq), (int)longest, LinTile<T, CLS>::C);
+  m.lin_state = c->pf_states;
+  const dim3 grid(m.li.H * m.li.slices, (unsigned)n_seq, (unsigned)m.lin_segs);
+  if (m.lin_segs > 1) {
+    CH_HIP(c->dev, raise_dyn_lds(c->dev, (const void*)k_linear_rows<T, CLS, true>, (int)lds));
+    launch_k(st, nullptr, k_linear_rows<T, CLS, true>, dim3(grid.x, grid.y, grid.z - 1), dim3(256), lds, m);
+  }
+  CH_HIP(c->dev, raise_dyn_lds(c->dev, (const void*)k_linear_rows<T, CLS, false>, (int)lds));
+  launch_k(st, rec, k_linear_rows<T, CLS, false>, grid, dim3(256), lds, m);
   return 0;
 }
 
 template <typename T>
-int mix_rows(Ctx* c, const Run& run, const PassSeq* seqs, size_t n_seq, const PassTiles& tiles, const PassRow* rows, size_t n_rows, size_t n_hist) {
+int mix_rows(Ctx* c, const Run& run, const PassSeq* seqs, size_t n_seq, size_t longest, const PassTiles& tiles, const PassRow* rows, size_t n_rows, size_t n_hist) {
   constexpr int P = sizeof(T) == 2 ? 1 : 3;
   const Layer& L = c->layers[run.layer];
   MixRows<T> m;
@@ -932,11 +944,11 @@ int mix_rows(Ctx* c, const Run& run, const PassSeq* seqs, size_t n_seq, const Pa
   if (L.li.H) {
     Prof p(c->dev, true, ST_PASS + ST_LIN, 0.0);
     if (L.li.D <= 64)
-      CH_TRY((launch_linear_cls<T, 64>(c, lin_st, p.rec(), m, n_seq)));
+      CH_TRY((launch_linear_cls<T, 64>(c, lin_st, p.rec(), m, n_seq, longest)));
     else if (L.li.D <= 128)
-      CH_TRY((launch_linear_cls<T, 128>(c, lin_st, p.rec(), m, n_seq)));
+      CH_TRY((launch_linear_cls<T, 128>(c, lin_st, p.rec(), m, n_seq, longest)));
     else
-      CH_TRY((launch_linear_cls<T, 256>(c, lin_st, p.rec(), m, n_seq)));
+      CH_TRY((launch_linear_cls<T, 256>(c, lin_st, p.rec(), m, n_seq, longest)));
   }
   if (lin_st != st) CH_HIP(c->dev, hipEventRecord(c->join, lin_st));
   if (L.at.H) launch_attn<T, false>(c, m, tiles);
@@ -962,9 +974,10 @@ int run_pass(Ctx* c, const std::vector<Part>& parts, float** logits) {
   PassTile* ht[2] = {(PassTile*)(hm + o_tile), (PassTile*)(hm + o_tile) + R};
   PassRow* hr = (PassRow*)(hm + o_row);
   int *hk = (int*)(hm + o_tok), *hw = (int*)(hm + o_want);
-  size_t n_tiles[2] = {0, 0}, M = 0, nw = 0;
+  size_t n_tiles[2] = {0, 0}, M = 0, nw = 0, longest = 0;
   for (size_t i = 0; i < parts.size(); i++) {
     const Part& p = parts[i];
+    longest = std::max(longest, p.n);
     const Seq& s = c->seqs[p.seq];
     hs[i] = PassSeq{(int)M, (int)p.n, (int)s.len, (int)M, s.slab};
     for (size_t b = 0; b < 2; b++)
@@ -1048,9 +1061,9 @@ int run_pass(Ctx* c, const std::vector<Part>& parts, float** logits) {
       launch_gemm_bf16(dev, p.rec(), c->planes, c->f32 ? GEMM_OUT_ACT_F32 : GEMM_OUT_ACT_BF16, g, c->pf_scratch);
     }
     if (c->f32)
-      CH_TRY(mix_rows<float>(c, run, ds, parts.size(), dt, dr, M, n_hist));
+      CH_TRY(mix_rows<float>(c, run, ds, parts.size(), longest, dt, dr, M, n_hist));
     else
-      CH_TRY(mix_rows<unsigned short>(c, run, ds, parts.size(), dt, dr, M, n_hist));
+      CH_TRY(mix_rows<unsigned short>(c, run, ds, parts.size(), longest, dt, dr, M, n_hist));
     {
       GemmBf16 g = residual(c->pf_cat, R * (size_t)c->ld_cat, L.w_o, L.ldc);
       if (!L.ff) {

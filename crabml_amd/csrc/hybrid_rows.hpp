@@ -164,7 +164,9 @@ struct MixRows {
   unsigned short* cat = nullptr;
   size_t cat_plane = 0;
   float* lin = nullptr;  // [rows][H * V] raw outputs of the linear branch
-  int n_tiles = 0, ldp = 0, ldc = 0, lin_off = 0;
+  float* lin_state = nullptr;  // [sequences][H * slices][lin_segs] states in front of the segments (LinTile::STATE floats each)
+  int lin_segs = 1;
+  int ldp = 0, ldc = 0, lin_off = 0;
   T* v_kept = nullptr;  // [rows][ld_vk] values that VMIX_KEEP leaves
   int ld_vk = 0;
   // latent attention: rows of this pass, then the earlier ones (PassSeq::hist_end)
@@ -479,6 +481,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RT == 1 && KC <= 128 ? 3 : 2
 //   o_i = d^(i+1) S^T q_i + sum_{j <= i} d^(i-j) (q_i . k_j) v_j          S <- d^n S + sum_j d^(n-1-j) k_j v_j^T
 // The state lives in the accumulators (transposed: value columns are matrix rows) and passes through LDS once per block for the first
 // term.  Decay powers, products with the state and the masked weights are f32 (mma_rows on an f32 side).
+// What bounds it is the chain of blocks, some 4.5 us each in a workgroup per head and slice, so where CUs are left over (lin_segments) a sequence's
+// blocks are shared out: a first launch (SUMS) leaves what each segment adds to the state, and every segment starts from the
+// sums in front of it.  2048 rows, 16 heads of 64 x 128: 143 us -> 28 + 51.
 template <typename T, int CLS>
 struct LinTile {
   static constexpr int C = sizeof(T) == 2 ? 64 : 32, PAD = 16 / sizeof(T);
@@ -486,8 +491,16 @@ struct LinTile {
   static constexpr size_t T_ELEMS = (size_t)2 * C * LD + (size_t)CLS * LC + LIN_SLICE * LC;
   static constexpr size_t F_ELEMS = (size_t)C * LP + LIN_SLICE * LS + C + LIN_POW + 7;
   static constexpr size_t LDS = T_ELEMS * sizeof(T) + F_ELEMS * sizeof(float);
+  static constexpr int STATE = CLS * LIN_SLICE;
 };
-template <typename T, int CLS>
+// Segments of a sequence of n rows: as many as fill two workgroups a CU, two blocks of `block` rows each at least
+__host__ inline int lin_segments(int n_cu, int units, int n, int block) {
+  const int fit = 2 * n_cu / units, most = (n + block - 1) / block / 2;
+  return fit < 2 || most < 2 ? 1 : fit < most ? fit : most;
+}
+// SUMS: no outputs; segment z's sums become the state in front of segment z + 1 (segment 0 starts from the slab's, which it copies for the
+// other launch: the last segment overwrites the slab)
+template <typename T, int CLS, bool SUMS>
 __global__ __launch_bounds__(256) void k_linear_rows(const MixRows<T> a) {
   typedef LinTile<T, CLS> L;
   constexpr int C = L::C, LD = L::LD, LC = L::LC, LP = L::LP, LS = L::LS, MT = C / 16, NG = 4 / MT, ND = CLS / 64;
@@ -506,8 +519,13 @@ __global__ __launch_bounds__(256) void k_linear_rows(const MixRows<T> a) {
   const int slice = blockIdx.x % g.slices, h = blockIdx.x / g.slices;
   const PassSeq sq = a.seqs[blockIdx.y];
   const int c0 = slice * LIN_SLICE;
-  float* S = (float*)(sq.slab + a.rs.s) + (size_t)h * g.D * g.V;
+  float* S = as_global((float*)(sq.slab + a.rs.s)) + (size_t)h * g.D * g.V;
   const T* base = a.proj + (size_t)sq.row0 * a.ldp;
+  const int seg = blockIdx.z, seg_blocks = ((sq.n + C - 1) / C + a.lin_segs - 1) / a.lin_segs;
+  const int first = seg * seg_blocks * C, end = min(first + seg_blocks * C, sq.n);
+  if (first >= sq.n || (SUMS && end == sq.n)) return;  // (whole workgroup)
+  const bool alone = seg == 0 && end == sq.n;          // the sequence's only segment: no other workgroup touches its state
+  float* slot = a.lin_state + ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * a.lin_segs * L::STATE + tid * 4;
   for (int i = tid; i < LIN_POW; i += 256) pow[i] = g.decay[h * LIN_POW + i];
   // state tile (value columns c0 + 16 i + 4 fk .., key column 16 (wave + 4 n) + fr)
   f32x4 s[2][ND];
@@ -516,64 +534,85 @@ __global__ __launch_bounds__(256) void k_linear_rows(const MixRows<T> a) {
 #pragma unroll
     for (int n = 0; n < ND; n++) {
       const int c = c0 + i * 16 + fk * 4, d = (wave + 4 * n) * 16 + fr;
-      s[i][n] = sq.pos0 > 0 && c < g.V && d < g.D ? *(const f32x4*)(S + (size_t)d * g.V + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+      const bool slab = (SUMS ? seg == 0 : alone) && sq.pos0 > 0;
+      s[i][n] = slab && c < g.V && d < g.D ? *(const f32x4*)(S + (size_t)d * g.V + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+      if (SUMS && seg == 0) *(f32x4*)(slot + (i * ND + n) * 1024) = s[i][n];
     }
+  if (!SUMS && !alone) {
+    float d = 1.f;
+    for (int i = 0; i < seg_blocks; i++) d *= g.decay[h * LIN_POW + C];
+    for (int z = seg ? 1 : 0; z <= seg; z++)
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int n = 0; n < ND; n++) {
+          const f32x4 u = *(const f32x4*)(slot + (size_t)z * L::STATE + (i * ND + n) * 1024);
+#pragma unroll
+          for (int e = 0; e < 4; e++) s[i][n][e] = __builtin_fmaf(s[i][n][e], d, u[e]);
+        }
+  }
   Oct<T> rq[NQ], rk[NQ], rv;
   auto request = [&](int r0) {
 #pragma unroll
     for (int u = 0; u < NQ; u++) {
       const int i = u * 256 + tid, r = r0 + i % C, c = i / C * 8;
-      const bool in = r < sq.n && c < g.D;
+      const bool in = r < end && c < g.D;
       const T* row = base + (size_t)r * a.ldp + h * g.D + c;
-      rq[u] = in ? oct_load(row + g.cq) : oct_zero<T>();
+      if constexpr (!SUMS) rq[u] = in ? oct_load(row + g.cq) : oct_zero<T>();
       rk[u] = in ? oct_load(row + g.ck) : oct_zero<T>();
     }
     const int r = r0 + tid % C, c = c0 + tid / C * 8;
-    rv = tid < C * (LIN_SLICE / 8) && r < sq.n && c < g.V ? oct_load(base + (size_t)r * a.ldp + g.cv + h * g.V + c) : oct_zero<T>();
+    rv = tid < C * (LIN_SLICE / 8) && r < end && c < g.V ? oct_load(base + (size_t)r * a.ldp + g.cv + h * g.V + c) : oct_zero<T>();
   };
-  request(0);
-  for (int r0 = 0; r0 < sq.n; r0 += C) {
-    const int n = sq.n - r0 < C ? sq.n - r0 : C;
+  request(first);
+  for (int r0 = first; r0 < end; r0 += C) {
+    const int n = end - r0 < C ? end - r0 : C;
     __syncthreads();  // the previous block's products are done with LDS (and pow is there)
 #pragma unroll
     for (int u = 0; u < NQ; u++) {
       const int i = u * 256 + tid, r = i % C, c = i / C * 8;
-      oct_store(qs + r * LD + c, rq[u]);
-      oct_store(ks + r * LD + c, rk[u]);
+      if constexpr (!SUMS) {
+        oct_store(qs + r * LD + c, rq[u]);
+        oct_store(ks + r * LD + c, rk[u]);
+      }
       oct_scatter(kt + c * LC + r, LC, rk[u]);
     }
     if (tid < C * (LIN_SLICE / 8)) oct_scatter(vt + (tid / C * 8) * LC + tid % C, LC, rv);
     if (tid < C) wj[tid] = tid < n ? pow[n - 1 - tid] : 0.f;
+    if constexpr (!SUMS) {
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+      for (int i = 0; i < 2; i++)
 #pragma unroll
-      for (int nn = 0; nn < ND; nn++)
+        for (int nn = 0; nn < ND; nn++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) st[(i * 16 + fk * 4 + e) * LS + (wave + 4 * nn) * 16 + fr] = s[i][nn][e];
-    __syncthreads();
-    if (r0 + C < sq.n) request(r0 + C);
-    const int mt = wave % MT;
-    // masked, decayed products of the block's rows
-    for (int j = wave / MT; j < MT; j += NG) {
-      f32x4 v = {0.f, 0.f, 0.f, 0.f};
-      if (j <= mt) v = mma_rows(qs + (mt * 16 + fr) * LD, ks + (j * 16 + fr) * LD, CLS, v);
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int i = mt * 16 + fk * 4 + e, d = i - (j * 16 + fr);
-        p[i * LP + j * 16 + fr] = d >= 0 ? v[e] * pow[d] : 0.f;
-      }
+          for (int e = 0; e < 4; e++) st[(i * 16 + fk * 4 + e) * LS + (wave + 4 * nn) * 16 + fr] = s[i][nn][e];
     }
     __syncthreads();
-    for (int j = wave / MT; j < 2; j += NG) {
-      f32x4 v = mma_rows(qs + (mt * 16 + fr) * LD, st + (j * 16 + fr) * LS, CLS, f32x4{0.f, 0.f, 0.f, 0.f});
+    if (r0 + C < end) request(r0 + C);
+    if constexpr (!SUMS) {
+      const int mt = wave % MT;
+      // masked, decayed products of the block's rows
+      for (int j = wave / MT; j < MT; j += NG) {
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+        if (j <= mt) v = mma_rows(qs + (mt * 16 + fr) * LD, ks + (j * 16 + fr) * LD, CLS, v);
 #pragma unroll
-      for (int e = 0; e < 4; e++) v[e] *= pow[mt * 16 + fk * 4 + e + 1];
-      v = mma_rows(p + (mt * 16 + fr) * LP, vt + (j * 16 + fr) * LC, C, v);
-      const int c = c0 + j * 16 + fr;
+        for (int e = 0; e < 4; e++) {
+          const int i = mt * 16 + fk * 4 + e, d = i - (j * 16 + fr);
+          p[i * LP + j * 16 + fr] = d >= 0 ? v[e] * pow[d] : 0.f;
+        }
+      }
+      __syncthreads();
+      for (int j = wave / MT; j < 2; j += NG) {
+        f32x4 v = mma_rows(qs + (mt * 16 + fr) * LD, st + (j * 16 + fr) * LS, CLS, f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int i = mt * 16 + fk * 4 + e;
-        if (i < n && c < g.V) a.lin[(size_t)(sq.row0 + r0 + i) * (g.H * g.V) + h * g.V + c] = v[e];
+        for (int e = 0; e < 4; e++) v[e] *= pow[mt * 16 + fk * 4 + e + 1];
+        v = mma_rows(p + (mt * 16 + fr) * LP, vt + (j * 16 + fr) * LC, C, v);
+        const int c = c0 + j * 16 + fr;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int i = mt * 16 + fk * 4 + e;
+          if (i < n && c < g.V) a.lin[(size_t)(sq.row0 + r0 + i) * (g.H * g.V) + h * g.V + c] = v[e];
+        }
       }
     }
 #pragma unroll
@@ -584,6 +623,14 @@ __global__ __launch_bounds__(256) void k_linear_rows(const MixRows<T> a) {
         s[i][nn] = mma_rows_w(vt + (i * 16 + fr) * LC, wj, kt + ((wave + 4 * nn) * 16 + fr) * LC, C, s[i][nn]);
       }
   }
+  if constexpr (SUMS) {
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int nn = 0; nn < ND; nn++) *(f32x4*)(slot + (size_t)(seg + 1) * L::STATE + (i * ND + nn) * 1024) = s[i][nn];
+    return;
+  }
+  if (end < sq.n) return;
 #pragma unroll
   for (int i = 0; i < 2; i++)
 #pragma unroll
