@@ -1,6 +1,7 @@
 // gemm_bf16.hip -- the kernel behind gemm_bf16.hpp
 #include <cmath>
 #include <cstdlib>
+#include <type_traits>
 
 #include "gemm_bf16.hpp"
 
@@ -13,9 +14,9 @@ __device__ __forceinline__ void store4(float* p, const float (&v)[4]) { *(f32x4*
 template <int BM, int BN, int WGM, int WGN, int ST, int P, int OUT, int NS>
 __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_bf16(const GemmBf16 g, int S, float* __restrict__ ws, unsigned* __restrict__ tick) {
   constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 16, TN = WN / 16;
-  constexpr int HR = BM < 64 ? BM : 64, LC = BN + 4;  // the epilogue's slab of rows in LDS
+  constexpr int HR = BM, LC = BN + 4;  // the epilogue's slab of rows in LDS
   constexpr int NT = 64 * WGM * WGN, FA = BM * 8 / NT, FB = BN * 8 / NT;  // threads; a step's requests per thread
-  static_assert(WN == 64 && HR % WM == 0 && BM * 8 % NT == 0 && BN * 8 % NT == 0, "a wave's columns are one square-sum piece; its rows lie in one slab");
+  static_assert(BM * 8 % NT == 0 && BN * 8 % NT == 0 && HR * BN / 8 % NT == 0, "whole requests, whole units of the epilogue");
   __shared__ __attribute__((aligned(16))) unsigned short lds[ST][(BM + BN) * 64];
   static_assert(sizeof(lds) >= (HR * LC + BM) * sizeof(float), "the epilogue reuses the tiles' LDS");
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_wg();
@@ -35,61 +36,72 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_bf16(const GemmBf16 g, 
     for (int j = 0; j < TN; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int steps = g.K / 64, all = steps * P;
   const int s_lo = (int)((long long)all * piece / S), s_hi = (int)((long long)all * (piece + 1) / S);
-  auto fetch = [&](int s, int buf) {
-    const int p = P == 1 ? 0 : s / steps, k0 = (P == 1 ? s : s - p * steps) * 64;
-    const unsigned short* ap = g.a + (P == 1 ? 0 : (size_t)(P - 1 - p) * g.a_plane) + k0;  // (the smallest plane first)
+  unsigned oa[FA], ob[FB];  // bytes behind the tile's first row
 #pragma unroll
-    for (int it = 0; it < FA; it++) {
-      const int slot = it * NT + tid, r = slot >> 3, c = (slot & 7) ^ ((r >> 1) & 7);
-      lds_dma16(ap + (size_t)(row0 + r) * g.K + c * 8, &lds[buf][(it * NT + wave * 64) * 8]);
-    }
-#pragma unroll
-    for (int it = 0; it < FB; it++) {
-      const int slot = it * NT + tid, r = slot >> 3, c = (slot & 7) ^ ((r >> 1) & 7);
-      lds_dma16(g.w + (size_t)(col0 + r) * g.K + k0 + c * 8, &lds[buf][BM * 64 + (it * NT + wave * 64) * 8]);
-    }
-  };
-  float factor = 1.f;  // of row tid, waiting for the epilogue
-  if (g.sq_in != nullptr && tid < BM) {
-    const float* q = g.sq_in + (size_t)(row0 + tid < g.M ? row0 + tid : g.M - 1) * g.n_sq;
-    float s = 0.f;
-#pragma unroll 8
-    for (int i = 0; i < g.n_sq; i++) s += q[i];
-    factor = (g.gain ? *g.gain : 1.0f) / sqrtf(s / (float)g.mean_n + g.eps);
+  for (int it = 0; it < FA; it++) {
+    const int slot = it * NT + tid, r = slot >> 3, c = (slot & 7) ^ ((r >> 1) & 7);
+    oa[it] = (unsigned)(r * g.K + c * 8) * 2;
   }
+#pragma unroll
+  for (int it = 0; it < FB; it++) {
+    const int slot = it * NT + tid, r = slot >> 3, c = (slot & 7) ^ ((r >> 1) & 7);
+    ob[it] = (unsigned)(r * g.K + c * 8) * 2;
+  }
+  const unsigned short *ta = g.a + (size_t)row0 * g.K, *tb = g.w + (size_t)col0 * g.K;
+  constexpr unsigned STAGE = (BM + BN) * 128;  // bytes of a step
+  const unsigned lds0 = lds_address(&lds[0][wave * 512]);
+  // step s's request i of FA + FB, to the stage at the LDS address `buf` (this wave's part)
+  auto request = [&](int s, unsigned buf, int i) {
+    const int p = P == 1 ? 0 : s / steps, k0 = (P == 1 ? s : s - p * steps) * 64;
+    if (i < FA)  // (the smallest plane first)
+      lds_dma16(ta + (P == 1 ? 0 : (size_t)(P - 1 - p) * g.a_plane) + k0, oa[i < FA ? i : 0], buf + i * NT * 16);
+    else
+      lds_dma16(tb + k0, ob[i < FA ? 0 : i - FA], buf + i * NT * 16);
+  };
   const int fr = lane & 15, fk = lane >> 4;
 #pragma unroll
   for (int i = 0; i < ST - 1; i++)
-    if (s_lo + i < s_hi) fetch(s_lo + i, i);
-  int buf = 0;
-  for (int s = s_lo; s < s_hi; s++) {
-    // step s has landed -- this wave's part (later steps' requests stay out), then everybody's -- and step s - 1 has been read by all
+    if (s_lo + i < s_hi) {
+#pragma unroll
+      for (int d = 0; d < FA + FB; d++) request(s_lo + i, lds0 + i * STAGE, d);
+    }
+  float factor = 1.f;  // of row tid, for the epilogue
+  if (g.sq_in != nullptr && tid < BM) {  // (behind the first requests: their latency covers it)
+    const float* q = g.sq_in + (size_t)(row0 + tid < g.M ? row0 + tid : g.M - 1) * g.n_sq;
+    float s = 0.f;
+    if (g.n_sq % 4 == 0) {
+#pragma unroll 8
+      for (int i = 0; i < g.n_sq; i += 4) {
+        const f32x4 v = *(const f32x4*)(q + i);
+#pragma unroll
+        for (int e = 0; e < 4; e++) s += v[e];
+      }
+    } else {
+#pragma unroll 16
+      for (int i = 0; i < g.n_sq; i++) s += q[i];
+    }
+    factor = (g.gain ? *g.gain : 1.0f) / sqrtf(s / (float)g.mean_n + g.eps);
+  }
+  int buf = 0;  // the stage that step s is in
+  auto step = [&](auto Mc, int s) {
+    const unsigned into = lds0 + (buf == 0 ? ST - 1 : buf - 1) * STAGE;
+    tile_step<bf16x8, TM, TN, decltype(Mc)::value ? FA + FB : 0>(
+        &lds[buf][0], wm * WM, &lds[buf][BM * 64], wn * WN, [&](int i, int j, bf16x8 x, bf16x8 y) { acc[i][j] = mfma_bf16(x, y, acc[i][j]); },
+        [&](int d) { request(s + ST - 1, into, d); });
+    buf = buf + 1 == ST ? 0 : buf + 1;
+  };
+  // In front of step s: it has landed -- this wave's part (later steps' requests stay out), then everybody's -- and step s - 1 has been read by all
+  int s = s_lo;
+  for (; s + ST - 1 < s_hi; s++) {
+    landed_barrier<(ST - 2) * (FA + FB)>();
+    step(std::true_type{}, s);
+  }
+  for (; s < s_hi; s++) {
     if (s + ST - 2 < s_hi)
       landed_barrier<(ST - 2) * (FA + FB)>();
     else
       landed_barrier<0>();
-    if (s + ST - 1 < s_hi) fetch(s + ST - 1, buf == 0 ? ST - 1 : buf - 1);
-    const unsigned short* la = &lds[buf][0];
-    const unsigned short* lb = la + BM * 64;
-#pragma unroll
-    for (int kk = 0; kk < 2; kk++) {
-      bf16x8 fa[TM], fb[TN];
-#pragma unroll
-      for (int i = 0; i < TM; i++) {
-        const int r = wm * WM + i * 16 + fr;
-        fa[i] = *(const bf16x8*)(la + r * 64 + (((kk * 4 + fk) ^ ((r >> 1) & 7)) * 8));
-      }
-#pragma unroll
-      for (int j = 0; j < TN; j++) {
-        const int r = wn * WN + j * 16 + fr;
-        fb[j] = *(const bf16x8*)(lb + r * 64 + (((kk * 4 + fk) ^ ((r >> 1) & 7)) * 8));
-      }
-#pragma unroll
-      for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = mfma_bf16(fa[i], fb[j], acc[i][j]);
-    }
-    buf = buf + 1 == ST ? 0 : buf + 1;
+    step(std::false_type{}, s);
   }
   if (S > 1 && !add_pieces<TM * TN, NT>((f32x4*)acc, S, piece, tile, ws, tick)) return;
   // epilogue: the tile goes through LDS in slabs of HR rows, so that a thread has eight neighbouring columns of a row
@@ -341,14 +353,14 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_bf16(const GemmBf16 g, 
   }
 }
 
-// Tile and k pieces.  A CU's time for a step of 64 (tile by tile, one workgroup after the other or side by side) and a workgroup's own
+// Tile and k pieces.  (128 rows: eight waves, two a SIMD -- 2048 x 2048 x 4096 61 -> 46 us against four.)  A CU's time for a step of 64 (tile by tile, one workgroup after the other or side by side) and a workgroup's own
 // chain of steps are what was measured; a cut of k costs the hand-over of the pieces.
 struct TileCost {
   int bm, resident;     // workgroups of this tile a CU holds
   double step, chain;   // us per step of 64: a workgroup's share of a busy CU; the latency of one alone
 };
 GemmPlan gemm_plan(int M, int col_tiles, int steps, int n_cu, size_t ws_floats) {
-  static const TileCost costs[] = {{256, 1, 1.03, 1.03}, {128, 1, 0.68, 0.68}, {64, 2, 0.42, 0.51}, {32, 2, 0.41, 0.41}};
+  static const TileCost costs[] = {{256, 1, 1.03, 1.03}, {128, 1, 0.58, 0.58}, {64, 2, 0.42, 0.51}, {32, 2, 0.41, 0.41}};
   GemmPlan best{128, 1};
   double best_cost = 1e30;
   for (const TileCost& t : costs) {
@@ -384,7 +396,7 @@ static void launch_t(hipStream_t st, crabml_hip_device::ProfRec* rec, const Gemm
   if (p.bm == 256)
     launch_k(st, rec, k_gemm_bf16<256, 128, 4, 2, 3, P, OUT, NS>, grid, dim3(512), 0, g, p.S, w.partials, w.ticks);
   else if (p.bm == 128)
-    launch_k(st, rec, k_gemm_bf16<128, 128, 2, 2, 4, P, OUT, NS>, grid, dim3(256), 0, g, p.S, w.partials, w.ticks);
+    launch_k(st, rec, k_gemm_bf16<128, 128, 4, 2, 4, P, OUT, NS>, grid, dim3(512), 0, g, p.S, w.partials, w.ticks);
   else if (p.bm == 64)
     launch_k(st, rec, k_gemm_bf16<64, 128, 2, 2, 3, P, OUT, NS>, grid, dim3(256), 0, g, p.S, w.partials, w.ticks);
   else

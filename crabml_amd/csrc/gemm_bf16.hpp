@@ -82,17 +82,54 @@ __device__ __forceinline__ void read8(const float* p, float (&o)[8]) {
   }
 }
 
-// 16 bytes per lane from memory into LDS at l + 16 lane (l: wave-uniform).  As assembly, because the compiler would wait for ALL of them
+__device__ __forceinline__ unsigned lds_address(const void* l) {
+  return (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(size_t)(const __attribute__((address_space(3))) void*)l);
+}
+// 16 bytes per lane from memory into LDS at the address `at` + 16 lane (wave-uniform).  As assembly, because the compiler would wait for ALL of them
 // in front of the next LDS read (it cannot tell the buffers apart); who waits for what is landed_barrier's business.
 // (m0, the LDS address of such a load, needs one wait state behind its write; nothing else here uses it.)
-__device__ __forceinline__ void lds_dma16(const void* g, const void* l) {
-  const unsigned at = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(size_t)(const __attribute__((address_space(3))) void*)l);
+__device__ __forceinline__ void lds_dma16(const void* g, unsigned at) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(at) : "memory");
+}
+// the same from `off` bytes behind a wave-uniform base
+__device__ __forceinline__ void lds_dma16(const void* base, unsigned off, unsigned at) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(at) : "memory");
 }
 // waits until at most N of this wave's memory requests are outstanding, then for the workgroup.  (__syncthreads would drain them all.)
 template <int N>
 __device__ __forceinline__ void landed_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+// One step of 64: TM x TN fragments of products of rows ra + 16 i of the stage at `la` and rows rb + 16 j of the one at `lb`.  LDS rows are 64
+// elements, their 16-byte pieces permuted by (row / 2) % 8.  request(d), d < NREQ, asks for a part of a later step: requests are spread over the
+// products, because 48 KB a step are 768 cycles of the CU's address path, and issued in a row behind the barrier they left the matrix
+// cores idle for 550 of a step's 2150 cycles (256 x 128 tile, 2048 x 11264 x 2048: 138 -> 115 us).
+template <typename V, int TM, int TN, int NREQ, typename Mul, typename Req>
+__device__ __forceinline__ void tile_step(const unsigned short* la, int ra, const unsigned short* lb, int rb, Mul mul, Req request) {
+  constexpr int GR = 2 * TM, SL = TM > 1 ? TM - 1 : 1;
+  const int fr = threadIdx.x & 15, fk = threadIdx.x >> 4 & 3;
+  V f[2][TN + TM];  // columns, rows
+  auto read = [&](int kk, int i) {
+    const int r = i < TN ? rb + i * 16 + fr : ra + (i - TN) * 16 + fr;
+    f[kk][i] = *(const V*)((i < TN ? lb : la) + r * 64 + (((kk * 4 + fk) ^ ((r >> 1) & 7)) * 8));
+  };
+#pragma unroll
+  for (int i = 0; i < TN + TM; i++) read(0, i);
+#pragma unroll
+  for (int q = 0; q < GR; q++) {
+    const int kk = q / TM, i = q % TM;
+#pragma unroll
+    for (int j = 0; j < TN; j++) mul(i, j, f[kk][TN + i], f[kk][j]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (q < SL) {  // the second half's fragments, behind all but the last group of the first
+#pragma unroll
+      for (int d = (TN + TM) * q / SL; d < (TN + TM) * (q + 1) / SL; d++) read(1, d);
+    }
+#pragma unroll
+    for (int d = NREQ * q / GR; d < NREQ * (q + 1) / GR; d++) request(d);
+    __builtin_amdgcn_sched_barrier(0);
+  }
 }
 
 // S > 1: k is cut into S pieces, one workgroup each.  A workgroup leaves its accumulators (F fragments a thread, NT threads) in ws

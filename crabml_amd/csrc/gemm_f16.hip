@@ -8,8 +8,10 @@
 // again (its results are not stored), a 16-byte piece past the end of k is a piece of zeros.  Weights are the first operand, so that a
 // lane's four results are neighbouring columns of one row and leave as one 16-byte store, without a way through LDS.
 //
-// Measured (203 rows, width 2048, ff 8192, one layer): q | k | v 16.6 us, wo 16.0, gate | up 31.8, ff_down 28.5 (430 TFLOP/s in the
-// gate | up launch); before, a launch of the row kernel per row and matrix: 21.3 ms a layer.
+// Measured (203 rows, width 2048, ff 8192, one layer): q | k | v 15.5 us, wo 15.0, gate | up 27.5, ff_down 28.8 (500 TFLOP/s in the
+// gate | up launch); 17.8, 17.2, 33.6, 28.5 with a step's requests in a row behind its barrier and four waves on a 128-row tile.
+#include <type_traits>
+
 #include "gemm_bf16.hpp"
 
 namespace crabml_hip {
@@ -57,46 +59,40 @@ __global__ __launch_bounds__(64 * WGM * WGN) void k_gemm_f16(const GemmF16 g, in
     for (int j = 0; j < TN; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int steps = (g.K + 63) / 64;
   const int s_lo = (int)((long long)steps * piece / S), s_hi = (int)((long long)steps * (piece + 1) / S);
-  auto fetch = [&](int s, int buf) {
+  constexpr unsigned STAGE = (BM + BN) * 128;  // bytes of a step
+  const unsigned lds0 = lds_address(&lds[0][wave * 512]);
+  auto request = [&](int s, unsigned into, int i) {  // step s's request i of FA + FB
     const int k0 = s * 64;
     const bool in = k0 + c8 < g.K;  // (K is a multiple of 8)
-#pragma unroll
-    for (int it = 0; it < FA; it++) lds_dma16(in ? pa[it] + k0 : g_zero_piece, &lds[buf][(it * NT + wave * 64) * 8]);
-#pragma unroll
-    for (int it = 0; it < FB; it++) lds_dma16(in ? pb[it] + k0 : g_zero_piece, &lds[buf][BM * 64 + (it * NT + wave * 64) * 8]);
+    lds_dma16(in ? (i < FA ? pa[i < FA ? i : 0] : pb[i < FA ? 0 : i - FA]) + k0 : g_zero_piece, into + i * NT * 16);
   };
   const int fr = lane & 15, fk = lane >> 4;
 #pragma unroll
   for (int i = 0; i < ST - 1; i++)
-    if (s_lo + i < s_hi) fetch(s_lo + i, i);
-  int buf = 0;
-  for (int s = s_lo; s < s_hi; s++) {
+    if (s_lo + i < s_hi) {
+#pragma unroll
+      for (int d = 0; d < FA + FB; d++) request(s_lo + i, lds0 + i * STAGE, d);
+    }
+  int buf = 0;  // the stage that step s is in
+  auto step = [&](auto Mc, int s) {
+    const unsigned into = lds0 + (buf == 0 ? ST - 1 : buf - 1) * STAGE;
+    tile_step<f16x8, TM, TN, decltype(Mc)::value ? FA + FB : 0>(
+        &lds[buf][0], wm * WM, &lds[buf][BM * 64], wn * WN,
+        [&](int i, int j, f16x8 x, f16x8 y) { acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(y, x, acc[i][j], 0, 0, 0); },
+        [&](int d) { request(s + ST - 1, into, d); });
+    buf = buf + 1 == ST ? 0 : buf + 1;
+  };
+  int s = s_lo;
+  for (; s + ST - 1 < s_hi; s++) {
+    landed_barrier<(ST - 2) * (FA + FB)>();
+    step(std::true_type{}, s);
+  }
+  for (; s < s_hi; s++) {
     if (s + ST - 2 < s_hi)
       landed_barrier<(ST - 2) * (FA + FB)>();
     else
       landed_barrier<0>();
-    if (s + ST - 1 < s_hi) fetch(s + ST - 1, buf == 0 ? ST - 1 : buf - 1);
-    const unsigned short* la = &lds[buf][0];
-    const unsigned short* lb = la + BM * 64;
-#pragma unroll
-    for (int kk = 0; kk < 2; kk++) {
-      f16x8 fa[TM], fb[TN];
-#pragma unroll
-      for (int i = 0; i < TM; i++) {
-        const int r = wm * WM + i * 16 + fr;
-        fa[i] = *(const f16x8*)(la + r * 64 + (((kk * 4 + fk) ^ ((r >> 1) & 7)) * 8));
-      }
-#pragma unroll
-      for (int j = 0; j < TN; j++) {
-        const int r = wn * WN + j * 16 + fr;
-        fb[j] = *(const f16x8*)(lb + r * 64 + (((kk * 4 + fk) ^ ((r >> 1) & 7)) * 8));
-      }
-#pragma unroll
-      for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[j], fa[i], acc[i][j], 0, 0, 0);
-    }
-    buf = buf + 1 == ST ? 0 : buf + 1;
+    step(std::false_type{}, s);
   }
   if (S > 1 && !add_pieces<TM * TN, NT>((f32x4*)acc, S, piece, tile, ws, tick)) return;
 #pragma unroll
@@ -144,7 +140,7 @@ bool launch_gemm_f16(crabml_hip_device* dev, crabml_hip_device::ProfRec* rec, co
   if (p.bm == 256)
     launch_k(st, rec, k_gemm_f16<256, 128, 4, 2, 3>, grid, dim3(512), 0, g, p.S, ws.partials, ws.ticks);
   else if (p.bm == 128)
-    launch_k(st, rec, k_gemm_f16<128, 128, 2, 2, 4>, grid, dim3(256), 0, g, p.S, ws.partials, ws.ticks);
+    launch_k(st, rec, k_gemm_f16<128, 128, 4, 2, 4>, grid, dim3(512), 0, g, p.S, ws.partials, ws.ticks);
   else if (p.bm == 64)
     launch_k(st, rec, k_gemm_f16<64, 128, 2, 2, 3>, grid, dim3(256), 0, g, p.S, ws.partials, ws.ticks);
   else
