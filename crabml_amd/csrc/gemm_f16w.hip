@@ -165,7 +165,7 @@ __device__ __forceinline__ f16x8 unpack_q6_k_f16(unsigned w, unsigned hw, f16x2 
 
 enum { WF_Q4_0 = 0, WF_Q8_0 = 1, WF_Q4_K = 2, WF_Q6_K = 3, WF_Q4_1 = 4 };  // the weight format of a GEMM
 
-template <int T_>
+template <int T_, int NW = 4>
 struct GemmF16Geo {
   static constexpr int T = T_, CW = 16 * T;    // column tiles per wave / prompt rows per workgroup
   static constexpr int KCH = 4;                // blocks per chunk
@@ -176,7 +176,7 @@ struct GemmF16Geo {
   static constexpr int CSTR = 80, GSTR = CW * CSTR;
   static_assert(GSTR % 256 == 0, "block planes must be whole bank rows apart");
   static constexpr int BUF = KCH * GSTR, LDS_BYTES = 2 * BUF;
-  static constexpr int B_LOADS = CW * KCH * 4 / 256;  // 16-byte pieces per thread and chunk (T)
+  static constexpr int B_LOADS = CW * KCH * 4 / (64 * NW);  // 16-byte pieces per thread and chunk
 };
 
 // Up to three weight matrices against the same rhs in ONE launch (wq | wk | wv: the 1024-row k / v GEMMs alone leave most of the
@@ -200,14 +200,14 @@ __device__ __forceinline__ float f16w_silu_mul(float g, float u, const unsigned 
   return (g / (1.0f + nexp)) * u;
 }
 // GU (F = 2, two matrices of the same shape: ffn_gate and ffn_up): fragment 0 holds 16 rows of the FIRST matrix, fragment 1 the same
-// 16 rows of the SECOND -- the workgroup owns 64 rows of both -- and the epilogue stores h = silu(g) * u (out[0]) instead of g and u:
+// 16 rows of the SECOND -- the workgroup owns 16 NW rows of both -- and the epilogue stores h = silu(g) * u (out[0]) instead of g and u:
 // the (rows, hidden) f32 pair never makes its trip through memory (llama2.rs:620-630).  One k piece only (silu is not linear).
-template <int WF, int F, int T_, bool GU = false>  // F 16-row fragments x T_ 16-column tiles per wave: the workgroup's four waves own 64 F consecutive weight rows
+template <int WF, int F, int T_, bool GU = false, int NW = 4>  // F 16-row fragments x T_ 16-column tiles per wave: the workgroup's NW waves own 16 NW F consecutive weight rows
 // ksplit > 1: that many workgroups per output tile, each over its piece of k, each writing its own partial buffer -- ffn_down and wo
 // have few row tiles and a long serial k loop (one wave per SIMD otherwise), and a short pass has few tiles altogether
-__global__ __launch_bounds__(256, 2) void k_gemm_f16w(F16wMats mats, const i32x4* __restrict__ xh, int nb, int n, int row_tiles, int ksplit) {
-  using G = GemmF16Geo<T_>;
-  constexpr int T = G::T, KCH = G::KCH;
+__global__ __launch_bounds__(64 * NW, 2) void k_gemm_f16w(F16wMats mats, const i32x4* __restrict__ xh, int nb, int n, int row_tiles, int ksplit) {
+  using G = GemmF16Geo<T_, NW>;
+  constexpr int T = G::T, KCH = G::KCH, NT = 64 * NW;
   extern __shared__ __attribute__((aligned(16))) unsigned char f16w_lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_wg();
   const int i = lane & 15, g = lane >> 4;
@@ -244,7 +244,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16w(F16wMats mats, const i32x4
   const int m = ti == 0 ? mats.m[0] : ti == 1 ? mats.m[1] : mats.m[2];
   const int rt_l = rt - (ti == 0 ? 0 : ti == 1 ? mats.tiles_end[0] : mats.tiles_end[1]);
   constexpr int FSTEP = GU ? 0 : 16;  // rows between a wave's fragments
-  const int r0 = GU ? rt_l * 64 + wave * 16 : rt_l * 64 * F + wave * 16 * F, c0 = ct * G::CW;
+  const int r0 = (rt_l * NW + wave) * (GU ? 16 : 16 * F), c0 = ct * G::CW;
   // this workgroup's chunks: [ch_lo, ch_lo + nchunks) of the row's ceil(nb / KCH)
   // (Q4_K: an even chunk is half 0 of its super-block -- the pieces start on super-block boundaries)
   const int all_chunks = (nb + KCH - 1) / KCH;
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16w(F16wMats mats, const i32x4
   // multiplied; B' (L2-resident) two chunks ahead in two register sets.  All ring indices are compile-time (chunk loop unrolled by 4).
   constexpr int NQ = (WF == WF_Q8_0 || WF == WF_Q6_K) ? 2 : 1;  // 16-byte quant loads per fragment and chunk
   i32x4 aq[4][NQ * F];
-  unsigned ad[4][F];   // Q4_0 / Q8_0: the block's scale; Q4_1: d | m << 16
+  unsigned ad[4][F];   // Q4_0 / Q8_0: the block's scale; Q4_1: d | m << 16 (of the last block, past the row's end)
   i32x4 hq[2][F];      // Q4_K: the super-block header of ring slots (0, 1) / (2, 3), fetched with the even slot; Q6_K: the 16 scales
   unsigned hd[2][F];   // Q6_K: d
   auto fetch_a = [&](auto Jc, int ch) {
@@ -297,18 +297,16 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16w(F16wMats mats, const i32x4
         const size_t blk = (size_t)(row < m ? row : m - 1) * nb + gkb;
 #pragma unroll
         for (int u = 0; u < NQ; u++) aq[J][NQ * f + u] = __builtin_nontemporal_load(wq + blk * NQ + u);
-        unsigned dv;
         if constexpr (WF == WF_Q4_1)
-          dv = __builtin_nontemporal_load((const unsigned*)wsc + blk);
+          ad[J][f] = __builtin_nontemporal_load((const unsigned*)wsc + blk);
         else
-          dv = __builtin_nontemporal_load(wd + blk);
-        ad[J][f] = kb < nb ? dv : 0u;  // past the row's end: scale 0 (and m 0), the slots add nothing
+          ad[J][f] = __builtin_nontemporal_load(wd + blk);
       }
     }
   };
-  // B': 128 columns x 256 bytes per chunk, 8 pieces per thread (piece p: column p / 16, 16 bytes p % 16 of the chunk): ONE 32-bit
+  // B': 128 columns x 256 bytes per chunk, 32 / NW pieces per thread (piece p: column p / 16, 16 bytes p % 16 of the chunk): ONE 32-bit
   // byte offset per thread, advanced by a chunk = 256 bytes per fetch (the fetches come in chunk order), against a scalar base per
-  // piece -- 16 columns further each (global_load ... s[base], v offset: no per-piece pointer registers).  Columns past n (a ragged
+  // piece -- NT / 16 columns further each (global_load ... s[base], v offset: no per-piece pointer registers).  Columns past n (a ragged
   // last tile) and the look-ahead of the last iterations read whatever follows in xh -- launch_gemm_f16w's contract keeps that
   // inside the allocation; finite or not, it meets only output columns that are never stored, zero weights, or is never consumed.
   // register sets of B' pieces in flight (one wave per SIMD: the longer look-ahead; the 32-byte-per-lane formats with two fragments:
@@ -316,7 +314,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16w(F16wMats mats, const i32x4
   constexpr int NBD = (F == 1 && WF == WF_Q4_0) ? 4 : (F == 2 && (WF == WF_Q8_0 || WF == WF_Q6_K)) ? 1 : 2;
   i32x4 rb[NBD][G::B_LOADS];
   const char* xbase = (const char*)xh + ((size_t)c0 * nb + (size_t)ch_lo * KCH) * 64;  // (uniform)
-  const unsigned xstep = 16u * (unsigned)nb * 64u;                                        // 16 columns
+  const unsigned xstep = (unsigned)(NT / 16) * (unsigned)nb * 64u;
   unsigned xoff = (unsigned)(tid >> 4) * (unsigned)nb * 64u + (unsigned)(tid & 15) * 16u;
   auto fetch_b = [&](i32x4 (&r)[G::B_LOADS], int ch) {
     (void)ch;
@@ -328,7 +326,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16w(F16wMats mats, const i32x4
     unsigned char* S = f16w_lds + buf * G::BUF;
 #pragma unroll
     for (int u = 0; u < G::B_LOADS; u++) {
-      const int p = tid + 256 * u, col = p >> 4, pc = p & 15;
+      const int p = tid + NT * u, col = p >> 4, pc = p & 15;
       *(i32x4*)(S + (pc >> 2) * G::GSTR + col * G::CSTR + (pc & 3) * 16) = r[u];
     }
   };
@@ -357,6 +355,10 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16w(F16wMats mats, const i32x4
     fetch_a(std::integral_constant<int, (J + 3) & 3>{}, ch + 3);
     const unsigned char* S = f16w_lds + (J & 1) * G::BUF + g * G::GSTR + i * G::CSTR;
     f16x2 d2[F];
+    // past the row's end: scale 0 (and m 0), the slots add nothing.  (Said here and not where the scale is requested: a choice there waits for it,
+    // a memory round trip a chunk -- 1400 of 4500 cycles.  512 rows, Q4_0: wo and ffn_down 79 -> 73 us on average,
+    // q | k | v 64 -> 60.)
+    const unsigned there = (ch_lo + ch) * KCH + g < nb ? ~0u : 0u;
 #pragma unroll
     for (int f = 0; f < F; f++) {
       if constexpr (WF == WF_Q4_K) {
@@ -376,11 +378,12 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16w(F16wMats mats, const i32x4
           cs[f].o_hi = f16x2{c[3], c[3]};
         }
       } else if constexpr (WF == WF_Q4_1) {
-        const unsigned dm = ad[J][f];
+        const unsigned dm = ad[J][f] & there;
         cs[f].c_lo = cs[f].c_hi = __builtin_bit_cast(f16x2, (dm & 0xffffu) | (dm << 16));
         cs[f].o_lo = cs[f].o_hi = __builtin_bit_cast(f16x2, (dm >> 16) | (dm & 0xffff0000u));
       } else {
-        d2[f] = __builtin_bit_cast(f16x2, ad[J][f] | (ad[J][f] << 16));
+        const unsigned d = ad[J][f] & there;
+        d2[f] = __builtin_bit_cast(f16x2, d | (d << 16));
       }
     }
     // B' fragments in groups of TG tiles, two groups in registers: group q + 1 is read from LDS while group q is multiplied (left
@@ -430,11 +433,12 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16w(F16wMats mats, const i32x4
   // D: lane (i, g) holds rows 4 g .. 4 g + 3 of column i of every tile
   if constexpr (GU) {
     if (mats.hq.planes != nullptr) {
-      // h = silu(g) * u of the workgroup's 64 rows x CW columns through LDS (the B' buffers are done), then ONE THREAD per
+      // h = silu(g) * u of the workgroup's 16 NW rows x CW columns through LDS (the B' buffers are done), then ONE THREAD per
       // (column, 32-row block) runs the row quantizer on it (quant_lane32's arithmetic, buf_q8_0.rs:87-134 / buf_q8_1.rs:90-129: the
       // block maximum and the integer sum do not depend on the order) and writes the block's quants, scale, sum and -- in the slot
       // order of ffn_down's GEMM -- its 32 pre-scaled halfs: h never exists as f32 in memory
-      constexpr int CS = 68;  // floats per column (64 rows + 4: 16-byte aligned columns, four banks apart)
+      constexpr int CS = 16 * NW + 4, HB = NW / 2;  // floats per column (16-byte aligned columns, four banks apart), blocks
+      static_assert((size_t)G::CW * CS * sizeof(float) <= (size_t)G::LDS_BYTES, "h fits where B' was");
       float* H = (float*)f16w_lds;
       __syncthreads();
 #pragma unroll
@@ -447,12 +451,12 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16w(F16wMats mats, const i32x4
       __syncthreads();
       const F16wHQuant& hq = mats.hq;
       const int nbh = m / 32;
-      for (int b = tid; b < G::CW * 2; b += 256) {
-        const int col = c0 + (b >> 1), hb = rt_l * 2 + (b & 1);
+      for (int b = tid; b < G::CW * HB; b += NT) {
+        const int col = c0 + b / HB, hb = rt_l * HB + b % HB;
         if (col >= n || hb >= nbh) continue;
         f32x4 v[8];
 #pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = *(const f32x4*)(H + (b >> 1) * CS + 32 * (b & 1) + 4 * j);
+        for (int j = 0; j < 8; j++) v[j] = *(const f32x4*)(H + (b / HB) * CS + 32 * (b % HB) + 4 * j);
         float amax = 0.0f;
 #pragma unroll
         for (int j = 0; j < 8; j++)
@@ -553,15 +557,15 @@ static bool f16w_raise_lds(const crabml_hip_device* dev, const void* fn, int byt
 }
 // xh: the rows' pre-scaled f16 planes (launch_rows_to_f16) inside an allocation of gemm_f16w_xh_bytes(b, k): the kernel reads whole
 // 128-column tiles and up to three chunks past the last column's end; returns false when the shape is not covered
-template <int WF, int F, int T, bool GU = false>
+template <int WF, int F, int T, bool GU = false, int NW = 4>
 static bool launch_f16w_t(crabml_hip_device* dev, const F16wMats& mats, int row_tiles, size_t k, const void* xh, size_t b, int ksplit) {
-  using G = GemmF16Geo<T>;
-  if (!f16w_raise_lds(dev, (const void*)k_gemm_f16w<WF, F, T, GU>, G::LDS_BYTES)) {  // (80 KB of dynamic LDS: raised once per device)
+  using G = GemmF16Geo<T, NW>;
+  if (!f16w_raise_lds(dev, (const void*)k_gemm_f16w<WF, F, T, GU, NW>, G::LDS_BYTES)) {  // (80 KB of dynamic LDS: raised once per device)
     (void)hipGetLastError();
     return false;
   }
   const int col_tiles = (int)((b + G::CW - 1) / G::CW);
-  k_gemm_f16w<WF, F, T, GU><<<dim3(row_tiles * col_tiles * ksplit), 256, G::LDS_BYTES, dev->stream>>>(mats, (const i32x4*)xh, (int)(k / 32), (int)b,
+  k_gemm_f16w<WF, F, T, GU, NW><<<dim3(row_tiles * col_tiles * ksplit), 64 * NW, G::LDS_BYTES, dev->stream>>>(mats, (const i32x4*)xh, (int)(k / 32), (int)b,
                                                                                           row_tiles, ksplit);
   return true;
 }
@@ -582,7 +586,7 @@ static bool launch_f16w_fmt(crabml_hip_device* dev, const F16wMats& mats, int ro
     switch (T) {
       case 2: return launch_f16w_t<WF, 2, 2, true>(dev, mats, row_tiles, k, xh, b, 1);
       case 4: return launch_f16w_t<WF, 2, 4, true>(dev, mats, row_tiles, k, xh, b, 1);
-      default: return launch_f16w_t<WF, 2, 8, true>(dev, mats, row_tiles, k, xh, b, 1);
+      default: return launch_f16w_t<WF, 2, 8, true, 8>(dev, mats, row_tiles, k, xh, b, 1);
     }
   }
   switch (T) {
@@ -631,6 +635,11 @@ bool launch_gemm_f16w(crabml_hip_device* dev, const crabml_hip_buf* const* w, co
   const bool gu = gu_exp_tab != nullptr && gu_done != nullptr && nw == 2 && m[0] == m[1] && !(variant & 64) &&
                   ((m[0] + 63) / 64) * col128 * 2 >= (size_t)dev->n_cu * 3;
   if (gu) F = 2;
+  // gate | up in full tiles: eight waves share a B' tile, which halves what the launch reads of B' (every row tile reads all of it, a
+  // gigabyte for 512 rows of 4096) and the staging a wave does.  512 rows, Q4_0 183 -> 173 us, the whole request 3973 -> 3785; Q4_K, 1024 rows a
+  // pass, 0.6 % of the request.  The other launches, cut in k to fill the chip with the smaller tiles, do not gain (ffn_down 115 -> 108,
+  // wo 35 -> 44); four fragments a wave, one wave a SIMD, lose (183 -> 211).
+  const int NW = gu && T == 8 ? 8 : 4;
   F16wMats mats{};
   mats.exp_tab = gu_exp_tab;
   const bool hquant = gu && hq != nullptr && hq->planes != nullptr && m[0] % 32 == 0;
@@ -654,7 +663,7 @@ bool launch_gemm_f16w(crabml_hip_device* dev, const crabml_hip_buf* const* w, co
       if (!gu) row_tiles += (int)((m[j] + 64 * F - 1) / (64 * F));
       before += b * m[j];
     }
-    if (gu) row_tiles = (int)((m[0] + 63) / 64);
+    if (gu) row_tiles = (int)((m[0] + 16 * NW - 1) / (16 * NW));
     mats.tiles_end[j] = row_tiles;
     parts.end4[j] = before / 4;
   }
