@@ -7,6 +7,8 @@
 // of steps go out before the activations are staged (the first block) or while the previous block is multiplied.  One pass over the
 // weights serves NB rhs rows; more rows are further grid rows (blockIdx.y) that hit the same weights in L2 / Infinity Cache.
 #pragma once
+#include <type_traits>
+
 #include "devutil.hpp"
 #include "kernels.hpp"
 
@@ -206,7 +208,8 @@ __device__ __forceinline__ void rows16_out(const GemvBf16& a, int row, int b, fl
 
 #define GEMV_BF16_LDS_FLOATS 8192  // rhs elements staged at a time, all rows together: a cut segment is a multiple of the steps in flight
 
-template <int NB, int R, int IN, int OUT, bool NT>  // NT: weights nontemporal (GemvBf16::resident)
+// UN: steps of 512 in flight; NT: weights nontemporal (GemvBf16::resident)
+template <int NB, int R, int UN, int IN, int OUT, bool NT>
 __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
   extern __shared__ __attribute__((aligned(16))) float gemv_lds[];  // [NB][2][seg / 2]
   __shared__ float red[4][NB];
@@ -214,7 +217,6 @@ __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
   const int row0 = (blockIdx.x * 4 + wave) * R, b0 = blockIdx.y * NB;
   const int seg = a.K < GEMV_BF16_LDS_FLOATS / NB ? a.K : GEMV_BF16_LDS_FLOATS / NB;  // elements per staged segment (512-multiple if cut)
   const int half = seg / 2;                                                           // floats per half-octet plane
-  constexpr int UN = R >= 4 || NB >= 8 ? 2 : 4;  // steps of 512 in flight
   const unsigned short* wr[R];
 #pragma unroll
   for (int r = 0; r < R; r++) {
@@ -222,16 +224,14 @@ __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
     wr[r] = a.w + (size_t)row * a.ldw;
   }
   i32x4 wv[UN][R];
-  auto request = [&](int k0) {
+  auto request = [&](int u, int k0) {
+    int k = k0 + u * 512 + lane * 8;
+    k = k < a.K ? k : 0;  // (a lane past the end requests the row's start and never uses it)
 #pragma unroll
-    for (int u = 0; u < UN; u++) {
-      int k = k0 + u * 512 + lane * 8;
-      k = k < a.K ? k : 0;  // (a lane past the end requests the row's start and never uses it)
-#pragma unroll
-      for (int r = 0; r < R; r++) wv[u][r] = ld<NT>((const i32x4*)(wr[r] + k));
-    }
+    for (int r = 0; r < R; r++) wv[u][r] = ld<NT>((const i32x4*)(wr[r] + k));
   };
-  request(0);
+#pragma unroll
+  for (int u = 0; u < UN; u++) request(u, 0);
   StreamElem elem;  // of lane r NB + b
   const int my_row = row0 + lane / NB, my_b = b0 + lane % NB;
   const bool mine = OUT == GEMV_OUT_STREAMS && lane < R * NB && my_row < a.N && my_b < a.nb;
@@ -298,13 +298,8 @@ __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
       }
     }
     __syncthreads();
-    for (int k0 = 0; k0 < n; k0 += UN * 512) {
-      i32x4 cur[UN][R];
-#pragma unroll
-      for (int u = 0; u < UN; u++)
-#pragma unroll
-        for (int r = 0; r < R; r++) cur[u][r] = wv[u][r];
-      if (s0 + k0 + UN * 512 < a.K) request(s0 + k0 + UN * 512);  // (also across a segment's end: seg % (UN * 512) == 0 then)
+    // UN steps; MORE: a step's registers take the one UN steps further as soon as it has been used.  (A check a step would end the loads in flight.)
+    auto steps = [&](auto Mc, int k0) {
 #pragma unroll
       for (int u = 0; u < UN; u++) {
         const int k = k0 + u * 512 + lane * 8;
@@ -318,7 +313,7 @@ __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
               float s = acc[r][b];
 #pragma unroll
               for (int e = 0; e < 2; e++) {
-                const unsigned p = (unsigned)cur[u][r][e], p2 = (unsigned)cur[u][r][e + 2];
+                const unsigned p = (unsigned)wv[u][r][e], p2 = (unsigned)wv[u][r][e + 2];
                 s = __builtin_fmaf(__builtin_bit_cast(float, p << 16), x0[2 * e], s);
                 s = __builtin_fmaf(__builtin_bit_cast(float, p & 0xffff0000u), x0[2 * e + 1], s);
                 s = __builtin_fmaf(__builtin_bit_cast(float, p2 << 16), x1[2 * e], s);
@@ -328,7 +323,14 @@ __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
             }
           }
         }
+        if constexpr (decltype(Mc)::value) request(u, s0 + k0 + UN * 512);  // (also across a segment's end: seg % (UN * 512) == 0 then)
       }
+    };
+    for (int k0 = 0; k0 < n; k0 += UN * 512) {
+      if (s0 + k0 + UN * 512 < a.K)
+        steps(std::true_type{}, k0);
+      else
+        steps(std::false_type{}, k0);
     }
   }
   float scale[NB];
@@ -718,12 +720,16 @@ inline void launch_gemv16_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, 
   a.resident ? launch_gemv16_n<SPL, IN, OUT, false>(st, rec, a, n_cu) : launch_gemv16_n<SPL, IN, OUT, true>(st, rec, a, n_cu);
 }
 
-template <int NB, int R, int IN, int OUT>
+template <int NB, int R, int IN, int OUT, int UN = NB >= 8 ? 2 : 4>
 inline void launch_gemv_bf16_t(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a) {
   const int cap = GEMV_BF16_LDS_FLOATS / NB, seg = a.K < cap ? a.K : cap;
-  launch_k(st, rec, a.resident ? k_gemv_bf16<NB, R, IN, OUT, false> : k_gemv_bf16<NB, R, IN, OUT, true>,
+  launch_k(st, rec, a.resident ? k_gemv_bf16<NB, R, UN, IN, OUT, false> : k_gemv_bf16<NB, R, UN, IN, OUT, true>,
            dim3((a.N + 4 * R - 1) / (4 * R), (a.nb + NB - 1) / NB), dim3(256), (size_t)NB * seg * sizeof(float), a);
 }
+// One row of the rhs: what bounds it is how early the weights are asked for, so a wave has 8 to 16 KB of them on their way while it stages
+// the rhs: four rows a wave where they still fill the chip (all of 2048 columns at once: gate | up of 16384 x 2048 15.0 -> 13.5 us against half
+// of them; 11264 x 2048 and 8192 x 2048 are better with two rows, 10.2 / 11.5 and 8.2 / 9.2), one row and twice the steps for few rows of
+// many columns (2048 x 8192 9.4 -> 8.5, 2048 x 4096 6.5 -> 6.3, against two rows).
 // rows of the rhs that share one pass over the weights: as many as there are, up to 8
 template <int IN, int OUT>
 inline void launch_gemv_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a) {
@@ -731,10 +737,14 @@ inline void launch_gemv_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, co
   if (a.nb <= 1) {
     if (wide)
       launch_gemv_bf16_t<1, 4, IN, OUT>(st, rec, a);
-    else if (a.N >= 2048 || OUT == GEMV_OUT_GLU)
+    else if (OUT == GEMV_OUT_GLU || (a.N >= 2048 && (a.N >= 4096 || a.K < 4096)))
       launch_gemv_bf16_t<1, 2, IN, OUT>(st, rec, a);
-    else if constexpr (OUT != GEMV_OUT_GLU)
-      launch_gemv_bf16_t<1, 1, IN, OUT>(st, rec, a);
+    else if constexpr (OUT != GEMV_OUT_GLU) {
+      if (a.K >= 4096)
+        launch_gemv_bf16_t<1, 1, IN, OUT, 8>(st, rec, a);
+      else
+        launch_gemv_bf16_t<1, 1, IN, OUT>(st, rec, a);
+    }
   } else if (a.nb <= 2) {
     launch_gemv_bf16_t<2, 2, IN, OUT>(st, rec, a);
   } else if (a.nb <= 4) {
