@@ -200,14 +200,17 @@ struct AttnTile {
 // one number per lane, and the accumulators of S^T, exponentiated, ARE the operand of the second product: k slot (lane / 16, i) of the
 // matrix instruction stands for key 4 (lane / 16) + i of a 16-key group, and V^T is read from LDS in the same order.  Scores live in
 // the log2 domain.
-template <typename T, int KC, int VC, int P, bool LAT, int RT>
-__global__ __launch_bounds__(256, sizeof(T) == 2 ? (RT == 1 && KC <= 128 ? 3 : 2) : 1) void k_attn_rows(const MixRows<T> a) {
+// KP: waves that share query rows; wave w + 4 takes the second half of a tile's keys, and the two meet once, at the end.
+template <typename T, int KC, int VC, int P, bool LAT, int RT, int KP>
+__global__ __launch_bounds__(256 * KP, sizeof(T) == 2 ? (KP == 2 && KC <= 128 ? 4 : RT == 1 && KC <= 128 ? 3 : 2) : 1) void k_attn_rows(const MixRows<T> a) {
   typedef AttnTile<T, KC, VC> A;
-  constexpr int KT = A::KT, LK = KC + A::PAD, LV = KT + A::PAD, VT = VC / 16, ST = KT / 16;
-  constexpr int NK = KT * KC / 8 / 256, NV = KT * VC / 8 / 256;  // octets of K and of V per thread and tile
+  constexpr int KT = A::KT, LK = KC + A::PAD, LV = KT + A::PAD, VT = VC / 16, ST = KT / 16 / KP, NTH = 256 * KP;
+  constexpr int NK = KT * KC / 8 / NTH, NV = KT * VC / 8 / NTH;  // octets of K and of V per thread and tile
   static_assert(NK >= 1 && NV >= 2 && NV % 2 == 0, "V octets are handled in pairs of keys");
-  __shared__ __attribute__((aligned(16))) T ks[KT * LK];
-  __shared__ __attribute__((aligned(16))) T vs[VC * LV];
+  static_assert(KP == 1 || (KP == 2 && RT == 1 && ST % 2 == 0), "keys enter the second product 32 at a time");
+  constexpr size_t TILES = (size_t)(KT * LK + VC * LV) * sizeof(T), MEET = KP == 2 ? (size_t)256 * (4 * VT + 2) * sizeof(float) : 0;
+  __shared__ __attribute__((aligned(16))) char attn_lds[TILES > MEET ? TILES : MEET];
+  T *ks = (T*)attn_lds, *vs = ks + KT * LK;
   const AttnGeom& g = a.at;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_wg(), fr = lane & 15, fk = lane >> 4;
   const PassTile t = a.tiles[blockIdx.x / g.H];  // (tiles that see the most keys first)
@@ -246,7 +249,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RT == 1 && KC <= 128 ? 3 : 2
     }
   };
   // this wave's rows, and the keys any of them sees
-  const int w0 = wave * 16 * RT, wn = min(16 * RT, t.n - w0);
+  const int w0 = (wave & 3) * 16 * RT, kof = KP == 2 ? (wave >> 2) * (KT / 2) : 0, wn = min(16 * RT, t.n - w0);
   const int wfirst = t.pos + w0, wlast = wfirst + wn - 1, wlo = attn_first(g, wfirst), wlast_lo = attn_first(g, wlast > 0 ? wlast : 0);
   bf16x8 q16[RT][sizeof(T) == 2 ? KC / 32 : 1];
   float q32[RT][sizeof(T) == 4 ? KC / 4 : 1];
@@ -284,12 +287,12 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RT == 1 && KC <= 128 ? 3 : 2
   unsigned ko[NK], vo[NV];
 #pragma unroll
   for (int u = 0; u < NK; u++) {
-    const int i = u * 256 + tid, c = i % (KC / 8) * 8, row = i / (KC / 8), cc = c < g.D ? c : 0;
+    const int i = u * NTH + tid, c = i % (KC / 8) * 8, row = i / (KC / 8), cc = c < g.D ? c : 0;
     ko[u] = LAT ? (cc < a.la.dim ? row * ldkv + cc : row * a.la.rot + cc - a.la.dim) : row * a.ldp + cc;
   }
 #pragma unroll
   for (int u = 0; u < NV; u++) {
-    const int i = (u >> 1) * 256 + tid, c = i / (KT / 2) * 8, row = i % (KT / 2) * 2 + (u & 1);
+    const int i = (u >> 1) * NTH + tid, c = i / (KT / 2) * 8, row = i % (KT / 2) * 2 + (u & 1);
     vo[u] = row * (LAT ? ldkv : a.ldp) + (c < g.V ? c : 0);
   }
   // (past the last key: that one again, which no row's probabilities count; past the last column: column 0, zero in K's tile, unused in V's)
@@ -300,7 +303,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RT == 1 && KC <= 128 ? 3 : 2
       const T* vb = LAT ? a.kv + row * ldkv + g.H * a.la.dim + h * g.V : a.proj + row * a.ldp + g.cv + kvh * g.V;
 #pragma unroll
       for (int u = 0; u < NK; u++) {
-        const int c = (u * 256 + tid) % (KC / 8) * 8;
+        const int c = (u * NTH + tid) % (KC / 8) * 8;
         rk[u] = oct_load((LAT ? one_of(c < a.la.dim || c >= g.D, kb, a.rot + row * a.la.rot) : kb) + ko[u]);
       }
 #pragma unroll
@@ -309,12 +312,12 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RT == 1 && KC <= 128 ? 3 : 2
     }
 #pragma unroll
     for (int u = 0; u < NK; u++) {
-      const int i = u * 256 + tid, c = i % (KC / 8) * 8, p = j0 + i / (KC / 8);
+      const int i = u * NTH + tid, c = i % (KC / 8) * 8, p = j0 + i / (KC / 8);
       rk[u] = oct_load(k_at(p < hi ? p : hi - 1, c < g.D ? c : 0));
     }
 #pragma unroll
     for (int u = 0; u < NV; u++) {  // octets u, u + 1: the same columns of two neighbouring keys
-      const int i = (u >> 1) * 256 + tid, c = i / (KT / 2) * 8, p = j0 + i % (KT / 2) * 2 + (u & 1);
+      const int i = (u >> 1) * NTH + tid, c = i / (KT / 2) * 8, p = j0 + i % (KT / 2) * 2 + (u & 1);
       rv[u] = oct_load(v_at(p < hi ? p : hi - 1, c < g.V ? c : 0));
     }
   };
@@ -323,12 +326,12 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RT == 1 && KC <= 128 ? 3 : 2
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < NK; u++) {
-      const int i = u * 256 + tid, c = i % (KC / 8) * 8;
+      const int i = u * NTH + tid, c = i % (KC / 8) * 8;
       oct_store(ks + i / (KC / 8) * LK + c, c < g.D ? rk[u] : oct_zero<T>());
     }
 #pragma unroll
     for (int u = 0; u < NV; u += 2) {
-      const int i = (u >> 1) * 256 + tid, c = i / (KT / 2) * 8, key = i % (KT / 2) * 2;
+      const int i = (u >> 1) * NTH + tid, c = i / (KT / 2) * 8, key = i % (KT / 2) * 2;
       T v0[8], v1[8];
       __builtin_memcpy(v0, &rv[u], sizeof v0);
       __builtin_memcpy(v1, &rv[u + 1], sizeof v1);
@@ -340,12 +343,13 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RT == 1 && KC <= 128 ? 3 : 2
     }
     __syncthreads();
     if (j0 + KT < hi) request(j0 + KT);
-    if (wn <= 0 || j0 > wlast || j0 + KT <= wlo) continue;  // (wave-uniform: nothing here for this wave's rows)
-    const bool edge = j0 + KT - 1 > wfirst || j0 < wlast_lo;
+    const int k0 = j0 + kof;  // this wave's keys of the tile: [k0, k0 + KT / KP)
+    if (wn <= 0 || k0 > wlast || k0 + KT / KP <= wlo) continue;  // (wave-uniform: nothing here for this wave's rows)
+    const bool edge = k0 + KT / KP - 1 > wfirst || k0 < wlast_lo;
     f32x4 s[RT][ST];
 #pragma unroll
     for (int j = 0; j < ST; j++) {
-      const T* kr = ks + (j * 16 + fr) * LK;
+      const T* kr = ks + (kof + j * 16 + fr) * LK;
 #pragma unroll
       for (int r = 0; r < RT; r++) s[r][j] = f32x4{0.f, 0.f, 0.f, 0.f};
       if constexpr (sizeof(T) == 2) {
@@ -368,7 +372,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RT == 1 && KC <= 128 ? 3 : 2
     }
 #pragma unroll
     for (int r = 0; r < RT; r++) {
-      const float d0 = (float)(pos[r] - j0 - fk * 4);  // distance to this lane's first key of the tile
+      const float d0 = (float)(pos[r] - k0 - fk * 4);  // distance to this lane's first key of the tile
 #pragma unroll
       for (int j = 0; j < ST; j++) s[r][j] *= scale2;
       if (g.amp) {
@@ -383,7 +387,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RT == 1 && KC <= 128 ? 3 : 2
         for (int j = 0; j < ST; j++)
 #pragma unroll
           for (int e = 0; e < 4; e++) {
-            const int p = j0 + j * 16 + fk * 4 + e;
+            const int p = k0 + j * 16 + fk * 4 + e;
             s[r][j][e] = p <= pos[r] && p >= first[r] ? s[r][j][e] : -INFINITY;
           }
       }
@@ -425,7 +429,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RT == 1 && KC <= 128 ? 3 : 2
 #pragma unroll
         for (int j = 0; j < VT; j++)
           if (VC <= 128 || j * 16 < g.V) {
-            const T* vr = vs + (j * 16 + fr) * LV + jj * 16 + fk * 4;
+            const T* vr = vs + (j * 16 + fr) * LV + kof + jj * 16 + fk * 4;
             bf16x8 vf;
             __builtin_memcpy(&vf, vr, 8);
             __builtin_memcpy((char*)&vf + 8, vr + 16, 8);
@@ -446,6 +450,25 @@ __global__ __launch_bounds__(256, sizeof(T) == 2 ? (RT == 1 && KC <= 128 ? 3 : 2
               for (int e = 0; e < 4; e++) o[r][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[e], s[r][jj][e], o[r][j], 0, 0, 0);
           }
     }
+  }
+  if constexpr (KP == 2) {
+    f32x4* mo = (f32x4*)attn_lds + (wave & 3) * 64 * VT + lane;  // [4][VT][64]
+    float* mm = (float*)attn_lds + 4 * 64 * 4 * VT + (wave & 3) * 128 + lane;
+    __syncthreads();
+    if (wave >= 4) {
+#pragma unroll
+      for (int j = 0; j < VT; j++) mo[j * 64] = o[0][j];
+      mm[0] = m[0];
+      mm[64] = l[0];
+    }
+    __syncthreads();
+    if (wave >= 4) return;
+    const float m1 = mm[0], top = fmaxf(m[0], m1), ref = top == -INFINITY ? 0.f : top;
+    const float w0 = __builtin_amdgcn_exp2f(m[0] - ref), w1 = __builtin_amdgcn_exp2f(m1 - ref);
+    m[0] = top;
+    l[0] = __builtin_fmaf(mm[64], w1, l[0] * w0);
+#pragma unroll
+    for (int j = 0; j < VT; j++) o[0][j] = o[0][j] * w0 + mo[j * 64] * w1;
   }
 #pragma unroll
   for (int r = 0; r < RT; r++) {

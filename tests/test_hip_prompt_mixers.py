@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 
 # decays that carry a state over a thousand rows, so that a segment that starts from the wrong one shows
 LINEAR = sh.config(72, 99, [sh.layer(2, 1, 16, 24, 300, 3, 24, 40, 48, decay=[0.999, 0.99, 0.9]), sh.layer(2, 2, 8, 8, 40, 1, 72, 8, None, decay=[0.998])])
-# 64 heads between 64 and 128 wide: eight tiles of 128 rows and more go to the larger tiles
+# heads between 64 and 128 wide: few tiles give two waves the same rows, eight tiles of 128 rows of 64 heads and more go to the larger tiles
+FEW_HEADS = sh.config(64, 77, [sh.layer(4, 2, 104, 128, 256, 1, 8, 8, None), sh.layer(2, 1, 128, 72, 1000, 1, 8, 8, None)])
 MANY_HEADS = sh.config(64, 77, [sh.layer(64, 2, 72, 80, 600, 1, 8, 8, None)])
 
 
@@ -44,9 +45,9 @@ def test_portions_and_neighbours(ca, hdev, linear, f32):
     close(got, np.concatenate([w[c:] for w, c in zip(want, cuts)]), f32)
 
 
-@pytest.mark.parametrize("n", [895, 897, 1040])
-def test_larger_query_tiles(ca, hdev, tmp_path, n):
-    m = Model(MANY_HEADS, tmp_path, seed=5)
+@pytest.mark.parametrize("heads,n", [("few", 51), ("few", 82), ("few", 83), ("few", 114), ("few", 115), ("few", 700), ("many", 895), ("many", 897), ("many", 1040)])
+def test_query_tiles(ca, hdev, tmp_path, heads, n):
+    m = Model(FEW_HEADS if heads == "few" else MANY_HEADS, tmp_path, seed=5)
     r = m.runner(ca, hdev, False, seq_len=1100)
     t = m.tokens(n, seed=n)
     s = r.open()
