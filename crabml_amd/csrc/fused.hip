@@ -467,12 +467,11 @@ StepF16 step_f16(const crabml_hip_llama* c, std::initializer_list<const crabml_h
 
 // What workgroups of `rows` consecutive rows each read of a Q4_0 / Q8_0 / Q4_1 matrix (prefetch.hpp)
 PrefetchPlan prefetch_rows(const crabml_hip_llama* c, const crabml_hip_buf* w, int rows) {
-  PrefetchPlan pf{};
-  if ((c->cfg.flags & CRABML_HIP_LLAMA_NO_PREFETCH) || (w->dtype != CRABML_HIP_Q4_0 && w->dtype != CRABML_HIP_Q8_0 && w->dtype != CRABML_HIP_Q4_1)) return pf;
-  const size_t blocks = w->k / 32 * rows;
-  prefetch_add(pf, w->ptr, blocks * (w->dtype == CRABML_HIP_Q8_0 ? 32 : 16), 0, (int)(w->m / rows));
-  prefetch_add(pf, (const char*)w->ptr + w->wl.off_scale, blocks * (w->dtype == CRABML_HIP_Q4_1 ? 4 : 2), 0, (int)(w->m / rows));
-  return pf;
+  if ((c->cfg.flags & CRABML_HIP_LLAMA_NO_PREFETCH) || (w->dtype != CRABML_HIP_Q4_0 && w->dtype != CRABML_HIP_Q8_0 && w->dtype != CRABML_HIP_Q4_1))
+    return PrefetchPlan{};
+  const size_t blocks = w->k / 32;
+  return prefetch_matrix((int)w->m, rows, w->ptr, blocks * (w->dtype == CRABML_HIP_Q8_0 ? 32 : 16), (const char*)w->ptr + w->wl.off_scale,
+                         blocks * (w->dtype == CRABML_HIP_Q4_1 ? 4 : 2));
 }
 
 // The front of a step (k_step_front): embedding, and what the first launch of layer 0 reads.  pick: behind the sampler's partials, for the

@@ -456,10 +456,9 @@ void step_linear(Ctx* c, crabml_hip_device::ProfRec* rec, GemvBf16 g) {
 // stay in a cache anyway.  One and two rows: the mixer is the longer for it by what the linear gains (8.8 -> 10.9 and 7.0 -> 5.5 us); 16 rows of
 // 4 layers of width 2048 18593 -> 17965 us for 154 tokens each.  (Latent layers, hosted by k_latent_attn: 0.3 %, not kept.)
 PrefetchPlan prefetch_out(const Ctx* c, const Layer& L, int B) {
-  PrefetchPlan pf{};
+  if (B <= 2 || c->weight_bytes <= RESIDENT_MALL) return PrefetchPlan{};
   const int rows = c->width >= 16384 ? 32 : 16;  // (a workgroup of launch_gemv16_bf16)
-  if (B > 2 && c->weight_bytes > RESIDENT_MALL) prefetch_add(pf, L.w_o, (size_t)rows * L.ldc * 2, 0, c->width / rows);
-  return pf;
+  return prefetch_matrix(c->width, rows, L.w_o, (size_t)L.ldc * 2, nullptr, 0);
 }
 
 MixStep mix_step(const Ctx* c, const Run& run, int B) {
@@ -1448,6 +1447,13 @@ int crabml_hip_hybrid_decode_greedy(crabml_hip_hybrid_t* c, size_t n, const size
 
 }  // extern "C"
 
+extern "C" int crabml_hip_debug_prefetch(int32_t m, int32_t rows, size_t row_bytes, size_t row_bytes2, size_t* bytes) {
+  if (!bytes || m < 1 || rows < 1) return CRABML_HIP_BAD_INPUT;
+  const crabml_hip::PrefetchPlan pf = crabml_hip::prefetch_matrix(m, rows, nullptr, row_bytes, nullptr, row_bytes2);
+  *bytes = 0;
+  for (int i = 0; i < pf.n; i++) *bytes += (size_t)pf.bytes[i] * pf.count[i];
+  return 0;
+}
 extern "C" int crabml_hip_debug_mix_shares(int32_t n_cu, int32_t per, int32_t rows, int32_t* shares) {
   if (!shares || n_cu < 1 || per < 1 || rows < 1) return CRABML_HIP_BAD_INPUT;
   *shares = crabml_hip::mix_shares(n_cu, per, rows);

@@ -1,12 +1,14 @@
 // prefetch.hpp -- the next launch's weights into the L2 they will be read through, by workgroups of a launch that leaves memory idle
 //
-// Attention, mixers, merges and the front of a step are chains of a few dependent round trips in a few workgroups.  Spare workgroups of those
-// launches touch every 128-byte line of the next linear's weights (one dword a lane: 64 lines a wave instruction, no register traffic).
+// A step's attention (k_attn, k_attn_s, k_attn_short) and mixers (k_mix_step) are chains of a few dependent round trips in a few workgroups.  Spare
+// workgroups of those launches touch every 128-byte line of the next linear's weights (one dword a lane: 64 lines a wave instruction, no register traffic).
 // Workgroup i of a launch runs on XCD i mod 8 and each XCD has an L2 of its own (4 MB), so a line helps most where the workgroup that will
 // read it runs: a plan lists the consumer's workgroups with the bytes each reads, and a spare workgroup takes those of its own XCD.
 // A cold launch that reads 8 / 16 / 32 MB takes 3.1 / 4.5 / 6.7 us, behind such a launch 1.7 / 2.0 / 2.7, and 2.6 / 3.8 / 5.9 where the lines
-// were touched from another XCD (they are in the Infinity Cache then).  Above what the L2s hold (64 MB: 10.2 against 12.4) it is not worth
-// its traffic.  No result depends on it, nor on where a workgroup runs.
+// were touched from another XCD (they are in the Infinity Cache then).  Above what the L2s hold there is nothing to win: lines are gone before they
+// are read, and the launch that hosts the traffic is the longer for it.  A run of steps of the hybrid decoder with 3 / 8 / 16 rows, with / without:
+// w_o of 16 MB 1.01 / 0.97 / 1.00, 32 MB 1.01 / 0.98 / 1.00, 48 MB 1.02 / 1.00 / 1.02, 64 MB 1.04 / 1.05 / 1.03, 96 MB 1.07 / 1.07 / 1.08, 128 MB 1.13 / 1.14 /
+// 1.15.  No result depends on it, nor on where a workgroup runs.
 #pragma once
 #include "devutil.hpp"
 
@@ -30,11 +32,20 @@ struct PrefetchArg<true> {
   typedef PrefetchPlan type;
 };
 inline void prefetch_add(PrefetchPlan& pf, const void* p, size_t bytes, int first, int count) {
-  if (pf.n == PrefetchPlan::MAX || bytes < 4 || bytes > (1u << 30) || count < 1) return;
+  if (pf.n == PrefetchPlan::MAX || bytes < 4 || count < 1) return;
   pf.p[pf.n] = (const char*)p;
   pf.bytes[pf.n] = (unsigned)bytes;
   pf.first[pf.n] = first;
   pf.count[pf.n++] = count;
+}
+constexpr size_t PREFETCH_MOST = (size_t)32 << 20;  // what the L2s hold
+// a matrix of which the next launch's workgroups take `rows` of the m rows each: row_bytes a row from p, and row_bytes2 from p2 (scales; 0: none)
+inline PrefetchPlan prefetch_matrix(int m, int rows, const void* p, size_t row_bytes, const void* p2, size_t row_bytes2) {
+  PrefetchPlan pf{};
+  if ((size_t)m * (row_bytes + row_bytes2) > PREFETCH_MOST) return pf;
+  prefetch_add(pf, p, row_bytes * rows, 0, m / rows);
+  prefetch_add(pf, p2, row_bytes2 * rows, 0, m / rows);
+  return pf;
 }
 
 // wg: this workgroup's place in the launch (x fastest); the launch's spare ones are [base, all)

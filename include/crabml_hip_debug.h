@@ -57,6 +57,9 @@ int crabml_hip_debug_gemm_ints(crabml_hip_device_t* dev, const crabml_hip_buf_t*
                                const crabml_hip_buf_t* x, size_t b, int32_t* dst, float* out);
 /* Rows of the rhs that one launch of the row kernels takes over a matrix of m rows (matmul_vec without a matrix-core kernel).  Host only. */
 int crabml_hip_debug_rhs_rows(size_t m, size_t* rows);
+/* Bytes that a step's attention or mixer launch touches ahead of the linear behind it: m rows, `rows` of them a workgroup, row_bytes + row_bytes2 a row.
+ * Host only. */
+int crabml_hip_debug_prefetch(int32_t m, int32_t rows, size_t row_bytes, size_t row_bytes2, size_t* bytes);
 /* Workgroups that share the cached rows of a (sequence, kv head, head block) in the hybrid decoder's step: `per` of those in the launch, up to
  * `rows` rows each, a device of n_cu CUs.  Host only. */
 int crabml_hip_debug_mix_shares(int32_t n_cu, int32_t per, int32_t rows, int32_t* shares);

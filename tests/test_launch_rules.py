@@ -34,3 +34,14 @@ def test_shares_of_cached_rows(n_cu):
             assert lib.crabml_hip_debug_mix_shares(n_cu, per, rows, ctypes.byref(n)) == 0
             assert 1 <= n.value <= -(-rows // 64) and n.value * per <= max(n_cu, per)
             assert n.value == -(-rows // 64) or (n.value + 1) * per > n_cu  # (no fewer than fit)
+
+
+@pytest.mark.parametrize("row_bytes,row_bytes2", [(4096, 0), (4096, 256), (2304, 144), (16384, 0), (32768, 2048)])
+def test_weights_touched_ahead_fit_the_l2s(row_bytes, row_bytes2):
+    """a matrix that the L2s hold (32 MB) is touched ahead whole, a larger one not at all"""
+    for rows in (2, 8, 16, 32):
+        for m in (32, 2048, 4096, 7264, 8192, 32768, 1 << 20):
+            n = ctypes.c_size_t()
+            assert lib.crabml_hip_debug_prefetch(m, rows, ctypes.c_size_t(row_bytes), ctypes.c_size_t(row_bytes2), ctypes.byref(n)) == 0
+            all_of_it = m * (row_bytes + row_bytes2)
+            assert n.value == (all_of_it if all_of_it <= 32 << 20 else 0), (m, rows, n.value)
