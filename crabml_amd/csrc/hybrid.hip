@@ -5,6 +5,7 @@
 #include <memory>
 
 #include "dequant.hpp"
+#include "graph_steps.hpp"
 #include "hybrid_latent.hpp"
 #include "hybrid_rows.hpp"
 #include "hybrid_step.hpp"
@@ -53,9 +54,6 @@ constexpr size_t LOGIT_ROWS = 256;  // rows of logits a pass keeps on the device
 // 8090 / 8149, 394 MB 12280 / 11520, 504 MB 17433 / 17121.
 constexpr size_t RESIDENT_L2 = (size_t)32 << 20, RESIDENT_MALL = (size_t)256 << 20;
 constexpr int META_SLOTS = 4;
-// steps of a greedy run behind one another in one graph: a graph's two ends cost 6 to 7 us between two launches (measured with graphs of 35 and
-// 140 small kernels)
-constexpr size_t STEPS_A_GRAPH = 8;
 
 }  // namespace
 
@@ -96,6 +94,8 @@ struct crabml_hip_hybrid {
   StepSeq* h_seq = nullptr;  // pinned ring of META_SLOTS * HYB_STEP_ROWS
   int h_seq_next = 0;
   std::map<int, std::pair<hipGraph_t, hipGraphExec_t>> graphs;  // (graph_key)
+  size_t single_steps[HYB_STEP_ROWS + 1] = {};  // greedy steps that a batch size has made one at a time
+  bool graph_steps_now = false;                 // test hook: several steps a graph from the first run on
   // prompt pass (allocated on first use)
   size_t rows_cap = 0, hist_cap = 0, meta_bytes = 0;
   char *meta = nullptr, *h_meta = nullptr;
@@ -602,8 +602,8 @@ int latent_step(Ctx* c, const Run& run, int B, bool prof) {
 }
 
 
-// the front of a step (k_front_rows); pick: behind the sampler's partials
-void enqueue_front(Ctx* c, int B, bool pick) {
+// the front of a step (k_front_rows); pick: behind the sampler's partials; embed: not where the next step brings its own front
+void enqueue_front(Ctx* c, int B, bool pick, bool embed) {
   const size_t stride = (size_t)HYB_STEP_ROWS * c->ldx;
   RowPick p;
   if (pick) {
@@ -614,20 +614,21 @@ void enqueue_front(Ctx* c, int B, bool pick) {
     p.count = c->st_count;
     p.out = c->st_out;
   }
-  k_front_rows<<<B, 1024, 0, c->dev->stream>>>(p, c->embed, c->st_seq, c->width, c->ldx, c->cfg.embed_scale, c->freq, c->st_x, c->keep_emb ? c->st_emb : nullptr,
+  k_front_rows<<<B, embed ? 1024 : 64, 0, c->dev->stream>>>(p, c->embed, c->st_seq, embed ? c->width : 0, c->ldx, c->cfg.embed_scale, c->freq, c->st_x, c->keep_emb ? c->st_emb : nullptr,
                                                c->runs[0].add_vec, streams_at_start(c, stride), c->st_in, rows16(c, B) ? c->st_x16 : nullptr,
                                                c->streams ? c->layers[c->runs[0].layer].norm1 : nullptr, c->st_xss, c->n_xss);
 }
 
-// one step of B rows: front, layers, classifier -- or, with the sampler, layers, classifier, sampler and the next step's front
-int enqueue_step(Ctx* c, int B, bool sample, bool prof) {
+// One step of B rows: front, layers, classifier, and the sampler if asked for.  Inside a graph of several steps the sampler's second stage and the next
+// step's front are one launch -- led: the step before ran this one's front; lead: this one runs the next one's.
+int enqueue_step(Ctx* c, int B, bool sample, bool prof, bool led = false, bool lead = false) {
   crabml_hip_device* dev = c->dev;
   hipStream_t st = dev->stream;
   const float eps = c->cfg.norm_eps;
   const size_t stride = (size_t)HYB_STEP_ROWS * c->ldx;
   const float* next_gain = nullptr;
   float* x_in = c->streams ? c->st_in : c->st_x;  // what a norm reads
-  if (!sample) enqueue_front(c, B, false);
+  if (!led) enqueue_front(c, B, false, true);
   for (size_t r = 0; r < c->runs.size(); r++) {
     const Run& run = c->runs[r];
     const Layer& L = c->layers[run.layer];
@@ -739,25 +740,22 @@ int enqueue_step(Ctx* c, int B, bool sample, bool prof) {
   head_rows(c, x_in, B, prof, false);
   if (sample) {
     k_argmax_partial<<<dim3(ARGMAX_BLOCKS, B), 256, 0, st>>>(c->st_logits, c->vocab, c->am_val, c->am_idx, 0, c->vocab);
-    enqueue_front(c, B, true);
+    enqueue_front(c, B, true, lead);
   }
   CH_HIP(dev, hipGetLastError());
   return 0;
 }
 
 int graph_key(int B, bool sample, int steps) { return (steps * (HYB_STEP_ROWS + 1) + B) * 2 + (sample ? 1 : 0); }
-// one decode step of B rows, or several of a greedy run, from its graph (captured when that batch size first comes up), or eagerly
-int run_step(Ctx* c, int B, bool sample, int steps = 1) {
+bool step_graphs(const Ctx* c) { return !(c->cfg.flags & CRABML_HIP_HYBRID_NO_GRAPH) && !c->dev->prof_on; }
+// the graph of one decode step of B rows, or of several of a greedy run, captured when it is first asked for
+int step_graph(Ctx* c, int B, bool sample, int steps, std::pair<hipGraph_t, hipGraphExec_t>* out) {
   crabml_hip_device* dev = c->dev;
-  if ((c->cfg.flags & CRABML_HIP_HYBRID_NO_GRAPH) || dev->prof_on) {
-    for (int i = 0; i < steps; i++) CH_TRY(enqueue_step(c, B, sample, true));
-    return 0;
-  }
   auto& slot = c->graphs[graph_key(B, sample, steps)];
   if (!slot.second) {
     CH_HIP(dev, hipStreamBeginCapture(dev->stream, hipStreamCaptureModeThreadLocal));
     int rc = 0;
-    for (int i = 0; i < steps && rc == 0; i++) rc = enqueue_step(c, B, sample, false);
+    for (int i = 0; i < steps && rc == 0; i++) rc = enqueue_step(c, B, sample, false, i > 0, i + 1 < steps);
     hipGraph_t graph = nullptr;
     const hipError_t e = hipStreamEndCapture(dev->stream, &graph);
     hipGraphExec_t exec = nullptr;
@@ -768,7 +766,32 @@ int run_step(Ctx* c, int B, bool sample, int steps = 1) {
     }
     slot = {graph, exec};
   }
-  CH_HIP(dev, hipGraphLaunch(slot.second, dev->stream));
+  *out = slot;
+  return 0;
+}
+// one decode step of B rows from its graph, or eagerly
+int run_step(Ctx* c, int B, bool sample) {
+  if (!step_graphs(c)) return enqueue_step(c, B, sample, true);
+  std::pair<hipGraph_t, hipGraphExec_t> g;
+  CH_TRY(step_graph(c, B, sample, 1, &g));
+  CH_HIP(c->dev, hipGraphLaunch(g.second, c->dev->stream));
+  return 0;
+}
+// Steps at a time of a greedy run of n: what a graph of several holds, where there is one or this run is the one that captures it (graph_steps.hpp)
+int greedy_graph(Ctx* c, int B, size_t n, int* steps, hipGraphExec_t* exec) {
+  *steps = 1;
+  if (!step_graphs(c)) return 0;
+  std::pair<hipGraph_t, hipGraphExec_t> g;
+  CH_TRY(step_graph(c, B, true, 1, &g));
+  size_t nodes = 0;
+  CH_HIP(c->dev, hipGraphGetNodes(g.first, nullptr, &nodes));
+  const int s = steps_a_graph(nodes, c->cfg.seq_len);
+  if (s == 1 || n < (size_t)s) return 0;
+  const auto have = c->graphs.find(graph_key(B, true, s));
+  if ((have == c->graphs.end() || !have->second.second) && !c->graph_steps_now && !steps_graph_earned(nodes, s, c->single_steps[B] + n)) return 0;
+  CH_TRY(step_graph(c, B, true, s, &g));
+  *steps = s;
+  *exec = g.second;
   return 0;
 }
 
@@ -1226,6 +1249,8 @@ int create_impl(Ctx* c, const crabml_hip_hybrid_layer_t* layers, const crabml_hi
   {
     const char *h = getenv("CRABML_HIP_TEST_HOOKS"), *e = getenv("CRABML_HIP_STREAM_WEIGHTS");  // test hook: small models through the large ones' loads
     if (h && h[0] == '1' && e && e[0] == '1') c->weight_bytes = SIZE_MAX;
+    const char* g = getenv("CRABML_HIP_GRAPH_STEPS");
+    c->graph_steps_now = h && h[0] == '1' && g && g[0] == '1';
   }
   const size_t B = HYB_STEP_ROWS;
   CH_TRY(dalloc_n(c, B, &c->st_seq));
@@ -1429,16 +1454,18 @@ int crabml_hip_hybrid_decode_greedy(crabml_hip_hybrid_t* c, size_t n, const size
       CH_BAIL(dev, CRABML_HIP_TENSOR_ERROR, "hybrid: %zu steps do not fit sequence %zu (%zu of %zu used)", n_steps, seqs[i], c->seqs[seqs[i]].len, c->cfg.seq_len);
   }
   if (n_steps == 0) return 0;
+  int steps = 1;
+  hipGraphExec_t several = nullptr;
+  CH_TRY(greedy_graph(c, (int)n, n_steps, &steps, &several));
   CH_TRY(step_begin(c, n, seqs, tokens));
   CH_HIP(dev, hipMemsetAsync(c->st_count, 0, HYB_STEP_ROWS * sizeof(int), dev->stream));
-  enqueue_front(c, (int)n, false);
-  // (a graph of several steps is captured where the run itself earns that back, about a tenth of a millisecond)
-  const bool several = n_steps >= 2 * STEPS_A_GRAPH || c->graphs.count(graph_key((int)n, true, (int)STEPS_A_GRAPH));
-  for (size_t s = 0; s < n_steps;) {
-    const int steps = several && n_steps - s >= STEPS_A_GRAPH ? (int)STEPS_A_GRAPH : 1;
-    CH_TRY(run_step(c, (int)n, true, steps));
-    s += steps;
+  size_t s = 0;
+  if (steps > 1) {
+    for (; s + steps <= n_steps; s += steps) CH_HIP(dev, hipGraphLaunch(several, dev->stream));
+  } else {
+    c->single_steps[n] += n_steps;
   }
+  for (; s < n_steps; s++) CH_TRY(run_step(c, (int)n, true));
   for (size_t i = 0; i < n; i++) c->seqs[seqs[i]].len += n_steps;
   CH_HIP(dev, hipMemcpyAsync(out_tokens, c->st_out, n_steps * n * sizeof(uint32_t), hipMemcpyDeviceToHost, dev->stream));
   CH_HIP(dev, hipStreamSynchronize(dev->stream));
@@ -1447,6 +1474,12 @@ int crabml_hip_hybrid_decode_greedy(crabml_hip_hybrid_t* c, size_t n, const size
 
 }  // extern "C"
 
+extern "C" int crabml_hip_debug_graph_steps(size_t nodes, size_t seq_len, size_t done, int32_t* steps, int32_t* earned) {
+  if (!steps || !earned) return CRABML_HIP_BAD_INPUT;
+  *steps = crabml_hip::steps_a_graph(nodes, seq_len);
+  *earned = crabml_hip::steps_graph_earned(nodes, *steps, done) ? 1 : 0;
+  return 0;
+}
 extern "C" int crabml_hip_debug_prefetch(int32_t m, int32_t rows, size_t row_bytes, size_t row_bytes2, size_t* bytes) {
   if (!bytes || m < 1 || rows < 1) return CRABML_HIP_BAD_INPUT;
   const crabml_hip::PrefetchPlan pf = crabml_hip::prefetch_matrix(m, rows, nullptr, row_bytes, nullptr, row_bytes2);

@@ -25,8 +25,8 @@ struct StepSeq {
   char* slab;
 };
 
-// A step's front: embedding and what the first norm reads, a workgroup per row.  With pick.pv it runs behind the sampler's partials at a step's end, for
-// the tokens that they name: combining them (every wave for itself), advancing and embedding were three launches of one memory round trip
+// A step's front: embedding and what the first norm reads, a workgroup per row.  With pick.pv it runs behind the sampler's partials, for the tokens
+// that they name (the next step's front; width 0 where that step is in another graph and brings its own): combining them (every wave for itself), advancing and embedding were three launches of one memory round trip
 // each, 13.6 of the 18.4 us that a 16-row step spent outside its layers and classifier (with several steps in a graph, 16 x 154 tokens of 4 layers of
 // width 2048: 20629 -> 19997 us; one sequence of 81 tokens on latent and windowed layers 12734 -> 12414).
 struct RowPick {

@@ -47,9 +47,29 @@ NILIVIK_WIDE = sh.config(4104, 67, [sh.layer(1, 1, 8, 8, 16, 1, 8, 8, 16)])  # (
 BIFAZEN = sb.config(200, 131, [sb.latent(2, 12, 4, 12, 20, 30, 40), sb.attention(2, 1, 8, 8, 9, 40)], streams=3)
 
 
+@pytest.mark.parametrize("config,tensors", [(NILIVIK, sh.random_tensors), (BIFAZEN, sb.random_tensors)])
+@pytest.mark.parametrize("rows", [1, 3])
+def test_several_steps_a_graph_when_runs_have_earned_it(ca, hdev, tmp_path, config, tensors, rows):
+    """short runs make their steps one at a time until they have made up for a graph of several, and the same tokens before and behind that"""
+    folder = sh.write_model(config, tensors(config, 7), str(tmp_path / "m"))
+    g, e = ca.load_model(folder, hdev, seq_len=300), ca.load_model(folder, hdev, seq_len=300, use_graph=False)
+    seqs = [[r.open() for _ in range(rows)] for r in (g, e)]
+    ids = list(range(1, rows + 1))
+    for n in (9, 30, 9, 60, 17, 100, 12):
+        a, b = g.decode_batch(seqs[0], ids, n), e.decode_batch(seqs[1], ids, n)
+        assert list(a) == list(b), n
+        ids = list(a[-rows:])
+    last = [r.step([(s, [t], [0]) for s, t in zip(q, ids)]) for r, q in zip((g, e), seqs)]
+    assert np.array_equal(last[0].view(np.uint32), last[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("now", [False, True])
 @pytest.mark.parametrize("config,tensors", [(NILIVIK, sh.random_tensors), (NILIVIK_WIDE, sh.random_tensors), (BIFAZEN, sb.random_tensors)])
 @pytest.mark.parametrize("f32", [False, True])
-def test_greedy_batches_equal_single_steps(ca, hdev, tmp_path, config, tensors, f32):
+def test_greedy_batches_equal_single_steps(ca, hdev, tmp_path, monkeypatch, config, tensors, f32, now):
+    if now:  # several steps a graph from the first run on
+        monkeypatch.setenv("CRABML_HIP_TEST_HOOKS", "1")
+        monkeypatch.setenv("CRABML_HIP_GRAPH_STEPS", "1")
     folder = sh.write_model(config, tensors(config, 5), str(tmp_path / "m"))
     g, e, h = (ca.load_model(folder, hdev, seq_len=64, f32=f32, **kw) for kw in ({}, {"use_graph": False}, {}))
     for rows in (1, 2, 3, 16):

@@ -45,3 +45,25 @@ def test_weights_touched_ahead_fit_the_l2s(row_bytes, row_bytes2):
             assert lib.crabml_hip_debug_prefetch(m, rows, ctypes.c_size_t(row_bytes), ctypes.c_size_t(row_bytes2), ctypes.byref(n)) == 0
             all_of_it = m * (row_bytes + row_bytes2)
             assert n.value == (all_of_it if all_of_it <= 32 << 20 else 0), (m, rows, n.value)
+
+
+def graph_steps(nodes, seq_len, done):
+    steps, earned = ctypes.c_int32(), ctypes.c_int32()
+    assert lib.crabml_hip_debug_graph_steps(ctypes.c_size_t(nodes), ctypes.c_size_t(seq_len), ctypes.c_size_t(done), ctypes.byref(steps), ctypes.byref(earned)) == 0
+    return steps.value, bool(earned.value)
+
+
+def test_a_capture_is_bounded_and_earned():
+    """several steps in a graph: a bounded number of launches, and none captured before the steps that it serves have won what the capture costs (at
+    least 1.4 us a launch; at most 7 us between two steps)"""
+    for nodes in (1, 14, 23, 31, 44, 63, 123, 161, 192, 193, 243, 1000):
+        for seq_len in (1, 2, 3, 15, 16, 400, 8192):
+            n = graph_steps(nodes, seq_len, 0)[0]
+            assert 1 <= n <= 8 and (n == 1 or (n * nodes <= 384 and 2 * n <= seq_len)), (nodes, seq_len)
+        n, first = graph_steps(nodes, 8192, 0)[0], next((d for d in range(1, 3000) if graph_steps(nodes, 8192, d)[1]), None)
+        if n == 1:
+            assert first is None and nodes > 192
+        else:
+            assert first * 7 * (n - 1) / n >= 1.4 * nodes * n, (nodes, n, first)
+    assert graph_steps(23, 400, 16) == (8, False) and graph_steps(123, 400, 64) == (3, False)  # (a short answer, a deeper model)
+    assert graph_steps(23, 400, 200) == (8, True)
