@@ -167,7 +167,9 @@ struct crabml_hip_llama {
   int multi_steps = 1;
   bool use_graph = false;
   bool capturing = false;
-  bool lead = false;  // a step ends with the next one's front (enqueue_front): steps that follow each other on this device without the host
+  bool chains = false;  // steps can follow each other on this device without the host: several in one graph
+  // the step being enqueued, inside a graph of several: the one before ran its front (enqueue_front); it ends with the next one's
+  bool led = false, lead = false;
   int attn_variant = 0;         // which of them the next enqueue emits: 0 = one workgroup per head, 1 = the long-context kernels,
                                 // 2 = split-KV attention with the merge inside the launch (ticket form: the mid range), 3 = k_attn_short
   size_t flash_ticket_until = 0;  // > 0: positions [attn_long_from, this) run variant 2
@@ -735,7 +737,7 @@ int enqueue_segment_t(crabml_hip_llama* c, int seg) {
   if ((seg & 1) == 0) {
     // embedding and attention rmsnorm (llama2.rs:222-234)
     if (l == 0) {
-      if (!c->lead) CH_TRY(enqueue_front(c, false));
+      if (!c->led) CH_TRY(enqueue_front(c, false));
     } else if (!norm_epi) {
       norm_quant((const float*)c->rms_att[l]->ptr, g.rms_norm_eps, tp);
     }
@@ -854,7 +856,7 @@ int enqueue_segment_generic(crabml_hip_llama* c, int seg) {
   }
   const int l = seg / 2;
   if ((seg & 1) == 0) {
-    if (l == 0 && !c->lead) CH_TRY(enqueue_front(c, false));
+    if (l == 0 && !c->led) CH_TRY(enqueue_front(c, false));
     norm((const float*)c->rms_att[l]->ptr, g.rms_norm_eps, tp && l > 0);
     const void* act = quant(c->xn, dim, c->qt, c->act_dim);
     QkvEpi e{c->qbuf, c->kc[l], c->vc[l], c->rope, pos_d, 1.0f / std::sqrt((float)hd), dim_l, kv_dim_l, hd,
@@ -923,7 +925,7 @@ int enqueue_segment_f16(crabml_hip_llama* c, int seg) {
   }
   const int l = seg / 2;
   if ((seg & 1) == 0) {
-    if (l == 0 && !c->lead) CH_TRY(enqueue_front(c, false));
+    if (l == 0 && !c->led) CH_TRY(enqueue_front(c, false));
     const QkvEpi e{c->qbuf, c->kc[l], c->vc[l], c->rope, c->state + 1, 1.0f / std::sqrt((float)hd), dim_l, kv_dim_l, hd,
                    (int)g.rope_dim, c->npairs, (int)g.seq_len, g.use_f16_kv_cache ? 1 : 0};
     CH_TRY(P0(1, dim_l + 2.0 * kv_dim_l, dim));
@@ -1081,7 +1083,7 @@ int enqueue_segment_k(crabml_hip_llama* c, int seg) {
   const int l = seg / 2;
   if ((seg & 1) == 0) {
     if (l == 0) {
-      if (!c->lead) CH_TRY(enqueue_front(c, false));
+      if (!c->led) CH_TRY(enqueue_front(c, false));
     } else if (!nepi) {
       norm_quant((const float*)c->rms_att[l]->ptr, g.rms_norm_eps, tp, QT);
     }
@@ -1240,7 +1242,12 @@ bool capture_steps(crabml_hip_llama* c, int variant, int steps, hipGraph_t* grap
   c->capturing = true;
   c->attn_variant = variant;
   int rc = 0;
-  for (int i = 0; i < steps && rc == 0; i++) rc = enqueue_step(c);
+  for (int i = 0; i < steps && rc == 0; i++) {
+    c->led = i > 0;
+    c->lead = i + 1 < steps;
+    rc = enqueue_step(c);
+  }
+  c->led = c->lead = false;
   c->capturing = false;
   c->attn_variant = 0;
   hipGraph_t graph = nullptr;
@@ -2385,7 +2392,7 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
       return hip_fail(dev, e, "llama init", __FILE__, __LINE__);
     }
   }
-  c->lead = tp == 1 && !c->ext_kv && !c->split_vocab;
+  c->chains = tp == 1 && !c->ext_kv && !c->split_vocab;
   // capture one decode step into a graph.
   // tp > 1 without a communicator = a rank of the single-device simulation: driven segment by segment, no graph.
   // tp > 1 over RCCL launches eagerly unless CRABML_HIP_LLAMA_TP_GRAPH asks for the collectives to be captured too.
@@ -2401,7 +2408,7 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
       ok = capture_steps(c, v, 1, &c->graph[v], &c->exec[v]);
       // several steps in a graph where a step is short enough for the gap between two graphs to show
       size_t nodes = 0;
-      if (!ok || !c->lead || hipGraphGetNodes(c->graph[v], nullptr, &nodes) != hipSuccess || nodes == 0) continue;
+      if (!ok || !c->chains || hipGraphGetNodes(c->graph[v], nullptr, &nodes) != hipSuccess || nodes == 0) continue;
       if (c->multi_steps == 1) c->multi_steps = (int)std::min({crabml_hip_llama::MULTI_STEPS + 0, crabml_hip_llama::MULTI_NODES / nodes, (size_t)g.seq_len / 2});
       if (c->multi_steps > 1) (void)capture_steps(c, v, c->multi_steps, &c->multi_graph[v], &c->multi_exec[v]);
     }
@@ -2467,7 +2474,6 @@ int crabml_hip_llama_forward(crabml_hip_llama_t* c, size_t token, size_t pos, fl
     CH_BAIL(dev, CRABML_HIP_BAD_INPUT, "llama: a tp rank without a communicator is driven by crabml_hip_llama_tp_sim_*");
   CH_TRY(check_step(c, token, pos));
   CH_TRY(set_state(c, token, pos, 0));
-  if (c->lead) CH_TRY(enqueue_front(c, false));
   CH_TRY(run_step(c, pos));
   c->kv_len++;
   if (logits) {
@@ -2494,7 +2500,6 @@ int crabml_hip_llama_decode_greedy(crabml_hip_llama_t* c, size_t token, size_t n
     CH_BAIL(dev, CRABML_HIP_TENSOR_ERROR, "llama: %zu steps do not fit the kv cache (%zu of %zu used)", n_steps, c->kv_len, c->cfg.seq_len);
   if (n_steps == 0) return 0;
   CH_TRY(set_state(c, token, c->kv_len, 0));
-  if (c->lead) CH_TRY(enqueue_front(c, false));
   CH_TRY(run_steps(c, c->kv_len, n_steps));
   c->kv_len += n_steps;
   int fault = 0;
@@ -2560,7 +2565,6 @@ int crabml_hip_llama_tp_sim_forward(crabml_hip_llama_t* const* ranks, int n, siz
   for (int r = 0; r < n; r++) ptrs.p[r] = ranks[r]->partial;
   const int dim = (int)ranks[0]->cfg.embedding_dim;
   for (int r = 0; r < n; r++) ranks[r]->attn_variant = variant_of(ranks[r], pos);
-  if (ranks[0]->lead) CH_TRY(enqueue_front(ranks[0], false));  // (n == 1)
   for (int s = 0; s < nseg; s++) {
     for (int r = 0; r < n; r++) CH_TRY(enqueue_segment(ranks[r], s));
     if (n > 1 && s + 1 < nseg) k_sim_allreduce<<<(dim + 255) / 256, 256, 0, dev->stream>>>(ptrs, n, dim);

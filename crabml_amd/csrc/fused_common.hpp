@@ -248,7 +248,7 @@ __global__ __launch_bounds__(1024) void k_norm_f32(float* __restrict__ x, const 
 // These were four launches at a step's two ends (combine the arg-max partials, embedding, norm, quantizer of a Q8_K rhs): each is one
 // round trip to memory behind 1.7 us of launch.  One workgroup does all of it: every wave combines the partials for itself (two
 // requests a lane), so the token is known without a barrier; the row's elements are requested together whatever the table's format is.
-// A context whose steps follow each other on the device (`lead`, fused.hip) runs it at the END of a step, for the next one.
+// Inside a graph of several steps (run_steps) it runs at the END of a step, for the next one; a graph's first step runs it without the partials.
 // With several steps in a graph (run_steps), us a request, before -> after: 57 tokens of the 15M-parameter model in Q8_0 6482 -> 6047, 88 tokens of 8
 // layers of the 8B shape in Q4_0 24840 -> 24232.
 enum { FRONT_ROW = 0, FRONT_Q8_0 = 1, FRONT_Q8_1 = 2, FRONT_Q8_K = 3 };  // what is left beside x: nothing, or the normed row's planes

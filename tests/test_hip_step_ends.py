@@ -107,3 +107,19 @@ def test_weights_past_the_caches_are_the_same_weights(ca, hdev, tmp_path, monkey
         for r, q in ((kept, a), (past, b)):
             for s in q:
                 r.close(s)
+
+
+@pytest.mark.parametrize("fmt,shape", [("Q4_0", "tiny-hd128"), ("Q8_0", "15m"), ("Q4_K", "tiny-hd128"), ("F16", "15m"), ("Q6_K", "tiny-gqa")])
+def test_a_step_by_itself_has_one_front(ca, fmt, shape):
+    """a program that samples on the host pays for no embedding and first norm but its own step's (in these formats the only launch that counts as one)"""
+    dev = ca.HipTensorDevice(0)
+    conf, w = synth.to_hip(synth.build_model(synth.SHAPES[shape], synth.TYPE_BY_NAME[fmt], seed=22), dev)
+    r = ca.HipLlamaRunner(conf, w, dev, 60, True, False)
+    r.forward(3, 0)
+    dev.prof_enable(True)
+    for i in range(3):
+        r.forward(5 + i, 1 + i)
+        assert sum(x["launches"] for x in dev.prof_read() if x["stage"] == 6) == 1, i
+    r.decode_greedy(9, 4)
+    assert sum(x["launches"] for x in dev.prof_read() if x["stage"] == 6) == 4
+    dev.prof_enable(False)
