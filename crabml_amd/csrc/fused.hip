@@ -23,6 +23,7 @@
 #include "fused_common.hpp"
 #include "fused_attention.hpp"
 #include "fused_ffn.hpp"
+#include "graph_steps.hpp"
 #include "fused_f16.hpp"
 #include "gemm_bf16.hpp"
 #include "prefill_rows.hpp"
@@ -159,12 +160,15 @@ struct crabml_hip_llama {
   // by attn_variant
   hipGraph_t graph[4] = {nullptr, nullptr, nullptr, nullptr};
   hipGraphExec_t exec[4] = {nullptr, nullptr, nullptr, nullptr};
-  // ... and of several steps (multi_steps) behind one another: a graph's two ends cost 6 to 7 us between two launches (measured with 35 and
-  // 140 small kernels), which a greedy run of a small model pays for every token
-  hipGraph_t multi_graph[4] = {nullptr, nullptr, nullptr, nullptr};
-  hipGraphExec_t multi_exec[4] = {nullptr, nullptr, nullptr, nullptr};
-  static constexpr size_t MULTI_STEPS = 8, MULTI_NODES = 384;  // (161 launches a step, 32 layers: the gap is half a percent, two steps)
-  int multi_steps = 1;
+  // ... and of several steps behind one another (graph_steps.hpp), when greedy runs have earned it
+  struct Several {
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+    int steps = 1;          // that it holds
+    size_t nodes = 0;       // launches of one step
+    size_t single = 0;      // greedy steps made one at a time
+  } several[4];
+  bool graph_steps_now = false;  // test hook: from the first run on
   bool use_graph = false;
   bool capturing = false;
   bool chains = false;  // steps can follow each other on this device without the host: several in one graph
@@ -1217,24 +1221,6 @@ int run_step(crabml_hip_llama* c, size_t pos) {
 }
 
 
-// `n` decode steps from cache position `pos` on: as many at a time as one graph holds, as long as they take the same attention form
-int run_steps(crabml_hip_llama* c, size_t pos, size_t n) {
-  for (size_t i = 0; i < n;) {
-    const int v = variant_of(c, pos + i);
-    size_t m = 0;
-    if (c->use_graph && c->multi_exec[v] && n - i >= (size_t)c->multi_steps)
-      while (m < (size_t)c->multi_steps && variant_of(c, pos + i + m) == v) m++;
-    if (m > 0 && m == (size_t)c->multi_steps) {
-      CH_HIP(c->dev, hipGraphLaunch(c->multi_exec[v], c->dev->stream));
-      i += m;
-    } else {
-      CH_TRY(run_step(c, pos + i));
-      i++;
-    }
-  }
-  return 0;
-}
-
 // `steps` decode steps of attention form `variant` as a graph (token / pos / step are read from device memory by the kernels)
 bool capture_steps(crabml_hip_llama* c, int variant, int steps, hipGraph_t* graph_out, hipGraphExec_t* exec_out) {
   hipStream_t st = c->dev->stream;
@@ -1260,6 +1246,25 @@ bool capture_steps(crabml_hip_llama* c, int variant, int steps, hipGraph_t* grap
   }
   if (graph) (void)hipGraphDestroy(graph);
   return false;
+}
+
+// `n` decode steps from cache position `pos` on: as many at a time as one graph holds, as long as they take the same attention form
+int run_steps(crabml_hip_llama* c, size_t pos, size_t n) {
+  for (size_t i = 0; i < n;) {
+    const int v = variant_of(c, pos + i);
+    size_t m = 1;  // steps of this form
+    while (i + m < n && variant_of(c, pos + i + m) == v) m++;
+    auto& s = c->several[v];
+    if (s.steps > 1 && m >= (size_t)s.steps && !s.exec && (c->graph_steps_now || steps_graph_earned(s.nodes, s.steps, s.single + m)) &&
+        !capture_steps(c, v, s.steps, &s.graph, &s.exec)) {
+      (void)hipGetLastError();
+      s.steps = 1;
+    }
+    for (; s.exec && m >= (size_t)s.steps; i += s.steps, m -= s.steps) CH_HIP(c->dev, hipGraphLaunch(s.exec, c->dev->stream));
+    if (!s.exec) s.single += m;
+    for (; m > 0; i++, m--) CH_TRY(run_step(c, pos + i));
+  }
+  return 0;
 }
 
 // ---- batched prefill ---------------------------------------------------------------------------------------
@@ -2406,12 +2411,11 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
     for (int v = 0; v < 4 && ok; v++) {
       if (!has[v]) continue;
       ok = capture_steps(c, v, 1, &c->graph[v], &c->exec[v]);
-      // several steps in a graph where a step is short enough for the gap between two graphs to show
-      size_t nodes = 0;
-      if (!ok || !c->chains || hipGraphGetNodes(c->graph[v], nullptr, &nodes) != hipSuccess || nodes == 0) continue;
-      if (c->multi_steps == 1) c->multi_steps = (int)std::min({crabml_hip_llama::MULTI_STEPS + 0, crabml_hip_llama::MULTI_NODES / nodes, (size_t)g.seq_len / 2});
-      if (c->multi_steps > 1) (void)capture_steps(c, v, c->multi_steps, &c->multi_graph[v], &c->multi_exec[v]);
+      auto& s = c->several[v];
+      if (ok && c->chains && hipGraphGetNodes(c->graph[v], nullptr, &s.nodes) == hipSuccess) s.steps = steps_a_graph(s.nodes, g.seq_len);
     }
+    const char *h = getenv("CRABML_HIP_TEST_HOOKS"), *e = getenv("CRABML_HIP_GRAPH_STEPS");
+    c->graph_steps_now = h && h[0] == '1' && e && e[0] == '1';
     (void)hipGetLastError();
     c->use_graph = ok;
     if (!ok && tp == 1) {  // fail loudly: the caller asked for the graph path
@@ -2445,8 +2449,8 @@ int crabml_hip_llama_destroy(crabml_hip_llama_t* c) {
   for (int v = 0; v < 4; v++) {
     if (c->exec[v]) (void)hipGraphExecDestroy(c->exec[v]);
     if (c->graph[v]) (void)hipGraphDestroy(c->graph[v]);
-    if (c->multi_exec[v]) (void)hipGraphExecDestroy(c->multi_exec[v]);
-    if (c->multi_graph[v]) (void)hipGraphDestroy(c->multi_graph[v]);
+    if (c->several[v].exec) (void)hipGraphExecDestroy(c->several[v].exec);
+    if (c->several[v].graph) (void)hipGraphDestroy(c->several[v].graph);
   }
   for (auto& a : c->allocs) pool_free(c->dev, a.first, a.second);
   for (auto* b : c->held) crabml_hip_buf_release(b);
@@ -2624,6 +2628,14 @@ int crabml_hip_llama_debug_graphs(crabml_hip_llama_t* c, size_t pos, int32_t* fo
   *form = variant_of(c, pos);
   *captured = 0;
   for (int v = 0; v < 4; v++) *captured |= c->exec[v] ? 1u << v : 0u;
+  return 0;
+}
+
+int crabml_hip_llama_debug_graph_steps(crabml_hip_llama_t* c, size_t pos, int32_t* steps, int32_t* captured) {
+  if (!c || !steps || !captured || pos >= c->cfg.seq_len) return CRABML_HIP_BAD_INPUT;
+  const auto& s = c->several[variant_of(c, pos)];
+  *steps = s.steps;
+  *captured = s.exec ? 1 : 0;
   return 0;
 }
 

@@ -137,6 +137,8 @@ int crabml_hip_debug_flash_attention_rows(crabml_hip_device_t* dev, const float*
 
 /* the attention form of the step that serves cache position `pos`, and the forms whose step this context captured (bit v: form v) */
 int crabml_hip_llama_debug_graphs(crabml_hip_llama_t* ctx, size_t pos, int32_t* form, uint32_t* captured);
+/* greedy steps a graph of several holds at cache position pos (1: none is made), and whether it has been captured */
+int crabml_hip_llama_debug_graph_steps(crabml_hip_llama_t* ctx, size_t pos, int32_t* steps, int32_t* captured);
 /* parity hook: copies the layer's K or V cache (raw f16/f32 bytes, [n_kv_heads][seq_len][head_dim]) */
 int crabml_hip_llama_debug_kv(crabml_hip_llama_t* ctx, size_t layer, int32_t which_v, void* dst, size_t nbytes);
 

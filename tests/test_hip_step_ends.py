@@ -25,7 +25,11 @@ WIDE = synth.ModelShape("wide", 4352, 512, 1, 34, 2, 600, 64, 1e-5, None)
 @pytest.mark.parametrize("fmt,shape", [("Q4_0", "tiny-hd128"), ("Q8_0", "15m"), ("Q4_1", "tiny-hd128"), ("Q4_K", "tiny-hd128"), ("Q4_K", "tiny-gqa"), ("F16", "15m"),
                                        ("Q5_K", "tiny-gqa"), ("F32", "tiny-gqa"), ("Q6_K", "tiny-gqa"), ("Q4_0", WIDE), ("Q4_K", WIDE), ("F16", WIDE)])
 @pytest.mark.parametrize("strict", [False, True])
-def test_greedy_runs_equal_single_steps(ca, fmt, shape, strict):
+@pytest.mark.parametrize("now", [False, True])
+def test_greedy_runs_equal_single_steps(ca, monkeypatch, fmt, shape, strict, now):
+    if now:  # several steps a graph from the first run on
+        monkeypatch.setenv("CRABML_HIP_TEST_HOOKS", "1")
+        monkeypatch.setenv("CRABML_HIP_GRAPH_STEPS", "1")
     dev = ca.HipTensorDevice(0, strict_order=strict)
     model = synth.build_model(shape if isinstance(shape, synth.ModelShape) else synth.SHAPES[shape], synth.TYPE_BY_NAME[fmt], seed=21)
     conf, w = synth.to_hip(model, dev)
@@ -123,3 +127,21 @@ def test_a_step_by_itself_has_one_front(ca, fmt, shape):
     r.decode_greedy(9, 4)
     assert sum(x["launches"] for x in dev.prof_read() if x["stage"] == 6) == 4
     dev.prof_enable(False)
+
+
+@pytest.mark.parametrize("fmt,shape", [("Q8_0", "15m"), ("Q4_K", "tiny-hd128")])
+def test_a_runner_captures_several_steps_when_runs_have_earned_it(ca, fmt, shape):
+    """none when it is made, none for short answers, and the same tokens before and behind"""
+    dev = ca.HipTensorDevice(0)
+    conf, w = synth.to_hip(synth.build_model(synth.SHAPES[shape], synth.TYPE_BY_NAME[fmt], seed=23), dev)
+    a, e = ca.HipLlamaRunner(conf, w, dev, 400, True), ca.HipLlamaRunner(conf, w, dev, 400, True, False)
+    assert [a.debug_graph_steps(p) for p in (0, 100, 399)] == [(8, False)] * 3 and e.debug_graph_steps(0) == (1, False)
+    token = 3
+    for n, captured in ((10, False), (9, False), (200, True), (20, True)):  # (a token makes at least 12 launches, 31 with 6 layers)
+        ids = a.decode_greedy(token, n)
+        assert ids == e.decode_greedy(token, n), n
+        token = ids[-1]
+        if n != 20:
+            assert any(a.debug_graph_steps(p)[1] for p in (0, 100, 399)) == captured, n
+    x, y = a.forward(token, 239), e.forward(token, 239)
+    assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
