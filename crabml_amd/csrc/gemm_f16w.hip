@@ -581,12 +581,13 @@ bool gemm_f16w_covers(uint32_t w_dtype, uint32_t act_qtype) {
 static int f16w_col_tiles_per_wave(size_t b, int variant) { return (variant & 512) ? 4 : (variant & 16) ? 8 : b <= 32 ? 2 : b <= 64 ? 4 : 8; }
 template <int WF>
 static bool launch_f16w_fmt(crabml_hip_device* dev, const F16wMats& mats, int row_tiles, size_t k, const void* xh, size_t b, int ksplit, int F,
-                            int variant, bool gu, int T) {
+                            int variant, bool gu, int T, int NW) {
   if (gu) {
     switch (T) {
       case 2: return launch_f16w_t<WF, 2, 2, true>(dev, mats, row_tiles, k, xh, b, 1);
       case 4: return launch_f16w_t<WF, 2, 4, true>(dev, mats, row_tiles, k, xh, b, 1);
-      default: return launch_f16w_t<WF, 2, 8, true, 8>(dev, mats, row_tiles, k, xh, b, 1);
+      default:
+        return NW == 8 ? launch_f16w_t<WF, 2, 8, true, 8>(dev, mats, row_tiles, k, xh, b, 1) : launch_f16w_t<WF, 2, 8, true>(dev, mats, row_tiles, k, xh, b, 1);
     }
   }
   switch (T) {
@@ -594,6 +595,17 @@ static bool launch_f16w_fmt(crabml_hip_device* dev, const F16wMats& mats, int ro
     case 4: return F == 2 ? launch_f16w_t<WF, 2, 4>(dev, mats, row_tiles, k, xh, b, ksplit) : launch_f16w_t<WF, 1, 4>(dev, mats, row_tiles, k, xh, b, ksplit);
     default: return F == 2 ? launch_f16w_t<WF, 2, 8>(dev, mats, row_tiles, k, xh, b, ksplit) : launch_f16w_t<WF, 1, 8>(dev, mats, row_tiles, k, xh, b, ksplit);
   }
+}
+// gate | up in full tiles: eight waves share a B' tile, which halves what the launch reads of B' (every row tile reads all of it, a gigabyte for 512
+// rows of 4096) and the staging a wave does -- one workgroup a CU, where those of four waves lie two on a CU.  It pays where the last round of CUs is
+// nearly full; into a part-empty one the smaller workgroups, which then have a CU each, fit better.  A whole pass of 3 layers, eight waves / four, by
+// rounds of CUs (128-row tiles / CUs): 0.5 1.00 to 1.04, 0.67 1.00 to 1.02, 0.75 0.96 to 1.00, 0.875 0.96 to 0.99, 1.0 0.98 to 1.01, 1.25 to 1.5 1.03 to
+// 1.10, 1.75 0.96 to 0.98, 2.0 0.97 to 1.01, 2.2 1.03 to 1.04, 2.6 0.97 to 0.99, 3.5 0.99 (Q8_0), 1.00, 1.015 (Q4_K, whose unpacking hides
+// less of the longer barrier).  (14336 rows of 4096, one launch of 300 rows: Q4_K 137 us with eight waves, 123 with four.)
+static bool f16w_eight_waves(uint32_t dt, size_t tiles, size_t n_cu) {
+  const size_t rounds = (tiles + n_cu - 1) / n_cu;
+  if (dt == CRABML_HIP_Q4_K && rounds > 3) return false;
+  return rounds == 1 ? 4 * tiles >= 3 * n_cu : 20 * tiles >= 17 * rounds * n_cu;
 }
 // nw weight matrices (one format, the same k) against the same rhs rows: out[j] (b, m[j]) = W[j] . x
 // ws (nullable), ws_floats: scratch for split launches.  When the output tiles alone leave the chip underfilled -- wo / ffn_down (few
@@ -635,11 +647,9 @@ bool launch_gemm_f16w(crabml_hip_device* dev, const crabml_hip_buf* const* w, co
   const bool gu = gu_exp_tab != nullptr && gu_done != nullptr && nw == 2 && m[0] == m[1] && !(variant & 64) &&
                   ((m[0] + 63) / 64) * col128 * 2 >= (size_t)dev->n_cu * 3;
   if (gu) F = 2;
-  // gate | up in full tiles: eight waves share a B' tile, which halves what the launch reads of B' (every row tile reads all of it, a
-  // gigabyte for 512 rows of 4096) and the staging a wave does.  512 rows, Q4_0 183 -> 173 us, the whole request 3973 -> 3785; Q4_K, 1024 rows a
-  // pass, 0.6 % of the request.  The other launches, cut in k to fill the chip with the smaller tiles, do not gain (ffn_down 115 -> 108,
-  // wo 35 -> 44); four fragments a wave, one wave a SIMD, lose (183 -> 211).
-  const int NW = gu && T == 8 ? 8 : 4;
+  // (gate | up alone.  512 rows, Q4_0 183 -> 173 us, the whole request 3973 -> 3785.  The other launches, cut in k to fill the chip with the smaller
+  // tiles, do not gain: ffn_down 115 -> 108, wo 35 -> 44; four fragments a wave, one wave a SIMD, lose: 183 -> 211.)
+  const int NW = gu && T == 8 && f16w_eight_waves(dt, (m[0] + 127) / 128 * col128, (size_t)dev->n_cu) ? 8 : 4;
   F16wMats mats{};
   mats.exp_tab = gu_exp_tab;
   const bool hquant = gu && hq != nullptr && hq->planes != nullptr && m[0] % 32 == 0;
@@ -678,15 +688,15 @@ bool launch_gemm_f16w(crabml_hip_device* dev, const crabml_hip_buf* const* w, co
       ksplit *= 2;
   bool ok;
   if (dt == CRABML_HIP_Q8_0)
-    ok = launch_f16w_fmt<WF_Q8_0>(dev, mats, row_tiles, k, xh, b, ksplit, F, variant, gu, T);
+    ok = launch_f16w_fmt<WF_Q8_0>(dev, mats, row_tiles, k, xh, b, ksplit, F, variant, gu, T, NW);
   else if (dt == CRABML_HIP_Q4_K)
-    ok = launch_f16w_fmt<WF_Q4_K>(dev, mats, row_tiles, k, xh, b, ksplit, F, variant, gu, T);
+    ok = launch_f16w_fmt<WF_Q4_K>(dev, mats, row_tiles, k, xh, b, ksplit, F, variant, gu, T, NW);
   else if (dt == CRABML_HIP_Q6_K)
-    ok = launch_f16w_fmt<WF_Q6_K>(dev, mats, row_tiles, k, xh, b, ksplit, F, variant, gu, T);
+    ok = launch_f16w_fmt<WF_Q6_K>(dev, mats, row_tiles, k, xh, b, ksplit, F, variant, gu, T, NW);
   else if (dt == CRABML_HIP_Q4_1)
-    ok = launch_f16w_fmt<WF_Q4_1>(dev, mats, row_tiles, k, xh, b, ksplit, F, variant, gu, T);
+    ok = launch_f16w_fmt<WF_Q4_1>(dev, mats, row_tiles, k, xh, b, ksplit, F, variant, gu, T, NW);
   else
-    ok = launch_f16w_fmt<WF_Q4_0>(dev, mats, row_tiles, k, xh, b, ksplit, F, variant, gu, T);
+    ok = launch_f16w_fmt<WF_Q4_0>(dev, mats, row_tiles, k, xh, b, ksplit, F, variant, gu, T, NW);
   if (ok && gu) *gu_done = hquant ? 2 : 1;
   if (ok && ksplit > 1 && defer_parts != nullptr && nw == 1) {
     *defer_parts = ksplit - 1;  // the caller's next row kernel adds the pieces (ws + s * b * m, s = 0 ..) in the same order
@@ -708,3 +718,9 @@ void launch_add_parts(hipStream_t st, float* out, const float* ws, size_t n, int
 }
 
 }  // namespace crabml_hip
+
+extern "C" int crabml_hip_debug_gateup_waves(uint32_t dtype, size_t hidden, size_t rows, int32_t n_cu, int32_t* waves) {
+  if (!waves || n_cu < 1) return CRABML_HIP_BAD_INPUT;
+  *waves = crabml_hip::f16w_eight_waves(dtype, (hidden + 127) / 128 * ((rows + 127) / 128), (size_t)n_cu) ? 8 : 4;
+  return 0;
+}

@@ -60,6 +60,8 @@ int crabml_hip_debug_rhs_rows(size_t m, size_t* rows);
 /* Steps of a greedy run that go into one graph where one step is `nodes` launches, and whether `done` steps -- made one at a time so far or about to be --
  * have earned its capture.  Host only. */
 int crabml_hip_debug_graph_steps(size_t nodes, size_t seq_len, size_t done, int32_t* steps, int32_t* earned);
+/* Waves of a workgroup of the fast prompt pass's gate | up launch over `rows` > 64 rows.  Host only. */
+int crabml_hip_debug_gateup_waves(uint32_t dtype, size_t hidden, size_t rows, int32_t n_cu, int32_t* waves);
 /* Bytes that a step's attention or mixer launch touches ahead of the linear behind it: m rows, `rows` of them a workgroup, row_bytes + row_bytes2 a row.
  * Host only. */
 int crabml_hip_debug_prefetch(int32_t m, int32_t rows, size_t row_bytes, size_t row_bytes2, size_t* bytes);

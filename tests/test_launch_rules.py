@@ -67,3 +67,16 @@ def test_a_capture_is_bounded_and_earned():
             assert first * 7 * (n - 1) / n >= 1.4 * nodes * n, (nodes, n, first)
     assert graph_steps(23, 400, 16) == (8, False) and graph_steps(123, 400, 64) == (3, False)  # (a short answer, a deeper model)
     assert graph_steps(23, 400, 200) == (8, True)
+
+
+Q4_0, Q8_0, Q4_K = 2, 8, 12
+
+
+@pytest.mark.parametrize("dtype,hidden,rows,waves", [
+    (Q4_K, 14336, 300, 4), (Q8_0, 14336, 300, 4), (Q4_0, 14336, 384, 4), (Q4_0, 14336, 640, 4), (Q8_0, 11008, 450, 4), (Q4_0, 8192, 700, 4), (Q4_0, 8192, 200, 4),
+    (Q4_K, 14336, 1024, 4), (Q4_0, 14336, 130, 8), (Q4_K, 14336, 256, 8), (Q8_0, 14336, 512, 8), (Q4_0, 14336, 768, 8), (Q8_0, 14336, 1024, 8), (Q4_0, 8192, 300, 8)])
+def test_gate_up_takes_eight_waves_where_they_won(dtype, hidden, rows, waves):
+    """sizes at which both were timed"""
+    n = ctypes.c_int32()
+    assert lib.crabml_hip_debug_gateup_waves(dtype, ctypes.c_size_t(hidden), ctypes.c_size_t(rows), 256, ctypes.byref(n)) == 0
+    assert n.value == waves
