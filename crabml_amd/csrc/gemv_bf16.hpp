@@ -208,8 +208,9 @@ __device__ __forceinline__ void rows16_out(const GemvBf16& a, int row, int b, fl
 
 #define GEMV_BF16_LDS_FLOATS 8192  // rhs elements staged at a time, all rows together: a cut segment is a multiple of the steps in flight
 
-// UN: steps of 512 in flight; NT: weights nontemporal (GemvBf16::resident)
-template <int NB, int R, int UN, int IN, int OUT, bool NT>
+// UN: steps of 512 in flight; NT: weights nontemporal (GemvBf16::resident); ROLL: a step's registers are refilled as soon as it has been used, else all
+// of them are asked for together in front of the products
+template <int NB, int R, int UN, int IN, int OUT, bool NT, bool ROLL>
 __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
   extern __shared__ __attribute__((aligned(16))) float gemv_lds[];  // [NB][2][seg / 2]
   __shared__ float red[4][NB];
@@ -298,8 +299,8 @@ __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
       }
     }
     __syncthreads();
-    // UN steps; MORE: a step's registers take the one UN steps further as soon as it has been used.  (A check a step would end the loads in flight.)
-    auto steps = [&](auto Mc, int k0) {
+    // UN steps; MORE: a step's registers take the one UN steps further.  (A check a step would end the loads in flight.)
+    auto steps = [&](auto Mc, int k0, const i32x4 (&w)[UN][R]) {
 #pragma unroll
       for (int u = 0; u < UN; u++) {
         const int k = k0 + u * 512 + lane * 8;
@@ -313,7 +314,7 @@ __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
               float s = acc[r][b];
 #pragma unroll
               for (int e = 0; e < 2; e++) {
-                const unsigned p = (unsigned)wv[u][r][e], p2 = (unsigned)wv[u][r][e + 2];
+                const unsigned p = (unsigned)w[u][r][e], p2 = (unsigned)w[u][r][e + 2];
                 s = __builtin_fmaf(__builtin_bit_cast(float, p << 16), x0[2 * e], s);
                 s = __builtin_fmaf(__builtin_bit_cast(float, p & 0xffff0000u), x0[2 * e + 1], s);
                 s = __builtin_fmaf(__builtin_bit_cast(float, p2 << 16), x1[2 * e], s);
@@ -327,10 +328,24 @@ __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
       }
     };
     for (int k0 = 0; k0 < n; k0 += UN * 512) {
-      if (s0 + k0 + UN * 512 < a.K)
-        steps(std::true_type{}, k0);
-      else
-        steps(std::false_type{}, k0);
+      const bool more = s0 + k0 + UN * 512 < a.K;
+      if constexpr (ROLL) {
+        if (more)
+          steps(std::true_type{}, k0, wv);
+        else
+          steps(std::false_type{}, k0, wv);
+      } else {
+        i32x4 cur[UN][R];
+#pragma unroll
+        for (int u = 0; u < UN; u++)
+#pragma unroll
+          for (int r = 0; r < R; r++) cur[u][r] = wv[u][r];
+        if (more) {
+#pragma unroll
+          for (int u = 0; u < UN; u++) request(u, s0 + k0 + UN * 512);
+        }
+        steps(std::false_type{}, k0, cur);
+      }
     }
   }
   float scale[NB];
@@ -720,16 +735,20 @@ inline void launch_gemv16_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, 
   a.resident ? launch_gemv16_n<SPL, IN, OUT, false>(st, rec, a, n_cu) : launch_gemv16_n<SPL, IN, OUT, true>(st, rec, a, n_cu);
 }
 
-template <int NB, int R, int IN, int OUT, int UN = NB >= 8 ? 2 : 4>
+template <int NB, int R, int IN, int OUT, int UN = NB >= 8 ? 2 : 4, bool ROLL = true>
 inline void launch_gemv_bf16_t(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a) {
   const int cap = GEMV_BF16_LDS_FLOATS / NB, seg = a.K < cap ? a.K : cap;
-  launch_k(st, rec, a.resident ? k_gemv_bf16<NB, R, UN, IN, OUT, false> : k_gemv_bf16<NB, R, UN, IN, OUT, true>,
+  launch_k(st, rec, a.resident ? k_gemv_bf16<NB, R, UN, IN, OUT, false, ROLL> : k_gemv_bf16<NB, R, UN, IN, OUT, true, ROLL>,
            dim3((a.N + 4 * R - 1) / (4 * R), (a.nb + NB - 1) / NB), dim3(256), (size_t)NB * seg * sizeof(float), a);
 }
 // One row of the rhs: what bounds it is how early the weights are asked for, so a wave has 8 to 16 KB of them on their way while it stages
 // the rhs: four rows a wave where they still fill the chip (all of 2048 columns at once: gate | up of 16384 x 2048 15.0 -> 13.5 us against half
 // of them; 11264 x 2048 and 8192 x 2048 are better with two rows, 10.2 / 11.5 and 8.2 / 9.2), one row and twice the steps for few rows of
 // many columns (2048 x 8192 9.4 -> 8.5, 2048 x 4096 6.5 -> 6.3, against two rows).
+// Two rows: where the columns are more than the steps in flight, the next ones are asked for together -- one by one, each behind twice the products, they
+// come too late (8192 .. 32000 x 4096 with the norm inside 33.2 -> 32.1, 43.3 -> 42.4, 14.75 -> 14.6 us, 2048 / 4096 x 8192 11.15 -> 11.0, 15.85 -> 15.6; with up to
+// 2048 columns the copy costs 13.1 against 11.9, 25.6 / 23.0).  A tail that is scaled and streams have more to do beside: 2048 x 4096 8.1 / 7.75,
+// 2048 x 8192 11.0 / 10.7 with the refill step by step.
 // rows of the rhs that share one pass over the weights: as many as there are, up to 8
 template <int IN, int OUT>
 inline void launch_gemv_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a) {
@@ -746,6 +765,9 @@ inline void launch_gemv_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, co
         launch_gemv_bf16_t<1, 1, IN, OUT>(st, rec, a);
     }
   } else if (a.nb <= 2) {
+    if constexpr (IN != GEMV_IN_SPLIT && OUT != GEMV_OUT_STREAMS) {
+      if (a.K > 4 * 512) return launch_gemv_bf16_t<2, 2, IN, OUT, 4, false>(st, rec, a);
+    }
     launch_gemv_bf16_t<2, 2, IN, OUT>(st, rec, a);
   } else if (a.nb <= 4) {
     launch_gemv_bf16_t<4, 2, IN, OUT>(st, rec, a);

@@ -40,3 +40,18 @@ def test_batched_steps(ca, hdev, tmp_path, design, width, ff, vocab, f32):
             d = got[:, i] - want[i]
             # the bounds of the designs' own tests
             assert np.sqrt((d * d).mean(axis=1)).max() <= (2e-5 if f32 else 2.5e-2) * np.sqrt((want[i] ** 2).mean()), (batch, i)
+
+
+# columns: those of the steps in flight, one octet more; one staged segment of one row, of two, of eight (8192, 4096, 1024 elements), and one octet more
+@pytest.mark.parametrize("m,k", [(70, 2048), (70, 2056), (515, 4096), (33, 4104), (66, 8200), (17, 1032), (16389, 2056)])
+def test_row_kernels_over_long_rows(ca, hdev, m, k):
+    rng = np.random.default_rng(k + m)
+    bits = sh.to_bf16(rng.standard_normal((m, k)).astype(np.float32))
+    w = sh.from_bf16(bits).astype(np.float64)
+    t = ca.HipTensor.from_cpu(bits.view(np.uint8).reshape(-1), [m, k], ca.GGMLType.BF16, hdev)
+    for b in (1, 2, 3, 5, 8, 9, 16):
+        x = rng.standard_normal((b, k)).astype(np.float32)
+        got = t.matmul_vec(ca.HipTensor.new(x.reshape(-1), [b, k], hdev)).export().reshape(b, m)
+        # (f32 sums of k products, k / 64 of them in a lane's chain: 2 + k / 64 roundings of 2^-24 each at the most, of the products' absolute values)
+        bound = (2 + k / 64) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T)
+        assert (np.abs(got - x.astype(np.float64) @ w.T) <= bound).all(), b
