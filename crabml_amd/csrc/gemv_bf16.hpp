@@ -749,6 +749,8 @@ inline void launch_gemv_bf16_t(hipStream_t st, crabml_hip_device::ProfRec* rec, 
 // come too late (8192 .. 32000 x 4096 with the norm inside 33.2 -> 32.1, 43.3 -> 42.4, 14.75 -> 14.6 us, 2048 / 4096 x 8192 11.15 -> 11.0, 15.85 -> 15.6; with up to
 // 2048 columns the copy costs 13.1 against 11.9, 25.6 / 23.0).  A tail that is scaled and streams have more to do beside: 2048 x 4096 8.1 / 7.75,
 // 2048 x 8192 11.0 / 10.7 with the refill step by step.
+// Eight rows (matmul_vec): the same, and more so: step by step 8192 x 2048 15.1 us against 9.9, 8192 x 8192 49.1 / 32.0, 32000 x 2048 49.4 / 39.4.  Four rows: step by
+// step 8.0 -> 7.4, 26.3 -> 23.6, 26.6 -> 23.7.
 // rows of the rhs that share one pass over the weights: as many as there are, up to 8
 template <int IN, int OUT>
 inline void launch_gemv_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a) {
@@ -772,7 +774,7 @@ inline void launch_gemv_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, co
   } else if (a.nb <= 4) {
     launch_gemv_bf16_t<4, 2, IN, OUT>(st, rec, a);
   } else {
-    launch_gemv_bf16_t<8, 2, IN, OUT>(st, rec, a);
+    launch_gemv_bf16_t<8, 2, IN, OUT, 2, false>(st, rec, a);
   }
 }
 
