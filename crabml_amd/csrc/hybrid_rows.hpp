@@ -201,8 +201,9 @@ struct AttnTile {
 // matrix instruction stands for key 4 (lane / 16) + i of a 16-key group, and V^T is read from LDS in the same order.  Scores live in
 // the log2 domain.
 // KP: waves that share query rows; wave w + 4 takes the second half of a tile's keys, and the two meet once, at the end.
+// (Waves a SIMD: left to itself the compiler takes 366 registers for heads of 128 in f32, one workgroup a CU: 48 heads, 900 rows 484 us against 407 with 208.)
 template <typename T, int KC, int VC, int P, bool LAT, int RT, int KP>
-__global__ __launch_bounds__(256 * KP, sizeof(T) == 2 ? (KP == 2 && KC <= 128 ? 4 : RT == 1 && KC <= 128 ? 3 : 2) : 1) void k_attn_rows(const MixRows<T> a) {
+__global__ __launch_bounds__(256 * KP, sizeof(T) == 2 ? (KP == 2 && KC <= 128 ? 4 : RT == 1 && KC <= 128 ? 3 : 2) : KC <= 128 ? 2 : 1) void k_attn_rows(const MixRows<T> a) {
   typedef AttnTile<T, KC, VC> A;
   constexpr int KT = A::KT, LK = KC + A::PAD, LV = KT + A::PAD, VT = VC / 16, ST = KT / 16 / KP, NTH = 256 * KP;
   constexpr int NK = KT * KC / 8 / NTH, NV = KT * VC / 8 / NTH;  // octets of K and of V per thread and tile

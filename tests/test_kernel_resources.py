@@ -32,3 +32,22 @@ def test_no_kernel_uses_scratch_or_spills(tmp_path):
                     bad.append((os.path.basename(o), m.group(1), int(m.group(2)), int(m.group(3))))
     assert n_kernels > 100, n_kernels
     assert not bad, bad
+
+
+@pytest.mark.skipif(not os.path.exists(os.path.join(LLVM, "llvm-objdump")), reason="needs the ROCm llvm tools")
+def test_prompt_attention_keeps_its_workgroups_on_a_cu(tmp_path):
+    """The hybrid decoder's prompt attention lives on the other workgroups of a CU while one waits for its tile: registers for two waves a SIMD at least (256
+    a lane, both files together), heads of up to 128 columns in f32 among them.  (With one, 48 heads of 128, 900 rows took 484 us for 407.)"""
+    obj = os.path.join(ROOT, "build", "obj", "hybrid.o")
+    if not os.path.exists(obj):
+        pytest.skip("objects not built (run __graft_entry__.build())")
+    local = tmp_path / "hybrid.o"
+    shutil.copy(obj, local)
+    subprocess.run([os.path.join(LLVM, "llvm-objdump"), "--offloading", str(local)], capture_output=True, cwd=tmp_path)
+    seen = {}
+    for co in glob.glob(str(local) + ".*amdgcn*"):
+        notes = subprocess.run([os.path.join(LLVM, "llvm-readelf"), "--notes", co], capture_output=True, text=True).stdout
+        for m in re.finditer(r"\.name:\s+\S*k_attn_rowsI([ft])Li(\d+)E\S*.*?\.vgpr_count:\s+(\d+)", notes, flags=re.S):
+            seen[m.group(1), int(m.group(2))] = max(seen.get((m.group(1), int(m.group(2))), 0), int(m.group(3)))
+    assert {("f", 64), ("f", 128), ("t", 64), ("t", 128), ("t", 192), ("t", 256)} <= set(seen)
+    assert all(n <= 256 for k, n in seen.items() if k != ("f", 256)), seen
