@@ -169,6 +169,7 @@ struct crabml_hip_llama {
     size_t single = 0;      // greedy steps made one at a time
   } several[4];
   bool graph_steps_now = false;  // test hook: from the first run on
+  size_t weight_bytes = 0;       // of the matrices that a step reads
   bool use_graph = false;
   bool capturing = false;
   bool chains = false;  // steps can follow each other on this device without the host: several in one graph
@@ -366,6 +367,7 @@ void launch_attn_flash(crabml_hip_llama* c, int l, signed char* xq, unsigned sho
   if (prof) prof_end(dev, &r[1]);
 }
 
+bool runs_attn_short(const crabml_hip_llama* c) { return c->attn_variant == 3 || (c->attn_variant == 0 && c->attn_short_from == 0); }
 void enqueue_attention(crabml_hip_llama* c, int l, signed char* xq, unsigned short* xd, void* xisum, const PrefetchPlan& pf,
                        int spare, bool prof, const AttnQ8K* k8 = nullptr) {
   crabml_hip_device* dev = c->dev;
@@ -375,7 +377,7 @@ void enqueue_attention(crabml_hip_llama* c, int l, signed char* xq, unsigned sho
   const int* pos_d = c->state + 1;
   crabml_hip_device::ProfRec ar{};
   crabml_hip_device::ProfRec* AR = prof ? &ar : nullptr;
-  if (c->attn_variant == 3 || (c->attn_variant == 0 && c->attn_short_from == 0)) {
+  if (runs_attn_short(c)) {
     if (prof) prof_begin(dev, &ar, CRABML_HIP_F32, 7, 0.0);
     launch_k(st, AR, attn_short_kernel(hd), dim3(n_heads + spare), dim3(512), 0, (const float*)c->qbuf, (const unsigned short*)c->kc[l], (const unsigned short*)c->vc[l],
              pos_d, c->attn, xq, xd, xisum, n_heads, n_kv, hd, seq_cap, pf, c->qt == CRABML_HIP_Q8_1 ? 1 : 0);
@@ -476,7 +478,7 @@ PrefetchPlan prefetch_rows(const crabml_hip_llama* c, const crabml_hip_buf* w, i
   if ((c->cfg.flags & CRABML_HIP_LLAMA_NO_PREFETCH) || (w->dtype != CRABML_HIP_Q4_0 && w->dtype != CRABML_HIP_Q8_0 && w->dtype != CRABML_HIP_Q4_1))
     return PrefetchPlan{};
   const size_t blocks = w->k / 32;
-  return prefetch_matrix((int)w->m, rows, w->ptr, blocks * (w->dtype == CRABML_HIP_Q8_0 ? 32 : 16), (const char*)w->ptr + w->wl.off_scale,
+  return prefetch_matrix(c->weight_bytes, runs_attn_short(c) ? PREFETCH_MODEL : SIZE_MAX, (int)w->m, rows, w->ptr, blocks * (w->dtype == CRABML_HIP_Q8_0 ? 32 : 16), (const char*)w->ptr + w->wl.off_scale,
                          blocks * (w->dtype == CRABML_HIP_Q4_1 ? 4 : 2));
 }
 
@@ -2158,6 +2160,7 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
   c->token_embed = hold(w->token_embed);
   c->rms_final = hold(w->rms_final_weight);
   c->output = hold(outw);
+  c->weight_bytes = outw->wl.total;
   for (size_t l = 0; l < g.n_layers; l++) {
     c->rms_att.push_back(hold(w->rms_att_weight[l]));
     c->rms_ffn.push_back(hold(w->rms_ffn_weight[l]));
@@ -2168,6 +2171,7 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
     c->gate.push_back(hold(w->ffn_gate_weight[l]));
     c->down.push_back(hold(w->ffn_down_weight[l]));
     c->up.push_back(hold(w->ffn_up_weight[l]));
+    for (const auto* m : {c->wq[l], c->wk[l], c->wv[l], c->wo[l], c->gate[l], c->up[l], c->down[l]}) c->weight_bytes += m->wl.total;
   }
   auto A = [&](size_t bytes, void** p) {
     if (rc == 0) rc = dalloc(c, bytes, p);

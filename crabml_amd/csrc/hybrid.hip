@@ -458,7 +458,7 @@ void step_linear(Ctx* c, crabml_hip_device::ProfRec* rec, GemvBf16 g) {
 PrefetchPlan prefetch_out(const Ctx* c, const Layer& L, int B) {
   if (B <= 2 || c->weight_bytes <= RESIDENT_MALL) return PrefetchPlan{};
   const int rows = c->width >= 16384 ? 32 : 16;  // (a workgroup of launch_gemv16_bf16)
-  return prefetch_matrix(c->width, rows, L.w_o, (size_t)L.ldc * 2, nullptr, 0);
+  return prefetch_matrix(c->weight_bytes, PREFETCH_MODEL_HYBRID, c->width, rows, L.w_o, (size_t)L.ldc * 2, nullptr, 0);
 }
 
 MixStep mix_step(const Ctx* c, const Run& run, int B) {
@@ -1248,7 +1248,7 @@ int create_impl(Ctx* c, const crabml_hip_hybrid_layer_t* layers, const crabml_hi
   }
   {
     const char *h = getenv("CRABML_HIP_TEST_HOOKS"), *e = getenv("CRABML_HIP_STREAM_WEIGHTS");  // test hook: small models through the large ones' loads
-    if (h && h[0] == '1' && e && e[0] == '1') c->weight_bytes = SIZE_MAX;
+    if (h && h[0] == '1' && e && e[0] == '1') c->weight_bytes = RESIDENT_MALL + 1;
     const char* g = getenv("CRABML_HIP_GRAPH_STEPS");
     c->graph_steps_now = h && h[0] == '1' && g && g[0] == '1';
   }
@@ -1480,9 +1480,9 @@ extern "C" int crabml_hip_debug_graph_steps(size_t nodes, size_t seq_len, size_t
   *earned = crabml_hip::steps_graph_earned(nodes, *steps, done) ? 1 : 0;
   return 0;
 }
-extern "C" int crabml_hip_debug_prefetch(int32_t m, int32_t rows, size_t row_bytes, size_t row_bytes2, size_t* bytes) {
+extern "C" int crabml_hip_debug_prefetch(int32_t hybrid, size_t model_bytes, int32_t m, int32_t rows, size_t row_bytes, size_t row_bytes2, size_t* bytes) {
   if (!bytes || m < 1 || rows < 1) return CRABML_HIP_BAD_INPUT;
-  const crabml_hip::PrefetchPlan pf = crabml_hip::prefetch_matrix(m, rows, nullptr, row_bytes, nullptr, row_bytes2);
+  const crabml_hip::PrefetchPlan pf = crabml_hip::prefetch_matrix(model_bytes, hybrid ? crabml_hip::PREFETCH_MODEL_HYBRID : crabml_hip::PREFETCH_MODEL, m, rows, nullptr, row_bytes, nullptr, row_bytes2);
   *bytes = 0;
   for (int i = 0; i < pf.n; i++) *bytes += (size_t)pf.bytes[i] * pf.count[i];
   return 0;

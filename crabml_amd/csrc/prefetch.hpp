@@ -39,10 +39,17 @@ inline void prefetch_add(PrefetchPlan& pf, const void* p, size_t bytes, int firs
   pf.count[pf.n++] = count;
 }
 constexpr size_t PREFETCH_MOST = (size_t)32 << 20;  // what the L2s hold
+// Models whose steps read more than this (PREFETCH_MODEL behind k_attn_short; the hybrid decoder PREFETCH_MODEL_HYBRID) do without: the short hosts take
+// longer than the linear gains, probably because every XCD touches pages all over a matrix and from some 4 GB of weights on their addresses are not at hand
+// (32 layers of the 8B shape, 4.2 GB: attention 4.6 -> 5.9 us, wo 5.6 -> 4.6, a token 1257 -> 1285).  k_attn and k_attn_s take long enough to hide it: the
+// strict device at the same 32 layers 652 tokens/s without, 668 with.  A token with / without: 8B shape in Q4_0, 1.3 GB 0.987,
+// 2.3 GB 0.983, 3.2 GB 0.985, 4.2 GB 1.031; in Q8_0, 3.3 GB 0.991, 4.3 GB 1.019, 6.1 GB 1.025; width 3072, 1.8 GB 0.974.  Hybrid decoder of width 2048, 3 / 8 / 16
+// rows: 0.65 GB 1.01 / 0.97 / 0.99, 1.2 GB 1.01 / 0.97 / 1.01, 2.2 GB 1.03 / 1.00 / 1.03, 4.3 GB 1.05 / 1.00 / 1.00, of width 4096, 4.2 GB 1.04 / 1.04 / 1.04.
+constexpr size_t PREFETCH_MODEL = (size_t)3584 << 20, PREFETCH_MODEL_HYBRID = (size_t)1536 << 20;
 // a matrix of which the next launch's workgroups take `rows` of the m rows each: row_bytes a row from p, and row_bytes2 from p2 (scales; 0: none)
-inline PrefetchPlan prefetch_matrix(int m, int rows, const void* p, size_t row_bytes, const void* p2, size_t row_bytes2) {
+inline PrefetchPlan prefetch_matrix(size_t model_bytes, size_t model_most, int m, int rows, const void* p, size_t row_bytes, const void* p2, size_t row_bytes2) {
   PrefetchPlan pf{};
-  if ((size_t)m * (row_bytes + row_bytes2) > PREFETCH_MOST) return pf;
+  if (model_bytes > model_most || (size_t)m * (row_bytes + row_bytes2) > PREFETCH_MOST) return pf;
   prefetch_add(pf, p, row_bytes * rows, 0, m / rows);
   prefetch_add(pf, p2, row_bytes2 * rows, 0, m / rows);
   return pf;

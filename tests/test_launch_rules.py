@@ -42,9 +42,18 @@ def test_weights_touched_ahead_fit_the_l2s(row_bytes, row_bytes2):
     for rows in (2, 8, 16, 32):
         for m in (32, 2048, 4096, 7264, 8192, 32768, 1 << 20):
             n = ctypes.c_size_t()
-            assert lib.crabml_hip_debug_prefetch(m, rows, ctypes.c_size_t(row_bytes), ctypes.c_size_t(row_bytes2), ctypes.byref(n)) == 0
+            assert lib.crabml_hip_debug_prefetch(m & 1, ctypes.c_size_t(1 << 30), m, rows, ctypes.c_size_t(row_bytes), ctypes.c_size_t(row_bytes2), ctypes.byref(n)) == 0
             all_of_it = m * (row_bytes + row_bytes2)
             assert n.value == (all_of_it if all_of_it <= 32 << 20 else 0), (m, rows, n.value)
+
+
+@pytest.mark.parametrize("hybrid,gigabytes,touched", [(0, 1.3, True), (0, 2.3, True), (0, 3.34, True), (0, 4.22, False), (0, 6.1, False), (1, 0.65, True), (1, 1.2, True),
+                                                      (1, 2.2, False), (1, 4.2, False)])
+def test_weights_are_touched_ahead_where_that_won(hybrid, gigabytes, touched):
+    """sizes of models at which a step was timed with and without"""
+    n = ctypes.c_size_t()
+    assert lib.crabml_hip_debug_prefetch(hybrid, ctypes.c_size_t(int(gigabytes * 1e9)), 4096, 32, ctypes.c_size_t(2048), ctypes.c_size_t(256), ctypes.byref(n)) == 0
+    assert (n.value > 0) == touched
 
 
 def graph_steps(nodes, seq_len, done):
