@@ -701,12 +701,12 @@ int enqueue_segment_t(crabml_hip_llama* c, int seg) {
                  eps_next,
                  ad.q, ad.d, ad.isum, ng, k / 32, Planes6{nullptr, 0}, NoTp{});
     } else if (c->ord) {
-      launch_k(st, R, k_gemv_res_ord<FMT>, dim3((dim + 7) / 8), dim3(256), (size_t)8 * ((k / 32 + 3) & ~3) * sizeof(float), planes_of(w), act_view<FMT>(a),
+      launch_k(st, R, k_gemv_res_ord<FMT>, dim3((dim + RES_ORD_ROWS - 1) / RES_ORD_ROWS), dim3(256), (size_t)8 * ((k / 32 + 3) & ~3) * sizeof(float), planes_of(w), act_view<FMT>(a),
                c->x, dim, k / 32);
     } else if (tp) {
-      launch_k(st, R, k_gemv_res<FMT, 1, false>, dim3((dim + 1) / 2), dim3(128), 0, planes_of(w), act_view<FMT>(a), dst, dim, k / 32);
+      launch_k(st, R, k_gemv_res<FMT, 1, false>, dim3((dim + RES_ROWS - 1) / RES_ROWS), dim3(128), 0, planes_of(w), act_view<FMT>(a), dst, dim, k / 32);
     } else {
-      launch_k(st, R, k_gemv_res<FMT, 1, true>, dim3((dim + 1) / 2), dim3(128), 0, planes_of(w), act_view<FMT>(a), dst, dim, k / 32);
+      launch_k(st, R, k_gemv_res<FMT, 1, true>, dim3((dim + RES_ROWS - 1) / RES_ROWS), dim3(128), 0, planes_of(w), act_view<FMT>(a), dst, dim, k / 32);
     }
     CH_TRY(P1(&pr));
     return 0;
@@ -769,7 +769,7 @@ int enqueue_segment_t(crabml_hip_llama* c, int seg) {
     CH_TRY(P1(&pr));
     // attention (llama2.rs:571-590) -> attn (f32) [+ Q8_0 planes for wo]; spare CUs prefetch wo
     const bool attn_quant = (hd % 32) == 0;
-    const PrefetchPlan wo = prefetch_rows(c, c->wo[l], norm_epi ? 32 / split_of(dim_l) : 2);
+    const PrefetchPlan wo = prefetch_rows(c, c->wo[l], res_rows(norm_epi, c->ord, split_of(dim_l)));
     enqueue_attention(c, l, attn_quant ? aa.q : (signed char*)nullptr, aa.d, aa.isum, wo, dev->n_cu > n_heads_l ? dev->n_cu - n_heads_l : 0, prof);
     // heads that are not whole quant blocks (head width 48 of the 15M-parameter model): wo's launch quantizes the row itself -- the same bits, one
     // launch fewer per layer (2 us of quantizer and its boundary: 7.46 -> 7.05 ms for 57 tokens of that model)
@@ -1070,9 +1070,9 @@ int enqueue_segment_k(crabml_hip_llama* c, int seg) {
       }
     }
     if (tp)
-      launch_k(st, R, k_gemv_res<FMT, 1, false>, dim3((dim + 1) / 2), dim3(128), 0, planes_k(w), a, dst, dim, k / BE);
+      launch_k(st, R, k_gemv_res<FMT, 1, false>, dim3((dim + RES_ROWS - 1) / RES_ROWS), dim3(128), 0, planes_k(w), a, dst, dim, k / BE);
     else
-      launch_k(st, R, k_gemv_res<FMT, 1, true>, dim3((dim + 1) / 2), dim3(128), 0, planes_k(w), a, dst, dim, k / BE);
+      launch_k(st, R, k_gemv_res<FMT, 1, true>, dim3((dim + RES_ROWS - 1) / RES_ROWS), dim3(128), 0, planes_k(w), a, dst, dim, k / BE);
     return P1();
   };
 
@@ -2632,6 +2632,12 @@ int crabml_hip_llama_debug_graphs(crabml_hip_llama_t* c, size_t pos, int32_t* fo
   *form = variant_of(c, pos);
   *captured = 0;
   for (int v = 0; v < 4; v++) *captured |= c->exec[v] ? 1u << v : 0u;
+  return 0;
+}
+
+int crabml_hip_debug_residual_rows(int32_t norm_epilogue, int32_t ordered, int32_t split, int32_t* rows) {
+  if (!rows || (split != 1 && split != 2)) return CRABML_HIP_BAD_INPUT;
+  *rows = res_rows(norm_epilogue != 0, ordered != 0, split);
   return 0;
 }
 

@@ -26,6 +26,10 @@ __global__ __launch_bounds__(128) void k_gemv_res(Planes w, typename ActOf<FMT>:
   }
 }
 
+// rows of wo / ffn_down that a workgroup takes: with the norm behind them a 32-row chunk or half of one (k_gemv_res_nq); k_gemv_res_ord; k_gemv_res.  (What
+// the attention launch touches ahead is cut the same way.)
+constexpr int RES_ORD_ROWS = 8, RES_ROWS = 2;
+inline int res_rows(bool norm_epi, bool ord, int split) { return norm_epi ? 32 / split : ord ? RES_ORD_ROWS : RES_ROWS; }
 // strict order: x[row] = (the row's block terms added in block order) + x[row]; 4 waves x 2 rows, dynamic LDS = 8 * nt floats
 template <int FMT>
 __global__ __launch_bounds__(256) void k_gemv_res_ord(Planes w, typename ActOf<FMT>::type act, float* __restrict__ x, int m, int nb) {

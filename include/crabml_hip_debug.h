@@ -62,6 +62,9 @@ int crabml_hip_debug_rhs_rows(size_t m, size_t* rows);
 int crabml_hip_debug_graph_steps(size_t nodes, size_t seq_len, size_t done, int32_t* steps, int32_t* earned);
 /* Waves of a workgroup of the fast prompt pass's gate | up launch over `rows` > 64 rows.  Host only. */
 int crabml_hip_debug_gateup_waves(uint32_t dtype, size_t hidden, size_t rows, int32_t n_cu, int32_t* waves);
+/* Rows of wo / ffn_down that a workgroup of a llama step takes: with the next norm in the launch or without, block-ordered sums (strict device), one or two
+ * workgroups a 32-row chunk.  The launch's grid and what attention touches ahead of it both come from this.  Host only. */
+int crabml_hip_debug_residual_rows(int32_t norm_epilogue, int32_t ordered, int32_t split, int32_t* rows);
 /* Bytes that a step's attention or mixer launch touches ahead of the linear behind it: m rows, `rows` of them a workgroup, row_bytes + row_bytes2 a row, in a
  * model (llama, hybrid) whose steps read model_bytes of weights.  Host only. */
 int crabml_hip_debug_prefetch(int32_t hybrid, size_t model_bytes, int32_t m, int32_t rows, size_t row_bytes, size_t row_bytes2, size_t* bytes);

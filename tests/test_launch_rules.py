@@ -56,6 +56,14 @@ def test_weights_are_touched_ahead_where_that_won(hybrid, gigabytes, touched):
     assert (n.value > 0) == touched
 
 
+def test_rows_of_the_residual_linears():
+    """k_gemv_res_nq: a chunk of 32 rows or half of one; k_gemv_res_ord: four waves of two rows; k_gemv_res: two waves of one"""
+    for args, want in {(1, 0, 1): 32, (1, 1, 1): 32, (1, 0, 2): 16, (1, 1, 2): 16, (0, 1, 1): 8, (0, 1, 2): 8, (0, 0, 1): 2, (0, 0, 2): 2}.items():
+        rows = ctypes.c_int32()
+        assert lib.crabml_hip_debug_residual_rows(*args, ctypes.byref(rows)) == 0
+        assert rows.value == want, args
+
+
 def graph_steps(nodes, seq_len, done):
     steps, earned = ctypes.c_int32(), ctypes.c_int32()
     assert lib.crabml_hip_debug_graph_steps(ctypes.c_size_t(nodes), ctypes.c_size_t(seq_len), ctypes.c_size_t(done), ctypes.byref(steps), ctypes.byref(earned)) == 0
