@@ -879,7 +879,8 @@ void launch_attn_cls(Ctx* c, crabml_hip_device::ProfRec* rec, MixRows<T> m, cons
     if (big) return launch_k(c->dev->stream, rec, k_attn_rows<T, KC, VC, P, LAT, 2, 1>, grid, dim3(256), 0, m);
   // Two waves share 16 query rows where the chain of key tiles is all there is: up to two such workgroups a CU (heads of 128, us, one wave / two: 16
   // heads 2048 rows 82 / 74, 1000 rows 42 / 34, 400 rows 22.7 / 21.1, 2048 rows in a window 52 / 48; more workgroups, 32 heads of
-  // 4 x 500 rows, 39 / 52; latent keys of 192 66 / 77).
+  // 4 x 500 rows, 39 / 52; latent keys of 192 66 / 77).  Heads of up to 64 have no such form: 512 threads would hold one octet of a V tile each,
+  // and V goes to LDS by pairs of keys.  Nor has f32 compute, whose tiles are half as many keys.
   if constexpr (sizeof(T) == 2 && KC == 128)
     if ((int)grid.x <= 2 * c->dev->n_cu) return launch_k(c->dev->stream, rec, k_attn_rows<T, KC, VC, P, LAT, 1, 2>, grid, dim3(512), 0, m);
   launch_k(c->dev->stream, rec, k_attn_rows<T, KC, VC, P, LAT, 1, 1>, grid, dim3(256), 0, m);

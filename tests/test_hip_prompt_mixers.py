@@ -3,7 +3,9 @@
 import numpy as np
 import pytest
 
+from crabml_amd import synth_bifazen as sb
 from crabml_amd import synth_hybrid as sh
+from tests import test_hip_bifazen as bifazen
 from tests.test_hip_hybrid import Model, close
 
 pytestmark = pytest.mark.gpu
@@ -45,7 +47,7 @@ def test_portions_and_neighbours(ca, hdev, linear, f32):
     close(got, np.concatenate([w[c:] for w, c in zip(want, cuts)]), f32)
 
 
-@pytest.mark.parametrize("heads,n", [("few", 51), ("few", 82), ("few", 83), ("few", 114), ("few", 115), ("few", 700), ("many", 895), ("many", 897), ("many", 1040)])
+@pytest.mark.parametrize("heads,n", [("few", 51), ("few", 82), ("few", 83), ("few", 114), ("few", 115), ("few", 700), ("many", 895), ("many", 897), ("many", 946), ("many", 947), ("many", 1040)])
 def test_query_tiles(ca, hdev, tmp_path, heads, n):
     m = Model(FEW_HEADS if heads == "few" else MANY_HEADS, tmp_path, seed=5)
     r = m.runner(ca, hdev, False, seq_len=1100)
@@ -53,3 +55,21 @@ def test_query_tiles(ca, hdev, tmp_path, heads, n):
     s = r.open()
     got = [r.step([(s, t[:50], list(range(50)))]), r.step([(s, t[50:], list(range(n - 50)))])]
     close(np.concatenate(got), m.oracle(t), False)
+
+
+# 64 heads: eight tiles of 128 rows and more go to the larger tiles -- with a latent key of up to 128 and of up to 192 columns, and in a window
+LATENT_128 = sb.config(64, 77, [sb.latent(64, 72, 20, 80, 32, 300, None)])
+LATENT_192 = sb.config(64, 77, [sb.latent(64, 120, 32, 104, 40, 1000, None)])
+WINDOW = sb.config(64, 77, [sb.attention(64, 2, 72, 80, 200, None)])
+
+
+@pytest.mark.parametrize("config", [LATENT_128, LATENT_192, WINDOW])
+@pytest.mark.parametrize("n", [946, 947, 1075])
+def test_query_tiles_of_latent_and_windowed_heads(ca, hdev, tmp_path, config, n):
+    """896, 897 and 1025 rows behind 50 that are in the cache: seven, eight and nine tiles, the last one whole, of one row and of one row"""
+    m = bifazen.Model(config, tmp_path, seed=6)
+    r = m.runner(ca, hdev, False, seq_len=1100)
+    t = m.tokens(n, seed=n)
+    s = r.open()
+    got = [r.step([(s, t[:50], list(range(50)))]), r.step([(s, t[50:], list(range(n - 50)))])]
+    bifazen.close(np.concatenate(got), m.oracle(t), False)
