@@ -127,7 +127,7 @@ struct crabml_hip_llama {
   char* act_attn = nullptr;  // Q8_0 planes of the attention output (dim_l)
   char* act_hid = nullptr;   // Q8_0 planes of the ffn hidden vector (hidden_l)
   float* rope = nullptr;     // [seq_len][npairs][2]
-  int* state = nullptr;      // token, pos, step, sink, serial (never reset), fault
+  int* state = nullptr;      // token, pos, step, (unused), serial (never reset), fault
   unsigned long long* slots = nullptr;  // dim/32 {chunk sum, epoch} granules of the norm epilogue
   unsigned long long* a8gran = nullptr;  // Q4_K layers: granules of the attention output (dim_l) and of h (hidden_l), through which
   unsigned long long* h8gran = nullptr;  // the producing kernels assemble Q8_K super-blocks (q8k_exchange_store)
@@ -1753,7 +1753,7 @@ int set_state(crabml_hip_llama* c, size_t token, size_t pos, int step, const uns
   st[0] = (int)token;
   st[1] = (int)pos;
   st[2] = step;
-  if (serial != nullptr) {  // token, pos, step, (prefetch sink), serial: the serial set from the host (lazy_ctx_begin)
+  if (serial != nullptr) {  // token, pos, step, (unused), serial: the serial set from the host (lazy_ctx_begin)
     int st5[5] = {st[0], st[1], st[2], 0, (int)*serial};
     // the ring slot holds 4 ints: the 5-int form takes two consecutive slots
     if (c->h_state_next == crabml_hip_llama::H_STATE_SLOTS) {

@@ -6,7 +6,7 @@
 // bits (split3): every f32 is the exact sum of its planes and every plane times a bf16 weight is exact in f32, so three planes give
 // true f32 products with f32 sums -- the weights ARE bf16 numbers -- at a fifth of the time the f32 matrix instruction would take.
 //
-// Mapping: BM x 128 output tile per workgroup (BM = 256: eight waves; else four), k in steps of 64.  A step's tiles go from memory
+// Mapping: BM x 128 output tile per workgroup (BM = 256 and 128: eight waves; else four), k in steps of 64.  A step's tiles go from memory
 // straight into LDS (global_load_lds, 16 bytes per lane); three or four steps are in LDS or on their way, and a wave waits for the oldest
 // only (s_waitcnt vmcnt(n)).  LDS holds rows of 128 bytes whose 16-byte chunks are permuted by (row / 2) % 8 -- on the SOURCE side, the LDS side of the instruction
 // being linear -- so that the 16 rows a fragment read touches spread over all 64 banks.  Operands are padded by their owners (k to 64,

@@ -1018,7 +1018,7 @@ int run_pass(Ctx* c, const std::vector<Part>& parts, float** logits) {
     }
     M += p.n;
   }
-  for (size_t b = 0; b < 2; b++)  // the tiles that see the most keys first
+  for (size_t b = 0; b < 2; b++)  // the last positions first: without a window or chunks the tiles that see the most keys
     std::stable_sort(ht[b], ht[b] + n_tiles[b], [](const PassTile& x, const PassTile& y) { return x.pos + x.n > y.pos + y.n; });
   size_t n_hist = 0;  // earlier positions that latent layers read again
   for (size_t i = 0; i < parts.size(); i++) {

@@ -207,7 +207,7 @@ typedef struct crabml_hip_llama crabml_hip_llama_t;
 /* config flags (crabml_hip_llama_config_t.flags).  A/B switches between kernel variants and test hooks share the word: they are
  * declared in crabml_hip_debug.h and are not part of the drop-in surface. */
 #define CRABML_HIP_LLAMA_NO_GRAPH 1 /* launch the kernels eagerly instead of replaying a hipGraph */
-#define CRABML_HIP_LLAMA_NO_PREFETCH 2 /* do not warm the Infinity Cache from the latency-bound stages */
+#define CRABML_HIP_LLAMA_NO_PREFETCH 2 /* no spare workgroups of attention that touch wo's weights ahead of it */
 #define CRABML_HIP_LLAMA_TP_GRAPH 8 /* tp_size > 1: capture the RCCL all-reduces into the hipGraph as well
                                        (default for tp: eager launches; falls back to eager if capture fails) */
 #define CRABML_HIP_LLAMA_EXACT_ATTENTION 4194304 /* fast mode, wherever attention would run with f32 sums (attn_long_from): keep the reference's serial
