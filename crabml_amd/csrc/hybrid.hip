@@ -95,6 +95,7 @@ struct crabml_hip_hybrid {
   int h_seq_next = 0;
   std::map<int, std::pair<hipGraph_t, hipGraphExec_t>> graphs;  // (graph_key)
   size_t single_steps[HYB_STEP_ROWS + 1] = {};  // greedy steps that a batch size has made one at a time
+  size_t step_nodes[HYB_STEP_ROWS + 1] = {};    // launches of a greedy step of a batch size
   bool graph_steps_now = false;                 // test hook: several steps a graph from the first run on
   // prompt pass (allocated on first use)
   size_t rows_cap = 0, hist_cap = 0, meta_bytes = 0;
@@ -783,8 +784,8 @@ int greedy_graph(Ctx* c, int B, size_t n, int* steps, hipGraphExec_t* exec) {
   if (!step_graphs(c)) return 0;
   std::pair<hipGraph_t, hipGraphExec_t> g;
   CH_TRY(step_graph(c, B, true, 1, &g));
-  size_t nodes = 0;
-  CH_HIP(c->dev, hipGraphGetNodes(g.first, nullptr, &nodes));
+  size_t& nodes = c->step_nodes[B];
+  if (!nodes) CH_HIP(c->dev, hipGraphGetNodes(g.first, nullptr, &nodes));
   const int s = steps_a_graph(nodes, c->cfg.seq_len);
   if (s == 1 || n < (size_t)s) return 0;
   const auto have = c->graphs.find(graph_key(B, true, s));
