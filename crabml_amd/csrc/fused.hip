@@ -160,13 +160,13 @@ struct crabml_hip_llama {
   // by attn_variant
   hipGraph_t graph[4] = {nullptr, nullptr, nullptr, nullptr};
   hipGraphExec_t exec[4] = {nullptr, nullptr, nullptr, nullptr};
-  // ... and of several steps behind one another (graph_steps.hpp), when greedy runs have earned it
+  // ... and of several steps behind one another (graph_steps.hpp), captured by greedy runs
   struct Several {
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    int steps = 1;          // that it holds
-    size_t nodes = 0;       // launches of one step
-    size_t single = 0;      // greedy steps made one at a time
+    int steps = 1;     // that the largest holds
+    size_t nodes = 0;  // launches of one step
+    unsigned have = 0, failed = 0;
+    hipGraph_t graph[GRAPH_SIZES] = {};
+    hipGraphExec_t exec[GRAPH_SIZES] = {};
   } several[4];
   bool graph_steps_now = false;  // test hook: from the first run on
   size_t weight_bytes = 0;       // of the matrices that a step reads
@@ -1257,14 +1257,22 @@ int run_steps(crabml_hip_llama* c, size_t pos, size_t n) {
     size_t m = 1;  // steps of this form
     while (i + m < n && variant_of(c, pos + i + m) == v) m++;
     auto& s = c->several[v];
-    if (s.steps > 1 && m >= (size_t)s.steps && !s.exec && (c->graph_steps_now || steps_graph_earned(s.nodes, s.steps, s.single + m)) &&
-        !capture_steps(c, v, s.steps, &s.graph, &s.exec)) {
-      (void)hipGetLastError();
-      s.steps = 1;
+    while (m > 0) {
+      const int z = next_size(m, c->graph_steps_now ? SIZE_MAX : i, s.steps, s.have, s.failed);
+      if (z >= 0 && !(s.have >> z & 1)) {
+        const bool ok = capture_steps(c, v, s.steps >> z, &s.graph[z], &s.exec[z]);
+        (ok ? s.have : s.failed) |= 1u << z;
+        (void)hipGetLastError();
+        continue;
+      }
+      const size_t made = z < 0 ? 1 : (size_t)(s.steps >> z);
+      if (z < 0)
+        CH_TRY(run_step(c, pos + i));
+      else
+        CH_HIP(c->dev, hipGraphLaunch(s.exec[z], c->dev->stream));
+      i += made;
+      m -= made;
     }
-    for (; s.exec && m >= (size_t)s.steps; i += s.steps, m -= s.steps) CH_HIP(c->dev, hipGraphLaunch(s.exec, c->dev->stream));
-    if (!s.exec) s.single += m;
-    for (; m > 0; i++, m--) CH_TRY(run_step(c, pos + i));
   }
   return 0;
 }
@@ -2453,8 +2461,10 @@ int crabml_hip_llama_destroy(crabml_hip_llama_t* c) {
   for (int v = 0; v < 4; v++) {
     if (c->exec[v]) (void)hipGraphExecDestroy(c->exec[v]);
     if (c->graph[v]) (void)hipGraphDestroy(c->graph[v]);
-    if (c->several[v].exec) (void)hipGraphExecDestroy(c->several[v].exec);
-    if (c->several[v].graph) (void)hipGraphDestroy(c->several[v].graph);
+    for (int z = 0; z < GRAPH_SIZES; z++) {
+      if (c->several[v].exec[z]) (void)hipGraphExecDestroy(c->several[v].exec[z]);
+      if (c->several[v].graph[z]) (void)hipGraphDestroy(c->several[v].graph[z]);
+    }
   }
   for (auto& a : c->allocs) pool_free(c->dev, a.first, a.second);
   for (auto* b : c->held) crabml_hip_buf_release(b);
@@ -2645,7 +2655,7 @@ int crabml_hip_llama_debug_graph_steps(crabml_hip_llama_t* c, size_t pos, int32_
   if (!c || !steps || !captured || pos >= c->cfg.seq_len) return CRABML_HIP_BAD_INPUT;
   const auto& s = c->several[variant_of(c, pos)];
   *steps = s.steps;
-  *captured = s.exec ? 1 : 0;
+  *captured = (int32_t)s.have;
   return 0;
 }
 

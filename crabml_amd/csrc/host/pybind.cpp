@@ -474,11 +474,11 @@ PYBIND11_MODULE(_host, m) {
                if (captured >> v & 1) forms.append(v);
              return py::make_tuple(form, forms);
            })
-      .def("debug_graph_steps",  // (steps of a greedy run in one graph at pos, captured)
+      .def("debug_graph_steps",  // (steps of a greedy run in the largest graph at pos, sizes captured)
            [](HipLlamaRunner& r, size_t pos) {
              int32_t steps = 0, captured = 0;
              r.device()->check(crabml_hip_llama_debug_graph_steps(r.raw(), pos, &steps, &captured));
-             return py::make_tuple(steps, captured != 0);
+             return py::make_tuple(steps, captured);
            })
       .def("debug_kv", [](HipLlamaRunner& r, size_t layer, bool v, bool f16) {
         std::vector<uint8_t> b = r.debug_kv(layer, v, f16);

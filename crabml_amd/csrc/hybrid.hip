@@ -94,8 +94,10 @@ struct crabml_hip_hybrid {
   StepSeq* h_seq = nullptr;  // pinned ring of META_SLOTS * HYB_STEP_ROWS
   int h_seq_next = 0;
   std::map<int, std::pair<hipGraph_t, hipGraphExec_t>> graphs;  // (graph_key)
-  size_t single_steps[HYB_STEP_ROWS + 1] = {};  // greedy steps that a batch size has made one at a time
-  size_t step_nodes[HYB_STEP_ROWS + 1] = {};    // launches of a greedy step of a batch size
+  struct {
+    int steps = 0;  // that the largest graph of a greedy run holds (0: not known yet)
+    unsigned have = 0, failed = 0;
+  } several[HYB_STEP_ROWS + 1];
   bool graph_steps_now = false;                 // test hook: several steps a graph from the first run on
   // prompt pass (allocated on first use)
   size_t rows_cap = 0, hist_cap = 0, meta_bytes = 0;
@@ -749,12 +751,12 @@ int enqueue_step(Ctx* c, int B, bool sample, bool prof, bool led = false, bool l
 
 int graph_key(int B, bool sample, int steps) { return (steps * (HYB_STEP_ROWS + 1) + B) * 2 + (sample ? 1 : 0); }
 bool step_graphs(const Ctx* c) { return !(c->cfg.flags & CRABML_HIP_HYBRID_NO_GRAPH) && !c->dev->prof_on; }
-// the graph of one decode step of B rows, or of several of a greedy run, captured when it is first asked for
-int step_graph(Ctx* c, int B, bool sample, int steps, std::pair<hipGraph_t, hipGraphExec_t>* out) {
+// the graph of one decode step of B rows, or of several of a greedy run, captured when it is first asked for; false: that failed
+bool step_graph(Ctx* c, int B, bool sample, int steps, std::pair<hipGraph_t, hipGraphExec_t>* out) {
   crabml_hip_device* dev = c->dev;
   auto& slot = c->graphs[graph_key(B, sample, steps)];
   if (!slot.second) {
-    CH_HIP(dev, hipStreamBeginCapture(dev->stream, hipStreamCaptureModeThreadLocal));
+    if (hipStreamBeginCapture(dev->stream, hipStreamCaptureModeThreadLocal) != hipSuccess) return false;
     int rc = 0;
     for (int i = 0; i < steps && rc == 0; i++) rc = enqueue_step(c, B, sample, false, i > 0, i + 1 < steps);
     hipGraph_t graph = nullptr;
@@ -763,36 +765,45 @@ int step_graph(Ctx* c, int B, bool sample, int steps, std::pair<hipGraph_t, hipG
     if (rc != 0 || e != hipSuccess || !graph || hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) != hipSuccess) {
       if (graph) (void)hipGraphDestroy(graph);
       (void)hipGetLastError();
-      CH_BAIL(dev, CRABML_HIP_UNEXPECTED, "hybrid: hipGraph capture / instantiate of the decode step failed");
+      return false;
     }
     slot = {graph, exec};
   }
   *out = slot;
+  return true;
+}
+int one_step_graph(Ctx* c, int B, bool sample, std::pair<hipGraph_t, hipGraphExec_t>* out) {
+  if (!step_graph(c, B, sample, 1, out)) CH_BAIL(c->dev, CRABML_HIP_UNEXPECTED, "hybrid: hipGraph capture / instantiate of the decode step failed");
   return 0;
 }
 // one decode step of B rows from its graph, or eagerly
 int run_step(Ctx* c, int B, bool sample) {
   if (!step_graphs(c)) return enqueue_step(c, B, sample, true);
   std::pair<hipGraph_t, hipGraphExec_t> g;
-  CH_TRY(step_graph(c, B, sample, 1, &g));
+  CH_TRY(one_step_graph(c, B, sample, &g));
   CH_HIP(c->dev, hipGraphLaunch(g.second, c->dev->stream));
   return 0;
 }
-// Steps at a time of a greedy run of n: what a graph of several holds, where there is one or this run is the one that captures it (graph_steps.hpp)
-int greedy_graph(Ctx* c, int B, size_t n, int* steps, hipGraphExec_t* exec) {
-  *steps = 1;
-  if (!step_graphs(c)) return 0;
+// n greedy steps: several at a time from the graphs of that (graph_steps.hpp), which the run captures as it goes
+int run_steps(Ctx* c, int B, size_t n) {
+  crabml_hip_device* dev = c->dev;
+  auto& v = c->several[B];
   std::pair<hipGraph_t, hipGraphExec_t> g;
-  CH_TRY(step_graph(c, B, true, 1, &g));
-  size_t& nodes = c->step_nodes[B];
-  if (!nodes) CH_HIP(c->dev, hipGraphGetNodes(g.first, nullptr, &nodes));
-  const int s = steps_a_graph(nodes, c->cfg.seq_len);
-  if (s == 1 || n < (size_t)s) return 0;
-  const auto have = c->graphs.find(graph_key(B, true, s));
-  if ((have == c->graphs.end() || !have->second.second) && !c->graph_steps_now && !steps_graph_earned(nodes, s, c->single_steps[B] + n)) return 0;
-  CH_TRY(step_graph(c, B, true, s, &g));
-  *steps = s;
-  *exec = g.second;
+  for (size_t made = 0; made < n;) {
+    const int z = next_size(n - made, c->graph_steps_now ? SIZE_MAX : made, v.steps, v.have, v.failed);
+    if (z < 0) {
+      CH_TRY(run_step(c, B, true));
+      made++;
+      continue;
+    }
+    if (!step_graph(c, B, true, v.steps >> z, &g)) {
+      v.failed |= 1u << z;
+      continue;
+    }
+    v.have |= 1u << z;
+    CH_HIP(dev, hipGraphLaunch(g.second, dev->stream));
+    made += (size_t)(v.steps >> z);
+  }
   return 0;
 }
 
@@ -1456,18 +1467,20 @@ int crabml_hip_hybrid_decode_greedy(crabml_hip_hybrid_t* c, size_t n, const size
       CH_BAIL(dev, CRABML_HIP_TENSOR_ERROR, "hybrid: %zu steps do not fit sequence %zu (%zu of %zu used)", n_steps, seqs[i], c->seqs[seqs[i]].len, c->cfg.seq_len);
   }
   if (n_steps == 0) return 0;
-  int steps = 1;
-  hipGraphExec_t several = nullptr;
-  CH_TRY(greedy_graph(c, (int)n, n_steps, &steps, &several));
+  auto& several = c->several[n];
+  if (step_graphs(c) && !several.steps) {
+    std::pair<hipGraph_t, hipGraphExec_t> one;
+    CH_TRY(one_step_graph(c, (int)n, true, &one));
+    size_t nodes = 0;
+    CH_HIP(dev, hipGraphGetNodes(one.first, nullptr, &nodes));
+    several.steps = steps_a_graph(nodes, c->cfg.seq_len);
+  }
   CH_TRY(step_begin(c, n, seqs, tokens));
   CH_HIP(dev, hipMemsetAsync(c->st_count, 0, HYB_STEP_ROWS * sizeof(int), dev->stream));
-  size_t s = 0;
-  if (steps > 1) {
-    for (; s + steps <= n_steps; s += steps) CH_HIP(dev, hipGraphLaunch(several, dev->stream));
-  } else {
-    c->single_steps[n] += n_steps;
-  }
-  for (; s < n_steps; s++) CH_TRY(run_step(c, (int)n, true));
+  if (step_graphs(c))
+    CH_TRY(run_steps(c, (int)n, n_steps));
+  else
+    for (size_t s = 0; s < n_steps; s++) CH_TRY(run_step(c, (int)n, true));
   for (size_t i = 0; i < n; i++) c->seqs[seqs[i]].len += n_steps;
   CH_HIP(dev, hipMemcpyAsync(out_tokens, c->st_out, n_steps * n * sizeof(uint32_t), hipMemcpyDeviceToHost, dev->stream));
   CH_HIP(dev, hipStreamSynchronize(dev->stream));
@@ -1476,10 +1489,10 @@ int crabml_hip_hybrid_decode_greedy(crabml_hip_hybrid_t* c, size_t n, const size
 
 }  // extern "C"
 
-extern "C" int crabml_hip_debug_graph_steps(size_t nodes, size_t seq_len, size_t done, int32_t* steps, int32_t* earned) {
-  if (!steps || !earned) return CRABML_HIP_BAD_INPUT;
-  *steps = crabml_hip::steps_a_graph(nodes, seq_len);
-  *earned = crabml_hip::steps_graph_earned(nodes, *steps, done) ? 1 : 0;
+extern "C" int crabml_hip_debug_graph_steps(size_t nodes, size_t seq_len, size_t left, size_t made, uint32_t have, int32_t* top, int32_t* next) {
+  if (!top || !next) return CRABML_HIP_BAD_INPUT;
+  *top = crabml_hip::steps_a_graph(nodes, seq_len);
+  *next = crabml_hip::next_size(left, made, *top, have, 0);
   return 0;
 }
 extern "C" int crabml_hip_debug_prefetch(int32_t hybrid, size_t model_bytes, int32_t m, int32_t rows, size_t row_bytes, size_t row_bytes2, size_t* bytes) {

@@ -57,9 +57,9 @@ int crabml_hip_debug_gemm_ints(crabml_hip_device_t* dev, const crabml_hip_buf_t*
                                const crabml_hip_buf_t* x, size_t b, int32_t* dst, float* out);
 /* Rows of the rhs that one launch of the row kernels takes over a matrix of m rows (matmul_vec without a matrix-core kernel).  Host only. */
 int crabml_hip_debug_rhs_rows(size_t m, size_t* rows);
-/* Steps of a greedy run that go into one graph where one step is `nodes` launches, and whether `done` steps -- made one at a time so far or about to be --
- * have earned its capture.  Host only. */
-int crabml_hip_debug_graph_steps(size_t nodes, size_t seq_len, size_t done, int32_t* steps, int32_t* earned);
+/* top: steps of a greedy run that go into one graph where one step is `nodes` launches.  next: which of the sizes top, top / 2, top / 4 comes next in a run that
+ * has made `made` steps and has `left` to make (its place; -1: a single step); have: the sizes that have been captured, bits by place.  Host only. */
+int crabml_hip_debug_graph_steps(size_t nodes, size_t seq_len, size_t left, size_t made, uint32_t have, int32_t* top, int32_t* next);
 /* Waves of a workgroup of the fast prompt pass's gate | up launch over `rows` > 64 rows.  Host only. */
 int crabml_hip_debug_gateup_waves(uint32_t dtype, size_t hidden, size_t rows, int32_t n_cu, int32_t* waves);
 /* Rows of wo / ffn_down that a workgroup of a llama step takes: with the next norm in the launch or without, block-ordered sums (strict device), one or two
@@ -142,7 +142,7 @@ int crabml_hip_debug_flash_attention_rows(crabml_hip_device_t* dev, const float*
 
 /* the attention form of the step that serves cache position `pos`, and the forms whose step this context captured (bit v: form v) */
 int crabml_hip_llama_debug_graphs(crabml_hip_llama_t* ctx, size_t pos, int32_t* form, uint32_t* captured);
-/* greedy steps a graph of several holds at cache position pos (1: none is made), and whether it has been captured */
+/* greedy steps the largest graph of several holds at cache position pos (1: none is made), and the sizes that have been captured, bits by place */
 int crabml_hip_llama_debug_graph_steps(crabml_hip_llama_t* ctx, size_t pos, int32_t* steps, int32_t* captured);
 /* parity hook: copies the layer's K or V cache (raw f16/f32 bytes, [n_kv_heads][seq_len][head_dim]) */
 int crabml_hip_llama_debug_kv(crabml_hip_llama_t* ctx, size_t layer, int32_t which_v, void* dst, size_t nbytes);

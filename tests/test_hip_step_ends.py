@@ -53,13 +53,13 @@ BIFAZEN = sb.config(200, 131, [sb.latent(2, 12, 4, 12, 20, 30, 40), sb.attention
 
 @pytest.mark.parametrize("config,tensors", [(NILIVIK, sh.random_tensors), (BIFAZEN, sb.random_tensors)])
 @pytest.mark.parametrize("rows", [1, 3])
-def test_several_steps_a_graph_when_runs_have_earned_it(ca, hdev, tmp_path, config, tensors, rows):
-    """short runs make their steps one at a time until they have made up for a graph of several, and the same tokens before and behind that"""
+def test_runs_capture_several_steps_a_graph_as_they_go(ca, hdev, tmp_path, config, tensors, rows):
+    """runs of all lengths capture graphs of eight, four and two steps behind their first ones: the same tokens before, during and behind that"""
     folder = sh.write_model(config, tensors(config, 7), str(tmp_path / "m"))
     g, e = ca.load_model(folder, hdev, seq_len=300), ca.load_model(folder, hdev, seq_len=300, use_graph=False)
     seqs = [[r.open() for _ in range(rows)] for r in (g, e)]
     ids = list(range(1, rows + 1))
-    for n in (9, 30, 9, 60, 17, 100, 12):
+    for n in (1, 3, 9, 30, 9, 60, 17, 7, 100, 12):
         a, b = g.decode_batch(seqs[0], ids, n), e.decode_batch(seqs[1], ids, n)
         assert list(a) == list(b), n
         ids = list(a[-rows:])
@@ -130,18 +130,17 @@ def test_a_step_by_itself_has_one_front(ca, fmt, shape):
 
 
 @pytest.mark.parametrize("fmt,shape", [("Q8_0", "15m"), ("Q4_K", "tiny-hd128")])
-def test_a_runner_captures_several_steps_when_runs_have_earned_it(ca, fmt, shape):
-    """none when it is made, none for short answers, and the same tokens before and behind"""
+def test_a_runner_captures_several_steps_as_it_runs(ca, fmt, shape):
+    """none when it is made, the sizes that a run has use for behind its first steps, and the same tokens before, during and behind that"""
     dev = ca.HipTensorDevice(0)
     conf, w = synth.to_hip(synth.build_model(synth.SHAPES[shape], synth.TYPE_BY_NAME[fmt], seed=23), dev)
     a, e = ca.HipLlamaRunner(conf, w, dev, 400, True), ca.HipLlamaRunner(conf, w, dev, 400, True, False)
-    assert [a.debug_graph_steps(p) for p in (0, 100, 399)] == [(8, False)] * 3 and e.debug_graph_steps(0) == (1, False)
+    assert [a.debug_graph_steps(p) for p in (0, 100, 399)] == [(8, 0)] * 3 and e.debug_graph_steps(0) == (1, 0)
     token = 3
-    for n, captured in ((10, False), (9, False), (200, True), (20, True)):  # (a token makes at least 12 launches, 31 with 6 layers)
+    for n, captured in ((1, 0), (3, 0), (7, 2), (8, 2), (6, 6), (194, 7), (20, 7)):  # (bits: eight steps, four, two)
         ids = a.decode_greedy(token, n)
         assert ids == e.decode_greedy(token, n), n
         token = ids[-1]
-        if n != 20:
-            assert any(a.debug_graph_steps(p)[1] for p in (0, 100, 399)) == captured, n
+        assert a.debug_graph_steps(0)[1] == captured and e.debug_graph_steps(0)[1] == 0, n
     x, y = a.forward(token, 239), e.forward(token, 239)
     assert np.array_equal(x.view(np.uint32), y.view(np.uint32))

@@ -64,26 +64,47 @@ def test_rows_of_the_residual_linears():
         assert rows.value == want, args
 
 
-def graph_steps(nodes, seq_len, done):
-    steps, earned = ctypes.c_int32(), ctypes.c_int32()
-    assert lib.crabml_hip_debug_graph_steps(ctypes.c_size_t(nodes), ctypes.c_size_t(seq_len), ctypes.c_size_t(done), ctypes.byref(steps), ctypes.byref(earned)) == 0
-    return steps.value, bool(earned.value)
+def graph_steps(nodes, seq_len, left=0, made=0, have=0):
+    top, place = ctypes.c_int32(), ctypes.c_int32()
+    assert lib.crabml_hip_debug_graph_steps(ctypes.c_size_t(nodes), ctypes.c_size_t(seq_len), ctypes.c_size_t(left), ctypes.c_size_t(made), have, ctypes.byref(top),
+                                            ctypes.byref(place)) == 0
+    return top.value, place.value
 
 
-def test_a_capture_is_bounded_and_earned():
-    """several steps in a graph: a bounded number of launches, and none captured before the steps that it serves have won what the capture costs (at
-    least 1.4 us a launch; at most 7 us between two steps)"""
+def test_graphs_of_several_steps_are_bounded():
     for nodes in (1, 14, 23, 31, 44, 63, 123, 161, 192, 193, 243, 1000):
         for seq_len in (1, 2, 3, 15, 16, 400, 8192):
-            n = graph_steps(nodes, seq_len, 0)[0]
+            n = graph_steps(nodes, seq_len)[0]
             assert 1 <= n <= 8 and (n == 1 or (n * nodes <= 384 and 2 * n <= seq_len)), (nodes, seq_len)
-        n, first = graph_steps(nodes, 8192, 0)[0], next((d for d in range(1, 3000) if graph_steps(nodes, 8192, d)[1]), None)
-        if n == 1:
-            assert first is None and nodes > 192
-        else:
-            assert first * 7 * (n - 1) / n >= 1.4 * nodes * n, (nodes, n, first)
-    assert graph_steps(23, 400, 16) == (8, False) and graph_steps(123, 400, 64) == (3, False)  # (a short answer, a deeper model)
-    assert graph_steps(23, 400, 200) == (8, True)
+    assert graph_steps(23, 8192)[0] == 8 and graph_steps(123, 8192)[0] == 3 and graph_steps(193, 8192)[0] == 1
+
+
+@pytest.mark.parametrize("nodes", [23, 50, 63, 90, 123, 180, 250])
+def test_a_run_captures_behind_its_own_steps(nodes):
+    """a capture (at most 2 us a launch) only while steps of the same run keep the GPU busy (4 us a launch), none that the run does not use, and the same run
+    once more goes through graphs from its first step on"""
+    top = graph_steps(nodes, 8192)[0]
+    for n in range(1, 120):
+        have, made, launches = 0, 0, 0
+        while made < n:
+            place = graph_steps(nodes, 8192, n - made, made, have)[1]
+            size = 1 if place < 0 else top >> place
+            assert size <= n - made and (place < 0 or size >= 2)
+            if place >= 0 and not have >> place & 1:
+                assert 4 * made >= 2 * size and (place == 0 or n - made < 2 * size), (n, made, size)
+                have |= 1 << place
+            made += size
+            launches += 1
+        assert made == n
+        if top > 1 and n >= 2 * top:
+            assert have & 1 and launches <= top // 2 + 1 + n // top + 3, (n, launches)
+        made = 0
+        while made < n:
+            place = graph_steps(nodes, 8192, n - made, made, have)[1]
+            if made == 0 and have:
+                assert place >= 0, n
+            have |= 1 << place if place >= 0 else 0
+            made += 1 if place < 0 else top >> place
 
 
 Q4_0, Q8_0, Q4_K = 2, 8, 12
