@@ -1348,7 +1348,7 @@ __global__ __launch_bounds__(512) void k_attn_flash_rows(const float* __restrict
   float m = -INFINITY, lsum = 0.f;
   // staging: thread t moves NP 16-byte pieces of the K tile per fill (piece = 8 dims of one position), and of the V tile the same 8 dims
   // of NV pairs of neighbouring positions, so that V^T takes whole dwords, a half-wave's side by side (halves of one position a
-  // lane, lanes along the dims, put 16 lanes on 4 banks: 32 heads of 128, 512 rows 23.6 -> 17.4 us, 1024 behind 1977 171 -> 113); a whole tile of compute lies between the
+  // lane, lanes along the dims, put 16 lanes on 4 banks: 32 heads of 128, 512 rows 23.6 -> 17.4 us, 953 behind 2048 171 -> 113); a whole tile of compute lies between the
   // request and the commit
   constexpr int PAIRS = HD / 8 * (BN / 2), NV = (PAIRS + 511) / 512;
   i32x4 vreg[2 * NV], kreg[NP];

@@ -8,8 +8,9 @@
 // again (its results are not stored), a 16-byte piece past the end of k is a piece of zeros.  Weights are the first operand, so that a
 // lane's four results are neighbouring columns of one row and leave as one 16-byte store, without a way through LDS.
 //
-// Measured (203 rows, width 2048, ff 8192, one layer): q | k | v 15.5 us, wo 15.0, gate | up 27.5, ff_down 28.8 (500 TFLOP/s in the
-// gate | up launch); 17.8, 17.2, 33.6, 28.5 with a step's requests in a row behind its barrier and four waves on a 128-row tile.
+// Measured (203 rows, width 2048, ff 8192, one layer): q | k | v 15.4 us, wo 15.0, gate | up 28.1, ff_down 29.4 (490 TFLOP/s in the
+// gate | up launch); 17.8, 17.2, 33.6, 28.5 with a step's requests in a row behind its barrier and four waves on a 128-row tile (ff_down, on 64-row
+// tiles in pieces of k, gained nothing).
 #include <type_traits>
 
 #include "gemm_bf16.hpp"

@@ -507,7 +507,7 @@ __global__ __launch_bounds__(256 * KP, sizeof(T) == 2 ? (KP == 2 && KC <= 128 ? 
 // term.  Decay powers, products with the state and the masked weights are f32 (mma_rows on an f32 side).
 // What bounds it is the chain of blocks, some 4.5 us each in a workgroup per head and slice, so where CUs are left over (lin_segments) a sequence's
 // blocks are shared out: a first launch (SUMS) leaves what each segment adds to the state, and every segment starts from the
-// sums in front of it.  2048 rows, 16 heads of 64 x 128: 143 us -> 28 + 51.
+// sums in front of it.  2048 rows, 16 heads of 64 x 128: 143 us -> 45 + 41.
 template <typename T, int CLS>
 struct LinTile {
   static constexpr int C = sizeof(T) == 2 ? 64 : 32, PAD = 16 / sizeof(T);
