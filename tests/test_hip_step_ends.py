@@ -144,3 +144,15 @@ def test_a_runner_captures_several_steps_as_it_runs(ca, fmt, shape):
         assert a.debug_graph_steps(0)[1] == captured and e.debug_graph_steps(0)[1] == 0, n
     x, y = a.forward(token, 239), e.forward(token, 239)
     assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
+
+
+@pytest.mark.parametrize("strict,layers,steps", [(False, 32, 2), (True, 32, 1), (False, 24, 3), (True, 24, 3)])
+def test_deep_models_chain_few_steps(ca, strict, layers, steps):
+    """steps of 5 launches a layer and some, up to 384 launches a graph; no pairs on the strict device"""
+    dev = ca.HipTensorDevice(0, strict_order=strict)
+    shape = synth.ModelShape("deep", 256, 512, layers, 2, 2, 300, 64, 1e-5, None)
+    conf, w = synth.to_hip(synth.build_model(shape, synth.Q4_0, seed=24), dev)
+    a, e = ca.HipLlamaRunner(conf, w, dev, 60, True), ca.HipLlamaRunner(conf, w, dev, 60, True, False)
+    assert a.debug_graph_steps(0) == (steps, 0)
+    assert a.decode_greedy(3, 25) == e.decode_greedy(3, 25)
+    assert a.debug_graph_steps(0)[1] == (1 if steps > 1 else 0)
