@@ -1,4 +1,5 @@
-// gemm_f16w.hip -- the FAST prompt pass's weight GEMM (crabml_hip_llama_prefill on the fast device; Q4_0 / Q8_0 weights x Q8_0 rows,
+// gemm_f16w.hip -- the FAST prompt pass's weight GEMM, its operands, and its kernel for up to 64 rows and widths that are no multiple of 256; the others:
+// gemm_f16w_wide.hip (crabml_hip_llama_prefill on the fast device; Q4_0 / Q8_0 weights x Q8_0 rows,
 // Q4_1 x Q8_1, Q4_K / Q6_K x Q8_K): weight-stationary on the f16 matrix cores.
 //
 // matmul_vec with a batched rhs is `C[b, m] = W[m, k] . x[b, k]` (matmul_vec.rs:41-76: the (b, k) rhs contract; llama2.rs:111-129).
@@ -35,14 +36,9 @@
 #include <cstdlib>
 #include <type_traits>
 
-#include "devutil.hpp"
-#include "f16w_rows.hpp"
-#include "kernels.hpp"
+#include "gemm_f16w.hpp"
 
 namespace crabml_hip {
-
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 // ---- B': the rows of a prompt pass as pre-scaled f16, in the GEMM's k-slot order: xh[col][kb][32] f16 ------------------------
 // (the slot orders and the conversion of one 8-slot group: f16w_rows.hpp, shared with the row kernels that write B' themselves)
@@ -92,79 +88,6 @@ __global__ __launch_bounds__(256) void k_addn_f32(F16wParts a) {
   ((f32x4*)o)[li] = v;
 }
 
-// one dword of a Q4_0 block (quant bytes 4 s .. 4 s + 3: low nibbles = elements 4 s .., high nibbles = 16 + 4 s ..; buf_q4_0.rs:24-33)
-// -> the lane's eight f16 k-slots (q - 8) * d.  0x6400 | n is the f16 number 1024 + n; -1032 makes it n - 8 exactly.
-// (x & 0x000F000F) | 0x64006400 as ONE v_and_or_b32: a VOP3 instruction takes a single scalar / literal operand, so the compiler
-// splits it unless one constant sits in a VGPR -- `magic` (loop-invariant, one register)
-__device__ __forceinline__ unsigned and_or_magic(unsigned x, unsigned magic) {
-  unsigned r;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(0x000F000Fu), "v"(magic));
-  return r;
-}
-__device__ __forceinline__ f16x8 unpack_q4_0_f16(unsigned w, f16x2 d2, unsigned magic) {
-  const f16x2 bias = {(_Float16)-1032.0f, (_Float16)-1032.0f};
-  const unsigned u0 = and_or_magic(w, magic), u1 = and_or_magic(w >> 8, magic);
-  const unsigned u2 = and_or_magic(w >> 4, magic), u3 = and_or_magic(w >> 12, magic);
-  const f16x2 p0 = (__builtin_bit_cast(f16x2, u0) + bias) * d2, p1 = (__builtin_bit_cast(f16x2, u1) + bias) * d2;
-  const f16x2 p2 = (__builtin_bit_cast(f16x2, u2) + bias) * d2, p3 = (__builtin_bit_cast(f16x2, u3) + bias) * d2;
-  return f16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-}
-
-// Q8_0: the bytes of a dword as f16 (b ^ 0x80 = b + 128 unsigned; 0x6400 | u = 1024 + u; -1152 makes it b exactly), pairs (b0, b2), (b1, b3)
-__device__ __forceinline__ unsigned and_or_magic8(unsigned x, unsigned magic) {
-  unsigned r;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(0x00FF00FFu), "v"(magic));
-  return r;
-}
-__device__ __forceinline__ f16x8 unpack_q8_0_f16(unsigned w0, unsigned w1, f16x2 d2, unsigned magic) {
-  const f16x2 bias = {(_Float16)-1152.0f, (_Float16)-1152.0f};
-  const unsigned x0 = w0 ^ 0x80808080u, x1 = w1 ^ 0x80808080u;
-  const unsigned u0 = and_or_magic8(x0, magic), u1 = and_or_magic8(x0 >> 8, magic);
-  const unsigned u2 = and_or_magic8(x1, magic), u3 = and_or_magic8(x1 >> 8, magic);
-  const f16x2 p0 = (__builtin_bit_cast(f16x2, u0) + bias) * d2, p1 = (__builtin_bit_cast(f16x2, u1) + bias) * d2;
-  const f16x2 p2 = (__builtin_bit_cast(f16x2, u2) + bias) * d2, p3 = (__builtin_bit_cast(f16x2, u3) + bias) * d2;
-  return f16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-}
-// Q4_K: one class dword of the lane's pair; cs = {d sc_lo, -dmin m_lo, d sc_hi, -dmin m_hi}, each in both halves
-struct Q4KF16Consts {
-  f16x2 c_lo, o_lo, c_hi, o_hi;
-};
-__device__ __forceinline__ f16x8 unpack_q4_k_f16(unsigned w, const Q4KF16Consts& cs, unsigned magic) {
-  const f16x2 bias = {(_Float16)-1024.0f, (_Float16)-1024.0f};
-  const unsigned u0 = and_or_magic(w, magic), u1 = and_or_magic(w >> 8, magic);
-  const unsigned u2 = and_or_magic(w >> 4, magic), u3 = and_or_magic(w >> 12, magic);
-  const f16x2 p0 = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, u0) + bias, cs.c_lo, cs.o_lo);
-  const f16x2 p1 = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, u1) + bias, cs.c_lo, cs.o_lo);
-  const f16x2 p2 = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, u2) + bias, cs.c_hi, cs.o_hi);
-  const f16x2 p3 = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, u3) + bias, cs.c_hi, cs.o_hi);
-  return f16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-}
-__device__ __forceinline__ Q4KF16Consts q4k_f16_consts(i32x4 hdr, int g) {
-  const unsigned f = q4k_pair_field((unsigned)hdr[1], (unsigned)hdr[2], (unsigned)hdr[3], g);
-  const float d = h2f((unsigned short)((unsigned)hdr[0] & 0xffffu)), dmin = h2f((unsigned short)((unsigned)hdr[0] >> 16));
-  const _Float16 c_lo = (_Float16)(d * (float)(f & 63u)), c_hi = (_Float16)(d * (float)((f >> 6) & 63u));  // (11 x 6 bits: exact in f32)
-  const _Float16 o_lo = (_Float16)-(dmin * (float)((f >> 12) & 63u)), o_hi = (_Float16)-(dmin * (float)(f >> 18));
-  return Q4KF16Consts{f16x2{c_lo, c_lo}, f16x2{o_lo, o_lo}, f16x2{c_hi, c_hi}, f16x2{o_hi, o_hi}};
-}
-
-// Q6_K: one dword of ql and the matching dword of qh, already shifted so that bits 0-1 of each byte belong to the low nibbles' quarter
-// and bits 4-5 to the high nibbles'
-__device__ __forceinline__ unsigned and_or_hi2(unsigned x, unsigned acc) {
-  unsigned r;
-  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(0x00300030u), "v"(acc));
-  return r;
-}
-__device__ __forceinline__ f16x8 unpack_q6_k_f16(unsigned w, unsigned hw, f16x2 c_lo, f16x2 c_hi, unsigned magic) {
-  const f16x2 bias = {(_Float16)-1056.0f, (_Float16)-1056.0f};  // 1024 + q -> q - 32
-  const unsigned u0 = and_or_hi2(hw << 4, and_or_magic(w, magic)), u1 = and_or_hi2(hw >> 4, and_or_magic(w >> 8, magic));
-  const unsigned u2 = and_or_hi2(hw, and_or_magic(w >> 4, magic)), u3 = and_or_hi2(hw >> 8, and_or_magic(w >> 12, magic));
-  const f16x2 p0 = (__builtin_bit_cast(f16x2, u0) + bias) * c_lo, p1 = (__builtin_bit_cast(f16x2, u1) + bias) * c_lo;
-  const f16x2 p2 = (__builtin_bit_cast(f16x2, u2) + bias) * c_hi, p3 = (__builtin_bit_cast(f16x2, u3) + bias) * c_hi;
-  return f16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-}
-
-enum { WF_Q4_0 = 0, WF_Q8_0 = 1, WF_Q4_K = 2, WF_Q6_K = 3, WF_Q4_1 = 4 };  // the weight format of a GEMM
-
 template <int T_, int NW = 4>
 struct GemmF16Geo {
   static constexpr int T = T_, CW = 16 * T;    // column tiles per wave / prompt rows per workgroup
@@ -179,26 +102,6 @@ struct GemmF16Geo {
   static constexpr int B_LOADS = CW * KCH * 4 / (64 * NW);  // 16-byte pieces per thread and chunk
 };
 
-// Up to three weight matrices against the same rhs in ONE launch (wq | wk | wv: the 1024-row k / v GEMMs alone leave most of the
-// chip idle for a whole serial k loop): row tile rt belongs to the first matrix whose cumulative tile count exceeds it.
-struct F16wMats {
-  const i32x4* wq[3];  // the quant plane
-  const char* wd[3];   // the scale plane (f16 per block; Q4_1: (d, m); Q4_K: the 16-byte headers; Q6_K: the qh plane)
-  const char* ws2[3];  // Q6_K: the int8 scales (16 per super-block) ...
-  const char* ws3[3];  // ... and d (f16 per super-block)
-  float* out[3];
-  float* out2[3];    // ksplit > 1: k piece s >= 1 writes its partial tiles to out2[j] + (s - 1) pstride (k_addn_f32 adds them)
-  size_t pstride;
-  const unsigned short* exp_tab;  // GU launches: the f16 exp table of silu (silu.rs:6-13)
-  F16wHQuant hq;                   // GU launches: h leaves as Q8_0 / Q8_1 planes (+ ffn_down's B') instead of f32 (planes == nullptr: f32)
-  int m[3];
-  int tiles_end[3];  // cumulative row tiles
-};
-// h = silu(g) * u (silu.rs:6-13, arithmetic.rs:57-66; fused_ffn.hpp silu_mul: the exp through the reference's f16 table)
-__device__ __forceinline__ float f16w_silu_mul(float g, float u, const unsigned short* __restrict__ exp_tab) {
-  const float nexp = h2f(exp_tab[f2h(-g)]);
-  return (g / (1.0f + nexp)) * u;
-}
 // GU (F = 2, two matrices of the same shape: ffn_gate and ffn_up): fragment 0 holds 16 rows of the FIRST matrix, fragment 1 the same
 // 16 rows of the SECOND -- the workgroup owns 16 NW rows of both -- and the epilogue stores h = silu(g) * u (out[0]) instead of g and u:
 // the (rows, hidden) f32 pair never makes its trip through memory (llama2.rs:620-630).  One k piece only (silu is not linear).
@@ -433,10 +336,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_gemm_f16w(F16wMats mats, const i
   // D: lane (i, g) holds rows 4 g .. 4 g + 3 of column i of every tile
   if constexpr (GU) {
     if (mats.hq.planes != nullptr) {
-      // h = silu(g) * u of the workgroup's 16 NW rows x CW columns through LDS (the B' buffers are done), then ONE THREAD per
-      // (column, 32-row block) runs the row quantizer on it (quant_lane32's arithmetic, buf_q8_0.rs:87-134 / buf_q8_1.rs:90-129: the
-      // block maximum and the integer sum do not depend on the order) and writes the block's quants, scale, sum and -- in the slot
-      // order of ffn_down's GEMM -- its 32 pre-scaled halfs: h never exists as f32 in memory
+      // h of the workgroup's 16 NW rows x CW columns through LDS (the B' buffers are done)
       constexpr int CS = 16 * NW + 4, HB = NW / 2;  // floats per column (16-byte aligned columns, four banks apart), blocks
       static_assert((size_t)G::CW * CS * sizeof(float) <= (size_t)G::LDS_BYTES, "h fits where B' was");
       float* H = (float*)f16w_lds;
@@ -449,58 +349,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_gemm_f16w(F16wMats mats, const i
         *(f32x4*)(H + (16 * t + i) * CS + wave * 16 + 4 * g) = hv;
       }
       __syncthreads();
-      const F16wHQuant& hq = mats.hq;
-      const int nbh = m / 32;
-      for (int b = tid; b < G::CW * HB; b += NT) {
-        const int col = c0 + b / HB, hb = rt_l * HB + b % HB;
-        if (col >= n || hb >= nbh) continue;
-        f32x4 v[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = *(const f32x4*)(H + (b / HB) * CS + 32 * (b % HB) + 4 * j);
-        float amax = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-#pragma unroll
-          for (int r = 0; r < 4; r++) amax = fmaxf(amax, fabsf(v[j][r]));
-        const float dd = amax / 127.0f;
-        const unsigned short dh = f2h(dd);
-        int q[32], sum = 0;
-#pragma unroll
-        for (int e = 0; e < 32; e++) {
-          const float x = v[e >> 2][e & 3];
-          if (hq.q81) {
-            q[e] = (int)fminf(fmaxf(x / dd, -128.0f), 127.0f);
-          } else {
-            q[e] = (int)(signed char)(unsigned char)((unsigned)rs_f32_as_i32(x / dd) & 0xffu);
-          }
-          sum += q[e];
-        }
-        char* p = hq.planes + (size_t)col * hq.stride;
-        i32x4 pk[2];
-#pragma unroll
-        for (int e = 0; e < 8; e++)
-          pk[e >> 2][e & 3] = (int)(((unsigned)q[4 * e] & 0xffu) | (((unsigned)q[4 * e + 1] & 0xffu) << 8) | (((unsigned)q[4 * e + 2] & 0xffu) << 16) |
-                                    (((unsigned)q[4 * e + 3] & 0xffu) << 24));
-        ((i32x4*)(p + (size_t)hb * 32))[0] = pk[0];
-        ((i32x4*)(p + (size_t)hb * 32))[1] = pk[1];
-        ((unsigned short*)(p + hq.off_d))[hb] = dh;
-        if (hq.q81)
-          ((unsigned short*)(p + hq.off_aux))[hb] = f2h((float)sum * dd);
-        else
-          ((int*)(p + hq.off_aux))[hb] = sum;
-        if (hq.xh != nullptr) {
-          const float ds = h2f(dh);
-          unsigned short* xr = hq.xh + ((size_t)col * nbh + hb) * 32;
-#pragma unroll
-          for (int s4 = 0; s4 < 4; s4++) {
-            unsigned short o[8];
-#pragma unroll
-            for (int e = 0; e < 8; e++) o[e] = f16w_value(q[f16w_slot_elem(8 * s4 + e)], ds);
-            *(i32x4*)(xr + 8 * s4) = i32x4{(int)(o[0] | ((unsigned)o[1] << 16)), (int)(o[2] | ((unsigned)o[3] << 16)),
-                                           (int)(o[4] | ((unsigned)o[5] << 16)), (int)(o[6] | ((unsigned)o[7] << 16))};
-          }
-        }
-      }
+      f16w_quantize_h<HB, G::CW, CS, NT>(H, mats.hq, c0, n, rt_l * HB, m);
       return;
     }
 #pragma unroll
@@ -569,7 +418,8 @@ static bool launch_f16w_t(crabml_hip_device* dev, const F16wMats& mats, int row_
                                                                                           row_tiles, ksplit);
   return true;
 }
-size_t gemm_f16w_xh_bytes(size_t rows, size_t k) { return ((rows + 127) / 128 * 128) * k * 2 + 4096; }
+// (tiles of 128 or 96 columns: at most 95 more than whole tiles of 128 hold)
+size_t gemm_f16w_xh_bytes(size_t rows, size_t k) { return ((rows + 127) / 128 * 128 + 96) * k * 2 + 4096; }
 // the weight formats the kernel covers, and the rows' format each pairs with (CpuTensorBuf::quantize's choice: buf/api.rs:142-159)
 bool gemm_f16w_covers(uint32_t w_dtype, uint32_t act_qtype) {
   if (act_qtype == CRABML_HIP_Q8_0) return w_dtype == CRABML_HIP_Q4_0 || w_dtype == CRABML_HIP_Q8_0;
@@ -628,8 +478,50 @@ bool launch_gemm_f16w(crabml_hip_device* dev, const crabml_hip_buf* const* w, co
     const char* e = getenv("CRABML_HIP_F16W");
     return h && h[0] == '1' && e ? atoi(e) : 0;
   }();
-  size_t mtot = 0;
-  for (int j = 0; j < nw; j++) mtot += m[j];
+  F16wMats mats{};
+  F16wParts parts{};
+  size_t mtot = 0, before = 0;  // rows; output elements of the matrices before j
+  mats.exp_tab = gu_exp_tab;
+  for (int j = 0; j < 3; j++) {
+    const int jj = j < nw ? j : nw - 1;
+    const char* wp = (const char*)w[jj]->ptr;
+    mats.wq[j] = (const i32x4*)wp;
+    mats.wd[j] = wp + w[jj]->wl.off_scale;
+    mats.ws2[j] = wp + w[jj]->wl.off_scale + w[jj]->wl.n_blocks * 64;  // (Q6_K: ql | qh | scales | d, common.hpp)
+    mats.ws3[j] = wp + w[jj]->wl.off_scale + w[jj]->wl.n_blocks * 80;
+    mats.out[j] = out[jj];
+    mats.out2[j] = ws + before;
+    mats.m[j] = (int)m[jj];
+    parts.out[j] = out[jj];
+    parts.part[j] = ws + before;
+    if (j < nw) {
+      mtot += m[j];
+      before += b * m[j];
+    }
+    parts.end4[j] = before / 4;
+  }
+  mats.pstride = parts.pstride = before;
+  int ksplit = 1;
+  auto finish = [&](bool gu, bool hquant) {
+    if (gu) *gu_done = hquant ? 2 : 1;
+    if (ksplit > 1 && defer_parts != nullptr && nw == 1) {
+      *defer_parts = ksplit - 1;  // the caller's next row kernel adds the pieces (ws + s * b * m, s = 0 ..) in the same order
+    } else if (ksplit > 1) {
+      parts.nparts = ksplit - 1;
+      k_addn_f32<<<(unsigned)((parts.end4[2] + 255) / 256), 256, 0, dev->stream>>>(parts);
+    }
+    return true;
+  };
+  {
+    // gate | up whose 64-row tiles give three CUs in four something to do: k stays whole (with or without the epilogue: the same sums)
+    const bool pair = nw == 2 && m[0] == m[1] && ((m[0] + 63) / 64) * ((b + 127) / 128) * 4 >= (size_t)dev->n_cu * 3;
+    const bool gu = pair && gu_exp_tab != nullptr && gu_done != nullptr;
+    const bool hquant = gu && hq != nullptr && hq->planes != nullptr && m[0] % 32 == 0;
+    if (hquant) mats.hq = *hq;
+    if (launch_f16w_wide(dev, dt, mats, m, nw, k, xh, b, pair, gu, ws != nullptr ? ws_floats : 0, &ksplit)) return finish(gu, hquant);
+    mats.hq = F16wHQuant{};
+    ksplit = 1;
+  }
   int T = f16w_col_tiles_per_wave(b, variant);
   size_t cw = 16 * (size_t)T, col128 = (b + cw - 1) / cw;  // (column tiles of the launch)
   // two fragments per wave (every B' fragment read from LDS feeds two MFMAs) when 128-row tiles still cover the chip
@@ -650,37 +542,18 @@ bool launch_gemm_f16w(crabml_hip_device* dev, const crabml_hip_buf* const* w, co
   // (gate | up alone.  512 rows, Q4_0 183 -> 173 us, the whole request 3973 -> 3785.  The other launches, cut in k to fill the chip with the smaller
   // tiles, do not gain: ffn_down 115 -> 108, wo 35 -> 44; four fragments a wave, one wave a SIMD, lose: 183 -> 211.)
   const int NW = gu && T == 8 && f16w_eight_waves(dt, (m[0] + 127) / 128 * col128, (size_t)dev->n_cu) ? 8 : 4;
-  F16wMats mats{};
-  mats.exp_tab = gu_exp_tab;
   const bool hquant = gu && hq != nullptr && hq->planes != nullptr && m[0] % 32 == 0;
   if (hquant) mats.hq = *hq;
-  F16wParts parts{};
   int row_tiles = 0;
-  size_t before = 0;  // output elements of the matrices before j
   for (int j = 0; j < 3; j++) {
-    const int jj = j < nw ? j : nw - 1;
-    const char* wp = (const char*)w[jj]->ptr;
-    mats.wq[j] = (const i32x4*)wp;
-    mats.wd[j] = wp + w[jj]->wl.off_scale;
-    mats.ws2[j] = wp + w[jj]->wl.off_scale + w[jj]->wl.n_blocks * 64;  // (Q6_K: ql | qh | scales | d, common.hpp)
-    mats.ws3[j] = wp + w[jj]->wl.off_scale + w[jj]->wl.n_blocks * 80;
-    mats.out[j] = out[jj];
-    mats.out2[j] = ws + before;
-    mats.m[j] = (int)m[jj];
-    parts.out[j] = out[jj];
-    parts.part[j] = ws + before;
-    if (j < nw) {
-      if (!gu) row_tiles += (int)((m[j] + 64 * F - 1) / (64 * F));
-      before += b * m[j];
-    }
-    if (gu) row_tiles = (int)((m[0] + 16 * NW - 1) / (16 * NW));
+    if (gu)
+      row_tiles = (int)((m[0] + 16 * NW - 1) / (16 * NW));
+    else if (j < nw)
+      row_tiles += (int)((m[j] + 64 * F - 1) / (64 * F));
     mats.tiles_end[j] = row_tiles;
-    parts.end4[j] = before / 4;
   }
-  mats.pstride = parts.pstride = before;
   // pieces of k: double while the launch is short of ~1.5 workgroups per CU, every piece keeps >= 4 chunks (and whole super-blocks),
   // and the partial buffers fit the scratch
-  int ksplit = 1;
   const size_t chunks = (k + 127) / 128;
   if (ws != nullptr && !(variant & 8) && k % 128 == 0 && !gu)
     while (ksplit < 8 && (size_t)row_tiles * col128 * ksplit < (size_t)dev->n_cu * 3 / 2 && chunks % (size_t)(4 * ksplit) == 0 &&
@@ -697,14 +570,7 @@ bool launch_gemm_f16w(crabml_hip_device* dev, const crabml_hip_buf* const* w, co
     ok = launch_f16w_fmt<WF_Q4_1>(dev, mats, row_tiles, k, xh, b, ksplit, F, variant, gu, T, NW);
   else
     ok = launch_f16w_fmt<WF_Q4_0>(dev, mats, row_tiles, k, xh, b, ksplit, F, variant, gu, T, NW);
-  if (ok && gu) *gu_done = hquant ? 2 : 1;
-  if (ok && ksplit > 1 && defer_parts != nullptr && nw == 1) {
-    *defer_parts = ksplit - 1;  // the caller's next row kernel adds the pieces (ws + s * b * m, s = 0 ..) in the same order
-  } else if (ok && ksplit > 1) {
-    parts.nparts = ksplit - 1;
-    k_addn_f32<<<(unsigned)((parts.end4[2] + 255) / 256), 256, 0, dev->stream>>>(parts);
-  }
-  return ok;
+  return ok && finish(gu, hquant);
 }
 
 void launch_add_parts(hipStream_t st, float* out, const float* ws, size_t n, int nparts) {

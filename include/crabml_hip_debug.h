@@ -60,8 +60,11 @@ int crabml_hip_debug_rhs_rows(size_t m, size_t* rows);
 /* top: steps of a greedy run that go into one graph where one step is `nodes` launches.  next: which of the sizes top, top / 2, top / 4 comes next in a run that
  * has made `made` steps and has `left` to make (its place; -1: a single step); have: the sizes that have been captured, bits by place.  Host only. */
 int crabml_hip_debug_graph_steps(size_t nodes, size_t seq_len, size_t left, size_t made, uint32_t have, int32_t* top, int32_t* next);
-/* Waves of a workgroup of the fast prompt pass's gate | up launch over `rows` > 64 rows.  Host only. */
+/* Waves of a workgroup of the fast prompt pass's gate | up launch over `rows` > 64 rows of a width that is no multiple of 256.  Host only. */
 int crabml_hip_debug_gateup_waves(uint32_t dtype, size_t hidden, size_t rows, int32_t n_cu, int32_t* waves);
+/* Tile of the fast prompt pass's weight GEMM over b > 64 rows, k a multiple of 256: fragments and column tiles of a wave, groups of waves along k in a
+ * workgroup, pieces of k in memory.  m0, m1, m2: the launch's matrices (0: none); pair: gate | up in one tile.  Host only. */
+int crabml_hip_debug_wide_tile(uint32_t dtype, size_t m0, size_t m1, size_t m2, size_t k, size_t b, int32_t pair, int32_t n_cu, size_t ws_floats, int32_t* tile);
 /* Rows of wo / ffn_down that a workgroup of a llama step takes: with the next norm in the launch or without, block-ordered sums (strict device), one or two
  * workgroups a 32-row chunk.  The launch's grid and what attention touches ahead of it both come from this.  Host only. */
 int crabml_hip_debug_residual_rows(int32_t norm_epilogue, int32_t ordered, int32_t split, int32_t* rows);

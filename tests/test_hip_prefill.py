@@ -412,3 +412,21 @@ def test_short_passes_in_pieces_of_k_equal_the_token_loop(ca, fmt, rows, width, 
     assert np.max(np.abs(first - want)) <= FAST_TOL[fmt][1] * np.max(np.abs(want))
     a.reset()
     assert np.array_equal(a.prefill(toks).view(np.uint32), first.view(np.uint32))  # (added in piece order, whoever ends first)
+
+
+# the wide weight GEMM (rows > 64, k a multiple of 256): a row more and a row less than its tiles of 96 and 128 columns; k of one, two, three (a group of waves
+# without a chunk), 11 and 16 super-blocks; matrices that end inside a tile of 128 or 256 rows
+@pytest.mark.parametrize("fmt", ["Q4_0", "Q8_0", "Q4_1", "Q4_K", "Q6_K"])
+@pytest.mark.parametrize("width,hidden,rows", [(256, 768, 65), (512, 768, 96), (512, 2816, 97), (1024, 1280, 129), (768, 4096, 193), (2048, 1024, 300)])
+def test_wide_prompt_gemm_at_the_edges_of_its_tiles(ca, fmt, width, hidden, rows):
+    shape = synth.ModelShape("wide", width, hidden, 1, width // 64, 2, 300, 512, 1e-5, None)
+    dev = ca.HipTensorDevice(0)
+    conf, w = synth.to_hip(synth.build_model(shape, synth.TYPE_BY_NAME[fmt], seed=37), dev)
+    a = ca.HipLlamaRunner(conf, w, dev, 512, True, prefill_chunk=512)
+    b = ca.HipLlamaRunner(conf, w, dev, 512, True, prefill_chunk=512, extra_flags=PREFILL_INT8_GEMM)
+    toks = [(19 * i + 7) % 300 for i in range(rows)]
+    got, want = np.array(a.prefill(toks)), np.array(b.prefill(toks))
+    # the operands' f16 roundings against exact block sums: the bound of the other prompt tests (FAST_TOL)
+    assert np.max(np.abs(got - want)) <= FAST_TOL[fmt][1] * np.max(np.abs(want))
+    a.reset()
+    assert np.array_equal(np.array(a.prefill(toks)).view(np.uint32), got.view(np.uint32))

@@ -118,3 +118,24 @@ def test_gate_up_takes_eight_waves_where_they_won(dtype, hidden, rows, waves):
     n = ctypes.c_int32()
     assert lib.crabml_hip_debug_gateup_waves(dtype, ctypes.c_size_t(hidden), ctypes.c_size_t(rows), 256, ctypes.byref(n)) == 0
     assert n.value == waves
+
+
+@pytest.mark.parametrize("k", [256, 512, 2816, 4096, 14336])
+@pytest.mark.parametrize("rows", [(4096, 0, 0), (4096, 1024, 1024), (1088, 1088, 0), (300, 0, 0)])
+def test_prompt_gemm_tiles_cover_k(rows, k):
+    """every plan of the wide prompt GEMM: pieces of whole super-blocks, none of them empty where they meet in memory, partial outputs inside the scratch, no
+    pieces in memory for gate | up, Q6_K without the tile its registers do not hold"""
+    out = (ctypes.c_int32 * 4)()
+    size = ctypes.c_size_t
+    for dtype in (Q4_0, 14):
+        for b in (65, 96, 97, 128, 203, 513, 1024, 3000):
+            for ws in (0, 1 << 22, 1 << 26):
+                for pair in (0, 1) if rows[1] == rows[0] else (0,):
+                    assert lib.crabml_hip_debug_wide_tile(dtype, size(rows[0]), size(rows[1]), size(rows[2]), size(k), size(b), pair, 256, size(ws), out) == 0
+                    f, t, groups, pieces = out
+                    assert (f, t, groups) in [(4, 8, 1), (4, 6, 1), (2, 8, 1), (2, 6, 1), (2, 8, 2), (2, 6, 2)]
+                    assert dtype != 14 or (f, t) != (4, 8)
+                    assert not pair or pieces == 1
+                    chunks = k // 128
+                    per = (-(-chunks // (groups * pieces)) + 1) // 2 * 2
+                    assert pieces == 1 or (per * (groups * pieces - 1) < chunks and (pieces - 1) * sum(rows) * b <= ws)
