@@ -106,15 +106,15 @@ struct GemvBf16 {
   // gain_out (nullable) and with its square sums by 16 columns
   unsigned short* out16 = nullptr;
   const float* gain_out = nullptr;
-  float* ss_out = nullptr;  // [nb][n_ss_out]
-  int n_ss_out = 0;
+  float* ss_out = nullptr;  // [nb][ld_ss_out]
+  int ld_ss_out = 0;
   int N = 0, K = 0, ldw = 0, ldx = 0, ldo = 0, nb = 1;  // K % 8 == 0
-  // GEMV_IN_RMS: elements the mean is over, eps, the gain (device); GEMV_IN_SPLIT: the same for the tail, with ss[b][n_ss] pieces
+  // GEMV_IN_RMS: elements the mean is over, eps, the gain (device); GEMV_IN_SPLIT: the same for the tail, with n_ss pieces of ss[b][ld_ss]
   // (GEMV_IN_BF16_RMS: such pieces too)
   int mean_n = 1;
   float eps = 0.f;
   const float* gain = nullptr;
-  int k_split = 0, n_ss = 0;
+  int k_split = 0, n_ss = 0, ld_ss = 0;  // (ld_ss: whole fours)
   const float* ss = nullptr;
   ActRanges act;
   const float* xielu = nullptr;  // {softplus(p), 1/2 + softplus(q)}
@@ -194,7 +194,9 @@ __device__ __forceinline__ float stream_elem_mix(const GemvBf16& a, int row, int
 __device__ __forceinline__ void stream_elem_out(const GemvBf16& a, int row, int b, const StreamElem& e, float v) {
   a.u[(size_t)b * a.ldo + row] = stream_elem_mix(a, row, b, e, v);
 }
-// v of 16 neighbouring columns in 16 lanes (zero outside the matrix): what the next linear reads, and its square sum.  Without out16: as f32.
+// columns of a piece of a row's square sum: a workgroup of the batched linears below owns as many at least
+__host__ __device__ inline int ss_columns(int rows) { return rows <= 8 ? 8 : 16; }
+// v of 8 or 16 neighbouring columns in as many lanes (zero outside the matrix): what the next linear reads, and its square sum.  Without out16: as f32.
 __device__ __forceinline__ void rows16_out(const GemvBf16& a, int row, int b, float v) {
   const bool in = b < a.nb && row < a.N;
   if (!a.out16) {
@@ -202,8 +204,13 @@ __device__ __forceinline__ void rows16_out(const GemvBf16& a, int row, int b, fl
     return;
   }
   if (in) a.out16[(size_t)b * a.ldo + row] = f2bf(a.gain_out ? v * a.gain_out[row] : v);
-  const float s = row16_sum_f32(v * v);
-  if (in && (row & 15) == 0) a.ss_out[(size_t)b * a.n_ss_out + (row >> 4)] = s;
+  float s = group_sum<8>(v * v);
+  if (a.nb <= 8) {  // (ss_columns)
+    if (in && (row & 7) == 0) a.ss_out[(size_t)b * a.ld_ss_out + (row >> 3)] = s;
+    return;
+  }
+  s += dpp_f<0x140>(s);
+  if (in && (row & 15) == 0) a.ss_out[(size_t)b * a.ld_ss_out + (row >> 4)] = s;
 }
 
 #define GEMV_BF16_LDS_FLOATS 8192  // rhs elements staged at a time, all rows together: a cut segment is a multiple of the steps in flight
@@ -256,7 +263,7 @@ __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
     for (int b = 0; b < NB; b++) {
       const int bb = b0 + b < a.nb ? b0 + b : a.nb - 1;
       float s = 0.f;
-      for (int i = lane; i < a.n_ss; i += 64) s += a.ss[(size_t)bb * a.n_ss + i];
+      for (int i = lane; i < a.n_ss; i += 64) s += a.ss[(size_t)bb * a.ld_ss + i];
       s = wave_sum_f32(s);
       tail[b] = 1.0f / sqrtf(s / (float)a.mean_n + a.eps);
     }
@@ -430,21 +437,30 @@ __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) { return
 // XG: f32 rows are requested and split in groups of four, as many as there are rows -- a group is a request, twelve conversions and three LDS
 // stores a lane and piece, which three rows of four groups paid for in full (f32 compute, us, 4 rows, all groups / one: 11264 x 2048
 // 17.3 / 12.2, gate | up of 16384 x 2048 18.5 / 16.1).
-template <int RT, int SPL, int W, int D, int IN, int OUT, bool NTW, int XG = 4>
+// XG = 1 and bf16 rows: up to eight of them, one request for a piece instead of two.
+// HALF (up to eight rows): a workgroup owns 8 weight rows, where 16 would leave half of the CUs without one (a CU draws some 25 KB/us, however much it asks
+// for).  A step is two neighbouring pieces of k: the upper eight rows of the weight tile are the same weights' second piece, so a request is as wide as
+// ever, and each piece of the rhs multiplies the whole tile -- the half of its product that the other piece's weights made is dropped.  Us a launch, 4
+// rows, streams behind it: 2048 x 8192 11.3 -> 9.4, 2048 x 2048 with a tail 6.3 -> 5.9.  (16 rows, whose rhs is as many bytes as the weights of 16 rows: 2048 x
+// 8192 12.2 -> 11.7, 2048 x 4096 6.2 -> 6.8; twice as many pieces of square sums to read cost the linears behind them more.)
+template <int RT, int SPL, int W, int D, int IN, int OUT, bool NTW, int XG = 4, bool HALF = false>
 __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
   constexpr int LD = 20, NT = 64 * W;
   constexpr bool XB = IN == GEMV_IN_BF16 || IN == GEMV_IN_BF16_RMS || IN == GEMV_IN_BF16_SPLIT, NORM = IN == GEMV_IN_RMS || IN == GEMV_IN_RMSV;
   constexpr bool PIECES = IN == GEMV_IN_BF16_RMS || IN == GEMV_IN_BF16_SPLIT, TAIL = IN == GEMV_IN_BF16_SPLIT;
-  constexpr int XR = XB ? 2 : XG;  // requests for a piece of the rhs
+  constexpr int XR = XB ? (XG == 1 ? 1 : 2) : XG;  // requests for a piece of the rhs
+  constexpr int WR = HALF ? 8 : 16 * RT, KP = HALF ? 2 : 1;  // weight rows of the workgroup; pieces of k a step
   static_assert(!XB || SPL == 1, "a bf16 rhs has one piece");
+  constexpr bool EIGHT = XB && XG == 1;
+  static_assert(!HALF || (EIGHT && RT == 1), "eight weight rows: up to eight bf16 rows");
   union Lds {
-    unsigned short in[W][RT + SPL][16 * 64];  // a wave's tiles: weights, rhs
+    unsigned short in[W][RT + SPL * KP][16 * 64];  // a wave's tiles: weights, rhs
     float tile[W][RT][16 * LD];
   };
   __shared__ __attribute__((aligned(16))) Lds lds;
   __shared__ float sums[W][16], scale[16];
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_wg(), fr = lane & 15, fk = lane >> 4;
-  const int row0 = blockIdx.x * 16 * RT;
+  const int row0 = blockIdx.x * WR;
   // where this lane's part of a request lies: 16 bytes, eight lanes a row (f32: sixteen)
   const int r8 = lane >> 3, c8 = lane & 7, r16 = lane >> 4, c16 = lane & 15;
   // (32-bit offsets from a scalar base)
@@ -454,7 +470,7 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
   for (int t = 0; t < RT; t++)
 #pragma unroll
     for (int j = 0; j < 2; j++) {
-      const int row = t * 16 + j * 8 + r8;
+      const int row = HALF ? r8 : t * 16 + j * 8 + r8;
       wo[t][j] = (unsigned)(row0 + row < a.N ? row : a.N - 1 - row0) * (unsigned)a.ldw * 2 + c8 * 16;
     }
 #pragma unroll
@@ -462,35 +478,35 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
     const int b = XB ? j * 8 + r8 : j * 4 + r16;
     xo[j] = (unsigned)(b < a.nb ? b : a.nb - 1) * (unsigned)a.ldx * (XB ? 2 : 4) + (XB ? c8 : c16) * 16;
   }
-  i32x4 wv[D][RT][2], xv[D][XR];
+  i32x4 wv[D][RT][2], xv[D][KP * XR];
   f32x4 gv[D];
+  const int pieces = a.K / 64, n = (pieces + KP - 1) / KP, last = n - 1;
   auto request = [&](int d, int i) {
-    const char *w = wb + i * 128, *x = xbase + i * (XB ? 128 : 256);
+    const char *w = wb + i * (128 * KP), *x = xbase + i * (XB ? 128 * KP : 256);
+    const int second = HALF && 2 * i + 1 >= pieces ? 0 : 128;  // (an odd piece at the end: itself again, not used)
 #pragma unroll
     for (int t = 0; t < RT; t++)
 #pragma unroll
-      for (int j = 0; j < 2; j++) wv[d][t][j] = ld<NTW>((const i32x4*)(w + wo[t][j]));
+      for (int j = 0; j < 2; j++) wv[d][t][j] = ld<NTW>((const i32x4*)(w + (HALF ? j * second : 0) + wo[t][j]));
 #pragma unroll
-    for (int j = 0; j < XR; j++) xv[d][j] = *(const i32x4*)(x + xo[j]);
+    for (int h = 0; h < KP; h++)
+#pragma unroll
+      for (int j = 0; j < XR; j++) xv[d][h * XR + j] = *(const i32x4*)(x + h * second + xo[j]);
     if constexpr (IN == GEMV_IN_RMSV) gv[d] = *(const f32x4*)(gb + i * 256 + (unsigned)c16 * 16);
   };
-  const int n = a.K / 64, last = n - 1;
-  // a row's sum of squares: NT / 16 threads, its first pieces requested ahead of the weights (loads come back in order)
-  constexpr int QT = NT / 16, QP = 4;
-  const int q_row = tid / QT, q_at = tid % QT;
-  const float* q_ss = PIECES ? a.ss + (size_t)(q_row < a.nb ? q_row : a.nb - 1) * a.n_ss : nullptr;
-  float q_v[QP];
-  if constexpr (PIECES) {
-#pragma unroll
-    for (int u = 0; u < QP; u++) q_v[u] = q_ss[q_at + u * QT < a.n_ss ? q_at + u * QT : 0];
-  }
+  // a row's sum of squares: QT threads, four pieces a request, the first ahead of the weights (loads come back in order)
+  constexpr int QT = EIGHT ? 64 : NT / 16;
+  const int q_row = tid / QT, q_at = tid % QT, n4 = (a.n_ss + 3) / 4;
+  const f32x4* q_ss = PIECES ? (const f32x4*)(a.ss + (size_t)(q_row < a.nb ? q_row : a.nb - 1) * a.ld_ss) : nullptr;
+  f32x4 q_v = {0.f, 0.f, 0.f, 0.f};
+  if constexpr (PIECES) q_v = q_ss[q_at < n4 ? q_at : 0];
   float tail[XR], sq[XR];  // of row 4 j + r16
   const float* t_ss[XR];
 #pragma unroll
   for (int j = 0; j < XR; j++) {
     tail[j] = sq[j] = 0.f;
     if constexpr (IN == GEMV_IN_SPLIT) {  // (the first pieces of every row: ahead of the weights, too)
-      t_ss[j] = a.ss + (size_t)(j * 4 + r16 < a.nb ? j * 4 + r16 : a.nb - 1) * a.n_ss;
+      t_ss[j] = a.ss + (size_t)(j * 4 + r16 < a.nb ? j * 4 + r16 : a.nb - 1) * a.ld_ss;
       tail[j] = t_ss[j][c16 < a.n_ss ? c16 : 0];
     }
   }
@@ -498,13 +514,22 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
 #pragma unroll
     for (int d = 0; d < D; d++) request(d, wave + d * W < n ? wave + d * W : last);  // (clamped: no branch between the requests)
   }
-  constexpr int ELEMS = (RT * 256 + NT - 1) / NT;
+  constexpr int RB = HALF ? 3 : 4, ELEMS = (WR * 16 + NT - 1) / NT;
+  // result j of the tile: weight row t 16 + r of the workgroup, row b of the rhs
+  auto of = [&](int j, int& t, int& b, int& r) {
+    t = j >> 8;
+    b = (j >> RB) & 15;
+    r = j & ((1 << RB) - 1);
+  };
   StreamElem elem[ELEMS];  // of this thread's results: element tid + NT i of the tile
   if constexpr (OUT == GEMV_OUT_STREAMS) {
 #pragma unroll
     for (int i = 0; i < ELEMS; i++) {
-      const int j = tid + i * NT, b = (j >> 4) & 15, row = row0 + (j >> 8) * 16 + (j & 15);
-      if (j < RT * 256 && b < a.nb && row < a.N) stream_elem_load(a, row, b, elem[i]);
+      const int j = tid + i * NT;
+      int t, b, r;
+      of(j, t, b, r);
+      const int row = row0 + t * 16 + r;
+      if (j < WR * 16 && b < a.nb && row < a.N) stream_elem_load(a, row, b, elem[i]);
     }
   }
   if constexpr (IN == GEMV_IN_SPLIT) {
@@ -515,11 +540,11 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
       tail[j] = 1.0f / sqrtf(row16_sum_f32(t) / (float)a.mean_n + a.eps);
     }
   }
-  f32x4 acc[RT], acc2[RT];  // (TAIL: what is normalized apart)
+  f32x4 acc[RT * KP], acc2[RT * KP];  // (TAIL: what is normalized apart)
 #pragma unroll
-  for (int t = 0; t < RT; t++) acc[t] = acc2[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < RT * KP; t++) acc[t] = acc2[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   unsigned short(*mine)[16 * 64] = lds.in[wave];
-  auto multiply = [&](const i32x4 (&wc)[RT][2], const i32x4 (&xc)[XR], const f32x4& gc, int i) {
+  auto multiply = [&](const i32x4 (&wc)[RT][2], const i32x4 (&xc)[KP * XR], const f32x4& gc, int i) {
 #pragma unroll
     for (int t = 0; t < RT; t++)
 #pragma unroll
@@ -529,10 +554,12 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
       }
     if constexpr (XB) {
 #pragma unroll
-      for (int j = 0; j < 2; j++) {
-        const int r = j * 8 + r8;
-        *(i32x4*)&mine[RT][r * 64 + ((c8 ^ ((r >> 1) & 7)) * 8)] = xc[j];
-      }
+      for (int h = 0; h < KP; h++)
+#pragma unroll
+        for (int j = 0; j < XR; j++) {  // (rows 8 .. 15 that are not there: whatever LDS holds, in columns that are not stored)
+          const int r = j * 8 + r8;
+          *(i32x4*)&mine[RT + h][r * 64 + ((c8 ^ ((r >> 1) & 7)) * 8)] = xc[h * XR + j];
+        }
     } else {
 #pragma unroll
       for (int j = 0; j < XR; j++) {
@@ -561,6 +588,26 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
       }
     }
     wave_lds_order();
+    if constexpr (HALF) {
+      bf16x8 w[2];
+#pragma unroll
+      for (int u = 0; u < 2; u++) w[u] = *(const bf16x8*)&mine[0][fr * 64 + (((u * 4 + fk) ^ ((fr >> 1) & 7)) * 8)];
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        if (2 * i + h >= pieces) break;  // (uniform)
+        const bool apart = TAIL && (2 * i + h) * 64 >= a.k_split;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          const bf16x8 x = *(const bf16x8*)&mine[1 + h][fr * 64 + (((u * 4 + fk) ^ ((fr >> 1) & 7)) * 8)];
+          if (apart)
+            acc2[h] = mfma_bf16(w[u], x, acc2[h]);
+          else
+            acc[h] = mfma_bf16(w[u], x, acc[h]);
+        }
+      }
+      wave_lds_order();
+      return;
+    }
 #pragma unroll
     for (int u = 0; u < 2; u++) {
       const int at = fr * 64 + (((u * 4 + fk) ^ ((fr >> 1) & 7)) * 8);
@@ -600,19 +647,25 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
     }
   }
   if constexpr (PIECES) {
-    float t = 0.f;
+    f32x4 t4 = {0.f, 0.f, 0.f, 0.f};
+    auto take = [&](int q, f32x4 v) {  // (behind the last piece: whatever is there)
 #pragma unroll
-    for (int u = 0; u < QP; u++) t += q_at + u * QT < a.n_ss ? q_v[u] : 0.f;
-    for (int i = q_at + QP * QT; i < a.n_ss; i += QT) t += q_ss[i];
-    t = row16_sum_f32(t);
+      for (int e = 0; e < 4; e++) t4[e] += 4 * q + e < a.n_ss ? v[e] : 0.f;
+    };
+    take(q_at, q_v);
+    for (int i = q_at + QT; i < n4; i += QT) take(i, q_ss[i]);
+    float t = row16_sum_f32((t4[0] + t4[1]) + (t4[2] + t4[3]));
     t += __shfl_xor(t, 16, 64);
     if constexpr (QT == 64) t += __shfl_xor(t, 32, 64);
-    if (q_at == 0) scale[q_row] = (!TAIL && a.gain ? *a.gain : 1.0f) / sqrtf(t / (float)a.mean_n + a.eps);
+    if (q_at == 0 && q_row < 16) scale[q_row] = (!TAIL && a.gain ? *a.gain : 1.0f) / sqrtf(t / (float)a.mean_n + a.eps);
   }
   __syncthreads();  // (the tiles of results take the place of the operands')
   if constexpr (TAIL) {
 #pragma unroll
-    for (int t = 0; t < RT; t++) acc[t] += acc2[t] * scale[fr];
+    for (int t = 0; t < RT * KP; t++) acc[t] += acc2[t] * scale[fr];
+  }
+  if constexpr (HALF) {
+    if (fk >= 2) acc[0] = acc[1];  // the second piece's weights are the tile's upper eight rows
   }
   // lane: weight rows 4 fk .. of rhs row fr
 #pragma unroll
@@ -627,15 +680,21 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
     }
     __syncthreads();
   }
-  if constexpr (OUT == GEMV_OUT_GLU) {
-    for (int i = tid; i < RT * 128; i += NT) {
-      const int t = i >> 7, b = (i >> 3) & 15, r = (i & 7) * 2, row = row0 + t * 16 + r;
-      float gate = 0.f, up = 0.f;
+  auto met = [&](int t, int b, int r) {  // the waves' sums
+    float v = 0.f;
 #pragma unroll
-      for (int w = 0; w < W; w++) {
-        gate += lds.tile[w][t][b * LD + r];
-        up += lds.tile[w][t][b * LD + r + 1];
-      }
+    for (int w = 0; w < W; w++) {
+      v += lds.tile[w][t][b * LD + r];
+      if constexpr (HALF) v += lds.tile[w][t][b * LD + 8 + r];
+    }
+    return v;
+  };
+  if constexpr (OUT == GEMV_OUT_GLU) {
+    for (int i = tid; i < WR * 8; i += NT) {
+      int t, b, r;
+      of(2 * i, t, b, r);
+      const int row = row0 + t * 16 + r;
+      float gate = met(t, b, r), up = met(t, b, r + 1);
       if constexpr (NORM || IN == GEMV_IN_BF16_RMS) {
         gate *= scale[b];
         up *= scale[b];
@@ -653,24 +712,22 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
   if constexpr (OUT == GEMV_OUT_STREAMS) {
 #pragma unroll
     for (int i = 0; i < ELEMS; i++) {
-      const int j = tid + i * NT, t = j >> 8, b = (j >> 4) & 15, r = j & 15, row = row0 + t * 16 + r;
-      if (j >= RT * 256) break;  // (whole waves)
+      const int j = tid + i * NT;
+      if (j >= WR * 16) break;  // (whole waves)
+      int t, b, r;
+      of(j, t, b, r);
+      const int row = row0 + t * 16 + r;
       float u = 0.f;
-      if (b < a.nb && row < a.N) {
-        float v = 0.f;
-#pragma unroll
-        for (int w = 0; w < W; w++) v += lds.tile[w][t][b * LD + r];
-        u = stream_elem_mix(a, row, b, elem[i], v);
-      }
+      if (b < a.nb && row < a.N) u = stream_elem_mix(a, row, b, elem[i], met(t, b, r));
       rows16_out(a, row, b, u);
     }
     return;
   }
-  for (int i = tid; i < RT * 256; i += NT) {
-    const int t = i >> 8, b = (i >> 4) & 15, r = i & 15, row = row0 + t * 16 + r;
-    float v = 0.f;
-#pragma unroll
-    for (int w = 0; w < W; w++) v += lds.tile[w][t][b * LD + r];
+  for (int i = tid; i < WR * 16; i += NT) {
+    int t, b, r;
+    of(i, t, b, r);
+    const int row = row0 + t * 16 + r;
+    float v = met(t, b, r);
     if constexpr (NORM || IN == GEMV_IN_BF16_RMS) v *= scale[b];
     if constexpr (OUT == GEMV_OUT_RESIDUAL) {
       float x = 0.f;
@@ -699,6 +756,12 @@ template <int RT, int SPL, int W, int IN, int OUT, bool NTW>
 inline void launch_gemv16_t(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a, int n_cu) {
   constexpr int D = IN < GEMV_IN_BF16 || RT == 2 ? 2 : OUT == GEMV_OUT_STREAMS ? 3 : 4;  // (registers: sixteen waves a CU)
   const dim3 grid((a.N + 16 * RT - 1) / (16 * RT));
+  if constexpr (IN >= GEMV_IN_BF16) {
+    if (a.nb <= 8) {
+      launch_k(st, rec, k_gemv16_bf16<RT, SPL, W, D, IN, OUT, NTW, 1>, grid, dim3(64 * W), 0, a);
+      return;
+    }
+  }
   if constexpr (SPL == 3) {
     if (a.nb <= 4) {
       launch_k(st, rec, k_gemv16_bf16<RT, SPL, W, D, IN, OUT, NTW, 1>, grid, dim3(64 * W), 0, a);
@@ -723,6 +786,11 @@ inline void launch_gemv16_n(hipStream_t st, crabml_hip_device::ProfRec* rec, con
     return;
   }
   if constexpr (IN >= GEMV_IN_BF16) {
+    if (deep && (a.N + 15) / 16 * 2 <= n_cu && a.nb <= 8) {
+      // (two steps out a wave: three or four make a whole decode step of 3 to 8 rows 0.5 to 3 % longer)
+      launch_k(st, rec, k_gemv16_bf16<1, SPL, 16, 2, IN, OUT, NTW, 1, true>, dim3((a.N + 7) / 8), dim3(1024), 0, a);
+      return;
+    }
     if (deep) {
       launch_gemv16_t<1, SPL, 16, IN, OUT, NTW>(st, rec, a, n_cu);
       return;

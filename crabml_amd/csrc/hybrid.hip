@@ -81,7 +81,7 @@ struct crabml_hip_hybrid {
   // the feed-forward's middle
   unsigned short *st_x16 = nullptr, *st_cat16 = nullptr, *st_u16 = nullptr;
   float* st_xss = nullptr;
-  int n_xss = 0;
+  int ld_xss = 0;
   float *st_in = nullptr, *st_vk = nullptr, *st_q = nullptr, *st_lpart = nullptr;  // streams: what the next linear reads; kept values; latent queries, partials
   int ld_vk = 0, ld_kv = 0, ld_lat = 0, ld_rot = 0;
   size_t hist = 0;  // earlier positions a latent layer can see
@@ -475,6 +475,7 @@ MixStep mix_step(const Ctx* c, const Run& run, int B) {
   m.cat = c->st_cat;
   m.cat16 = rows16(c, B) ? c->st_cat16 : nullptr;
   m.ss = c->st_ss;
+  m.ld_ss = up(L.li.H * L.li.slices, 4);
   m.part = c->st_part;
   m.tick = c->st_tick;
   m.v_kept = c->st_vk;
@@ -531,7 +532,8 @@ void normed_linear(Ctx* c, crabml_hip_device::ProfRec* rec, GemvBf16 g) {
   if (rows16(c, g.nb)) {
     g.x16 = c->st_x16;
     g.ss = c->st_xss;
-    g.n_ss = c->n_xss;
+    g.n_ss = (c->width + ss_columns(g.nb) - 1) / ss_columns(g.nb);
+    g.ld_ss = c->ld_xss;
     if (c->streams) g.gain = nullptr;  // (in the rows already)
   }
   if (c->streams)
@@ -545,7 +547,7 @@ void next_rows16(Ctx* c, GemvBf16* g, const float* gain) {
   g->out16 = c->st_x16;
   g->gain_out = c->streams ? gain : nullptr;
   g->ss_out = c->st_xss;
-  g->n_ss_out = c->n_xss;
+  g->ld_ss_out = c->ld_xss;
 }
 
 // the classifier on f32 rows, or (a step's own, f32_rows = false) on the rows the last linear left
@@ -619,7 +621,7 @@ void enqueue_front(Ctx* c, int B, bool pick, bool embed) {
   }
   k_front_rows<<<B, embed ? 1024 : 64, 0, c->dev->stream>>>(p, c->embed, c->st_seq, embed ? c->width : 0, c->ldx, c->cfg.embed_scale, c->freq, c->st_x, c->keep_emb ? c->st_emb : nullptr,
                                                c->runs[0].add_vec, streams_at_start(c, stride), c->st_in, rows16(c, B) ? c->st_x16 : nullptr,
-                                               c->streams ? c->layers[c->runs[0].layer].norm1 : nullptr, c->st_xss, c->n_xss);
+                                               c->streams ? c->layers[c->runs[0].layer].norm1 : nullptr, c->st_xss, c->ld_xss);
 }
 
 // One step of B rows: front, layers, classifier, and the sampler if asked for.  Inside a graph of several steps the sampler's second stage and the next
@@ -677,6 +679,7 @@ int enqueue_step(Ctx* c, int B, bool sample, bool prof, bool led = false, bool l
       g.eps = eps;
       g.k_split = L.lin_off;
       g.n_ss = L.li.H * L.li.slices;
+      g.ld_ss = up(g.n_ss, 4);
       g.ss = c->st_ss;
       if (!L.ff) {
         g.add_rows = add_rows;
@@ -1221,7 +1224,7 @@ int create_impl(Ctx* c, const crabml_hip_hybrid_layer_t* layers, const crabml_hi
       }
       tick = std::max(tick, slots);
     }
-    ss = std::max(ss, (size_t)HYB_STEP_ROWS * L.li.H * L.li.slices);
+    ss = std::max(ss, (size_t)HYB_STEP_ROWS * up(L.li.H * L.li.slices, 4));
   }
   // the order of layer runs, and each run's place in a sequence's slab
   auto add_run = [&](size_t layer, bool first, size_t t) {
@@ -1278,9 +1281,9 @@ int create_impl(Ctx* c, const crabml_hip_hybrid_layer_t* layers, const crabml_hi
   CH_TRY(dalloc_n(c, B * c->ld_cat, &c->st_cat));
   CH_TRY(dalloc_n(c, B * c->ld_u, &c->st_u));
   if (!c->f32) {
-    c->n_xss = (c->width + 15) / 16;
+    c->ld_xss = up((c->width + 7) / 8, 4);
     CH_TRY(dalloc_n(c, B * c->ldx, &c->st_x16));
-    CH_TRY(dalloc_n(c, B * c->n_xss, &c->st_xss));
+    CH_TRY(dalloc_n(c, B * c->ld_xss, &c->st_xss));
     CH_TRY(dalloc_n(c, B * c->ld_cat, &c->st_cat16));
     CH_TRY(dalloc_n(c, B * c->ld_u, &c->st_u16));
   }

@@ -39,7 +39,7 @@ struct RowPick {
 __global__ __launch_bounds__(1024) void k_front_rows(const RowPick pick, const unsigned short* __restrict__ table, StepSeq* __restrict__ seq, int width, int ldx,
                                                      float scale, const double* __restrict__ freq, float* __restrict__ x, float* __restrict__ emb,
                                                      const float* __restrict__ add_vec, const StreamMix sm, float* __restrict__ u,
-                                                     unsigned short* __restrict__ x16, const float* __restrict__ gain, float* __restrict__ xss, int n_xss) {
+                                                     unsigned short* __restrict__ x16, const float* __restrict__ gain, float* __restrict__ xss, int ld_xss) {
   const int b = blockIdx.x, tid = threadIdx.x;
   int token = seq[b].token, pos = seq[b].pos;
   if (pick.pv) {
@@ -85,8 +85,10 @@ __global__ __launch_bounds__(1024) void k_front_rows(const RowPick pick, const u
       }
       if (!x16) continue;
       if (in) x16[(size_t)b * ldx + c] = f2bf(gain ? r * gain[c] : r);
-      const float q = row16_sum_f32(r * r);
-      if (in && (c & 15) == 0) xss[(size_t)b * n_xss + (c >> 4)] = q;
+      const int sc = ss_columns(gridDim.x);
+      float q = group_sum<8>(r * r);
+      if (sc == 16) q += dpp_f<0x140>(q);
+      if (in && c % sc == 0) xss[(size_t)b * ld_xss + c / sc] = q;
     }
   }
 }
@@ -99,7 +101,8 @@ struct MixStep {
   const float* proj = nullptr;  // [B][ldp]
   float* cat = nullptr;         // [B][ldc]: attention columns from 0, linear columns from lin_off
   unsigned short* cat16 = nullptr;  // the same as bf16, instead (nullable)
-  float* ss = nullptr;          // [B][H * slices] square sums of the linear branch
+  float* ss = nullptr;          // [B][ld_ss]: H * slices square sums of the linear branch
+  int ld_ss = 0;
   float* part = nullptr;        // attention partials
   float* v_kept = nullptr;      // [B][ld_vk] values that VMIX_KEEP leaves
   int ld_vk = 0;
@@ -446,7 +449,7 @@ __device__ __forceinline__ void mix_linear(const MixStep& a, int blk, float* lds
     }
     const bool in = used && lane < LIN_SLICE && oc < g.V;
     const float ss = wave_sum_f32(in ? r * r : 0.f);
-    if (used && lane == 0) a.ss[(size_t)b * g.H * g.slices + h * g.slices + slice] = ss;
+    if (used && lane == 0) a.ss[(size_t)b * a.ld_ss + h * g.slices + slice] = ss;
     if (in) cat_out(a.cat, a.cat16, (size_t)b * a.ldc + a.lin_off + occ, r * factor);
   }
 }

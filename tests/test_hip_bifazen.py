@@ -205,6 +205,21 @@ def test_many_heads_times_many_sequences(ca, hdev, tmp_path, f32):
         close(r.step([(s, [t[-k]], [0]) for s, t in zip(seqs, toks)]), [w[-k] for w in want], f32)
 
 
+# as the hybrid decoder's test of that name, into residual streams
+@pytest.mark.parametrize("rows", [3, 8, 9])
+@pytest.mark.parametrize("streams", [1, 4, 6])
+def test_decode_linears_of_few_columns_and_long_rows(ca, hdev, tmp_path, streams, rows):
+    c = sb.config(84, 90, [sb.latent(18, 16, 8, 116, 40, 70, 2112), sb.attention(16, 2, 16, 130, 24, 4096)], streams=streams)
+    m = Model(c, tmp_path / "m", seed=streams)
+    r = m.runner(ca, hdev, False)
+    toks = [m.tokens(7 + i, seed=400 + i) for i in range(rows)]
+    want = [m.oracle(t) for t in toks]
+    seqs = [r.open() for _ in toks]
+    r.step([(s, t[:-3], []) for s, t in zip(seqs, toks)])
+    for k in (3, 2, 1):
+        close(r.step([(s, [t[-k]], [0]) for s, t in zip(seqs, toks)]), [w[-k] for w in want], False)
+
+
 def test_rows_of_a_batch_do_not_change_each_other(ca, hdev, models):
     m = models("plain")
     r = m.runner(ca, hdev, True)

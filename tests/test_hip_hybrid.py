@@ -167,6 +167,22 @@ def test_unequal_batch_against_each_alone(ca, hdev, models, name, f32):
     close(got, [w[-2] for w in want], f32)
 
 
+# three to eight rows, long rows of a few columns: the linears whose workgroups own eight weight rows (a piece of k without a partner at 2112, widths that end inside
+# a workgroup, the linear branch's norm inside the row); nine: sixteen of them
+@pytest.mark.parametrize("rows", [3, 8, 9])
+@pytest.mark.parametrize("width", [84, 200])
+def test_decode_linears_of_few_columns_and_long_rows(ca, hdev, tmp_path, width, rows):
+    c = sh.config(width, 90, [sh.layer(8, 1, 16, 128, 24, 9, 16, 120, 2112), sh.layer(2, 1, 16, 16, 24, 2, 16, 16, 4096)])
+    m = Model(c, tmp_path / "m", seed=width)
+    r = m.runner(ca, hdev, False)
+    toks = [m.tokens(7 + i, seed=400 + i) for i in range(rows)]
+    want = [m.oracle(t) for t in toks]
+    seqs = [r.open() for _ in toks]
+    r.step([(s, t[:-3], []) for s, t in zip(seqs, toks)])
+    for k in (3, 2, 1):
+        close(r.step([(s, [t[-k]], [0]) for s, t in zip(seqs, toks)]), [w[-k] for w in want], False)
+
+
 def test_rows_of_a_batch_do_not_change_each_other(ca, hdev, models):
     """the same sequence in the same step function: its logits do not move when others are added or leave"""
     m = models("plain")
