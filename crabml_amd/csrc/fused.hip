@@ -16,6 +16,7 @@
 //   k_gemv_res     wo / ffn_down matmul_vec + add_inplace(residual)
 //   k_gateup       ffn_gate/ffn_up matmul_vec + silu_inplace + mul_inplace
 //   k_step_front   greedy sampler (last maximum) + token/position advance, embedding, first norm (+ quantize)
+#include <atomic>
 #include <chrono>
 #include <thread>
 #include <cmath>
@@ -23,6 +24,7 @@
 #include "fused_common.hpp"
 #include "fused_attention.hpp"
 #include "fused_ffn.hpp"
+#include "fused_small.hpp"
 #include "graph_steps.hpp"
 #include "fused_f16.hpp"
 #include "gemm_bf16.hpp"
@@ -129,6 +131,9 @@ struct crabml_hip_llama {
   float* rope = nullptr;     // [seq_len][npairs][2]
   int* state = nullptr;      // token, pos, step, (unused), serial (never reset), fault
   unsigned long long* slots = nullptr;  // dim/32 {chunk sum, epoch} granules of the norm epilogue
+  SmallLayer* small = nullptr;  // all layers in one launch (fused_small.hpp): their table ...
+  unsigned long long* small_gran = nullptr;  // ... granules
+  int small_wgs = 0;                         // ... and workgroups, as reserved (small_reserve)
   unsigned long long* a8gran = nullptr;  // Q4_K layers: granules of the attention output (dim_l) and of h (hidden_l), through which
   unsigned long long* h8gran = nullptr;  // the producing kernels assemble Q8_K super-blocks (q8k_exchange_store)
   bool q8k_producers = false;            // attention / gate-up emit the Q8_K planes of wo's / ffn_down's rhs themselves
@@ -1202,8 +1207,64 @@ int allreduce(crabml_hip_llama* c, int seg) {
   return 0;
 }
 
+// Workgroups of the one launch wait for each other and take a CU each (118 VGPRs, 16 waves): what the contexts of a process hold together stays within half
+// of a device's CUs, however many streams run, and the rest is left to launches whose workgroups wait as well.  A context past that
+// (five of 24 workgroups, four of 32, are within) keeps its launches per layer: the same bits.
+std::atomic<int>& small_reserved(int ordinal) {
+  static std::atomic<int> held[64];
+  return held[ordinal & 63];
+}
+bool small_reserve(crabml_hip_device* dev, int n) {
+  std::atomic<int>& held = small_reserved(dev->ordinal);
+  for (int now = held.load(); now + n <= dev->n_cu / 2;)
+    if (held.compare_exchange_weak(now, now + n)) return true;
+  return false;
+}
+// Small models: every layer in one launch, in the attention form that it has (fused_small.hpp)
+int enqueue_small_layers(crabml_hip_llama* c) {
+  crabml_hip_device* dev = c->dev;
+  const auto& g = c->cfg;
+  const int dim = (int)g.embedding_dim, total = dim + 2 * c->kv_dim_l;
+  const ActPtrs ad = act_ptrs(c->act_dim, dim, c->qt);
+  SmallStep a;
+  a.layers = c->small;
+  a.g_qkv = c->small_gran;
+  a.g_attn = a.g_qkv + total;
+  a.g_x1 = a.g_attn + dim;
+  a.g_x2 = a.g_x1 + dim / 32 * SMALL_XG;
+  a.g_h = a.g_x2 + dim / 32 * SMALL_XG;
+  a.state = c->state;
+  a.fault = c->state + 5;
+  a.x = c->x;
+  a.q = ad.q;
+  a.d = ad.d;
+  a.isum = (int*)ad.isum;
+  a.rope = c->rope;
+  a.exp_tab = (const unsigned short*)dev->exp_table;
+  a.L = (int)g.n_layers;
+  a.dim = dim;
+  a.kv_dim = c->kv_dim_l;
+  a.hd = c->hd;
+  a.hidden = c->hidden_l;
+  a.n_heads = c->n_heads_l;
+  a.n_kv = c->n_kv_l;
+  a.seq_cap = (int)g.seq_len;
+  a.rope_dim = (int)g.rope_dim;
+  a.npairs = c->npairs;
+  a.q_scale = 1.0f / std::sqrt((float)c->hd);
+  a.eps = g.rms_norm_eps;
+  small_kernel(c->wtype)<<<c->small_wgs, 1024, 0, dev->stream>>>(a);
+  CH_HIP(dev, hipGetLastError());
+  return 0;
+}
+
 int enqueue_step(crabml_hip_llama* c) {
   const int n = n_segments(c);
+  if (c->small && runs_attn_short(c) && !(c->dev->prof_on && !c->use_graph && !c->capturing)) {
+    if (!c->led) CH_TRY(enqueue_front(c, false));
+    CH_TRY(enqueue_small_layers(c));
+    return enqueue_segment(c, n - 1);
+  }
   for (int s = 0; s < n; s++) {
     CH_TRY(enqueue_segment(c, s));
     if (c->tp > 1 && s + 1 < n) CH_TRY(allreduce(c, s));
@@ -2370,6 +2431,16 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
     A(dim_l * 8, (void**)&c->a8gran);
     A(hidden_l * 8, (void**)&c->h8gran);
   }
+  // (heads of one workgroup each from the first position on, the hop-free norms, rows in one piece: what the one launch does)
+  const size_t small_n = g.embedding_dim + 2 * kv_dim_l + g.embedding_dim + g.embedding_dim / 32 * 2 * SMALL_XG + hidden_l / 32 * SMALL_HG;
+  if (c->defer_norm && c->attn_short_from == 0 && g.use_f16_kv_cache && !mixed && !c->attn_row_apart && ext_kc == nullptr && !dry &&
+      !(g.flags & (CRABML_HIP_LLAMA_NO_SMALL_LAYERS | CRABML_HIP_LLAMA_SPLIT_CHUNKS_ALWAYS | CRABML_HIP_LLAMA_SPLIT_CHUNKS_NEVER)) &&
+      small_fits(g.n_layers, g.embedding_dim, kv_dim_l, hidden_l, n_heads_l, hd) &&
+      small_reserve(dev, small_workers((int)g.embedding_dim, (int)kv_dim_l, (int)hidden_l, (int)n_heads_l))) {
+    c->small_wgs = small_workers((int)g.embedding_dim, (int)kv_dim_l, (int)hidden_l, (int)n_heads_l);
+    A(g.n_layers * sizeof(SmallLayer), (void**)&c->small);
+    A(small_n * 8, (void**)&c->small_gran);
+  }
   c->out_cap = (int)g.seq_len;
   A((size_t)c->out_cap * 4, (void**)&c->out_tokens);
   A(ARGMAX_BLOCKS * 4, (void**)&c->am_val);
@@ -2401,6 +2472,15 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
     // vocabulary split: the entries of the other ranks' shards read -inf (an element-wise max over the ranks is the all-gather)
     if (e == hipSuccess && c->split_vocab) e = hipMemsetD32Async((hipDeviceptr_t)c->logits, (int)0xff800000u, g.vocab_size, dev->stream);
     if (e == hipSuccess) e = hipMemsetAsync(c->slots, 0, (g.embedding_dim / 16 + g.embedding_dim) * 8, dev->stream);
+    std::vector<SmallLayer> layers;
+    if (c->small) {
+      for (size_t l = 0; l < g.n_layers; l++)
+        layers.push_back(SmallLayer{planes_of(c->wq[l]), planes_of(c->wk[l]), planes_of(c->wv[l]), planes_of(c->wo[l]), planes_of(c->gate[l]), planes_of(c->up[l]),
+                                    planes_of(c->down[l]), (const float*)c->rms_ffn[l]->ptr,
+                                    (const float*)(l + 1 < g.n_layers ? c->rms_att[l + 1] : c->rms_final)->ptr, (unsigned short*)c->kc[l], (unsigned short*)c->vc[l]});
+      if (e == hipSuccess) e = hipMemcpyAsync(c->small, layers.data(), layers.size() * sizeof(SmallLayer), hipMemcpyHostToDevice, dev->stream);
+      if (e == hipSuccess) e = hipMemsetAsync(c->small_gran, 0, small_n * 8, dev->stream);
+    }
     if (e == hipSuccess && c->a8gran) e = hipMemsetAsync(c->a8gran, 0, dim_l * 8, dev->stream);
     if (e == hipSuccess && c->h8gran) e = hipMemsetAsync(c->h8gran, 0, hidden_l * 8, dev->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(dev->stream);
@@ -2469,6 +2549,7 @@ int crabml_hip_llama_destroy(crabml_hip_llama_t* c) {
       if (c->several[v].graph[z]) (void)hipGraphDestroy(c->several[v].graph[z]);
     }
   }
+  if (c->small_wgs) small_reserved(c->dev->ordinal) -= c->small_wgs;
   for (auto& a : c->allocs) pool_free(c->dev, a.first, a.second);
   for (auto* b : c->held) crabml_hip_buf_release(b);
   if (c->h_state) (void)hipHostFree(c->h_state);
@@ -2941,3 +3022,17 @@ bool lazy_ctx_has_host_logits(const crabml_hip_llama* c) { return c != nullptr &
 int lazy_ctx_fault_value(const crabml_hip_llama* c) { return c->dev->dry ? 0 : c->h_state[crabml_hip_llama::H_STATE_SLOTS * 4]; }
 
 }  // namespace crabml_hip
+
+extern "C" int crabml_hip_debug_exp_of_f16(crabml_hip_device_t* dev, uint16_t* computed, uint16_t* table) {
+  using namespace crabml_hip;
+  if (!dev || !computed || !table) return CRABML_HIP_BAD_INPUT;
+  void* d = nullptr;
+  CH_HIP(dev, hipMalloc(&d, 65536 * 2));
+  k_exp_of_f16<<<256, 256, 0, dev->stream>>>((const unsigned short*)dev->exp_table, (unsigned short*)d);
+  int rc = 0;
+  if (hipMemcpyAsync(computed, d, 65536 * 2, hipMemcpyDeviceToHost, dev->stream) != hipSuccess ||
+      hipMemcpyAsync(table, dev->exp_table, 65536 * 2, hipMemcpyDeviceToHost, dev->stream) != hipSuccess || hipStreamSynchronize(dev->stream) != hipSuccess)
+    rc = CRABML_HIP_UNEXPECTED;
+  (void)hipFree(d);
+  return rc;
+}

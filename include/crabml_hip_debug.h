@@ -62,6 +62,8 @@ int crabml_hip_debug_rhs_rows(size_t m, size_t* rows);
 int crabml_hip_debug_graph_steps(size_t nodes, size_t seq_len, size_t left, size_t made, uint32_t have, int32_t* top, int32_t* next);
 /* Waves of a workgroup of the fast prompt pass's gate | up launch over `rows` > 64 rows of a width that is no multiple of 256.  Host only. */
 int crabml_hip_debug_gateup_waves(uint32_t dtype, size_t hidden, size_t rows, int32_t n_cu, int32_t* waves);
+/* f16(exp(x)) of every f16 x as the one-launch decode step of a small model computes it, and the device's table of it: 65536 values each. */
+int crabml_hip_debug_exp_of_f16(crabml_hip_device_t* dev, uint16_t* computed, uint16_t* table);
 /* Tile of the fast prompt pass's weight GEMM over b > 64 rows, k a multiple of 256: fragments and column tiles of a wave, groups of waves along k in a
  * workgroup, pieces of k in memory.  m0, m1, m2: the launch's matrices (0: none); pair: gate | up in one tile.  Host only. */
 int crabml_hip_debug_wide_tile(uint32_t dtype, size_t m0, size_t m1, size_t m2, size_t k, size_t b, int32_t pair, int32_t n_cu, size_t ws_floats, int32_t* tile);
@@ -136,6 +138,8 @@ int crabml_hip_debug_flash_attention_rows(crabml_hip_device_t* dev, const float*
                                                               own launch (k_rows_to_f16) instead of by the kernels that quantize the rows,
                                                               and the k pieces of a split wo / ffn_down GEMM are added by their own launch
                                                               (k_addn_f32) instead of by the norm kernel that consumes them (bit-identical) */
+#define CRABML_HIP_LLAMA_NO_SMALL_LAYERS 134217728 /* A/B: a small model's decode step keeps its launches per layer instead of one launch for all
+                                                         of them (bit-identical) */
 #define CRABML_HIP_LLAMA_PREFILL_NO_GU_EPILOGUE 67108864 /* A/B, fast prompt pass: gate | up leave g and u and SiLU * mul (+ quantize) stays its own
                                                            launch, instead of being the f16 GEMM's epilogue (bit-identical) */
 #define CRABML_HIP_LLAMA_NO_K_NORM_IN 16777216 /* A/B, fast Q4_K step: wo gathers the row's sums and quantizes its output to Q8_K itself (two

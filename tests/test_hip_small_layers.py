@@ -1,0 +1,62 @@
+"""A small model's decode step with all its layers in one launch, against the step of five launches a layer, bit for bit."""
+import ctypes
+from concurrent.futures import ThreadPoolExecutor
+
+import numpy as np
+import pytest
+
+from crabml_amd import synth
+
+pytestmark = pytest.mark.gpu
+FIVE = 134217728  # CRABML_HIP_LLAMA_NO_SMALL_LAYERS
+
+
+# the smallest; heads of eight columns, as many as there are workgroups; heads that fill part of their lanes; the widest rows of each kind, with one key head
+# and with as many as fit; workgroups without rows of wo or without rows of gate and up
+@pytest.mark.parametrize("dim,hidden,layers,heads,kv_heads", [(32, 32, 1, 1, 1), (256, 96, 2, 32, 8), (288, 768, 3, 6, 6), (896, 1024, 2, 14, 1), (512, 1024, 3, 8, 4),
+                                                              (64, 992, 2, 2, 1), (320, 64, 5, 5, 5)])
+@pytest.mark.parametrize("fmt", ["Q8_0", "Q4_0"])
+def test_one_launch_equals_five_a_layer(ca, fmt, dim, hidden, layers, heads, kv_heads):
+    dev = ca.HipTensorDevice(0)
+    shape = synth.ModelShape("small", dim, hidden, layers, heads, kv_heads, 300, 160, 1e-5, None)
+    conf, w = synth.to_hip(synth.build_model(shape, synth.TYPE_BY_NAME[fmt], seed=31), dev)
+    seq = 150  # (past the first 64 and the next 128 positions, and to the last)
+    one, eager, five = (ca.HipLlamaRunner(conf, w, dev, seq, True, g, extra_flags=f) for g, f in ((True, 0), (False, 0), (True, FIVE)))
+    pos, token = 0, 3
+    for n in (1, 5, 58, 2, 70):
+        ids = one.decode_greedy(token, n)
+        assert ids == five.decode_greedy(token, n) == eager.decode_greedy(token, n), (pos, n)
+        pos, token = pos + n, ids[-1]
+    while pos < seq:
+        x, y, z = one.forward(token, pos), five.forward(token, pos), eager.forward(token, pos)
+        assert np.isfinite(x).all() and np.array_equal(x.view(np.uint32), y.view(np.uint32)) and np.array_equal(x.view(np.uint32), z.view(np.uint32)), pos
+        pos, token = pos + 1, (token * 7 + pos) % 300
+    # a prompt behind it, and steps behind the prompt
+    prompt = [(5 * i + 1) % 300 for i in range(40)]
+    one.reset()
+    five.reset()
+    x, y = one.prefill(prompt), five.prefill(prompt)
+    assert np.array_equal(np.asarray(x).view(np.uint32), np.asarray(y).view(np.uint32))
+    assert one.decode_greedy(9, 30) == five.decode_greedy(9, 30)
+
+
+def test_contexts_past_the_reserved_workgroups(ca):
+    """more contexts than half of the CUs hold, each on a stream of its own and all of them under way at once"""
+    shape = synth.ModelShape("small", 288, 768, 2, 6, 6, 300, 160, 1e-5, None)
+    model, runners = synth.build_model(shape, synth.Q8_0, seed=32), []
+    for i in range(8):
+        dev = ca.HipTensorDevice(0)
+        runners.append(ca.HipLlamaRunner(*synth.to_hip(model, dev), dev, 100, True))
+    with ThreadPoolExecutor(8) as pool:
+        ids = list(pool.map(lambda r: r.decode_greedy(3, 90), runners))
+    assert all(x == ids[0] for x in ids)
+
+
+def test_the_computed_exp_is_the_table(ca):
+    """the step's exp against the device's table, every f16"""
+    lib = ctypes.CDLL(ca.LIB_PATH)
+    dev = ca.HipTensorDevice(0)
+    got, table = np.zeros(65536, np.uint16), np.zeros(65536, np.uint16)
+    assert lib.crabml_hip_debug_exp_of_f16(ctypes.c_void_p(dev.raw_handle()), got.ctypes.data_as(ctypes.c_void_p), table.ctypes.data_as(ctypes.c_void_p)) == 0
+    nan = (table & 0x7fff) > 0x7c00
+    assert np.array_equal(got[~nan], table[~nan]) and np.all((got[nan] & 0x7fff) > 0x7c00)
