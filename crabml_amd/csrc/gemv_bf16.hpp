@@ -114,7 +114,7 @@ struct GemvBf16 {
   int mean_n = 1;
   float eps = 0.f;
   const float* gain = nullptr;
-  int k_split = 0, n_ss = 0, ld_ss = 0;  // (ld_ss: whole fours)
+  int k_split = 0, n_ss = 0, ld_ss = 0;  // (ld_ss: even)
   const float* ss = nullptr;
   ActRanges act;
   const float* xielu = nullptr;  // {softplus(p), 1/2 + softplus(q)}
@@ -439,10 +439,12 @@ __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) { return
 // 17.3 / 12.2, gate | up of 16384 x 2048 18.5 / 16.1).
 // XG = 1 and bf16 rows: up to eight of them, one request for a piece instead of two.
 // HALF (up to eight rows): a workgroup owns 8 weight rows, where 16 would leave half of the CUs without one (a CU draws some 25 KB/us, however much it asks
-// for).  A step is two neighbouring pieces of k: the upper eight rows of the weight tile are the same weights' second piece, so a request is as wide as
-// ever, and each piece of the rhs multiplies the whole tile -- the half of its product that the other piece's weights made is dropped.  Us a launch, 4
+// for).  A step is the next two pieces of k that the wave would take of 16 rows, their eight weight rows one above the other in the tile, and each is
+// multiplied by its piece of the rhs in turn (the lower and the upper half of the product are the same).  Us a launch, 4
 // rows, streams behind it: 2048 x 8192 11.3 -> 9.4, 2048 x 2048 with a tail 6.3 -> 5.9.  (16 rows, whose rhs is as many bytes as the weights of 16 rows: 2048 x
 // 8192 12.2 -> 11.7, 2048 x 4096 6.2 -> 6.8; twice as many pieces of square sums to read cost the linears behind them more.)
+// The sums of bf16 rows are the same in every form: pieces of k by wave, waves in order, square sums of 16 columns: a sequence's logits do not
+// depend on how many others, three to sixteen rows in all, share its step.
 template <int RT, int SPL, int W, int D, int IN, int OUT, bool NTW, int XG = 4, bool HALF = false>
 __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
   constexpr int LD = 20, NT = 64 * W;
@@ -480,10 +482,11 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
   }
   i32x4 wv[D][RT][2], xv[D][KP * XR];
   f32x4 gv[D];
-  const int pieces = a.K / 64, n = (pieces + KP - 1) / KP, last = n - 1;
+  const int n = a.K / 64, last = n - 1;
+  constexpr int S = KP * W;  // pieces from a step of this wave's to its next
   auto request = [&](int d, int i) {
-    const char *w = wb + i * (128 * KP), *x = xbase + i * (XB ? 128 * KP : 256);
-    const int second = HALF && 2 * i + 1 >= pieces ? 0 : 128;  // (an odd piece at the end: itself again, not used)
+    const char *w = wb + i * 128, *x = xbase + i * (XB ? 128 : 256);
+    const int second = HALF && i + W < n ? 128 * W : 0;  // (none: itself again, not used)
 #pragma unroll
     for (int t = 0; t < RT; t++)
 #pragma unroll
@@ -494,12 +497,21 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
       for (int j = 0; j < XR; j++) xv[d][h * XR + j] = *(const i32x4*)(x + h * second + xo[j]);
     if constexpr (IN == GEMV_IN_RMSV) gv[d] = *(const f32x4*)(gb + i * 256 + (unsigned)c16 * 16);
   };
-  // a row's sum of squares: QT threads, four pieces a request, the first ahead of the weights (loads come back in order)
-  constexpr int QT = EIGHT ? 64 : NT / 16;
-  const int q_row = tid / QT, q_at = tid % QT, n4 = (a.n_ss + 3) / 4;
-  const f32x4* q_ss = PIECES ? (const f32x4*)(a.ss + (size_t)(q_row < a.nb ? q_row : a.nb - 1) * a.ld_ss) : nullptr;
-  f32x4 q_v = {0.f, 0.f, 0.f, 0.f};
-  if constexpr (PIECES) q_v = q_ss[q_at < n4 ? q_at : 0];
+  // a row's sum of squares: NT / 16 threads, its first pieces requested ahead of the weights (loads come back in order).  Pieces of 8 columns: as pairs
+  constexpr int QT = NT / 16, QP = 4, QC = EIGHT && !TAIL ? 2 : 1;
+  const int q_row = tid / QT, q_at = tid % QT, n_ss = (a.n_ss + QC - 1) / QC;
+  const float* q_ss = PIECES ? a.ss + (size_t)(q_row < a.nb ? q_row : a.nb - 1) * a.ld_ss : nullptr;
+  auto square = [&](int i) -> f32x2 {
+    if constexpr (QC == 1)
+      return f32x2{q_ss[i], 0.f};
+    else
+      return *(const f32x2*)(q_ss + 2 * i);
+  };
+  f32x2 q_v[QP];
+  if constexpr (PIECES) {
+#pragma unroll
+    for (int u = 0; u < QP; u++) q_v[u] = square(q_at + u * QT < n_ss ? q_at + u * QT : 0);
+  }
   float tail[XR], sq[XR];  // of row 4 j + r16
   const float* t_ss[XR];
 #pragma unroll
@@ -512,7 +524,7 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
   }
   if (wave < n) {
 #pragma unroll
-    for (int d = 0; d < D; d++) request(d, wave + d * W < n ? wave + d * W : last);  // (clamped: no branch between the requests)
+    for (int d = 0; d < D; d++) request(d, wave + d * S < n ? wave + d * S : last);  // (clamped: no branch between the requests)
   }
   constexpr int RB = HALF ? 3 : 4, ELEMS = (WR * 16 + NT - 1) / NT;
   // result j of the tile: weight row t 16 + r of the workgroup, row b of the rhs
@@ -540,9 +552,9 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
       tail[j] = 1.0f / sqrtf(row16_sum_f32(t) / (float)a.mean_n + a.eps);
     }
   }
-  f32x4 acc[RT * KP], acc2[RT * KP];  // (TAIL: what is normalized apart)
+  f32x4 acc[RT], acc2[RT];  // (TAIL: what is normalized apart)
 #pragma unroll
-  for (int t = 0; t < RT * KP; t++) acc[t] = acc2[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < RT; t++) acc[t] = acc2[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   unsigned short(*mine)[16 * 64] = lds.in[wave];
   auto multiply = [&](const i32x4 (&wc)[RT][2], const i32x4 (&xc)[KP * XR], const f32x4& gc, int i) {
 #pragma unroll
@@ -589,20 +601,20 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
     }
     wave_lds_order();
     if constexpr (HALF) {
-      bf16x8 w[2];
-#pragma unroll
-      for (int u = 0; u < 2; u++) w[u] = *(const bf16x8*)&mine[0][fr * 64 + (((u * 4 + fk) ^ ((fr >> 1) & 7)) * 8)];
 #pragma unroll
       for (int h = 0; h < 2; h++) {
-        if (2 * i + h >= pieces) break;  // (uniform)
-        const bool apart = TAIL && (2 * i + h) * 64 >= a.k_split;
+        const int at = i + h * W;
+        if (at >= n) break;  // (uniform)
+        const bool apart = TAIL && at * 64 >= a.k_split;
+        const int r = h * 8 + (fr & 7);
 #pragma unroll
         for (int u = 0; u < 2; u++) {
+          const bf16x8 w = *(const bf16x8*)&mine[0][r * 64 + (((u * 4 + fk) ^ ((r >> 1) & 7)) * 8)];
           const bf16x8 x = *(const bf16x8*)&mine[1 + h][fr * 64 + (((u * 4 + fk) ^ ((fr >> 1) & 7)) * 8)];
           if (apart)
-            acc2[h] = mfma_bf16(w[u], x, acc2[h]);
+            acc2[0] = mfma_bf16(w, x, acc2[0]);
           else
-            acc[h] = mfma_bf16(w[u], x, acc[h]);
+            acc[0] = mfma_bf16(w, x, acc[0]);
         }
       }
       wave_lds_order();
@@ -626,17 +638,17 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
     }
     wave_lds_order();
   };
-  for (int i = wave; i < n; i += D * W) {
-    if (i + D * W < n) {
+  for (int i = wave; i < n; i += D * S) {
+    if (i + D * S < n) {
 #pragma unroll
       for (int d = 0; d < D; d++) {
-        multiply(wv[d], xv[d], gv[d], i + d * W);
-        request(d, i + (D + d) * W < n ? i + (D + d) * W : last);
+        multiply(wv[d], xv[d], gv[d], i + d * S);
+        request(d, i + (D + d) * S < n ? i + (D + d) * S : last);
       }
     } else {
 #pragma unroll
       for (int d = 0; d < D; d++)
-        if (i + d * W < n) multiply(wv[d], xv[d], gv[d], i + d * W);
+        if (i + d * S < n) multiply(wv[d], xv[d], gv[d], i + d * S);
     }
   }
   if constexpr (NORM) {
@@ -647,25 +659,23 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
     }
   }
   if constexpr (PIECES) {
-    f32x4 t4 = {0.f, 0.f, 0.f, 0.f};
-    auto take = [&](int q, f32x4 v) {  // (behind the last piece: whatever is there)
-#pragma unroll
-      for (int e = 0; e < 4; e++) t4[e] += 4 * q + e < a.n_ss ? v[e] : 0.f;
+    float t = 0.f;
+    auto take = [&](int q, f32x2 v) {  // (behind the last piece: whatever is there)
+      const float second = QC == 2 && 2 * q + 1 < a.n_ss ? v[1] : 0.f;
+      t += q < n_ss ? (QC == 2 ? v[0] + second : v[0]) : 0.f;
     };
-    take(q_at, q_v);
-    for (int i = q_at + QT; i < n4; i += QT) take(i, q_ss[i]);
-    float t = row16_sum_f32((t4[0] + t4[1]) + (t4[2] + t4[3]));
+#pragma unroll
+    for (int u = 0; u < QP; u++) take(q_at + u * QT, q_v[u]);
+    for (int i = q_at + QP * QT; i < n_ss; i += QT) take(i, square(i));
+    t = row16_sum_f32(t);
     t += __shfl_xor(t, 16, 64);
     if constexpr (QT == 64) t += __shfl_xor(t, 32, 64);
-    if (q_at == 0 && q_row < 16) scale[q_row] = (!TAIL && a.gain ? *a.gain : 1.0f) / sqrtf(t / (float)a.mean_n + a.eps);
+    if (q_at == 0) scale[q_row] = (!TAIL && a.gain ? *a.gain : 1.0f) / sqrtf(t / (float)a.mean_n + a.eps);
   }
   __syncthreads();  // (the tiles of results take the place of the operands')
   if constexpr (TAIL) {
 #pragma unroll
-    for (int t = 0; t < RT * KP; t++) acc[t] += acc2[t] * scale[fr];
-  }
-  if constexpr (HALF) {
-    if (fk >= 2) acc[0] = acc[1];  // the second piece's weights are the tile's upper eight rows
+    for (int t = 0; t < RT; t++) acc[t] += acc2[t] * scale[fr];
   }
   // lane: weight rows 4 fk .. of rhs row fr
 #pragma unroll
@@ -683,10 +693,7 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
   auto met = [&](int t, int b, int r) {  // the waves' sums
     float v = 0.f;
 #pragma unroll
-    for (int w = 0; w < W; w++) {
-      v += lds.tile[w][t][b * LD + r];
-      if constexpr (HALF) v += lds.tile[w][t][b * LD + 8 + r];
-    }
+    for (int w = 0; w < W; w++) v += lds.tile[w][t][b * LD + r];
     return v;
   };
   if constexpr (OUT == GEMV_OUT_GLU) {

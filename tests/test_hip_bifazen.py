@@ -220,6 +220,26 @@ def test_decode_linears_of_few_columns_and_long_rows(ca, hdev, tmp_path, streams
         close(r.step([(s, [t[-k]], [0]) for s, t in zip(seqs, toks)]), [w[-k] for w in want], False)
 
 
+# as the hybrid decoder's test of that name
+@pytest.mark.parametrize("streams", [1, 4])
+def test_bf16_logits_do_not_depend_on_the_rows_of_a_step(ca, hdev, tmp_path, streams):
+    c = sb.config(84, 90, [sb.latent(18, 16, 8, 116, 40, 70, 2112), sb.attention(16, 2, 16, 130, 24, 4096)], streams=streams)
+    m = Model(c, tmp_path / "m", seed=streams)
+    r = m.runner(ca, hdev, False)
+    toks = [m.tokens(12, seed=500 + i) for i in range(16)]
+    got = []
+    for rows in (3, 8, 9, 16):
+        seqs = [r.open() for _ in range(rows)]
+        for s, t in zip(seqs, toks):
+            r.step([(s, t[:-3], [])])
+        got.append(np.stack([r.step([(s, [t[-k]], [0]) for s, t in zip(seqs, toks)])[:3] for k in (3, 2, 1)]))
+        for s in seqs:
+            r.close(s)
+    assert np.isfinite(got[0]).all()
+    for other in got[1:]:
+        assert np.array_equal(other.view(np.uint32), got[0].view(np.uint32))
+
+
 def test_rows_of_a_batch_do_not_change_each_other(ca, hdev, models):
     m = models("plain")
     r = m.runner(ca, hdev, True)

@@ -183,6 +183,27 @@ def test_decode_linears_of_few_columns_and_long_rows(ca, hdev, tmp_path, width, 
         close(r.step([(s, [t[-k]], [0]) for s, t in zip(seqs, toks)]), [w[-k] for w in want], False)
 
 
+# bf16 steps of three to sixteen rows: the same sums, whatever form a linear takes (workgroups of eight weight rows or sixteen, square sums by 8 columns or 16: 84 and
+# 200 are no multiple of 16, 2112 an odd number of pieces of k)
+@pytest.mark.parametrize("width", [84, 200, 1032])
+def test_bf16_logits_do_not_depend_on_the_rows_of_a_step(ca, hdev, tmp_path, width):
+    c = sh.config(width, 90, [sh.layer(8, 1, 16, 128, 24, 9, 16, 120, 2112), sh.layer(2, 1, 16, 16, 24, 2, 16, 16, 4096)])
+    m = Model(c, tmp_path / "m", seed=width)
+    r = m.runner(ca, hdev, False)
+    toks = [m.tokens(12, seed=500 + i) for i in range(16)]
+    got = []
+    for rows in (3, 8, 9, 16):
+        seqs = [r.open() for _ in range(rows)]
+        for s, t in zip(seqs, toks):
+            r.step([(s, t[:-3], [])])
+        got.append(np.stack([r.step([(s, [t[-k]], [0]) for s, t in zip(seqs, toks)])[:3] for k in (3, 2, 1)]))
+        for s in seqs:
+            r.close(s)
+    assert np.isfinite(got[0]).all()
+    for other in got[1:]:
+        assert np.array_equal(other.view(np.uint32), got[0].view(np.uint32))
+
+
 def test_rows_of_a_batch_do_not_change_each_other(ca, hdev, models):
     """the same sequence in the same step function: its logits do not move when others are added or leave"""
     m = models("plain")
