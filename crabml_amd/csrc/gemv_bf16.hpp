@@ -785,20 +785,26 @@ inline void launch_gemv16_t(hipStream_t st, crabml_hip_device::ProfRec* rec, con
   }
   launch_k(st, rec, k_gemv16_bf16<RT, SPL, W, D, IN, OUT, NTW>, grid, dim3(64 * W), 0, a);
 }
+// bf16: of the rhs
+inline bool gemv16_deep(int N, int K, int n_cu) { return (N + 15) / 16 < n_cu && K >= 2048; }
+inline int gemv16_rows(bool bf16, int N, int K, int nb, int n_cu) {
+  if (N >= 16384) return 32;
+  return bf16 && nb <= 8 && gemv16_deep(N, K, n_cu) && (N + 15) / 16 * 2 <= n_cu ? 8 : 16;
+}
 template <int SPL, int IN, int OUT, bool NTW>
 inline void launch_gemv16_n(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a, int n_cu) {
-  const bool two = a.N >= 16384, deep = !two && (a.N + 15) / 16 < n_cu && a.K >= 2048;
-  if (two) {
+  const int rows = gemv16_rows(IN >= GEMV_IN_BF16, a.N, a.K, a.nb, n_cu);
+  if (rows == 32) {
     launch_gemv16_t<2, SPL, 8, IN, OUT, NTW>(st, rec, a, n_cu);
     return;
   }
   if constexpr (IN >= GEMV_IN_BF16) {
-    if (deep && (a.N + 15) / 16 * 2 <= n_cu && a.nb <= 8) {
+    if (rows == 8) {
       // (two steps out a wave: three or four make a whole decode step of 3 to 8 rows 0.5 to 3 % longer)
       launch_k(st, rec, k_gemv16_bf16<1, SPL, 16, 2, IN, OUT, NTW, 1, true>, dim3((a.N + 7) / 8), dim3(1024), 0, a);
       return;
     }
-    if (deep) {
+    if (gemv16_deep(a.N, a.K, n_cu)) {
       launch_gemv16_t<1, SPL, 16, IN, OUT, NTW>(st, rec, a, n_cu);
       return;
     }

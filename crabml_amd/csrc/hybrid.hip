@@ -460,8 +460,7 @@ void step_linear(Ctx* c, crabml_hip_device::ProfRec* rec, GemvBf16 g) {
 // 4 layers of width 2048 18593 -> 17965 us for 154 tokens each.  (Latent layers, hosted by k_latent_attn: 0.3 %, not kept.)
 PrefetchPlan prefetch_out(const Ctx* c, const Layer& L, int B) {
   if (B <= 2 || c->weight_bytes <= RESIDENT_MALL) return PrefetchPlan{};
-  const int rows = c->width >= 16384 ? 32 : 16;  // (a workgroup of launch_gemv16_bf16)
-  return prefetch_matrix(c->weight_bytes, PREFETCH_MODEL_HYBRID, c->width, rows, L.w_o, (size_t)L.ldc * 2, nullptr, 0);
+  return prefetch_matrix(c->weight_bytes, PREFETCH_MODEL_HYBRID, c->width, gemv16_rows(rows16(c, B), c->width, L.ldc, B, c->dev->n_cu), L.w_o, (size_t)L.ldc * 2, nullptr, 0);
 }
 
 MixStep mix_step(const Ctx* c, const Run& run, int B) {
@@ -1496,6 +1495,11 @@ extern "C" int crabml_hip_debug_graph_steps(size_t nodes, size_t seq_len, size_t
   if (!top || !next) return CRABML_HIP_BAD_INPUT;
   *top = crabml_hip::steps_a_graph(nodes, seq_len);
   *next = crabml_hip::next_size(left, made, *top, have, 0);
+  return 0;
+}
+extern "C" int crabml_hip_debug_step_linear_rows(int32_t bf16, int32_t n, int32_t k, int32_t nb, int32_t n_cu, int32_t* rows) {
+  if (!rows || n < 1 || k < 1 || nb < 3 || n_cu < 1) return CRABML_HIP_BAD_INPUT;
+  *rows = crabml_hip::gemv16_rows(bf16 != 0, n, k, nb, n_cu);
   return 0;
 }
 extern "C" int crabml_hip_debug_prefetch(int32_t hybrid, size_t model_bytes, int32_t m, int32_t rows, size_t row_bytes, size_t row_bytes2, size_t* bytes) {

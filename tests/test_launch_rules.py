@@ -64,6 +64,16 @@ def test_rows_of_the_residual_linears():
         assert rows.value == want, args
 
 
+def test_rows_of_a_steps_linears():
+    """bf16 rows: eight weight rows a workgroup for up to eight of them where sixteen leave half of the CUs idle and the rows are long, thirty-two from 16384 on; f32
+    rows never eight.  What the mixer touches ahead of w_o is cut by the same rule."""
+    for (bf16, n, k, nb), want in {(1, 2048, 8192, 3): 8, (1, 2048, 2048, 8): 8, (1, 2048, 2048, 9): 16, (1, 2049, 8192, 4): 16, (1, 2048, 2047, 4): 16, (1, 72, 4096, 4): 8,
+                                   (0, 2048, 8192, 4): 16, (0, 16384, 2048, 4): 32, (1, 16384, 2048, 4): 32, (1, 16383, 2048, 16): 16}.items():
+        rows = ctypes.c_int32()
+        assert lib.crabml_hip_debug_step_linear_rows(bf16, n, k, nb, 256, ctypes.byref(rows)) == 0
+        assert rows.value == want, (bf16, n, k, nb)
+
+
 def graph_steps(nodes, seq_len, left=0, made=0, have=0):
     top, place = ctypes.c_int32(), ctypes.c_int32()
     assert lib.crabml_hip_debug_graph_steps(ctypes.c_size_t(nodes), ctypes.c_size_t(seq_len), ctypes.c_size_t(left), ctypes.c_size_t(made), have, ctypes.byref(top),
