@@ -133,7 +133,9 @@ struct crabml_hip_llama {
   unsigned long long* slots = nullptr;  // dim/32 {chunk sum, epoch} granules of the norm epilogue
   SmallLayer* small = nullptr;  // all layers in one launch (fused_small.hpp): their table ...
   unsigned long long* small_gran = nullptr;  // ... granules
-  int small_wgs = 0;                         // ... and workgroups, as reserved (small_reserve)
+  int small_wgs = 0;                         // ... and workgroups, as reserved (small_reserve; 0: launches per layer)
+  int small_polls = SMALL_POLLS;
+  bool small_unseen = false;  // steps in one launch each whose fault word nobody has looked at
   unsigned long long* a8gran = nullptr;  // Q4_K layers: granules of the attention output (dim_l) and of h (hidden_l), through which
   unsigned long long* h8gran = nullptr;  // the producing kernels assemble Q8_K super-blocks (q8k_exchange_store)
   bool q8k_producers = false;            // attention / gate-up emit the Q8_K planes of wo's / ffn_down's rhs themselves
@@ -1208,8 +1210,10 @@ int allreduce(crabml_hip_llama* c, int seg) {
 }
 
 // Workgroups of the one launch wait for each other and take a CU each (118 VGPRs, 16 waves): what the contexts of a process hold together stays within half
-// of a device's CUs, however many streams run, and the rest is left to launches whose workgroups wait as well.  A context past that
-// (five of 24 workgroups, four of 32, are within) keeps its launches per layer: the same bits.
+// of a device's CUs, so that these launches never wait for each other's CUs, however many streams run.  A context past that (of 256 CUs four contexts of 27
+// workgroups, the 15M model's, are within), and for as long as it lives, keeps its launches per layer: the same bits.  Launches of other contexts whose
+// workgroups wait as well, and other processes, are not counted: where they and this one hold CUs that the other needs, the call takes 0.4 s longer, once
+// (small_recover).
 std::atomic<int>& small_reserved(int ordinal) {
   static std::atomic<int> held[64];
   return held[ordinal & 63];
@@ -1251,6 +1255,7 @@ int enqueue_small_layers(crabml_hip_llama* c) {
   a.seq_cap = (int)g.seq_len;
   a.rope_dim = (int)g.rope_dim;
   a.npairs = c->npairs;
+  a.polls = c->small_polls;
   a.q_scale = 1.0f / std::sqrt((float)c->hd);
   a.eps = g.rms_norm_eps;
   small_kernel(c->wtype)<<<c->small_wgs, 1024, 0, dev->stream>>>(a);
@@ -1260,7 +1265,7 @@ int enqueue_small_layers(crabml_hip_llama* c) {
 
 int enqueue_step(crabml_hip_llama* c) {
   const int n = n_segments(c);
-  if (c->small && runs_attn_short(c) && !(c->dev->prof_on && !c->use_graph && !c->capturing)) {
+  if (c->small_wgs && runs_attn_short(c) && !(c->dev->prof_on && !c->use_graph && !c->capturing)) {
     if (!c->led) CH_TRY(enqueue_front(c, false));
     CH_TRY(enqueue_small_layers(c));
     return enqueue_segment(c, n - 1);
@@ -1309,6 +1314,57 @@ bool capture_steps(crabml_hip_llama* c, int variant, int steps, hipGraph_t* grap
   }
   if (graph) (void)hipGraphDestroy(graph);
   return false;
+}
+
+// a decode step of every attention form that some position of this context runs (variant_of changes at these numbers of cached positions only), as a graph
+bool capture_forms(crabml_hip_llama* c) {
+  bool has[4] = {};
+  for (size_t n : {(size_t)1, c->attn_short_from, c->attn_short_until, c->attn_long_from, c->flash_ticket_until})
+    if (n >= 1 && n <= c->cfg.seq_len) has[variant_of(c, n - 1)] = true;
+  bool ok = true;
+  for (int v = 0; v < 4 && ok; v++) {
+    if (!has[v]) continue;
+    ok = capture_steps(c, v, 1, &c->graph[v], &c->exec[v]);
+    auto& s = c->several[v];
+    if (ok && c->chains && hipGraphGetNodes(c->graph[v], nullptr, &s.nodes) == hipSuccess) s.steps = steps_a_graph(s.nodes, c->cfg.seq_len);
+    // Strict device: no pairs.  32 layers of the 8B shape in Q4_0, us a token, single steps / pairs 1454 / 1479 (in Q4_K 1983 / 1978; three steps of 24
+    // layers 1127 / 1122, eight of 8 layers 416 / 410; fast device, pairs of 32 layers 1227 / 1223).  Why is not known.
+    if (c->dev->strict_order && s.steps < 3) s.steps = 1;
+  }
+  (void)hipGetLastError();
+  return ok;
+}
+void drop_graphs(crabml_hip_llama* c) {
+  for (int v = 0; v < 4; v++) {
+    if (c->exec[v]) (void)hipGraphExecDestroy(c->exec[v]);
+    if (c->graph[v]) (void)hipGraphDestroy(c->graph[v]);
+    c->exec[v] = nullptr;
+    c->graph[v] = nullptr;
+    auto& s = c->several[v];
+    for (int z = 0; z < GRAPH_SIZES; z++) {
+      if (s.exec[z]) (void)hipGraphExecDestroy(s.exec[z]);
+      if (s.graph[z]) (void)hipGraphDestroy(s.graph[z]);
+    }
+    s = {};
+  }
+}
+void small_release(crabml_hip_llama* c) {
+  if (c->small_wgs) small_reserved(c->dev->ordinal) -= c->small_wgs;
+  c->small_wgs = 0;
+}
+// A one-launch step's workgroups did not meet (the stream is idle, the fault word was SMALL_FAULT): the context goes on in launches per layer.  *again: the call's
+// steps can be made once more from where they began; not where steps in front of them, whose rows of the cache they read, may be what was lost.
+int small_recover(crabml_hip_llama* c, bool* again) {
+  crabml_hip_device* dev = c->dev;
+  *again = !c->small_unseen;
+  c->small_unseen = false;
+  small_release(c);
+  CH_HIP(dev, hipMemsetAsync(c->state + 5, 0, sizeof(int), dev->stream));
+  if (c->use_graph) {
+    drop_graphs(c);
+    c->use_graph = capture_forms(c);
+  }
+  return 0;
 }
 
 // `n` decode steps from cache position `pos` on: as many at a time as one graph holds, as long as they take the same attention form
@@ -1836,6 +1892,32 @@ int set_state(crabml_hip_llama* c, size_t token, size_t pos, int step, const uns
     return 0;
   }
   CH_HIP(c->dev, hipMemcpyAsync(c->state, st, 3 * sizeof(int), hipMemcpyHostToDevice, c->dev->stream));
+  return 0;
+}
+
+// behind a call's steps: waits for them, and what the context's fault word says then
+int read_fault(crabml_hip_llama* c, int* fault) {
+  CH_HIP(c->dev, hipMemcpyAsync(fault, c->state + 5, sizeof(int), hipMemcpyDeviceToHost, c->dev->stream));
+  CH_HIP(c->dev, hipStreamSynchronize(c->dev->stream));
+  return 0;
+}
+template <class Finish, class Again>
+int finish_call(crabml_hip_llama* c, const Finish& finish, const Again& again) {
+  crabml_hip_device* dev = c->dev;
+  int fault = 0;
+  CH_TRY(finish(&fault));
+  if (fault == SMALL_FAULT) {
+    bool repeat = false;
+    CH_TRY(small_recover(c, &repeat));
+    if (!repeat)
+      CH_BAIL(dev, CRABML_HIP_UNEXPECTED, "llama: an earlier step of this context was lost (the workgroups of its one launch did not meet: timed out); its cached rows are not to be used");
+    CH_TRY(again());
+    fault = 0;
+    CH_TRY(finish(&fault));
+  }
+  if (fault == 2) CH_BAIL(dev, CRABML_HIP_UNEXPECTED, "llama: a tensor-parallel peer's partial sums never arrived (poll timed out)");
+  if (fault) CH_BAIL(dev, CRABML_HIP_UNEXPECTED, "llama: a norm-epilogue gather timed out (workgroups not co-resident?)");
+  c->small_unseen = false;
   return 0;
 }
 
@@ -2440,6 +2522,9 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
     c->small_wgs = small_workers((int)g.embedding_dim, (int)kv_dim_l, (int)hidden_l, (int)n_heads_l);
     A(g.n_layers * sizeof(SmallLayer), (void**)&c->small);
     A(small_n * 8, (void**)&c->small_gran);
+    // test hook: so few polls that the workgroups do not meet
+    const char *h = getenv("CRABML_HIP_TEST_HOOKS"), *e = getenv("CRABML_HIP_SMALL_POLLS");
+    if (h && h[0] == '1' && e && atoi(e) > 0) c->small_polls = atoi(e);
   }
   c->out_cap = (int)g.seq_len;
   A((size_t)c->out_cap * 4, (void**)&c->out_tokens);
@@ -2496,22 +2581,9 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
   const bool want_graph = !(g.flags & CRABML_HIP_LLAMA_NO_GRAPH) &&
                           (tp == 1 || c->tp_dry || p2p_comm || (c->comm != nullptr && (g.flags & CRABML_HIP_LLAMA_TP_GRAPH)));
   if (want_graph) {
-    bool has[4] = {};  // the forms that some position of this context runs (variant_of changes at these numbers of cached positions only)
-    for (size_t n : {(size_t)1, c->attn_short_from, c->attn_short_until, c->attn_long_from, c->flash_ticket_until})
-      if (n >= 1 && n <= g.seq_len) has[variant_of(c, n - 1)] = true;
-    bool ok = true;
-    for (int v = 0; v < 4 && ok; v++) {
-      if (!has[v]) continue;
-      ok = capture_steps(c, v, 1, &c->graph[v], &c->exec[v]);
-      auto& s = c->several[v];
-      if (ok && c->chains && hipGraphGetNodes(c->graph[v], nullptr, &s.nodes) == hipSuccess) s.steps = steps_a_graph(s.nodes, g.seq_len);
-      // Strict device: no pairs.  32 layers of the 8B shape in Q4_0, us a token, single steps / pairs 1454 / 1479 (in Q4_K 1983 / 1978; three steps of 24
-      // layers 1127 / 1122, eight of 8 layers 416 / 410; fast device, pairs of 32 layers 1227 / 1223).  Why is not known.
-      if (dev->strict_order && s.steps < 3) s.steps = 1;
-    }
+    const bool ok = capture_forms(c);
     const char *h = getenv("CRABML_HIP_TEST_HOOKS"), *e = getenv("CRABML_HIP_GRAPH_STEPS");
     c->graph_steps_now = h && h[0] == '1' && e && e[0] == '1';
-    (void)hipGetLastError();
     c->use_graph = ok;
     if (!ok && tp == 1) {  // fail loudly: the caller asked for the graph path
       crabml_hip_llama_destroy(c);
@@ -2541,15 +2613,8 @@ int crabml_hip_llama_destroy(crabml_hip_llama_t* c) {
     (void)hipSetDevice(c->dev->ordinal);
     (void)hipStreamSynchronize(c->dev->stream);
   }
-  for (int v = 0; v < 4; v++) {
-    if (c->exec[v]) (void)hipGraphExecDestroy(c->exec[v]);
-    if (c->graph[v]) (void)hipGraphDestroy(c->graph[v]);
-    for (int z = 0; z < GRAPH_SIZES; z++) {
-      if (c->several[v].exec[z]) (void)hipGraphExecDestroy(c->several[v].exec[z]);
-      if (c->several[v].graph[z]) (void)hipGraphDestroy(c->several[v].graph[z]);
-    }
-  }
-  if (c->small_wgs) small_reserved(c->dev->ordinal) -= c->small_wgs;
+  drop_graphs(c);
+  small_release(c);
   for (auto& a : c->allocs) pool_free(c->dev, a.first, a.second);
   for (auto* b : c->held) crabml_hip_buf_release(b);
   if (c->h_state) (void)hipHostFree(c->h_state);
@@ -2578,15 +2643,19 @@ int crabml_hip_llama_forward(crabml_hip_llama_t* c, size_t token, size_t pos, fl
   CH_TRY(set_state(c, token, pos, 0));
   CH_TRY(run_step(c, pos));
   c->kv_len++;
-  if (logits) {
-    int fault = 0;
-    CH_HIP(dev, hipMemcpyAsync(logits, c->logits, c->cfg.vocab_size * 4, hipMemcpyDeviceToHost, dev->stream));
-    CH_HIP(dev, hipMemcpyAsync(&fault, c->state + 5, sizeof(int), hipMemcpyDeviceToHost, dev->stream));
-    CH_HIP(dev, hipStreamSynchronize(dev->stream));
-    if (fault == 2) CH_BAIL(dev, CRABML_HIP_UNEXPECTED, "llama: a tensor-parallel peer's partial sums never arrived (poll timed out)");
-    if (fault) CH_BAIL(dev, CRABML_HIP_UNEXPECTED, "llama: a norm-epilogue gather timed out (workgroups not co-resident?)");
+  if (!logits) {
+    c->small_unseen |= c->small_wgs != 0;
+    return 0;
   }
-  return 0;
+  auto finish = [&](int* fault) {
+    CH_HIP(dev, hipMemcpyAsync(logits, c->logits, c->cfg.vocab_size * 4, hipMemcpyDeviceToHost, dev->stream));
+    return read_fault(c, fault);
+  };
+  auto again = [&] {
+    CH_TRY(set_state(c, token, pos, 0));
+    return run_step(c, pos);
+  };
+  return finish_call(c, finish, again);
 }
 
 int crabml_hip_llama_decode_greedy(crabml_hip_llama_t* c, size_t token, size_t n_steps, uint32_t* out_tokens) {
@@ -2602,15 +2671,18 @@ int crabml_hip_llama_decode_greedy(crabml_hip_llama_t* c, size_t token, size_t n
     CH_BAIL(dev, CRABML_HIP_TENSOR_ERROR, "llama: %zu steps do not fit the kv cache (%zu of %zu used)", n_steps, c->kv_len, c->cfg.seq_len);
   if (n_steps == 0) return 0;
   CH_TRY(set_state(c, token, c->kv_len, 0));
-  CH_TRY(run_steps(c, c->kv_len, n_steps));
+  const size_t pos = c->kv_len;
+  CH_TRY(run_steps(c, pos, n_steps));
   c->kv_len += n_steps;
-  int fault = 0;
-  CH_HIP(dev, hipMemcpyAsync(out_tokens, c->out_tokens, n_steps * 4, hipMemcpyDeviceToHost, dev->stream));
-  CH_HIP(dev, hipMemcpyAsync(&fault, c->state + 5, sizeof(int), hipMemcpyDeviceToHost, dev->stream));
-  CH_HIP(dev, hipStreamSynchronize(dev->stream));
-  if (fault == 2) CH_BAIL(dev, CRABML_HIP_UNEXPECTED, "llama: a tensor-parallel peer's partial sums never arrived (poll timed out)");
-  if (fault) CH_BAIL(dev, CRABML_HIP_UNEXPECTED, "llama: a norm-epilogue gather timed out (workgroups not co-resident?)");
-  return 0;
+  auto finish = [&](int* fault) {
+    CH_HIP(dev, hipMemcpyAsync(out_tokens, c->out_tokens, n_steps * 4, hipMemcpyDeviceToHost, dev->stream));
+    return read_fault(c, fault);
+  };
+  auto again = [&] {
+    CH_TRY(set_state(c, token, pos, 0));
+    return run_steps(c, pos, n_steps);
+  };
+  return finish_call(c, finish, again);
 }
 
 
@@ -2703,6 +2775,7 @@ size_t crabml_hip_llama_kv_len(const crabml_hip_llama_t* c) { return c ? c->kv_l
 int crabml_hip_llama_reset(crabml_hip_llama_t* c) {
   if (!c) return CRABML_HIP_BAD_INPUT;
   c->kv_len = 0;
+  c->small_unseen = false;
   if (c->flash_tick) {  // a step that faulted half-way may have left arrivals behind
     CH_USE(c->dev);
     CH_FLUSH(c->dev);
@@ -2740,6 +2813,12 @@ int crabml_hip_llama_debug_graph_steps(crabml_hip_llama_t* c, size_t pos, int32_
   const auto& s = c->several[variant_of(c, pos)];
   *steps = s.steps;
   *captured = (int32_t)s.have;
+  return 0;
+}
+
+int crabml_hip_llama_debug_small_layers(crabml_hip_llama_t* c, int32_t* workgroups) {
+  if (!c || !workgroups) return CRABML_HIP_BAD_INPUT;
+  *workgroups = c->small_wgs;
   return 0;
 }
 

@@ -16,13 +16,17 @@
 // a row (small_fits).  The arithmetic is that of the five launches, term by term and in their order: k_qkv, k_attn_short, k_gemv_res_nq<DEFER>,
 // k_gateup_q<DEFER>; the last ffn_down normalizes exactly, as there.  All bits are theirs.
 // A granule buffer is written once a layer.  Whoever writes it again has, through the chain of gathers, waited for everything that its readers made of
-// it, so one copy of each is enough.  Polls are bounded and raise the context's fault flag, and a raised flag ends the others' waits.
+// it, so one copy of each is enough.  Polls are bounded -- at a quarter of what the other launches of the step wait for each other, so that where the two
+// kinds hold CUs that the other needs it is this one that leaves -- and raise the context's fault word, and a raised word ends the others'
+// waits.  The host then runs the call again in launches per layer and stays with them (small_give_up).
 #pragma once
 
 namespace crabml_hip {
 
 #define SMALL_WGS 32
 #define SMALL_LAYERS 64
+#define SMALL_POLLS (1 << 19)  // some 0.4 s
+#define SMALL_FAULT 3
 
 struct SmallLayer {
   Planes wq, wk, wv, wo, gate, up, down;
@@ -40,7 +44,7 @@ struct SmallStep {
   int* isum;
   const float* rope;
   const unsigned short* exp_tab;
-  int L, dim, kv_dim, hd, hidden, n_heads, n_kv, seq_cap, rope_dim, npairs;
+  int L, dim, kv_dim, hd, hidden, n_heads, n_kv, seq_cap, rope_dim, npairs, polls;
   float q_scale, eps;
 };
 // granules of a block: eight of four quants, scale | sum, and -- x1, x2 -- the block's sum of squares
@@ -105,9 +109,9 @@ __global__ __launch_bounds__(1024) void k_small_layers(const SmallStep a) {
   auto poll = [&](const unsigned long long* p, unsigned epoch) -> unsigned {
     unsigned long long g = ld_granule(p);
     for (int tries = 1; (unsigned)(g >> 32) != epoch && !dead; tries++) {
-      if ((tries & 255) == 0 && (tries >= 1 << 21 || __hip_atomic_load(a.fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+      if (tries >= a.polls || ((tries & 255) == 0 && __hip_atomic_load(a.fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
         dead = true;
-        *a.fault = 1;  // a workgroup never arrived: flagged, not hung
+        *a.fault = SMALL_FAULT;  // a workgroup never arrived: flagged, not hung
       }
       g = ld_granule(p);
     }

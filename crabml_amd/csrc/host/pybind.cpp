@@ -480,6 +480,12 @@ PYBIND11_MODULE(_host, m) {
              r.device()->check(crabml_hip_llama_debug_graph_steps(r.raw(), pos, &steps, &captured));
              return py::make_tuple(steps, captured);
            })
+      .def("debug_small_layers",  // workgroups of the one launch for all layers (0: launches per layer)
+           [](HipLlamaRunner& r) {
+             int32_t n = 0;
+             r.device()->check(crabml_hip_llama_debug_small_layers(r.raw(), &n));
+             return n;
+           })
       .def("debug_kv", [](HipLlamaRunner& r, size_t layer, bool v, bool f16) {
         std::vector<uint8_t> b = r.debug_kv(layer, v, f16);
         return py::array_t<uint8_t>(b.size(), b.data());

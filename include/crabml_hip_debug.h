@@ -154,6 +154,8 @@ int crabml_hip_debug_flash_attention_rows(crabml_hip_device_t* dev, const float*
 int crabml_hip_llama_debug_graphs(crabml_hip_llama_t* ctx, size_t pos, int32_t* form, uint32_t* captured);
 /* greedy steps the largest graph of several holds at cache position pos (1: none is made), and the sizes that have been captured, bits by place */
 int crabml_hip_llama_debug_graph_steps(crabml_hip_llama_t* ctx, size_t pos, int32_t* steps, int32_t* captured);
+/* workgroups of the launch that makes all of a small model's layers, as this context reserved them; 0: its step is launches per layer */
+int crabml_hip_llama_debug_small_layers(crabml_hip_llama_t* ctx, int32_t* workgroups);
 /* parity hook: copies the layer's K or V cache (raw f16/f32 bytes, [n_kv_heads][seq_len][head_dim]) */
 int crabml_hip_llama_debug_kv(crabml_hip_llama_t* ctx, size_t layer, int32_t which_v, void* dst, size_t nbytes);
 

@@ -52,6 +52,41 @@ def test_contexts_past_the_reserved_workgroups(ca):
     assert all(x == ids[0] for x in ids)
 
 
+@pytest.mark.parametrize("graph", [True, False])
+def test_workgroups_that_do_not_meet(ca, monkeypatch, graph):
+    """one poll instead of half a million: no gather is met.  The call that finds out is made again in launches per layer, and the context stays with them; steps
+    that nobody has looked at cannot be made again: an error, once"""
+    shape = synth.ModelShape("small", 288, 768, 3, 6, 6, 300, 160, 1e-5, None)
+    model = synth.build_model(shape, synth.Q8_0, seed=33)
+    dev = ca.HipTensorDevice(0)
+    conf, w = synth.to_hip(model, dev)
+    five = ca.HipLlamaRunner(conf, w, dev, 100, True, graph, extra_flags=FIVE)
+    ids = five.decode_greedy(3, 40)
+    logits = five.forward(ids[-1], 40).view(np.uint32)
+    monkeypatch.setenv("CRABML_HIP_TEST_HOOKS", "1")
+    monkeypatch.setenv("CRABML_HIP_SMALL_POLLS", "1")
+    by_steps, by_run, unseen = (ca.HipLlamaRunner(conf, w, dev, 100, True, graph) for _ in range(3))
+    assert by_steps.debug_small_layers() == by_run.debug_small_layers() == unseen.debug_small_layers() == 27
+    token = 3
+    for pos in range(40):
+        x = by_steps.forward(token, pos)
+        token = int(ca.sample_argmax(x))
+        assert token == ids[pos]
+    assert np.array_equal(by_steps.forward(ids[-1], 40).view(np.uint32), logits)
+    assert by_run.decode_greedy(3, 40) == ids and np.array_equal(by_run.forward(ids[-1], 40).view(np.uint32), logits)
+    unseen.forward_async(3, 0)
+    with pytest.raises(ca.CrabmlError, match="not to be used"):
+        unseen.forward(ids[0], 1)
+    unseen.reset()
+    assert unseen.decode_greedy(3, 40) == ids
+    assert by_steps.debug_small_layers() == by_run.debug_small_layers() == unseen.debug_small_layers() == 0
+    # what they had reserved is there again
+    monkeypatch.delenv("CRABML_HIP_SMALL_POLLS")
+    more = [ca.HipLlamaRunner(conf, w, dev, 100, True, graph) for _ in range(4)]
+    assert [r.debug_small_layers() for r in more] == [27] * 4
+    assert all(r.decode_greedy(3, 40) == ids for r in more)
+
+
 def test_the_computed_exp_is_the_table(ca):
     """the step's exp against the device's table, every f16"""
     lib = ctypes.CDLL(ca.LIB_PATH)
