@@ -20,8 +20,10 @@ def test_one_launch_equals_five_a_layer(ca, fmt, dim, hidden, layers, heads, kv_
     dev = ca.HipTensorDevice(0)
     shape = synth.ModelShape("small", dim, hidden, layers, heads, kv_heads, 300, 160, 1e-5, None)
     conf, w = synth.to_hip(synth.build_model(shape, synth.TYPE_BY_NAME[fmt], seed=31), dev)
-    seq = 150  # (past the first 64 and the next 128 positions, and to the last)
+    seq = 150  # (past the first 64 positions, and to the last)
     one, eager, five = (ca.HipLlamaRunner(conf, w, dev, seq, True, g, extra_flags=f) for g, f in ((True, 0), (False, 0), (True, FIVE)))
+    wgs = max((dim + 2 * (dim // heads * kv_heads) + 31) // 32, hidden // 32, heads)
+    assert (one.debug_small_layers(), eager.debug_small_layers(), five.debug_small_layers()) == (wgs, wgs, 0)
     pos, token = 0, 3
     for n in (1, 5, 58, 2, 70):
         ids = one.decode_greedy(token, n)
@@ -40,6 +42,46 @@ def test_one_launch_equals_five_a_layer(ca, fmt, dim, hidden, layers, heads, kv_
     assert one.decode_greedy(9, 30) == five.decode_greedy(9, 30)
 
 
+# several passes of 128 over a head's cached rows, to the end of the cache (heads of 48) and across the position from which the step's attention is k_attn_flash
+# (heads of 64: 57344 / 64 = 896 cached)
+@pytest.mark.parametrize("dim,heads,seq,until", [(288, 6, 640, 640), (512, 8, 912, 895)])
+@pytest.mark.parametrize("fmt", ["Q8_0", "Q4_0"])
+def test_one_launch_equals_five_a_layer_at_every_position(ca, fmt, dim, heads, seq, until):
+    dev = ca.HipTensorDevice(0)
+    shape = synth.ModelShape("small", dim, 768, 2, heads, heads // 2, 300, seq, 1e-5, None)
+    conf, w = synth.to_hip(synth.build_model(shape, synth.TYPE_BY_NAME[fmt], seed=34), dev)
+    one, five = (ca.HipLlamaRunner(conf, w, dev, seq, True, extra_flags=f) for f in (0, FIVE))
+    assert one.debug_small_layers() > 0 and five.debug_small_layers() == 0
+    assert [one.debug_graphs(p)[0] == 0 for p in (0, until - 1, min(until, seq - 1))] == [True, True, until == seq]
+    pos, token = 0, 3
+    for n in (190, 3, 127, 3, 125, 3, until - 467):
+        assert one.decode_greedy(token, n) == (ids := five.decode_greedy(token, n)), (pos, n)
+        pos, token = pos + n, ids[-1]
+        x, y = one.forward(token, pos), five.forward(token, pos)
+        assert np.array_equal(x.view(np.uint32), y.view(np.uint32)), pos
+        pos += 1
+    while pos < seq:
+        x, y = one.forward(token, pos), five.forward(token, pos)
+        assert np.isfinite(x).all() and np.array_equal(x.view(np.uint32), y.view(np.uint32)), pos
+        pos, token = pos + 1, (token * 7 + pos) % 300
+    for layer in range(2):
+        for v in (False, True):
+            assert np.array_equal(one.debug_kv(layer, v, True), five.debug_kv(layer, v, True))
+
+
+@pytest.mark.parametrize("fmt,out", [("Q8_0", "Q6_K"), ("Q4_0", "Q6_K"), ("Q4_0", "F16"), ("Q8_0", "Q4_1")])
+def test_a_classifier_of_another_type_reads_the_row_behind_the_one_launch(ca, fmt, out):
+    dev = ca.HipTensorDevice(0)
+    shape = synth.ModelShape("small", 256, 512, 3, 4, 2, 300, 60, 1e-5, None)
+    conf, w = synth.to_hip(synth.build_model(shape, synth.TYPE_BY_NAME[fmt], seed=35, output_type=synth.TYPE_BY_NAME[out]), dev)
+    one, five = (ca.HipLlamaRunner(conf, w, dev, 60, True, extra_flags=f) for f in (0, FIVE))
+    assert one.debug_small_layers() > 0 and five.debug_small_layers() == 0
+    assert one.decode_greedy(3, 40) == five.decode_greedy(3, 40)
+    for pos in range(40, 60):
+        x, y = one.forward(pos, pos), five.forward(pos, pos)
+        assert np.isfinite(x).all() and np.array_equal(x.view(np.uint32), y.view(np.uint32)), pos
+
+
 def test_contexts_past_the_reserved_workgroups(ca):
     """more contexts than half of the CUs hold, each on a stream of its own and all of them under way at once"""
     shape = synth.ModelShape("small", 288, 768, 2, 6, 6, 300, 160, 1e-5, None)
@@ -47,9 +89,13 @@ def test_contexts_past_the_reserved_workgroups(ca):
     for i in range(8):
         dev = ca.HipTensorDevice(0)
         runners.append(ca.HipLlamaRunner(*synth.to_hip(model, dev), dev, 100, True))
+    assert [r.debug_small_layers() for r in runners] == [27] * 4 + [0] * 4
+    dev = ca.HipTensorDevice(0)
+    want = ca.HipLlamaRunner(*synth.to_hip(model, dev), dev, 100, True, extra_flags=FIVE).decode_greedy(3, 90)
     with ThreadPoolExecutor(8) as pool:
         ids = list(pool.map(lambda r: r.decode_greedy(3, 90), runners))
-    assert all(x == ids[0] for x in ids)
+    assert all(x == want for x in ids)
+    assert [r.debug_small_layers() for r in runners] == [27] * 4 + [0] * 4  # (all of them met)
 
 
 @pytest.mark.parametrize("graph", [True, False])
