@@ -429,32 +429,34 @@ bool gemm_f16w_covers(uint32_t w_dtype, uint32_t act_qtype) {
 // wave tile: T column tiles of 16 prompt rows -- 8 (128-row workgroup tiles) from 65 rows up; short passes (a short prompt, the ragged
 // tail of a long one) take 4 / 2: the MFMAs of an empty column tile cost what a full one's do
 static int f16w_col_tiles_per_wave(size_t b, int variant) { return (variant & 512) ? 4 : (variant & 16) ? 8 : b <= 32 ? 2 : b <= 64 ? 4 : 8; }
+// (K-quants past 64 rows are gemm_f16w_wide.hip's, but for Q6_K launches of fewer than 2M weights and for what its launcher refuses)
 template <int WF>
-static bool launch_f16w_fmt(crabml_hip_device* dev, const F16wMats& mats, int row_tiles, size_t k, const void* xh, size_t b, int ksplit, int F,
-                            int variant, bool gu, int T, int NW) {
+static bool launch_f16w_fmt(crabml_hip_device* dev, const F16wMats& mats, int row_tiles, size_t k, const void* xh, size_t b, int ksplit, int F, bool gu, int T,
+                            int NW) {
   if (gu) {
-    switch (T) {
-      case 2: return launch_f16w_t<WF, 2, 2, true>(dev, mats, row_tiles, k, xh, b, 1);
-      case 4: return launch_f16w_t<WF, 2, 4, true>(dev, mats, row_tiles, k, xh, b, 1);
-      default:
-        return NW == 8 ? launch_f16w_t<WF, 2, 8, true, 8>(dev, mats, row_tiles, k, xh, b, 1) : launch_f16w_t<WF, 2, 8, true>(dev, mats, row_tiles, k, xh, b, 1);
+    if constexpr (WF != WF_Q4_K) {
+      if (T == 8) {
+        if constexpr (WF != WF_Q6_K)
+          if (NW == 8) return launch_f16w_t<WF, 2, 8, true, 8>(dev, mats, row_tiles, k, xh, b, 1);
+        return launch_f16w_t<WF, 2, 8, true>(dev, mats, row_tiles, k, xh, b, 1);
+      }
     }
+    return T == 2 ? launch_f16w_t<WF, 2, 2, true>(dev, mats, row_tiles, k, xh, b, 1) : launch_f16w_t<WF, 2, 4, true>(dev, mats, row_tiles, k, xh, b, 1);
   }
-  switch (T) {
-    case 2: return F == 2 ? launch_f16w_t<WF, 2, 2>(dev, mats, row_tiles, k, xh, b, ksplit) : launch_f16w_t<WF, 1, 2>(dev, mats, row_tiles, k, xh, b, ksplit);
-    case 4: return F == 2 ? launch_f16w_t<WF, 2, 4>(dev, mats, row_tiles, k, xh, b, ksplit) : launch_f16w_t<WF, 1, 4>(dev, mats, row_tiles, k, xh, b, ksplit);
-    default: return F == 2 ? launch_f16w_t<WF, 2, 8>(dev, mats, row_tiles, k, xh, b, ksplit) : launch_f16w_t<WF, 1, 8>(dev, mats, row_tiles, k, xh, b, ksplit);
-  }
+  if constexpr (WF != WF_Q4_K)
+    if (T == 8) return F == 2 ? launch_f16w_t<WF, 2, 8>(dev, mats, row_tiles, k, xh, b, ksplit) : launch_f16w_t<WF, 1, 8>(dev, mats, row_tiles, k, xh, b, ksplit);
+  if (T == 2) return F == 2 ? launch_f16w_t<WF, 2, 2>(dev, mats, row_tiles, k, xh, b, ksplit) : launch_f16w_t<WF, 1, 2>(dev, mats, row_tiles, k, xh, b, ksplit);
+  return F == 2 ? launch_f16w_t<WF, 2, 4>(dev, mats, row_tiles, k, xh, b, ksplit) : launch_f16w_t<WF, 1, 4>(dev, mats, row_tiles, k, xh, b, ksplit);
 }
 // gate | up in full tiles: eight waves share a B' tile, which halves what the launch reads of B' (every row tile reads all of it, a gigabyte for 512
 // rows of 4096) and the staging a wave does -- one workgroup a CU, where those of four waves lie two on a CU.  It pays where the last round of CUs is
-// nearly full; into a part-empty one the smaller workgroups, which then have a CU each, fit better.  A whole pass of 3 layers, eight waves / four, by
-// rounds of CUs (128-row tiles / CUs): 0.5 1.00 to 1.04, 0.67 1.00 to 1.02, 0.75 0.96 to 1.00, 0.875 0.96 to 0.99, 1.0 0.98 to 1.01, 1.25 to 1.5 1.03 to
-// 1.10, 1.75 0.96 to 0.98, 2.0 0.97 to 1.01, 2.2 1.03 to 1.04, 2.6 0.97 to 0.99, 3.5 0.99 (Q8_0), 1.00, 1.015 (Q4_K, whose unpacking hides
-// less of the longer barrier).  (14336 rows of 4096, one launch of 300 rows: Q4_K 137 us with eight waves, 123 with four.)
-static bool f16w_eight_waves(uint32_t dt, size_t tiles, size_t n_cu) {
+// nearly full; into a part-empty one the smaller workgroups, which then have a CU each, fit better.  A whole pass of 3 layers of width 4096, eight waves / four,
+// by rounds of CUs (128-row tiles / CUs): 0.5 1.00 to 1.04, 0.67 1.00 to 1.02, 0.75 0.96 to 1.00, 0.875 0.96 to 0.99, 1.0 0.98 to 1.01, 1.25 to 1.5 1.03 to
+// 1.10, 1.75 0.96 to 0.98, 2.0 0.97 to 1.01, 2.2 1.03 to 1.04, 2.6 0.97 to 0.99, 3.5 0.99 to 1.00.  Widths that are no multiple of 256, which alone come here,
+// Q4_0 / Q8_0, where the rule says eight: gate | up of 8640 x 3200 0.80 0.95 / 0.97, 1.86 0.99 / 0.97; 10240 x 3200 0.94 0.98 / 0.97, 1.88 1.01 / 0.99; 7680 x 2880
+// 0.94 0.99 / 1.00, 1.88 1.045 / 1.02 (the one that loses); 6400 x 1600 0.98 1.01 / 0.99; 16384 x 1600 1.0 0.98 / 0.95, 2.0 0.99 / 0.97.
+static bool f16w_eight_waves(size_t tiles, size_t n_cu) {
   const size_t rounds = (tiles + n_cu - 1) / n_cu;
-  if (dt == CRABML_HIP_Q4_K && rounds > 3) return false;
   return rounds == 1 ? 4 * tiles >= 3 * n_cu : 20 * tiles >= 17 * rounds * n_cu;
 }
 // nw weight matrices (one format, the same k) against the same rhs rows: out[j] (b, m[j]) = W[j] . x
@@ -473,7 +475,8 @@ bool launch_gemm_f16w(crabml_hip_device* dev, const crabml_hip_buf* const* w, co
   if ((dt == CRABML_HIP_Q4_K || dt == CRABML_HIP_Q6_K) && k % 256 != 0) return false;
   for (int j = 0; j < nw; j++)
     if (w[j]->dtype != dt || m[j] % 4 != 0) return false;
-  static const int variant = [] {  // lab hook (CRABML_HIP_TEST_HOOKS=1 CRABML_HIP_F16W=n): 1 = two fragments, 3 = one; +8 = never split k; +16 = T = 8 always; +32 = k pieces of >= 8 chunks; +64 = no gate | up epilogue; +512 = T = 4 always; +1024 = narrow launches as <2, 4>
+  // lab hook, for the launches of this file's kernel (CRABML_HIP_TEST_HOOKS=1 CRABML_HIP_F16W=n)
+  static const int variant = [] {  // 1 = two fragments, 3 = one; +8 = never split k; +16 = T = 8 always; +32 = k pieces of >= 8 chunks; +64 = no gate | up epilogue; +512 = T = 4 always; +1024 = narrow launches as <2, 4>
     const char* h = getenv("CRABML_HIP_TEST_HOOKS");
     const char* e = getenv("CRABML_HIP_F16W");
     return h && h[0] == '1' && e ? atoi(e) : 0;
@@ -523,6 +526,7 @@ bool launch_gemm_f16w(crabml_hip_device* dev, const crabml_hip_buf* const* w, co
     ksplit = 1;
   }
   int T = f16w_col_tiles_per_wave(b, variant);
+  if (dt == CRABML_HIP_Q4_K && T == 8) T = 4;  // (refused by the wide launcher)
   size_t cw = 16 * (size_t)T, col128 = (b + cw - 1) / cw;  // (column tiles of the launch)
   // two fragments per wave (every B' fragment read from LDS feeds two MFMAs) when 128-row tiles still cover the chip
   int F = ((mtot + 127) / 128) * col128 >= (size_t)dev->n_cu ? 2 : 1;
@@ -541,7 +545,7 @@ bool launch_gemm_f16w(crabml_hip_device* dev, const crabml_hip_buf* const* w, co
   if (gu) F = 2;
   // (gate | up alone.  512 rows, Q4_0 183 -> 173 us, the whole request 3973 -> 3785.  The other launches, cut in k to fill the chip with the smaller
   // tiles, do not gain: ffn_down 115 -> 108, wo 35 -> 44; four fragments a wave, one wave a SIMD, lose: 183 -> 211.)
-  const int NW = gu && T == 8 && f16w_eight_waves(dt, (m[0] + 127) / 128 * col128, (size_t)dev->n_cu) ? 8 : 4;
+  const int NW = gu && T == 8 && dt != CRABML_HIP_Q6_K && f16w_eight_waves((m[0] + 127) / 128 * col128, (size_t)dev->n_cu) ? 8 : 4;
   const bool hquant = gu && hq != nullptr && hq->planes != nullptr && m[0] % 32 == 0;
   if (hquant) mats.hq = *hq;
   int row_tiles = 0;
@@ -561,15 +565,15 @@ bool launch_gemm_f16w(crabml_hip_device* dev, const crabml_hip_buf* const* w, co
       ksplit *= 2;
   bool ok;
   if (dt == CRABML_HIP_Q8_0)
-    ok = launch_f16w_fmt<WF_Q8_0>(dev, mats, row_tiles, k, xh, b, ksplit, F, variant, gu, T, NW);
+    ok = launch_f16w_fmt<WF_Q8_0>(dev, mats, row_tiles, k, xh, b, ksplit, F, gu, T, NW);
   else if (dt == CRABML_HIP_Q4_K)
-    ok = launch_f16w_fmt<WF_Q4_K>(dev, mats, row_tiles, k, xh, b, ksplit, F, variant, gu, T, NW);
+    ok = launch_f16w_fmt<WF_Q4_K>(dev, mats, row_tiles, k, xh, b, ksplit, F, gu, T, NW);
   else if (dt == CRABML_HIP_Q6_K)
-    ok = launch_f16w_fmt<WF_Q6_K>(dev, mats, row_tiles, k, xh, b, ksplit, F, variant, gu, T, NW);
+    ok = launch_f16w_fmt<WF_Q6_K>(dev, mats, row_tiles, k, xh, b, ksplit, F, gu, T, NW);
   else if (dt == CRABML_HIP_Q4_1)
-    ok = launch_f16w_fmt<WF_Q4_1>(dev, mats, row_tiles, k, xh, b, ksplit, F, variant, gu, T, NW);
+    ok = launch_f16w_fmt<WF_Q4_1>(dev, mats, row_tiles, k, xh, b, ksplit, F, gu, T, NW);
   else
-    ok = launch_f16w_fmt<WF_Q4_0>(dev, mats, row_tiles, k, xh, b, ksplit, F, variant, gu, T, NW);
+    ok = launch_f16w_fmt<WF_Q4_0>(dev, mats, row_tiles, k, xh, b, ksplit, F, gu, T, NW);
   return ok && finish(gu, hquant);
 }
 
@@ -585,8 +589,8 @@ void launch_add_parts(hipStream_t st, float* out, const float* ws, size_t n, int
 
 }  // namespace crabml_hip
 
-extern "C" int crabml_hip_debug_gateup_waves(uint32_t dtype, size_t hidden, size_t rows, int32_t n_cu, int32_t* waves) {
+extern "C" int crabml_hip_debug_gateup_waves(size_t hidden, size_t rows, int32_t n_cu, int32_t* waves) {
   if (!waves || n_cu < 1) return CRABML_HIP_BAD_INPUT;
-  *waves = crabml_hip::f16w_eight_waves(dtype, (hidden + 127) / 128 * ((rows + 127) / 128), (size_t)n_cu) ? 8 : 4;
+  *waves = crabml_hip::f16w_eight_waves((hidden + 127) / 128 * ((rows + 127) / 128), (size_t)n_cu) ? 8 : 4;
   return 0;
 }

@@ -60,8 +60,9 @@ int crabml_hip_debug_rhs_rows(size_t m, size_t* rows);
 /* top: steps of a greedy run that go into one graph where one step is `nodes` launches.  next: which of the sizes top, top / 2, top / 4 comes next in a run that
  * has made `made` steps and has `left` to make (its place; -1: a single step); have: the sizes that have been captured, bits by place.  Host only. */
 int crabml_hip_debug_graph_steps(size_t nodes, size_t seq_len, size_t left, size_t made, uint32_t have, int32_t* top, int32_t* next);
-/* Waves of a workgroup of the fast prompt pass's gate | up launch over `rows` > 64 rows of a width that is no multiple of 256.  Host only. */
-int crabml_hip_debug_gateup_waves(uint32_t dtype, size_t hidden, size_t rows, int32_t n_cu, int32_t* waves);
+/* Waves of a workgroup of the fast prompt pass's gate | up launch with SiLU * mul inside, over `rows` > 64 rows of a width that is no multiple of 256 (Q4_0, Q8_0,
+ * Q4_1).  Host only. */
+int crabml_hip_debug_gateup_waves(size_t hidden, size_t rows, int32_t n_cu, int32_t* waves);
 /* f16(exp(x)) of every f16 x as the one-launch decode step of a small model computes it, and the device's table of it: 65536 values each. */
 int crabml_hip_debug_exp_of_f16(crabml_hip_device_t* dev, uint16_t* computed, uint16_t* table);
 /* Tile of the fast prompt pass's weight GEMM over b > 64 rows, k a multiple of 256: fragments and column tiles of a wave, groups of waves along k in a

@@ -360,7 +360,8 @@ NO_GU_EPILOGUE = 67108864  # CRABML_HIP_LLAMA_PREFILL_NO_GU_EPILOGUE
                                          ("Q4_0", "wide-ffn", 200), ("Q4_K", "wide-ffn", 173), ("Q8_0", "wide-ffn", 130),
                                          ("Q4_0", "ffn-14336", 200), ("Q4_K", "ffn-14336", 129), ("Q6_K", "ffn-14336", 256), ("Q4_0", "ffn-14368", 130),
                                          ("Q8_0", "ffn-14432", 200), ("Q4_1", "ffn-15424", 255), ("Q4_K", "ffn-14336", 300), ("Q8_0", "ffn-14368", 300),
-                                         ("Q4_0", "dim-4096", 200), ("Q4_1", "dim-4096", 70), ("Q8_0", "dim-8192", 130)])
+                                         ("Q4_0", "narrow-14336", 200), ("Q8_0", "narrow-14432", 200), ("Q4_1", "narrow-15424", 255), ("Q4_0", "narrow-14368", 130),
+                                         ("Q8_0", "narrow-14368", 300), ("Q4_0", "dim-4096", 200), ("Q4_1", "dim-4096", 70), ("Q8_0", "dim-8192", 130)])
 def test_fast_prompt_pass_rows_write_their_own_f16_planes(ca, fmt, shape, n):
     """The kernels that quantize the rows of a fast prompt pass (norm + quantize, SiLU * mul + quantize, the stand-alone quantizer for
     the attention output and for Q8_K rows) also leave the pre-scaled f16 planes the next weight GEMM reads (f16w_rows.hpp), in that
@@ -374,9 +375,11 @@ def test_fast_prompt_pass_rows_write_their_own_f16_planes(ca, fmt, shape, n):
     # SiLU * mul epilogue (one pass of > 128 rows; the 48-row passes keep the separate launch)
     # dim-4096 / dim-8192: rows of 4096 / 8192 elements take the 256-thread norm + quantize kernel (k_norm_quant_rows_w: a thread owns
     # half a quant block / a whole one) -- against the 1024-thread kernel behind the flag, on the fast AND the strict device
-    # ffn-*: the gate | up launch's workgroups of eight waves (129 to 256 rows), with 32, 96 and 64 rows in the last 128-row tile; 300 rows: four waves
+    # ffn-*: feed-forwards that end 32, 96 and 64 rows into a tile of 128.  narrow-*: the same behind a width of 576, which is no multiple of 256: the gate | up
+    # launch's workgroups of eight waves (129 to 256 rows), and four (300 rows), of gemm_f16w.hip
     shp = (synth.ModelShape("wide-ffn", 512, 12288, 1, 4, 2, 512, 256, 1e-5, None) if shape == "wide-ffn"
            else synth.ModelShape(shape, 512, int(shape[4:]), 1, 4, 2, 512, 512, 1e-5, None) if shape.startswith("ffn-")
+           else synth.ModelShape(shape, 576, int(shape[7:]), 1, 9, 3, 512, 512, 1e-5, None) if shape.startswith("narrow-")
            else synth.ModelShape("dim-4096", 4096, 1024, 1, 32, 8, 512, 256, 1e-5, None) if shape == "dim-4096"
            else synth.ModelShape("dim-8192", 8192, 1024, 1, 64, 8, 512, 256, 1e-5, None) if shape == "dim-8192" else synth.SHAPES[shape])
     model = (synth.build_model(shp, synth.Q4_K, k_m_mix=True, **kw) if fmt == "Q4_K_M" else synth.build_model(shp, getattr(synth, fmt), **kw))
