@@ -130,6 +130,7 @@ struct crabml_hip_device {
   int n_cu = 256;
   int numa_node = -1;         // the host NUMA node the GPU hangs off (sysfs), -1 = unknown
   bool strict_order = false;  // CRABML_HIP_FLAG_STRICT_ORDER
+  int wide_tile = -1;         // test hook: the tile of every quantized prompt GEMM that gemm_f16w_wide.hip covers (-1: the rule)
   std::mutex mu;
   std::string last_error;
   // caching allocator: size class -> free blocks (single stream => stream-ordered reuse is safe)

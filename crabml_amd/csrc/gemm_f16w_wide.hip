@@ -382,12 +382,15 @@ bool launch_f16w_wide(crabml_hip_device* dev, uint32_t dt, F16wMats mats, const 
   if (b <= 64 || k % 256 != 0) return false;
   size_t weights = 0;
   for (int j = 0; j < nw; j++) weights += m[j] * k;
-  // formats of two quant loads a fragment, a launch of a few workgroups: gemm_f16w.hip's 64-row tiles come out even or ahead (models of 512 x 1024, two layers:
-  // Q6_K 4 % of a pass, Q8_0 1 %; 2048 x 2048 this kernel, 2 to 20 %)
-  if ((dt == CRABML_HIP_Q8_0 || dt == CRABML_HIP_Q6_K) && weights < (size_t)2 << 20) return false;
+  const bool forced = dev->wide_tile >= 0 && !(dt == CRABML_HIP_Q6_K && dev->wide_tile == 0);
+  // formats of two quant loads a fragment, a launch of a few workgroups: gemm_f16w.hip's 64-row tiles come out even or ahead.  A pass of four layers of which
+  // this kernel takes every launch / none below the line, Q8_0 (Q6_K), 77, 130, 300, 700 rows: width 512 1.08 1.07 1.06 1.00 (1.08 1.08 1.08 1.03), 768 1.02
+  // 1.02 1.01 0.95 (1.02 1.02 1.03 0.97), 1024 1.04 1.04 1.02 0.96 (1.03 1.02 1.04 0.99), 1280 and 1536, where the narrow launches alone are below it, 1.00
+  // 1.00 1.00 1.00 (1.00 to 1.03); models of 2048 x 2048, all above it, 0.80 to 0.98.
+  if (!forced && (dt == CRABML_HIP_Q8_0 || dt == CRABML_HIP_Q6_K) && weights < (size_t)2 << 20) return false;
   for (int j = 0; j < nw; j++)
     if (m[j] * k >= (size_t)1 << 32) return false;  // (32-bit offsets into the quants)
-  const int tile = f16w_wide_tile(dt == CRABML_HIP_Q6_K, m, nw, k, b, pair, (size_t)dev->n_cu, ws_floats, ksplit);
+  const int tile = forced ? dev->wide_tile : f16w_wide_tile(dt == CRABML_HIP_Q6_K, m, nw, k, b, pair, (size_t)dev->n_cu, ws_floats, ksplit);
   switch (dt) {
     case CRABML_HIP_Q4_0: return launch_wide_fmt<WF_Q4_0>(dev, tile, gu, mats, m, nw, k, xh, b, *ksplit);
     case CRABML_HIP_Q8_0: return launch_wide_fmt<WF_Q8_0>(dev, tile, gu, mats, m, nw, k, xh, b, *ksplit);

@@ -275,6 +275,7 @@ int crabml_hip_device_create(const crabml_hip_device_options_t* opts, crabml_hip
       }
     }
   }
+  if (const char* e = hooks_on ? getenv("CRABML_HIP_WIDE_TILE") : nullptr) dev->wide_tile = atoi(e) < 6 ? atoi(e) : -1;
   if (opts && opts->stream) {
     dev->stream = (hipStream_t)opts->stream;
     dev->own_stream = false;

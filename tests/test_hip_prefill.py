@@ -417,8 +417,8 @@ def test_short_passes_in_pieces_of_k_equal_the_token_loop(ca, fmt, rows, width, 
     assert np.array_equal(a.prefill(toks).view(np.uint32), first.view(np.uint32))  # (added in piece order, whoever ends first)
 
 
-# the wide weight GEMM (rows > 64, k a multiple of 256): a row more and a row less than its tiles of 96 and 128 columns; k of one, two, three (a group of waves
-# without a chunk), 11 and 16 super-blocks; matrices that end inside a tile of 128 or 256 rows
+# the wide weight GEMM (rows > 64, k a multiple of 256) by its own rule: a row more and a row less than its tiles of 96 and 128 columns; k of one, two, three, 11 and 16
+# super-blocks; matrices that end inside a tile of 128 or 256 rows.  (Q8_0, Q6_K: launches of fewer than 2M weights are gemm_f16w.hip's.)
 @pytest.mark.parametrize("fmt", ["Q4_0", "Q8_0", "Q4_1", "Q4_K", "Q6_K"])
 @pytest.mark.parametrize("width,hidden,rows", [(256, 768, 65), (512, 768, 96), (512, 2816, 97), (1024, 1280, 129), (768, 4096, 193), (2048, 1024, 300)])
 def test_wide_prompt_gemm_at_the_edges_of_its_tiles(ca, fmt, width, hidden, rows):
@@ -433,3 +433,47 @@ def test_wide_prompt_gemm_at_the_edges_of_its_tiles(ca, fmt, width, hidden, rows
     assert np.max(np.abs(got - want)) <= FAST_TOL[fmt][1] * np.max(np.abs(want))
     a.reset()
     assert np.array_equal(np.array(a.prefill(toks)).view(np.uint32), got.view(np.uint32))
+
+
+# every tile of the wide weight GEMM in every launch of a pass: two layers, all rows of the cache.  Width 256: k of one super-block (a group of waves without a
+# chunk); 768: three (groups of four and two chunks).  Feed-forwards of 4160 / 4352 rows run gate | up in one tile, of 1280 (five super-blocks) apart.  Rows of a
+# column more and less than tiles of 96 and 128 columns; matrices that end inside a tile of rows
+@pytest.mark.parametrize("fmt", ["Q4_0", "Q8_0", "Q4_1", "Q4_K", "Q6_K"])
+@pytest.mark.parametrize("width,hidden,rows", [(256, 4160, 257), (256, 4160, 383), (768, 1280, 65), (768, 1280, 97), (768, 1280, 193)])
+def test_every_tile_of_the_wide_prompt_gemm(ca, monkeypatch, fmt, width, hidden, rows):
+    if fmt in ("Q4_K", "Q6_K") and hidden == 4160:
+        hidden = 4352
+    shape = synth.ModelShape("tiles", width, hidden, 2, width // 64, width // 256, 300, 512, 1e-5, None)
+    model, toks = synth.build_model(shape, synth.TYPE_BY_NAME[fmt], seed=38), [(19 * i + 7) % 300 for i in range(rows)]
+
+    def run(tile, flags=0):
+        monkeypatch.setenv("CRABML_HIP_TEST_HOOKS", "1")
+        monkeypatch.setenv("CRABML_HIP_WIDE_TILE", str(tile))
+        dev = ca.HipTensorDevice(0)
+        conf, w = synth.to_hip(model, dev)
+        r = ca.HipLlamaRunner(conf, w, dev, 512, True, prefill_chunk=512, extra_flags=flags)
+        logits = np.array(r.prefill(toks))
+        kv = [r.debug_kv(layer, v, True).view(np.float16).reshape(width // 256, 512, 64)[:, :rows] for layer in range(2) for v in (False, True)]
+        return logits, kv
+
+    def rows_off(got, want):  # relative error of each position's row, in the 2-norm
+        got, want = (x.astype(np.float64).transpose(1, 0, 2).reshape(rows, -1) for x in (got, want))
+        return np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+
+    want, want_kv = run(-1, PREFILL_INT8_GEMM)
+    by_order = {}  # k in one piece, in two: the same sums whatever the tile
+    for tile in range(1 if fmt == "Q6_K" else 0, 6):
+        got, kv = run(tile)
+        assert np.max(np.abs(got - want)) <= FAST_TOL[fmt][1] * np.max(np.abs(want)), tile
+        # the first layer's keys and values: two (K-quants: three) f16 roundings a product against exact block sums, and the cache's own: each 2^-11 at most and
+        # 2^-11 / sqrt 3 at the root mean square, independent of each other; four times that
+        for i in (0, 1):
+            assert rows_off(kv[i], want_kv[i]).max() <= 4 * 2 * 2**-11 / 3**0.5, (tile, i, rows_off(kv[i], want_kv[i]).max())
+        # the second layer's, behind four quantizers: at the root mean square over the positions the bound of the logits.  A level that falls the other way
+        # is worth more in a short row: four times the bound for one position, where a row that another position's was taken for is off by more than one
+        for i in (2, 3):
+            off = rows_off(kv[i], want_kv[i])
+            assert np.sqrt(np.mean(off**2)) <= FAST_TOL[fmt][1] and off.max() <= 4 * FAST_TOL[fmt][1], (tile, i, off.max())
+        first = by_order.setdefault(tile // 4, (tile, got, kv))
+        assert np.array_equal(got.view(np.uint32), first[1].view(np.uint32)), (tile, first[0])
+        assert all(np.array_equal(x.view(np.uint16), y.view(np.uint16)) for x, y in zip(kv, first[2])), (tile, first[0])
