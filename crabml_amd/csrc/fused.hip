@@ -3105,6 +3105,8 @@ int lazy_ctx_fault_value(const crabml_hip_llama* c) { return c->dev->dry ? 0 : c
 extern "C" int crabml_hip_debug_exp_of_f16(crabml_hip_device_t* dev, uint16_t* computed, uint16_t* table) {
   using namespace crabml_hip;
   if (!dev || !computed || !table) return CRABML_HIP_BAD_INPUT;
+  CH_LIVE(dev);
+  CH_USE(dev);
   void* d = nullptr;
   CH_HIP(dev, hipMalloc(&d, 65536 * 2));
   k_exp_of_f16<<<256, 256, 0, dev->stream>>>((const unsigned short*)dev->exp_table, (unsigned short*)d);

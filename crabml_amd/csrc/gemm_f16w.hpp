@@ -99,7 +99,7 @@ struct F16wMats {
   int tiles_end[3];  // cumulative row tiles
 };
 // h = silu(g) * u (silu.rs:6-13, arithmetic.rs:57-66; fused_ffn.hpp silu_mul: the exp through the reference's f16 table.  Computed instead, the same bits
-// for every f16, the launch takes as long: 512 rows of 14336 x 4096 133 -> 139 us.)
+// for every f16, the launch takes longer: 512 rows of 14336 x 4096 133 -> 139 us.)
 __device__ __forceinline__ float f16w_silu_mul(float g, float u, const unsigned short* __restrict__ exp_tab) {
   const float nexp = h2f(exp_tab[f2h(-g)]);
   return (g / (1.0f + nexp)) * u;
