@@ -429,7 +429,7 @@ bool gemm_f16w_covers(uint32_t w_dtype, uint32_t act_qtype) {
 // wave tile: T column tiles of 16 prompt rows -- 8 (128-row workgroup tiles) from 65 rows up; short passes (a short prompt, the ragged
 // tail of a long one) take 4 / 2: the MFMAs of an empty column tile cost what a full one's do
 static int f16w_col_tiles_per_wave(size_t b, int variant) { return (variant & 512) ? 4 : (variant & 16) ? 8 : b <= 32 ? 2 : b <= 64 ? 4 : 8; }
-// (K-quants past 64 rows are gemm_f16w_wide.hip's, but for Q6_K launches of fewer than 2M weights and for what its launcher refuses)
+// (gate | up in one tile past 64 rows is gemm_f16w_wide.hip's where k is a multiple of 256, as it is of K-quants, but for what its launcher refuses)
 template <int WF>
 static bool launch_f16w_fmt(crabml_hip_device* dev, const F16wMats& mats, int row_tiles, size_t k, const void* xh, size_t b, int ksplit, int F, bool gu, int T,
                             int NW) {
@@ -459,6 +459,68 @@ static bool f16w_eight_waves(size_t tiles, size_t n_cu) {
   const size_t rounds = (tiles + n_cu - 1) / n_cu;
   return rounds == 1 ? 4 * tiles >= 3 * n_cu : 20 * tiles >= 17 * rounds * n_cu;
 }
+// How k_gemm_f16w would take a launch: column tiles and fragments of a wave, gate | up in one tile (pair), pieces of k
+struct F16wPlan {
+  int T, F, ksplit;
+  bool pair;
+  size_t cols, row_tiles;
+};
+static F16wPlan f16w_plan(uint32_t dt, const size_t* m, int nw, size_t k, size_t b, size_t n_cu, size_t ws_floats, int variant) {
+  F16wPlan p{};
+  size_t mtot = 0;
+  for (int j = 0; j < nw; j++) mtot += m[j];
+  p.T = f16w_col_tiles_per_wave(b, variant);
+  // Q4_K past 64 rows, where only launches of few workgroups come here: 64 columns a tile take 0.57 to 0.9 of the time of 128 (1.13 at the worst, 1536 x 4096 of 65)
+  if (dt == CRABML_HIP_Q4_K && p.T == 8) p.T = 4;
+  p.cols = (b + 16 * (size_t)p.T - 1) / (16 * (size_t)p.T);
+  // two fragments per wave (every B' fragment read from LDS feeds two MFMAs) when 128-row tiles still cover the chip
+  p.F = ((mtot + 127) / 128) * p.cols >= n_cu ? 2 : 1;
+  if ((variant & 1024) && p.F == 1 && p.T == 8 && b >= 128) {  // lab: narrow launches as two fragments x four column tiles
+    p.F = 2;
+    p.T = 4;
+    p.cols = (b + 63) / 64;
+  }
+  if ((variant & 7) == 1) p.F = 2;
+  if ((variant & 7) == 3) p.F = 1;
+  // gate | up with the SiLU * mul epilogue (out[0] = h, out[1] untouched): when 64-row tiles of both matrices cover the chip without
+  // cutting k
+  p.pair = nw == 2 && m[0] == m[1] && !(variant & 64) && ((m[0] + 63) / 64) * p.cols * 2 >= n_cu * 3;
+  for (int j = 0; j < nw; j++) p.row_tiles += (m[j] + 64 * p.F - 1) / (64 * p.F);
+  // pieces of k: double while the launch is short of ~1.5 workgroups per CU, every piece keeps >= 4 chunks (and whole super-blocks),
+  // and the partial buffers fit the scratch
+  const size_t chunks = (k + 127) / 128;
+  p.ksplit = 1;
+  if (!(variant & 8) && k % 128 == 0)
+    while (p.ksplit < 8 && p.row_tiles * p.cols * p.ksplit < n_cu * 3 / 2 && chunks % (size_t)(4 * p.ksplit) == 0 &&
+           chunks / (size_t)(2 * p.ksplit) >= (size_t)((variant & 32) ? 8 : 4) && (size_t)(2 * p.ksplit - 1) * mtot * b <= ws_floats)
+      p.ksplit *= 2;
+  return p;
+}
+// gate | up whose 64-row tiles give three CUs in four something to do: in gemm_f16w_wide.hip's tiles k stays whole then, with or without the epilogue
+static bool f16w_wide_pair(const size_t* m, int nw, size_t b, size_t n_cu) { return nw == 2 && m[0] == m[1] && ((m[0] + 63) / 64) * ((b + 127) / 128) * 4 >= n_cu * 3; }
+// Which kernel.  gemm_f16w_wide.hip's wants whole super-blocks of k, and workgroups enough: launches of few of them are faster with the 64-row tiles of this file's
+// (a layer of 256 x 768 at 128 rows, q | k | v: Q4_0 7.7 us against 6.0, Q4_K 7.9 / 4.3; 1280 x 1280 Q4_K 11.6 / 9.2, Q4_0 11.1 / 12.8; 1536 x 1536 Q4_0 11.9 /
+// 10.1, Q8_0 and Q6_K alike; 3072 x 3072 Q4_0 13.0 / 11.0, at 300 rows 13.6 / 24.2).  Both are estimated: a constant, what a chunk of k takes over the rounds of
+// CUs, the rounds behind the first, and pieces of k, which cost a launch to add them unless the consumer does.  Fitted to 2880 launches of five formats (q | k | v, wo,
+// gate | up, ffn_down of twelve models of 256 x 768 to 4096 x 11008, 65 to 1000 rows); the kernel chosen takes 0.1 to 0.2 % longer than the faster one on
+// average (26 launches more than 5 %, 1.24 times as long at the worst).  Whole passes of six layers of 256 to 2048, 65 to 1000 rows, that take every launch with
+// gemm_f16w_wide.hip: up to 1.17 of the time of this file's kernel alone (256 wide), 0.92 on average by this rule and none of 400 longer by more than runs differ.
+static float f16w_narrow_us(uint32_t dt, const size_t* m, int nw, size_t b, size_t k, size_t n_cu, bool deferred, const F16wPlan& p) {
+  size_t total = 0;
+  for (int j = 0; j < nw; j++) total += m[j];
+  const bool small = p.T == 4;  // (Q4_K)
+  const float alone = p.F == 1 ? (small ? .56f : .82f) : small ? 1.f : 1.37f, shared = p.F == 1 ? (small ? .95f : 1.6f) : small ? 1.63f : 2.4f;
+  const float format = dt == CRABML_HIP_Q4_1 ? 1.03f : dt == CRABML_HIP_Q8_0 ? 1.12f : dt == CRABML_HIP_Q6_K ? 1.2f : 1.f;
+  float rounds;
+  const float chunk = f16w_chunk_us(p.row_tiles * p.cols * p.ksplit, n_cu, alone, shared, &rounds);
+  return (small ? 3.3f : 4.3f) + (small ? .4f : 3.2f) * (rounds - 1.f) + format * chunk * (float)(k / 128 / p.ksplit) +
+         (p.ksplit == 1 ? 0.f : deferred ? 1.1e-6f * (float)p.ksplit * (float)(total * b) : 3.9f + 1.2e-6f * (float)p.ksplit * (float)(total * b));
+}
+static bool f16w_takes_wide(uint32_t dt, const size_t* m, int nw, size_t k, size_t b, size_t n_cu, size_t ws_floats, bool deferred, const F16wPlan& p) {
+  if (b <= 64 || k % 256 != 0) return false;
+  if (p.pair || f16w_wide_pair(m, nw, b, n_cu)) return true;
+  return f16w_wide_us(dt, m, nw, k, b, n_cu, ws_floats, deferred) <= f16w_narrow_us(dt, m, nw, b, k, n_cu, deferred, p);
+}
 // nw weight matrices (one format, the same k) against the same rhs rows: out[j] (b, m[j]) = W[j] . x
 // ws (nullable), ws_floats: scratch for split launches.  When the output tiles alone leave the chip underfilled -- wo / ffn_down (few
 // row tiles, a long k), any short pass -- the k range is cut into 2 / 4 / 8 pieces, one workgroup each: piece 0 writes out, the
@@ -483,7 +545,7 @@ bool launch_gemm_f16w(crabml_hip_device* dev, const crabml_hip_buf* const* w, co
   }();
   F16wMats mats{};
   F16wParts parts{};
-  size_t mtot = 0, before = 0;  // rows; output elements of the matrices before j
+  size_t before = 0;  // output elements of the matrices before j
   mats.exp_tab = gu_exp_tab;
   for (int j = 0; j < 3; j++) {
     const int jj = j < nw ? j : nw - 1;
@@ -497,10 +559,7 @@ bool launch_gemm_f16w(crabml_hip_device* dev, const crabml_hip_buf* const* w, co
     mats.m[j] = (int)m[jj];
     parts.out[j] = out[jj];
     parts.part[j] = ws + before;
-    if (j < nw) {
-      mtot += m[j];
-      before += b * m[j];
-    }
+    if (j < nw) before += b * m[j];
     parts.end4[j] = before / 4;
   }
   mats.pstride = parts.pstride = before;
@@ -515,37 +574,20 @@ bool launch_gemm_f16w(crabml_hip_device* dev, const crabml_hip_buf* const* w, co
     }
     return true;
   };
-  {
-    // gate | up whose 64-row tiles give three CUs in four something to do: k stays whole (with or without the epilogue: the same sums)
-    const bool pair = nw == 2 && m[0] == m[1] && ((m[0] + 63) / 64) * ((b + 127) / 128) * 4 >= (size_t)dev->n_cu * 3;
-    const bool gu = pair && gu_exp_tab != nullptr && gu_done != nullptr;
+  if (ws == nullptr) ws_floats = 0;
+  const F16wPlan plan = f16w_plan(dt, m, nw, k, b, (size_t)dev->n_cu, ws_floats, variant);
+  if (f16w_takes_wide(dt, m, nw, k, b, (size_t)dev->n_cu, ws_floats, defer_parts != nullptr && nw == 1, plan) || dev->wide_tile >= 0) {
+    const bool pair = f16w_wide_pair(m, nw, b, (size_t)dev->n_cu), gu = pair && gu_exp_tab != nullptr && gu_done != nullptr;
     const bool hquant = gu && hq != nullptr && hq->planes != nullptr && m[0] % 32 == 0;
     if (hquant) mats.hq = *hq;
-    if (launch_f16w_wide(dev, dt, mats, m, nw, k, xh, b, pair, gu, ws != nullptr ? ws_floats : 0, &ksplit)) return finish(gu, hquant);
+    if (launch_f16w_wide(dev, dt, mats, m, nw, k, xh, b, pair, gu, ws_floats, &ksplit)) return finish(gu, hquant);
     mats.hq = F16wHQuant{};
-    ksplit = 1;
   }
-  int T = f16w_col_tiles_per_wave(b, variant);
-  if (dt == CRABML_HIP_Q4_K && T == 8) T = 4;  // (refused by the wide launcher)
-  size_t cw = 16 * (size_t)T, col128 = (b + cw - 1) / cw;  // (column tiles of the launch)
-  // two fragments per wave (every B' fragment read from LDS feeds two MFMAs) when 128-row tiles still cover the chip
-  int F = ((mtot + 127) / 128) * col128 >= (size_t)dev->n_cu ? 2 : 1;
-  if ((variant & 1024) && F == 1 && T == 8 && b >= 128) {  // lab: narrow launches as two fragments x four column tiles
-    F = 2;
-    T = 4;
-    cw = 64;
-    col128 = (b + cw - 1) / cw;
-  }
-  if ((variant & 7) == 1) F = 2;
-  if ((variant & 7) == 3) F = 1;
-  // gate | up with the SiLU * mul epilogue (out[0] = h, out[1] untouched): when 64-row tiles of both matrices cover the chip without
-  // cutting k
-  const bool gu = gu_exp_tab != nullptr && gu_done != nullptr && nw == 2 && m[0] == m[1] && !(variant & 64) &&
-                  ((m[0] + 63) / 64) * col128 * 2 >= (size_t)dev->n_cu * 3;
-  if (gu) F = 2;
+  const bool gu = plan.pair && gu_exp_tab != nullptr && gu_done != nullptr;
+  const int T = plan.T, F = gu ? 2 : plan.F;
   // (gate | up alone.  512 rows, Q4_0 183 -> 173 us, the whole request 3973 -> 3785.  The other launches, cut in k to fill the chip with the smaller
   // tiles, do not gain: ffn_down 115 -> 108, wo 35 -> 44; four fragments a wave, one wave a SIMD, lose: 183 -> 211.)
-  const int NW = gu && T == 8 && dt != CRABML_HIP_Q6_K && f16w_eight_waves((m[0] + 127) / 128 * col128, (size_t)dev->n_cu) ? 8 : 4;
+  const int NW = gu && T == 8 && dt != CRABML_HIP_Q6_K && f16w_eight_waves((m[0] + 127) / 128 * plan.cols, (size_t)dev->n_cu) ? 8 : 4;
   const bool hquant = gu && hq != nullptr && hq->planes != nullptr && m[0] % 32 == 0;
   if (hquant) mats.hq = *hq;
   int row_tiles = 0;
@@ -556,13 +598,7 @@ bool launch_gemm_f16w(crabml_hip_device* dev, const crabml_hip_buf* const* w, co
       row_tiles += (int)((m[j] + 64 * F - 1) / (64 * F));
     mats.tiles_end[j] = row_tiles;
   }
-  // pieces of k: double while the launch is short of ~1.5 workgroups per CU, every piece keeps >= 4 chunks (and whole super-blocks),
-  // and the partial buffers fit the scratch
-  const size_t chunks = (k + 127) / 128;
-  if (ws != nullptr && !(variant & 8) && k % 128 == 0 && !gu)
-    while (ksplit < 8 && (size_t)row_tiles * col128 * ksplit < (size_t)dev->n_cu * 3 / 2 && chunks % (size_t)(4 * ksplit) == 0 &&
-           chunks / (size_t)(2 * ksplit) >= (size_t)((variant & 32) ? 8 : 4) && (size_t)(2 * ksplit - 1) * before <= ws_floats)
-      ksplit *= 2;
+  ksplit = gu ? 1 : plan.ksplit;
   bool ok;
   if (dt == CRABML_HIP_Q8_0)
     ok = launch_f16w_fmt<WF_Q8_0>(dev, mats, row_tiles, k, xh, b, ksplit, F, gu, T, NW);
@@ -592,5 +628,13 @@ void launch_add_parts(hipStream_t st, float* out, const float* ws, size_t n, int
 extern "C" int crabml_hip_debug_gateup_waves(size_t hidden, size_t rows, int32_t n_cu, int32_t* waves) {
   if (!waves || n_cu < 1) return CRABML_HIP_BAD_INPUT;
   *waves = crabml_hip::f16w_eight_waves((hidden + 127) / 128 * ((rows + 127) / 128), (size_t)n_cu) ? 8 : 4;
+  return 0;
+}
+extern "C" int crabml_hip_debug_prompt_gemm(uint32_t dtype, size_t m0, size_t m1, size_t m2, size_t k, size_t b, int32_t n_cu, size_t ws_floats, int32_t deferred, int32_t* wide) {
+  using namespace crabml_hip;
+  if (!wide || n_cu < 1 || m0 == 0 || b <= 64 || k == 0 || k % 256 != 0) return CRABML_HIP_BAD_INPUT;
+  const size_t m[3] = {m0, m1, m2};
+  const int nw = m2 ? 3 : m1 ? 2 : 1;
+  *wide = f16w_takes_wide(dtype, m, nw, k, b, (size_t)n_cu, ws_floats, deferred != 0 && nw == 1, f16w_plan(dtype, m, nw, k, b, (size_t)n_cu, ws_floats, 0));
   return 0;
 }

@@ -164,7 +164,15 @@ __device__ __forceinline__ void f16w_quantize_h(const float* H, const F16wHQuant
   }
 }
 
-// gemm_f16w_wide.hip: passes of more than 64 rows, k a multiple of 256.  false: not covered.  ksplit: the pieces of k that a launch of its own or the consumer adds
+// what a chunk of k takes a launch over its rounds of CUs, where a workgroup's takes `alone` with a CU to itself and `shared` beside another (0: it has one to itself)
+inline float f16w_chunk_us(size_t wgs, size_t n_cu, float alone, float shared, float* rounds) {
+  const size_t slots = n_cu * (shared > 0.f ? 2 : 1), rest = wgs % slots;
+  *rounds = (float)(wgs / slots) + (rest != 0);
+  return (float)(wgs / slots) * (shared > 0.f ? shared : alone) + (rest == 0 ? 0.f : rest <= n_cu ? alone : shared);
+}
+// gemm_f16w_wide.hip, passes of more than 64 rows, k a multiple of 256.  Estimated time of the launch that it would make, us; deferred: pieces of k are the consumer's
+float f16w_wide_us(uint32_t dt, const size_t* m, int nw, size_t k, size_t b, size_t n_cu, size_t ws_floats, bool deferred);
+// false: not covered.  ksplit: the pieces of k that a launch of its own or the consumer adds
 bool launch_f16w_wide(crabml_hip_device* dev, uint32_t dt, F16wMats mats, const size_t* m, int nw, size_t k, const void* xh, size_t b, bool pair, bool gu,
                       size_t ws_floats, int* ksplit);
 

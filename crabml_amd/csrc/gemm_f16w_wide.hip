@@ -335,8 +335,8 @@ struct WideTile {
 };
 static constexpr WideTile WIDE_TILES[6] = {{4, 8, 1, 1.61f, 3.1f}, {4, 6, 1, 1.36f, 2.49f}, {2, 8, 1, 1.05f, 1.78f}, {2, 6, 1, .85f, 1.49f}, {2, 8, 2, 1.77f, 0.f}, {2, 6, 2, 1.44f, 0.f}};
 // rows[0 .. nw): of the matrices; pair: gate | up, whose tiles hold rows of both and whose k stays in one workgroup (the same choice with and without the
-// epilogue: the same sums); six_bits: Q6_K, whose registers hold no tile of 4 x 8; -> index into WIDE_TILES
-static int f16w_wide_tile(bool six_bits, const size_t* rows, int nw, size_t k, size_t b, bool pair, size_t n_cu, size_t ws_floats, int* ksplit) {
+// epilogue: the same sums); six_bits: Q6_K, whose registers hold no tile of 4 x 8; -> index into WIDE_TILES; parts: chunks' time, rounds of CUs
+static int f16w_wide_tile(bool six_bits, const size_t* rows, int nw, size_t k, size_t b, bool pair, size_t n_cu, size_t ws_floats, int* ksplit, float (&parts)[2]) {
   size_t total = 0;
   for (int j = 0; j < nw; j++) total += rows[j];
   int best = -1;
@@ -351,18 +351,30 @@ static int f16w_wide_tile(bool six_bits, const size_t* rows, int nw, size_t k, s
     for (int ks = 1; ks <= (pair ? 1 : 8); ks *= 2) {
       const size_t pieces = (size_t)(ks * w.kg), chunks = (((k / 128 + pieces - 1) / pieces) + 1) & ~(size_t)1;
       if (ks > 1 && (chunks * (pieces - 1) >= k / 128 || (size_t)(ks - 1) * total * b > ws_floats)) break;
-      const size_t wgs = tiles * cols * ks, slots = n_cu * (w.shared > 0.f ? 2 : 1), rest = wgs % slots;
-      const float rounds = (float)(wgs / slots) + (rest != 0);
-      float us = (float)(wgs / slots) * (w.shared > 0.f ? w.shared : w.alone) + (rest == 0 ? 0.f : rest <= n_cu ? w.alone : w.shared);
-      us = us * (float)chunks + 4.6f + 3.7f * (rounds - 1.f) + (ks > 1 ? 4.f + 1.2e-6f * (float)ks * (float)(total * b) : 0.f);
+      float rounds;
+      const float chunks_us = f16w_chunk_us(tiles * cols * ks, n_cu, w.alone, w.shared, &rounds) * (float)chunks;
+      const float us = chunks_us + 4.6f + 3.7f * (rounds - 1.f) + (ks > 1 ? 4.f + 1.2e-6f * (float)ks * (float)(total * b) : 0.f);
       if (best < 0 || us < least) {
         best = c;
         least = us;
         *ksplit = ks;
+        parts[0] = chunks_us;
+        parts[1] = rounds;
       }
     }
   }
   return best;
+}
+// By format, against launch_gemm_f16w's own estimate (f16w_narrow_us): fitted to which of the two kernels is the faster one (there)
+float f16w_wide_us(uint32_t dt, const size_t* m, int nw, size_t k, size_t b, size_t n_cu, size_t ws_floats, bool deferred) {
+  size_t total = 0;
+  for (int j = 0; j < nw; j++) total += m[j];
+  float parts[2] = {};
+  int ks = 1;
+  f16w_wide_tile(dt == CRABML_HIP_Q6_K, m, nw, k, b, false, n_cu, ws_floats, &ks, parts);
+  const float format = dt == CRABML_HIP_Q4_0 ? .76f : dt == CRABML_HIP_Q4_1 ? .78f : dt == CRABML_HIP_Q8_0 ? 1.31f : dt == CRABML_HIP_Q4_K ? .92f : 1.42f;
+  return 4.7f + 2.5f * (parts[1] - 1.f) + format * parts[0] +
+         (ks == 1 ? 0.f : deferred ? .9e-6f * (float)ks * (float)(total * b) : 3.3f + 1.5e-6f * (float)ks * (float)(total * b));
 }
 template <int WF>
 static bool launch_wide_fmt(crabml_hip_device* dev, int tile, bool gu, F16wMats& mats, const size_t* m, int nw, size_t k, const void* xh, size_t b, int ksplit) {
@@ -380,17 +392,11 @@ static bool launch_wide_fmt(crabml_hip_device* dev, int tile, bool gu, F16wMats&
 bool launch_f16w_wide(crabml_hip_device* dev, uint32_t dt, F16wMats mats, const size_t* m, int nw, size_t k, const void* xh, size_t b, bool pair, bool gu,
                       size_t ws_floats, int* ksplit) {
   if (b <= 64 || k % 256 != 0) return false;
-  size_t weights = 0;
-  for (int j = 0; j < nw; j++) weights += m[j] * k;
-  const bool forced = dev->wide_tile >= 0 && !(dt == CRABML_HIP_Q6_K && dev->wide_tile == 0);
-  // formats of two quant loads a fragment, a launch of a few workgroups: gemm_f16w.hip's 64-row tiles come out even or ahead.  A pass of four layers of which
-  // this kernel takes every launch / none below the line, Q8_0 (Q6_K), 77, 130, 300, 700 rows: width 512 1.08 1.07 1.06 1.00 (1.08 1.08 1.08 1.03), 768 1.02
-  // 1.02 1.01 0.95 (1.02 1.02 1.03 0.97), 1024 1.04 1.04 1.02 0.96 (1.03 1.02 1.04 0.99), 1280 and 1536, where the narrow launches alone are below it, 1.00
-  // 1.00 1.00 1.00 (1.00 to 1.03); models of 2048 x 2048, all above it, 0.80 to 0.98.
-  if (!forced && (dt == CRABML_HIP_Q8_0 || dt == CRABML_HIP_Q6_K) && weights < (size_t)2 << 20) return false;
   for (int j = 0; j < nw; j++)
     if (m[j] * k >= (size_t)1 << 32) return false;  // (32-bit offsets into the quants)
-  const int tile = forced ? dev->wide_tile : f16w_wide_tile(dt == CRABML_HIP_Q6_K, m, nw, k, b, pair, (size_t)dev->n_cu, ws_floats, ksplit);
+  float parts[2];
+  const bool forced = dev->wide_tile >= 0 && !(dt == CRABML_HIP_Q6_K && dev->wide_tile == 0);
+  const int tile = forced ? dev->wide_tile : f16w_wide_tile(dt == CRABML_HIP_Q6_K, m, nw, k, b, pair, (size_t)dev->n_cu, ws_floats, ksplit, parts);
   switch (dt) {
     case CRABML_HIP_Q4_0: return launch_wide_fmt<WF_Q4_0>(dev, tile, gu, mats, m, nw, k, xh, b, *ksplit);
     case CRABML_HIP_Q8_0: return launch_wide_fmt<WF_Q8_0>(dev, tile, gu, mats, m, nw, k, xh, b, *ksplit);
@@ -408,7 +414,8 @@ extern "C" int crabml_hip_debug_wide_tile(uint32_t dtype, size_t m0, size_t m1, 
   using namespace crabml_hip;
   if (!tile || n_cu < 1 || m0 == 0 || b <= 64 || k == 0 || k % 256 != 0) return CRABML_HIP_BAD_INPUT;
   const size_t rows[3] = {m0, m1, m2};
-  const WideTile& w = WIDE_TILES[f16w_wide_tile(dtype == CRABML_HIP_Q6_K, rows, m2 ? 3 : m1 ? 2 : 1, k, b, pair != 0, (size_t)n_cu, ws_floats, tile + 3)];
+  float parts[2];
+  const WideTile& w = WIDE_TILES[f16w_wide_tile(dtype == CRABML_HIP_Q6_K, rows, m2 ? 3 : m1 ? 2 : 1, k, b, pair != 0, (size_t)n_cu, ws_floats, tile + 3, parts)];
   tile[0] = w.f;
   tile[1] = w.t;
   tile[2] = w.kg;

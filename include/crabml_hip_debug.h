@@ -68,6 +68,8 @@ int crabml_hip_debug_exp_of_f16(crabml_hip_device_t* dev, uint16_t* computed, ui
 /* Tile of the fast prompt pass's weight GEMM over b > 64 rows, k a multiple of 256: fragments and column tiles of a wave, groups of waves along k in a
  * workgroup, pieces of k in memory.  m0, m1, m2: the launch's matrices (0: none); pair: gate | up in one tile.  Host only. */
 int crabml_hip_debug_wide_tile(uint32_t dtype, size_t m0, size_t m1, size_t m2, size_t k, size_t b, int32_t pair, int32_t n_cu, size_t ws_floats, int32_t* tile);
+/* Whether that GEMM runs such a tile (1) or the kernel of short passes and other widths (0).  deferred: pieces of k are added by the consumer.  Host only. */
+int crabml_hip_debug_prompt_gemm(uint32_t dtype, size_t m0, size_t m1, size_t m2, size_t k, size_t b, int32_t n_cu, size_t ws_floats, int32_t deferred, int32_t* wide);
 /* Rows of wo / ffn_down that a workgroup of a llama step takes: with the next norm in the launch or without, block-ordered sums (strict device), one or two
  * workgroups a 32-row chunk.  The launch's grid and what attention touches ahead of it both come from this.  Host only. */
 int crabml_hip_debug_residual_rows(int32_t norm_epilogue, int32_t ordered, int32_t split, int32_t* rows);

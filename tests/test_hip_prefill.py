@@ -418,7 +418,7 @@ def test_short_passes_in_pieces_of_k_equal_the_token_loop(ca, fmt, rows, width, 
 
 
 # the wide weight GEMM (rows > 64, k a multiple of 256) by its own rule: a row more and a row less than its tiles of 96 and 128 columns; k of one, two, three, 11 and 16
-# super-blocks; matrices that end inside a tile of 128 or 256 rows.  (Q8_0, Q6_K: launches of fewer than 2M weights are gemm_f16w.hip's.)
+# super-blocks; matrices that end inside a tile of 128 or 256 rows.  (Launches of few workgroups are gemm_f16w.hip's.)
 @pytest.mark.parametrize("fmt", ["Q4_0", "Q8_0", "Q4_1", "Q4_K", "Q6_K"])
 @pytest.mark.parametrize("width,hidden,rows", [(256, 768, 65), (512, 768, 96), (512, 2816, 97), (1024, 1280, 129), (768, 4096, 193), (2048, 1024, 300)])
 def test_wide_prompt_gemm_at_the_edges_of_its_tiles(ca, fmt, width, hidden, rows):

@@ -117,6 +117,20 @@ def test_a_run_captures_behind_its_own_steps(nodes):
             made += 1 if place < 0 else top >> place
 
 
+@pytest.mark.parametrize("dtype,rows,k,b,narrow_us,wide_us", [
+    (2, (256, 0, 0), 256, 300, 5.9, 7.8), (2, (256, 64, 64), 256, 128, 6.0, 7.7), (2, (768, 768, 0), 256, 300, 6.4, 8.4), (2, (1536, 0, 0), 1536, 128, 10.1, 11.9),
+    (2, (3072, 0, 0), 3072, 65, 10.4, 13.5), (2, (3072, 0, 0), 3072, 300, 24.2, 13.6), (2, (1280, 320, 320), 1280, 300, 13.4, 11.4), (2, (3072, 0, 0), 8192, 300, 47.3, 27.1),
+    (2, (4096, 1024, 1024), 4096, 128, 26.9, 20.3), (3, (1536, 0, 0), 1536, 128, 9.8, 12.2), (3, (1536, 384, 384), 1536, 1000, 31.7, 14.3), (8, (1536, 0, 0), 4096, 300, 21.3, 13.3),
+    (8, (4096, 0, 0), 4096, 1000, 56.7, 39.6), (12, (256, 64, 64), 256, 65, 4.3, 7.2), (12, (1280, 0, 0), 3584, 65, 11.5, 16.4), (12, (1536, 0, 0), 1536, 300, 7.0, 12.8),
+    (12, (4096, 0, 0), 11008, 65, 50.6, 22.6), (12, (2048, 512, 512), 2048, 700, 34.1, 17.1), (14, (1280, 0, 0), 3584, 65, 17.4, 21.5), (14, (1536, 384, 384), 1536, 65, 12.6, 15.9),
+    (14, (1536, 384, 384), 1536, 1000, 33.6, 17.6), (14, (3072, 0, 0), 8192, 65, 22.5, 15.6)])
+def test_prompt_gemm_runs_the_faster_kernel(dtype, rows, k, b, narrow_us, wide_us):
+    """launches that were timed with both"""
+    wide, size = ctypes.c_int32(), ctypes.c_size_t
+    assert lib.crabml_hip_debug_prompt_gemm(dtype, size(rows[0]), size(rows[1]), size(rows[2]), size(k), size(b), 256, size(2048 * max(sum(rows), 4096)), 1, ctypes.byref(wide)) == 0
+    assert wide.value == (wide_us < narrow_us)
+
+
 @pytest.mark.parametrize("hidden,rows,waves", [
     (14336, 300, 4), (14336, 384, 4), (14336, 640, 4), (11008, 450, 4), (8192, 700, 4), (8192, 200, 4), (8640, 200, 4), (8640, 512, 4), (7680, 896, 4),
     (14336, 130, 8), (14336, 256, 8), (14336, 512, 8), (14336, 768, 8), (14336, 1024, 8), (8192, 300, 8), (8640, 300, 8), (8640, 850, 8), (16384, 200, 8)])
