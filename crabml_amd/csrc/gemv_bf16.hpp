@@ -114,7 +114,7 @@ struct GemvBf16 {
   int mean_n = 1;
   float eps = 0.f;
   const float* gain = nullptr;
-  int k_split = 0, n_ss = 0, ld_ss = 0;  // (ld_ss: even)
+  int k_split = 0, n_ss = 0, ld_ss = 0;  // (ld_ss: whole fours)
   const float* ss = nullptr;
   ActRanges act;
   const float* xielu = nullptr;  // {softplus(p), 1/2 + softplus(q)}
@@ -497,21 +497,14 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
       for (int j = 0; j < XR; j++) xv[d][h * XR + j] = *(const i32x4*)(x + h * second + xo[j]);
     if constexpr (IN == GEMV_IN_RMSV) gv[d] = *(const f32x4*)(gb + i * 256 + (unsigned)c16 * 16);
   };
-  // a row's sum of squares: NT / 16 threads, its first pieces requested ahead of the weights (loads come back in order).  Pieces of 8 columns: as pairs
-  constexpr int QT = NT / 16, QP = 4, QC = EIGHT && !TAIL ? 2 : 1;
-  const int q_row = tid / QT, q_at = tid % QT, n_ss = (a.n_ss + QC - 1) / QC;
-  const float* q_ss = PIECES ? a.ss + (size_t)(q_row < a.nb ? q_row : a.nb - 1) * a.ld_ss : nullptr;
-  auto square = [&](int i) -> f32x2 {
-    if constexpr (QC == 1)
-      return f32x2{q_ss[i], 0.f};
-    else
-      return *(const f32x2*)(q_ss + 2 * i);
-  };
-  f32x2 q_v[QP];
-  if constexpr (PIECES) {
-#pragma unroll
-    for (int u = 0; u < QP; u++) q_v[u] = square(q_at + u * QT < n_ss ? q_at + u * QT : 0);
-  }
+  // A row's sum of squares, by pieces of 16 columns (two of 8): piece q + QT u belongs to term q, in the order of u, the terms meet by neighbours, pairs, ...  A lane
+  // requests 16 bytes -- QC neighbouring terms of one u, QU of which a row's QR threads have at a time -- the first ahead of the weights (loads come back in order).
+  constexpr bool QTWO = EIGHT && !TAIL;
+  constexpr int QT = NT / 16, QC = QTWO ? 2 : 4, QL = QT / QC, QR = QTWO ? 64 : QT, QU = QR / QL;
+  const int q_row = tid / QR, q_at = tid % QR, q_j = q_at % QL, q_u = q_at / QL, n4 = (a.n_ss + 3) / 4;
+  const f32x4* q_ss = PIECES ? (const f32x4*)(a.ss + (size_t)(q_row < a.nb ? q_row : a.nb - 1) * a.ld_ss) : nullptr;
+  f32x4 q_v = {0.f, 0.f, 0.f, 0.f};
+  if constexpr (PIECES) q_v = q_ss[q_u * QL + q_j < n4 ? q_u * QL + q_j : 0];
   float tail[XR], sq[XR];  // of row 4 j + r16
   const float* t_ss[XR];
 #pragma unroll
@@ -659,18 +652,28 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
     }
   }
   if constexpr (PIECES) {
-    float t = 0.f;
-    auto take = [&](int q, f32x2 v) {  // (behind the last piece: whatever is there)
-      const float second = QC == 2 && 2 * q + 1 < a.n_ss ? v[1] : 0.f;
-      t += q < n_ss ? (QC == 2 ? v[0] + second : v[0]) : 0.f;
-    };
+    float term[QC] = {};
+    for (int u0 = 0; u0 * QL < n4; u0 += QU) {
+      const int at = (u0 + q_u) * QL + q_j;
+      if (u0 > 0) q_v = q_ss[at < n4 ? at : 0];
+      float v[4];
 #pragma unroll
-    for (int u = 0; u < QP; u++) take(q_at + u * QT, q_v[u]);
-    for (int i = q_at + QP * QT; i < n_ss; i += QT) take(i, square(i));
-    t = row16_sum_f32(t);
-    t += __shfl_xor(t, 16, 64);
-    if constexpr (QT == 64) t += __shfl_xor(t, 32, 64);
-    if (q_at == 0) scale[q_row] = (!TAIL && a.gain ? *a.gain : 1.0f) / sqrtf(t / (float)a.mean_n + a.eps);
+      for (int e = 0; e < 4; e++) v[e] = 4 * at + e < a.n_ss ? q_v[e] : 0.f;  // (behind the last piece: whatever is there)
+      float p[QC];
+#pragma unroll
+      for (int c = 0; c < QC; c++) p[c] = QTWO ? v[2 * c] + v[2 * c + 1] : v[c];
+#pragma unroll
+      for (int s = 0; s < QU; s++) {
+        if ((u0 + s) * QL >= n4) break;  // (uniform)
+#pragma unroll
+        for (int c = 0; c < QC; c++) term[c] += s == 0 ? p[c] : __shfl(p[c], (lane & ~(QR - 1)) + s * QL + q_j, 64);  // (what is used is in the lanes of u = 0)
+      }
+    }
+    float t = QC == 2 ? term[0] + term[1] : (term[0] + term[1]) + (term[QC - 2] + term[QC - 1]);
+    t = group_sum<8>(t);
+    if constexpr (QL >= 16) t += dpp_f<0x140>(t);
+    if constexpr (QL == 32) t += __shfl_xor(t, 16, 64);
+    if (q_at == 0 && q_row < 16) scale[q_row] = (!TAIL && a.gain ? *a.gain : 1.0f) / sqrtf(t / (float)a.mean_n + a.eps);
   }
   __syncthreads();  // (the tiles of results take the place of the operands')
   if constexpr (TAIL) {
