@@ -1,5 +1,5 @@
-// gemm_f16w.hip -- the FAST prompt pass's weight GEMM, its operands, and its kernel for up to 64 rows and widths that are no multiple of 256; the others:
-// gemm_f16w_wide.hip (crabml_hip_llama_prefill on the fast device; Q4_0 / Q8_0 weights x Q8_0 rows,
+// gemm_f16w.hip -- the FAST prompt pass's weight GEMM, its operands, and its kernel for up to 64 rows, widths that are no multiple of 256 and launches of few
+// workgroups; the others: gemm_f16w_wide.hip (crabml_hip_llama_prefill on the fast device; Q4_0 / Q8_0 weights x Q8_0 rows,
 // Q4_1 x Q8_1, Q4_K / Q6_K x Q8_K): weight-stationary on the f16 matrix cores.
 //
 // matmul_vec with a batched rhs is `C[b, m] = W[m, k] . x[b, k]` (matmul_vec.rs:41-76: the (b, k) rhs contract; llama2.rs:111-129).

@@ -1,5 +1,5 @@
 // gemm_f16w_wide.hip -- the fast prompt pass's weight GEMM (gemm_f16w.hip: operands, formats, k-slot orders) for passes of more than 64 rows whose k
-// is a multiple of 256.
+// is a multiple of 256, where the launch has workgroups enough (f16w_takes_wide).
 //
 // What bounds it: the matrix cores, if everything beside them stays out of their way.  gemm_f16w.hip's waves hold two 16-row fragments, so every B'
 // fragment read from LDS feeds two products: 8 waves read 64 KB per 32 slots of k, the 512 cycles that their products take.  Here

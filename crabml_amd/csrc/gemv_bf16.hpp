@@ -441,7 +441,7 @@ __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) { return
 // HALF (up to eight rows): a workgroup owns 8 weight rows, where 16 would leave half of the CUs without one (a CU draws some 25 KB/us, however much it asks
 // for).  A step is the next two pieces of k that the wave would take of 16 rows, their eight weight rows one above the other in the tile, and each is
 // multiplied by its piece of the rhs in turn (the lower and the upper half of the product are the same).  Us a launch, 4
-// rows, streams behind it: 2048 x 8192 11.3 -> 8.5, 2048 x 2048 with a tail 6.3 -> 5.6.  (16 rows, whose rhs is as many bytes as the weights of 16 rows: 2048 x
+// rows, streams behind it: 2048 x 8192 11.3 -> 8.5, 2048 x 2048 with a tail 6.3 -> 5.4.  (16 rows, whose rhs is as many bytes as the weights of 16 rows: 2048 x
 // 8192 12.2 -> 11.7, 2048 x 4096 6.2 -> 6.8; twice as many pieces of square sums to read cost the linears behind them more.)
 // The sums of bf16 rows are the same in every form: pieces of k by wave, waves in order, square sums of 16 columns: a sequence's logits do not
 // depend on how many others, three to sixteen rows in all, share its step.
