@@ -1212,7 +1212,7 @@ int allreduce(crabml_hip_llama* c, int seg) {
 // Workgroups of the one launch wait for each other and take a CU each (118 VGPRs, 16 waves): what the contexts of a process hold together stays within half
 // of a device's CUs, so that these launches never wait for each other's CUs, however many streams run.  A context past that (of 256 CUs four contexts of 27
 // workgroups, the 15M model's, are within), and for as long as it lives, keeps its launches per layer: the same bits.  Launches of other contexts whose
-// workgroups wait as well, and other processes, are not counted: where they and this one hold CUs that the other needs, the call takes 0.4 s longer, once
+// workgroups wait as well, and other processes, are not counted: where they and this one hold CUs that the other needs, the call takes 0.2 s longer, once
 // (small_recover).
 std::atomic<int>& small_reserved(int ordinal) {
   static std::atomic<int> held[64];

@@ -16,8 +16,8 @@
 // a row (small_fits).  The arithmetic is that of the five launches, term by term and in their order: k_qkv, k_attn_short, k_gemv_res_nq<DEFER>,
 // k_gateup_q<DEFER>; the last ffn_down normalizes exactly, as there.  All bits are theirs.
 // A granule buffer is written once a layer.  Whoever writes it again has, through the chain of gathers, waited for everything that its readers made of
-// it, so one copy of each is enough.  Polls are bounded -- at a quarter of what the other launches of the step wait for each other, so that where the two
-// kinds hold CUs that the other needs it is this one that leaves -- and raise the context's fault word, and a raised word ends the others'
+// it, so one copy of each is enough.  Polls are bounded -- at half of the other launches' number and without their sleeps between, so that where the two
+// kinds hold CUs that the other needs it is this one that leaves, after 0.2 s -- and raise the context's fault word, and a raised word ends the others'
 // waits.  The host then runs the call again in launches per layer and stays with them (small_give_up).
 #pragma once
 
@@ -25,7 +25,7 @@ namespace crabml_hip {
 
 #define SMALL_WGS 32
 #define SMALL_LAYERS 64
-#define SMALL_POLLS (1 << 19)  // some 0.4 s
+#define SMALL_POLLS (1 << 20)  // 0.17 us each
 #define SMALL_FAULT 3
 
 struct SmallLayer {

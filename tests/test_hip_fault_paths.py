@@ -50,3 +50,39 @@ def test_lost_co_residency_raises_instead_of_hanging(flags, name):
         pytest.skip("the runtime did not confine the process (CU mask not honoured): the condition cannot be produced here")
     assert "FAULT" in out and "timed out" in out, out
     assert "USABLE" in out, out
+
+
+SMALL = r"""
+import sys, time
+sys.path.insert(0, %r)
+import numpy as np
+import crabml_amd as ca
+from crabml_amd import synth
+shape = synth.ModelShape("small", 288, 768, 6, 6, 6, 300, 64, 1e-5, None)
+dev = ca.HipTensorDevice(0)
+conf, w = synth.to_hip(synth.build_model(shape, synth.Q8_0, seed=6), dev)
+five = ca.HipLlamaRunner(conf, w, dev, 64, True, extra_flags=134217728)
+ids = five.decode_greedy(3, 20)
+one = ca.HipLlamaRunner(conf, w, dev, 64, True)
+print("WORKGROUPS", one.debug_small_layers(), flush=True)
+t0 = time.time()
+got = one.decode_greedy(3, 20)
+print("SECONDS %%.3f" %% (time.time() - t0), "NOW", one.debug_small_layers(), "SAME" if got == ids else "DIFFERENT", flush=True)
+t0 = time.time()
+x, y = one.forward(ids[-1], 20), five.forward(ids[-1], 20)
+print("AGAIN %%.2f" %% (time.time() - t0), "SAME" if np.array_equal(x.view(np.uint32), y.view(np.uint32)) else "DIFFERENT", flush=True)
+""" % ROOT
+
+
+def test_a_small_models_launch_without_room_is_made_again_in_launches_per_layer():
+    """27 workgroups of a CU each on 16 CUs: the ones that are there wait for the others until their polls run out; the same tokens within seconds, and launches per
+    layer from then on"""
+    env = dict(os.environ, HSA_CU_MASK="0:0-15", CRABML_HIP_TEST_HOOKS="1", CRABML_HIP_ASSUME_CUS="256")
+    p = subprocess.run([sys.executable, "-c", SMALL], env=env, capture_output=True, text=True, timeout=100)
+    assert p.returncode == 0, (p.stdout[-2000:], p.stderr[-2000:])
+    print(p.stdout)
+    assert "WORKGROUPS 27" in p.stdout and p.stdout.count("SAME") == 2 and "DIFFERENT" not in p.stdout, p.stdout
+    if "NOW 27" in p.stdout:
+        pytest.skip("the runtime did not confine the process (CU mask not honoured): the condition cannot be produced here")
+    assert "NOW 0" in p.stdout, p.stdout
+    assert float(p.stdout.split("SECONDS ")[1].split()[0]) < 5 and float(p.stdout.split("AGAIN ")[1].split()[0]) < 1, p.stdout

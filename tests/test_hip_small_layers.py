@@ -100,7 +100,7 @@ def test_contexts_past_the_reserved_workgroups(ca):
 
 @pytest.mark.parametrize("graph", [True, False])
 def test_workgroups_that_do_not_meet(ca, monkeypatch, graph):
-    """one poll instead of half a million: no gather is met.  The call that finds out is made again in launches per layer, and the context stays with them; steps
+    """one poll instead of a million: no gather is met.  The call that finds out is made again in launches per layer, and the context stays with them; steps
     that nobody has looked at cannot be made again: an error, once"""
     shape = synth.ModelShape("small", 288, 768, 3, 6, 6, 300, 160, 1e-5, None)
     model = synth.build_model(shape, synth.Q8_0, seed=33)
