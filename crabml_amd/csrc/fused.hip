@@ -136,6 +136,7 @@ struct crabml_hip_llama {
   int small_wgs = 0;                         // ... and workgroups, as reserved (small_reserve; 0: launches per layer)
   int small_polls = SMALL_POLLS;
   bool small_unseen = false;  // steps in one launch each whose fault word nobody has looked at
+  bool small_lost = false;    // such a step was lost: the cache holds rows that are none, until it is reset
   unsigned long long* a8gran = nullptr;  // Q4_K layers: granules of the attention output (dim_l) and of h (hidden_l), through which
   unsigned long long* h8gran = nullptr;  // the producing kernels assemble Q8_K super-blocks (q8k_exchange_store)
   bool q8k_producers = false;            // attention / gate-up emit the Q8_K planes of wo's / ffn_down's rhs themselves
@@ -1895,6 +1896,11 @@ int set_state(crabml_hip_llama* c, size_t token, size_t pos, int step, const uns
   return 0;
 }
 
+int check_cache(crabml_hip_llama* c) {
+  if (c->small_lost)
+    CH_BAIL(c->dev, CRABML_HIP_UNEXPECTED, "llama: an earlier step of this context was lost (the workgroups of its one launch did not meet: timed out); its cached rows are not to be used, reset it");
+  return 0;
+}
 // behind a call's steps: waits for them, and what the context's fault word says then
 int read_fault(crabml_hip_llama* c, int* fault) {
   CH_HIP(c->dev, hipMemcpyAsync(fault, c->state + 5, sizeof(int), hipMemcpyDeviceToHost, c->dev->stream));
@@ -1909,8 +1915,8 @@ int finish_call(crabml_hip_llama* c, const Finish& finish, const Again& again) {
   if (fault == SMALL_FAULT) {
     bool repeat = false;
     CH_TRY(small_recover(c, &repeat));
-    if (!repeat)
-      CH_BAIL(dev, CRABML_HIP_UNEXPECTED, "llama: an earlier step of this context was lost (the workgroups of its one launch did not meet: timed out); its cached rows are not to be used");
+    c->small_lost = !repeat;
+    CH_TRY(check_cache(c));
     CH_TRY(again());
     fault = 0;
     CH_TRY(finish(&fault));
@@ -2628,7 +2634,7 @@ static int check_step(crabml_hip_llama* c, size_t token, size_t pos) {
   if (token >= c->cfg.vocab_size) CH_BAIL(dev, CRABML_HIP_BAD_INPUT, "llama: token %zu out of range", token);
   if (pos != c->kv_len) CH_BAIL(dev, CRABML_HIP_BAD_INPUT, "llama: pos %zu != kv cache length %zu", pos, c->kv_len);
   if (pos >= c->cfg.seq_len) CH_BAIL(dev, CRABML_HIP_TENSOR_ERROR, "llama: kv cache is full (%zu)", c->cfg.seq_len);
-  return 0;
+  return check_cache(c);
 }
 
 int crabml_hip_llama_forward(crabml_hip_llama_t* c, size_t token, size_t pos, float* logits) {
@@ -2670,6 +2676,7 @@ int crabml_hip_llama_decode_greedy(crabml_hip_llama_t* c, size_t token, size_t n
   if (c->kv_len + n_steps > c->cfg.seq_len || n_steps > (size_t)c->out_cap)
     CH_BAIL(dev, CRABML_HIP_TENSOR_ERROR, "llama: %zu steps do not fit the kv cache (%zu of %zu used)", n_steps, c->kv_len, c->cfg.seq_len);
   if (n_steps == 0) return 0;
+  CH_TRY(check_cache(c));
   CH_TRY(set_state(c, token, c->kv_len, 0));
   const size_t pos = c->kv_len;
   CH_TRY(run_steps(c, pos, n_steps));
@@ -2697,6 +2704,7 @@ int crabml_hip_llama_prefill(crabml_hip_llama_t* c, const uint32_t* tokens, size
     if (tokens[i] >= c->cfg.vocab_size) CH_BAIL(dev, CRABML_HIP_BAD_INPUT, "llama: token %u out of range", tokens[i]);
   if (c->kv_len + n > c->cfg.seq_len)
     CH_BAIL(dev, CRABML_HIP_TENSOR_ERROR, "llama: %zu prompt tokens do not fit the kv cache (%zu of %zu used)", n, c->kv_len, c->cfg.seq_len);
+  CH_TRY(check_cache(c));
   if (c->tp > 1) {  // token loop
     for (size_t i = 0; i < n; i++) CH_TRY(crabml_hip_llama_forward(c, tokens[i], c->kv_len, i + 1 == n ? logits : nullptr));
     return 0;
@@ -2714,7 +2722,19 @@ int crabml_hip_llama_prefill(crabml_hip_llama_t* c, const uint32_t* tokens, size
   }
   if (logits) {
     CH_HIP(dev, hipMemcpyAsync(logits, c->logits, c->cfg.vocab_size * 4, hipMemcpyDeviceToHost, dev->stream));
-    CH_HIP(dev, hipStreamSynchronize(dev->stream));
+    if (c->small_unseen) {  // (steps in front of the prompt: their rows are in these logits)
+      int fault = 0;
+      CH_TRY(read_fault(c, &fault));
+      if (fault == SMALL_FAULT) {
+        bool again;
+        CH_TRY(small_recover(c, &again));
+        c->small_lost = true;
+        return check_cache(c);
+      }
+      c->small_unseen = false;
+    } else {
+      CH_HIP(dev, hipStreamSynchronize(dev->stream));
+    }
   }
   return 0;
 }
@@ -2775,7 +2795,7 @@ size_t crabml_hip_llama_kv_len(const crabml_hip_llama_t* c) { return c ? c->kv_l
 int crabml_hip_llama_reset(crabml_hip_llama_t* c) {
   if (!c) return CRABML_HIP_BAD_INPUT;
   c->kv_len = 0;
-  c->small_unseen = false;
+  c->small_unseen = c->small_lost = false;
   if (c->flash_tick) {  // a step that faulted half-way may have left arrivals behind
     CH_USE(c->dev);
     CH_FLUSH(c->dev);

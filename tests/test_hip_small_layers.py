@@ -101,7 +101,7 @@ def test_contexts_past_the_reserved_workgroups(ca):
 @pytest.mark.parametrize("graph", [True, False])
 def test_workgroups_that_do_not_meet(ca, monkeypatch, graph):
     """one poll instead of a million: no gather is met.  The call that finds out is made again in launches per layer, and the context stays with them; steps
-    that nobody has looked at cannot be made again: an error, once"""
+    that nobody has looked at cannot be made again: an error until the context is reset"""
     shape = synth.ModelShape("small", 288, 768, 3, 6, 6, 300, 160, 1e-5, None)
     model = synth.build_model(shape, synth.Q8_0, seed=33)
     dev = ca.HipTensorDevice(0)
@@ -111,8 +111,8 @@ def test_workgroups_that_do_not_meet(ca, monkeypatch, graph):
     logits = five.forward(ids[-1], 40).view(np.uint32)
     monkeypatch.setenv("CRABML_HIP_TEST_HOOKS", "1")
     monkeypatch.setenv("CRABML_HIP_SMALL_POLLS", "1")
-    by_steps, by_run, unseen = (ca.HipLlamaRunner(conf, w, dev, 100, True, graph) for _ in range(3))
-    assert by_steps.debug_small_layers() == by_run.debug_small_layers() == unseen.debug_small_layers() == 27
+    by_steps, by_run, unseen, prompt = (ca.HipLlamaRunner(conf, w, dev, 100, True, graph) for _ in range(4))
+    assert [r.debug_small_layers() for r in (by_steps, by_run, unseen, prompt)] == [27] * 4
     token = 3
     for pos in range(40):
         x = by_steps.forward(token, pos)
@@ -121,11 +121,15 @@ def test_workgroups_that_do_not_meet(ca, monkeypatch, graph):
     assert np.array_equal(by_steps.forward(ids[-1], 40).view(np.uint32), logits)
     assert by_run.decode_greedy(3, 40) == ids and np.array_equal(by_run.forward(ids[-1], 40).view(np.uint32), logits)
     unseen.forward_async(3, 0)
-    with pytest.raises(ca.CrabmlError, match="not to be used"):
-        unseen.forward(ids[0], 1)
+    for call in (lambda: unseen.forward(ids[0], 1), lambda: unseen.forward(ids[0], 2), lambda: unseen.decode_greedy(ids[0], 2), lambda: unseen.prefill([1, 2])):
+        with pytest.raises(ca.CrabmlError, match="not to be used"):
+            call()
     unseen.reset()
     assert unseen.decode_greedy(3, 40) == ids
-    assert by_steps.debug_small_layers() == by_run.debug_small_layers() == unseen.debug_small_layers() == 0
+    prompt.forward_async(3, 0)
+    with pytest.raises(ca.CrabmlError, match="not to be used"):
+        prompt.prefill([1, 2, 3])
+    assert [r.debug_small_layers() for r in (by_steps, by_run, unseen, prompt)] == [0] * 4
     # what they had reserved is there again
     monkeypatch.delenv("CRABML_HIP_SMALL_POLLS")
     more = [ca.HipLlamaRunner(conf, w, dev, 100, True, graph) for _ in range(4)]
