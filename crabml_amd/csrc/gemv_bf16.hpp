@@ -125,6 +125,9 @@ struct GemvBf16 {
   bool resident = false;  // the weights of all linears that run in turn fit a cache: they are read so that they stay in it (else nontemporal)
   StreamMix sm;                 // STREAMS: out = stream 0, u[b][ldo] = what the next linear reads
   float* u = nullptr;
+  // a k shared by two workgroups of the batched linear: their sums as {value, launch} granules [tiles][2][256], and arrivals [tiles][4], two a launch, zero at first
+  unsigned long long* half = nullptr;
+  unsigned* meet = nullptr;
 };
 
 __device__ __forceinline__ float act_sigmoid(float z) { return 1.0f / (1.0f + __expf(-z)); }
@@ -162,12 +165,20 @@ __device__ __forceinline__ float gelu_tanh(float z) {
 }
 __device__ __forceinline__ float soft_cap(float z, float cap) { return cap > 0.0f ? cap * tanhf(z / cap) : z; }
 
-__device__ __forceinline__ float gemv_residual(const GemvBf16& a, int row, int b, float v) {
-  float* o = a.out + (size_t)b * a.ldo + row;
-  float s = *o + v;
-  if (a.add_rows) s += a.add_rows[(size_t)b * a.ld_add + row];
-  if (a.add_vec) s += a.add_vec[row];
-  *o = s;
+// GEMV_OUT_RESIDUAL: what the thread that will have (row, b) needs, requested ahead of the products
+struct ResidualElem {
+  float old = 0.f, rows = 0.f, vec = 0.f;
+};
+__device__ __forceinline__ void residual_load(const GemvBf16& a, int row, int b, ResidualElem& e) {
+  e.old = a.out[(size_t)b * a.ldo + row];
+  if (a.add_rows) e.rows = a.add_rows[(size_t)b * a.ld_add + row];
+  if (a.add_vec) e.vec = a.add_vec[row];
+}
+__device__ __forceinline__ float residual_out(const GemvBf16& a, int row, int b, const ResidualElem& e, float v) {
+  float s = e.old + v;
+  if (a.add_rows) s += e.rows;
+  if (a.add_vec) s += e.vec;
+  a.out[(size_t)b * a.ldo + row] = s;
   return s;
 }
 template <int OUT>
@@ -175,7 +186,6 @@ __device__ __forceinline__ void gemv_out(const GemvBf16& a, int row, int b, floa
   float* o = a.out + (size_t)b * a.ldo + row;
   if constexpr (OUT == GEMV_OUT_STORE) *o = v;
   if constexpr (OUT == GEMV_OUT_ACT) *o = act_ranges(a.bias ? v + a.bias[row] : v, row, a.act);
-  if constexpr (OUT == GEMV_OUT_RESIDUAL) (void)gemv_residual(a, row, b, v);
   if constexpr (OUT == GEMV_OUT_XIELU) *o = xielu_apply(v, a.xielu[0], a.xielu[1]);
   if constexpr (OUT == GEMV_OUT_SOFTCAP) *o = soft_cap(v, a.cap);
 }
@@ -197,13 +207,14 @@ __device__ __forceinline__ void stream_elem_out(const GemvBf16& a, int row, int 
 // columns of a piece of a row's square sum: a workgroup of the batched linears below owns as many at least
 __host__ __device__ inline int ss_columns(int rows) { return rows <= 8 ? 8 : 16; }
 // v of 8 or 16 neighbouring columns in as many lanes (zero outside the matrix): what the next linear reads, and its square sum.  Without out16: as f32.
-__device__ __forceinline__ void rows16_out(const GemvBf16& a, int row, int b, float v) {
+// gain: gain_out[row] (1 without)
+__device__ __forceinline__ void rows16_out(const GemvBf16& a, int row, int b, float v, float gain) {
   const bool in = b < a.nb && row < a.N;
   if (!a.out16) {
     if (in) a.u[(size_t)b * a.ldo + row] = v;
     return;
   }
-  if (in) a.out16[(size_t)b * a.ldo + row] = f2bf(a.gain_out ? v * a.gain_out[row] : v);
+  if (in) a.out16[(size_t)b * a.ldo + row] = f2bf(a.gain_out ? v * gain : v);
   float s = group_sum<8>(v * v);
   if (a.nb <= 8) {  // (ss_columns)
     if (in && (row & 7) == 0) a.ss_out[(size_t)b * a.ld_ss_out + (row >> 3)] = s;
@@ -242,7 +253,9 @@ __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
   for (int u = 0; u < UN; u++) request(u, 0);
   StreamElem elem;  // of lane r NB + b
   const int my_row = row0 + lane / NB, my_b = b0 + lane % NB;
-  const bool mine = OUT == GEMV_OUT_STREAMS && lane < R * NB && my_row < a.N && my_b < a.nb;
+  const bool mine = (OUT == GEMV_OUT_STREAMS || OUT == GEMV_OUT_RESIDUAL) && lane < R * NB && my_row < a.N && my_b < a.nb;
+  ResidualElem res;
+  if constexpr (OUT == GEMV_OUT_RESIDUAL) residual_load(a, my_row < a.N ? my_row : a.N - 1, my_b < a.nb ? my_b : a.nb - 1, res);  // (no branch on the lane)
   if constexpr (OUT == GEMV_OUT_STREAMS) {
     static_assert(R * NB <= 64, "a lane per result");
     if (mine) stream_elem_load(a, my_row, my_b, elem);
@@ -376,7 +389,7 @@ __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
       }
     return;
   }
-  if constexpr (OUT == GEMV_OUT_STREAMS) {
+  if constexpr (OUT == GEMV_OUT_STREAMS || OUT == GEMV_OUT_RESIDUAL) {
     float y = 0.f;
 #pragma unroll
     for (int r = 0; r < R; r++)
@@ -385,7 +398,11 @@ __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
         const float v = wave_sum_f32(acc[r][b]) * scale[b];
         y = lane == r * NB + b ? v : y;
       }
-    if (mine) stream_elem_out(a, my_row, my_b, elem, y);
+    if constexpr (OUT == GEMV_OUT_STREAMS) {
+      if (mine) stream_elem_out(a, my_row, my_b, elem, y);
+    } else {
+      if (mine) (void)residual_out(a, my_row, my_b, res, y);
+    }
     return;
   }
 #pragma unroll
@@ -443,9 +460,12 @@ __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) { return
 // multiplied by its piece of the rhs in turn (the lower and the upper half of the product are the same).  Us a launch, 4
 // rows, streams behind it: 2048 x 8192 11.3 -> 8.5, 2048 x 2048 with a tail 6.3 -> 5.4.  (16 rows, whose rhs is as many bytes as the weights of 16 rows: 2048 x
 // 8192 12.2 -> 11.7, 2048 x 4096 6.2 -> 6.8; twice as many pieces of square sums to read cost the linears behind them more.)
-// The sums of bf16 rows are the same in every form: pieces of k by wave, waves in order, square sums of 16 columns: a sequence's logits do not
-// depend on how many others, three to sixteen rows in all, share its step.
-template <int RT, int SPL, int W, int D, int IN, int OUT, bool NTW, int XG = 4, bool HALF = false>
+// KS = 2 (nine rows and more, the same matrices from GEMV16_SHARED_K columns on): two workgroups of eight waves share a tile's k, each with the pieces that eight of the sixteen
+// waves would take, and meet at the end (below): 16 rows, residual behind it, 2048 x 8192 12.0 -> 9.0 us, 2048 x 4096 7.4 -> 6.4, 1280 x 4096 7.1 -> 6.0; 2048 x 2048 5.0 -> 5.1.
+// The sums of bf16 rows are the same in every form: pieces of k by wave, waves in order (from GEMV16_SHARED_K columns on those of narrow matrices in two halves), square
+// sums of 16 columns: a sequence's logits do not depend on how many others, three to sixteen rows in all, share its step.
+#define GEMV16_SHARED_K 3072
+template <int RT, int SPL, int W, int D, int IN, int OUT, bool NTW, int XG = 4, bool HALF = false, int KS = 1>
 __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
   constexpr int LD = 20, NT = 64 * W;
   constexpr bool XB = IN == GEMV_IN_BF16 || IN == GEMV_IN_BF16_RMS || IN == GEMV_IN_BF16_SPLIT, NORM = IN == GEMV_IN_RMS || IN == GEMV_IN_RMSV;
@@ -461,8 +481,12 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
   };
   __shared__ __attribute__((aligned(16))) Lds lds;
   __shared__ float sums[W][16], scale[16];
+  static_assert(KS == 1 || (KS == 2 && RT == 1 && !HALF && XB && W >= 4), "two workgroups a tile: one of 16 weight rows, bf16 rows");
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_wg(), fr = lane & 15, fk = lane >> 4;
-  const int row0 = blockIdx.x * WR;
+  // (KS = 2: the two of a tile are eight workgroups apart, on one XCD: what was touched there for the tile's rows serves both)
+  const int tile = KS == 2 ? (blockIdx.x >> 4) * 8 + (blockIdx.x & 7) : blockIdx.x, part = KS == 2 ? (blockIdx.x >> 3) & 1 : 0;
+  if (KS == 2 && tile * WR >= a.N) return;
+  const int row0 = tile * WR, kw = part * W + wave;  // kw: this wave's place among those of k
   // where this lane's part of a request lies: 16 bytes, eight lanes a row (f32: sixteen)
   const int r8 = lane >> 3, c8 = lane & 7, r16 = lane >> 4, c16 = lane & 15;
   // (32-bit offsets from a scalar base)
@@ -483,7 +507,7 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
   i32x4 wv[D][RT][2], xv[D][KP * XR];
   f32x4 gv[D];
   const int n = a.K / 64, last = n - 1;
-  constexpr int S = KP * W;  // pieces from a step of this wave's to its next
+  constexpr int S = KP * W * KS;  // pieces from a step of this wave's to its next
   auto request = [&](int d, int i) {
     const char *w = wb + i * 128, *x = xbase + i * (XB ? 128 : 256);
     const int second = HALF && i + W < n ? 128 * W : 0;  // (none: itself again, not used)
@@ -515,10 +539,18 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
       tail[j] = t_ss[j][c16 < a.n_ss ? c16 : 0];
     }
   }
-  if (wave < n) {
+  unsigned launch = 0;
+  if constexpr (KS == 2) launch = __hip_atomic_load(a.meet + tile * 4 + (wave & 3), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (kw < n) {
 #pragma unroll
-    for (int d = 0; d < D; d++) request(d, wave + d * S < n ? wave + d * S : last);  // (clamped: no branch between the requests)
+    for (int d = 0; d < D; d++) request(d, kw + d * S < n ? kw + d * S : last);  // (clamped: no branch between the requests)
   }
+  float out_c[2] = {0.f, 0.f};  // (asked for here: behind the products they would be one more round trip of every workgroup)
+  if constexpr (OUT == GEMV_OUT_XIELU) {
+    out_c[0] = a.xielu[0];
+    out_c[1] = a.xielu[1];
+  }
+  const float gain1 = PIECES && !TAIL && a.gain ? *a.gain : 1.0f;
   constexpr int RB = HALF ? 3 : 4, ELEMS = (WR * 16 + NT - 1) / NT;
   // result j of the tile: weight row t 16 + r of the workgroup, row b of the rhs
   auto of = [&](int j, int& t, int& b, int& r) {
@@ -527,6 +559,18 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
     r = j & ((1 << RB) - 1);
   };
   StreamElem elem[ELEMS];  // of this thread's results: element tid + NT i of the tile
+  ResidualElem res[ELEMS];
+  float gain_next[ELEMS];
+  if constexpr (OUT == GEMV_OUT_RESIDUAL || OUT == GEMV_OUT_STREAMS) {
+#pragma unroll
+    for (int i = 0; i < ELEMS; i++) {
+      int t, b, r;
+      of(tid + i * NT < WR * 16 ? tid + i * NT : 0, t, b, r);
+      const int row = row0 + t * 16 + r < a.N ? row0 + t * 16 + r : a.N - 1;
+      gain_next[i] = a.gain_out ? a.gain_out[row] : 1.f;
+      if constexpr (OUT == GEMV_OUT_RESIDUAL) residual_load(a, row, b < a.nb ? b : a.nb - 1, res[i]);
+    }
+  }
   if constexpr (OUT == GEMV_OUT_STREAMS) {
 #pragma unroll
     for (int i = 0; i < ELEMS; i++) {
@@ -631,7 +675,7 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
     }
     wave_lds_order();
   };
-  for (int i = wave; i < n; i += D * S) {
+  for (int i = kw; i < n; i += D * S) {
     if (i + D * S < n) {
 #pragma unroll
       for (int d = 0; d < D; d++) {
@@ -673,7 +717,7 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
     t = group_sum<8>(t);
     if constexpr (QL >= 16) t += dpp_f<0x140>(t);
     if constexpr (QL == 32) t += __shfl_xor(t, 16, 64);
-    if (q_at == 0 && q_row < 16) scale[q_row] = (!TAIL && a.gain ? *a.gain : 1.0f) / sqrtf(t / (float)a.mean_n + a.eps);
+    if (q_at == 0 && q_row < 16) scale[q_row] = gain1 / sqrtf(t / (float)a.mean_n + a.eps);
   }
   __syncthreads();  // (the tiles of results take the place of the operands')
   if constexpr (TAIL) {
@@ -695,10 +739,58 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
   }
   auto met = [&](int t, int b, int r) {  // the waves' sums
     float v = 0.f;
+    if constexpr (HALF) {
+      float v2 = 0.f;
+#pragma unroll
+      for (int w = 0; w < W / 2; w++) v += lds.tile[w][t][b * LD + r];
+      if (a.K < GEMV16_SHARED_K) v2 = v;
+#pragma unroll
+      for (int w = W / 2; w < W; w++) v2 += lds.tile[w][t][b * LD + r];
+      return a.K < GEMV16_SHARED_K ? v2 : v + v2;
+    }
 #pragma unroll
     for (int w = 0; w < W; w++) v += lds.tile[w][t][b * LD + r];
     return v;
   };
+  float both = 0.f;
+  if constexpr (KS == 2) {
+    // A wave's 64 results leave as {value, launch} granules before it counts itself in; of the two workgroups' waves the later one takes the other's,
+    // which are on their way or there -- it waits for stores that have been issued, never for a workgroup -- and goes on alone.
+    if (wave >= 4) return;
+    int t, b, r;
+    of(tid, t, b, r);
+    const float v = met(t, b, r);
+    const unsigned tag = (launch >> 1) + 1u;  // (two arrivals a launch: both workgroups see the same half, whether the other one has come or not)
+    unsigned long long* g = a.half + (size_t)tile * 512 + tid;
+    __hip_atomic_store(g + part * 256, ((unsigned long long)tag << 32) | __builtin_bit_cast(unsigned, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    unsigned n_before = 0;
+    if (lane == 0) n_before = __hip_atomic_fetch_add(a.meet + tile * 4 + wave, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if ((__builtin_amdgcn_readfirstlane(n_before) & 1u) == 0) return;
+    unsigned long long o;
+    do {
+      o = __hip_atomic_load(g + (part ^ 1) * 256, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } while ((unsigned)(o >> 32) != tag);
+    const float ov = __builtin_bit_cast(float, (unsigned)o);
+    both = v + ov;  // (the same whichever is later)
+  }
+  if constexpr (OUT == GEMV_OUT_GLU && KS == 2) {
+    int t, b, r;
+    of(tid, t, b, r);
+    const int row = row0 + r;
+    float up = dpp_f<0xB1>(both), gate = both;  // (of the neighbour)
+    if constexpr (IN == GEMV_IN_BF16_RMS) {
+      gate *= scale[b];
+      up *= scale[b];
+    }
+    if ((r & 1) == 0 && b < a.nb && row < a.N) {
+      const size_t o = (size_t)b * a.ldo + row / 2;
+      if (a.out16)
+        a.out16[o] = f2bf(gelu_tanh(gate) * up);
+      else
+        a.out[o] = gelu_tanh(gate) * up;
+    }
+    return;
+  }
   if constexpr (OUT == GEMV_OUT_GLU) {
     for (int i = tid; i < WR * 8; i += NT) {
       int t, b, r;
@@ -728,43 +820,48 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
       of(j, t, b, r);
       const int row = row0 + t * 16 + r;
       float u = 0.f;
-      if (b < a.nb && row < a.N) u = stream_elem_mix(a, row, b, elem[i], met(t, b, r));
-      rows16_out(a, row, b, u);
+      if (b < a.nb && row < a.N) u = stream_elem_mix(a, row, b, elem[i], KS == 2 ? both : met(t, b, r));
+      rows16_out(a, row, b, u, gain_next[i]);
     }
     return;
   }
-  for (int i = tid; i < WR * 16; i += NT) {
+#pragma unroll
+  for (int i = 0; i < ELEMS; i++) {
+    const int j = tid + i * NT;
+    if (j >= WR * 16) break;  // (whole waves)
     int t, b, r;
-    of(i, t, b, r);
+    of(j, t, b, r);
     const int row = row0 + t * 16 + r;
-    float v = met(t, b, r);
+    float v = KS == 2 ? both : met(t, b, r);
     if constexpr (NORM || IN == GEMV_IN_BF16_RMS) v *= scale[b];
     if constexpr (OUT == GEMV_OUT_RESIDUAL) {
       float x = 0.f;
-      if (b < a.nb && row < a.N) x = gemv_residual(a, row, b, v);
-      if (a.out16) rows16_out(a, row, b, x);
+      if (b < a.nb && row < a.N) x = residual_out(a, row, b, res[i], v);
+      if (a.out16) rows16_out(a, row, b, x, gain_next[i]);
       continue;
     }
     if (b < a.nb && row < a.N) {
       if constexpr (OUT == GEMV_OUT_XIELU) {
-        if (a.out16) {
-          a.out16[(size_t)b * a.ldo + row] = f2bf(xielu_apply(v, a.xielu[0], a.xielu[1]));
-          continue;
-        }
+        const float y = xielu_apply(v, out_c[0], out_c[1]);
+        if (a.out16)
+          a.out16[(size_t)b * a.ldo + row] = f2bf(y);
+        else
+          a.out[(size_t)b * a.ldo + row] = y;
+        continue;
       }
       gemv_out<OUT>(a, row, b, v);
     }
   }
 }
 
-// 32 rows a workgroup where that still fills the chip, else 16; sixteen waves where 16 rows leave CUs without a workgroup and k is long
-// enough for each of them to have a few steps.  One piece of the rhs: bf16 rows, but for a classifier behind a prompt pass.
+// f32 rows, and linears of bf16 rows into the residual: 32 rows a workgroup where that still fills the chip, else 16; sixteen waves where 16 rows leave CUs without
+// a workgroup and k is long enough for each of them to have a few steps.  One piece of the rhs: bf16 rows, but for a classifier behind a prompt pass.
 // Three pieces of more than eight f32 rows: two steps of requests hold 140 registers a thread, one workgroup a CU; where there are more workgroups than
 // CUs, two of them with one step out each are faster (us, 12 rows: 11264 x 2048 18.0 -> 16.4, 8192 x 1024 8.7 -> 6.9), elsewhere they are
 // not (2048 x 8192, 128 workgroups: 16.2 -> 19.8).
-template <int RT, int SPL, int W, int IN, int OUT, bool NTW>
+template <int RT, int SPL, int W, int IN, int OUT, bool NTW, int D0 = 0>
 inline void launch_gemv16_t(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a, int n_cu) {
-  constexpr int D = IN < GEMV_IN_BF16 || RT == 2 ? 2 : OUT == GEMV_OUT_STREAMS ? 3 : 4;  // (registers: sixteen waves a CU)
+  constexpr int D = D0 ? D0 : IN < GEMV_IN_BF16 || RT == 2 ? 2 : OUT == GEMV_OUT_STREAMS ? 3 : 4;  // (registers: sixteen waves a CU)
   const dim3 grid((a.N + 16 * RT - 1) / (16 * RT));
   if constexpr (IN >= GEMV_IN_BF16) {
     if (a.nb <= 8) {
@@ -790,12 +887,46 @@ inline void launch_gemv16_t(hipStream_t st, crabml_hip_device::ProfRec* rec, con
 }
 // bf16: of the rhs
 inline bool gemv16_deep(int N, int K, int n_cu) { return (N + 15) / 16 < n_cu && K >= 2048; }
+inline bool gemv16_narrow(int N, int K, int n_cu) { return gemv16_deep(N, K, n_cu) && (N + 15) / 16 * 2 <= n_cu; }
 inline int gemv16_rows(bool bf16, int N, int K, int nb, int n_cu) {
   if (N >= 16384) return 32;
-  return bf16 && nb <= 8 && gemv16_deep(N, K, n_cu) && (N + 15) / 16 * 2 <= n_cu ? 8 : 16;
+  return bf16 && nb <= 8 && gemv16_narrow(N, K, n_cu) ? 8 : 16;
+}
+// what k shared by two workgroups needs (GemvBf16::half, meet)
+inline size_t gemv16_half_bytes(int n_cu) { return (size_t)(n_cu / 2) * 512 * sizeof(unsigned long long); }
+inline size_t gemv16_meet_bytes(int n_cu) { return (size_t)(n_cu / 2) * 4 * sizeof(unsigned); }
+// More rows of weights than 16 a CU, bf16 rows with a norm: as many tiles of 16 a workgroup as make one round of workgroups.  The rhs comes through the L2s once a
+// workgroup, as many bytes as 16 rows of weights, and a second round that leaves most CUs without work costs as much as the first.  Us a launch of 16 / 4 rows,
+// workgroups of 16 rows / these: 4608 x 512 5.5 / 4.2 and 4.9 / 3.9, 11264 x 512 7.7 / 4.9 and 6.9 / 4.7, 8192 x 1024 6.95 / 5.6 and 6.1 / 5.4, 12288 x 1024 9.4 / 6.8 and
+// 8.25 / 6.5, 4608 x 2048 8.4 / 7.2 and 6.7 / 6.4, 8192 x 2048 9.2 / 8.65 and 7.8 / 7.8, 9216 x 2048 11.4 / 9.6 and 9.65 / 9.1, 11264 x 2048 12.1 / 10.4 and 10.3 / 10.3,
+// 14336 x 2048 14.8 / 13.3 and 12.8 / 12.9.  Sixteen waves where each has two pieces of k, else eight that start sooner (9216 x 1024 6.35 / 6.2).  More than four
+// tiles a CU: two workgroups of 48 rows on each in turn (against 32 rows: 32000 x 512 11.2 / 9.1, x 1024 14.5 / 13.5, x 2048 24.9 / 24.0, x 4096 48.5 / 44.0).
+// From 4096 columns on eight rows and fewer are as fast or faster in workgroups of 16 (8192 x 4096 12.6 / 15.2).
+template <int SPL, int IN, int OUT, bool NTW>
+inline bool launch_gemv16_round(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a, int n_cu) {
+  const int tiles = (a.N + 15) / 16, per = (tiles + n_cu - 1) / n_cu;
+  if (per > 4) {
+    launch_gemv16_t<3, SPL, 8, IN, OUT, NTW, 1>(st, rec, a, n_cu);
+    return true;
+  }
+  if (per < 2 || a.K >= 4096) return false;
+  if (per == 2 && a.K <= 1024)
+    launch_gemv16_t<2, SPL, 16, IN, OUT, NTW, 1>(st, rec, a, n_cu);
+  else if (per == 2)
+    launch_gemv16_t<2, SPL, 16, IN, OUT, NTW, 2>(st, rec, a, n_cu);
+  else if (per == 3 && a.K <= 1024)
+    launch_gemv16_t<3, SPL, 8, IN, OUT, NTW, 1>(st, rec, a, n_cu);
+  else if (per == 3)
+    launch_gemv16_t<3, SPL, 16, IN, OUT, NTW, 1>(st, rec, a, n_cu);
+  else
+    launch_gemv16_t<4, SPL, 8, IN, OUT, NTW, 1>(st, rec, a, n_cu);
+  return true;
 }
 template <int SPL, int IN, int OUT, bool NTW>
 inline void launch_gemv16_n(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a, int n_cu) {
+  if constexpr (IN == GEMV_IN_BF16_RMS) {
+    if (launch_gemv16_round<SPL, IN, OUT, NTW>(st, rec, a, n_cu)) return;
+  }
   const int rows = gemv16_rows(IN >= GEMV_IN_BF16, a.N, a.K, a.nb, n_cu);
   if (rows == 32) {
     launch_gemv16_t<2, SPL, 8, IN, OUT, NTW>(st, rec, a, n_cu);
@@ -805,6 +936,10 @@ inline void launch_gemv16_n(hipStream_t st, crabml_hip_device::ProfRec* rec, con
     if (rows == 8) {
       // (two steps out a wave: three or four, of neighbouring pieces of k, made a whole decode step of 3 to 8 rows 0.5 to 3 % longer)
       launch_k(st, rec, k_gemv16_bf16<1, SPL, 16, 2, IN, OUT, NTW, 1, true>, dim3((a.N + 7) / 8), dim3(1024), 0, a);
+      return;
+    }
+    if (gemv16_narrow(a.N, a.K, n_cu) && a.K >= GEMV16_SHARED_K) {
+      launch_k(st, rec, k_gemv16_bf16<1, SPL, 8, 2, IN, OUT, NTW, 4, false, 2>, dim3((a.N + 127) / 128 * 16), dim3(512), 0, a);
       return;
     }
     if (gemv16_deep(a.N, a.K, n_cu)) {

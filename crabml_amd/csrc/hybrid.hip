@@ -86,6 +86,8 @@ struct crabml_hip_hybrid {
   int ld_vk = 0, ld_kv = 0, ld_lat = 0, ld_rot = 0;
   size_t hist = 0;  // earlier positions a latent layer can see
   unsigned* st_tick = nullptr;
+  unsigned long long* st_half = nullptr;  // GemvBf16::half, meet
+  unsigned* st_meet = nullptr;
   unsigned* st_out = nullptr;
   size_t st_out_cap = 0;
   float* am_val = nullptr;
@@ -447,6 +449,8 @@ bool rows16(const Ctx* c, int B) { return B > 2 && !c->f32; }
 template <int IN, int IN16, int OUT>
 void step_linear(Ctx* c, crabml_hip_device::ProfRec* rec, GemvBf16 g) {
   g.resident = c->weight_bytes <= (g.nb > 2 ? RESIDENT_MALL : RESIDENT_L2);
+  g.half = c->st_half;
+  g.meet = c->st_meet;
   if (g.nb <= 2)
     launch_gemv_bf16<IN, OUT>(c->dev->stream, rec, g);
   else if (c->f32)
@@ -1285,6 +1289,8 @@ int create_impl(Ctx* c, const crabml_hip_hybrid_layer_t* layers, const crabml_hi
     CH_TRY(dalloc_n(c, B * c->ld_xss, &c->st_xss));
     CH_TRY(dalloc_n(c, B * c->ld_cat, &c->st_cat16));
     CH_TRY(dalloc_n(c, B * c->ld_u, &c->st_u16));
+    CH_TRY(dalloc_n(c, gemv16_half_bytes(dev->n_cu) / sizeof(unsigned long long), &c->st_half));
+    CH_TRY(dalloc_n(c, gemv16_meet_bytes(dev->n_cu) / sizeof(unsigned), &c->st_meet));
   }
   CH_TRY(dalloc_n(c, ss, &c->st_ss));
   CH_TRY(dalloc_n(c, part, &c->st_part));

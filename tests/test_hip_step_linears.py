@@ -42,6 +42,27 @@ def test_batched_steps(ca, hdev, tmp_path, design, width, ff, vocab, f32):
             assert np.sqrt((d * d).mean(axis=1)).max() <= (2e-5 if f32 else 2.5e-2) * np.sqrt((want[i] ** 2).mean()), (batch, i)
 
 
+# the classifier in one round of workgroups of 32, 48 and 64 rows, a tile and four rows past each line (of few columns: eight or sixteen waves with a piece of k each or
+# none; of 2090: sixteen with two and a third that some have), two workgroups to a k of 3104 and 3072 columns with a tile that 72 and 2048 rows do not fill and fill
+@pytest.mark.parametrize("width,ff,vocab", [(72, 3100, 4100), (72, 90, 8196), (72, 90, 12292), (72, 90, 16388), (2090, 90, 4100), (2090, 90, 8196), (2090, 90, 12292), (2048, 3072, 50)])
+def test_one_round_of_workgroups(ca, hdev, tmp_path, width, ff, vocab):
+    config, tensors, oracle = nilivik(width, ff, vocab)
+    bits = tensors(config, 12, pool=1 << 20)
+    r = ca.load_model(sh.write_model(config, bits, str(tmp_path)), hdev, seq_len=16)
+    toks = np.random.default_rng(vocab + ff).integers(0, vocab, (16, 3))
+    want = oracle.forward(config, {k: sh.from_bf16(v) for k, v in bits.items()}, toks[0])
+    seen = []
+    for batch in (3, 8, 9, 16):
+        seqs = [r.open() for _ in range(batch)]
+        got = np.array([r.step([(s, [int(toks[i, t])], [0]) for i, s in enumerate(seqs)])[0] for t in range(3)])
+        for s in seqs:
+            r.close(s)
+        d = got - want
+        assert np.sqrt((d * d).mean(axis=1)).max() <= 2.5e-2 * np.sqrt((want ** 2).mean()), batch  # (the design's own bound)
+        seen.append(got)
+    assert all(np.array_equal(s, seen[0]) for s in seen)  # (bit for bit: a sequence's logits do not depend on how many share its step)
+
+
 # columns: those of the steps in flight, one octet more; one staged segment of one row, of two, of eight (8192, 4096, 1024 elements), and one octet more
 @pytest.mark.parametrize("m,k", [(70, 2048), (70, 2056), (515, 4096), (33, 4104), (66, 8200), (17, 1032), (16389, 2056)])
 def test_row_kernels_over_long_rows(ca, hdev, m, k):
