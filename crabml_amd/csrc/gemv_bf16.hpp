@@ -226,14 +226,14 @@ __device__ __forceinline__ void rows16_out(const GemvBf16& a, int row, int b, fl
 
 #define GEMV_BF16_LDS_FLOATS 8192  // rhs elements staged at a time, all rows together: a cut segment is a multiple of the steps in flight
 
-// UN: steps of 512 in flight; NT: weights nontemporal (GemvBf16::resident); ROLL: a step's registers are refilled as soon as it has been used, else all
+// WV: waves of a workgroup; UN: steps of 512 in flight; NT: weights nontemporal (GemvBf16::resident); ROLL: a step's registers are refilled as soon as it has been used, else all
 // of them are asked for together in front of the products
-template <int NB, int R, int UN, int IN, int OUT, bool NT, bool ROLL>
-__global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
+template <int WV, int NB, int R, int UN, int IN, int OUT, bool NT, bool ROLL>
+__global__ __launch_bounds__(64 * WV) void k_gemv_bf16(const GemvBf16 a) {
   extern __shared__ __attribute__((aligned(16))) float gemv_lds[];  // [NB][2][seg / 2]
-  __shared__ float red[4][NB];
+  __shared__ float red[WV][NB];
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_wg();
-  const int row0 = (blockIdx.x * 4 + wave) * R, b0 = blockIdx.y * NB;
+  const int row0 = (blockIdx.x * WV + wave) * R, b0 = blockIdx.y * NB;
   const int seg = a.K < GEMV_BF16_LDS_FLOATS / NB ? a.K : GEMV_BF16_LDS_FLOATS / NB;  // elements per staged segment (512-multiple if cut)
   const int half = seg / 2;                                                           // floats per half-octet plane
   const unsigned short* wr[R];
@@ -289,7 +289,7 @@ __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
       const int bb = b0 + b < a.nb ? b0 + b : a.nb - 1;
       const float* xr = a.x + (size_t)bb * a.ldx + s0;
       float* lo = gemv_lds + b * 2 * half;
-      for (int q = tid; q < n / 8; q += 256) {
+      for (int q = tid; q < n / 8; q += 64 * WV) {
         f32x4 v0 = *(const f32x4*)(xr + q * 8), v1 = *(const f32x4*)(xr + q * 8 + 4);
         if constexpr (IN == GEMV_IN_RMS || IN == GEMV_IN_RMSV) {
 #pragma unroll
@@ -373,7 +373,9 @@ __global__ __launch_bounds__(256) void k_gemv_bf16(const GemvBf16 a) {
   for (int b = 0; b < NB; b++) {
     scale[b] = 1.f;
     if constexpr (IN == GEMV_IN_RMS || IN == GEMV_IN_RMSV) {
-      const float s = (red[0][b] + red[1][b]) + (red[2][b] + red[3][b]);
+      float s = 0.f;
+#pragma unroll
+      for (int w = 0; w < WV; w += 4) s += (red[w][b] + red[w + 1][b]) + (red[w + 2][b] + red[w + 3][b]);
       scale[b] = (IN == GEMV_IN_RMS ? *a.gain : 1.0f) / sqrtf(s / (float)a.mean_n + a.eps);
     }
   }
@@ -954,46 +956,86 @@ inline void launch_gemv16_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, 
   a.resident ? launch_gemv16_n<SPL, IN, OUT, false>(st, rec, a, n_cu) : launch_gemv16_n<SPL, IN, OUT, true>(st, rec, a, n_cu);
 }
 
-template <int NB, int R, int IN, int OUT, int UN = NB >= 8 ? 2 : 4, bool ROLL = true>
+template <int WV, int NB, int R, int UN, int IN, int OUT, bool ROLL = true>
 inline void launch_gemv_bf16_t(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a) {
   const int cap = GEMV_BF16_LDS_FLOATS / NB, seg = a.K < cap ? a.K : cap;
-  launch_k(st, rec, a.resident ? k_gemv_bf16<NB, R, UN, IN, OUT, false, ROLL> : k_gemv_bf16<NB, R, UN, IN, OUT, true, ROLL>,
-           dim3((a.N + 4 * R - 1) / (4 * R), (a.nb + NB - 1) / NB), dim3(256), (size_t)NB * seg * sizeof(float), a);
+  launch_k(st, rec, a.resident ? k_gemv_bf16<WV, NB, R, UN, IN, OUT, false, ROLL> : k_gemv_bf16<WV, NB, R, UN, IN, OUT, true, ROLL>,
+           dim3((a.N + WV * R - 1) / (WV * R), (a.nb + NB - 1) / NB), dim3(64 * WV), (size_t)NB * seg * sizeof(float), a);
 }
-// One row of the rhs: what bounds it is how early the weights are asked for, so a wave has 8 to 16 KB of them on their way while it stages
-// the rhs: four rows a wave where they still fill the chip (all of 2048 columns at once: gate | up of 16384 x 2048 15.0 -> 13.5 us against half
-// of them; 11264 x 2048 and 8192 x 2048 are better with two rows, 10.2 / 11.5 and 8.2 / 9.2), one row and twice the steps for few rows of
-// many columns (2048 x 8192 9.4 -> 8.5, 2048 x 4096 6.5 -> 6.3, against two rows).
-// Two rows: where the columns are more than the steps in flight, the next ones are asked for together -- one by one, each behind twice the products, they
-// come too late (8192 .. 32000 x 4096 with the norm inside 33.2 -> 32.1, 43.3 -> 42.4, 14.75 -> 14.6 us, 2048 / 4096 x 8192 11.15 -> 11.0, 15.85 -> 15.6; with up to
-// 2048 columns the copy costs 13.1 against 11.9, 25.6 / 23.0).  A tail that is scaled and streams have more to do beside: 2048 x 4096 8.1 / 7.75,
-// 2048 x 8192 11.0 / 10.7 with the refill step by step.
-// Eight rows (matmul_vec): the same, and more so: step by step 8192 x 2048 15.1 us against 9.9, 8192 x 8192 49.1 / 32.0, 32000 x 2048 49.4 / 39.4.  Four rows: step by
-// step 8.0 -> 7.4, 26.3 -> 23.6, 26.6 -> 23.7.
+// One row of the rhs: every workgroup stages it for itself, so eight waves with a row each are faster than four with one, two or four (half as many copies of the rhs
+// through the L2s and half as many workgroups to start, as many requests out from the beginning); a wave has no more requests out than its row has steps -- more are the row's
+// start again, 0.1 to 0.2 us each -- and eight where there are more than eight to make.  What else: two rows a wave where there are more than 8192 of less than 2048
+// columns (four of at most 512), four waves up to 1024 rows of longer ones and from 16384 rows of 2048 columns on.  Us a launch, four waves of as many rows as
+// was best for them and four or eight steps out / these: 2048 x 512 3.25 / 2.8, 32000 x 512 9.7 / 7.5, 32000 x 128 8.5 / 5.2, 4096 x 1024 4.4 / 4.0, 3648 x 2048 5.5 / 5.0,
+// 8192 x 2048 7.7 / 7.4, 11264 x 2048 9.7 / 9.3, 32000 x 2048 23.1 / 20.2, 2048 x 8192 7.75 / 7.5, 2048 x 4096 5.2 / 5.1; gate | up of 16384 x 2048 13.7 / 12.7, 8192 x 512 4.6 / 4.1.
+template <int IN, int OUT>
+inline void launch_gemv1_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a) {
+  constexpr bool NARROW = OUT == GEMV_OUT_RESIDUAL || OUT == GEMV_OUT_STREAMS;  // (as many rows as the model is wide)
+  if constexpr (OUT == GEMV_OUT_GLU) {
+    if (a.K <= 512)
+      launch_gemv_bf16_t<8, 1, 2, 1, IN, OUT>(st, rec, a);
+    else if (a.K <= 1024)
+      launch_gemv_bf16_t<8, 1, 2, 2, IN, OUT>(st, rec, a);
+    else if (a.N >= 2048)
+      launch_gemv_bf16_t<8, 1, 2, 4, IN, OUT>(st, rec, a);
+    else
+      launch_gemv_bf16_t<4, 1, 2, 4, IN, OUT>(st, rec, a);
+    return;
+  } else {
+    if constexpr (!NARROW) {
+      if (a.K <= 512 && a.N >= 16384) return launch_gemv_bf16_t<8, 1, 4, 1, IN, OUT>(st, rec, a);
+      if (a.K <= 512 && a.N > 8192) return launch_gemv_bf16_t<8, 1, 2, 1, IN, OUT>(st, rec, a);
+      if (a.K < 2048 && a.N > 8192)
+        return a.K <= 1024 ? launch_gemv_bf16_t<8, 1, 2, 2, IN, OUT>(st, rec, a) : launch_gemv_bf16_t<8, 1, 2, 4, IN, OUT>(st, rec, a);
+    }
+    if (a.K <= 512)
+      launch_gemv_bf16_t<8, 1, 1, 1, IN, OUT>(st, rec, a);
+    else if (a.K <= 1024)
+      launch_gemv_bf16_t<8, 1, 1, 2, IN, OUT>(st, rec, a);
+    else if (a.N <= 1024 && a.K >= 4096)
+      launch_gemv_bf16_t<4, 1, 1, 8, IN, OUT>(st, rec, a);
+    else if (a.K > 4096)
+      launch_gemv_bf16_t<8, 1, 1, 8, IN, OUT>(st, rec, a);
+    else if (a.N <= 1024 || a.N >= 16384)
+      launch_gemv_bf16_t<4, 1, 1, 4, IN, OUT>(st, rec, a);
+    else
+      launch_gemv_bf16_t<8, 1, 1, 4, IN, OUT>(st, rec, a);
+  }
+}
+// Two rows: the same (2048 x 512 3.95 / 3.6, 1280 x 4096 5.5 / 4.8, 2048 x 8192 9.5 / 8.4, 8192 x 4096 14.3 / 13.25), but two rows of weights a wave where there are more than
+// 4096 of up to 1024 columns or more than 2048 of up to 2048 (32000 x 512 13.6 / 11.7, x 2048 22.4 and 23.85 with a row each).
+template <int IN, int OUT>
+inline void launch_gemv2_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a) {
+  if constexpr (OUT == GEMV_OUT_GLU) {
+    if (a.K <= 1024)
+      launch_gemv_bf16_t<8, 2, 2, 2, IN, OUT>(st, rec, a);
+    else
+      launch_gemv_bf16_t<8, 2, 2, 4, IN, OUT>(st, rec, a);
+  } else {
+    if (a.K <= 1024 && a.N > 4096)
+      launch_gemv_bf16_t<4, 2, 2, 2, IN, OUT>(st, rec, a);
+    else if (a.K <= 1024)
+      launch_gemv_bf16_t<8, 2, 1, 2, IN, OUT>(st, rec, a);
+    else if (a.K <= 2048 && a.N > 2048)
+      launch_gemv_bf16_t<4, 2, 2, 4, IN, OUT>(st, rec, a);
+    else
+      launch_gemv_bf16_t<8, 2, 1, 4, IN, OUT>(st, rec, a);
+  }
+}
+// Eight rows (matmul_vec): the next steps' requests together, behind the products; step by step 8192 x 2048 15.1 us against 9.9, 8192 x 8192 49.1 / 32.0, 32000 x 2048
+// 49.4 / 39.4.  Four rows: step by step 8.0 -> 7.4, 26.3 -> 23.6, 26.6 -> 23.7.
 // rows of the rhs that share one pass over the weights: as many as there are, up to 8
 template <int IN, int OUT>
 inline void launch_gemv_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a) {
-  const bool wide = a.N >= 16384;  // enough rows to give a wave four and still fill the chip
-  if (a.nb <= 1) {
-    if (wide)
-      launch_gemv_bf16_t<1, 4, IN, OUT>(st, rec, a);
-    else if (OUT == GEMV_OUT_GLU || (a.N >= 2048 && (a.N >= 4096 || a.K < 4096)))
-      launch_gemv_bf16_t<1, 2, IN, OUT>(st, rec, a);
-    else if constexpr (OUT != GEMV_OUT_GLU) {
-      if (a.K >= 4096)
-        launch_gemv_bf16_t<1, 1, IN, OUT, 8>(st, rec, a);
-      else
-        launch_gemv_bf16_t<1, 1, IN, OUT>(st, rec, a);
-    }
-  } else if (a.nb <= 2) {
-    if constexpr (IN != GEMV_IN_SPLIT && OUT != GEMV_OUT_STREAMS) {
-      if (a.K > 4 * 512) return launch_gemv_bf16_t<2, 2, IN, OUT, 4, false>(st, rec, a);
-    }
-    launch_gemv_bf16_t<2, 2, IN, OUT>(st, rec, a);
-  } else if (a.nb <= 4) {
-    launch_gemv_bf16_t<4, 2, IN, OUT>(st, rec, a);
-  } else {
-    launch_gemv_bf16_t<8, 2, IN, OUT, 2, false>(st, rec, a);
+  if (a.nb <= 1)
+    launch_gemv1_bf16<IN, OUT>(st, rec, a);
+  else if (a.nb <= 2)
+    launch_gemv2_bf16<IN, OUT>(st, rec, a);
+  else if constexpr (IN == GEMV_IN_PLAIN && OUT == GEMV_OUT_STORE) {
+    if (a.nb <= 4)
+      launch_gemv_bf16_t<4, 4, 2, 4, IN, OUT>(st, rec, a);
+    else
+      launch_gemv_bf16_t<4, 8, 2, 2, IN, OUT, false>(st, rec, a);
   }
 }
 

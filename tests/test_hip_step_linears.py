@@ -76,3 +76,19 @@ def test_row_kernels_over_long_rows(ca, hdev, m, k):
         # (f32 sums of k products, k / 64 of them in a lane's chain: 2 + k / 64 roundings of 2^-24 each at the most, of the products' absolute values)
         bound = (2 + k / 64) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T)
         assert (np.abs(got - x.astype(np.float64) @ w.T) <= bound).all(), b
+
+
+# one and two rows, either side of every line of the forms: 512, 1024, 2048 and 4096 columns; 1024, 4096, 8192 and 16384 rows of weights
+@pytest.mark.parametrize("k", [8, 512, 520, 1024, 1032, 2040, 2048, 2056, 4096, 4104])
+@pytest.mark.parametrize("m", [3, 1024, 1025, 4097, 8193, 16384])
+def test_row_forms(ca, hdev, m, k):
+    rng = np.random.default_rng(k + m)
+    bits = sh.to_bf16(rng.standard_normal((m, k)).astype(np.float32))
+    w = sh.from_bf16(bits)
+    t = ca.HipTensor.from_cpu(bits.view(np.uint8).reshape(-1), [m, k], ca.GGMLType.BF16, hdev)
+    x = rng.standard_normal((2, k)).astype(np.float32)
+    # (as above, the sums of the reference in 32 bits as well: k more roundings at the most)
+    bound = (2 + k / 64 + k) * 2.0 ** -24 * (np.abs(x) @ np.abs(w).T)
+    for b in (1, 2):
+        got = t.matmul_vec(ca.HipTensor.new(x[:b].reshape(-1), [b, k], hdev)).export().reshape(b, m)
+        assert (np.abs(got - x[:b] @ w.T) <= bound[:b]).all(), b
