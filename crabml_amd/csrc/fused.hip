@@ -428,41 +428,57 @@ void enqueue_attention(crabml_hip_llama* c, int l, signed char* xq, unsigned sho
 }
 
 // ---- F16 layers on the fast device (fused_f16.hpp) ---------------------------------------------------------
-// Rows a wave takes: two (gate and up: two of each) where that still leaves eight waves per CU, else one -- a launch is over in one round
-// either way, and a short one wants more waves rather than longer ones.
-template <int R, int UN, int IN, int OUT>
+// Every workgroup stages the rhs for itself, so eight waves of a row (gate and up: one of each; q | k | v: the pair that is rotated) are faster than four of two or four rows:
+// half the copies through the L2s, as many requests out from the start.  As many steps out as the rows have, up to four (more are the row's start again); four rows a
+// wave where a classifier has many short ones; four waves for q | k | v from 4096 columns on.  ffn_down stages nothing: four waves, two rows where there are many.  Us a launch,
+// four waves and the steps out that were best for them / these: q | k | v 3072 x 2048 5.4 / 4.8, 864 x 288 3.2 / 3.0; wo 2048 x 2048 4.2 / 3.6, 512 x 512 2.6 / 2.2; gate | up of
+// 2 x 8192 x 2048 13.4 / 12.4, 2 x 14336 x 4096 38.1 / 35.4; ffn_down 2048 x 8192 7.6 / 7.4, 512 x 1024 3.1 / 2.6; 32000 x 2048 24.5 / 20.9, 32000 x 288 7.3 / 5.9.
+template <int WV, int R, int UN, int IN, int OUT>
 void launch_step_f16_t(crabml_hip_device* dev, crabml_hip_device::ProfRec* rec, const StepF16& a, const QkvEpi& e) {
-  const int per_wg = 4 * (OUT == F16_OUT_GU ? R / 2 : R);
+  const int per_wg = WV * (OUT == F16_OUT_GU ? R / 2 : R);
   const dim3 grid((unsigned)((a.m + per_wg - 1) / per_wg));
   const size_t lds = IN == F16_IN_HALF ? 0 : ((size_t)a.k * 2 + 15) & ~(size_t)15;
   if constexpr (IN != F16_IN_HALF) {
     if (a.k > 4096) {
-      launch_k(dev->stream, rec, k_step_f16<R, UN, 8, IN, OUT>, grid, dim3(256), lds, a, e);
+      launch_k(dev->stream, rec, k_step_f16<WV, R, UN, 32 / WV, IN, OUT>, grid, dim3(64 * WV), lds, a, e);
       return;
     }
   }
-  launch_k(dev->stream, rec, k_step_f16<R, UN, 2, IN, OUT>, grid, dim3(256), lds, a, e);
+  launch_k(dev->stream, rec, k_step_f16<WV, R, UN, 8 / WV, IN, OUT>, grid, dim3(64 * WV), lds, a, e);
+}
+template <int WV, int R, int IN, int OUT>
+void launch_step_f16_u(crabml_hip_device* dev, crabml_hip_device::ProfRec* rec, const StepF16& a, const QkvEpi& e) {
+  if (a.k <= 512)
+    launch_step_f16_t<WV, R, 1, IN, OUT>(dev, rec, a, e);
+  else if (a.k <= 1024)
+    launch_step_f16_t<WV, R, 2, IN, OUT>(dev, rec, a, e);
+  else
+    launch_step_f16_t<WV, R, 4, IN, OUT>(dev, rec, a, e);
 }
 template <int IN, int OUT>
 void launch_step_f16(crabml_hip_device* dev, crabml_hip_device::ProfRec* rec, const StepF16& a, const QkvEpi& e = QkvEpi{}) {
   const bool wide = a.m >= 16 * dev->n_cu;
-  if constexpr (OUT == F16_OUT_QKV)
-    launch_step_f16_t<2, 4, IN, OUT>(dev, rec, a, e);
-  else if constexpr (OUT == F16_OUT_GU) {
-    if (wide)
-      launch_step_f16_t<4, 2, IN, OUT>(dev, rec, a, e);
+  if constexpr (OUT == F16_OUT_QKV) {
+    if (a.k >= 4096)
+      launch_step_f16_t<4, 2, 4, IN, OUT>(dev, rec, a, e);
     else
-      launch_step_f16_t<2, 4, IN, OUT>(dev, rec, a, e);
+      launch_step_f16_u<8, 2, IN, OUT>(dev, rec, a, e);
+  } else if constexpr (OUT == F16_OUT_GU) {
+    launch_step_f16_u<8, 2, IN, OUT>(dev, rec, a, e);
   } else if constexpr (OUT == F16_OUT_STORE) {  // (a classifier)
-    if (wide)
-      launch_step_f16_t<4, 2, IN, OUT>(dev, rec, a, e);
+    if (wide && a.k <= 512)
+      launch_step_f16_t<8, 4, 1, IN, OUT>(dev, rec, a, e);
+    else if (wide && a.k <= 1024)
+      launch_step_f16_t<8, 2, 2, IN, OUT>(dev, rec, a, e);
     else
-      launch_step_f16_t<1, 4, IN, OUT>(dev, rec, a, e);
+      launch_step_f16_u<8, 1, IN, OUT>(dev, rec, a, e);
+  } else if constexpr (IN == F16_IN_HALF) {
+    if (wide)
+      launch_step_f16_t<4, 2, 4, IN, OUT>(dev, rec, a, e);
+    else
+      launch_step_f16_u<4, 1, IN, OUT>(dev, rec, a, e);
   } else {
-    if (wide)
-      launch_step_f16_t<2, 4, IN, OUT>(dev, rec, a, e);
-    else
-      launch_step_f16_t<1, 8, IN, OUT>(dev, rec, a, e);
+    launch_step_f16_u<8, 1, IN, OUT>(dev, rec, a, e);
   }
 }
 StepF16 step_f16(const crabml_hip_llama* c, std::initializer_list<const crabml_hip_buf*> w, int m, int k, const float* x, const float* gain, float eps, float* out) {

@@ -5,7 +5,7 @@
 //
 // Mapping: a wave owns R weight rows and strides k 512 elements at a time (8 per lane: one aligned 16-byte request per row), UN steps in
 // flight; the first requests go out before the rhs is looked at.  The rhs is what the reference multiplies by (buf/api.rs:142-159: the row
-// rounded to f16): a workgroup of four waves normalizes (x / rms) * w, or rounds, the whole row into LDS itself -- 2 bytes per element, read
+// rounded to f16): a workgroup of eight waves (four: launch_step_f16) normalizes (x / rms) * w, or rounds, the whole row into LDS itself -- 2 bytes per element, read
 // back as contiguous 16-byte pieces -- which is 8-16 KB from L2 per workgroup beside its 16-64 KB of weights and hides behind them.
 // ffn_down's rhs leaves the gate | up launch as f16 already and is read from L2 in place.  Products are exact in f32 (v_fma_mix_f32), sums
 // f32.  Bound: the weights' bytes, plus a launch's ramp.
@@ -30,13 +30,13 @@ struct StepF16 {
   const unsigned short* exp_tab = nullptr;
 };
 
-// NIT: rhs pieces of 8 elements a thread holds while the norm is taken (k <= NIT * 2048)
-template <int R, int UN, int NIT, int IN, int OUT>
-__global__ __launch_bounds__(256) void k_step_f16(const StepF16 a, const QkvEpi e) {
+// WV: waves of a workgroup; NIT: rhs pieces of 8 elements a thread holds while the norm is taken (k <= NIT * WV * 512)
+template <int WV, int R, int UN, int NIT, int IN, int OUT>
+__global__ __launch_bounds__(64 * WV) void k_step_f16(const StepF16 a, const QkvEpi e) {
   extern __shared__ __attribute__((aligned(16))) unsigned short rhs[];  // [k], NORM and ROUND
-  __shared__ float red[4];
+  __shared__ float red[WV];
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_wg();
-  const int unit = blockIdx.x * 4 + wave;  // this wave's rows: R unit .. (GU: R / 2 of either matrix)
+  const int unit = blockIdx.x * WV + wave;  // this wave's rows: R unit .. (GU: R / 2 of either matrix)
   const unsigned short* wr[R];
   bool live[R];
 #pragma unroll
@@ -80,7 +80,7 @@ __global__ __launch_bounds__(256) void k_step_f16(const StepF16 a, const QkvEpi 
     f32x4 v[NIT][2], gn[NIT][2];
 #pragma unroll
     for (int it = 0; it < NIT; it++) {
-      const int i = (it * 256 + tid) * 8, at = i < a.k ? i : 0;
+      const int i = (it * (64 * WV) + tid) * 8, at = i < a.k ? i : 0;
 #pragma unroll
       for (int h = 0; h < 2; h++) {
         v[it][h] = *(const f32x4*)(a.x + at + 4 * h);
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(256) void k_step_f16(const StepF16 a, const QkvEpi 
       float sq = 0.f;
 #pragma unroll
       for (int it = 0; it < NIT; it++)
-        if ((it * 256 + tid) * 8 < a.k) {
+        if ((it * (64 * WV) + tid) * 8 < a.k) {
 #pragma unroll
           for (int h = 0; h < 2; h++)
 #pragma unroll
@@ -101,11 +101,14 @@ __global__ __launch_bounds__(256) void k_step_f16(const StepF16 a, const QkvEpi 
       sq = wave_sum_f32(sq);
       if (lane == 0) red[wave] = sq;
       __syncthreads();
-      rms = sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)a.k + a.eps);
+      sq = 0.f;
+#pragma unroll
+      for (int w = 0; w < WV; w += 4) sq += (red[w] + red[w + 1]) + (red[w + 2] + red[w + 3]);
+      rms = sqrtf(sq / (float)a.k + a.eps);
     }
 #pragma unroll
     for (int it = 0; it < NIT; it++) {
-      const int i = (it * 256 + tid) * 8;
+      const int i = (it * (64 * WV) + tid) * 8;
       if (i < a.k) {
         unsigned short t[8];
 #pragma unroll

@@ -87,3 +87,9 @@ def test_decode_step_against_the_scalar_order(ca, dim, hidden, heads, kv, vocab,
     # 1.2e-3 over these models where the fast device takes one launch per op, four such steps allowed
     err = np.linalg.norm(logits[1] - logits[0], axis=1) / np.linalg.norm(logits[0], axis=1)
     assert np.max(err) <= 4 * 2.0 ** -11, err
+
+
+# either side of 512, 1024 and 4096 columns; classifiers either side of sixteen rows a CU
+@pytest.mark.parametrize("dim,hidden,heads,kv,vocab", [(520, 512, 5, 5, 4095), (1024, 1032, 8, 2, 4096), (1032, 4096, 6, 3, 70), (512, 1024, 8, 2, 16400)])
+def test_decode_step_forms_against_the_scalar_order(ca, dim, hidden, heads, kv, vocab):
+    test_decode_step_against_the_scalar_order(ca, dim, hidden, heads, kv, vocab, True)
