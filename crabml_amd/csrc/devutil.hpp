@@ -217,21 +217,14 @@ struct Q8KLane {
   float d;
 };
 __device__ __forceinline__ Q8KLane q8k_wave_quant(const f32x4 v, int lane) {
-  // first element of maximal |x|: the lane's own first maximum (strict `>` scan), the wave maximum by DPP, then
-  // the lowest lane that holds it (ballot) hands over its element
-  float loc_abs = 0.f, loc_val = 0.f;
+  // first element of maximal |x| -- of its value only the sign is not known yet: the wave maximum by DPP, the lowest lane that holds it (ballot), that
+  // lane's first element that does.  (NaN is never the maximum.)
+  const float best_abs = wave_max_f32(fmaxf(fmaxf(fmaxf(0.f, fabsf(v[0])), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+  float mine = 0.f;
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    float a = fabsf(v[i]);
-    if (a > loc_abs) {
-      loc_abs = a;
-      loc_val = v[i];
-    }
-  }
-  const float best_abs = wave_max_f32(loc_abs);
-  const unsigned long long holders = __ballot(loc_abs == best_abs);
-  const int first = holders ? __builtin_ctzll(holders) : 0;
-  const float best_val = rl_f(loc_val, first);
+  for (int i = 3; i >= 0; i--) mine = fabsf(v[i]) == best_abs ? v[i] : mine;
+  const unsigned long long holders = __ballot(fabsf(mine) == best_abs);
+  const float best_val = rl_f(mine, holders ? __builtin_ctzll(holders) : 0);
   const float scale = -128.0f / best_val;
   Q8KLane o;
   o.d = best_abs == 0.0f ? 0.0f : 1.0f / scale;
@@ -239,18 +232,15 @@ __device__ __forceinline__ Q8KLane q8k_wave_quant(const f32x4 v, int lane) {
   int s = 0;
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    int t = 0;
-    if (best_abs != 0.0f) {
-      float r = roundf(scale * v[i]);  // half away from zero
-      r = fminf(r, 127.0f);
-      t = rs_f32_as_i32(r);
-      t = t < -128 ? -128 : t;  // `as i8` saturates
-    }
+    // half away from zero: the largest number below 1/2 moves exactly what rounds up past the next integer (every |r| to 131), the conversion cuts off.
+    // min(127) takes NaN to 127, `as i8` saturates.
+    float r = scale * v[i];
+    r = fmaxf(fminf(r + __builtin_copysignf(0.49999997f, r), 127.0f), -128.0f);
+    const int t = best_abs != 0.0f ? (int)r : 0;
     qi[i] = t;
     s += t;
   }
-  o.packed = ((unsigned)qi[0] & 0xffu) | (((unsigned)qi[1] & 0xffu) << 8) | (((unsigned)qi[2] & 0xffu) << 16) |
-             (((unsigned)qi[3] & 0xffu) << 24);
+  o.packed = ((unsigned)qi[0] & 0xffu) | (((unsigned)qi[1] & 0xffu) << 8) | (((unsigned)qi[2] & 0xffu) << 16) | ((unsigned)qi[3] << 24);
   s += dpp_i<0xB1>(s);
   s += dpp_i<0x4E>(s);
   o.quad_sum = s;
@@ -259,13 +249,19 @@ __device__ __forceinline__ Q8KLane q8k_wave_quant(const f32x4 v, int lane) {
 
 // The class-major copy of a super-block's quants (plane `qp`, common.hpp): q8k_wave_quant leaves lane L the four consecutive
 // elements 4 L .. 4 L + 3; element 4 j + k of 32-group c = L / 8 (j = L % 8) goes to byte 4 ((4 j + k) % 8) + (4 j + k) / 8 =
-// 16 (j & 1) + 4 k + j / 2 of the group.  sb_base: the super-block's 256 bytes (global memory or LDS).
-__device__ __forceinline__ void q8k_store_class_major(signed char* sb_base, int lane, unsigned packed) {
-  signed char* p = sb_base + 32 * (lane >> 3) + 16 * (lane & 1) + ((lane & 7) >> 1);
-  p[0] = (signed char)(packed & 0xffu);
-  p[4] = (signed char)((packed >> 8) & 0xffu);
-  p[8] = (signed char)((packed >> 16) & 0xffu);
-  p[12] = (signed char)(packed >> 24);
+// 16 (j & 1) + 4 k + j / 2 of the group: four bytes of four lanes of one parity are transposed (two exchanges), after which a lane holds dword
+// 4 (j & 1) + j / 2 of its group.  sb_base: the super-block's 256 bytes (global memory or LDS), 4-byte aligned.  All lanes of the wave.
+__device__ __forceinline__ unsigned q8k_class_major(int lane, unsigned packed) {
+  const unsigned a = (unsigned)dpp_i<0x4E>((int)packed);  // of lane ^ 2
+  packed = __builtin_amdgcn_perm(a, packed, lane & 2 ? 0x03070105u : 0x06020400u);
+  const unsigned b = (unsigned)dpp_i<0x1B>(dpp_i<0x141>((int)packed));  // of lane ^ 4 (half row mirrored, quads mirrored)
+  return __builtin_amdgcn_perm(b, packed, lane & 4 ? 0x03020706u : 0x05040100u);
+}
+__device__ __forceinline__ int q8k_class_major_at(int lane) { return (lane >> 3) * 8 + (lane & 1) * 4 + ((lane >> 1) & 3); }
+// (`in`: lanes that store; whole groups of 8)
+__device__ __forceinline__ void q8k_store_class_major(signed char* sb_base, int lane, unsigned packed, bool in = true) {
+  const unsigned d = q8k_class_major(lane, packed);
+  if (in) ((unsigned*)sb_base)[q8k_class_major_at(lane)] = d;
 }
 
 }  // namespace crabml_hip

@@ -24,6 +24,7 @@
 #include "fused_common.hpp"
 #include "fused_attention.hpp"
 #include "fused_ffn.hpp"
+#include "fused_kquant.hpp"
 #include "fused_small.hpp"
 #include "graph_steps.hpp"
 #include "fused_f16.hpp"
@@ -142,7 +143,7 @@ struct crabml_hip_llama {
   bool q8k_producers = false;            // attention / gate-up emit the Q8_K planes of wo's / ffn_down's rhs themselves
   unsigned tp_salt = 0;      // P2P group: epoch salt of this context (see TpP2P::salt)
   bool tp_dry = false;       // CRABML_HIP_LLAMA_TP_DRY_RUN: a lone rank that skips the all-reduces (timing only)
-  bool k_norm_in = false;    // fast Q4_K step: gate | up normalizes and quantizes wo's f32 row itself (k_gateup_k_lds<.., NORMIN>)
+  bool kq = false;           // Q4_K and Q6_K layers, fast step on one device: every launch quantizes its rhs itself (fused_kquant.hpp)
   bool kfused = false;       // Q4_K layers, fast mode: fused GEMV kernels with the Q4_K inner loop (enqueue_segment_k)
   bool f16_step = false;     // F16 layers, fast mode, one GPU: the linears with their row operations folded in (enqueue_segment_f16)
   bool attn_row_apart = false;  // test hook: the attention row of odd head widths through the quantizer's own launch
@@ -515,7 +516,7 @@ int enqueue_front(crabml_hip_llama* c, bool pick) {
   const bool prof = dev->prof_on && !c->use_graph && !c->capturing;
   crabml_hip_device::ProfRec nr{};
   const bool k = c->kfused && c->wtype == CRABML_HIP_Q4_K;
-  const int front = !c->kfused && (c->f16_step || c->generic) ? FRONT_ROW : k ? FRONT_Q8_K : c->wtype == CRABML_HIP_Q4_1 ? FRONT_Q8_1 : FRONT_Q8_0;
+  const int front = c->kq ? FRONT_SUMS : !c->kfused && (c->f16_step || c->generic) ? FRONT_ROW : k ? FRONT_Q8_K : c->wtype == CRABML_HIP_Q4_1 ? FRONT_Q8_1 : FRONT_Q8_0;
   TokenPick tp;
   tp.token = c->state;
   if (pick) {
@@ -529,7 +530,8 @@ int enqueue_front(crabml_hip_llama* c, bool pick) {
     tp.out = c->out_tokens;
   }
   const ActLayout al = act_layout(k ? CRABML_HIP_Q8_K : front == FRONT_Q8_1 ? CRABML_HIP_Q8_1 : CRABML_HIP_Q8_0, (size_t)dim);
-  const FrontOut o{(signed char*)c->act_dim, (signed char*)(c->act_dim + al.off_p), (void*)(c->act_dim + al.off_d), (void*)(c->act_dim + al.off_aux)};
+  FrontOut o{(signed char*)c->act_dim, (signed char*)(c->act_dim + al.off_p), (void*)(c->act_dim + al.off_d), (void*)(c->act_dim + al.off_aux)};
+  if (front == FRONT_SUMS) o.d = c->rsums;
   auto go = [&](auto kernel) {
     launch_k(dev->stream, prof ? &nr : nullptr, kernel, dim3(1), dim3(1024), front == FRONT_ROW ? 0 : norm_lds_bytes(dim),
              (const char*)c->token_embed->ptr, (int)c->token_embed->dtype, c->token_embed->wl.off_scale, tp, dim, c->x, (const float*)c->rms_att[0]->ptr,
@@ -538,6 +540,7 @@ int enqueue_front(crabml_hip_llama* c, bool pick) {
   if (prof) CH_TRY(prof_begin(dev, &nr, CRABML_HIP_F32, 6, 8.0 * dim));
   const bool narrow = dim <= 4096;
   switch (front) {
+    case FRONT_SUMS: narrow ? go(k_step_front<4, FRONT_SUMS>) : go(k_step_front<12, FRONT_SUMS>); break;
     case FRONT_ROW: narrow ? go(k_step_front<4, FRONT_ROW>) : go(k_step_front<12, FRONT_ROW>); break;
     case FRONT_Q8_0: narrow ? go(k_step_front<4, FRONT_Q8_0>) : go(k_step_front<12, FRONT_Q8_0>); break;
     case FRONT_Q8_1: narrow ? go(k_step_front<4, FRONT_Q8_1>) : go(k_step_front<12, FRONT_Q8_1>); break;
@@ -1041,21 +1044,19 @@ int enqueue_segment_k(crabml_hip_llama* c, int seg) {
   // wnext / eps_next: the RMSNorm that consumes this GEMV's output (norm epilogue only); xin: the f32 rhs
   // qmode: 0 = rhs planes from global memory, 1 = quantize the f32 rhs in the kernel's prologue, 2 = copy finished planes
   auto gemv_out = [&](const crabml_hip_buf* w, const Act& a, const float* xin, int k, uint32_t stage, const float* wnext,
-                      float eps_next, int qmode, bool x_only = false) -> int {
+                      float eps_next, int qmode) -> int {
     CH_TRY(P0(stage, dim, k));
     if constexpr (FMT == CRABML_HIP_Q4_K) {
       if (nepi) {
         NormGather ng{c->slots, c->slots + dim / 16, c->state + 4, c->state + 5, n_segments(c), seg, c->rsums};
         ActLayout al = act_layout(QT, (size_t)dim);
         ng.qp = (signed char*)(c->act_dim + al.off_p);
-        signed char* oq = x_only ? nullptr : (signed char*)c->act_dim;  // (x_only: the consumer quantizes, nq_epilogue)
+        signed char* oq = (signed char*)c->act_dim;
         void* od = (void*)(c->act_dim + al.off_d);
         void* ob = (void*)(c->act_dim + al.off_aux);
-        // (x_only: no hop pairs the halves of a chunk -- two 16-row workgroups per chunk whenever that still fits the chip twice)
         const int split = (g.flags & CRABML_HIP_LLAMA_SPLIT_CHUNKS_ALWAYS)  ? 2
                           : (g.flags & CRABML_HIP_LLAMA_SPLIT_CHUNKS_NEVER) ? 1
                           : (k / 32 >= 256 && dim / 32 <= dev->n_cu)        ? 2
-                          : (x_only && dim / 32 <= dev->n_cu)               ? 2
                                                                             : 1;
         const size_t lds = (size_t)k + (size_t)(k / 256) * 4 + (size_t)(k / 16) * 2;
         if (ordk) {  // (qmode is 1 or 2 here: `qin` holds on every ordered context)
@@ -1143,8 +1144,7 @@ int enqueue_segment_k(crabml_hip_llama* c, int seg) {
       enqueue_attention(c, l, nullptr, nullptr, nullptr, PrefetchPlan{}, 0, prof);
     }
     if (!qin) launch_quantize_act(st, QT, c->attn, (size_t)dim_l, c->act_attn);
-    CH_TRY(gemv_out(c->wo[l], act_k(c->act_attn, dim_l), c->attn, dim_l, 2, (const float*)c->rms_ffn[l]->ptr, 1e-5f, aq8 ? 2 : qin ? 1 : 0,
-                    qout && c->k_norm_in));
+    CH_TRY(gemv_out(c->wo[l], act_k(c->act_attn, dim_l), c->attn, dim_l, 2, (const float*)c->rms_ffn[l]->ptr, 1e-5f, aq8 ? 2 : qin ? 1 : 0));
   } else {
     if (!nepi) norm_quant((const float*)c->rms_ffn[l]->ptr, 1e-5f, tp, QT);  // llama2.rs:611
     CH_TRY(P0(3, 2.0 * hidden_l, dim));
@@ -1156,24 +1156,19 @@ int enqueue_segment_k(crabml_hip_llama* c, int seg) {
       if (ordk && qout)
         launch_k(st, R, k_gateup_k_lds<true, true>, dim3(hidden_l / 32), dim3(1024), ldso, planes_k(c->gate[l]), planes_k(c->up[l]),
                  act_k(c->act_dim, dim), (const unsigned short*)dev->exp_table, c->h, hidden_l, dim / 256, hx, (signed char*)c->act_hid,
-                 (float*)(c->act_hid + alh.off_d), (short*)(c->act_hid + alh.off_aux), (signed char*)(c->act_hid + alh.off_p), (const float*)nullptr, (const float*)nullptr, 0.f, (const float*)nullptr, 1);
+                 (float*)(c->act_hid + alh.off_d), (short*)(c->act_hid + alh.off_aux), (signed char*)(c->act_hid + alh.off_p));
       else if (ordk)
         launch_k(st, R, k_gateup_k_lds<false, true>, dim3(hidden_l / 32), dim3(1024), ldso, planes_k(c->gate[l]), planes_k(c->up[l]),
                  act_k(c->act_dim, dim), (const unsigned short*)dev->exp_table, c->h, hidden_l, dim / 256, hx, (signed char*)nullptr,
-                 (float*)nullptr, (short*)nullptr, (signed char*)nullptr, (const float*)nullptr, (const float*)nullptr, 0.f, (const float*)nullptr, 1);
-      else if (qout && c->k_norm_in)  // wo left x only (below): this launch normalizes and quantizes the row itself
-        launch_k(st, R, k_gateup_k_lds<true, false, true>, dim3(hidden_l / 32), dim3(1024), lds, planes_k(c->gate[l]), planes_k(c->up[l]),
-                 act_k(c->act_dim, dim), (const unsigned short*)dev->exp_table, c->h, hidden_l, dim / 256, hx, (signed char*)c->act_hid,
-                 (float*)(c->act_hid + alh.off_d), (short*)(c->act_hid + alh.off_aux), (signed char*)(c->act_hid + alh.off_p), (const float*)c->x,
-                 (const float*)c->rms_ffn[l]->ptr, 1e-5f, (const float*)c->rsums, dim / 32 <= dev->n_cu ? 2 : 1);
+                 (float*)nullptr, (short*)nullptr, (signed char*)nullptr);
       else if (qout)
         launch_k(st, R, k_gateup_k_lds<true>, dim3(hidden_l / 32), dim3(1024), lds, planes_k(c->gate[l]), planes_k(c->up[l]),
                  act_k(c->act_dim, dim), (const unsigned short*)dev->exp_table, c->h, hidden_l, dim / 256, hx, (signed char*)c->act_hid,
-                 (float*)(c->act_hid + alh.off_d), (short*)(c->act_hid + alh.off_aux), (signed char*)(c->act_hid + alh.off_p), (const float*)nullptr, (const float*)nullptr, 0.f, (const float*)nullptr, 1);
+                 (float*)(c->act_hid + alh.off_d), (short*)(c->act_hid + alh.off_aux), (signed char*)(c->act_hid + alh.off_p));
       else
         launch_k(st, R, k_gateup_k_lds<false>, dim3((hidden_l + 31) / 32), dim3(1024), lds, planes_k(c->gate[l]), planes_k(c->up[l]),
                  act_k(c->act_dim, dim), (const unsigned short*)dev->exp_table, c->h, hidden_l, dim / 256, hx, (signed char*)nullptr,
-                 (float*)nullptr, (short*)nullptr, (signed char*)nullptr, (const float*)nullptr, (const float*)nullptr, 0.f, (const float*)nullptr, 1);
+                 (float*)nullptr, (short*)nullptr, (signed char*)nullptr);
     } else {
       launch_k(st, R, k_gateup<FMT>, dim3((hidden_l + 1) / 2), dim3(128), 0, planes_k(c->gate[l]), planes_k(c->up[l]),
                act_k(c->act_dim, dim), (const unsigned short*)dev->exp_table, c->h, hidden_l, dim / BE);
@@ -1187,7 +1182,106 @@ int enqueue_segment_k(crabml_hip_llama* c, int seg) {
   return 0;
 }
 
+// Q4_K (with Q6_K attn_v / ffn_down: *_K_M files) and Q6_K layers in the fast step: five launches a layer, none of which waits for another's workgroups
+template <bool SIX>
+int enqueue_segment_kq(crabml_hip_llama* c, int seg) {
+  crabml_hip_device* dev = c->dev;
+  hipStream_t st = dev->stream;
+  const auto& g = c->cfg;
+  const int dim = (int)g.embedding_dim, hd = c->hd, kv_dim = c->kv_dim_l, hidden = c->hidden_l, L = (int)g.n_layers, nsb = dim / 256;
+  const bool prof = dev->prof_on && !c->use_graph && !c->capturing;
+  crabml_hip_device::ProfRec pr{};
+  crabml_hip_device::ProfRec* R = prof ? &pr : nullptr;
+  auto P0 = [&](uint32_t stage, double rows, const crabml_hip_buf* w, double k) {
+    return prof ? prof_begin(dev, &pr, w->dtype, stage, rows * k * (double)block_bytes(w->dtype) / 256.0 + 4.0 * k + 4.0 * rows) : 0;
+  };
+  auto P1 = [&]() { return prof ? prof_end(dev, &pr) : 0; };
+  auto mat = [](const crabml_hip_buf* b) { return KqMat{(const char*)b->ptr, b->wl.off_scale}; };
+  auto res = [&](const crabml_hip_buf* w, const float* in, int k, uint32_t stage) -> int {
+    CH_TRY(P0(stage, dim, w, k));
+    const dim3 grid(dim / 16), wg(1024);
+    const size_t lds = kq_lds_bytes(k, false);
+    const KqMat m = mat(w);
+    // (pieces out: as many as a row has a lane, up to four -- of seven 10.0 us with two, 9.5 with four, 11.0 with seven)
+#define CRABML_KQ_RES(SIX_)                                                                                                       \
+  k <= 2048   ? launch_k(st, R, k_kq_res<SIX_, 1, 1>, grid, wg, lds, m, in, k / 256, c->x, c->rsums)                                     \
+  : k <= 4096 ? launch_k(st, R, k_kq_res<SIX_, 1, 2>, grid, wg, lds, m, in, k / 256, c->x, c->rsums)                                     \
+              : launch_k(st, R, k_kq_res<SIX_, 4, 4>, grid, wg, lds, m, in, k / 256, c->x, c->rsums)
+    if (SIX || w->dtype == CRABML_HIP_Q6_K)
+      CRABML_KQ_RES(true);
+    else
+      CRABML_KQ_RES(false);
+#undef CRABML_KQ_RES
+    return P1();
+  };
+  if (seg == 2 * L) {
+    const ActLayout al = act_layout(CRABML_HIP_Q8_K, (size_t)dim);
+    auto norm = [&](auto kernel) {
+      kernel<<<1, 1024, norm_lds_bytes(dim), st>>>(c->x, nullptr, (const float*)c->rms_final->ptr, dim, g.rms_norm_eps, c->xn, c->act_dim, al.total, al.off_d, al.off_aux,
+                                                   al.off_p, 1, nullptr, 0, nullptr, 0, 0);
+    };
+    dim <= 4096 ? norm(k_norm_quant_rows_k<4>) : norm(k_norm_quant_rows_k<12>);
+    if (prof)
+      CH_TRY(prof_begin(dev, &pr, c->output->dtype, 5,
+                        (double)c->vocab_l * (double)(dim / block_elems(c->output->dtype)) * (double)block_bytes(c->output->dtype) + 4.0 * dim + 4.0 * c->vocab_l));
+    CH_TRY(enqueue_classifier_and_sampler(c, c->act_dim, R));
+    return P1();
+  }
+  const int l = seg / 2, rounds = (dim / 32 + 63) / 64;
+  const size_t lds = kq_lds_bytes(dim, false);
+  if ((seg & 1) == 0) {
+    if (l == 0 && !c->led) CH_TRY(enqueue_front(c, false));
+    const QkvEpi e{c->qbuf, c->kc[l], c->vc[l], c->rope, c->state + 1, 1.0f / std::sqrt((float)hd), dim, kv_dim, hd,
+                   (int)g.rope_dim, c->npairs, (int)g.seq_len, g.use_f16_kv_cache != 0 ? 1 : 0};
+    const int pairs = dim / 2 + kv_dim;
+    int nw = (pairs + dev->n_cu - 1) / dev->n_cu;
+    nw = std::min(16, std::max({nw, std::min(nsb, 8), 4}));
+    const dim3 grid((unsigned)((pairs + nw - 1) / nw)), wg(64 * nw);
+    const bool v6 = !SIX && c->wv[l]->dtype == CRABML_HIP_Q6_K;
+    const float* wn = (const float*)c->rms_att[l]->ptr;
+    CH_TRY(P0(1, dim + 2 * kv_dim, c->wq[l], dim));
+    auto go = [&](auto kernel) {
+      launch_k(st, R, kernel, grid, wg, kq_lds_bytes(dim, v6), mat(c->wq[l]), mat(c->wk[l]), mat(c->wv[l]), (const float*)c->x, wn, g.rms_norm_eps, (const float*)c->rsums, nsb, e);
+    };
+    auto by_rows = [&](auto v) {
+      constexpr bool V6 = decltype(v)::value;
+      if (nsb <= nw && rounds <= 2)
+        go(k_kq_qkv<SIX, V6, 1, 2>);
+      else if (nsb <= 2 * nw && rounds <= 2)
+        go(k_kq_qkv<SIX, V6, 2, 2>);
+      else
+        go(k_kq_qkv<SIX, V6, 4, 4>);
+    };
+    if constexpr (SIX)
+      by_rows(std::false_type{});
+    else if (v6)
+      by_rows(std::true_type{});
+    else
+      by_rows(std::false_type{});
+    CH_TRY(P1());
+    enqueue_attention(c, l, nullptr, nullptr, nullptr, PrefetchPlan{}, 0, prof);
+    CH_TRY(res(c->wo[l], c->attn, dim, 2));
+  } else {
+    CH_TRY(P0(3, 2.0 * hidden, c->gate[l], dim));
+    auto go = [&](auto kernel) {
+      launch_k(st, R, kernel, dim3((unsigned)((hidden + 31) / 32)), dim3(1024), lds, mat(c->gate[l]), mat(c->up[l]), (const float*)c->x, (const float*)c->rms_ffn[l]->ptr, 1e-5f,
+               (const float*)c->rsums, nsb, (const unsigned short*)dev->exp_table, c->h, hidden);
+    };
+    if constexpr (SIX)
+      go(k_kq_gateup<SIX, 1, 2>);
+    else if (nsb <= 16)
+      go(k_kq_gateup<SIX, 1, 2>);
+    else
+      go(k_kq_gateup<SIX, 2, 4>);
+    CH_TRY(P1());
+    CH_TRY(res(c->down[l], c->h, hidden, 4));
+  }
+  CH_HIP(dev, hipGetLastError());
+  return 0;
+}
+
 int enqueue_segment(crabml_hip_llama* c, int seg) {
+  if (c->kq) return c->wtype == CRABML_HIP_Q6_K ? enqueue_segment_kq<true>(c, seg) : enqueue_segment_kq<false>(c, seg);
   if (c->kfused)
     return c->wtype == CRABML_HIP_Q4_K ? enqueue_segment_k<CRABML_HIP_Q4_K>(c, seg) : enqueue_segment_k<CRABML_HIP_Q4_1>(c, seg);
   if (c->f16_step) return enqueue_segment_f16(c, seg);
@@ -2527,10 +2621,12 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
   }
   c->q8k_producers = c->norm_epi_k && !(g.flags & (CRABML_HIP_LLAMA_NO_RHS_PROLOGUE | CRABML_HIP_LLAMA_NO_Q8K_PRODUCERS)) && dim_l % 256 == 0 &&
                      hidden_l % 256 == 0 && (hd == 64 || hd == 128 || hd == 256) && (int)(hidden_l / 32) <= 2 * dev->n_cu;
-  // the fast Q4_K step: wo leaves x only, gate | up normalizes and quantizes the row itself (k_gateup_k_lds<.., NORMIN>; the same bits)
-  c->k_norm_in = c->q8k_producers && wt == CRABML_HIP_Q4_K && tp == 1 && !ord && !dev->strict_order && g.embedding_dim % 256 == 0 && g.embedding_dim / 256 <= 32 &&
-                 !(g.flags & (CRABML_HIP_LLAMA_NO_K_NORM_IN | CRABML_HIP_LLAMA_SPLIT_CHUNKS_ALWAYS | CRABML_HIP_LLAMA_SPLIT_CHUNKS_NEVER));
-  if (c->k_norm_in && !c->rsums) A(g.embedding_dim / 16 * 4, (void**)&c->rsums);
+  c->kq = !dev->strict_order && tp == 1 && out_qt == CRABML_HIP_Q8_K && ((wt == CRABML_HIP_Q4_K && c->kfused) || (wt == CRABML_HIP_Q6_K && !mixed)) &&
+          // (wider rows of Q6_K: more than the 64 registers that gate | up's two workgroups a CU have)
+          g.embedding_dim % 256 == 0 && g.embedding_dim <= (wt == CRABML_HIP_Q6_K ? 4096 : 8192) && hidden_l % 256 == 0 && kq_lds_bytes((int)hidden_l, false) <= 60 * 1024 &&
+          !(g.flags & (CRABML_HIP_LLAMA_NO_K_NORM_IN | CRABML_HIP_LLAMA_NO_KQUANT_FUSION | CRABML_HIP_LLAMA_NO_NORM_EPILOGUE | CRABML_HIP_LLAMA_NO_RHS_PROLOGUE |
+                       CRABML_HIP_LLAMA_NO_Q8K_PRODUCERS | CRABML_HIP_LLAMA_Q8K_ATTN_PRODUCER | CRABML_HIP_LLAMA_SPLIT_CHUNKS_ALWAYS | CRABML_HIP_LLAMA_SPLIT_CHUNKS_NEVER));
+  if (c->kq && !c->rsums) A(g.embedding_dim / 16 * 4, (void**)&c->rsums);
   if (c->q8k_producers) {
     A(dim_l * 8, (void**)&c->a8gran);
     A(hidden_l * 8, (void**)&c->h8gran);

@@ -102,9 +102,9 @@ __device__ __forceinline__ void q8k_exchange_store(const Q8KExchange& ex, const 
     }
   }
   const Q8KLane o = q8k_wave_quant(v, lane);
+  q8k_store_class_major(oqp + sb * 256, lane, o.packed, mine);
   if (mine) {
     ((unsigned*)oq)[sb * 64 + lane] = o.packed;
-    q8k_store_class_major(oqp + sb * 256, lane, o.packed);
     if ((lane & 3) == 0) obs[sb * 16 + (lane >> 2)] = (short)o.quad_sum;
   }
   if (lane == 0 && first == sb * 256) od[sb] = o.d;
@@ -251,7 +251,7 @@ __global__ __launch_bounds__(1024) void k_norm_f32(float* __restrict__ x, const 
 // Inside a graph of several steps (run_steps) it runs at the END of a step, for the next one; a graph's first step runs it without the partials.
 // With several steps in a graph (run_steps), us a request, before -> after: 57 tokens of the 15M-parameter model in Q8_0 6482 -> 6047, 88 tokens of 8
 // layers of the 8B shape in Q4_0 24840 -> 24232.
-enum { FRONT_ROW = 0, FRONT_Q8_0 = 1, FRONT_Q8_1 = 2, FRONT_Q8_K = 3 };  // what is left beside x: nothing, or the normed row's planes
+enum { FRONT_ROW = 0, FRONT_Q8_0 = 1, FRONT_Q8_1 = 2, FRONT_Q8_K = 3, FRONT_SUMS = 4 };  // what is left beside x: nothing, the normed row's planes, sums of squares of 16
 struct TokenPick {  // pv == nullptr: the token is *token
   const float* pv = nullptr;
   const int* pi = nullptr;
@@ -293,11 +293,11 @@ __device__ __forceinline__ void embed_row(const char* __restrict__ w, int dtype,
 template <int NIT, int FRONT>
 __global__ __launch_bounds__(1024) void k_step_front(const char* __restrict__ table, int dtype, size_t off_scale, TokenPick pick, int dim, float* __restrict__ x,
                                                      const float* __restrict__ wn, float eps, FrontOut o, int half) {
-  extern __shared__ float lds[];
+  extern __shared__ __attribute__((aligned(16))) float lds[];
   __shared__ float s_rms;
   const int tid = threadIdx.x, lane = tid & 63;
   float xv[NIT], wv[NIT];
-  if constexpr (FRONT != FRONT_ROW) {
+  if constexpr (FRONT != FRONT_ROW && FRONT != FRONT_SUMS) {
 #pragma unroll
     for (int it = 0; it < NIT; it++) wv[it] = it * 1024 + tid < dim ? wn[it * 1024 + tid] : 0.f;
   }
@@ -324,6 +324,24 @@ __global__ __launch_bounds__(1024) void k_step_front(const char* __restrict__ ta
   for (int it = 0; it < NIT; it++)
     if (it * 1024 + tid < dim) x[it * 1024 + tid] = xv[it];
   NormLds L{lds, lds + dim};
+  if constexpr (FRONT == FRONT_SUMS) {  // (the halves of norm_quant_regs' chunks, as k_kq_res leaves them)
+#pragma unroll
+    for (int it = 0; it < NIT; it++)
+      if (it * 1024 + tid < dim) lds[it * 1024 + tid] = xv[it];
+    __syncthreads();
+    for (int i = tid; i < dim / 16; i += 1024) {
+      float s = -0.0f;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const f32x4 t = ((const f32x4*)lds)[i * 4 + j];
+        s += t[0] * t[0];
+        s += t[1] * t[1];
+        s += t[2] * t[2];
+        s += t[3] * t[3];
+      }
+      ((float*)o.d)[i] = s;
+    }
+  }
   if constexpr (FRONT == FRONT_Q8_0 || FRONT == FRONT_Q8_1)
     norm_quant_regs<NIT, true, FRONT == FRONT_Q8_1>(xv, wv, dim, eps, L, &s_rms, o.q, (unsigned short*)o.d, o.aux, nullptr, half);
   if constexpr (FRONT == FRONT_Q8_K) {

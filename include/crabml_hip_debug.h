@@ -148,8 +148,8 @@ int crabml_hip_debug_flash_attention_rows(crabml_hip_device_t* dev, const float*
                                                          of them (bit-identical) */
 #define CRABML_HIP_LLAMA_PREFILL_NO_GU_EPILOGUE 67108864 /* A/B, fast prompt pass: gate | up leave g and u and SiLU * mul (+ quantize) stays its own
                                                            launch, instead of being the f16 GEMM's epilogue (bit-identical) */
-#define CRABML_HIP_LLAMA_NO_K_NORM_IN 16777216 /* A/B, fast Q4_K step: wo gathers the row's sums and quantizes its output to Q8_K itself (two
-                                                  in-launch hops) instead of leaving x for gate | up to normalize and quantize (bit-identical) */
+#define CRABML_HIP_LLAMA_NO_K_NORM_IN 16777216 /* A/B, fast Q4_K / Q6_K step: the launches that produce a row leave its Q8_K planes (in-launch hops; Q6_K:
+                                                  per-op launches) instead of f32 rows that the reading launch normalizes and quantizes (bit-identical) */
 #define CRABML_HIP_LLAMA_SPLIT_CHUNKS_ALWAYS 16 /* test / tuning hooks for the norm epilogue: two workgroups per */
 #define CRABML_HIP_LLAMA_SPLIT_CHUNKS_NEVER 32  /* 32-row chunk always / never (default: only for long rows)   */
 

@@ -458,6 +458,25 @@ def test_q4_k_m_mix_on_the_fused_kernels_equals_the_per_op_segments(ca, flags):
     assert list(fused.decode_greedy(3, 20)) == list(per_op.decode_greedy(3, 20))
 
 
+# width, hidden, heads, kv heads: a super-block; one, two and four of them a wave of q | k | v, and rounds of 64 chunk sums likewise; ffn_down's rows of one piece a lane,
+# two, four, and more super-blocks than four a wave; a last workgroup of q | k | v that the rows do not fill
+@pytest.mark.parametrize("dim,hidden,heads,kv", [(256, 16640, 4, 2), (512, 256, 8, 1), (2048, 2304, 16, 5), (2304, 4096, 18, 3), (4096, 4352, 32, 8), (4352, 512, 34, 17), (8192, 1024, 64, 8)])
+@pytest.mark.parametrize("fmt", ["Q4_K", "Q6_K", "mix"])
+def test_k_quant_step_equals_the_per_op_segments(ca, fmt, dim, hidden, heads, kv):
+    """Q4_K, Q6_K and *_K_M layers whose launches quantize their rhs themselves: the logits of the per-op launches (flag 256), bit for bit."""
+    if heads % kv:
+        kv = 1
+    shape = synth.ModelShape("kq", dim, hidden, 2, heads, kv, 512, 64)
+    model = synth.build_model(shape, synth.Q6_K if fmt == "Q6_K" else synth.Q4_K, seed=dim + hidden, k_m_mix=fmt == "mix")
+    dev = ca.HipTensorDevice(0)
+    conf, w = synth.to_hip(model, dev)
+    fused, per_op = ca.HipLlamaRunner(conf, w, dev, 64, True), ca.HipLlamaRunner(conf, w, dev, 64, True, extra_flags=256)
+    for i, t in enumerate(PROMPT):
+        a, b = fused.forward(t % 512, i), per_op.forward(t % 512, i)
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), f"step {i}"
+    assert list(fused.decode_greedy(3, 12)) == list(per_op.decode_greedy(3, 12))
+
+
 @pytest.mark.parametrize("n_kv,hd", [(8, 128), (2, 128), (1, 128), (8, 64), (4, 64), (1, 64)])
 def test_flash_attention_tracks_the_exact_long_context_kernels(ca, n_kv, hd):
     """The fast step's default long-context attention (k_attn_flash: split-KV, f32 exp and accumulation, last-arriver merge)
