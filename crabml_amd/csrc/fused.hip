@@ -783,7 +783,7 @@ int enqueue_segment_t(crabml_hip_llama* c, int seg) {
     const RmsTail rtq{c->rsums, dim / 32, 1.0f / (float)dim, g.rms_norm_eps};
     if (c->ord)
       launch_k(st, R, k_qkv_ord<FMT>, dim3((total_rows / 2 + 3) / 4), dim3(256), (size_t)8 * ((dim / 32 + 3) & ~3) * sizeof(float), planes_of(c->wq[l]),
-               planes_of(c->wk[l]), planes_of(c->wv[l]), act_view<FMT>(ad), dim / 32, e, Planes6{nullptr, 0});
+               planes_of(c->wk[l]), planes_of(c->wv[l]), act_view<FMT>(ad), dim / 32, e);
     else if (defer_down && l > 0) {
       if constexpr (!Q81)
         launch_k(st, R, k_qkv<FMT, true>, dim3((total_rows / 2 + 1) / 2), dim3(128), 0, planes_of(c->wq[l]), planes_of(c->wk[l]),
@@ -1034,9 +1034,6 @@ int enqueue_segment_k(crabml_hip_llama* c, int seg) {
   };
   float* dst = tp ? c->partial : c->x;
   const bool nepi = FMT == CRABML_HIP_Q4_K && c->norm_epi_k;
-  // strict-order device, Q4_K layers (c->ord): the same five launches with every sum in the reference's order -- nine-term records per
-  // super-block added in order (q4k_class_terms / q4k_ordered_sum, gemv_core.hpp), the reference's norm order in the epilogue
-  const bool ordk = FMT == CRABML_HIP_Q4_K && c->ord;
   // wnext / eps_next: the RMSNorm that consumes this GEMV's output (norm epilogue only)
   // the rhs of wo / ffn_down quantized by the consuming kernel itself (no quantizer launch)
   const bool qin = nepi && !(g.flags & CRABML_HIP_LLAMA_NO_RHS_PROLOGUE) && dim_l % 256 == 0 && hidden_l % 256 == 0;
@@ -1059,22 +1056,6 @@ int enqueue_segment_k(crabml_hip_llama* c, int seg) {
                           : (k / 32 >= 256 && dim / 32 <= dev->n_cu)        ? 2
                                                                             : 1;
         const size_t lds = (size_t)k + (size_t)(k / 256) * 4 + (size_t)(k / 16) * 2;
-        if (ordk) {  // (qmode is 1 or 2 here: `qin` holds on every ordered context)
-          const size_t ldso = ((lds + 15) & ~(size_t)15) + (size_t)(32 / split) * (size_t)q4k_rec_stride(k / 256) * sizeof(float);
-#define CRABML_NQ_KO(SPLIT_, QIN_, GRID_)                                                                                                \
-  launch_k(st, R, k_gemv_res_nq<FMT, SPLIT_, QIN_, false, false, true>, dim3(GRID_), dim3(1024), ldso, planes_k(w), a, xin, c->x, wnext, \
-           eps_next, oq, od, ob, ng, k / BE, six(w), NoTp{})
-          if (split == 2 && qmode == 2)
-            CRABML_NQ_KO(2, 2, dim / 16);
-          else if (split == 2)
-            CRABML_NQ_KO(2, 1, dim / 16);
-          else if (qmode == 2)
-            CRABML_NQ_KO(1, 2, dim / 32);
-          else
-            CRABML_NQ_KO(1, 1, dim / 32);
-#undef CRABML_NQ_KO
-          return P1();
-        }
 #define CRABML_NQ_K(SPLIT_, QIN_, GRID_, LDS_)                                                                                          \
   launch_k(st, R, k_gemv_res_nq<FMT, SPLIT_, QIN_>, dim3(GRID_), dim3(1024), LDS_, planes_k(w), a, xin, c->x, wnext, eps_next, oq, od, ob, \
            ng, k / BE, six(w), NoTp{})
@@ -1122,12 +1103,8 @@ int enqueue_segment_k(crabml_hip_llama* c, int seg) {
              (int)g.rope_dim, c->npairs, seq_cap, kv16 ? 1 : 0};
     const int total_rows = dim_l + 2 * kv_dim_l;
     CH_TRY(P0(1, total_rows, dim));
-    if (ordk)
-      launch_k(st, R, k_qkv_ord<FMT>, dim3((total_rows / 2 + 3) / 4), dim3(256), (size_t)8 * (size_t)q4k_rec_stride(dim / BE) * sizeof(float),
-               planes_k(c->wq[l]), planes_k(c->wk[l]), planes_k(c->wv[l]), act_k(c->act_dim, dim), dim / BE, e, six(c->wv[l]));
-    else
-      launch_k(st, R, k_qkv<FMT>, dim3((total_rows / 2 + 1) / 2), dim3(128), 0, planes_k(c->wq[l]), planes_k(c->wk[l]),
-               planes_k(c->wv[l]), act_k(c->act_dim, dim), dim / BE, e, six(c->wv[l]), RmsTail{nullptr, 0, 0.f, 0.f}, 0);
+    launch_k(st, R, k_qkv<FMT>, dim3((total_rows / 2 + 1) / 2), dim3(128), 0, planes_k(c->wq[l]), planes_k(c->wk[l]),
+             planes_k(c->wv[l]), act_k(c->act_dim, dim), dim / BE, e, six(c->wv[l]), RmsTail{nullptr, 0, 0.f, 0.f}, 0);
     CH_TRY(P1());
     // Q8_K producers: the (short-context) attention kernel assembles the planes of wo's rhs itself; wo copies them
     const bool aq8 = qout && (g.flags & CRABML_HIP_LLAMA_Q8K_ATTN_PRODUCER) && c->attn_variant == 0 && c->attn_s_rows > 0;
@@ -1152,16 +1129,7 @@ int enqueue_segment_k(crabml_hip_llama* c, int seg) {
       const size_t lds = (size_t)dim + (size_t)(dim / 256) * 4 + (size_t)(dim / 16) * 2;
       const ActLayout alh = act_layout(QT, (size_t)hidden_l);
       const Q8KExchange hx{c->h8gran, c->state + 4, c->state + 5, n_segments(c), seg};
-      const size_t ldso = ((lds + 15) & ~(size_t)15) + (size_t)64 * (size_t)q4k_rec_stride(dim / 256) * sizeof(float);
-      if (ordk && qout)
-        launch_k(st, R, k_gateup_k_lds<true, true>, dim3(hidden_l / 32), dim3(1024), ldso, planes_k(c->gate[l]), planes_k(c->up[l]),
-                 act_k(c->act_dim, dim), (const unsigned short*)dev->exp_table, c->h, hidden_l, dim / 256, hx, (signed char*)c->act_hid,
-                 (float*)(c->act_hid + alh.off_d), (short*)(c->act_hid + alh.off_aux), (signed char*)(c->act_hid + alh.off_p));
-      else if (ordk)
-        launch_k(st, R, k_gateup_k_lds<false, true>, dim3(hidden_l / 32), dim3(1024), ldso, planes_k(c->gate[l]), planes_k(c->up[l]),
-                 act_k(c->act_dim, dim), (const unsigned short*)dev->exp_table, c->h, hidden_l, dim / 256, hx, (signed char*)nullptr,
-                 (float*)nullptr, (short*)nullptr, (signed char*)nullptr);
-      else if (qout)
+      if (qout)
         launch_k(st, R, k_gateup_k_lds<true>, dim3(hidden_l / 32), dim3(1024), lds, planes_k(c->gate[l]), planes_k(c->up[l]),
                  act_k(c->act_dim, dim), (const unsigned short*)dev->exp_table, c->h, hidden_l, dim / 256, hx, (signed char*)c->act_hid,
                  (float*)(c->act_hid + alh.off_d), (short*)(c->act_hid + alh.off_aux), (signed char*)(c->act_hid + alh.off_p));
@@ -1182,8 +1150,11 @@ int enqueue_segment_k(crabml_hip_llama* c, int seg) {
   return 0;
 }
 
-// Q4_K (with Q6_K attn_v / ffn_down: *_K_M files) and Q6_K layers in the fast step: five launches a layer, none of which waits for another's workgroups
-template <bool SIX>
+// flags that ask for other launches than enqueue_segment_kq's
+constexpr uint64_t KQ_NOT = CRABML_HIP_LLAMA_NO_K_NORM_IN | CRABML_HIP_LLAMA_NO_KQUANT_FUSION | CRABML_HIP_LLAMA_NO_NORM_EPILOGUE | CRABML_HIP_LLAMA_NO_RHS_PROLOGUE |
+                            CRABML_HIP_LLAMA_NO_Q8K_PRODUCERS | CRABML_HIP_LLAMA_Q8K_ATTN_PRODUCER | CRABML_HIP_LLAMA_SPLIT_CHUNKS_ALWAYS | CRABML_HIP_LLAMA_SPLIT_CHUNKS_NEVER;
+// Q4_K (with Q6_K attn_v / ffn_down: *_K_M files) and Q6_K layers: five launches a layer, none of which waits for another's workgroups.  ORD: the strict-order device's sums
+template <bool SIX, bool ORD>
 int enqueue_segment_kq(crabml_hip_llama* c, int seg) {
   crabml_hip_device* dev = c->dev;
   hipStream_t st = dev->stream;
@@ -1200,13 +1171,13 @@ int enqueue_segment_kq(crabml_hip_llama* c, int seg) {
   auto res = [&](const crabml_hip_buf* w, const float* in, int k, uint32_t stage) -> int {
     CH_TRY(P0(stage, dim, w, k));
     const dim3 grid(dim / 16), wg(1024);
-    const size_t lds = kq_lds_bytes(k, false);
+    const size_t lds = ORD ? kq_rec_at(k, false) + kq_rec_bytes(16, k / 256, false) : kq_lds_bytes(k, false);
     const KqMat m = mat(w);
-    // (pieces out: as many as a row has a lane, up to four -- of seven 10.0 us with two, 9.5 with four, 11.0 with seven)
+    // (pieces out: as many as a row has a lane, up to four -- of seven 9.6 us with two, 9.0 with four, 10.5 with seven)
 #define CRABML_KQ_RES(SIX_)                                                                                                       \
-  k <= 2048   ? launch_k(st, R, k_kq_res<SIX_, 1, 1>, grid, wg, lds, m, in, k / 256, c->x, c->rsums)                                     \
-  : k <= 4096 ? launch_k(st, R, k_kq_res<SIX_, 1, 2>, grid, wg, lds, m, in, k / 256, c->x, c->rsums)                                     \
-              : launch_k(st, R, k_kq_res<SIX_, 4, 4>, grid, wg, lds, m, in, k / 256, c->x, c->rsums)
+  k <= 2048   ? launch_k(st, R, k_kq_res<SIX_, 1, 1, ORD>, grid, wg, lds, m, in, k / 256, c->x, c->rsums)                                     \
+  : k <= 4096 ? launch_k(st, R, k_kq_res<SIX_, 1, 2, ORD>, grid, wg, lds, m, in, k / 256, c->x, c->rsums)                                     \
+              : launch_k(st, R, k_kq_res<SIX_, 4, 4, ORD>, grid, wg, lds, m, in, k / 256, c->x, c->rsums)
     if (SIX || w->dtype == CRABML_HIP_Q6_K)
       CRABML_KQ_RES(true);
     else
@@ -1218,7 +1189,7 @@ int enqueue_segment_kq(crabml_hip_llama* c, int seg) {
     const ActLayout al = act_layout(CRABML_HIP_Q8_K, (size_t)dim);
     auto norm = [&](auto kernel) {
       kernel<<<1, 1024, norm_lds_bytes(dim), st>>>(c->x, nullptr, (const float*)c->rms_final->ptr, dim, g.rms_norm_eps, c->xn, c->act_dim, al.total, al.off_d, al.off_aux,
-                                                   al.off_p, 1, nullptr, 0, nullptr, 0, 0);
+                                                   al.off_p, ORD ? 0 : 1, nullptr, 0, nullptr, 0, 0);
     };
     dim <= 4096 ? norm(k_norm_quant_rows_k<4>) : norm(k_norm_quant_rows_k<12>);
     if (prof)
@@ -1228,34 +1199,29 @@ int enqueue_segment_kq(crabml_hip_llama* c, int seg) {
     return P1();
   }
   const int l = seg / 2, rounds = (dim / 32 + 63) / 64;
-  const size_t lds = kq_lds_bytes(dim, false);
   if ((seg & 1) == 0) {
     if (l == 0 && !c->led) CH_TRY(enqueue_front(c, false));
     const QkvEpi e{c->qbuf, c->kc[l], c->vc[l], c->rope, c->state + 1, 1.0f / std::sqrt((float)hd), dim, kv_dim, hd,
                    (int)g.rope_dim, c->npairs, (int)g.seq_len, g.use_f16_kv_cache != 0 ? 1 : 0};
     const int pairs = dim / 2 + kv_dim;
-    int nw = (pairs + dev->n_cu - 1) / dev->n_cu;
-    nw = std::min(16, std::max({nw, std::min(nsb, 8), 4}));
+    const int nw = std::min(16, std::max({(pairs + dev->n_cu - 1) / dev->n_cu, (nsb + 1) / 2, std::min(nsb, 8), 4}));
     const dim3 grid((unsigned)((pairs + nw - 1) / nw)), wg(64 * nw);
     const bool v6 = !SIX && c->wv[l]->dtype == CRABML_HIP_Q6_K;
     const float* wn = (const float*)c->rms_att[l]->ptr;
+    const size_t lds = ORD ? kq_rec_at(dim, v6) + kq_rec_bytes(2 * nw, nsb, true) : kq_lds_bytes(dim, v6);
     CH_TRY(P0(1, dim + 2 * kv_dim, c->wq[l], dim));
     auto go = [&](auto kernel) {
-      launch_k(st, R, kernel, grid, wg, kq_lds_bytes(dim, v6), mat(c->wq[l]), mat(c->wk[l]), mat(c->wv[l]), (const float*)c->x, wn, g.rms_norm_eps, (const float*)c->rsums, nsb, e);
+      launch_k(st, R, kernel, grid, wg, lds, mat(c->wq[l]), mat(c->wk[l]), mat(c->wv[l]), (const float*)c->x, wn, g.rms_norm_eps, (const float*)c->rsums, nsb, e);
     };
     auto by_rows = [&](auto v) {
       constexpr bool V6 = decltype(v)::value;
       if (nsb <= nw && rounds <= 2)
-        go(k_kq_qkv<SIX, V6, 1, 2>);
-      else if (nsb <= 2 * nw && rounds <= 2)
-        go(k_kq_qkv<SIX, V6, 2, 2>);
+        go(k_kq_qkv<SIX, V6, 1, 2, ORD>);
       else
-        go(k_kq_qkv<SIX, V6, 4, 4>);
+        go(k_kq_qkv<SIX, V6, 2, 4, ORD>);
     };
-    if constexpr (SIX)
-      by_rows(std::false_type{});
-    else if (v6)
-      by_rows(std::true_type{});
+    if (v6)
+      by_rows(std::bool_constant<!SIX>{});
     else
       by_rows(std::false_type{});
     CH_TRY(P1());
@@ -1263,16 +1229,17 @@ int enqueue_segment_kq(crabml_hip_llama* c, int seg) {
     CH_TRY(res(c->wo[l], c->attn, dim, 2));
   } else {
     CH_TRY(P0(3, 2.0 * hidden, c->gate[l], dim));
+    const size_t lds = ORD ? kq_rec_at(dim, false) + kq_rec_bytes(64, nsb, true) : kq_lds_bytes(dim, false);
     auto go = [&](auto kernel) {
       launch_k(st, R, kernel, dim3((unsigned)((hidden + 31) / 32)), dim3(1024), lds, mat(c->gate[l]), mat(c->up[l]), (const float*)c->x, (const float*)c->rms_ffn[l]->ptr, 1e-5f,
                (const float*)c->rsums, nsb, (const unsigned short*)dev->exp_table, c->h, hidden);
     };
     if constexpr (SIX)
-      go(k_kq_gateup<SIX, 1, 2>);
+      go(k_kq_gateup<SIX, 1, 2, ORD>);
     else if (nsb <= 16)
-      go(k_kq_gateup<SIX, 1, 2>);
+      go(k_kq_gateup<SIX, 1, 2, ORD>);
     else
-      go(k_kq_gateup<SIX, 2, 4>);
+      go(k_kq_gateup<SIX, 2, 4, ORD>);
     CH_TRY(P1());
     CH_TRY(res(c->down[l], c->h, hidden, 4));
   }
@@ -1281,7 +1248,7 @@ int enqueue_segment_kq(crabml_hip_llama* c, int seg) {
 }
 
 int enqueue_segment(crabml_hip_llama* c, int seg) {
-  if (c->kq) return c->wtype == CRABML_HIP_Q6_K ? enqueue_segment_kq<true>(c, seg) : enqueue_segment_kq<false>(c, seg);
+  if (c->kq) return c->ord ? enqueue_segment_kq<false, true>(c, seg) : c->wtype == CRABML_HIP_Q6_K ? enqueue_segment_kq<true, false>(c, seg) : enqueue_segment_kq<false, false>(c, seg);
   if (c->kfused)
     return c->wtype == CRABML_HIP_Q4_K ? enqueue_segment_k<CRABML_HIP_Q4_K>(c, seg) : enqueue_segment_k<CRABML_HIP_Q4_1>(c, seg);
   if (c->f16_step) return enqueue_segment_f16(c, seg);
@@ -2360,33 +2327,20 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
     generic = true;
   }
   generic = generic || (mixed && !mix_fused);
-  // strict order, pure Q4_K layers on one device (round 6): the five fused launches of the fast Q4_K step in their ORDERED form -- nine
-  // f32 terms per super-block (eight exact class sums x d, and dmin x sumi) parked in LDS and added in super-block order, the
-  // reference's norm order in the wo / ffn_down epilogue (k_qkv_ord, k_gemv_res_nq<.., ORD>, k_gateup_k_lds<.., ORD>); bit-identical
-  // to the per-op segments they replace (16 launches per layer).  The term tables must fit LDS.
-  // (a *_K_M mix too: its Q6_K attn_v / ffn_down rows leave the same records, rows_terms_q6k)
-  bool ordk = dev->strict_order && wt == CRABML_HIP_Q4_K && (!mixed || mix_v_down_q6k) && out_qt == CRABML_HIP_Q8_K && tp == 1 &&
-              !(g.flags & (CRABML_HIP_LLAMA_NO_NORM_EPILOGUE | CRABML_HIP_LLAMA_NO_KQUANT_FUSION | CRABML_HIP_LLAMA_NO_RHS_PROLOGUE)) &&
-              g.embedding_dim % 256 == 0 && dim_l % 256 == 0 && hidden_l % 256 == 0 && (int)(g.embedding_dim / 32) <= dev->n_cu;
+  // strict order, Q4_K layers on one device (a *_K_M mix too): the five launches of the fast K-quant step with every sum in the reference's order (fused_kquant.hpp, ORD),
+  // bit-identical to the per-op segments (16 launches per layer).  The records must fit LDS.
+  bool ordk = dev->strict_order && wt == CRABML_HIP_Q4_K && (!mixed || mix_v_down_q6k) && out_qt == CRABML_HIP_Q8_K && tp == 1 && !(g.flags & KQ_NOT) &&
+              g.embedding_dim % 256 == 0 && hidden_l % 256 == 0 && g.embedding_dim <= 8192;
   if (ordk && !dry) {
-    auto planes_b = [](size_t k) { return ((k + k / 256 * 4 + k / 16 * 2) + 15) & ~(size_t)15; };
-    const int split_dn = (g.flags & CRABML_HIP_LLAMA_SPLIT_CHUNKS_ALWAYS) ? 2 : (g.flags & CRABML_HIP_LLAMA_SPLIT_CHUNKS_NEVER) ? 1 : hidden_l / 32 >= 256 ? 2 : 1;
-    const int split_wo = (g.flags & CRABML_HIP_LLAMA_SPLIT_CHUNKS_ALWAYS) ? 2 : (g.flags & CRABML_HIP_LLAMA_SPLIT_CHUNKS_NEVER) ? 1 : dim_l / 32 >= 256 ? 2 : 1;
-    const size_t gu = planes_b(g.embedding_dim) + (size_t)64 * (size_t)q4k_rec_stride((int)(g.embedding_dim / 256)) * 4;
-    const size_t dn = planes_b(hidden_l) + (size_t)(32 / split_dn) * (size_t)q4k_rec_stride((int)(hidden_l / 256)) * 4;
-    const size_t wo = planes_b(dim_l) + (size_t)(32 / split_wo) * (size_t)q4k_rec_stride((int)(dim_l / 256)) * 4;
-    const size_t nq = dn > wo ? dn : wo;
-    bool fits = gu <= 150 * 1024 && nq <= 150 * 1024;
-    if (fits && gu > 48 * 1024)
-      fits = raise_dyn_lds(dev, (const void*)k_gateup_k_lds<true, true>, (int)gu) == hipSuccess &&
-             raise_dyn_lds(dev, (const void*)k_gateup_k_lds<false, true>, (int)gu) == hipSuccess;
-    if (fits && nq > 48 * 1024)
-      fits = raise_dyn_lds(dev, (const void*)k_gemv_res_nq<CRABML_HIP_Q4_K, 1, 1, false, false, true>, (int)nq) == hipSuccess &&
-             raise_dyn_lds(dev, (const void*)k_gemv_res_nq<CRABML_HIP_Q4_K, 1, 2, false, false, true>, (int)nq) == hipSuccess &&
-             raise_dyn_lds(dev, (const void*)k_gemv_res_nq<CRABML_HIP_Q4_K, 2, 1, false, false, true>, (int)nq) == hipSuccess &&
-             raise_dyn_lds(dev, (const void*)k_gemv_res_nq<CRABML_HIP_Q4_K, 2, 2, false, false, true>, (int)nq) == hipSuccess;
+    auto bytes = [](int rows, size_t k, bool norm, bool both) { return (int)(kq_rec_at((int)k, both) + kq_rec_bytes(rows, (int)k / 256, norm)); };
+    const int gu = bytes(64, g.embedding_dim, true, false), in = bytes(32, g.embedding_dim, true, true),
+              rs = std::max(bytes(16, g.embedding_dim, false, false), bytes(16, hidden_l, false, false));
+    auto room = [&](auto kernel, int n) { return n <= 150 * 1024 && (n <= 48 * 1024 || raise_dyn_lds(dev, (const void*)kernel, n) == hipSuccess); };
+    ordk = room(k_kq_gateup<false, 1, 2, true>, gu) && room(k_kq_gateup<false, 2, 4, true>, gu) && room(k_kq_qkv<false, false, 1, 2, true>, in) &&
+           room(k_kq_qkv<false, false, 2, 4, true>, in) && room(k_kq_qkv<false, true, 1, 2, true>, in) && room(k_kq_qkv<false, true, 2, 4, true>, in) &&
+           room(k_kq_res<false, 1, 1, true>, rs) && room(k_kq_res<false, 1, 2, true>, rs) && room(k_kq_res<false, 4, 4, true>, rs) &&
+           room(k_kq_res<true, 1, 1, true>, rs) && room(k_kq_res<true, 1, 2, true>, rs) && room(k_kq_res<true, 4, 4, true>, rs);
     (void)hipGetLastError();
-    if (!fits) ordk = false;
   }
   if (ordk) ord = true;
   if (ordk && mixed) generic = false;
@@ -2621,11 +2575,10 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
   }
   c->q8k_producers = c->norm_epi_k && !(g.flags & (CRABML_HIP_LLAMA_NO_RHS_PROLOGUE | CRABML_HIP_LLAMA_NO_Q8K_PRODUCERS)) && dim_l % 256 == 0 &&
                      hidden_l % 256 == 0 && (hd == 64 || hd == 128 || hd == 256) && (int)(hidden_l / 32) <= 2 * dev->n_cu;
-  c->kq = !dev->strict_order && tp == 1 && out_qt == CRABML_HIP_Q8_K && ((wt == CRABML_HIP_Q4_K && c->kfused) || (wt == CRABML_HIP_Q6_K && !mixed)) &&
-          // (wider rows of Q6_K: more than the 64 registers that gate | up's two workgroups a CU have)
-          g.embedding_dim % 256 == 0 && g.embedding_dim <= (wt == CRABML_HIP_Q6_K ? 4096 : 8192) && hidden_l % 256 == 0 && kq_lds_bytes((int)hidden_l, false) <= 60 * 1024 &&
-          !(g.flags & (CRABML_HIP_LLAMA_NO_K_NORM_IN | CRABML_HIP_LLAMA_NO_KQUANT_FUSION | CRABML_HIP_LLAMA_NO_NORM_EPILOGUE | CRABML_HIP_LLAMA_NO_RHS_PROLOGUE |
-                       CRABML_HIP_LLAMA_NO_Q8K_PRODUCERS | CRABML_HIP_LLAMA_Q8K_ATTN_PRODUCER | CRABML_HIP_LLAMA_SPLIT_CHUNKS_ALWAYS | CRABML_HIP_LLAMA_SPLIT_CHUNKS_NEVER));
+  // (wider rows of Q6_K: more than the 64 registers that gate | up's two workgroups a CU have)
+  c->kq = ordk || (!dev->strict_order && tp == 1 && out_qt == CRABML_HIP_Q8_K && ((wt == CRABML_HIP_Q4_K && c->kfused) || (wt == CRABML_HIP_Q6_K && !mixed)) &&
+                   g.embedding_dim % 256 == 0 && g.embedding_dim <= (wt == CRABML_HIP_Q6_K ? 4096 : 8192) && hidden_l % 256 == 0 &&
+                   kq_lds_bytes((int)hidden_l, false) <= 60 * 1024 && !(g.flags & KQ_NOT));
   if (c->kq && !c->rsums) A(g.embedding_dim / 16 * 4, (void**)&c->rsums);
   if (c->q8k_producers) {
     A(dim_l * 8, (void**)&c->a8gran);

@@ -7,8 +7,9 @@
 // wave per super-block and some 60 instructions (q8k_wave_quant).  Bound: the weights' bytes, plus a launch's ramp.
 // Every row's pieces are added by lane, ascending, as k_gemv_q4_k / k_gemv_q6_k add them, the norm's sums in k_norm_f32's order: the planes and logits are the per-op
 // launches' bit for bit.
-// Us a launch of the 8B shape, Q4_K, with planes from the producer / these: q | k | v 5.6 / 6.2, wo 5.6 / 5.2, gate | up 16.6 / 13.6 (4.9 TB/s), ffn_down 11.2 / 9.5; a token of
-// four layers 268 -> 250, of Q6_K (fourteen launches a layer and the attention before) 405 -> 333; width 2048, six layers, Q4_K 222 -> 205, Q6_K 367 -> 255.
+// Us a launch of the 8B shape, Q4_K, with planes from the producer / these: q | k | v 5.6 / 5.8, wo 5.6 / 4.4, gate | up 16.6 / 13.7 (4.8 TB/s), ffn_down 11.2 / 9.0; on the
+// strict-order device (ORD) 6.5 / 9.4, 10.7 / 5.6, 19.0 / 18.0, 16.2 / 13.3.  A token of four layers 269 -> 242, of Q6_K (fourteen launches a layer and the attention before)
+// 407 -> 297; width 2048, six layers, Q4_K 222 -> 192, Q6_K 363 -> 214.
 #pragma once
 #include "fused_ffn.hpp"
 
@@ -135,14 +136,81 @@ __device__ __forceinline__ void kq_norm_request(KqNorm<U, R>& n, const float* __
     n.w[u] = ((const f32x4*)w)[sb * 64 + lane];
   }
 }
+// ORD (strict-order device): rms_norm.rs:35-40's own order -- a chunk's 32 squares as one scan from -0.0, the chunks' sums one after the other.  The first half of every scan comes
+// with x (csums); the row goes to LDS (t, in front of the records; chunks 36 floats apart: lanes read their chunks' 16-byte pieces from different banks) and one wave goes on with
+// the second halves, a lane a chunk, and adds the sums lane by lane.
+inline __host__ __device__ size_t kq_ord_bytes(int nsb) { return (size_t)nsb * 8 * 36 * 4; }
 template <int U, int R>
-__device__ __forceinline__ void kq_norm_quant(KqNorm<U, R>& n, const KqLds& l, float eps, int nsb, int lane, int wave, int nw) {
+__device__ __forceinline__ float kq_ordered_rms(KqNorm<U, R>& n, float* __restrict__ t, float eps, int nsb, int lane, int wave, int nw) {
+  __shared__ __attribute__((aligned(16))) float s_chunk[64 * R];
+  __shared__ float s_rms;
+  const int nch = nsb * 8;
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    const int sb = wave + u * nw;
+    if (sb < nsb) *(f32x4*)(t + (sb * 8 + (lane >> 3)) * 36 + (lane & 7) * 4) = n.x[u];
+  }
+  __syncthreads();
+  if (wave == 0) {
+    float s[R];
+#pragma unroll
+    for (int r = 0; r < R; r += 2) {  // (two rounds together: their scans hide each other; the first weights are on their way to most registers)
+      f32x4 v[2][2];
+#pragma unroll
+      for (int h = 0; h < 2; h++) s[r + h] = n.c[r + h][0];
+#pragma unroll
+      for (int j = 0; j < 4; j += 2) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          const int c = (r + h) * 64 + lane;
+#pragma unroll
+          for (int i = 0; i < 2; i++) v[h][i] = *(const f32x4*)(t + (c < nch ? c : nch - 1) * 36 + 16 + (j + i) * 4);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+#pragma unroll
+          for (int h = 0; h < 2; h++) s[r + h] += v[h][i >> 2][i & 3] * v[h][i >> 2][i & 3];
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) s_chunk[r * 64 + lane] = r * 64 + lane < nch ? s[r] : 0.0f;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    float sum = 0.0f;
+    f32x4 q[2];  // (eight sums are read while eight are added; sums past the row are +0.0)
+    q[0] = ((const f32x4*)s_chunk)[0];
+    q[1] = ((const f32x4*)s_chunk)[1];
+#pragma unroll 1
+    for (int c = 0; c < nch; c += 8) {
+      const float* next = s_chunk + (c + 8 < 64 * R ? c + 8 : 0);
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        const f32x4 v = q[i];
+        q[i] = ((const f32x4*)next)[i];
+        sum += v[0];
+        sum += v[1];
+        sum += v[2];
+        sum += v[3];
+      }
+    }
+    if (lane == 0) s_rms = sqrtf(sum / (float)(nsb * 256) + eps);
+  }
+  __syncthreads();
+  return s_rms;
+}
+template <int U, int R, bool ORD>
+__device__ __forceinline__ void kq_norm_quant(KqNorm<U, R>& n, const KqLds& l, float* __restrict__ t, float eps, int nsb, int lane, int wave, int nw) {
 #pragma unroll
   for (int u = 0; u < U; u++) asm volatile("" : "+v"(n.x[u]), "+v"(n.w[u]));  // (else the compiler moves the requests into the branch that uses them)
-  float sum = 0.0f;
+  float rms;
+  if constexpr (ORD) {
+    rms = kq_ordered_rms(n, t, eps, nsb, lane, wave, nw);
+  } else {
+    float sum = 0.0f;
 #pragma unroll
-  for (int r = 0; r < R; r++) sum += wave_sum_f32(r * 64 + lane < nsb * 8 ? n.c[r][0] + n.c[r][1] : 0.0f);  // (rounds past the row add +0.0)
-  const float rms = sqrtf(sum / (float)(nsb * 256) + eps);
+    for (int r = 0; r < R; r++) sum += wave_sum_f32(r * 64 + lane < nsb * 8 ? n.c[r][0] + n.c[r][1] : 0.0f);  // (rounds past the row add +0.0)
+    rms = sqrtf(sum / (float)(nsb * 256) + eps);
+  }
 #pragma unroll
   for (int u = 0; u < U; u++) {
     const int sb = wave + u * nw;
@@ -192,9 +260,59 @@ __device__ __forceinline__ void kq_rows(KqPiece<SIX> (&p)[P][R], const KqMat& m,
   }
 }
 
+// ORD: the rows' records (q4k_class_terms, gemv_core.hpp) to T, `stride` floats a row, one lane a row adds them (q4k_ordered_sum)
+template <bool SIX>
+__device__ __forceinline__ void kq_class_terms(const KqPiece<SIX>& p, const Q4KX& x, int c, bool live, float* __restrict__ t) {
+  if constexpr (!SIX) {
+    q4k_class_terms<false>(p.w, x, c, live, t);
+  } else {
+    const int sh = 8 * ((c & 1) + (c & 2));
+    q6k_class_terms(p.ql, p.qh, (int)(signed char)(p.sc[0] >> sh), (int)(signed char)(p.sc[1] >> sh), p.d, x.xl, x.xh, x.d8, c, live, t);
+  }
+}
+template <bool SIX, int R, int P>
+__device__ __forceinline__ void kq_terms(KqPiece<SIX> (&p)[P][R], const KqMat& m, const ActQ8_K& act, int row0, int last, int nsb, int lane, float* __restrict__ T, int stride) {
+  const int np = nsb * 8;
+  auto steps = [&](auto More, int c0) {
+#pragma unroll
+    for (int j = 0; j < P; j++) {
+      const int c = c0 + j * 64 + lane, cc = c < np ? c : np - 1;
+      if (!decltype(More)::value && c0 + j * 64 >= np) break;  // (uniform)
+      const Q4KX x = kq_loadx<SIX>(act, cc);
+#pragma unroll
+      for (int r = 0; r < R; r++) kq_class_terms<SIX>(p[j][r], x, cc, c < np, T + (size_t)r * stride + (cc >> 3) * 12);
+      if constexpr (decltype(More)::value) {
+        const int n = c + P * 64 < np ? c + P * 64 : np - 1;
+#pragma unroll
+        for (int r = 0; r < R; r++) p[j][r] = kq_load<SIX>(m, row0 + r < last ? row0 + r : last, nsb, n);
+      }
+    }
+  };
+  for (int c0 = 0; c0 < np; c0 += P * 64) {
+    if (c0 + P * 64 < np)
+      steps(std::true_type{}, c0);
+    else
+      steps(std::false_type{}, c0);
+  }
+}
+// floats from the planes on: the records of so many rows, or in front of them the row itself
+inline __host__ __device__ size_t kq_rec_at(int k, bool both) { return (kq_lds_bytes(k, both) + 15) & ~(size_t)15; }
+inline __host__ __device__ size_t kq_rec_bytes(int rows, int nsb, bool norm) {
+  const size_t r = (size_t)rows * q4k_rec_stride(nsb) * 4;
+  return norm && kq_ord_bytes(nsb) > r ? kq_ord_bytes(nsb) : r;
+}
+
+// Every wave of the workgroup has asked for its share of the rhs before any goes on to weights: a CU takes its waves' requests in turn, 16 cycles each, and the last wave's
+// share came 1900 cycles behind the first one's (us a launch without / with: q | k | v 6.2 / 5.8, wo 5.2 / 4.4, ffn_down 9.5 / 9.0; width 2048: wo 3.7 / 3.2, gate | up 6.6 / 6.1).
+__device__ __forceinline__ void kq_rhs_first() {
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 // q | k | v: a wave a pair of rows (the pair that is rotated).  SIX: Q6_K; V6: q and k Q4_K, v Q6_K (*_K_M files).  A workgroup of 4 to 16 waves: one round of workgroups, and a super-block a wave
-// where that is up to eight (3072 x 2048 4.9 us with four, 4.4 with eight, 4.6 with twelve; 6144 x 4096 8.4 with eight, 6.2 with twelve, 6.8 with sixteen).
-template <bool SIX, bool V6, int U, int R>
+// where that is up to eight (3072 x 2048 4.5 us with four, 4.0 with eight, 4.4 with twelve; 6144 x 4096 7.7 with eight, 5.8 with twelve, 6.8 with sixteen).
+template <bool SIX, bool V6, int U, int R, bool ORD = false>
 __global__ __launch_bounds__(1024) void k_kq_qkv(KqMat wq, KqMat wk, KqMat wv, const float* __restrict__ x, const float* __restrict__ wnorm, float eps,
                                                  const float* __restrict__ csums, int nsb, QkvEpi e) {
   extern __shared__ i32x4 lds_act[];
@@ -216,20 +334,38 @@ __global__ __launch_bounds__(1024) void k_kq_qkv(KqMat wq, KqMat wk, KqMat wv, c
   }
   KqNorm<U, R> n;
   kq_norm_request(n, x, wnorm, csums, nsb, lane, wave, nw);
+  kq_rhs_first();
   const QkvPre pre = qkv_preload_nb(e, row0);
   KqPiece<SIX> p[2][2];
-  KqPiece<true> p6[V6 ? 2 : 1][V6 ? 2 : 1];
+  constexpr int P6 = ORD ? 1 : 2;  // (registers)
+  KqPiece<true> p6[V6 ? P6 : 1][V6 ? 2 : 1];
   if (V6 && v6) {
-    if constexpr (V6) kq_request<true, 2, 2>(p6, w, local, m - 1, nsb, lane);
+    if constexpr (V6) kq_request<true, 2, P6>(p6, w, local, m - 1, nsb, lane);
   } else {
     kq_request<SIX, 2, 2>(p, w, local, m - 1, nsb, lane);
   }
-  kq_norm_quant(n, l, eps, nsb, lane, wave, nw);
+  float* T = (float*)((char*)lds_act + kq_rec_at(nsb * 256, V6));
+  kq_norm_quant<U, R, ORD>(n, l, T, eps, nsb, lane, wave, nw);
   __syncthreads();
   if (!live) return;
+  if constexpr (ORD) {
+    const int stride = q4k_rec_stride(nsb);
+    float* Tw = T + (size_t)wave * 2 * stride;
+    if (V6 && v6) {
+      if constexpr (V6) kq_terms<true, 2, P6>(p6, w, kq_act(l), local, m - 1, nsb, lane, Tw, stride);
+    } else {
+      kq_terms<SIX, 2, 2>(p, w, kq_act(l), local, m - 1, nsb, lane, Tw, stride);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    const float s = q4k_ordered_sum(Tw + (size_t)(lane & 1) * stride, nsb);
+    const float s1 = __shfl(s, 1, 64);
+    if (lane == 0) qkv_epilogue(e, pre, row0, s, s1);
+    return;
+  }
   float acc[2] = {0.f, 0.f};
   if (V6 && v6) {
-    if constexpr (V6) kq_rows<true, 2, 2>(p6, w, kq_act(l), local, m - 1, nsb, lane, acc);
+    if constexpr (V6) kq_rows<true, 2, P6>(p6, w, kq_act(l), local, m - 1, nsb, lane, acc);
   } else {
     kq_rows<SIX, 2, 2>(p, w, kq_act(l), local, m - 1, nsb, lane, acc);
   }
@@ -237,9 +373,9 @@ __global__ __launch_bounds__(1024) void k_kq_qkv(KqMat wq, KqMat wk, KqMat wv, c
   if (lane == 0) qkv_epilogue(e, pre, row0, s0, s1);
 }
 
-// gate | up + SiLU * mul: two rows of each a wave, 32 a workgroup of sixteen waves, two of them a CU (64 registers); h leaves as f32
-template <bool SIX, int U, int R>
-__global__ __launch_bounds__(1024, 8) void k_kq_gateup(KqMat wg, KqMat wu, const float* __restrict__ x, const float* __restrict__ wnorm, float eps,
+// gate | up + SiLU * mul: two rows of each a wave, 32 a workgroup of sixteen waves, two of them a CU (64 registers; one where the records of long rows fill its LDS); h leaves as f32
+template <bool SIX, int U, int R, bool ORD = false>
+__global__ __launch_bounds__(1024, ORD && U > 1 ? 4 : 8) void k_kq_gateup(KqMat wg, KqMat wu, const float* __restrict__ x, const float* __restrict__ wnorm, float eps,
                                                        const float* __restrict__ csums, int nsb, const unsigned short* __restrict__ exp_tab, float* __restrict__ h, int m) {
   extern __shared__ i32x4 lds_act[];
   const KqLds l = kq_lds(lds_act, nsb, !SIX, SIX);
@@ -247,12 +383,26 @@ __global__ __launch_bounds__(1024, 8) void k_kq_gateup(KqMat wg, KqMat wu, const
   const int row0 = (blockIdx.x * 16 + wave) * 2;
   KqNorm<U, R> n;
   kq_norm_request(n, x, wnorm, csums, nsb, lane, wave, 16);
+  kq_rhs_first();
   KqPiece<SIX> p[1][2];
   kq_request<SIX, 2, 1>(p, wg, row0, m - 1, nsb, lane);
-  kq_norm_quant(n, l, eps, nsb, lane, wave, 16);
+  float* T = (float*)((char*)lds_act + kq_rec_at(nsb * 256, false));  // rows 0 .. 31: gate, 32 .. 63: up
+  kq_norm_quant<U, R, ORD>(n, l, T, eps, nsb, lane, wave, 16);
   __syncthreads();
-  if (row0 >= m) return;
   const ActQ8_K act = kq_act(l);
+  if constexpr (ORD) {  // (host: m is a multiple of 32)
+    const int stride = q4k_rec_stride(nsb);
+    kq_terms<SIX, 2, 1>(p, wg, act, row0, m - 1, nsb, lane, T + (size_t)wave * 2 * stride, stride);
+    kq_request<SIX, 2, 1>(p, wu, row0, m - 1, nsb, lane);
+    kq_terms<SIX, 2, 1>(p, wu, act, row0, m - 1, nsb, lane, T + (size_t)(32 + wave * 2) * stride, stride);
+    __syncthreads();
+    if (wave != 0) return;
+    const float s = q4k_ordered_sum<3>(T + (size_t)lane * stride, nsb);  // (three records ahead: a fourth does not fit the 64 registers)
+    const float u = __shfl(s, (lane & 31) + 32, 64);
+    if (lane < 32) h[(int)blockIdx.x * 32 + lane] = silu_mul(s, u, exp_tab);
+    return;
+  }
+  if (row0 >= m) return;
   float ag[2] = {0.f, 0.f}, au[2] = {0.f, 0.f};
   kq_rows<SIX, 2, 1>(p, wg, act, row0, m - 1, nsb, lane, ag);
   kq_request<SIX, 2, 1>(p, wu, row0, m - 1, nsb, lane);
@@ -264,34 +414,8 @@ __global__ __launch_bounds__(1024, 8) void k_kq_gateup(KqMat wg, KqMat wu, const
   }
 }
 
-// wo, ffn_down: x += W . quantized(in), a row a wave, 16 a workgroup; the workgroup's sum of squares of x goes to csums (a plain store, read by the next launch)
-template <bool SIX, int U, int P>
-__global__ __launch_bounds__(1024) void k_kq_res(KqMat w, const float* __restrict__ in, int nsb, float* __restrict__ x, float* __restrict__ csums) {
-  extern __shared__ i32x4 lds_act[];
-  __shared__ __attribute__((aligned(16))) float hv[16];
-  const KqLds l = kq_lds(lds_act, nsb, !SIX, SIX);
-  const int lane = threadIdx.x & 63, wave = wave_in_wg(), row = blockIdx.x * 16 + wave;
-  f32x4 v[U];
-#pragma unroll
-  for (int u = 0; u < U; u++) v[u] = ((const f32x4*)in)[(wave + u * 16 < nsb ? wave + u * 16 : 0) * 64 + lane];
-  KqPiece<SIX> p[P][1];
-  kq_request<SIX, 1, P>(p, w, row, row, nsb, lane);
-  const float res = x[blockIdx.x * 16 + (lane & 15)];  // (wave 0's; no branch)
-#pragma unroll
-  for (int u = 0; u < U; u++) asm volatile("" : "+v"(v[u]));  // (as in kq_norm_quant)
-#pragma unroll
-  for (int u = 0; u < U; u++) {
-    if (wave + u * 16 >= nsb) break;  // (wave-uniform)
-    kq_quant(l, wave + u * 16, v[u], lane);
-  }
-  for (int sb = wave + U * 16; sb < nsb; sb += 16) kq_quant(l, sb, ((const f32x4*)in)[sb * 64 + lane], lane);
-  __syncthreads();
-  float acc[1] = {0.f};
-  kq_rows<SIX, 1, P>(p, w, kq_act(l), row, row, nsb, lane, acc);
-  const float s = wave_sum_f32(acc[0]);
-  if (lane == 0) hv[wave] = s;
-  __syncthreads();
-  if (wave != 0) return;
+// the end of a workgroup's 16 rows: hv their dots, res what they are added to; one wave
+__device__ __forceinline__ void kq_res_out(float* hv, float res, float* __restrict__ x, float* __restrict__ csums, int lane) {
   if (lane < 16) {
     const float xv = hv[lane] + res;  // x = matmul_out + x (llama2.rs:266 / :636)
     x[blockIdx.x * 16 + lane] = xv;
@@ -309,6 +433,50 @@ __global__ __launch_bounds__(1024) void k_kq_res(KqMat w, const float* __restric
     cs += t[3] * t[3];
   }
   if (lane == 0) csums[blockIdx.x] = cs;
+}
+// wo, ffn_down: x += W . quantized(in), a row a wave, 16 a workgroup; the workgroup's sum of squares of x goes to csums (a plain store, read by the next launch)
+template <bool SIX, int U, int P, bool ORD = false>
+__global__ __launch_bounds__(1024) void k_kq_res(KqMat w, const float* __restrict__ in, int nsb, float* __restrict__ x, float* __restrict__ csums) {
+  extern __shared__ i32x4 lds_act[];
+  __shared__ __attribute__((aligned(16))) float hv[16];
+  const KqLds l = kq_lds(lds_act, nsb, !SIX, SIX);
+  const int lane = threadIdx.x & 63, wave = wave_in_wg(), row = blockIdx.x * 16 + wave;
+  f32x4 v[U];
+#pragma unroll
+  for (int u = 0; u < U; u++) v[u] = ((const f32x4*)in)[(wave + u * 16 < nsb ? wave + u * 16 : 0) * 64 + lane];
+  KqPiece<SIX> p[P][1];
+  kq_rhs_first();
+  kq_request<SIX, 1, P>(p, w, row, row, nsb, lane);
+  const float res = x[blockIdx.x * 16 + (lane & 15)];  // (wave 0's; no branch)
+#pragma unroll
+  for (int u = 0; u < U; u++) asm volatile("" : "+v"(v[u]));  // (as in kq_norm_quant)
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    if (wave + u * 16 >= nsb) break;  // (wave-uniform)
+    kq_quant(l, wave + u * 16, v[u], lane);
+  }
+  for (int sb = wave + U * 16; sb < nsb; sb += 16) kq_quant(l, sb, ((const f32x4*)in)[sb * 64 + lane], lane);
+  __syncthreads();
+  if constexpr (ORD) {
+    const int stride = q4k_rec_stride(nsb);
+    float* T = (float*)((char*)lds_act + kq_rec_at(nsb * 256, false));
+    kq_terms<SIX, 1, P>(p, w, kq_act(l), row, row, nsb, lane, T + (size_t)wave * stride, stride);
+    __syncthreads();
+    if (wave != 0) return;
+    const float s = q4k_ordered_sum(T + (size_t)(lane & 15) * stride, nsb);
+    if (lane < 16) hv[lane] = s;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    kq_res_out(hv, res, x, csums, lane);
+    return;
+  }
+  float acc[1] = {0.f};
+  kq_rows<SIX, 1, P>(p, w, kq_act(l), row, row, nsb, lane, acc);
+  const float s = wave_sum_f32(acc[0]);
+  if (lane == 0) hv[wave] = s;
+  __syncthreads();
+  if (wave != 0) return;
+  kq_res_out(hv, res, x, csums, lane);
 }
 
 }  // namespace crabml_hip
