@@ -92,9 +92,11 @@ __global__ __launch_bounds__(256) void k_latent_append(const MixRows<T> a) {
 #define LAT_SPLITS 16      // most workgroups that share a sequence's cached rows
 #define LAT_SLICE 64       // latent columns per workgroup of k_latent_query
 #define LAT_MAX_ROW 768    // rank + rot
+#define LAT_VALUE 512      // threads of k_latent_value
 template <typename T>
-struct LatTile {
-  static constexpr int KT = sizeof(T) == 2 ? 64 : 32, PAD = 16 / sizeof(T), LP = KT + 4;
+struct LatTile {  // rows of a tile, waves of k_latent_attn, waves that share a score's columns
+  static constexpr int KT = sizeof(T) == 2 ? 64 : 32, NW = sizeof(T) == 2 ? 16 : 8, KS = NW / (KT / 16);
+  static constexpr int PAD = 16 / sizeof(T), LP = KT + 4, PP = KT + PAD;
 };
 struct LatStep {
   AttnGeom at;
@@ -102,7 +104,7 @@ struct LatStep {
   RunState rs;
   const StepSeq* seq = nullptr;
   const float* proj = nullptr;  // [B][ldp]
-  float* q = nullptr;           // [B][H][rank + rot]
+  void* q = nullptr;            // [B][H][rank + rot] in the cache's type
   float* part = nullptr;        // [B][H][LAT_SPLITS][rank + 2]: unnormalized sums, maximum, denominator
   float* cat = nullptr;         // [B][ldc]
   unsigned short* cat16 = nullptr;  // the same as bf16, instead (nullable)
@@ -155,9 +157,9 @@ __global__ __launch_bounds__(256) void k_latent_query(const LatStep a) {
       const float cs = lat_lds[2 * p], sn = lat_lds[2 * p + 1];
       const float u = src[0] * cs - src[1] * sn, v = src[1] * cs + src[0] * sn;
       if (h < g.H) {
-        float* d = a.q + ((size_t)b * g.H + h) * row_w + l.rank + 2 * p;
-        d[0] = u;
-        d[1] = v;
+        T* d = (T*)a.q + ((size_t)b * g.H + h) * row_w + l.rank + 2 * p;
+        d[0] = kv_from<T>(u);
+        d[1] = kv_from<T>(v);
       } else {
         c[l.rank + 2 * p] = kv_from<T>(u);
         c[l.rank + 2 * p + 1] = kv_from<T>(v);
@@ -197,26 +199,33 @@ __global__ __launch_bounds__(256) void k_latent_query(const LatStep a) {
   if (rr < r1) {
 #pragma unroll
     for (int e = 0; e < 4; e++)
-      if (fk * 4 + e < a.B) a.q[((size_t)(fk * 4 + e) * g.H + h) * row_w + rr] = acc[e];
+      if (fk * 4 + e < a.B) ((T*)a.q)[((size_t)(fk * 4 + e) * g.H + h) * row_w + rr] = kv_from<T>(acc[e]);
   }
 }
 
-// out += P V over one tile: P [16][KT] f32 (LDS), V [KT][ld] (LDS rows of the cache); this lane's column of V
-__device__ __forceinline__ f32x4 latent_pv(const float* p, const unsigned short* v, int ld, f32x4 acc) {
+// acc += A B^T over 32 columns; element e of a lane's octet goes with the same one of the others
+__device__ __forceinline__ f32x4 latent_qk(const Oct<unsigned short>& q, const Oct<unsigned short>& k, f32x4 acc) {
+  return mfma_bf16(__builtin_bit_cast(bf16x8, q.d[0]), __builtin_bit_cast(bf16x8, k.d[0]), acc);
+}
+__device__ __forceinline__ f32x4 latent_qk(const Oct<float>& q, const Oct<float>& k, f32x4 acc) {
+  float a[8], b[8];
+  oct_floats(q, a);
+  oct_floats(k, b);
+#pragma unroll
+  for (int e = 0; e < 8; e++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], acc, 0, 0, 0);
+  return acc;
+}
+// out += P V over one tile: P [16][PP] (LDS), V [KT][ld] (LDS rows of the cache); this lane's column of V
+__device__ __forceinline__ f32x4 latent_pv(const unsigned short* p, const unsigned short* v, int ld, f32x4 acc) {
   const int fr = threadIdx.x & 15, fk = threadIdx.x >> 4 & 3;
 #pragma unroll
   for (int k = 0; k < LatTile<unsigned short>::KT; k += 32) {
-    float w[8];
-    read8(p + fr * LatTile<unsigned short>::LP + k + fk * 8, w);
-    bf16x8 fa, fb;
+    bf16x8 fb;
     unsigned short t[8];
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-      fa[e] = (__bf16)w[e];
-      t[e] = v[(size_t)(k + fk * 8 + e) * ld];
-    }
+    for (int e = 0; e < 8; e++) t[e] = v[(size_t)(k + fk * 8 + e) * ld];
     __builtin_memcpy(&fb, t, 16);
-    acc = mfma_bf16(fa, fb, acc);
+    acc = mfma_bf16(*(const bf16x8*)(p + fr * LatTile<unsigned short>::PP + k + fk * 8), fb, acc);
   }
   return acc;
 }
@@ -224,127 +233,115 @@ __device__ __forceinline__ f32x4 latent_pv(const float* p, const float* v, int l
   const int fr = threadIdx.x & 15, fk = threadIdx.x >> 4 & 3;
 #pragma unroll
   for (int k = 0; k < LatTile<float>::KT; k += 4)
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(p[fr * LatTile<float>::LP + k + fk], v[(size_t)(k + fk) * ld], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(p[fr * LatTile<float>::PP + k + fk], v[(size_t)(k + fk) * ld], acc, 0, 0, 0);
   return acc;
 }
 
-// NT: latent columns up to 64 NT
+// NT: latent columns up to 16 NW NT.  A chain of one or a few tiles in a few workgroups, so what bounds it is each link's length, and a tile goes over all
+// waves a workgroup can have: a wave asks for 16 rows' share of the columns as the score's matrix instructions take them, scores them from its registers
+// (the waves that share a row tile meet in LDS) and lays them down for P V on the way; the next tile is asked for before the softmax.  16 heads, rank 512 + 64,
+// us a launch, staged through LDS by four waves / so: one sequence of 33 to 81 rows 10.5 / 7.2, four of 700 11.7 / 7.9.
 template <typename T, int NT>
-__global__ __launch_bounds__(256) void k_latent_attn(const LatStep a) {
-  constexpr int KT = LatTile<T>::KT, LP = LatTile<T>::LP;
+__global__ __launch_bounds__(64 * LatTile<T>::NW) void k_latent_attn(const LatStep a) {
+  constexpr int KT = LatTile<T>::KT, LP = LatTile<T>::LP, PP = LatTile<T>::PP, NW = LatTile<T>::NW, KS = LatTile<T>::KS, RT = KT / 16;
+  constexpr int NS = LAT_MAX_ROW / 32 / KS, HW = LAT_HEADS / NW, UQ = (LAT_HEADS * LAT_MAX_ROW / 8 + 64 * NW - 1) / (64 * NW);
   extern __shared__ __attribute__((aligned(16))) char latt_lds[];
-  __shared__ float alpha[LAT_HEADS];
+  __shared__ __attribute__((aligned(16))) float alpha[LAT_HEADS];
   const AttnGeom& g = a.at;
   const LatGeom& l = a.la;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_in_wg(), fr = lane & 15, fk = lane >> 4;
   const int split = blockIdx.x, h0 = blockIdx.y * LAT_HEADS, b = blockIdx.z;
   const int row_w = l.rank + l.rot, w32 = (row_w + 31) & ~31, ld = w32 + LatTile<T>::PAD, cpr = w32 / 8;
-  T* q_s = (T*)latt_lds;               // [16][ld]
-  T* k_s = q_s + LAT_HEADS * ld;       // [KT][ld]
-  float* p_s = (float*)(k_s + KT * ld);  // [16][LP]
+  T* q_s = (T*)latt_lds;                   // [16][ld]
+  T* k_s = q_s + LAT_HEADS * ld;           // [KT][ld]
+  float* s_s = (float*)(k_s + KT * ld);    // [KS][16][LP]
+  T* p_s = (T*)(s_s + KS * LAT_HEADS * LP);  // [16][PP]
   const int nh = g.H - h0 < LAT_HEADS ? g.H - h0 : LAT_HEADS;
-  const float* q = a.q + ((size_t)b * g.H + h0) * row_w;
+  const T* q = (const T*)a.q + ((size_t)b * g.H + h0) * row_w;
   const StepSeq sq = a.seq[b];
+  Oct<T> qv[UQ];
+#pragma unroll
+  for (int u = 0; u < UQ; u++) {
+    const int i = tid + u * 64 * NW, r = i / cpr, c = i % cpr * 8;
+    qv[u] = oct_zero<T>();
+    if (r < nh && c < row_w) qv[u] = oct_load(q + (size_t)r * row_w + c);
+  }
   const LatRange rg = latent_range<T>(g, a.splits, sq.pos);
   const int lo = split * rg.per, hi = lo + rg.per < rg.n ? lo + rg.per : rg.n;
   if (lo >= hi) return;  // (whole workgroup)
   const T* cache = as_global((const T*)(sq.slab + a.rs.k));
-  // a tile's octets in row order, 256 at a time: thread t starts at (row tr0, octet tc0) and goes on by (dr, dc)
-  const int tr0 = tid / cpr, tc0 = tid % cpr, dr = 256 / cpr, dc = 256 % cpr;
-  constexpr int UN = sizeof(T) == 2 ? 9 : 5;  // octets in flight per thread
-  auto stage = [&](int t0, int n, int rows, const T* src, T* dst) {  // rows of LDS; those from n on are zero
-    int r = tr0, c = tc0;
-    while (true) {
-      Oct<T> v[UN];
-      int at[UN];
+  const int rt = wave % RT, ks = wave / RT, nks = (w32 / 32 + KS - 1) / KS, k0 = ks * nks * 32;
+  Oct<T> kv[NS];
+  auto fetch = [&](int t0) {  // rows that are not there and columns past the row's end are zero
+    const int row = t0 + rt * 16 + fr;
 #pragma unroll
-      for (int u = 0; u < UN; u++) {
-        at[u] = r < rows ? r * ld + c * 8 : -1;
-        v[u] = oct_zero<T>();
-        if (r < n && r < rows && c * 8 < row_w) v[u] = oct_load(src + (size_t)(t0 + r) * row_w + c * 8);
-        r += dr;
-        c += dc;
-        if (c >= cpr) {
-          c -= cpr;
-          r++;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < UN; u++)
-        if (at[u] >= 0) oct_store(dst + at[u], v[u]);
-      if (__all(r >= rows)) return;
+    for (int s = 0; s < NS; s++) {
+      const int k = k0 + s * 32 + fk * 8;
+      kv[s] = oct_zero<T>();
+      if (s < nks && row < hi && k < row_w) kv[s] = oct_load(cache + (size_t)row * row_w + k);
     }
   };
-  {
-    constexpr int UQ = LAT_HEADS * LAT_MAX_ROW / 8 / 256;
-    int r = tr0, c = tc0, at[UQ];
-    float v[UQ][8];
+  fetch(lo);
 #pragma unroll
-    for (int u = 0; u < UQ; u++) {
-      at[u] = r < LAT_HEADS ? r * ld + c * 8 : -1;
-#pragma unroll
-      for (int e = 0; e < 8; e++) v[u][e] = 0.f;
-      if (r < nh && c * 8 < row_w) read8(q + (size_t)r * row_w + c * 8, v[u]);
-      r += dr;
-      c += dc;
-      if (c >= cpr) {
-        c -= cpr;
-        r++;
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < UQ; u++)
-      if (at[u] >= 0) {
-        T t[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++) t[e] = kv_from<T>(v[u][e]);
-        __builtin_memcpy(q_s + at[u], t, sizeof t);
-      }
+  for (int u = 0; u < UQ; u++) {
+    const int i = tid + u * 64 * NW, r = i / cpr;
+    if (r < LAT_HEADS) oct_store(q_s + r * ld + i % cpr * 8, qv[u]);
   }
   f32x4 o[NT];
 #pragma unroll
   for (int j = 0; j < NT; j++) o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m[4], den[4];  // of heads 4 wave .. 4 wave + 3
+  float m[HW], den[HW];  // of heads HW wave ..
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
+  for (int i = 0; i < HW; i++) {
     m[i] = -INFINITY;
     den[i] = 0.f;
   }
+  __syncthreads();
   for (int t0 = lo; t0 < hi; t0 += KT) {
-    __syncthreads();  // the previous tile has been read
-    stage(t0, hi - t0, KT, cache, k_s);
-    __syncthreads();
-    if (wave < KT / 16) {
-      f32x4 s = {0.f, 0.f, 0.f, 0.f};
-      for (int k = 0; k < w32; k += 32) s = mma_rows(q_s + fr * ld + k, k_s + (wave * 16 + fr) * ld + k, 32, s);
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int e = 0; e < 4; e++) p_s[(fk * 4 + e) * LP + wave * 16 + fr] = t0 + wave * 16 + fr < hi ? s[e] * g.scale : -INFINITY;
+    for (int u = 0; u < NS; u++) {
+      const int k = k0 + u * 32;
+      if (u < nks && k < w32) {  // (uniform)
+        s = latent_qk(oct_load(q_s + fr * ld + k + fk * 8), kv[u], s);
+        oct_store(k_s + (rt * 16 + fr) * ld + k + fk * 8, kv[u]);
+      }
     }
+#pragma unroll
+    for (int e = 0; e < 4; e++) s_s[(ks * LAT_HEADS + fk * 4 + e) * LP + rt * 16 + fr] = s[e];
+    if (t0 + KT < hi) fetch(t0 + KT);
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int h = wave * 4 + i;
-      const float s = lane < KT ? p_s[h * LP + lane] : -INFINITY;
-      const float mx = fmaxf(m[i], wave_max_f32(s));  // (a tile has at least one row: finite)
-      const float e = __expf(s - mx), w = __expf(m[i] - mx);
+    for (int i = 0; i < HW; i++) {
+      const int h = wave * HW + i;
+      float v = -INFINITY;
+      if (lane < KT && t0 + lane < hi) {
+        v = 0.f;
+#pragma unroll
+        for (int u = 0; u < KS; u++) v += s_s[(u * LAT_HEADS + h) * LP + lane];
+        v *= g.scale;
+      }
+      const float mx = fmaxf(m[i], wave_max_f32(v));  // (a tile has at least one row: finite)
+      const float e = __expf(v - mx), w = __expf(m[i] - mx);
       den[i] = __builtin_fmaf(den[i], w, wave_sum_f32(e));
       m[i] = mx;
-      if (lane < KT) p_s[h * LP + lane] = e;
+      if (lane < KT) p_s[h * PP + lane] = kv_from<T>(e);
       if (lane == 0) alpha[h] = w;
     }
     __syncthreads();
     const f32x4 w = *(const f32x4*)&alpha[fk * 4];
 #pragma unroll
     for (int j = 0; j < NT; j++) {
-      const int c = (wave + 4 * j) * 16;
+      const int c = (wave + NW * j) * 16;
       if (c < l.rank) o[j] = latent_pv(p_s, k_s + c + fr, ld, o[j] * w);
     }
+    if (t0 + KT < hi) __syncthreads();  // the tile has been read
   }
   const int pw = l.rank + 2;
   float* part = a.part + (((size_t)b * g.H + h0) * LAT_SPLITS + split) * pw;
 #pragma unroll
   for (int j = 0; j < NT; j++) {
-    const int c = (wave + 4 * j) * 16 + fr;
+    const int c = (wave + NW * j) * 16 + fr;
     if (c < l.rank) {
 #pragma unroll
       for (int e = 0; e < 4; e++)
@@ -352,8 +349,8 @@ __global__ __launch_bounds__(256) void k_latent_attn(const LatStep a) {
     }
   }
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int h = wave * 4 + i;
+  for (int i = 0; i < HW; i++) {
+    const int h = wave * HW + i;
     if (lane == 0 && h < nh) {
       part[(size_t)h * LAT_SPLITS * pw + l.rank] = m[i];
       part[(size_t)h * LAT_SPLITS * pw + l.rank + 1] = den[i];
@@ -361,9 +358,10 @@ __global__ __launch_bounds__(256) void k_latent_attn(const LatStep a) {
   }
 }
 
-// grid: (H * slices of VS value columns, B); SP: splits
+// grid: (H * slices of VS value columns, B); SP: splits.  One round trip for the splits' maxima, denominators and sums and the weights (in two, with four waves:
+// 6.7 us for one sequence and 7.6 for four of 16 heads, rank 512; so 4.9 and 5.8).
 template <typename T, int SP, int VS>
-__global__ __launch_bounds__(256) void k_latent_value(const LatStep a) {
+__global__ __launch_bounds__(LAT_VALUE) void k_latent_value(const LatStep a) {
   __shared__ __attribute__((aligned(16))) float x[LAT_MAX_ROW];
   const AttnGeom& g = a.at;
   const LatGeom& l = a.la;
@@ -377,8 +375,8 @@ __global__ __launch_bounds__(256) void k_latent_value(const LatStep a) {
   while (lpr < 64 && lpr * 8 < l.rank) lpr <<= 1;
   const int rows = 64 / lpr, sub = lane / lpr, k0 = lane % lpr * 8;
   const unsigned short* wv = l.w_kv + (size_t)(g.H * l.dim + h * g.V) * l.ldl;
-  // a wave's VS / 4 rows, `rows` at a time: their first octets are on their way while the splits are merged
-  constexpr int RW = VS / 4;
+  // a wave's RW rows, `rows` at a time: their first octets are on their way while the splits are merged
+  constexpr int RW = VS / (LAT_VALUE / 64);
   i32x4 wf[RW];
   const int kf = k0 < l.ldl ? k0 : 0;
 #pragma unroll
@@ -386,13 +384,17 @@ __global__ __launch_bounds__(256) void k_latent_value(const LatStep a) {
     const int v = v0 + wave * RW + j * rows + sub;
     if (j * rows < RW) wf[j] = *(const i32x4*)(wv + (size_t)(v < v1 ? v : v1 - 1) * l.ldl + kf);
   }
-  float w[SP], ds[SP], top = -INFINITY, den = 0.f;
+  float w[SP], ds[SP], p[SP], top = -INFINITY, den = 0.f;
 #pragma unroll
   for (int s = 0; s < SP; s++) {  // (requests without branches; a split that is not there counts nothing)
-    const float* p = part + (size_t)s * pw + l.rank;
-    w[s] = p[0];
-    ds[s] = p[1];
+    w[s] = part[(size_t)s * pw + l.rank];
+    ds[s] = part[(size_t)s * pw + l.rank + 1];
   }
+  auto column = [&](int i) {
+#pragma unroll
+    for (int s = 0; s < SP; s++) p[s] = part[(size_t)s * pw + (i < l.rank ? i : 0)];
+  };
+  column(tid);  // (in the same round trip: most ranks have no other)
 #pragma unroll
   for (int s = 0; s < SP; s++) {
     w[s] = s < active ? w[s] : -INFINITY;
@@ -404,10 +406,9 @@ __global__ __launch_bounds__(256) void k_latent_value(const LatStep a) {
     den = __builtin_fmaf(s < active ? ds[s] : 0.f, w[s], den);
   }
   const float inv = 1.0f / den;
-  for (int i = tid; i < l.ldl; i += 256) {
-    float p[SP], o = 0.f;
-#pragma unroll
-    for (int s = 0; s < SP; s++) p[s] = part[(size_t)s * pw + (i < l.rank ? i : 0)];
+  for (int i = tid; i < l.ldl; i += LAT_VALUE) {
+    if (i != tid) column(i);
+    float o = 0.f;
 #pragma unroll
     for (int s = 0; s < SP; s++) o = __builtin_fmaf(s < active ? p[s] : 0.f, w[s], o);
     x[i] = i < l.rank ? o * inv : 0.f;
@@ -441,21 +442,21 @@ inline int latent_splits(int B, int H) { return B * H >= 512 ? LAT_SPLITS / 2 : 
 template <typename T>
 inline size_t latent_attn_lds(const LatGeom& l) {
   const size_t ld = align_up((size_t)(l.rank + l.rot), 32) + LatTile<T>::PAD;
-  return (LAT_HEADS + LatTile<T>::KT) * ld * sizeof(T) + (size_t)LAT_HEADS * LatTile<T>::LP * sizeof(float);
+  return (LAT_HEADS + LatTile<T>::KT) * ld * sizeof(T) + (size_t)LAT_HEADS * (LatTile<T>::KS * LatTile<T>::LP * sizeof(float) + LatTile<T>::PP * sizeof(T));
 }
 template <typename T, int NT>
 inline int launch_latent_attn_t(crabml_hip_device* dev, crabml_hip_device::ProfRec* rec, const LatStep& a) {
   const size_t lds = latent_attn_lds<T>(a.la);
   CH_HIP(dev, raise_dyn_lds(dev, (const void*)k_latent_attn<T, NT>, (int)lds));
-  launch_k(dev->stream, rec, k_latent_attn<T, NT>, dim3(a.splits, (a.at.H + LAT_HEADS - 1) / LAT_HEADS, a.B), dim3(256), lds, a);
+  launch_k(dev->stream, rec, k_latent_attn<T, NT>, dim3(a.splits, (a.at.H + LAT_HEADS - 1) / LAT_HEADS, a.B), dim3(64 * LatTile<T>::NW), lds, a);
   return 0;
 }
 template <typename T>
 inline int launch_latent_attn(crabml_hip_device* dev, crabml_hip_device::ProfRec* rec, const LatStep& a) {
-  if (a.la.rank <= 128) return launch_latent_attn_t<T, 2>(dev, rec, a);
-  if (a.la.rank <= 256) return launch_latent_attn_t<T, 4>(dev, rec, a);
-  if (a.la.rank <= 512) return launch_latent_attn_t<T, 8>(dev, rec, a);
-  return launch_latent_attn_t<T, 12>(dev, rec, a);
+  constexpr int N = 16 / LatTile<T>::NW;  // of 256 columns
+  if (a.la.rank <= 256) return launch_latent_attn_t<T, N>(dev, rec, a);
+  if (a.la.rank <= 512) return launch_latent_attn_t<T, 2 * N>(dev, rec, a);
+  return launch_latent_attn_t<T, 3 * N>(dev, rec, a);
 }
 template <typename T>
 inline void launch_latent_query(hipStream_t st, crabml_hip_device::ProfRec* rec, const LatStep& a) {
@@ -465,9 +466,9 @@ inline void launch_latent_query(hipStream_t st, crabml_hip_device::ProfRec* rec,
 template <typename T>
 inline void launch_latent_value(hipStream_t st, crabml_hip_device::ProfRec* rec, const LatStep& a) {
   if (a.splits == LAT_SPLITS)
-    launch_k(st, rec, k_latent_value<T, LAT_SPLITS, 32>, dim3(a.at.H * ((a.at.V + 31) / 32), a.B), dim3(256), 0, a);
+    launch_k(st, rec, k_latent_value<T, LAT_SPLITS, 32>, dim3(a.at.H * ((a.at.V + 31) / 32), a.B), dim3(LAT_VALUE), 0, a);
   else
-    launch_k(st, rec, k_latent_value<T, LAT_SPLITS / 2, 64>, dim3(a.at.H * ((a.at.V + 63) / 64), a.B), dim3(256), 0, a);
+    launch_k(st, rec, k_latent_value<T, LAT_SPLITS / 2, 64>, dim3(a.at.H * ((a.at.V + 63) / 64), a.B), dim3(LAT_VALUE), 0, a);
 }
 
 }  // namespace crabml_hip

@@ -298,6 +298,22 @@ def test_long_decoding(ca, hdev, tmp_path, window, n, start):
         close(np.concatenate(got), want[at], f32)
 
 
+@pytest.mark.parametrize("rank,rot", [(8, 2), (256, 16), (512, 64), (704, 64)])
+def test_latent_rows_of_every_width(ca, hdev, tmp_path, rank, rot):
+    """cached rows of one 32-column step of the scores up to the widest, by one tile and by several of a workgroup, a second block of heads of one"""
+    c = sb.config(48, 70, [sb.latent(17, 16, rot, 16, rank, 1200, None)], streams=1)
+    m = Model(c, tmp_path / "m", seed=rank)
+    t = m.tokens(1093, seed=rot)
+    want = m.oracle(t)
+    for f32 in (True, False):
+        r = m.runner(ca, hdev, f32, seq_len=1200)
+        for start, n in ((30, 4), (1084, 9)):
+            s = r.open()
+            r.step([(s, t[:start], [])])
+            close(np.concatenate([r.step([(s, [x], [0])]) for x in t[start:start + n]]), want[start:start + n], f32)
+            r.close(s)
+
+
 # ---- single mechanisms -----------------------------------------------------------------------------------------------------------------
 def pointed_at(config, seed, key_token, query_token):
     """random weights of a one-layer model in which query_token's query (every head) points at key_token's key"""
