@@ -737,6 +737,7 @@ int launch_gemv_strict(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m
     const char* e = getenv("CRABML_HIP_STRICT_SCALAR");
     return h && h[0] == '1' && e && e[0] == '1';
   }();
+  if (!scalar_only && launch_gemm_exact_kq(dev, w, m, k, act, b, out, add_all)) return 0;
   const size_t per = rhs_rows_per_launch(m);
   for (size_t b0 = 0; b0 < b; b0 += per) {
     const size_t rows = b - b0 < per ? b - b0 : per;

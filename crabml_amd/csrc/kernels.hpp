@@ -43,6 +43,11 @@ int launch_gemv(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m, size_
 // gemv_strict.hip: same contract, block terms added in the reference's scalar order (bit-exact; slow)
 int launch_gemv_strict(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m, size_t k, const void* act, size_t b,
                        float* out, const float* add = nullptr);  // add: out[i] = sum + add[i] (the residual; may alias out)
+// gemm_exact_kq.hip: the same for several rows of the rhs on the matrix cores (Q4_K); false where the row kernels take it.  From KQX_ROWS rows on: the rows of
+// a tile cost the same from one to sixteen, a row kernel's row by row.  A prompt on four layers, us, row kernels / this: 8B shape 3 rows 764 / 783, 4 rows 837 / 784,
+// 6 rows 1012 / 782, 16 rows 1867 / 797, 128 rows 11636 / 2229; 2048 x 8192 3 rows 451 / 461, 4 rows 487 / 466, 16 rows 790 / 479, 128 rows 3642 / 950.
+bool launch_gemm_exact_kq(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m, size_t k, const void* act, size_t b, float* out, const float* add);
+#define KQX_ROWS 4
 // weight upload: scatter the pieces of `n_blocks` GGUF blocks (`bb` bytes each) starting at block `blk0` into their
 // planes (byte moves only).  Piece s = bytes [2 src_off2, 2 src_off2 + 2 len2) of a block -> base + dst_off[s],
 // one `stride2`-unit record per block (stride2 = len2 unless two pieces share a record: Q5_K's header); bytes covered by no

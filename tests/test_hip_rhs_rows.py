@@ -57,3 +57,24 @@ def test_lane_per_row_kernel_over_several_launches(ca, fmt, m, rows):
     for r in range(rows):
         one = w.matmul_vec(ca.HipTensor.new(x[r], [256], dev)).export()
         assert np.array_equal(got[r].view(np.uint32), one.view(np.uint32)), r
+
+
+# rows of the rhs: one, two and four of the kernel's tiles, their remainders, several workgroups; rows of the matrix: less than a tile, remainders, tiles that do
+# and do not divide by the eight XCDs; super-blocks: fewer than are on their way at once, a remainder, many
+@pytest.mark.parametrize("m,k,rows", [(1, 256, 4), (15, 768, 16), (130, 1280, 17), (100, 512, 32), (256, 1024, 33), (77, 2304, 64), (129, 256, 65), (48, 14336, 130)])
+@pytest.mark.parametrize("levels", ["random", "largest"])
+def test_strict_q4_k_on_the_matrix_cores(ca, m, k, rows, levels):
+    """several rows against one row at a time (the row kernels, which the oracle covers); `largest`: every level 15, scale and minimum 63, quant -128 or 127"""
+    rng = np.random.default_rng(m + rows)
+    dev = ca.HipTensorDevice(0, False, 0, True)
+    raw = synth.random_blocks(rng, m * k, synth.TYPE_BY_NAME["Q4_K"])
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    if levels == "largest":
+        raw = raw.copy()
+        raw.reshape(-1, 144)[:, 4:] = 255
+        x = np.where(rng.random((rows, 1)) < 0.5, 1.0, np.where(rng.random((rows, k)) < 0.5, -1.0, 0.99)).astype(np.float32)
+    w = ca.HipTensor.from_cpu(raw, [m, k], ca.GGMLType.Q4K, dev)
+    got = w.matmul_vec(ca.HipTensor.new(x.reshape(-1), [rows, k], dev)).export().reshape(rows, m)
+    for r in range(rows):
+        one = w.matmul_vec(ca.HipTensor.new(x[r], [k], dev)).export()
+        assert np.array_equal(got[r].view(np.uint32), one.view(np.uint32)), r
