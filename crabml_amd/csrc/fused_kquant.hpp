@@ -8,7 +8,7 @@
 // Every row's pieces are added by lane, ascending, as k_gemv_q4_k / k_gemv_q6_k add them, the norm's sums in k_norm_f32's order: the planes and logits are the per-op
 // launches' bit for bit.
 // Us a launch of the 8B shape, Q4_K, with planes from the producer / these: q | k | v 5.6 / 5.8, wo 5.6 / 4.4, gate | up 16.6 / 13.7 (4.8 TB/s), ffn_down 11.2 / 9.0; on the
-// strict-order device (ORD) 6.5 / 9.4, 10.7 / 5.6, 19.0 / 18.0, 16.2 / 13.3.  A token of four layers 269 -> 242, of Q6_K (fourteen launches a layer and the attention before)
+// strict-order device (ORD) 6.5 / 8.8, 10.7 / 5.5, 19.0 / 18.0, 16.2 / 12.4.  A token of four layers 269 -> 242, of Q6_K (fourteen launches a layer and the attention before)
 // 407 -> 297; width 2048, six layers, Q4_K 222 -> 192, Q6_K 363 -> 214.
 #pragma once
 #include "fused_ffn.hpp"
@@ -260,7 +260,7 @@ __device__ __forceinline__ void kq_rows(KqPiece<SIX> (&p)[P][R], const KqMat& m,
   }
 }
 
-// ORD: the rows' records (q4k_class_terms, gemv_core.hpp) to T, `stride` floats a row, one lane a row adds them (q4k_ordered_sum)
+// ORD: the rows' records (q4k_class_terms, gemv_core.hpp) to T, `stride` floats a row, a lane a chain adds them (q4k_ordered_sum16)
 template <bool SIX>
 __device__ __forceinline__ void kq_class_terms(const KqPiece<SIX>& p, const Q4KX& x, int c, bool live, float* __restrict__ t) {
   if constexpr (!SIX) {
@@ -358,8 +358,8 @@ __global__ __launch_bounds__(1024) void k_kq_qkv(KqMat wq, KqMat wk, KqMat wv, c
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_wave_barrier();
-    const float s = q4k_ordered_sum(Tw + (size_t)(lane & 1) * stride, nsb);
-    const float s1 = __shfl(s, 1, 64);
+    const float s = q4k_ordered_sum16(Tw + (size_t)(lane >> 4 & 1) * stride, nsb, lane);
+    const float s1 = rl_f(s, 16);
     if (lane == 0) qkv_epilogue(e, pre, row0, s, s1);
     return;
   }
@@ -397,7 +397,7 @@ __global__ __launch_bounds__(1024, ORD && U > 1 ? 4 : 8) void k_kq_gateup(KqMat 
     kq_terms<SIX, 2, 1>(p, wu, act, row0, m - 1, nsb, lane, T + (size_t)(32 + wave * 2) * stride, stride);
     __syncthreads();
     if (wave != 0) return;
-    const float s = q4k_ordered_sum<3>(T + (size_t)lane * stride, nsb);  // (three records ahead: a fourth does not fit the 64 registers)
+    const float s = q4k_ordered_sum<3>(T + (size_t)lane * stride, nsb);  // (three records ahead: a fourth does not fit the 64 registers.  A lane a chain: 19.3 us, not 19.0)
     const float u = __shfl(s, (lane & 31) + 32, 64);
     if (lane < 32) h[(int)blockIdx.x * 32 + lane] = silu_mul(s, u, exp_tab);
     return;
@@ -461,12 +461,12 @@ __global__ __launch_bounds__(1024) void k_kq_res(KqMat w, const float* __restric
     const int stride = q4k_rec_stride(nsb);
     float* T = (float*)((char*)lds_act + kq_rec_at(nsb * 256, false));
     kq_terms<SIX, 1, P>(p, w, kq_act(l), row, row, nsb, lane, T + (size_t)wave * stride, stride);
-    __syncthreads();
-    if (wave != 0) return;
-    const float s = q4k_ordered_sum(T + (size_t)(lane & 15) * stride, nsb);
-    if (lane < 16) hv[lane] = s;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_wave_barrier();
+    const float s = q4k_ordered_sum16(T + (size_t)wave * stride, nsb, lane);
+    if (lane == 0) hv[wave] = s;
+    __syncthreads();
+    if (wave != 0) return;
     kq_res_out(hv, res, x, csums, lane);
     return;
   }

@@ -589,6 +589,34 @@ __device__ __forceinline__ float q4k_ordered_sum(const float* __restrict__ t, in
   for (int l = 0; l < 8; l++) sumf += sums[l];
   return sumf;
 }
+// The same with a lane per chain: lane l of a group of 16 runs chain l (8: the minimum term) of the group's row, and the group adds the nine ends in order
+// (every lane gets the sum).  A row's nine chains in one lane keep the wave for nine times as many adds: us a launch so / a lane a chain, 8B shape,
+// classifier 57.3 / 49.2, ffn_down (one wave for the workgroup's 16 rows) 13.5 / 12.5, q | k | v 10.4 / 9.7.
+__device__ __forceinline__ float q4k_ordered_sum16(const float* __restrict__ t, int nsb, int lane) {
+  const int l = (lane & 15) < 9 ? lane & 15 : 8;
+  const float sign = l == 8 ? -1.0f : 1.0f;  // (x * +-1 is exact: s - x and s + x, rounded once)
+  t += l;
+  float s = 0.0f;
+  int sb = 0;
+  for (; sb + 8 <= nsb; sb += 8) {
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) v[u] = t[(sb + u) * 12];
+#pragma unroll
+    for (int u = 0; u < 8; u++) s = __builtin_fmaf(v[u], sign, s);
+  }
+  for (; sb < nsb; sb++) s = __builtin_fmaf(t[sb * 12], sign, s);
+  float sum = dpp_f<0x158>(s);  // (row_newbcast: lane n of the 16 to all of them)
+  sum += dpp_f<0x150>(s);
+  sum += dpp_f<0x151>(s);
+  sum += dpp_f<0x152>(s);
+  sum += dpp_f<0x153>(s);
+  sum += dpp_f<0x154>(s);
+  sum += dpp_f<0x155>(s);
+  sum += dpp_f<0x156>(s);
+  sum += dpp_f<0x157>(s);
+  return sum;
+}
 // the records of R rows of a Q4_K matrix: T[r * stride + sb * 12 ..]; lane = one 16-byte piece, as rows_partial_q4k
 template <int R, bool HDR_DPP>
 __device__ __forceinline__ void rows_terms_q4k(const i32x4* __restrict__ wq, const i32x4* __restrict__ wh, const ActQ8_K& act, int row0, int m,

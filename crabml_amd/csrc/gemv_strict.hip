@@ -435,10 +435,10 @@ __global__ __launch_bounds__(256) void k_gemv_exact_q4k(const char* __restrict__
     rows_terms_q4k<R, true>(wq, wh, act, row0, m, nsb, lane, T, stride);
     __builtin_amdgcn_s_waitcnt(0xC07F);
     __builtin_amdgcn_wave_barrier();
-    if (lane < R && row0 + lane < m) {
-      const float sumf = q4k_ordered_sum(T + (size_t)lane * stride, nsb);
-      out[row0 + lane] = add ? sumf + add[row0 + lane] : sumf;
-    }
+    static_assert(R <= 4, "a group of 16 lanes per row");
+    const int r = lane >> 4, row = row0 + r;
+    const float sumf = q4k_ordered_sum16(T + (size_t)(r < R ? r : R - 1) * stride, nsb, lane);
+    if ((lane & 15) == 0 && r < R && row < m) out[row] = add ? sumf + add[row] : sumf;
     return;
   }
   // Q5_K (planes in the file's element order): the activation dwords masked to one byte per v_dot4
@@ -774,6 +774,10 @@ int launch_gemv_strict(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m
           const size_t lk = (size_t)WAVES * R * (k / 256) * 12 * sizeof(float);
           if (lk > 48 * 1024) {
             done = false;
+          } else if (w->dtype == CRABML_HIP_Q4_K && m >= 32768 && 2 * lk <= 48 * 1024) {
+            // four rows a wave where that leaves a CU its 32 waves: the rhs is read once for all of them, and their chains run side by side (128256 x 4096: 49.2 us
+            // with two, 45.7 with four; 57.3 with a row's nine chains in one lane)
+            STRICT_LAUNCH((k_gemv_exact_q4k<false, 2 * R>), (k_gemv_exact_q4k<false, 2 * R, true>), (unsigned)((m + 2 * R * WAVES - 1) / (2 * R * WAVES)), 64 * WAVES, 2 * lk, wp, w->wl.off_scale, ak, o, add, (int)m, (int)(k / 256));
           } else if (w->dtype == CRABML_HIP_Q4_K) {
             STRICT_LAUNCH((k_gemv_exact_q4k<false, R>), (k_gemv_exact_q4k<false, R, true>), grid, 64 * WAVES, lk, wp, w->wl.off_scale, ak, o, add, (int)m, (int)(k / 256));
           } else {

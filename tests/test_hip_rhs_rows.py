@@ -78,3 +78,17 @@ def test_strict_q4_k_on_the_matrix_cores(ca, m, k, rows, levels):
     for r in range(rows):
         one = w.matmul_vec(ca.HipTensor.new(x[r], [k], dev)).export()
         assert np.array_equal(got[r].view(np.uint32), one.view(np.uint32)), r
+
+
+@pytest.mark.parametrize("k", [256, 2304])
+def test_strict_q4_k_rows_of_large_matrices(ca, k):
+    """from 32768 rows of the matrix on a wave takes four of them, below two: the same bits"""
+    m, rng, dev = 32773, np.random.default_rng(k), ca.HipTensorDevice(0, False, 0, True)
+    raw = synth.random_blocks(rng, m * k, synth.TYPE_BY_NAME["Q4_K"])
+    x = ca.HipTensor.new(rng.standard_normal(k).astype(np.float32), [k], dev)
+    got = ca.HipTensor.from_cpu(raw, [m, k], ca.GGMLType.Q4K, dev).matmul_vec(x).export()
+    size = raw.size // m
+    for first, n in ((0, 77), (16384, 64), (m - 77, 77)):
+        part = raw.reshape(-1)[first * size:(first + n) * size].copy()
+        want = ca.HipTensor.from_cpu(part, [n, k], ca.GGMLType.Q4K, dev).matmul_vec(x).export()
+        assert np.array_equal(got[first:first + n].view(np.uint32), want.view(np.uint32)), first
