@@ -207,6 +207,39 @@ __device__ __forceinline__ T ld(const T* p) {
     return *p;
 }
 
+// Q8_0 / Q8_1 quantizer of 32-element blocks, 8 lanes of 4 consecutive elements each (buf_q8_0.rs:87-134, buf_q8_1.rs:90-129; quant_lane32's arithmetic,
+// fused_common.hpp: the maximum and the integer sum do not depend on the order).  aux: the sum of the quants, or Q8_1's s as f16 bits; all lanes of the block get d and aux.
+struct QLane4 {
+  unsigned packed;
+  unsigned short d;
+  int aux;
+};
+template <bool Q81>
+__device__ __forceinline__ QLane4 quant_quad8(const f32x4 v) {
+  float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+  amax = fmaxf(amax, dpp_f<0xB1>(amax));
+  amax = fmaxf(amax, dpp_f<0x4E>(amax));
+  amax = fmaxf(amax, dpp_f<0x141>(amax));
+  const float dd = amax / 127.0f;
+  QLane4 o;
+  o.d = f2h(dd);
+  int q[4], s = 0;
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    if constexpr (Q81)
+      q[e] = (int)fminf(fmaxf(v[e] / dd, -128.0f), 127.0f);  // Rust f32::max / min return the non-NaN operand
+    else
+      q[e] = (int)(signed char)(unsigned char)((unsigned)rs_f32_as_i32(v[e] / dd) & 0xffu);  // `as i8` from i32 wraps
+    s += q[e];
+  }
+  s += dpp_i<0xB1>(s);
+  s += dpp_i<0x4E>(s);
+  s += dpp_i<0x141>(s);
+  o.aux = Q81 ? (int)f2h((float)s * dd) : s;
+  o.packed = ((unsigned)q[0] & 0xffu) | (((unsigned)q[1] & 0xffu) << 8) | (((unsigned)q[2] & 0xffu) << 16) | ((unsigned)q[3] << 24);
+  return o;
+}
+
 // Q8_K quantizer of one 256-element super-block by one wave, 4 consecutive elements per lane
 // (buf_q8_k.rs:84-131: scale = -128 / (the FIRST element of maximal |x|), round half away from zero, min(127),
 // `as i8` saturation).  Returns the 4 quants packed into a dword; `quad_sum` = this lane's quad's sum of 16 quants

@@ -72,4 +72,21 @@ __device__ __forceinline__ void rows_to_f16_piece(const char* __restrict__ p, si
 // the f16 value of a quant: q * d in f32 (Q8_0 / Q8_1: d is the STORED f16 scale -- exact product, one rounding), rounded once
 __device__ __forceinline__ unsigned short f16w_value(int q, float d) { return f2h((float)q * d); }
 
+// four of a row's B' values from the quants 0 .. 3 of a dword that stand 0, 2, 1, 3 there
+__device__ __forceinline__ void f16w_store4(unsigned short* at, unsigned quants, float d) {
+  const unsigned short v0 = f16w_value((int)(signed char)(quants & 0xffu), d), v1 = f16w_value((int)(signed char)((quants >> 8) & 0xffu), d);
+  const unsigned short v2 = f16w_value((int)(signed char)((quants >> 16) & 0xffu), d), v3 = f16w_value((int)(signed char)(quants >> 24), d);
+  *(unsigned long long*)at = (unsigned long long)(v0 | ((unsigned)v2 << 16)) | ((unsigned long long)(v1 | ((unsigned)v3 << 16)) << 32);
+}
+// B' of super-block sb from a wave's quantizer (q8k_wave_quant: lane has the quants of elements 4 lane .. 4 lane + 3): f16w_pos_q8k's places, eight bytes a
+// lane -- order 2 keeps four consecutive elements together, order 1 the four of a class, which is what the class-major dword holds
+__device__ __forceinline__ void f16w_store_q8k(unsigned short* __restrict__ xrow, int order, int sb, int lane, unsigned packed, float d) {
+  if (order == 1) {
+    const int l = (lane & 1) * 4 + ((lane >> 1) & 3);  // (the dword's class: q8k_class_major_at)
+    f16w_store4(xrow + (4 * (2 * sb + (l >> 2)) + (lane >> 4)) * 32 + 8 * (l & 3) + 4 * (lane >> 3 & 1), q8k_class_major(lane, packed), d);
+  } else {
+    f16w_store4(xrow + (4 * (2 * sb + (lane >> 5)) + 2 * (lane >> 3 & 1) + (lane >> 2 & 1)) * 32 + 8 * (lane & 3) + 4 * (lane >> 4 & 1), packed, d);
+  }
+}
+
 }  // namespace crabml_hip

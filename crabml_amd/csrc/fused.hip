@@ -1187,11 +1187,8 @@ int enqueue_segment_kq(crabml_hip_llama* c, int seg) {
   };
   if (seg == 2 * L) {
     const ActLayout al = act_layout(CRABML_HIP_Q8_K, (size_t)dim);
-    auto norm = [&](auto kernel) {
-      kernel<<<1, 1024, norm_lds_bytes(dim), st>>>(c->x, nullptr, (const float*)c->rms_final->ptr, dim, g.rms_norm_eps, c->xn, c->act_dim, al.total, al.off_d, al.off_aux,
-                                                   al.off_p, ORD ? 0 : 1, nullptr, 0, nullptr, 0, 0);
-    };
-    dim <= 4096 ? norm(k_norm_quant_rows_k<4>) : norm(k_norm_quant_rows_k<12>);
+    launch_norm_quant_rows<CRABML_HIP_Q8_K>(st, 1, dim, c->x, (const float*)nullptr, (const float*)c->rms_final->ptr, dim, g.rms_norm_eps, c->act_dim, al.total, al.off_d,
+                                            al.off_aux, al.off_p, ORD ? 0 : 1, (unsigned short*)nullptr, 0, (const float*)nullptr, (size_t)0, 0);
     if (prof)
       CH_TRY(prof_begin(dev, &pr, c->output->dtype, 5,
                         (double)c->vocab_l * (double)(dim / block_elems(c->output->dtype)) * (double)block_bytes(c->output->dtype) + 4.0 * dim + 4.0 * c->vocab_l));
@@ -1713,75 +1710,26 @@ int prefill_chunk(crabml_hip_llama* c, const uint32_t* tokens, size_t B, size_t 
   // Q8_0 / Q8_1 rhs: residual add + RMSNorm + quantize as one launch per row (k_norm_quant_rows), SiLU * mul + quantize as one
   // (k_gateup_epi_quant): the (rows, dim) / (rows, hidden) f32 intermediates make one trip through memory instead of three
   const bool fuse_rows = (c->qt == CRABML_HIP_Q8_0 || c->qt == CRABML_HIP_Q8_1) && !(g.flags & CRABML_HIP_LLAMA_NO_PREFILL_ROW_FUSION);
-  // Q8_K rhs (K-quant layers): the same for residual add + RMSNorm + quantize (k_norm_quant_rows_k); SiLU * mul keeps its own launch
-  // (from 192 rows: one 1024-thread workgroup per row is a chain of four barriers -- below, the four small launches run 1-2 % faster)
-  const bool fuse_k = c->qt == CRABML_HIP_Q8_K && dim % 256 == 0 && B >= 192 && !(g.flags & CRABML_HIP_LLAMA_NO_PREFILL_ROW_FUSION);
+  // Q8_K rhs (K-quant layers): the same for residual add + RMSNorm + quantize; SiLU * mul keeps its own launch
+  const bool fuse_k = c->qt == CRABML_HIP_Q8_K && dim % 256 == 0 && !(g.flags & CRABML_HIP_LLAMA_NO_PREFILL_ROW_FUSION);
   const bool fuse_norm = fuse_rows || fuse_k;
   const ActLayout ald = act_layout(c->qt == CRABML_HIP_F32 ? CRABML_HIP_Q8_0 : c->qt, (size_t)dim);
   const ActLayout alh = act_layout(c->qt == CRABML_HIP_F32 ? CRABML_HIP_Q8_0 : c->qt, (size_t)hidden);
   // pending = the wo / ffn_down output that has not been added to x yet (folded into the next norm)
   // nparts: `pending` is piece 0 of a GEMM cut into k pieces, the others wait in pf_split (gemm's defer)
   auto norm_quant_rows = [&](const float* wn, float eps, float* pending, const crabml_hip_buf* next, int nparts = 0) -> const void* {
-    const bool q81 = c->qt == CRABML_HIP_Q8_1;
     int order = 0;
     unsigned short* xh = (unsigned short*)xh_target(next, dim, &order);
-    const size_t pstride = B * (size_t)dim;
-    // Q8_0 / Q8_1 rows of 4096 / 8192 elements: the 256-thread form (a thread owns half a quant block / a whole one; prefill_rows.hpp)
-    static const bool rows_1024 = [] {  // lab hook (CRABML_HIP_TEST_HOOKS=1 CRABML_HIP_NORM_ROWS_1024=1): the 1024-thread kernel
-      const char* h = getenv("CRABML_HIP_TEST_HOOKS");
-      const char* e = getenv("CRABML_HIP_NORM_ROWS_1024");
-      return h && h[0] == '1' && e && e[0] == '1';
-    }();
-    if (!fuse_k && !rows_1024 && (dim == 4096 || dim == 8192) && !(g.flags & CRABML_HIP_LLAMA_PREFILL_SEPARATE_F16_ROWS)) {
-#define CRABML_NQW(E_, Q_)                                                                                                            \
-  k_norm_quant_rows_w<E_, Q_><<<rows, 256, 0, st>>>(c->pf_x, pending, wn, dim, eps, c->pf_act_dim, ald.total, ald.off_d, ald.off_aux, \
-                                                    half, xh, c->pf_split, pstride, nparts)
-      if (dim == 4096) {
-        if (q81)
-          CRABML_NQW(16, true);
-        else
-          CRABML_NQW(16, false);
-      } else {
-        if (q81)
-          CRABML_NQW(32, true);
-        else
-          CRABML_NQW(32, false);
-      }
-#undef CRABML_NQW
-      xh_of = xh ? c->pf_act_dim : nullptr;
-      xh_order = order;
-      return c->pf_act_dim;
-    }
-    if (fuse_k) {
-      if (dim <= 4096)
-        k_norm_quant_rows_k<4><<<rows, 1024, norm_lds, st>>>(c->pf_x, pending, wn, dim, eps, c->pf_xn, c->pf_act_dim, ald.total, ald.off_d,
-                                                            ald.off_aux, ald.off_p, half, xh, order, c->pf_split, pstride, nparts);
-      else
-        k_norm_quant_rows_k<12><<<rows, 1024, norm_lds, st>>>(c->pf_x, pending, wn, dim, eps, c->pf_xn, c->pf_act_dim, ald.total, ald.off_d,
-                                                             ald.off_aux, ald.off_p, half, xh, order, c->pf_split, pstride, nparts);
-      xh_of = xh ? c->pf_act_dim : nullptr;
-      xh_order = order;
-      return c->pf_act_dim;
-    }
-#define CRABML_NQR(NIT_, Q_)                                                                                                         \
-  if (xh || nparts > 0)                                                                                                              \
-    k_norm_quant_rows_h<NIT_, Q_><<<rows, 1024, norm_lds, st>>>(c->pf_x, pending, wn, dim, eps, c->pf_act_dim, ald.total, ald.off_d,  \
-                                                                ald.off_aux, half, xh, c->pf_split, pstride, nparts);                \
-  else                                                                                                                               \
-    k_norm_quant_rows<NIT_, Q_><<<rows, 1024, norm_lds, st>>>(c->pf_x, pending, wn, dim, eps, c->pf_act_dim, ald.total, ald.off_d,    \
-                                                              ald.off_aux, half)
-    if (dim <= 4096) {
-      if (q81)
-        CRABML_NQR(4, true);
-      else
-        CRABML_NQR(4, false);
-    } else {
-      if (q81)
-        CRABML_NQR(12, true);
-      else
-        CRABML_NQR(12, false);
-    }
-#undef CRABML_NQR
+    auto launch = [&](auto qt) {
+      launch_norm_quant_rows<decltype(qt)::value>(st, B, dim, c->pf_x, (const float*)pending, wn, dim, eps, c->pf_act_dim, ald.total, ald.off_d, ald.off_aux, ald.off_p, half,
+                                                  xh, order, (const float*)c->pf_split, B * (size_t)dim, nparts);
+    };
+    if (fuse_k)
+      launch(std::integral_constant<int, CRABML_HIP_Q8_K>{});
+    else if (c->qt == CRABML_HIP_Q8_1)
+      launch(std::integral_constant<int, CRABML_HIP_Q8_1>{});
+    else
+      launch(std::integral_constant<int, CRABML_HIP_Q8_0>{});
     xh_of = xh ? c->pf_act_dim : nullptr;
     xh_order = order;
     return c->pf_act_dim;

@@ -224,7 +224,18 @@ static bool launch_t(crabml_hip_device* dev, const KqxArgs& a) {
 // false: not covered (the caller's row kernels take it)
 bool launch_gemm_exact_kq(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m, size_t k, const void* act, size_t b, float* out, const float* add) {
   const int nsb = (int)(k / 256);
-  const int nt = b <= 16 ? 1 : b <= 32 ? 2 : 4;
+  // tiles of 16 rows a workgroup: a workgroup of one, two and four costs as 26 : 50 : 81 (a prompt on four layers of the 8B shape, us: 77 rows 1753 / 1979 / 2146, 64 rows
+  // 1558 / 1442 / 1401, 100 rows 2320 / 2437 / 2170, 17 rows 995 / 1015 / 1399), empty tiles included
+  const size_t tiles = (b + 15) / 16;
+  int nt = 1;
+  size_t least = tiles * 26;
+  for (int n : {2, 4}) {
+    const size_t cost = (tiles + n - 1) / n * (n == 2 ? 50 : 81);
+    if (cost < least) {
+      least = cost;
+      nt = n;
+    }
+  }
   if (w->dtype != CRABML_HIP_Q4_K || b < KQX_ROWS || m == 0 || nsb == 0) return false;
   const ActLayout al = act_layout(CRABML_HIP_Q8_K, k);
   KqxArgs a;

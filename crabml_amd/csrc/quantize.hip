@@ -16,65 +16,27 @@
 
 namespace crabml_hip {
 
-// one 32-lane group per block; 256 threads = 8 blocks per workgroup
-__global__ __launch_bounds__(256) void k_quantize_q8_0(const float* __restrict__ x, signed char* __restrict__ q,
-                                                       unsigned short* __restrict__ d, int* __restrict__ isum,
-                                                       size_t nblocks, size_t row_elems, size_t row_bytes, unsigned short* __restrict__ xh) {
+// eight lanes per block, four consecutive elements each: a wave's request and its stores are whole lines (a lane per element: 512 rows of 4096 with B'
+// 8.6 us)
+template <bool Q81>
+__global__ __launch_bounds__(256) void k_quantize_q8(const float* __restrict__ x, char* __restrict__ planes, size_t off_d, size_t off_aux, size_t nblocks,
+                                                     size_t row_elems, size_t row_bytes, unsigned short* __restrict__ xh) {
   // blockIdx.y: row of a batch (x rows of row_elems floats; one set of planes every row_bytes bytes)
   // xh (nullable): the row's pre-scaled f16 plane for the fast prompt pass's GEMM (f16w_rows.hpp), written next to the planes
-  x += blockIdx.y * row_elems;
-  q += blockIdx.y * row_bytes;
-  d = (unsigned short*)((char*)d + blockIdx.y * row_bytes);
-  isum = (int*)((char*)isum + blockIdx.y * row_bytes);
-  size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  size_t blk = gid >> 5;
-  int j = (int)(gid & 31);
-  bool live = blk < nblocks;
-  float v = live ? x[blk * 32 + j] : 0.f;
-  float amax = half_max_f32(fabsf(v));  // (256-thread blocks of whole waves: all lanes converged)
-  float dd = amax / 127.0f;
-  float t = v / dd;
-  int qi = rs_f32_as_i32(t);
-  signed char q8 = (signed char)(unsigned char)((unsigned)qi & 0xffu);  // `as i8` from i32 wraps
-  int s = half_sum_i32((int)q8);
-  if (live) {
-    q[blk * 32 + j] = q8;
-    if (j == 0) {
-      d[blk] = f2h(dd);
-      isum[blk] = s;
-    }
-    if (xh) xh[blockIdx.y * row_elems + blk * 32 + f16w_slot_of_elem(j)] = f16w_value((int)q8, h2f(f2h(dd)));
+  char* p = planes + blockIdx.y * row_bytes;
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, blk = i >> 3;
+  const bool live = blk < nblocks;
+  const QLane4 o = quant_quad8<Q81>(((const f32x4*)(x + blockIdx.y * row_elems))[live ? i : 0]);
+  if (!live) return;  // (whole blocks)
+  ((unsigned*)p)[i] = o.packed;
+  if ((i & 7) == 0) {
+    ((unsigned short*)(p + off_d))[blk] = o.d;
+    if constexpr (Q81)
+      ((unsigned short*)(p + off_aux))[blk] = (unsigned short)o.aux;
+    else
+      ((int*)(p + off_aux))[blk] = o.aux;
   }
-}
-
-__global__ __launch_bounds__(256) void k_quantize_q8_1(const float* __restrict__ x, signed char* __restrict__ q,
-                                                       unsigned short* __restrict__ d, unsigned short* __restrict__ sp,
-                                                       size_t nblocks, size_t row_elems, size_t row_bytes, unsigned short* __restrict__ xh) {
-  x += blockIdx.y * row_elems;
-  q += blockIdx.y * row_bytes;
-  d = (unsigned short*)((char*)d + blockIdx.y * row_bytes);
-  sp = (unsigned short*)((char*)sp + blockIdx.y * row_bytes);
-  size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  size_t blk = gid >> 5;
-  int j = (int)(gid & 31);
-  bool live = blk < nblocks;
-  float v = live ? x[blk * 32 + j] : 0.f;
-  float amax = half_max_f32(fabsf(v));
-  float dd = amax / 127.0f;
-  float sv = v / dd;
-  // Rust f32::max / f32::min return the non-NaN operand: NaN.max(-128) = -128
-  float c = fminf(fmaxf(sv, -128.0f), 127.0f);
-  int qi = (int)c;  // |c| <= 128: exact truncation
-  int s = half_sum_i32(qi);
-  if (live) {
-    q[blk * 32 + j] = (signed char)qi;
-    if (j == 0) {
-      d[blk] = f2h(dd);
-      // s accumulates small integers in f32 in the reference (exact), then `s *= d`
-      sp[blk] = f2h((float)s * dd);
-    }
-    if (xh) xh[blockIdx.y * row_elems + blk * 32 + f16w_slot_of_elem(j)] = f16w_value(qi, h2f(f2h(dd)));
-  }
+  if (xh) f16w_store4(xh + blockIdx.y * row_elems + blk * 32 + 8 * (i & 3) + 4 * (i >> 2 & 1), o.packed, h2f(o.d));
 }
 
 // one wave per 256-element super-block, 4 consecutive elements per lane
@@ -95,12 +57,7 @@ __global__ __launch_bounds__(256) void k_quantize_q8_k(const float* __restrict__
   q8k_store_class_major(qp + blk * 256, lane, o.packed);  // the plane the Q4_K kernels read
   if ((lane & 3) == 0) bsums[blk * 16 + (lane >> 2)] = (short)o.quad_sum;
   if (lane == 0) d[blk] = o.d;
-  if (xh) {  // (xh_order 1 / 2: the k-slot order of Q4_K / Q6_K weights)
-    unsigned short* xr = xh + blockIdx.y * row_elems;
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-      xr[f16w_pos_q8k(xh_order, (int)blk, 4 * lane + i)] = f16w_value((int)(signed char)((o.packed >> (8 * i)) & 0xffu), o.d);
-  }
+  if (xh) f16w_store_q8k(xh + blockIdx.y * row_elems, xh_order, (int)blk, lane, o.packed, o.d);  // (xh_order 1 / 2: the k-slot order of Q4_K / Q6_K weights)
 }
 
 __global__ __launch_bounds__(256) void k_quantize_f16(const float* __restrict__ x, unsigned short* __restrict__ h,
@@ -124,18 +81,14 @@ void launch_quantize_act_rows(hipStream_t st, uint32_t qtype, const float* x, si
   const unsigned ry = (unsigned)rows;
   char* p = (char*)planes;
   switch (qtype) {
-    case CRABML_HIP_Q8_0: {
-      size_t nb = n / 32;
-      unsigned grid = (unsigned)((nb * 32 + 255) / 256);
-      k_quantize_q8_0<<<dim3(grid, ry), 256, 0, st>>>(x, (signed char*)p, (unsigned short*)(p + al.off_d), (int*)(p + al.off_aux),
-                                           nb, n, al.total, (unsigned short*)xh);
-      break;
-    }
+    case CRABML_HIP_Q8_0:
     case CRABML_HIP_Q8_1: {
-      size_t nb = n / 32;
-      unsigned grid = (unsigned)((nb * 32 + 255) / 256);
-      k_quantize_q8_1<<<dim3(grid, ry), 256, 0, st>>>(x, (signed char*)p, (unsigned short*)(p + al.off_d),
-                                           (unsigned short*)(p + al.off_aux), nb, n, al.total, (unsigned short*)xh);
+      const size_t nb = n / 32;
+      const dim3 grid((unsigned)((nb * 8 + 255) / 256), ry);
+      if (qtype == CRABML_HIP_Q8_0)
+        k_quantize_q8<false><<<grid, 256, 0, st>>>(x, p, al.off_d, al.off_aux, nb, n, al.total, (unsigned short*)xh);
+      else
+        k_quantize_q8<true><<<grid, 256, 0, st>>>(x, p, al.off_d, al.off_aux, nb, n, al.total, (unsigned short*)xh);
       break;
     }
     case CRABML_HIP_Q8_K: {

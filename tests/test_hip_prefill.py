@@ -251,6 +251,24 @@ def test_prefill_row_fusion_k_quants_equals_the_separate_launches(ca, fmt):
             assert list(a.decode_greedy(nxt, 5)) == list(b.decode_greedy(nxt, 5))
 
 
+# rows around the row kernel's groups of 1024 elements: less than one, a part of the next, all twelve; Q8_0, Q8_1 and Q8_K
+@pytest.mark.parametrize("fmt,width", [("Q8_0", 64), ("Q4_1", 960), ("Q8_0", 1088), ("Q4_0", 2112), ("Q4_1", 4160), ("Q8_0", 8256), ("Q8_0", 12288),
+                                       ("Q4_K", 256), ("Q6_K", 1280), ("Q4_K", 2304), ("Q4_K", 4352), ("Q4_K", 8448), ("Q6_K", 12288)])
+def test_row_kernel_of_every_width_equals_the_separate_launches(ca, fmt, width):
+    """residual add + RMSNorm + quantize (+ the next GEMM's f16 planes from 32 rows on) as one launch against one launch each (flag 262144): the same bits"""
+    shape = synth.ModelShape("rows", width, 256, 2, width // 64, 1, 96, 64, 1e-5, None)
+    model = synth.build_model(shape, synth.TYPE_BY_NAME[fmt], seed=width)
+    toks = [(5 * i + 1) % 96 for i in range(40)]
+    for strict in (False, True):
+        dev = ca.HipTensorDevice(0, False, 0, strict)
+        conf, w = synth.to_hip(model, dev)
+        a, b = ca.HipLlamaRunner(conf, w, dev, 64, True), ca.HipLlamaRunner(conf, w, dev, 64, True, extra_flags=262144)
+        for n in (3, 40):
+            a.reset(), b.reset()
+            la, lb = a.prefill(toks[:n]), b.prefill(toks[:n])
+            assert np.array_equal(la.view(np.uint32), lb.view(np.uint32)), (strict, n)
+
+
 PREFILL_INT8_GEMM = 524288  # CRABML_HIP_LLAMA_PREFILL_INT8_GEMM (include/crabml_hip_debug.h)
 
 
