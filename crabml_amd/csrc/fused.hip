@@ -523,6 +523,8 @@ int enqueue_front(crabml_hip_llama* c, bool pick) {
     tp.pv = c->am_val;
     tp.pi = c->am_idx;
     tp.nparts = ARGMAX_BLOCKS;
+    if (c->vocab_l <= ARGMAX_ONE) tp.logits = c->logits + c->vocab_off;
+    tp.n = c->vocab_l;
     tp.out_cap = c->out_cap;
     tp.pos = c->state + 1;
     tp.step = c->state + 2;
@@ -533,7 +535,7 @@ int enqueue_front(crabml_hip_llama* c, bool pick) {
   FrontOut o{(signed char*)c->act_dim, (signed char*)(c->act_dim + al.off_p), (void*)(c->act_dim + al.off_d), (void*)(c->act_dim + al.off_aux)};
   if (front == FRONT_SUMS) o.d = c->rsums;
   auto go = [&](auto kernel) {
-    launch_k(dev->stream, prof ? &nr : nullptr, kernel, dim3(1), dim3(1024), front == FRONT_ROW ? 0 : norm_lds_bytes(dim),
+    launch_k(dev->stream, prof ? &nr : nullptr, kernel, dim3(1), dim3(1024), 0,
              (const char*)c->token_embed->ptr, (int)c->token_embed->dtype, c->token_embed->wl.off_scale, tp, dim, c->x, (const float*)c->rms_att[0]->ptr,
              g.rms_norm_eps, o, dev->strict_order ? 0 : 1);
   };
@@ -577,6 +579,7 @@ int enqueue_classifier_and_sampler(crabml_hip_llama* c, const void* cls_act, cra
     CH_HIP(dev, hipGetLastError());
     return 0;
   }
+  if (c->lead && c->vocab_l <= ARGMAX_ONE) return enqueue_front(c, true);  // (which reads the logits itself)
   k_argmax_partial<<<ARGMAX_BLOCKS, 256, 0, st>>>(out, c->vocab_l, c->am_val, c->am_idx, c->vocab_off, 0);
   if (c->lead) return enqueue_front(c, true);
   if (c->split_vocab && c->comm && c->comm->p2p)

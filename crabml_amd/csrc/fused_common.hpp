@@ -252,7 +252,9 @@ __global__ __launch_bounds__(1024) void k_norm_f32(float* __restrict__ x, const 
 // With several steps in a graph (run_steps), us a request, before -> after: 57 tokens of the 15M-parameter model in Q8_0 6482 -> 6047, 88 tokens of 8
 // layers of the 8B shape in Q4_0 24840 -> 24232.
 enum { FRONT_ROW = 0, FRONT_Q8_0 = 1, FRONT_Q8_1 = 2, FRONT_Q8_K = 3, FRONT_SUMS = 4 };  // what is left beside x: nothing, the normed row's planes, sums of squares of 16
-struct TokenPick {  // pv == nullptr: the token is *token
+struct TokenPick {  // pv == nullptr: the token is *token; logits: the n of them in place of the partials
+  const float* logits = nullptr;
+  int n = 0;
   const float* pv = nullptr;
   const int* pi = nullptr;
   int nparts = 0, out_cap = 0;
@@ -263,13 +265,18 @@ struct FrontOut {
   signed char *q = nullptr, *qp = nullptr;  // (qp: class-major copy, Q8_K)
   void *d = nullptr, *aux = nullptr;        // scales; block sums
 };
-template <int NIT>
+// a thread's elements of the row: QUADS of four, 4096 apart, or one every 1024
+template <bool QUADS>
+__device__ __forceinline__ int front_elem(int it) {
+  return QUADS ? (it >> 2) * 4096 + (int)threadIdx.x * 4 + (it & 3) : it * 1024 + (int)threadIdx.x;
+}
+template <int NIT, bool QUADS>
 __device__ __forceinline__ void embed_row(const char* __restrict__ w, int dtype, size_t off_scale, size_t base, int dim, float (&v)[NIT]) {
   // (one format at a time: with the format's switch inside the loop each element's request waited for the one before it)
   auto all = [&](auto t) {
 #pragma unroll
     for (int it = 0; it < NIT; it++) {
-      const int i = it * 1024 + (int)threadIdx.x;
+      const int i = front_elem<QUADS>(it);
       const float e = dequant_elem(w, decltype(t)::value, off_scale, base + (i < dim ? i : dim - 1));
       v[it] = i < dim ? e : 0.f;
     }
@@ -285,28 +292,58 @@ __device__ __forceinline__ void embed_row(const char* __restrict__ w, int dtype,
     default:
 #pragma unroll 1
       for (int it = 0; it < NIT; it++) {
-        const int i = it * 1024 + (int)threadIdx.x;
+        const int i = front_elem<QUADS>(it);
         v[it] = i < dim ? dequant_elem(w, dtype, off_scale, base + i) : 0.f;
       }
   }
 }
+// A scan of squares from -0.0 through 4 or 8 lanes of four elements each (last = 3 or 7), handed from lane to lane: the group's last lane has it
+__device__ __forceinline__ float quad_square_scan(const f32x4 v, int lane, int last) {
+  const f32x4 q = v * v;
+  float t = (((-0.0f + q[0]) + q[1]) + q[2]) + q[3];
+  for (int k = 1; k <= last; k++) {
+    const float u = (((dpp_f<0x111>(t) + q[0]) + q[1]) + q[2]) + q[3];  // (row_shr:1: the lane before goes first)
+    t = (lane & last) == k ? u : t;
+  }
+  return t;
+}
+// sums of nchunks chunks in norm_quant_regs' order, by every wave for itself
+__device__ __forceinline__ float chunk_sums(const float* cs, int nchunks, int lane, int half) {
+  float sum = 0.0f;
+  for (int base = 0; base < nchunks; base += 64) {
+    const float v = base + lane < nchunks ? cs[base + lane] : 0.0f;
+    if (half) {
+      sum += wave_sum_f32(v);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 64; i++) sum += rl_f(v, i);
+    }
+  }
+  return sum;
+}
 template <int NIT, int FRONT>
 __global__ __launch_bounds__(1024) void k_step_front(const char* __restrict__ table, int dtype, size_t off_scale, TokenPick pick, int dim, float* __restrict__ x,
                                                      const float* __restrict__ wn, float eps, FrontOut o, int half) {
-  extern __shared__ __attribute__((aligned(16))) float lds[];
-  __shared__ float s_rms;
+  constexpr bool QUADS = FRONT != FRONT_ROW;  // (rows of whole chunks)
+  __shared__ float s_pick[16], s_chunks[NIT * 32];
+  __shared__ int s_pick_at[16];
   const int tid = threadIdx.x, lane = tid & 63;
-  float xv[NIT], wv[NIT];
-  if constexpr (FRONT != FRONT_ROW && FRONT != FRONT_SUMS) {
+  float xv[NIT];
+  f32x4 wv[NIT / 4];
+  if constexpr (QUADS && FRONT != FRONT_SUMS) {
 #pragma unroll
-    for (int it = 0; it < NIT; it++) wv[it] = it * 1024 + tid < dim ? wn[it * 1024 + tid] : 0.f;
+    for (int j = 0; j < NIT / 4; j++) wv[j] = ((const f32x4*)wn)[j * 4096 + tid * 4 < dim ? j * 1024 + tid : 0];
   }
   int token;
   if (pick.pv != nullptr) {
     float bv = -INFINITY;
     int bi = -1;
-    for (int i = lane; i < pick.nparts; i += 64) argmax_combine(bv, bi, pick.pv[i], pick.pi[i]);
-    argmax_wave(bv, bi);
+    if (pick.logits != nullptr) {
+      bi = argmax_row(pick.logits, pick.n, s_pick, s_pick_at);
+    } else {
+      for (int i = lane; i < pick.nparts; i += 64) argmax_combine(bv, bi, pick.pv[i], pick.pi[i]);
+      argmax_wave(bv, bi);
+    }
     token = bi;
     if (tid == 0) {
       *pick.token = bi;
@@ -319,40 +356,51 @@ __global__ __launch_bounds__(1024) void k_step_front(const char* __restrict__ ta
   } else {
     token = *pick.token;
   }
-  embed_row<NIT>(table, dtype, off_scale, (size_t)token * dim, dim, xv);
-#pragma unroll
-  for (int it = 0; it < NIT; it++)
-    if (it * 1024 + tid < dim) x[it * 1024 + tid] = xv[it];
-  NormLds L{lds, lds + dim};
-  if constexpr (FRONT == FRONT_SUMS) {  // (the halves of norm_quant_regs' chunks, as k_kq_res leaves them)
+  embed_row<NIT, QUADS>(table, dtype, off_scale, (size_t)token * dim, dim, xv);
+  if constexpr (!QUADS) {
 #pragma unroll
     for (int it = 0; it < NIT; it++)
-      if (it * 1024 + tid < dim) lds[it * 1024 + tid] = xv[it];
-    __syncthreads();
-    for (int i = tid; i < dim / 16; i += 1024) {
-      float s = -0.0f;
+      if (it * 1024 + tid < dim) x[it * 1024 + tid] = xv[it];
+    return;
+  }
+  f32x4 v[NIT / 4];
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const f32x4 t = ((const f32x4*)lds)[i * 4 + j];
-        s += t[0] * t[0];
-        s += t[1] * t[1];
-        s += t[2] * t[2];
-        s += t[3] * t[3];
-      }
-      ((float*)o.d)[i] = s;
+  for (int j = 0; j < NIT / 4; j++) {
+    const int i = j * 1024 + tid;
+    v[j] = f32x4{xv[4 * j], xv[4 * j + 1], xv[4 * j + 2], xv[4 * j + 3]};
+    if (i * 4 < dim) ((f32x4*)x)[i] = v[j];
+    const float t = quad_square_scan(v[j], lane, half || FRONT == FRONT_SUMS ? 3 : 7);
+    if constexpr (FRONT == FRONT_SUMS) {  // (the halves of norm_quant_regs' chunks, as k_kq_res leaves them)
+      if ((lane & 3) == 3 && i * 4 < dim) ((float*)o.d)[i >> 2] = t;
+    } else {
+      const float low = dpp_f<0x114>(t);  // (row_shr:4: rows 0..15's)
+      if ((lane & 7) == 7 && i * 4 < dim) s_chunks[i >> 3] = half ? low + t : t;
     }
   }
-  if constexpr (FRONT == FRONT_Q8_0 || FRONT == FRONT_Q8_1)
-    norm_quant_regs<NIT, true, FRONT == FRONT_Q8_1>(xv, wv, dim, eps, L, &s_rms, o.q, (unsigned short*)o.d, o.aux, nullptr, half);
-  if constexpr (FRONT == FRONT_Q8_K) {
-    norm_quant_regs<NIT, false>(xv, wv, dim, eps, L, &s_rms, nullptr, nullptr, nullptr, L.xs, half);  // (xs has been read by then)
-    __syncthreads();
-    for (int sb = tid >> 6; sb < dim / 256; sb += 16) {  // k_quantize_q8_k's wave per super-block
-      const Q8KLane k = q8k_wave_quant(((const f32x4*)L.xs)[sb * 64 + lane], lane);
-      ((unsigned*)o.q)[sb * 64 + lane] = k.packed;
+  if constexpr (FRONT == FRONT_SUMS) return;
+  __syncthreads();
+  const float rms = sqrtf(chunk_sums(s_chunks, dim / 32, lane, half) / (float)dim + eps);
+#pragma unroll
+  for (int j = 0; j < NIT / 4; j++) {
+    const int i = j * 1024 + tid;
+    if (j * 4096 + (tid & ~63) * 4 >= dim) break;  // (wave-uniform)
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[j][e] = (v[j][e] / rms) * wv[j][e];
+    if constexpr (FRONT == FRONT_Q8_K) {
+      const int sb = i >> 6;
+      const Q8KLane k = q8k_wave_quant(v[j], lane);
+      ((unsigned*)o.q)[i] = k.packed;
       q8k_store_class_major(o.qp + sb * 256, lane, k.packed);
-      if ((lane & 3) == 0) ((short*)o.aux)[sb * 16 + (lane >> 2)] = (short)k.quad_sum;
+      if ((lane & 3) == 0) ((short*)o.aux)[i >> 2] = (short)k.quad_sum;
       if (lane == 0) ((float*)o.d)[sb] = k.d;
+    } else {
+      const QLane4 k = quant_quad8<FRONT == FRONT_Q8_1>(v[j]);
+      if (i * 4 >= dim) continue;  // (whole chunks)
+      ((unsigned*)o.q)[i] = k.packed;
+      if ((lane & 7) == 0) {
+        ((unsigned short*)o.d)[i >> 3] = k.d;
+        store_qaux<FRONT == FRONT_Q8_1>(o.aux, i >> 3, k.aux);
+      }
     }
   }
 }

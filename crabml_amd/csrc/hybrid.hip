@@ -610,6 +610,8 @@ int latent_step(Ctx* c, const Run& run, int B, bool prof) {
 }
 
 
+// the next step's front reads the logits itself (rows of them start on 16 bytes)
+bool front_picks(const Ctx* c) { return c->vocab <= ARGMAX_ONE && c->vocab % 4 == 0; }
 // the front of a step (k_front_rows); pick: behind the sampler's partials; embed: not where the next step brings its own front
 void enqueue_front(Ctx* c, int B, bool pick, bool embed) {
   const size_t stride = (size_t)HYB_STEP_ROWS * c->ldx;
@@ -618,6 +620,8 @@ void enqueue_front(Ctx* c, int B, bool pick, bool embed) {
     p.pv = c->am_val;
     p.pi = c->am_idx;
     p.nparts = ARGMAX_BLOCKS;
+    if (embed && front_picks(c)) p.logits = c->st_logits;
+    p.n = p.ld = c->vocab;
     p.out_cap = (int)c->st_out_cap;
     p.count = c->st_count;
     p.out = c->st_out;
@@ -748,7 +752,7 @@ int enqueue_step(Ctx* c, int B, bool sample, bool prof, bool led = false, bool l
   }
   head_rows(c, x_in, B, prof, false);
   if (sample) {
-    k_argmax_partial<<<dim3(ARGMAX_BLOCKS, B), 256, 0, st>>>(c->st_logits, c->vocab, c->am_val, c->am_idx, 0, c->vocab);
+    if (!lead || !front_picks(c)) k_argmax_partial<<<dim3(ARGMAX_BLOCKS, B), 256, 0, st>>>(c->st_logits, c->vocab, c->am_val, c->am_idx, 0, c->vocab);
     enqueue_front(c, B, true, lead);
   }
   CH_HIP(dev, hipGetLastError());

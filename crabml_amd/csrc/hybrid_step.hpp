@@ -30,6 +30,8 @@ struct StepSeq {
 // each, 13.6 of the 18.4 us that a 16-row step spent outside its layers and classifier (with several steps in a graph, 16 x 154 tokens of 4 layers of
 // width 2048: 20629 -> 19997 us; one sequence of 81 tokens on latent and windowed layers 12734 -> 12414).
 struct RowPick {
+  const float* logits = nullptr;  // [rows][ld]: n of them in place of the partials
+  int n = 0, ld = 0;
   const float* pv = nullptr;  // [rows][nparts]
   const int* pi = nullptr;
   int nparts = 0, out_cap = 0;
@@ -45,8 +47,14 @@ __global__ __launch_bounds__(1024) void k_front_rows(const RowPick pick, const u
   if (pick.pv) {
     float bv = -INFINITY;
     int bi = -1;
-    for (int i = tid & 63; i < pick.nparts; i += 64) argmax_combine(bv, bi, pick.pv[b * pick.nparts + i], pick.pi[b * pick.nparts + i]);
-    argmax_wave(bv, bi);
+    if (pick.logits) {  // (a whole workgroup)
+      __shared__ float sv[16];
+      __shared__ int si[16];
+      bi = argmax_row(pick.logits + (size_t)b * pick.ld, pick.n, sv, si);
+    } else {
+      for (int i = tid & 63; i < pick.nparts; i += 64) argmax_combine(bv, bi, pick.pv[b * pick.nparts + i], pick.pi[b * pick.nparts + i]);
+      argmax_wave(bv, bi);
+    }
     token = bi < 0 ? 0 : bi;
     pos++;
     __syncthreads();  // (every wave has the old position)

@@ -50,27 +50,12 @@ __global__ __launch_bounds__(256) void k_norm_quant_rows(float* __restrict__ x, 
       xv[j] = av[j] + xv[j];  // x = matmul_out + x (llama2.rs:266 / :636)
       if (i < n4) xr[i] = xv[j];
     }
-    const f32x4 q = xv[j] * xv[j];
-    float t = (((-0.0f + q[0]) + q[1]) + q[2]) + q[3];
-    for (int k = 1; k <= last; k++) {
-      const float u = (((dpp_f<0x111>(t) + q[0]) + q[1]) + q[2]) + q[3];  // (row_shr:1: the lane before goes first)
-      t = (lane & last) == k ? u : t;
-    }
+    const float t = quad_square_scan(xv[j], lane, last);
     const float low = dpp_f<0x114>(t);  // (row_shr:4: rows 0..15's)
     if ((lane & 7) == 7 && i < n4) cs_lds[i >> 3] = half ? low + t : t;
   }
   __syncthreads();
-  float sum = 0.0f;
-  for (int base = 0; base < cols / 32; base += 64) {
-    const float v = base + lane < cols / 32 ? cs_lds[base + lane] : 0.0f;
-    if (half) {
-      sum += wave_sum_f32(v);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 64; i++) sum += rl_f(v, i);
-    }
-  }
-  const float rms = sqrtf(sum / (float)cols + eps);
+  const float rms = sqrtf(chunk_sums(cs_lds, cols / 32, lane, half) / (float)cols + eps);
   char* p = planes + r * row_stride;
   unsigned short* xo = xh + r * (size_t)cols;
 #pragma unroll

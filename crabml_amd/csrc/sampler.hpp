@@ -16,12 +16,51 @@ __device__ __forceinline__ void argmax_combine(float& cv, int& ci, float ov, int
   }
 }
 __device__ __forceinline__ void argmax_wave(float& v, int& i) {  // over the 64 lanes; every lane gets it
+  argmax_combine(v, i, dpp_f<0xB1>(v), dpp_i<0xB1>(i));
+  argmax_combine(v, i, dpp_f<0x4E>(v), dpp_i<0x4E>(i));
+  argmax_combine(v, i, dpp_f<0x141>(v), dpp_i<0x141>(i));
+  argmax_combine(v, i, dpp_f<0x140>(v), dpp_i<0x140>(i));
+  float bv = rl_f(v, 0);
+  int bi = __builtin_amdgcn_readlane(i, 0);
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(v, o, 64);
-    const int oi = __shfl_xor(i, o, 64);
-    argmax_combine(v, i, ov, oi);
+  for (int r = 16; r < 64; r += 16) argmax_combine(bv, bi, rl_f(v, r), __builtin_amdgcn_readlane(i, r));
+  v = bv;
+  i = bi;
+}
+// The whole row of logits by one workgroup of 1024 (the front of the next step): where one round of requests covers it that is shorter than a launch of
+// partials in front of it.  sv, si: LDS, 16 each; every thread gets the index (-1: an empty row).
+#define ARGMAX_ONE 32768
+__device__ __forceinline__ int argmax_row(const float* __restrict__ logits, int n, float* sv, int* si) {
+  constexpr int U = ARGMAX_ONE / 4096;
+  const int tid = threadIdx.x, n4 = n / 4;
+  float bv = -INFINITY;
+  int bi = -1;
+  f32x4 q[U];
+  if (n4 > 0) {  // (uniform)
+#pragma unroll
+    for (int u = 0; u < U; u++) q[u] = ((const f32x4*)logits)[u * 1024 + tid < n4 ? u * 1024 + tid : n4 - 1];
+#pragma unroll
+    for (int u = 0; u < U; u++) {  // (ascending indices: whatever is not smaller takes the place.  The last four once more past the end change nothing)
+      const int i = (u * 1024 + tid < n4 ? u * 1024 + tid : n4 - 1) * 4;
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const bool take = !(bv > q[u][e]);
+        bv = take ? q[u][e] : bv;
+        bi = take ? i + e : bi;
+      }
+    }
   }
+  if (tid < n % 4) argmax_combine(bv, bi, logits[n4 * 4 + tid], n4 * 4 + tid);
+  argmax_wave(bv, bi);
+  if ((tid & 63) == 0) {
+    sv[tid >> 6] = bv;
+    si[tid >> 6] = bi;
+  }
+  __syncthreads();
+  bv = sv[tid & 15];
+  bi = si[tid & 15];
+  argmax_wave(bv, bi);
+  return bi;
 }
 // base: global index of logits[0] (a vocabulary shard of a tensor-parallel classifier; 0 otherwise).  blockIdx.y: row of a batch
 // (row_stride floats apart; its partials follow the previous row's)
