@@ -73,10 +73,24 @@ inline size_t sample_argmax(const std::vector<float>& p) {
   const size_t n = p.size();
 #if defined(__x86_64__)
   if (n >= 64 && __builtin_cpu_supports("avx2")) {
-    bool clean = false;
-    const float mx = max_avx2(p.data(), n, &clean);
+    // chunk by chunk, and back through the last one that holds the maximum alone (through all of 128256 logits, an element at a time, the way back took several
+    // times as long as the maximum)
+    const size_t CHUNK = 4096;
+    size_t at = 0, end = 0;
+    float mx = 0.0f;
+    bool clean = true;
+    for (size_t lo = 0; lo < n && clean;) {
+      const size_t hi = n - lo < 2 * CHUNK ? n : lo + CHUNK;
+      const float m = max_avx2(p.data() + lo, hi - lo, &clean);
+      if (lo == 0 || m >= mx) {
+        mx = m;
+        at = lo;
+        end = hi;
+      }
+      lo = hi;
+    }
     if (clean)
-      for (size_t k = n; k-- > 0;)
+      for (size_t k = end; k-- > at;)
         if (p[k] == mx) return k;
   } else
 #endif

@@ -27,21 +27,21 @@ __device__ __forceinline__ void argmax_wave(float& v, int& i) {  // over the 64 
   v = bv;
   i = bi;
 }
-// The whole row of logits by one workgroup of 1024 (the front of the next step): where one round of requests covers it that is shorter than a launch of
-// partials in front of it.  sv, si: LDS, 16 each; every thread gets the index (-1: an empty row).
-#define ARGMAX_ONE 32768
+// The whole row of logits by one workgroup of 1024 (the front of the next step), in rounds of 32768: up to four of them are shorter than a launch of partials
+// in front of it.  Us, partials and front / front: 32000 logits 4.6 + 4.7 / 5.5 (width 288), 128256 4.8 + 5.7 / 9.8 (width 4096).  sv, si: LDS, 16 each; every thread gets the index (-1: an empty row).
+#define ARGMAX_ONE 131072
 __device__ __forceinline__ int argmax_row(const float* __restrict__ logits, int n, float* sv, int* si) {
-  constexpr int U = ARGMAX_ONE / 4096;
+  constexpr int U = 8;
   const int tid = threadIdx.x, n4 = n / 4;
   float bv = -INFINITY;
   int bi = -1;
-  f32x4 q[U];
-  if (n4 > 0) {  // (uniform)
+  for (int i0 = 0; i0 < n4; i0 += U * 1024) {
+    f32x4 q[U];
 #pragma unroll
-    for (int u = 0; u < U; u++) q[u] = ((const f32x4*)logits)[u * 1024 + tid < n4 ? u * 1024 + tid : n4 - 1];
+    for (int u = 0; u < U; u++) q[u] = ((const f32x4*)logits)[i0 + u * 1024 + tid < n4 ? i0 + u * 1024 + tid : n4 - 1];
 #pragma unroll
     for (int u = 0; u < U; u++) {  // (ascending indices: whatever is not smaller takes the place.  The last four once more past the end change nothing)
-      const int i = (u * 1024 + tid < n4 ? u * 1024 + tid : n4 - 1) * 4;
+      const int i = (i0 + u * 1024 + tid < n4 ? i0 + u * 1024 + tid : n4 - 1) * 4;
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const bool take = !(bv > q[u][e]);

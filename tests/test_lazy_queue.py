@@ -370,6 +370,24 @@ def test_the_runners_greedy_sampler_keeps_the_last_maximum():
             assert ca.sample_argmax(p) == ref(p), (n, case)
 
 
+@pytest.mark.parametrize("n", [4096, 8191, 8192, 8193, 12289])
+def test_the_greedy_sampler_over_several_chunks(n):
+    """the maximum comes chunk by chunk (4096, the last one up to twice that): equal maxima in and across chunks, a NaN in any of them, no finite logit"""
+    rng = np.random.default_rng(n)
+    for at in (0, 4095, 4096, n // 2, n - 1):
+        p = rng.standard_normal(n).astype(np.float32)
+        p[[at, at // 2]] = 9.0
+        assert ca.sample_argmax(p) == at
+        q = p.copy()
+        q[at] = np.nan
+        best = 0
+        for i in range(1, n):
+            if not (q[best] > q[i]):
+                best = i
+        assert ca.sample_argmax(q) == best
+    assert ca.sample_argmax(np.full(n, -np.inf, np.float32)) == n - 1
+
+
 def test_rust_lifetimes_do_not_change_what_the_matcher_sees():
     """The op stream with every handle released where rustc would release it (forward_rs): every token is still served by the fused
     step -- the queue's own references keep operands alive, caches moved out of and back into their Option are the same handles."""
