@@ -374,7 +374,7 @@ def test_the_runners_greedy_sampler_keeps_the_last_maximum():
 def test_the_greedy_sampler_over_several_chunks(n):
     """the maximum comes chunk by chunk (4096, the last one up to twice that): equal maxima in and across chunks, a NaN in any of them, no finite logit"""
     rng = np.random.default_rng(n)
-    for at in (0, 4095, 4096, n // 2, n - 1):
+    for at in sorted({0, 4095, min(4096, n - 1), n // 2, n - 1}):
         p = rng.standard_normal(n).astype(np.float32)
         p[[at, at // 2]] = 9.0
         assert ca.sample_argmax(p) == at
