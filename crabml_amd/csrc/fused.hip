@@ -2447,11 +2447,12 @@ static int llama_create_impl(crabml_hip_device_t* dev, const crabml_hip_llama_co
         if (rc == 0 && !dry && hipMemsetAsync(c->flash_tick, 0, n_kv_l * 4, dev->stream) != hipSuccess) rc = CRABML_HIP_UNEXPECTED;
         c->attn_flash = rc == 0;
         if (c->attn_flash) c->attn_long_ok = true;
-        // Below ~768 cached positions the merge inside the launch (last-arriving workgroup of a kv head, ticket word) beats the
-        // second launch -- 7.4 vs 5.1 + 4.1 us per layer at 128 positions, 8.7 vs 10.0 at 512, 10.8 vs 9.95 at 1024
-        // (profiles/r05_flash_ticket_sweep.md; same partials, same merge order: bit-identical): a third graph variant serves that range.
+        // Below 1200 cached positions the merge inside the launch (last-arriving workgroup of a kv head, ticket word) beats the second launch (same
+        // partials, same merge: bit-identical): a third graph variant serves that range.  A step of four layers of the 8B shape in Q4_0, us, two launches /
+        // one: 470 positions 227.0 / 221.5, 700 227.3 / 222.5, 900 226.4 / 225.3, 1200 227.7 / 228.7, 2000 230.0 / 235.3; of width 2048 in F16 700 178.3 /
+        // 173.5, 900 178.4 / 174.7, 1200 178.8 / 177.5, 2000 179.8 / 181.1.
         if (c->attn_flash && !c->flash_ticket) {
-          size_t until = 768;
+          size_t until = 1200;
           if (const char* hooks = getenv("CRABML_HIP_TEST_HOOKS"))  // tuning hook: 0 = never
             if (hooks[0] == '1')
               if (const char* e = getenv("CRABML_HIP_FLASH_TICKET_UNTIL")) until = (size_t)atol(e);

@@ -1015,11 +1015,23 @@ __device__ __forceinline__ float flash_row_sum(float v) {
 #define FLASH_MAX_SLICES 32
 template <int G>
 struct FlashGeom {
-  static constexpr int NW = G == 8 ? 4 : 8;  // waves per workgroup (LDS: NW * RPI classes x G x HD floats)
+  static constexpr int NW = G == 8 ? 4 : 8;  // waves per workgroup
 };
 __host__ __device__ inline size_t flash_lds_bytes(int G, int hd) {
-  const int nw = G == 8 ? 4 : 8, rpi = 64 / (hd / 8), ncls = nw * rpi;
-  return (size_t)ncls * G * hd * 4 + (size_t)ncls * G * 4 * 3 + 64;
+  const int nw = G == 8 ? 4 : 8;
+  return (size_t)nw * G * (hd + 2) * 4 + 64;
+}
+// a head's slices meet: lane s has slice s's maximum and denominator, o[s] is this lane's column of slice s.  Every wave for itself; returns the sum, L its denominator
+template <int N>
+__device__ __forceinline__ float flash_meet(const float (&o)[N], float m, float l, int S, int lane, float& L) {
+  m = lane < S ? m : -INFINITY;
+  const float M = wave_max_f32(m), w = m == -INFINITY ? 0.0f : __expf(m - M);
+  L = wave_sum_f32(lane < S ? l * w : 0.0f);
+  float r = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; i++)
+    if (i < S) r = __builtin_fmaf(o[i], rl_f(w, i), r);
+  return r;
 }
 __host__ __device__ inline size_t flash_part_floats(int G, int hd) { return (size_t)G * (hd + 2); }
 template <int G, int HD, bool Q81, bool TICKET>
@@ -1029,15 +1041,14 @@ __global__ __launch_bounds__(FlashGeom<G>::NW * 64) void k_attn_flash(const floa
                                                                      float* __restrict__ out, signed char* __restrict__ xq,
                                                                      unsigned short* __restrict__ xd, void* __restrict__ xisum, int seq_cap,
                                                                      int Smax, int min_rows) {
-  constexpr int NW = FlashGeom<G>::NW, LPR = HD / 8, RPI = 64 / LPR, NCLS = NW * RPI, U = 4, NT = NW * 64;
+  constexpr int NW = FlashGeom<G>::NW, LPR = HD / 8, RPI = 64 / LPR, U = 4, NT = NW * 64;
   static_assert(HD == 64 || HD == 128, "a K / V row is 8 or 16 lanes x 16 bytes");
   typedef _Float16 h2 __attribute__((ext_vector_type(2)));
   extern __shared__ __attribute__((aligned(16))) float fl_lds[];
-  float* sacc = fl_lds;                 // [NCLS][G][HD]
-  float* sm = sacc + NCLS * G * HD;     // [NCLS][G]
-  float* sl = sm + NCLS * G;            // [NCLS][G]
-  float* sw = sl + NCLS * G;            // [NCLS][G] merge weights
-  int* s_last = (int*)(sw + NCLS * G);
+  float* sacc = fl_lds;            // [NW][G][HD]
+  float* sm = sacc + NW * G * HD;  // [NW][G]
+  float* sl = sm + NW * G;         // [NW][G]
+  int* s_last = (int*)(sl + NW * G);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int rc = lane / LPR, dl = lane % LPR;
   const int j = blockIdx.x / Smax, sp = blockIdx.x % Smax;
@@ -1116,48 +1127,44 @@ __global__ __launch_bounds__(FlashGeom<G>::NW * 64) void k_attn_flash(const floa
       }
     }
   }
-  // ---- the NCLS (wave, row class) states meet in LDS ---------------------------------------------------------------
-  const int cls = wave * RPI + rc;
+  // ---- a wave's row classes meet in its lanes, the waves in LDS (each class by itself there: 64 KB and a barrier more) ----
 #pragma unroll
   for (int g = 0; g < G; g++) {
-    f32x4* dst = (f32x4*)(sacc + ((size_t)cls * G + g) * HD + 8 * dl);
-    dst[0] = f32x4{acc[g][0], acc[g][1], acc[g][2], acc[g][3]};
-    dst[1] = f32x4{acc[g][4], acc[g][5], acc[g][6], acc[g][7]};
-    if (dl == 0) {
-      sm[cls * G + g] = m[g];
-      sl[cls * G + g] = l[g];
+    const float M = wave_max_f32(m[g]), f = m[g] == -INFINITY ? 0.0f : __expf(m[g] - M);
+    l[g] = sum_groups<LPR>(l[g] * f);
+#pragma unroll
+    for (int i = 0; i < 8; i++) acc[g][i] *= f;
+    sum_groups<LPR>(acc[g]);
+    if (LPR == 16 || (lane & 8) == 0)
+      *(f32x2*)(sacc + (wave * G + g) * HD + 8 * dl + (lane >> 5) * 4 + ((lane >> 4) & 1) * 2) = f32x2{acc[g][0], acc[g][1]};
+    if (lane == 0) {
+      sm[wave * G + g] = M;
+      sl[wave * G + g] = l[g];
     }
   }
   __syncthreads();
-  if (tid < NCLS * G) {  // merge weights e^(m_c - M) per (class, head); tid = c * G + g
-    const int g = tid % G;
-    float M = -INFINITY;
-    for (int c = 0; c < NCLS; c++) M = fmaxf(M, sm[c * G + g]);
-    const float mc = sm[tid];
-    sw[tid] = mc == -INFINITY ? 0.0f : __expf(mc - M);
-  }
-  __syncthreads();
   float* mypart = part + (size_t)blockIdx.x * (G * (HD + 2));
+  auto leave = [&](int at, float v) {
+    if constexpr (TICKET)
+      __hip_atomic_store(mypart + at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else
+      mypart[at] = v;
+  };
   for (int idx = tid; idx < G * HD; idx += NT) {
     const int g = idx / HD, d = idx % HD;
-    float o = 0.f;
-#pragma unroll 8
-    for (int c = 0; c < NCLS; c++) o = __builtin_fmaf(sacc[((size_t)c * G + g) * HD + d], sw[c * G + g], o);
-    if constexpr (TICKET)
-      __hip_atomic_store(mypart + g * (HD + 2) + d, o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else
-      mypart[g * (HD + 2) + d] = o;
-  }
-  if (tid < G) {
-    float M = -INFINITY, L = 0.f;
-    for (int c = 0; c < NCLS; c++) M = fmaxf(M, sm[c * G + tid]);
-    for (int c = 0; c < NCLS; c++) L = __builtin_fmaf(sl[c * G + tid], sw[c * G + tid], L);
-    if constexpr (TICKET) {
-      __hip_atomic_store(mypart + tid * (HD + 2) + HD, M, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(mypart + tid * (HD + 2) + HD + 1, L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    } else {
-      mypart[tid * (HD + 2) + HD] = M;
-      mypart[tid * (HD + 2) + HD + 1] = L;
+    float M = sm[g], o = 0.f, L = 0.f;
+#pragma unroll
+    for (int c = 1; c < NW; c++) M = fmaxf(M, sm[c * G + g]);
+#pragma unroll
+    for (int c = 0; c < NW; c++) {
+      const float mc = sm[c * G + g], e = mc == -INFINITY ? 0.0f : __expf(mc - M);
+      o = __builtin_fmaf(sacc[(c * G + g) * HD + d], e, o);
+      L = __builtin_fmaf(sl[c * G + g], e, L);
+    }
+    leave(g * (HD + 2) + d, o);
+    if (d == 0) {
+      leave(g * (HD + 2) + HD, M);
+      leave(g * (HD + 2) + HD + 1, L);
     }
   }
   if constexpr (!TICKET) return;  // the merge is its own launch (k_attn_flash_merge)
@@ -1173,55 +1180,28 @@ __global__ __launch_bounds__(FlashGeom<G>::NW * 64) void k_attn_flash(const floa
   }
   __syncthreads();
   if (*s_last == 0) return;
-  // ---- merge (one workgroup per kv head): every load of the hand-off is requested before anything waits on one --------------
+  // ---- merge (one workgroup per kv head, a wave on 64 columns of one head): one round trip, no barrier.  With this and the classes' meeting above, us a
+  // launch of 8 kv heads x 4 x 128: 512 positions 9.4 -> 8.7; without the ticket at 3000 7.6 -> 7.3 --------------------------------
   const float* pj = part + (size_t)j * Smax * (G * (HD + 2));
-  float* mg_m = sacc;                                  // [S][G]  (sacc is done with)
-  float* mg_l = sacc + FLASH_MAX_SLICES * G;           // [S][G]
-  float* mg_w = sacc + 2 * FLASH_MAX_SLICES * G;       // [S][G] e^(m_s - M)
-  float* mg_M = sacc + 3 * FLASH_MAX_SLICES * G;       // [G] {1 / L}
-  constexpr int SB = 16;                               // partial values per thread and batch
-  auto load_o = [&](int idx, int s0, float (&ov)[SB]) {
+  for (int idx = tid; idx < G * HD; idx += NT) {  // (one pass unless G * HD > NT)
     const int g = idx / HD, d = idx % HD;
+    const float* pg = pj + g * (HD + 2);
+    auto take = [&](int s2, int at) {
+      return __hip_atomic_load(pg + (size_t)(s2 < S ? s2 : S - 1) * (G * (HD + 2)) + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    float L, o;
+    auto meet = [&](auto n) {
+      constexpr int N = decltype(n)::value;
+      const float ms = take(lane, HD), ls = take(lane, HD + 1);
+      float ov[N];
 #pragma unroll
-    for (int i = 0; i < SB; i++) {
-      const int s2 = s0 + i < S ? s0 + i : S - 1;
-      ov[i] = __hip_atomic_load(pj + (size_t)s2 * (G * (HD + 2)) + g * (HD + 2) + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-  };
-  float ov[SB];
-  if (tid < G * HD) load_o(tid, 0, ov);
-  for (int t = tid; t < S * G; t += NT) {  // the slices' {m, l} -> LDS
-    const float* ps = pj + (size_t)(t / G) * (G * (HD + 2)) + (t % G) * (HD + 2) + HD;
-    mg_m[t] = __hip_atomic_load(ps, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    mg_l[t] = __hip_atomic_load(ps + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  __syncthreads();
-  if (tid < G) {  // per head: M, the slices' weights e^(m_s - M), L
-    float M = -INFINITY, L = 0.f;
-    for (int s2 = 0; s2 < S; s2++) M = fmaxf(M, mg_m[s2 * G + tid]);
-    for (int s2 = 0; s2 < S; s2++) {
-      const float ms = mg_m[s2 * G + tid];
-      const float w = ms == -INFINITY ? 0.0f : __expf(ms - M);
-      mg_w[s2 * G + tid] = w;
-      L = __builtin_fmaf(mg_l[s2 * G + tid], w, L);
-    }
-    mg_M[tid] = L;
-  }
-  __syncthreads();
-  for (int idx = tid; idx < G * HD; idx += NT) {  // (whole waves stay together: 64 | G * HD; one pass unless G * HD > NT)
-    const int g = idx / HD, d = idx % HD;
-    if (idx != tid) load_o(idx, 0, ov);
-    float o = 0.f;
-#pragma unroll
-    for (int i = 0; i < SB; i++)
-      if (i < S) o = __builtin_fmaf(ov[i], mg_w[i * G + g], o);
-    for (int s0 = SB; s0 < S; s0 += SB) {  // contexts past SB slices: one more batch
-      load_o(idx, s0, ov);
-#pragma unroll
-      for (int i = 0; i < SB; i++)
-        if (s0 + i < S) o = __builtin_fmaf(ov[i], mg_w[(s0 + i) * G + g], o);
-    }
-    const float L = mg_M[g];
+      for (int i = 0; i < N; i++) ov[i] = take(i, d);
+      o = flash_meet<N>(ov, ms, ls, S, lane, L);
+    };
+    if (S <= FLASH_MAX_SLICES / 2)
+      meet(std::integral_constant<int, FLASH_MAX_SLICES / 2>{});
+    else
+      meet(std::integral_constant<int, FLASH_MAX_SLICES>{});
     const float val = o / L;
     const int e = (j * G + g) * HD + d;
     out[e] = val;
@@ -1243,8 +1223,6 @@ __global__ __launch_bounds__(HD) void k_attn_flash_merge(const float* __restrict
                                                         float* __restrict__ out, signed char* __restrict__ xq,
                                                         unsigned short* __restrict__ xd, void* __restrict__ xisum, int G, int Smax,
                                                         int min_rows) {
-  __shared__ float s_w[FLASH_MAX_SLICES];
-  __shared__ float s_L;
   const int head = blockIdx.x, j = head / G, g = head % G, d = threadIdx.x;
   const float* pj = part + ((size_t)j * Smax * G + g) * (HD + 2);  // slice s of this head: pj + s * G * (HD + 2)
   const size_t sstr = (size_t)G * (HD + 2);
@@ -1253,25 +1231,13 @@ __global__ __launch_bounds__(HD) void k_attn_flash_merge(const float* __restrict
   float ov[FLASH_MAX_SLICES];
 #pragma unroll
   for (int i = 0; i < FLASH_MAX_SLICES; i++) ov[i] = pj[(size_t)(i < Smax ? i : Smax - 1) * sstr + d];
-  const int sl = d < Smax ? d : Smax - 1;  // lanes 0 .. Smax - 1 of wave 0 own one slice's {m, l}
-  float ms = pj[(size_t)sl * sstr + HD], ls = pj[(size_t)sl * sstr + HD + 1];
+  const int lane = d & 63, sl = lane < Smax ? lane : Smax - 1;  // lanes 0 .. Smax - 1 own one slice's {m, l}
+  const float ms = pj[(size_t)sl * sstr + HD], ls = pj[(size_t)sl * sstr + HD + 1];
   const int seq = *pos_d + 1;
   const int S = min(Smax, max(1, (seq + min_rows - 1) / min_rows));  // k_attn_flash's own rule
-  if (d < 64) {  // wave 0: M, the slices' weights e^(m_s - M), L -- the k_attn_flash merge's operations in its order
-    if (d >= S) ms = -INFINITY;
-    const float M = wave_max_f32(ms);
-    const float w = ms == -INFINITY ? 0.0f : __expf(ms - M);
-    if (d < FLASH_MAX_SLICES) s_w[d] = w;
-    float L = 0.f;
-    for (int s2 = 0; s2 < S; s2++) L = __builtin_fmaf(rl_f(ls, s2), rl_f(w, s2), L);
-    if (d == 0) s_L = L;
-  }
-  __syncthreads();
-  float o = 0.f;
-#pragma unroll
-  for (int i = 0; i < FLASH_MAX_SLICES; i++)
-    if (i < S) o = __builtin_fmaf(ov[i], s_w[i], o);
-  const float val = o / s_L;
+  float L;
+  const float o = flash_meet<FLASH_MAX_SLICES>(ov, ms, ls, S, lane, L);
+  const float val = o / L;
   const int e = head * HD + d;
   out[e] = val;
   if (xq != nullptr) {
