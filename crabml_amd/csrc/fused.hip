@@ -1696,7 +1696,7 @@ int prefill_chunk(crabml_hip_llama* c, const uint32_t* tokens, size_t B, size_t 
     }
     if (gemm_f16({w}, {(size_t)m}, (size_t)k, act, {out})) return 0;
     if (!strict) {
-      if (!gemm_exact_hook && B >= 16 && (w->dtype == CRABML_HIP_Q4_0 || w->dtype == CRABML_HIP_Q8_0 || w->dtype == CRABML_HIP_Q4_1 || w->dtype == CRABML_HIP_Q4_K) &&
+      if (!gemm_exact_hook && (B >= 16 || gemm_mfma_few(w->dtype, B, (size_t)m, (size_t)k)) && (w->dtype == CRABML_HIP_Q4_0 || w->dtype == CRABML_HIP_Q8_0 || w->dtype == CRABML_HIP_Q4_1 || w->dtype == CRABML_HIP_Q4_K) &&
           launch_gemm_mfma(dev, w, m, k, act, B, out, nullptr, nullptr, true, c->pf_split, c->pf_split_floats, defer))
         return 0;
       return launch_gemv(dev, w, m, k, act, B, out);

@@ -865,7 +865,7 @@ bool launch_gemm_mfma(crabml_hip_device* dev, const crabml_hip_buf* w, size_t m,
   if (w->dtype != CRABML_HIP_Q4_0 && w->dtype != CRABML_HIP_Q8_0 && w->dtype != CRABML_HIP_Q4_K && w->dtype != CRABML_HIP_Q6_K &&
       w->dtype != CRABML_HIP_Q4_1 && w->dtype != CRABML_HIP_Q8_K)
     return false;
-  if (b < 16 || m == 0 || k % 32 != 0) return false;
+  if ((b < 16 && !(fused_add && !dev->strict_order && gemm_mfma_few(w->dtype, b, m, k))) || m == 0 || k % 32 != 0) return false;
   hipStream_t st = dev->stream;
   const char* wp = (const char*)w->ptr;
   // pieces of k while the tiles leave CUs without work, each at least `least` chunks long.  24 rows, us a launch without / with the pieces:

@@ -85,6 +85,14 @@ bool launch_gemm_f16w(crabml_hip_device* dev, const crabml_hip_buf* const* w, co
 struct GemmScratch;
 bool launch_gemm_f16(crabml_hip_device* dev, crabml_hip_device::ProfRec* rec, const void* const* w, const size_t* n, int nw, size_t k,
                      const void* act, size_t act_stride, size_t rows, float* const* out, const GemmScratch& ws);
+// Up to 15 rows of a fast prompt pass on the matrix cores: a row kernel's time grows with each row and weight, a tile's with the weights alone, behind its
+// pieces of k.  Estimated us: 0.085 a row and million weights against 8 + 0.26 a million (Q4_1, whose terms have two products more, 0.6).  A prompt on four
+// layers of the 8B shape, row kernels / by this rule: Q4_0 5 rows 668 / 669, 7 rows 767 / 678, 12 rows 981 / 692; Q8_0 5 rows 886 / 759, 15 rows 1619 / 798; Q4_K 12
+// rows 1154 / 701; of 2048 x 8192 Q4_0 8 rows 429 / 426, 12 rows 483 / 442, Q8_0 12 rows 565 / 460.
+inline bool gemm_mfma_few(uint32_t dtype, size_t b, size_t m, size_t k) {
+  const double w = 1e-6 * (double)m * (double)k;
+  return (double)b * w * 0.085 > 8.0 + (dtype == CRABML_HIP_Q4_1 ? 0.6 : 0.26) * w;
+}
 // batched rhs on the matrix cores (gemm_mfma.hip); false = not covered.  fused_add (the FAST prompt pass only): a Q4_0 / Q8_0 block term takes its
 // second product and the add as one fma, and k may be cut into pieces -- an explicit argument, never device state: matmul_vec itself is
 // bit-exact and must not pick it up by accident

@@ -435,6 +435,23 @@ def test_short_passes_in_pieces_of_k_equal_the_token_loop(ca, fmt, rows, width, 
     assert np.array_equal(a.prefill(toks).view(np.uint32), first.view(np.uint32))  # (added in piece order, whoever ends first)
 
 
+# the fewest rows that take matrix-core tiles: the feed-forward alone (5 rows, 50 million weights a matrix), with wo and q (9), most of the row tile empty
+@pytest.mark.parametrize("fmt", ["Q4_0", "Q8_0", "Q4_1", "Q4_K"])
+@pytest.mark.parametrize("rows,hidden", [(5, 12288), (9, 4096), (15, 4352)])
+def test_passes_of_few_rows_equal_the_token_loop(ca, fmt, rows, hidden):
+    shape = synth.ModelShape("few", 4096, hidden, 1, 32, 2, 300, 64, 1e-5, None)
+    dev = ca.HipTensorDevice(0)
+    conf, w = synth.to_hip(synth.build_model(shape, synth.TYPE_BY_NAME[fmt], seed=92), dev)
+    a, b = ca.HipLlamaRunner(conf, w, dev, 64, True), ca.HipLlamaRunner(conf, w, dev, 64, True)
+    toks = [(13 * i + 5) % 300 for i in range(rows)]
+    want = [b.forward(t, i) for i, t in enumerate(toks)][-1]
+    first = a.prefill(toks)
+    # (as above: the same exact block terms, other sums)
+    assert np.max(np.abs(first - want)) <= FAST_TOL[fmt][1] * np.max(np.abs(want))
+    a.reset()
+    assert np.array_equal(a.prefill(toks).view(np.uint32), first.view(np.uint32))
+
+
 # the wide weight GEMM (rows > 64, k a multiple of 256) by its own rule: a row more and a row less than its tiles of 96 and 128 columns; k of one, two, three, 11 and 16
 # super-blocks; matrices that end inside a tile of 128 or 256 rows.  (Launches of few workgroups are gemm_f16w.hip's.)
 @pytest.mark.parametrize("fmt", ["Q4_0", "Q8_0", "Q4_1", "Q4_K", "Q6_K"])
