@@ -11,26 +11,9 @@ __device__ __forceinline__ int f16w_slot_of_elem(int j) {
   const int hi = j >> 4, s = (j >> 2) & 3, r = j & 3;
   return 8 * s + 4 * hi + ((r >> 1) | ((r & 1) << 1));
 }
-// orders 1 (Q4_K weights) / 2 (Q6_K weights), Q8_K rows: position (halfs from the row's start) of element E of super-block sb
-__device__ __forceinline__ int f16w_pos_q8k(int order, int sb, int E) {
-  int cc, g, s, hi, k;
-  if (order == 1) {
-    const int l = E & 7;
-    g = E >> 6;
-    hi = (E >> 5) & 1;
-    k = (E >> 3) & 3;
-    s = l & 3;
-    cc = 2 * sb + (l >> 2);
-  } else {
-    const int r2 = E & 63;
-    hi = (E >> 6) & 1;
-    g = 2 * (r2 >> 5) + ((r2 >> 4) & 1);
-    s = (r2 >> 2) & 3;
-    k = r2 & 3;
-    cc = 2 * sb + (E >> 7);
-  }
-  return (4 * cc + g) * 32 + 8 * s + 4 * hi + ((k >> 1) | ((k & 1) << 1));
-}
+// orders 1 (Q4_K weights) / 2 (Q6_K weights), Q8_K rows: element E of super-block sb sits at half (4 cc + g) * 32 + 8 s + 4 hi + {0, 2, 1, 3}[k] of the row, with
+//   order 1: l = E % 8, k = E / 8 % 4, hi = E / 32 % 2, g = E / 64, s = l % 4, cc = 2 sb + l / 4
+//   order 2: k = E % 4, s = E / 4 % 4, g = E / 16 % 4, hi = E / 64 % 2, cc = 2 sb + E / 128
 // order 0: inside a block, slot 8 s + e (s = 0..3 = the dword of the weight block the slot pairs with) holds element
 //   e = 0, 1: 4 s, 4 s + 2     e = 2, 3: 4 s + 1, 4 s + 3     e = 4, 5: 16 + 4 s, 16 + 4 s + 2     e = 6, 7: 16 + 4 s + 1, 16 + 4 s + 3
 // -- the order in which unpack_q4_0_f16 takes the nibbles out of a dword (two masks per packed pair, no byte permute)
@@ -78,7 +61,7 @@ __device__ __forceinline__ void f16w_store4(unsigned short* at, unsigned quants,
   const unsigned short v2 = f16w_value((int)(signed char)((quants >> 16) & 0xffu), d), v3 = f16w_value((int)(signed char)(quants >> 24), d);
   *(unsigned long long*)at = (unsigned long long)(v0 | ((unsigned)v2 << 16)) | ((unsigned long long)(v1 | ((unsigned)v3 << 16)) << 32);
 }
-// B' of super-block sb from a wave's quantizer (q8k_wave_quant: lane has the quants of elements 4 lane .. 4 lane + 3): f16w_pos_q8k's places, eight bytes a
+// B' of super-block sb from a wave's quantizer (q8k_wave_quant: lane has the quants of elements 4 lane .. 4 lane + 3): their places above, eight bytes a
 // lane -- order 2 keeps four consecutive elements together, order 1 the four of a class, which is what the class-major dword holds
 __device__ __forceinline__ void f16w_store_q8k(unsigned short* __restrict__ xrow, int order, int sb, int lane, unsigned packed, float d) {
   if (order == 1) {
