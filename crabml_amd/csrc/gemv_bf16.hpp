@@ -523,10 +523,11 @@ __global__ __launch_bounds__(64 * W) void k_gemv16_bf16(const GemvBf16 a) {
       for (int j = 0; j < XR; j++) xv[d][h * XR + j] = *(const i32x4*)(x + h * second + xo[j]);
     if constexpr (IN == GEMV_IN_RMSV) gv[d] = *(const f32x4*)(gb + i * 256 + (unsigned)c16 * 16);
   };
-  // A row's sum of squares, by pieces of 16 columns (two of 8): piece q + QT u belongs to term q, in the order of u, the terms meet by neighbours, pairs, ...  A lane
+  // A row's sum of squares, by pieces of 16 columns (two of 8): piece q + QT u belongs to term q, in the order of u, the terms meet by neighbours, pairs, ...  As many
+  // terms as four a wave of all that share k, so that two workgroups of eight waves have sixteen waves' sum.  A lane
   // requests 16 bytes -- QC neighbouring terms of one u, QU of which a row's QR threads have at a time -- the first ahead of the weights (loads come back in order).
   constexpr bool QTWO = EIGHT && !TAIL;
-  constexpr int QT = NT / 16, QC = QTWO ? 2 : 4, QL = QT / QC, QR = QTWO ? 64 : QT, QU = QR / QL;
+  constexpr int QT = 4 * W * KS, QC = QTWO ? 2 : 4, QL = QT / QC, QR = QTWO ? 64 : NT / 16, QU = QR / QL;
   const int q_row = tid / QR, q_at = tid % QR, q_j = q_at % QL, q_u = q_at / QL, n4 = (a.n_ss + 3) / 4;
   const f32x4* q_ss = PIECES ? (const f32x4*)(a.ss + (size_t)(q_row < a.nb ? q_row : a.nb - 1) * a.ld_ss) : nullptr;
   f32x4 q_v = {0.f, 0.f, 0.f, 0.f};

@@ -63,6 +63,34 @@ def test_one_round_of_workgroups(ca, hdev, tmp_path, width, ff, vocab):
     assert all(np.array_equal(s, seen[0]) for s in seen)  # (bit for bit: a sequence's logits do not depend on how many share its step)
 
 
+# k shared by two workgroups (nine rows and more) behind every input and in front of every output that takes it, and by the halves of one (up to eight): the output
+# projection with 68 and 64 pieces of the linear branch's square sum, without any, into the residual and into streams; normed linears of 3104 columns (194 pieces of the
+# square sum) in front of xIELU, GELU * up and the classifier
+@pytest.mark.parametrize("design,oracle,config", [
+    (sh, ho, sh.config(200, 50, [sh.layer(8, 1, 16, 128, 24, 17, 16, 128, 90)] * 2)),
+    (sh, ho, sh.config(84, 50, [sh.layer(16, 4, 16, 128, 24, 16, 16, 128, 90)] * 2)),
+    (sh, ho, sh.config(3104, 50, [sh.layer(4, 2, 24, 40, 100, 3, 16, 24, 90)])),
+    (sb, bo, sb.config(3104, 50, [sb.latent(4, 16, 6, 24, 40, 50, 90), sb.attention(4, 2, 24, 40, 50, 90)], streams=3)),
+    (sb, bo, sb.config(84, 90, [sb.latent(18, 16, 8, 200, 40, 70, 90), sb.attention(16, 2, 16, 200, 24, 90)], streams=2))])
+def test_shared_k_gives_the_bits_of_few_rows(ca, hdev, tmp_path, design, oracle, config):
+    bits = design.random_tensors(config, 13, pool=1 << 20)
+    r = ca.load_model(sh.write_model(config, bits, str(tmp_path)), hdev, seq_len=16)
+    toks = np.random.default_rng(config["width"]).integers(0, config["vocab"], (16, 10))
+    floats = {k: sh.from_bf16(v) for k, v in bits.items()}
+    want = np.array([oracle.forward(config, floats, t) for t in toks[:3]])
+    seen = []
+    for batch in (3, 8, 9, 16):
+        seqs = [r.open() for _ in range(batch)]
+        got = np.array([r.step([(s, [int(toks[i, t])], [0]) for i, s in enumerate(seqs)])[:3] for t in range(10)]).transpose(1, 0, 2)  # [sequence, step, vocab]
+        for s in seqs:
+            r.close(s)
+        d = got - want
+        assert np.sqrt((d * d).mean(axis=2)).max() <= 2.5e-2 * np.sqrt((want ** 2).mean()), batch  # (the designs' own bound)
+        seen.append(got)
+    for other in seen[1:]:
+        assert np.array_equal(other.view(np.uint32), seen[0].view(np.uint32))
+
+
 # columns: those of the steps in flight, one octet more; one staged segment of one row, of two, of eight (8192, 4096, 1024 elements), and one octet more
 @pytest.mark.parametrize("m,k", [(70, 2048), (70, 2056), (515, 4096), (33, 4104), (66, 8200), (17, 1032), (16389, 2056)])
 def test_row_kernels_over_long_rows(ca, hdev, m, k):
