@@ -966,9 +966,12 @@ inline void launch_gemv_bf16_t(hipStream_t st, crabml_hip_device::ProfRec* rec, 
 // One row of the rhs: every workgroup stages it for itself, so eight waves with a row each are faster than four with one, two or four (half as many copies of the rhs
 // through the L2s and half as many workgroups to start, as many requests out from the beginning); a wave has no more requests out than its row has steps -- more are the row's
 // start again, 0.1 to 0.2 us each -- and eight where there are more than eight to make.  What else: two rows a wave where there are more than 8192 of less than 2048
-// columns (four of at most 512), four waves up to 1024 rows of longer ones and from 16384 rows of 2048 columns on.  Us a launch, four waves of as many rows as
+// columns (four of at most 512), four waves up to 1024 rows of longer ones and, but for an rhs that is staged with a gain per element (GEMV_IN_RMSV: twice the bytes a
+// workgroup), from 16384 rows of 2048 columns on.  Us a launch, four waves of as many rows as
 // was best for them and four or eight steps out / these: 2048 x 512 3.25 / 2.8, 32000 x 512 9.7 / 7.5, 32000 x 128 8.5 / 5.2, 4096 x 1024 4.4 / 4.0, 3648 x 2048 5.5 / 5.0,
-// 8192 x 2048 7.7 / 7.4, 11264 x 2048 9.7 / 9.3, 32000 x 2048 23.1 / 20.2, 2048 x 8192 7.75 / 7.5, 2048 x 4096 5.2 / 5.1; gate | up of 16384 x 2048 13.7 / 12.7, 8192 x 512 4.6 / 4.1.
+// 8192 x 2048 7.7 / 7.4, 11264 x 2048 9.7 / 9.3, 2048 x 8192 7.75 / 7.5, 2048 x 4096 5.2 / 5.1; gate | up of 16384 x 2048 13.7 / 12.7, 8192 x 512 4.6 / 4.1.
+// A row a wave from 16384 rows on, four waves / eight: with one gain 32000 x 2048 20.7 / 20.7, x 4096 38.8 / 40.5, 128256 x 4096 146 / 153; with a gain per element 16384 x
+// 2048 14.0 / 12.7, 32000 x 2048 23.6 / 21.4, x 4096 43.9 / 40.6, 128256 x 4096 164 / 150 (four rows a wave: 14.6, 24.2, 41.8, 156).
 template <int IN, int OUT>
 inline void launch_gemv1_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a) {
   constexpr bool NARROW = OUT == GEMV_OUT_RESIDUAL || OUT == GEMV_OUT_STREAMS;  // (as many rows as the model is wide)
@@ -997,7 +1000,7 @@ inline void launch_gemv1_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, c
       launch_gemv_bf16_t<4, 1, 1, 8, IN, OUT>(st, rec, a);
     else if (a.K > 4096)
       launch_gemv_bf16_t<8, 1, 1, 8, IN, OUT>(st, rec, a);
-    else if (a.N <= 1024 || a.N >= 16384)
+    else if (a.N <= 1024 || (a.N >= 16384 && IN != GEMV_IN_RMSV))
       launch_gemv_bf16_t<4, 1, 1, 4, IN, OUT>(st, rec, a);
     else
       launch_gemv_bf16_t<8, 1, 1, 4, IN, OUT>(st, rec, a);

@@ -120,3 +120,22 @@ def test_row_forms(ca, hdev, m, k):
     for b in (1, 2):
         got = t.matmul_vec(ca.HipTensor.new(x[:b].reshape(-1), [b, k], hdev)).export().reshape(b, m)
         assert (np.abs(got - x[:b] @ w.T) <= bound[:b]).all(), b
+
+
+# one and two rows of both designs, the norm's gain one number or a vector: classifiers from 16384 rows on of more than 1024 columns
+@pytest.mark.parametrize("width,ff,vocab", [(1032, 90, 16388), (2048, 90, 16384)])
+@pytest.mark.parametrize("design", [nilivik, bifazen])
+def test_one_and_two_rows(ca, hdev, tmp_path, design, width, ff, vocab):
+    config, tensors, oracle = design(width, ff, vocab)
+    bits = tensors(config, 14, pool=1 << 20)
+    r = ca.load_model(sh.write_model(config, bits, str(tmp_path)), hdev, seq_len=16)
+    floats = {k: sh.from_bf16(v) for k, v in bits.items()}
+    toks = np.random.default_rng(width + ff).integers(0, vocab, (2, 3))
+    want = np.array([oracle.forward(config, floats, t) for t in toks])
+    for batch in (1, 2):
+        seqs = [r.open() for _ in range(batch)]
+        got = np.array([r.step([(s, [int(toks[i, t])], [0]) for i, s in enumerate(seqs)]) for t in range(3)]).transpose(1, 0, 2)
+        for s in seqs:
+            r.close(s)
+        d = got - want[:batch]
+        assert np.sqrt((d * d).mean(axis=2)).max() <= 2.5e-2 * np.sqrt((want ** 2).mean()), batch  # (the designs' own bound)
