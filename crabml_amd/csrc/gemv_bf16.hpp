@@ -965,13 +965,16 @@ inline void launch_gemv_bf16_t(hipStream_t st, crabml_hip_device::ProfRec* rec, 
 }
 // One row of the rhs: every workgroup stages it for itself, so eight waves with a row each are faster than four with one, two or four (half as many copies of the rhs
 // through the L2s and half as many workgroups to start, as many requests out from the beginning); a wave has no more requests out than its row has steps -- more are the row's
-// start again, 0.1 to 0.2 us each -- and eight where there are more than eight to make.  What else: two rows a wave where there are more than 8192 of less than 2048
+// start again, 0.1 to 0.2 us each -- and eight where there are more than eight to make, if the rows are at most 2048 or long enough for a round with less than eight to make
+// to be a small part (four / eight steps out: 2048 x 5120 6.6 / 6.4, 8192 x 5120 14.9 / 15.5, 16384 x 5120 26.6 / 27.2, 3072 x 8192 10.6 / 10.3, 8192 x 8192 22.7 / 22.6).  What else: two rows a wave where there are more than 8192 of less than 2048
 // columns (four of at most 512), four waves up to 1024 rows of longer ones and, but for an rhs that is staged with a gain per element (GEMV_IN_RMSV: twice the bytes a
 // workgroup), from 16384 rows of 2048 columns on.  Us a launch, four waves of as many rows as
 // was best for them and four or eight steps out / these: 2048 x 512 3.25 / 2.8, 32000 x 512 9.7 / 7.5, 32000 x 128 8.5 / 5.2, 4096 x 1024 4.4 / 4.0, 3648 x 2048 5.5 / 5.0,
 // 8192 x 2048 7.7 / 7.4, 11264 x 2048 9.7 / 9.3, 2048 x 8192 7.75 / 7.5, 2048 x 4096 5.2 / 5.1; gate | up of 16384 x 2048 13.7 / 12.7, 8192 x 512 4.6 / 4.1.
 // A row a wave from 16384 rows on, four waves / eight: with one gain 32000 x 2048 20.7 / 20.7, x 4096 38.8 / 40.5, 128256 x 4096 146 / 153; with a gain per element 16384 x
 // 2048 14.0 / 12.7, 32000 x 2048 23.6 / 21.4, x 4096 43.9 / 40.6, 128256 x 4096 164 / 150 (four rows a wave: 14.6, 24.2, 41.8, 156).
+// gate | up: eight waves with a pair each, but four up to 2048 rows of more than 1024 columns, a workgroup of four waves a CU (four / eight: 2048 x 1024 3.6 / 3.5, x 2048
+// 4.5 / 4.7, x 3072 5.6 / 6.1; 2560 x 2048 5.2 / 4.9, 16384 x 2048 13.3 / 12.8).
 template <int IN, int OUT>
 inline void launch_gemv1_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a) {
   constexpr bool NARROW = OUT == GEMV_OUT_RESIDUAL || OUT == GEMV_OUT_STREAMS;  // (as many rows as the model is wide)
@@ -980,7 +983,7 @@ inline void launch_gemv1_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, c
       launch_gemv_bf16_t<8, 1, 2, 1, IN, OUT>(st, rec, a);
     else if (a.K <= 1024)
       launch_gemv_bf16_t<8, 1, 2, 2, IN, OUT>(st, rec, a);
-    else if (a.N >= 2048)
+    else if (a.N > 2048)
       launch_gemv_bf16_t<8, 1, 2, 4, IN, OUT>(st, rec, a);
     else
       launch_gemv_bf16_t<4, 1, 2, 4, IN, OUT>(st, rec, a);
@@ -998,24 +1001,30 @@ inline void launch_gemv1_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, c
       launch_gemv_bf16_t<8, 1, 1, 2, IN, OUT>(st, rec, a);
     else if (a.N <= 1024 && a.K >= 4096)
       launch_gemv_bf16_t<4, 1, 1, 8, IN, OUT>(st, rec, a);
-    else if (a.K > 4096)
+    else if (a.K > 4096 && (a.N <= 2048 || a.K >= 8192))
       launch_gemv_bf16_t<8, 1, 1, 8, IN, OUT>(st, rec, a);
-    else if (a.N <= 1024 || (a.N >= 16384 && IN != GEMV_IN_RMSV))
+    else if (a.N <= 1024 || (a.N >= 16384 && a.K <= 4096 && IN != GEMV_IN_RMSV))
       launch_gemv_bf16_t<4, 1, 1, 4, IN, OUT>(st, rec, a);
     else
       launch_gemv_bf16_t<8, 1, 1, 4, IN, OUT>(st, rec, a);
   }
 }
 // Two rows: the same (2048 x 512 3.95 / 3.6, 1280 x 4096 5.5 / 4.8, 2048 x 8192 9.5 / 8.4, 8192 x 4096 14.3 / 13.25), but two rows of weights a wave where there are more than
-// 4096 of up to 1024 columns or more than 2048 of up to 2048 (32000 x 512 13.6 / 11.7, x 2048 22.4 and 23.85 with a row each).
+// 4096 of up to 1024 columns or more than 2048 of up to 2048 (a row each / two, four waves: 4096 x 1024 4.97 / 5.08, 8192 x 1024 6.9 / 6.7, 32000 x 1024 17.9 / 14.8; 2048 x 2048
+// 4.9 / 5.15, 3648 x 2048 6.36 / 6.35, 32000 x 2048 24.3 / 23.0); where they are more and longer and the rhs is staged with a gain per element, two each in eight waves (3136 x
+// 2560 7.6 / 6.9, 3136 x 4096 9.1 / 8.6, 32000 x 4096 46.7 / 41.8; 2048 x 4096 6.6 / 7.85).  gate | up: four waves up to 2048 rows, else eight (2048 x 2048 5.1 / 5.6,
+// 2048 x 1024 4.25 / 4.4, 2560 x 2048 6.05 / 5.8, 16384 x 1024 9.9 / 9.4, x 2048 15.5 / 14.5).
 template <int IN, int OUT>
 inline void launch_gemv2_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a) {
   if constexpr (OUT == GEMV_OUT_GLU) {
-    if (a.K <= 1024)
-      launch_gemv_bf16_t<8, 2, 2, 2, IN, OUT>(st, rec, a);
+    if (a.N > 2048)
+      a.K <= 1024 ? launch_gemv_bf16_t<8, 2, 2, 2, IN, OUT>(st, rec, a) : launch_gemv_bf16_t<8, 2, 2, 4, IN, OUT>(st, rec, a);
     else
-      launch_gemv_bf16_t<8, 2, 2, 4, IN, OUT>(st, rec, a);
+      a.K <= 1024 ? launch_gemv_bf16_t<4, 2, 2, 2, IN, OUT>(st, rec, a) : launch_gemv_bf16_t<4, 2, 2, 4, IN, OUT>(st, rec, a);
   } else {
+    if constexpr (IN == GEMV_IN_RMSV) {
+      if (a.K > 2048 && a.N > 2048) return launch_gemv_bf16_t<8, 2, 2, 4, IN, OUT>(st, rec, a);
+    }
     if (a.K <= 1024 && a.N > 4096)
       launch_gemv_bf16_t<4, 2, 2, 2, IN, OUT>(st, rec, a);
     else if (a.K <= 1024)

@@ -122,8 +122,10 @@ def test_row_forms(ca, hdev, m, k):
         assert (np.abs(got - x[:b] @ w.T) <= bound[:b]).all(), b
 
 
-# one and two rows of both designs, the norm's gain one number or a vector: classifiers from 16384 rows on of more than 1024 columns
-@pytest.mark.parametrize("width,ff,vocab", [(1032, 90, 16388), (2048, 90, 16384)])
+# one and two rows of both designs, the norm's gain one number or a vector: classifiers from 16384 rows on of more than 1024 and of more than 4096 columns, of more than 2048
+# rows; gate | up of 2048 rows and a pair more, of few columns and many; residuals behind more than 4096 columns, of 2048 rows and more, and behind 8192
+@pytest.mark.parametrize("width,ff,vocab", [(1032, 90, 16388), (2048, 90, 16384), (4104, 90, 16384), (2056, 1024, 2049), (2056, 1026, 2048), (328, 1024, 50), (328, 1026, 50),
+                                            (2056, 4104, 50), (2048, 4104, 50), (2056, 8192, 50)])
 @pytest.mark.parametrize("design", [nilivik, bifazen])
 def test_one_and_two_rows(ca, hdev, tmp_path, design, width, ff, vocab):
     config, tensors, oracle = design(width, ff, vocab)
