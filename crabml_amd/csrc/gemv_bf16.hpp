@@ -902,19 +902,30 @@ inline size_t gemv16_meet_bytes(int n_cu) { return (size_t)(n_cu / 2) * 4 * size
 // workgroup, as many bytes as 16 rows of weights, and a second round that leaves most CUs without work costs as much as the first.  Us a launch of 16 / 4 rows,
 // workgroups of 16 rows / these: 4608 x 512 5.5 / 4.2 and 4.9 / 3.9, 11264 x 512 7.7 / 4.9 and 6.9 / 4.7, 8192 x 1024 6.95 / 5.6 and 6.1 / 5.4, 12288 x 1024 9.4 / 6.8 and
 // 8.25 / 6.5, 4608 x 2048 8.4 / 7.2 and 6.7 / 6.4, 8192 x 2048 9.2 / 8.65 and 7.8 / 7.8, 9216 x 2048 11.4 / 9.6 and 9.65 / 9.1, 11264 x 2048 12.1 / 10.4 and 10.3 / 10.3,
-// 14336 x 2048 14.8 / 13.3 and 12.8 / 12.9.  Sixteen waves where each has two pieces of k, else eight that start sooner (9216 x 1024 6.35 / 6.2).  More than four
-// tiles a CU: two workgroups of 48 rows on each in turn (against 32 rows: 32000 x 512 11.2 / 9.1, x 1024 14.5 / 13.5, x 2048 24.9 / 24.0, x 4096 48.5 / 44.0).
+// 14336 x 2048 14.8 / 13.3 and 12.8 / 12.9.  Three tiles: sixteen waves where each has two pieces of k, else eight that start sooner
+// (9216 x 1024 6.35 / 6.2).  Two tiles: eight waves with a step each out (16 / 3 rows, workgroups of 16 rows / sixteen waves / these: 4112 x 128 3.26 3.47 3.28 and 3.06 3.31 3.11,
+// 8192 x 512 5.9 4.5 4.3 and 5.3 4.3 4.1, 4112 x 1280 6.9 7.2 5.8 and 5.8 6.5 5.3, 8192 x 1536 8.2 8.0 6.9 and 6.8 7.2 6.7, 8192 x 3072 13.6 12.2 10.8 and 11.2 11.4 10.4), but
+// sixteen with two where rows are 4 KB, which begin on the same memory channels (4608 x 2048 8.45 7.3 7.4 and 6.75 6.5 6.9, 8192 x 2048 9.4 8.8 9.4 and 7.9 7.9 9.1).
+// More than four tiles a CU: workgroups of 48 rows (against 32 rows, two steps out: 32000 x 512 11.2 / 9.1, x 1024 14.5 / 13.5, x 2048 24.9 / 24.0, x 4096 48.5 / 44.0) -- or
+// of 32 with a step out, where 48 leave CUs with one workgroup of the two that fit (16400 rows; 16 rows, 32 rows and two steps / 48 / these: x 512 7.4 6.4 5.75, x 1280 11.6
+// 11.7 10.6, x 3072 21.4 22.9 21.2) or go on in a second round over long rows (32000 x 2560 32.5 30.1 29.8, x 3072 33.6 34.2 33.3, 65536 x 5120 110 111 110, 3 rows 28.3 27.6 26.4,
+// 30.6 32.0 31.0, 97 102 98; x 2048 25.2 24.5 24.0, 65536 x 2048 48.1 45.4 46.7 with 3 rows; one full round: 20000 x 2560 24.3 21.1 22.3).  Never with rows of 8 KB (32000 x
+// 4096 49.8 44.4 48.7).
 // From 4096 columns on eight rows and fewer are as fast or faster in workgroups of 16 (8192 x 4096 12.6 / 15.2).
 template <int SPL, int IN, int OUT, bool NTW>
 inline bool launch_gemv16_round(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a, int n_cu) {
   const int tiles = (a.N + 15) / 16, per = (tiles + n_cu - 1) / n_cu;
   if (per > 4) {
-    launch_gemv16_t<3, SPL, 8, IN, OUT, NTW, 1>(st, rec, a, n_cu);
+    const int wgs = (a.N + 47) / 48;
+    if (a.K % 4096 != 0 && (2 * wgs < 3 * n_cu || (a.K > 2048 && wgs > 2 * n_cu)))
+      launch_gemv16_t<2, SPL, 8, IN, OUT, NTW, 1>(st, rec, a, n_cu);
+    else
+      launch_gemv16_t<3, SPL, 8, IN, OUT, NTW, 1>(st, rec, a, n_cu);
     return true;
   }
   if (per < 2 || a.K >= 4096) return false;
-  if (per == 2 && a.K <= 1024)
-    launch_gemv16_t<2, SPL, 16, IN, OUT, NTW, 1>(st, rec, a, n_cu);
+  if (per == 2 && a.K % 2048 != 0)
+    launch_gemv16_t<2, SPL, 8, IN, OUT, NTW, 1>(st, rec, a, n_cu);
   else if (per == 2)
     launch_gemv16_t<2, SPL, 16, IN, OUT, NTW, 2>(st, rec, a, n_cu);
   else if (per == 3 && a.K <= 1024)

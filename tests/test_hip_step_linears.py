@@ -42,9 +42,11 @@ def test_batched_steps(ca, hdev, tmp_path, design, width, ff, vocab, f32):
             assert np.sqrt((d * d).mean(axis=1)).max() <= (2e-5 if f32 else 2.5e-2) * np.sqrt((want[i] ** 2).mean()), (batch, i)
 
 
-# the classifier in one round of workgroups of 32, 48 and 64 rows, a tile and four rows past each line (of few columns: eight or sixteen waves with a piece of k each or
-# none; of 2090: sixteen with two and a third that some have), two workgroups to a k of 3104 and 3072 columns with a tile that 72 and 2048 rows do not fill and fill
-@pytest.mark.parametrize("width,ff,vocab", [(72, 3100, 4100), (72, 90, 8196), (72, 90, 12292), (72, 90, 16388), (2090, 90, 4100), (2090, 90, 8196), (2090, 90, 12292), (2048, 3072, 50)])
+# the classifier in one round of workgroups of 32, 48 and 64 rows, a tile and four rows past each line (of few columns: eight waves with a piece of k each or none; of
+# 2090: eight or sixteen with several, of 2048: sixteen with two), in rounds of 32 and 48 (either side of one and a half of those a CU, of two of them with long rows, rows
+# of 8 KB); two workgroups to a k of 3104 and 3072 columns with a tile that 72 and 2048 rows do not fill and fill
+@pytest.mark.parametrize("width,ff,vocab", [(72, 3100, 4100), (72, 90, 8196), (72, 90, 12292), (72, 90, 16388), (2090, 90, 4100), (2090, 90, 8196), (2090, 90, 12292), (2048, 3072, 50),
+                                            (2048, 90, 4100), (72, 90, 18434), (2090, 90, 24580), (4096, 90, 16388)])
 def test_one_round_of_workgroups(ca, hdev, tmp_path, width, ff, vocab):
     config, tensors, oracle = nilivik(width, ff, vocab)
     bits = tensors(config, 12, pool=1 << 20)
