@@ -1048,19 +1048,15 @@ inline void launch_gemv2_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, c
 }
 // Eight rows (matmul_vec): the next steps' requests together, behind the products; step by step 8192 x 2048 15.1 us against 9.9, 8192 x 8192 49.1 / 32.0, 32000 x 2048
 // 49.4 / 39.4.  Four rows: step by step 8.0 -> 7.4, 26.3 -> 23.6, 26.6 -> 23.7.
-// rows of the rhs that share one pass over the weights: as many as there are, up to 8
+// rows of the rhs that share one pass over the weights: as many as there are, up to 8; in front of and behind anything else two (a step's linears have no more here)
 template <int IN, int OUT>
 inline void launch_gemv_bf16(hipStream_t st, crabml_hip_device::ProfRec* rec, const GemvBf16& a) {
-  if (a.nb <= 1)
-    launch_gemv1_bf16<IN, OUT>(st, rec, a);
-  else if (a.nb <= 2)
-    launch_gemv2_bf16<IN, OUT>(st, rec, a);
-  else if constexpr (IN == GEMV_IN_PLAIN && OUT == GEMV_OUT_STORE) {
-    if (a.nb <= 4)
-      launch_gemv_bf16_t<4, 4, 2, 4, IN, OUT>(st, rec, a);
-    else
-      launch_gemv_bf16_t<4, 8, 2, 2, IN, OUT, false>(st, rec, a);
+  if (a.nb <= 1) return launch_gemv1_bf16<IN, OUT>(st, rec, a);
+  if constexpr (IN == GEMV_IN_PLAIN && OUT == GEMV_OUT_STORE) {
+    if (a.nb > 4) return launch_gemv_bf16_t<4, 8, 2, 2, IN, OUT, false>(st, rec, a);
+    if (a.nb > 2) return launch_gemv_bf16_t<4, 4, 2, 4, IN, OUT>(st, rec, a);
   }
+  launch_gemv2_bf16<IN, OUT>(st, rec, a);
 }
 
 }  // namespace crabml_hip

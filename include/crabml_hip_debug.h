@@ -74,7 +74,7 @@ int crabml_hip_debug_prompt_gemm(uint32_t dtype, size_t m0, size_t m1, size_t m2
  * workgroups a 32-row chunk.  The launch's grid and what attention touches ahead of it both come from this.  Host only. */
 int crabml_hip_debug_residual_rows(int32_t norm_epilogue, int32_t ordered, int32_t split, int32_t* rows);
 /* Weight rows that a workgroup of a hybrid step's linear over nb > 2 rows takes: n weight rows of k columns, the rhs bf16 rows or f32.  The launch's grid and what the
- * mixer touches ahead of it both come from this.  Host only. */
+ * mixer touches ahead of it both come from this; bf16 rows behind a norm go by another rule from more than 16 rows a CU on (32, 48 or 64).  Host only. */
 int crabml_hip_debug_step_linear_rows(int32_t bf16, int32_t n, int32_t k, int32_t nb, int32_t n_cu, int32_t* rows);
 /* Bytes that a step's attention or mixer launch touches ahead of the linear behind it: m rows, `rows` of them a workgroup, row_bytes + row_bytes2 a row, in a
  * model (llama, hybrid) whose steps read model_bytes of weights.  Host only. */

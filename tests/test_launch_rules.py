@@ -65,7 +65,7 @@ def test_rows_of_the_residual_linears():
 
 
 def test_rows_of_a_steps_linears():
-    """bf16 rows: eight weight rows a workgroup for up to eight of them where sixteen leave half of the CUs idle and the rows are long, thirty-two from 16384 on; f32
+    """bf16 rows (behind no norm, or where there are no more than sixteen weight rows a CU): eight weight rows a workgroup for up to eight of them where sixteen leave half of the CUs idle and the rows are long, thirty-two from 16384 on; f32
     rows never eight.  What the mixer touches ahead of w_o is cut by the same rule."""
     for (bf16, n, k, nb), want in {(1, 2048, 8192, 3): 8, (1, 2048, 2048, 8): 8, (1, 2048, 2048, 9): 16, (1, 2049, 8192, 4): 16, (1, 2048, 2047, 4): 16, (1, 72, 4096, 4): 8,
                                    (0, 2048, 8192, 4): 16, (0, 16384, 2048, 4): 32, (1, 16384, 2048, 4): 32, (1, 16383, 2048, 16): 16}.items():
