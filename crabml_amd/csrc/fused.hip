@@ -434,6 +434,13 @@ void enqueue_attention(crabml_hip_llama* c, int l, signed char* xq, unsigned sho
 // wave where a classifier has many short ones; four waves for q | k | v from 4096 columns on.  ffn_down stages nothing: four waves, two rows where there are many.  Us a launch,
 // four waves and the steps out that were best for them / these: q | k | v 3072 x 2048 5.4 / 4.8, 864 x 288 3.2 / 3.0; wo 2048 x 2048 4.2 / 3.6, 512 x 512 2.6 / 2.2; gate | up of
 // 2 x 8192 x 2048 13.4 / 12.4, 2 x 14336 x 4096 38.1 / 35.4; ffn_down 2048 x 8192 7.6 / 7.4, 512 x 1024 3.1 / 2.6; 32000 x 2048 24.5 / 20.9, 32000 x 288 7.3 / 5.9.
+// More than 2048 columns: two steps out where four end in a round that has one or two to make -- a request past the end is the row's start again -- and for q | k | v below 4096,
+// two rows a wave in a classifier of many rows that are not a multiple of 8 KB.  Us a launch, as it was with four waves / eight and four steps out / these: gate | up of 2 x
+// 8192 x 2560 16.0 / 16.4 / 15.1, x 3072 17.4 / 18.3 / 16.7, 2 x 4096 x 5120 16.4 / 16.7 / 15.6 (x 3584 20.6 / 20.3 / 19.8, x 6144 36.1 / 34.2 / 34.5: four); q | k | v 4608 x 3072
+// 9.1 / 9.7 / 8.0, 5376 x 3584 9.9 / 10.7 / 9.4, 6144 x 4096 11.2 / 11.5 / 11.1, 12288 x 8192 37.2 / 40.5 / 39.7; 32000 x 3072 30.5 / 31.6 / 29.7, x 5120 53.4 / 62.4 / 51.4, x
+// 7168 71.1 / 78.9 / 69.7, x 4096 42.5 / 39.9 / 40.3, x 8192 95.2 / 84.1 / 91.6.  ffn_down of up to 1024 rows from 4096 columns on: eight steps out (four / eight 1024 x 4096 4.05 /
+// 3.76, 512 x 8192 5.2 / 4.8; 2048 x 4096 4.75 / 4.88).  Two rows a wave of it from sixteen a CU on: 8192 x 8192 24.2 / 23.8, x 14336 39.8 / 36.8, 4096 x 14336 20.2 / 20.0, 5120
+// x 8192 15.4 / 16.5.
 template <int WV, int R, int UN, int IN, int OUT>
 void launch_step_f16_t(crabml_hip_device* dev, crabml_hip_device::ProfRec* rec, const StepF16& a, const QkvEpi& e) {
   const int per_wg = WV * (OUT == F16_OUT_GU ? R / 2 : R);
@@ -448,10 +455,10 @@ void launch_step_f16_t(crabml_hip_device* dev, crabml_hip_device::ProfRec* rec, 
   launch_k(dev->stream, rec, k_step_f16<WV, R, UN, 8 / WV, IN, OUT>, grid, dim3(64 * WV), lds, a, e);
 }
 template <int WV, int R, int IN, int OUT>
-void launch_step_f16_u(crabml_hip_device* dev, crabml_hip_device::ProfRec* rec, const StepF16& a, const QkvEpi& e) {
+void launch_step_f16_u(crabml_hip_device* dev, crabml_hip_device::ProfRec* rec, const StepF16& a, const QkvEpi& e, bool two = false) {
   if (a.k <= 512)
     launch_step_f16_t<WV, R, 1, IN, OUT>(dev, rec, a, e);
-  else if (a.k <= 1024)
+  else if (a.k <= 1024 || two)
     launch_step_f16_t<WV, R, 2, IN, OUT>(dev, rec, a, e);
   else
     launch_step_f16_t<WV, R, 4, IN, OUT>(dev, rec, a, e);
@@ -463,19 +470,22 @@ void launch_step_f16(crabml_hip_device* dev, crabml_hip_device::ProfRec* rec, co
     if (a.k >= 4096)
       launch_step_f16_t<4, 2, 4, IN, OUT>(dev, rec, a, e);
     else
-      launch_step_f16_u<8, 2, IN, OUT>(dev, rec, a, e);
+      launch_step_f16_u<8, 2, IN, OUT>(dev, rec, a, e, a.k > 2048);
   } else if constexpr (OUT == F16_OUT_GU) {
-    launch_step_f16_u<8, 2, IN, OUT>(dev, rec, a, e);
+    const int last = (a.k + 511) / 512 % 4;  // steps of a last round of four
+    launch_step_f16_u<8, 2, IN, OUT>(dev, rec, a, e, a.k > 2048 && (last == 1 || last == 2));
   } else if constexpr (OUT == F16_OUT_STORE) {  // (a classifier)
     if (wide && a.k <= 512)
       launch_step_f16_t<8, 4, 1, IN, OUT>(dev, rec, a, e);
-    else if (wide && a.k <= 1024)
+    else if (wide && (a.k <= 1024 || (a.k > 2048 && a.k % 4096 != 0)))
       launch_step_f16_t<8, 2, 2, IN, OUT>(dev, rec, a, e);
     else
       launch_step_f16_u<8, 1, IN, OUT>(dev, rec, a, e);
   } else if constexpr (IN == F16_IN_HALF) {
     if (wide)
       launch_step_f16_t<4, 2, 4, IN, OUT>(dev, rec, a, e);
+    else if (a.m <= 1024 && a.k >= 4096)
+      launch_step_f16_t<4, 1, 8, IN, OUT>(dev, rec, a, e);
     else
       launch_step_f16_u<4, 1, IN, OUT>(dev, rec, a, e);
   } else {

@@ -89,7 +89,8 @@ def test_decode_step_against_the_scalar_order(ca, dim, hidden, heads, kv, vocab,
     assert np.max(err) <= 4 * 2.0 ** -11, err
 
 
-# either side of 512, 1024 and 4096 columns; classifiers either side of sixteen rows a CU
-@pytest.mark.parametrize("dim,hidden,heads,kv,vocab", [(544, 512, 4, 4, 4095), (1024, 1056, 8, 2, 4096), (1056, 4096, 8, 4, 70), (512, 1024, 8, 2, 16400)])
+# either side of 512, 1024, 2048 and 4096 columns; classifiers either side of sixteen rows a CU, of rows of 4096 columns and of others; ffn_down of up to 1024 long rows
+@pytest.mark.parametrize("dim,hidden,heads,kv,vocab", [(544, 512, 4, 4, 4095), (1024, 1056, 8, 2, 4096), (1056, 4096, 8, 4, 70), (512, 1024, 8, 2, 16400), (2080, 544, 20, 4, 4100),
+                                                       (2560, 512, 20, 4, 4095), (3584, 544, 28, 4, 4100), (1024, 4096, 8, 2, 70), (4096, 512, 32, 8, 4100), (5120, 512, 40, 8, 4100)])
 def test_decode_step_forms_against_the_scalar_order(ca, dim, hidden, heads, kv, vocab):
     test_decode_step_against_the_scalar_order(ca, dim, hidden, heads, kv, vocab, True)
