@@ -458,14 +458,16 @@ def test_q4_k_m_mix_on_the_fused_kernels_equals_the_per_op_segments(ca, flags):
     assert list(fused.decode_greedy(3, 20)) == list(per_op.decode_greedy(3, 20))
 
 
-# width, hidden, heads, kv heads: a super-block; one, two and four of them a wave of q | k | v, and rounds of 64 chunk sums likewise; ffn_down's rows of one piece a lane,
-# two, four, and more super-blocks than four a wave; a last workgroup of q | k | v that the rows do not fill
-@pytest.mark.parametrize("dim,hidden,heads,kv", [(256, 16640, 4, 2), (512, 256, 8, 1), (2048, 2304, 16, 5), (2304, 4096, 18, 3), (4096, 4352, 32, 8), (4352, 512, 34, 17), (8192, 1024, 64, 8)])
-@pytest.mark.parametrize("fmt,strict", [("Q4_K", False), ("Q6_K", False), ("mix", False), ("Q4_K", True), ("mix", True)])
+# width, hidden, heads, kv heads: a super-block; one and two of them a wave of q | k | v, and two and four rounds of 64 chunk sums; ffn_down's rows of one piece a lane,
+# two, four, and more super-blocks than four a wave; a last workgroup of q | k | v that the rows do not fill (2496 pairs, ten waves)
+KQ_SHAPES = [(256, 16640, 4, 2), (512, 256, 8, 1), (2048, 2304, 16, 4), (2304, 4096, 18, 3), (3328, 512, 52, 13), (4096, 4352, 32, 8), (4352, 512, 34, 17), (8192, 1024, 64, 8)]
+
+
+# (Q6_K rows of more than 4096 elements run the per-op launches themselves)
+@pytest.mark.parametrize("fmt,strict,dim,hidden,heads,kv", [(f, strict, *shape) for f, strict in [("Q4_K", False), ("Q6_K", False), ("mix", False), ("Q4_K", True), ("mix", True)]
+                                                            for shape in KQ_SHAPES if f != "Q6_K" or shape[0] <= 4096])
 def test_k_quant_step_equals_the_per_op_segments(ca, fmt, strict, dim, hidden, heads, kv):
     """Q4_K, Q6_K and *_K_M layers whose launches quantize their rhs themselves: the logits of the per-op launches (flag 256), bit for bit."""
-    if heads % kv:
-        kv = 1
     shape = synth.ModelShape("kq", dim, hidden, 2, heads, kv, 512, 64)
     model = synth.build_model(shape, synth.Q6_K if fmt == "Q6_K" else synth.Q4_K, seed=dim + hidden, k_m_mix=fmt == "mix")
     dev = ca.HipTensorDevice(0, False, 0, strict)
