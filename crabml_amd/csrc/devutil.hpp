@@ -291,7 +291,7 @@ __device__ __forceinline__ unsigned q8k_class_major(int lane, unsigned packed) {
   return __builtin_amdgcn_perm(b, packed, lane & 4 ? 0x03020706u : 0x05040100u);
 }
 __device__ __forceinline__ int q8k_class_major_at(int lane) { return (lane >> 3) * 8 + (lane & 1) * 4 + ((lane >> 1) & 3); }
-// (`in`: lanes that store; whole groups of 8)
+// (`in`: lanes that store, each a whole dword of its own)
 __device__ __forceinline__ void q8k_store_class_major(signed char* sb_base, int lane, unsigned packed, bool in = true) {
   const unsigned d = q8k_class_major(lane, packed);
   if (in) ((unsigned*)sb_base)[q8k_class_major_at(lane)] = d;

@@ -1781,8 +1781,9 @@ int prefill_chunk(crabml_hip_llama* c, const uint32_t* tokens, size_t B, size_t 
     k_qkv_epi_rows<<<dim3((pairs + 255) / 256, rows), 256, 0, st>>>(c->pf_q, c->pf_k, c->pf_v, e);
     int along = 0;
     // (a pass whose every row sees fewer cached positions than the decode step's switch to the f32 kernels -- attn_long_from --
-    // keeps the exact tile kernel, so that prefill(prompt) and a token loop over the same short prompt agree bit for bit -- where the step
-    // runs the exact chain there too: not Q4_0 / Q8_0 layers with deferred norms, which run k_attn_short)
+    // keeps the exact tile kernel, so that prefill(prompt) and a token loop over the same short prompt agree bit for bit on strict devices, and on fast
+    // ones while every matrix stays on the row kernels (up to 4 rows, up to 15 in small matrices: gemm_mfma_few) and the step runs the exact chain
+    // there too: not Q4_0 / Q8_0 layers with deferred norms, which run k_attn_short)
     if (c->attn_flash_rows && kv16 && pos0 + B >= c->attn_long_from) {
       // fast step: causal flash attention on the f16 matrix cores (k_attn_flash_rows; the deviation stated for k_attn_flash)
       const dim3 fg((unsigned)((B + 63) / 64), (unsigned)n_heads);

@@ -273,8 +273,10 @@ int crabml_hip_llama_decode_greedy(crabml_hip_llama_t* ctx, size_t token, size_t
  * BLOCKS), the logits of the last prompt token.  The reference's own `_batched` flag is ignored (llama2.rs:114)
  * and its batch_matmul has no causal mask for n_batch > 1; here every row attends to the cache up to its own
  * position, which is what the token loop computes.  Weight matrices see the prompt as a (rows, k) rhs: the
- * matmul_vec contract (matmul_vec.rs:6-8), on the matrix cores for Q4_0 / Q8_0 weights and >= 16 rows.  Strict-order
- * devices: bit-identical to the token loop.  tp_size > 1: falls back to the token loop. */
+ * matmul_vec contract (matmul_vec.rs:6-8).  Fast devices run it on the matrix cores: F16 weights from 2 rows on, Q4_0 / Q8_0 /
+ * Q4_1 / Q4_K from 16 rows on, in large matrices from 5 (another association of the same f32 sums), those and Q6_K from 32 rows
+ * on with the block scales folded into f16 operands; fewer rows and other formats go row by row.  Strict-order devices:
+ * bit-identical to the token loop.  tp_size > 1: falls back to the token loop. */
 int crabml_hip_llama_prefill(crabml_hip_llama_t* ctx, const uint32_t* tokens, size_t n, float* logits);
 size_t crabml_hip_llama_kv_len(const crabml_hip_llama_t* ctx);
 int crabml_hip_llama_reset(crabml_hip_llama_t* ctx); /* empties the KV caches */
