@@ -8,7 +8,7 @@
 // Every row's pieces are added by lane, ascending, as k_gemv_q4_k / k_gemv_q6_k add them, the norm's sums in k_norm_f32's order: the planes and logits are the per-op
 // launches' bit for bit.
 // Us a launch of the 8B shape, Q4_K, with planes from the producer / these: q | k | v 5.6 / 5.8, wo 5.6 / 4.4, gate | up 16.6 / 13.7 (4.8 TB/s), ffn_down 11.2 / 9.0; on the
-// strict-order device (ORD) 6.5 / 8.8, 10.7 / 5.5, 19.0 / 18.0, 16.2 / 12.4.  A token of four layers 269 -> 242, of Q6_K (fourteen launches a layer and the attention before)
+// strict-order device (ORD) 7.2 / 9.6, 11.3 / 5.6, 19.8 / 18.7, 16.8 / 12.4 (in a kernel trace).  A token of four layers 269 -> 242, of Q6_K (fourteen launches a layer and the attention before)
 // 407 -> 297; width 2048, six layers, Q4_K 222 -> 192, Q6_K 363 -> 214.
 #pragma once
 #include "fused_ffn.hpp"
